@@ -6,12 +6,14 @@ objects are linked into one shared library next to this file.
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libtokspur_hip.so")
 HOST_LIB = os.path.join(HERE, "libtokspur_graph.so")
+BINDING = os.path.join(HERE, "_native.so")
 
 HIP_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++20", "-fPIC", "-ffp-contract=off", "-fno-gpu-rdc",
@@ -52,6 +54,16 @@ def build(verbose=False, jobs=8):
     return LIB
 
 
+def build_binding():
+    """The CPython module over the C ABI that capi.Device calls through: binding.cpp -> _native.so, next to the library it links."""
+    cmd = ["g++", "-std=c++20", "-O2", "-fPIC", "-shared", "-Wall", os.path.join(HERE, "binding.cpp"), "-I", sysconfig.get_path("include"),
+           "-L", HERE, "-ltokspur_hip", "-Wl,-rpath,$ORIGIN", "-Wl,--allow-shlib-undefined", "-o", BINDING]
+    proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if proc.returncode:
+        raise RuntimeError(f"Python binding build failed:\n{proc.stdout}")
+    return BINDING
+
+
 def build_host():
     """The C++ host side over the C ABI (tokspur::HipGraph, the GGUF reader and the Pack v3 builder / adopter): host/*.cpp -> libtokspur_graph.so."""
     root = os.path.dirname(HERE)
@@ -84,4 +96,5 @@ def build_native_tests():
 
 if __name__ == "__main__":
     print(build(verbose="-v" in sys.argv))
+    print(build_binding())
     print(build_host())

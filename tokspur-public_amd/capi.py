@@ -2,9 +2,12 @@
 
 The library must have been built (python -m build step or __graft_entry__.build()); loading fails
 loudly when libtokspur_hip.so is missing — there is no fallback path of any kind. `Device` wraps
-torch tensors as device buffers and calls every device entry point on torch's current stream.
+torch tensors as device buffers and calls every device entry point on torch's current stream. Host
+functions go through ctypes, device entry points through the compiled module `_native` (binding.cpp),
+which costs a fifth of it per call.
 """
 import ctypes as C
+import importlib
 import os
 
 import numpy as np
@@ -53,6 +56,20 @@ def dll():
         _dll.tsp_last_error.restype = C.c_char_p
         _dll.tsp_abi_version.restype = C.c_uint32
     return _dll
+
+
+_module = None
+
+
+def native():
+    """The compiled binding of the device entry points."""
+    global _module
+    if _module is None:
+        dll()
+        if not os.path.exists(os.path.join(HERE, "_native.so")):
+            raise RuntimeError(f"{HERE}/_native.so is missing: build it with __graft_entry__.build() — there is no fallback")
+        _module = importlib.import_module("._native", __package__)
+    return _module
 
 
 def check(status):
@@ -214,7 +231,9 @@ class Device:
             raise RuntimeError("no GPU: the HIP path cannot run and there is no CPU fallback")
         self.dev = torch.device("cuda", torch.cuda.current_device())
         self.err = torch.zeros(1, dtype=torch.int32, device=self.dev)
-        dll()
+        self.native = native()
+        # the handle of the current device's current stream; torch's stream object costs 2.7 us to make, these two calls 0.15
+        self._raw_stream, self._current_device = torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice
 
     # -- memory
     def upload(self, a):
@@ -244,8 +263,11 @@ class Device:
     def nbytes(t):
         return t.numel() * t.element_size()
 
+    def _stream(self):
+        return self._raw_stream(self._current_device())
+
     def stream(self):
-        return C.c_void_p(self.torch.cuda.current_stream().cuda_stream)
+        return C.c_void_p(self._stream())
 
     def sync(self):
         self.torch.cuda.synchronize()
@@ -262,8 +284,7 @@ class Device:
     # -- operators
     def dequantize(self, t, blocks, nelem):
         out = self.empty(nelem)
-        check(dll().tsp_dequantize(C.c_uint32(t), self.ptr(blocks), C.c_uint64(self.nbytes(blocks)), self.ptr(out),
-                                   C.c_uint64(nelem), self.ptr(self.err), self.stream()))
+        check(self.native.dequantize(t, blocks, blocks.nbytes, out, nelem, self.err, self._stream()))
         return out
 
     def dequantize_planar(self, spec, planar):
@@ -274,35 +295,29 @@ class Device:
     def gemv(self, t, matrix, x, columns, rows, layout=LAYOUT_GGUF, y=None, matrix_bytes=None):
         y = self.empty(rows) if y is None else y
         nbytes = self.nbytes(matrix) if matrix_bytes is None else matrix_bytes
-        check(dll().tsp_gemv(C.c_uint32(t), C.c_uint32(layout), self.ptr(matrix), C.c_uint64(nbytes), self.ptr(x), self.ptr(y),
-                             C.c_uint32(columns), C.c_uint32(rows), self.ptr(self.err), self.stream()))
+        check(self.native.gemv(t, layout, matrix, nbytes, x, y, columns, rows, self.err, self._stream()))
         return y
 
     def gemv_rows(self, t, matrix, x, y, count, columns, rows, x_stride, y_stride, layout=LAYOUT_GGUF):
-        check(dll().tsp_gemv_rows(C.c_uint32(t), C.c_uint32(layout), self.ptr(matrix), C.c_uint64(self.nbytes(matrix)), self.ptr(x),
-                                  C.c_uint64(x_stride), self.ptr(y), C.c_uint64(y_stride), C.c_uint32(count), C.c_uint32(columns),
-                                  C.c_uint32(rows), self.ptr(self.err), self.stream()))
+        check(self.native.gemv_rows(t, layout, matrix, matrix.nbytes, x, x_stride, y, y_stride, count, columns, rows, self.err, self._stream()))
         return y
 
     def q8_matvec_many(self, matrix, x, columns, rows, width, layout=LAYOUT_GGUF, y=None):
         y = self.empty((width, rows)) if y is None else y
-        check(dll().tsp_q8_matvec_many(C.c_uint32(layout), self.ptr(matrix), C.c_uint64(self.nbytes(matrix)), self.ptr(x), self.ptr(y),
-                                       C.c_uint32(columns), C.c_uint32(rows), C.c_uint32(width), self.ptr(self.err), self.stream()))
+        check(self.native.q8_matvec_many(layout, matrix, matrix.nbytes, x, y, columns, rows, width, self.err, self._stream()))
         return y
 
     def routed_gemv(self, t, matrices, ids, x, columns, rows, experts, selected, broadcast):
         y = self.empty((selected, rows))
-        check(dll().tsp_routed_gemv(C.c_uint32(t), self.ptr(matrices), C.c_uint64(self.nbytes(matrices)), self.ptr(ids), self.ptr(x),
-                                    self.ptr(y), C.c_uint32(columns), C.c_uint32(rows), C.c_uint32(experts), C.c_uint32(selected),
-                                    C.c_int(bool(broadcast)), self.ptr(self.err), self.stream()))
+        check(self.native.routed_gemv(t, matrices, matrices.nbytes, ids, x, y, columns, rows, experts, selected, bool(broadcast), self.err,
+                                      self._stream()))
         return y
 
     def router_f32_batch(self, weights, x, tokens, columns, experts, x_stride=None, out=None, out_stride=None):
         """logits[t, e] = sum_k weights[e, k] * x[t, k] for a whole chunk of token rows in one f32 GEMM."""
         out = self.empty((tokens, experts)) if out is None else out
-        check(dll().tsp_router_f32_batch(self.ptr(weights), self.ptr(x), C.c_uint64(columns * 4 if x_stride is None else x_stride),
-                                         self.ptr(out), C.c_uint64(experts * 4 if out_stride is None else out_stride), C.c_uint32(columns),
-                                         C.c_uint32(experts), C.c_uint32(tokens), self.ptr(self.err), self.stream()))
+        check(self.native.router_f32_batch(weights, x, columns * 4 if x_stride is None else x_stride, out,
+                                           experts * 4 if out_stride is None else out_stride, columns, experts, tokens, self.err, self._stream()))
         return out
 
     def route(self, logits, selected, mode=0, normalize=True, tokens=None, out=None):
@@ -311,89 +326,68 @@ class Device:
         n = 1 if tokens is None else tokens
         ids, w = out if out is not None else (self.zeros((n, selected), "int32"), self.zeros((n, selected)))
         if tokens is None:
-            check(dll().tsp_route(self.ptr(logits), self.ptr(ids), self.ptr(w), C.c_uint32(experts), C.c_uint32(selected), C.c_uint32(mode),
-                                  C.c_int(bool(normalize)), self.ptr(self.err), self.stream()))
+            check(self.native.route(logits, ids, w, experts, selected, mode, bool(normalize), self.err, self._stream()))
         else:
-            check(dll().tsp_route_batch(self.ptr(logits), self.ptr(ids), self.ptr(w), C.c_uint32(experts), C.c_uint32(selected),
-                                        C.c_uint32(tokens), C.c_uint32(mode), C.c_int(bool(normalize)), self.ptr(self.err), self.stream()))
+            check(self.native.route_batch(logits, ids, w, experts, selected, tokens, mode, bool(normalize), self.err, self._stream()))
         return ids, w
 
     def mixture(self, expert_out, weights, shared, shared_logit, channels, selected, tokens=1, out=None, out_stride=None):
         out = self.empty((tokens, channels)) if out is None else out
         stride = channels * 4 if out_stride is None else out_stride
-        check(dll().tsp_mixture_batch(self.ptr(expert_out), self.ptr(weights), self.ptr(shared), self.ptr(shared_logit), self.ptr(out),
-                                      C.c_uint64(stride), C.c_uint32(channels), C.c_uint32(selected), C.c_uint32(tokens),
-                                      self.ptr(self.err), self.stream()))
+        check(self.native.mixture_batch(expert_out, weights, shared, shared_logit, out, stride, channels, selected, tokens, self.err, self._stream()))
         return out
 
     def swiglu(self, gate, up, scale=1.0, out=None):
         out = self.empty(gate.shape) if out is None else out
-        check(dll().tsp_swiglu(self.ptr(gate), self.ptr(up), self.ptr(out), C.c_uint64(gate.numel()), C.c_float(scale),
-                               self.ptr(self.err), self.stream()))
+        check(self.native.swiglu(gate, up, out, gate.numel(), scale, self.err, self._stream()))
         return out
 
     def rms(self, x, gains, group_width, epsilon, gate=None, out=None):
         out = self.empty(x.shape) if out is None else out
         shared = int(gains.numel() == group_width and x.numel() != group_width)
         if gate is None:
-            check(dll().tsp_rms(self.ptr(x), self.ptr(gains), self.ptr(out), C.c_uint64(x.numel()), C.c_uint32(group_width), C.c_int(shared),
-                                C.c_float(epsilon), self.ptr(self.err), self.stream()))
+            check(self.native.rms(x, gains, out, x.numel(), group_width, shared, epsilon, self.err, self._stream()))
         else:
-            check(dll().tsp_rms_sigmoid_gate(self.ptr(x), self.ptr(gains), self.ptr(gate), self.ptr(out), C.c_uint64(x.numel()), C.c_uint32(group_width),
-                                             C.c_int(shared), C.c_float(epsilon), self.ptr(self.err), self.stream()))
+            check(self.native.rms_sigmoid_gate(x, gains, gate, out, x.numel(), group_width, shared, epsilon, self.err, self._stream()))
         return out
 
     def activate(self, x, kind, scale=1.0, out=None):
         out = self.empty(x.shape) if out is None else out
-        check(dll().tsp_activate(self.ptr(x), self.ptr(out), C.c_uint64(x.numel()), C.c_uint32(kind), C.c_float(scale), self.ptr(self.err), self.stream()))
+        check(self.native.activate(x, out, x.numel(), kind, scale, self.err, self._stream()))
         return out
 
     def multiply(self, x, gate, sigmoid_gate=False, out=None):
         out = self.empty(x.shape) if out is None else out
-        check(dll().tsp_multiply(self.ptr(x), self.ptr(gate), self.ptr(out), C.c_uint64(x.numel()), C.c_int(bool(sigmoid_gate)), self.ptr(self.err), self.stream()))
+        check(self.native.multiply(x, gate, out, x.numel(), bool(sigmoid_gate), self.err, self._stream()))
         return out
 
     def residual_read(self, normalized, scores, inject, branches, channels, out=None, scales=None):
         out = self.empty(channels) if out is None else out
         scales = self.empty(branches) if scales is None else scales
-        check(dll().tsp_residual_read(self.ptr(normalized), self.ptr(scores), self.ptr(inject), self.ptr(out), self.ptr(scales), C.c_uint32(branches),
-                                      C.c_uint32(channels), self.ptr(self.err), self.stream()))
+        check(self.native.residual_read(normalized, scores, inject, out, scales, branches, channels, self.err, self._stream()))
         return out, scales
 
     def residual_write(self, streams, x, scales, branches, channels, out=None):
         out = self.empty(streams.shape) if out is None else out
-        check(dll().tsp_residual_write(self.ptr(streams), self.ptr(x), self.ptr(scales), self.ptr(out), C.c_uint32(branches), C.c_uint32(channels),
-                                       self.ptr(self.err), self.stream()))
+        check(self.native.residual_write(streams, x, scales, out, branches, channels, self.err, self._stream()))
         return out
 
     def grouped_routes(self, ids, experts, selected, tokens, fill=0xDEADBEEF):
         token_map = self.full((experts, tokens), np.int32(np.uint32(fill).view(np.int32)), "int32")
         counts = self.zeros(experts, "int32")
-        check(dll().tsp_grouped_routes(self.ptr(ids), self.ptr(token_map), self.ptr(counts), C.c_uint32(experts), C.c_uint32(selected),
-                                       C.c_uint32(tokens), self.ptr(self.err), self.stream()))
+        check(self.native.grouped_routes(ids, token_map, counts, experts, selected, tokens, self.err, self._stream()))
         return token_map, counts
 
     def grouped_tasks(self, counts, experts, selected, tokens, tile=32):
         bound = tokens * selected // tile + experts
         tasks = self.zeros(2 + 2 * bound, "int32")
-        check(dll().tsp_grouped_tasks(self.ptr(counts), self.ptr(tasks), C.c_uint32(experts), C.c_uint32(selected), C.c_uint32(tokens),
-                                      C.c_uint32(tile), self.ptr(self.err), self.stream()))
+        check(self.native.grouped_tasks(counts, tasks, experts, selected, tokens, tile, self.err, self._stream()))
         return tasks
 
     def union_build(self, ids, experts, selected, tokens, hidden, channels, poison=0xBAADF00D):
         meta = self.full(2320, np.int32(np.uint32(poison).view(np.int32)), "int32")
-        check(dll().tsp_planar_union_build(self.ptr(ids), self.ptr(meta), C.c_uint32(experts), C.c_uint32(selected), C.c_uint32(tokens),
-                                           C.c_uint32(hidden), C.c_uint32(channels), self.ptr(self.err), self.stream()))
+        check(self.native.planar_union_build(ids, meta, experts, selected, tokens, hidden, channels, self.err, self._stream()))
         return meta
-
-
-class SmallMoe(C.Structure):
-    _fields_ = [("pair_lo", C.c_void_p), ("pair_hi", C.c_void_p), ("down", C.c_void_p),
-                ("gate_kind", C.c_uint32), ("up_kind", C.c_uint32), ("down_kind", C.c_uint32),
-                ("channels", C.c_uint32), ("hidden", C.c_uint32), ("experts", C.c_uint32), ("selected", C.c_uint32),
-                ("tokens", C.c_uint32), ("ids", C.c_void_p), ("x", C.c_void_p), ("x_stride_bytes", C.c_uint64),
-                ("h", C.c_void_p), ("h_stride_bytes", C.c_uint64), ("y", C.c_void_p), ("y_stride_bytes", C.c_uint64),
-                ("union_meta", C.c_void_p), ("error_word", C.c_void_p)]
 
 
 COLOC_KINDS = {12: (2, 3), 13: (4, 5), 8: (6, 7)}
@@ -415,27 +409,22 @@ class PlanarMoeWeights:
         self.union_meta = dev.zeros(2320, "int32")
 
 
-def _small_moe(dev, w, ids, x, tokens, selected, h, y, x_stride=None, h_stride=None, y_stride=None):
+def _routed_m8(dev, with_down, w, ids, x, tokens, selected, h, y, shared=None, shared_h=None, shared_y=None, shared_y_stride=None,
+               x_stride=None, h_stride=None, y_stride=None):
     gate_kind, up_kind = COLOC_KINDS[w.gu_type]
-    m = SmallMoe(w.pair_lo.data_ptr(), w.pair_hi.data_ptr(), w.down.data_ptr() if y is not None else None,
-                 gate_kind, up_kind, DOWN_KINDS[w.dn_type], w.channels, w.hidden, w.experts, selected, tokens,
-                 ids.data_ptr(), x.data_ptr(), w.channels * 4 if x_stride is None else x_stride,
-                 h.data_ptr(), w.hidden * 4 if h_stride is None else h_stride,
-                 y.data_ptr() if y is not None else None, w.channels * 4 if y_stride is None else y_stride,
-                 w.union_meta.data_ptr(), dev.err.data_ptr())
-    return m
+    row, h_row = w.channels * 4, w.hidden * 4
+    gate, up, down = (None, None, None) if shared is None else (shared.gate, shared.up, shared.down)
+    check(dev.native.routed_m8(
+        with_down, w.pair_lo, w.pair_hi, w.down if with_down else None, gate_kind, up_kind, DOWN_KINDS[w.dn_type], w.channels, w.hidden, w.experts,
+        selected, tokens, ids, x, row if x_stride is None else x_stride, h, h_row if h_stride is None else h_stride, y,
+        row if y_stride is None else y_stride, w.union_meta, dev.err, gate, up, down, shared_h, h_row, shared_y,
+        row if shared_y_stride is None else shared_y_stride, dev._stream()))
 
 
 def planar_moe_gate_up_swiglu_m8(dev, w, ids, x, tokens, selected, h=None, **strides):
     h = dev.empty((tokens * selected, w.hidden)) if h is None else h
-    m = _small_moe(dev, w, ids, x, tokens, selected, h, None, **strides)
-    check(dll().tsp_planar_moe_gate_up_swiglu_m8(C.byref(m), dev.stream()))
+    _routed_m8(dev, False, w, ids, x, tokens, selected, h, None, **strides)
     return h
-
-
-class SharedRows(C.Structure):
-    _fields_ = [("gate", C.c_void_p), ("up", C.c_void_p), ("down", C.c_void_p), ("h", C.c_void_p), ("h_stride_bytes", C.c_uint64),
-                ("y", C.c_void_p), ("y_stride_bytes", C.c_uint64)]
 
 
 def planar_moe_routed_m8(dev, w, ids, x, tokens, selected, h=None, y=None, shared=None, shared_h=None, shared_y=None, shared_y_stride=None,
@@ -444,34 +433,20 @@ def planar_moe_routed_m8(dev, w, ids, x, tokens, selected, h=None, y=None, share
     its rows [tokens, channels] come back as the third result."""
     h = dev.empty((tokens * selected, w.hidden)) if h is None else h
     y = dev.empty((tokens * selected, w.channels)) if y is None else y
-    m = _small_moe(dev, w, ids, x, tokens, selected, h, y, **strides)
     if shared is None:
-        check(dll().tsp_planar_moe_routed_m8(C.byref(m), dev.stream()))
+        _routed_m8(dev, True, w, ids, x, tokens, selected, h, y, **strides)
         return h, y
     shared_h = dev.empty((tokens, w.hidden)) if shared_h is None else shared_h
     shared_y = dev.empty((tokens, w.channels)) if shared_y is None else shared_y
-    e = SharedRows(shared.gate.data_ptr(), shared.up.data_ptr(), shared.down.data_ptr(), shared_h.data_ptr(), w.hidden * 4,
-                   shared_y.data_ptr(), w.channels * 4 if shared_y_stride is None else shared_y_stride)
-    check(dll().tsp_planar_moe_routed_m8_shared(C.byref(m), C.byref(e), dev.stream()))
+    _routed_m8(dev, True, w, ids, x, tokens, selected, h, y, shared, shared_h, shared_y, shared_y_stride, **strides)
     return h, y, shared_y
-
-
-class GroupedMoe(C.Structure):
-    _fields_ = [("pair_lo", C.c_void_p), ("pair_hi", C.c_void_p), ("down", C.c_void_p),
-                ("gate_kind", C.c_uint32), ("up_kind", C.c_uint32), ("down_kind", C.c_uint32),
-                ("channels", C.c_uint32), ("hidden", C.c_uint32), ("experts", C.c_uint32), ("selected", C.c_uint32),
-                ("tokens", C.c_uint32), ("ids", C.c_void_p), ("x", C.c_void_p), ("x_stride_bytes", C.c_uint64),
-                ("y", C.c_void_p), ("y_stride_bytes", C.c_uint64), ("token_map", C.c_void_p), ("counts", C.c_void_p),
-                ("tasks", C.c_void_p), ("workspace", C.c_void_p), ("workspace_bytes", C.c_uint64), ("error_word", C.c_void_p)]
 
 
 def dense_mm_q8(dev, layout, matrix, x, tokens, columns, rows, out=None, x_stride=None, out_stride=None):
     """Dense Q8_0 GEMM (`dense_mm_q8`): out[t] = W x[t], GGUF rows or q8_lanes_v1 rows, f32 rows with byte strides."""
     out = dev.empty((tokens, rows)) if out is None else out
-    check(dll().tsp_dense_mm_q8(C.c_uint32(layout), dev.ptr(matrix), C.c_uint64(dev.nbytes(matrix)), dev.ptr(x),
-                                C.c_uint64(columns * 4 if x_stride is None else x_stride), dev.ptr(out),
-                                C.c_uint64(rows * 4 if out_stride is None else out_stride), C.c_uint32(tokens), C.c_uint32(columns),
-                                C.c_uint32(rows), dev.ptr(dev.err), dev.stream()))
+    check(dev.native.dense_mm_q8(layout, matrix, matrix.nbytes, x, columns * 4 if x_stride is None else x_stride, out,
+                                 rows * 4 if out_stride is None else out_stride, tokens, columns, rows, dev.err, dev._stream()))
     return out
 
 
@@ -487,10 +462,9 @@ def dense_mm_q8_staged(dev, layout, matrix, x, tokens, columns, rows, out=None, 
     f.restype = C.c_uint64
     out = dev.empty((tokens, rows)) if out is None else out
     workspace = dev.empty(f(C.c_uint32(tokens), C.c_uint32(columns), C.c_uint32(rows)), "uint8") if workspace is None else workspace
-    check(dll().tsp_dense_mm_q8_staged(C.c_uint32(layout), dev.ptr(matrix), C.c_uint64(dev.nbytes(matrix)), dev.ptr(x),
-                                       C.c_uint64(columns * 4 if x_stride is None else x_stride), dev.ptr(out),
-                                       C.c_uint64(rows * 4 if out_stride is None else out_stride), C.c_uint32(tokens), C.c_uint32(columns),
-                                       C.c_uint32(rows), dev.ptr(workspace), C.c_uint64(dev.nbytes(workspace)), dev.ptr(dev.err), dev.stream()))
+    check(dev.native.dense_mm_q8_staged(layout, matrix, matrix.nbytes, x, columns * 4 if x_stride is None else x_stride, out,
+                                        rows * 4 if out_stride is None else out_stride, tokens, columns, rows, workspace, workspace.nbytes, dev.err,
+                                        dev._stream()))
     return out
 
 
@@ -511,12 +485,10 @@ def grouped_mm(dev, encoding, matrices, ids, x, columns, rows, experts, selected
         scratch = {"token_map": dev.zeros(experts * tokens, "int32"), "counts": dev.zeros(experts, "int32"),
                    "tasks": dev.zeros(2 + 2 * (routes // 32 + experts), "int32"),
                    "workspace": dev.empty(f(C.c_uint32(tokens), C.c_uint32(selected), C.c_uint32(experts), C.c_uint32(columns), C.c_int(bool(broadcast))), "uint8")}
-    check(dll().tsp_grouped_mm(C.c_uint32(encoding), C.c_uint32(layout), dev.ptr(matrices), C.c_uint64(dev.nbytes(matrices)), dev.ptr(ids),
-                               dev.ptr(x), C.c_uint64(columns * 4 if x_stride is None else x_stride), dev.ptr(out),
-                               C.c_uint64(rows * 4 if out_stride is None else out_stride), dev.ptr(scratch["token_map"]), dev.ptr(scratch["counts"]),
-                               dev.ptr(scratch["tasks"]), C.c_uint32(columns), C.c_uint32(rows), C.c_uint32(experts), C.c_uint32(selected),
-                               C.c_uint32(tokens), C.c_int(bool(broadcast)), dev.ptr(scratch["workspace"]), C.c_uint64(dev.nbytes(scratch["workspace"])),
-                               dev.ptr(dev.err), dev.stream()))
+    check(dev.native.grouped_mm(encoding, layout, matrices, matrices.nbytes, ids, x, columns * 4 if x_stride is None else x_stride, out,
+                                rows * 4 if out_stride is None else out_stride, scratch["token_map"], scratch["counts"], scratch["tasks"], columns,
+                                rows, experts, selected, tokens, bool(broadcast), scratch["workspace"], scratch["workspace"].nbytes, dev.err,
+                                dev._stream()))
     return out, scratch
 
 
@@ -536,10 +508,8 @@ def dense_mm(dev, encoding, layout, matrix, x, tokens, columns, rows, out=None, 
         workspace = dev.empty(dense_mm_workspace_bytes(tokens, columns), "uint8")
     xs = (columns * (2 if in_bf16 else 4)) if x_stride is None else x_stride
     os_ = (rows * (2 if out_bf16 else 4)) if out_stride is None else out_stride
-    check(dll().tsp_dense_mm(C.c_uint32(encoding), C.c_uint32(layout), dev.ptr(matrix), C.c_uint64(dev.nbytes(matrix)), dev.ptr(x),
-                             C.c_uint64(xs), C.c_int(bool(in_bf16)), dev.ptr(out), C.c_uint64(os_), C.c_int(bool(out_bf16)),
-                             C.c_uint32(tokens), C.c_uint32(columns), C.c_uint32(rows), dev.ptr(workspace),
-                             C.c_uint64(dev.nbytes(workspace)), dev.ptr(dev.err), dev.stream()))
+    check(dev.native.dense_mm(encoding, layout, matrix, matrix.nbytes, x, xs, bool(in_bf16), out, os_, bool(out_bf16), tokens, columns, rows,
+                              workspace, workspace.nbytes, dev.err, dev._stream()))
     return out
 
 
@@ -558,10 +528,6 @@ class GroupedScratch:
         self.workspace = dev.empty(size, "uint8")
 
 
-class SharedExpert(C.Structure):
-    _fields_ = [("gate", C.c_void_p), ("up", C.c_void_p), ("down", C.c_void_p), ("y", C.c_void_p), ("y_stride_bytes", C.c_uint64)]
-
-
 class PlanarSharedExpert:
     """One always-on expert in the routed experts' formats: Q4_K gate and up as one Pack v3 expert each, Q6_K planes down."""
 
@@ -578,19 +544,17 @@ def planar_nax_grouped_moe(dev, w, ids, x, tokens, selected, scratch, y=None, x_
     rows come back as the second result."""
     y = dev.empty((tokens * selected, w.channels)) if y is None else y
     gate_kind, up_kind = COLOC_KINDS[w.gu_type]
-    m = GroupedMoe(w.pair_lo.data_ptr(), w.pair_hi.data_ptr(), w.down.data_ptr(), gate_kind, up_kind, DOWN_KINDS[w.dn_type],
-                   w.channels, w.hidden, w.experts, selected, tokens, ids.data_ptr(), x.data_ptr(),
-                   w.channels * 4 if x_stride is None else x_stride, y.data_ptr(), w.channels * 4 if y_stride is None else y_stride,
-                   scratch.token_map.data_ptr(), scratch.counts.data_ptr(), scratch.tasks.data_ptr(), scratch.workspace.data_ptr(),
-                   dev.nbytes(scratch.workspace), dev.err.data_ptr())
-    if shared is None:
-        check(dll().tsp_planar_nax_grouped_moe(C.byref(m), dev.stream()))
-        return y
-    shared_y = dev.empty((tokens, w.channels)) if shared_y is None else shared_y
-    e = SharedExpert(shared.gate.data_ptr(), shared.up.data_ptr(), shared.down.data_ptr(), shared_y.data_ptr(),
-                     w.channels * 4 if shared_y_stride is None else shared_y_stride)
-    check(dll().tsp_planar_nax_grouped_moe_shared(C.byref(m), C.byref(e), dev.stream()))
-    return y, shared_y
+    row = w.channels * 4
+    gate, up, down = None, None, None
+    if shared is not None:
+        gate, up, down = shared.gate, shared.up, shared.down
+        shared_y = dev.empty((tokens, w.channels)) if shared_y is None else shared_y
+    check(dev.native.grouped_moe(
+        w.pair_lo, w.pair_hi, w.down, gate_kind, up_kind, DOWN_KINDS[w.dn_type], w.channels, w.hidden, w.experts, selected, tokens, ids, x,
+        row if x_stride is None else x_stride, y, row if y_stride is None else y_stride, scratch.token_map, scratch.counts, scratch.tasks,
+        scratch.workspace, scratch.workspace.nbytes, dev.err, gate, up, down, shared_y, row if shared_y_stride is None else shared_y_stride,
+        dev._stream()))
+    return y if shared is None else (y, shared_y)
 
 
 class KernelTime(C.Structure):
@@ -636,8 +600,7 @@ def logit_topk(dev, logits, rows, vocabulary, stride_bytes=None, scratch=None, o
     stride_bytes = vocabulary * 4 if stride_bytes is None else stride_bytes
     scratch = dev.empty(logit_topk_scratch_bytes(rows, vocabulary), "uint8") if scratch is None else scratch
     out = dev.empty(logit_topk_output_bytes(rows), "uint8") if out is None else out
-    check(dll().tsp_logit_topk(dev.ptr(logits), C.c_uint64(stride_bytes), C.c_uint32(rows), C.c_uint32(vocabulary), dev.ptr(scratch),
-                               C.c_uint64(dev.nbytes(scratch)), dev.ptr(out), C.c_uint64(dev.nbytes(out)), dev.stream()))
+    check(dev.native.logit_topk(logits, stride_bytes, rows, vocabulary, scratch, scratch.nbytes, out, out.nbytes, dev._stream()))
     return out
 
 
@@ -646,14 +609,13 @@ def logit_topk_static(dev, logits, rows, vocabulary, stride_bytes=None, out=None
     argument, nothing allocated by the call when `out` is given)."""
     stride_bytes = vocabulary * 4 if stride_bytes is None else stride_bytes
     out = dev.empty(logit_topk_output_bytes(rows), "uint8") if out is None else out
-    check(dll().tsp_logit_topk_static(dev.ptr(logits), C.c_uint64(stride_bytes), C.c_uint32(rows), C.c_uint32(vocabulary), dev.ptr(out),
-                                      C.c_uint64(dev.nbytes(out)), dev.stream()))
+    check(dev.native.logit_topk_static(logits, stride_bytes, rows, vocabulary, out, out.nbytes, dev._stream()))
     return out
 
 
 def calibration_copy(dev, dst, src):
     """Plain copy kernel of a known size (scales a profiler's HBM byte counters)."""
-    check(dll().tsp_calibration_copy(dev.ptr(dst), dev.ptr(src), C.c_uint64(dev.nbytes(src)), dev.stream()))
+    check(dev.native.calibration_copy(dst, src, src.nbytes, dev._stream()))
 
 
 def as_u32(t):
