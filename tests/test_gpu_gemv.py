@@ -289,3 +289,15 @@ def test_q8_matvec_many(gpu, tsp, orc, synth, width, cols, rows):
     assert scaled_error(got_l, want) <= TOL and gpu.error() == 0
     with pytest.raises(tsp.FormatError):
         gpu.q8_matvec_many(gpu.upload(w), gpu.upload(x), cols, rows, 3)
+
+
+@pytest.mark.parametrize("cols,rows,count", [(4, 1, 3), (252, 5, 2), (2048, 512, 1), (2052, 3, 1), (2560, 1, 9), (4100, 2, 2), (2046, 3, 2)])
+def test_gemv_f32_rows(gpu, synth, cols, rows, count):
+    """Float rows in 16-byte pieces: fewer pieces than lanes, a second batch of 2048 columns, many token rows against one
+    matrix row; 2046 columns stay with the per-element kernel. Error bound: f32 sums in any order, n/64 + 8 roundings."""
+    w, x = synth.activations_f32(1900 + cols, (rows, cols)), synth.activations_f32(1901 + cols, (count, cols))
+    y = gpu.empty((count, rows))
+    gpu.gemv_rows(0, gpu.upload(w.view(np.uint8)), gpu.upload(x), y, count, cols, rows, cols * 4, rows * 4)
+    want = x.astype(np.float64) @ w.astype(np.float64).T
+    scale = np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T
+    assert (np.abs(y.cpu().numpy() - want) <= (cols / 64 + 8) * 2.0 ** -24 * scale).all() and gpu.error() == 0

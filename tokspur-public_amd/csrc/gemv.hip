@@ -67,6 +67,44 @@ __global__ __launch_bounds__(256) void gemv_generic(GemvArgs a) {
     }
 }
 
+// ------------------------------------------------------------------------------------ F32
+
+// Rows of floats (a router projection of one token, the one row of a shared expert's gate against many tokens): a wave per
+// row and slice, 16-byte loads. Bound by latency at these sizes (4 MB at 512 x 2048), so everything a wave needs for 2048
+// columns, eight pieces of the row and eight of the activations, is requested before the first product: the per-element
+// form walked its row in 32 dependent rounds of 4-byte loads. Two waves per workgroup, so that 512 rows are 256 workgroups,
+// one per compute unit. 512 x 2048: 12.6 -> 3.7 us; one row against 2048 tokens: 15.5 -> 4.0 us.
+typedef float f32v4 __attribute__((ext_vector_type(4)));
+__global__ __launch_bounds__(128) void gemv_f32(GemvArgs a) {
+    const uint8_t* w; const float* x; float* y;
+    if (!resolve(a, w, x, y)) return;
+    const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    for (uint32_t row = blockIdx.x * 2 + wave; row < a.rows; row += gridDim.x * 2) {
+        const f32v4* data = reinterpret_cast<const f32v4*>(w + uint64_t(row) * a.columns * 4);
+        const f32v4* xs = reinterpret_cast<const f32v4*>(x);
+        const uint32_t quads = a.columns / 4;
+        f32v4 acc{};
+        for (uint32_t q0 = lane; q0 < quads; q0 += 8 * kWave) {
+            f32v4 wv[8], xv[8];
+#pragma unroll
+            for (uint32_t j = 0; j < 8; ++j) {
+                const uint32_t q = q0 + j * kWave;  // past the end: the last piece again, without a branch, against zeros
+                wv[j] = data[q < quads ? q : quads - 1];
+                xv[j] = xs[q < quads ? q : quads - 1];
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < 8; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf(wv[j][e], q0 + j * kWave < quads ? xv[j][e] : 0.0f, acc[e]);
+        }
+        const float total = wave_sum((acc[0] + acc[1]) + (acc[2] + acc[3]));
+        if (lane == 0) {
+            if (nonfinite(total)) atomicOr(a.error_word, TSP_ERRBIT_NONFINITE);
+            y[row] = total;
+        }
+    }
+}
+
 // ------------------------------------------------------------------------------------ Q4_K
 
 // Sum over aligned groups of N lanes (N = 8, 16, 32, 64); every lane of a group gets the sum.
@@ -280,6 +318,12 @@ int launch_gemv(uint32_t encoding, uint32_t layout, GemvArgs a, hipStream_t stre
 #undef TSP_Q4K_CASE
     }
     TSP_REQUIRE(layout == TSP_LAYOUT_GGUF, "no GEMV kernel for this layout/encoding/shape");
+    // 16-byte pieces of every row of either operand
+    if (encoding == 0 && aligned && a.columns % 4 == 0 && reinterpret_cast<uintptr_t>(a.x) % 16 == 0 && a.x_stride % 16 == 0) {
+        const dim3 grid(grid_rows(a.rows, 2), a.count);
+        TSP_LAUNCH("gemv_f32", stream, gemv_f32<<<grid, 128, 0, stream>>>(a));
+        return launch_status("gemv_f32");
+    }
     const dim3 grid(grid_rows(a.rows, 4), a.count);
     const bool ok = dispatch_encoding(encoding, [&]<uint32_t T>() { TSP_LAUNCH("gemv_generic", stream, gemv_generic<T><<<grid, 256, 0, stream>>>(a)); });
     TSP_REQUIRE(ok, "no owned numerical decoder for this encoding");
