@@ -413,3 +413,31 @@ def test_destination_contents_after_a_refused_batch(gpu, tsp):
     assert gpu.error() == tsp.ERRBIT_NONFINITE
     gpu.clear_error()
     assert got[0] == inf and got[1] == 2.0
+
+
+@pytest.mark.parametrize("experts,selected,grid", [(512, 10, 0), (512, 10, 0.25), (512, 10, 2), (70, 10, 0.5), (4, 4, 0), (512, 33, 0.1), (512, 64, 0)])
+def test_route_batch_candidates_and_ties(gpu, orc, experts, selected, grid):
+    """The candidates that pass a row's bound rank themselves as long as they are at most 64; coarse grids of logits make many
+    ties, up to more candidates than that (the rounds of arg-max take over). Ids are the oracle's."""
+    rng = np.random.default_rng(experts + selected)
+    logits = rng.normal(size=(9, experts)).astype(np.float32)
+    if grid:
+        logits = (np.round(logits / grid) * grid).astype(np.float32)
+    ids, weights = gpu.route(gpu.upload(logits), selected, 0, True, tokens=9)
+    for t in range(9):
+        want, want_w = orc.route_reference(logits[t].astype(np.float64), selected, 0, True)[:2]
+        assert np.array_equal(u32(ids)[t], want)
+        assert np.abs(weights.cpu().numpy()[t] - want_w).max() <= 1e-6  # f32 exponentials and one division
+    assert gpu.error() == 0
+
+
+@pytest.mark.parametrize("tokens,columns,experts", [(8, 2048, 512), (17, 2560, 100), (129, 1024, 512), (203, 2080, 300), (300, 96, 512), (1025, 64, 512)])
+def test_router_f32_batch_sliced(gpu, synth, tokens, columns, experts):
+    """Fewer tokens than a round of 64 x 64 tiles: each of the three tile sizes whose waves split the columns, columns that do
+    not divide among eight waves, ragged edges; the bound of the large form (f32 sums of 2080 products)."""
+    w = synth.activations_f32(synth.tensor_seed(5, 100 + tokens), (experts, columns))
+    x = synth.activations_f32(synth.tensor_seed(6, 100 + tokens), (tokens, columns))
+    got = gpu.router_f32_batch(gpu.upload(w), gpu.upload(x), tokens, columns, experts).cpu().numpy()
+    want = x.astype(np.float64) @ w.astype(np.float64).T
+    scale = np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T
+    assert (np.abs(got - want) <= 2e-6 * scale).all() and gpu.error() == 0

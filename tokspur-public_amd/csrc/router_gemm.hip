@@ -5,7 +5,7 @@
 // Both operands stay f32 from memory to the accumulator: the products run on the f32 matrix-core instruction
 // (v_mfma_f32_32x32x2_f32), which rounds once per fused multiply-add like the scalar code does.
 //
-// One workgroup of eight waves owns a 64 token x 64 expert tile. Per 64-column step both 64 x 64 operand tiles go
+// Many tokens: one workgroup of eight waves owns a 64 token x 64 expert tile. Per 64-column step both 64 x 64 operand tiles go
 // global -> registers -> LDS (rows padded to 68 floats so that the 16-byte fragment reads of a wave spread over all
 // banks), double buffered with one barrier per step; waves 0-3 multiply the first 32 columns of the step, waves 4-7 the
 // last 32, so every SIMD holds two waves that hide each other's LDS latency. The two halves are added in a fixed order
@@ -127,6 +127,81 @@ __global__ __launch_bounds__(512) void router_f32_gemm(RouterArgs a) {
     }
 }
 
+// Fewer tokens than fill the chip with 64 x 64 tiles (eight of them for a draft's tokens): a workgroup owns ET * 16 experts x
+// TT * 16 tokens, its eight waves a slice of the columns each, and the eight partial tiles are added in LDS in wave order.
+// Operands go straight from memory into the fragments of v_mfma_f32_16x16x4_f32: lane l holds four consecutive columns of
+// row l % 16 of either operand, one column per instruction, so no LDS round trip stands between a wave's requests and its
+// products and all a wave needs is in flight a batch of kUnits steps ahead. Bound by the latency of one trip to memory and the matrix
+// rate of f32 (4 x 32 cycles per 16 columns and tile pair) at eight waves per tile. 512 experts x
+// 2048 columns: 8 tokens 41.8 -> 7.6 us, 203 tokens 42.6 -> 12.8, 400 tokens 42.9 -> 17.2.
+constexpr uint32_t kSlices = 8;
+typedef float acc4 __attribute__((ext_vector_type(4)));
+
+template <int ET, int TT>
+__global__ __launch_bounds__(512) void router_f32_sliced(RouterArgs a) {
+    __shared__ __attribute__((aligned(16))) float sums[kSlices * ET * TT * 256];
+    const uint32_t token0 = (blockIdx.x / a.expert_tiles) * (TT * 16), expert0 = (blockIdx.x % a.expert_tiles) * (ET * 16);
+    const uint32_t tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
+    const uint32_t r16 = lane % 16, k4 = lane / 16;
+    const float* xrow[TT];
+    const float* wrow[ET];
+#pragma unroll
+    for (int t = 0; t < TT; ++t) xrow[t] = a.input + uint64_t(min(token0 + t * 16 + r16, a.tokens - 1)) * a.input_stride + k4 * 4;
+#pragma unroll
+    for (int e = 0; e < ET; ++e) wrow[e] = a.weights + uint64_t(min(expert0 + e * 16 + r16, a.experts - 1)) * a.columns + k4 * 4;
+    acc4 acc[ET][TT] = {};
+    // 16-column units of this wave's slice
+    const uint32_t units = a.columns / 16, per_wave = (units + kSlices - 1) / kSlices;
+    const uint32_t first = wave * per_wave, last = min(first + per_wave, units);
+    constexpr uint32_t kUnits = 8 / (ET * TT > 2 ? 2 : 1);
+    for (uint32_t u0 = first; u0 < last; u0 += kUnits) {
+        acc4 fx[kUnits][TT], fw[kUnits][ET];
+#pragma unroll
+        for (uint32_t j = 0; j < kUnits; ++j) {
+            const uint32_t k = min(u0 + j, last - 1) * 16;  // past the slice: its last unit again, not multiplied
+#pragma unroll
+            for (int t = 0; t < TT; ++t) fx[j][t] = *reinterpret_cast<const acc4*>(xrow[t] + k);
+#pragma unroll
+            for (int e = 0; e < ET; ++e) fw[j][e] = *reinterpret_cast<const acc4*>(wrow[e] + k);
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kUnits; ++j) {
+            if (u0 + j >= last) break;  // uniform over the wave
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+                for (int e = 0; e < ET; ++e)
+#pragma unroll
+                    for (int t = 0; t < TT; ++t) acc[e][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(fx[j][t][c], fw[j][e][c], acc[e][t], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < ET; ++e)
+#pragma unroll
+        for (int t = 0; t < TT; ++t) *reinterpret_cast<acc4*>(sums + ((wave * ET + e) * TT + t) * 256 + lane * 4) = acc[e][t];
+    __syncthreads();
+    uint32_t bad = 0;
+    for (uint32_t i = tid; i < ET * TT * 256; i += 512) {  // value i: register i % 4 of lane (i / 4) % 64 of tile i / 256
+        float value = sums[i];
+#pragma unroll
+        for (uint32_t s = 1; s < kSlices; ++s) value += sums[s * ET * TT * 256 + i];
+        const uint32_t l = i / 4 % 64, t = i / 256 % TT, e = i / 256 / TT;
+        const uint32_t token = token0 + t * 16 + (l / 16) * 4 + i % 4, expert = expert0 + e * 16 + l % 16;  // D[i][j]: j = lane % 16
+        if (token < a.tokens && expert < a.experts) {
+            bad |= nonfinite(value) ? TSP_ERRBIT_NONFINITE : 0u;
+            a.output[uint64_t(token) * a.output_stride + expert] = value;
+        }
+    }
+    publish_error(bad, a.error_word);
+}
+
+template <int ET, int TT>
+void launch_sliced(RouterArgs a, hipStream_t s) {
+    a.expert_tiles = (a.experts + ET * 16 - 1) / (ET * 16);
+    const uint32_t tiles = a.expert_tiles * ((a.tokens + TT * 16 - 1) / (TT * 16));
+    TSP_LAUNCH("router_f32_gemm", s, router_f32_sliced<ET, TT><<<tiles, 512, 0, s>>>(a));
+}
+
 std::atomic<uint64_t> g_lds_raised{0};
 
 }  // namespace
@@ -162,6 +237,13 @@ extern "C" int tsp_router_f32_batch(const float* weights, const float* input, ui
     a.tiles_per_xcd = (a.tiles + 7) / 8;
     a.error_word = error_word;
     const auto s = static_cast<hipStream_t>(stream);
-    TSP_LAUNCH("router_f32_gemm", s, router_f32_gemm<<<a.tiles_per_xcd * 8, 512, kLdsBytes, s>>>(a));
+    // The sliced form as long as one round of its tiles (256 compute units) covers the product, on the smallest tile for which
+    // that holds: 16 x 16 (9 us a round at 2048 columns), 16 experts x 32 tokens (13 us), 32 x 32 (17 us); two rounds of the
+    // largest (35 us, 1024 tokens of 512 experts) still beat the 43 us that the 64 x 64 form takes up to a full round of its own.
+    const auto tiles = [&](uint32_t e, uint32_t t) { return uint64_t((experts + e - 1) / e) * ((tokens + t - 1) / t); };
+    if (tiles(16, 16) <= 256) launch_sliced<1, 1>(a, s);
+    else if (tiles(16, 32) <= 256) launch_sliced<1, 2>(a, s);
+    else if (tiles(32, 32) <= 512) launch_sliced<2, 2>(a, s);
+    else TSP_LAUNCH("router_f32_gemm", s, router_f32_gemm<<<a.tiles_per_xcd * 8, 512, kLdsBytes, s>>>(a));
     return launch_status("router_f32_gemm");
 }
