@@ -243,3 +243,30 @@ def test_config2_moe_verify(gpu, tsp, orc, synth):
     value, at, actual, expected, row_rms = reference_metric(out, want)
     print(f"config2: reference metric |a-e|/max(1,|e|) = {value:.3e} at element {at} (got {actual:.8g}, reference {expected:.8g}, "
           f"row rms {row_rms:.3g}: {abs(actual - expected) / row_rms:.2e} of the row scale)")
+
+
+@pytest.mark.parametrize("tokens", [1, 2, 5, 8])
+@pytest.mark.parametrize("dn,channels,hidden,experts,selected", [(8, 2560, 640, 16, 10), (7, 2560, 160, 8, 4), (14, 1280, 768, 8, 4), (8, 256, 32, 4, 2),
+                                                                 (7, 768, 2560, 4, 2), (8, 1792, 96, 64, 16)])
+def test_routed_m8_streamed(gpu, tsp, orc, synth, dn, channels, hidden, experts, selected, tokens):
+    """The streaming kernels: rows of 1 to 10 super-blocks, down rows that do not fill their last 128 columns (160, 96, 32), more
+    rows than one pass holds (every token on expert 0), shares that span several records, strided rows and canaries; a row's
+    bits do not depend on which tokens ride along."""
+    gate, up = synth.matrix(12, 51, hidden * experts, channels), synth.matrix(12, 52, hidden * experts, channels)
+    down = synth.matrix(dn, 53, channels * experts, hidden)
+    w = tsp.PlanarMoeWeights(gpu, 12, dn, channels, hidden, experts, gate, up, down)
+    rng = np.random.default_rng(tokens + channels)
+    ids = np.array([[0] + list(1 + rng.permutation(experts - 1)[:selected - 1]) for _ in range(tokens)], dtype=np.uint32)
+    x = (synth.activations_f32(54 + tokens, (tokens, channels + 8)) * 0.1).astype(np.float32)
+    routes = tokens * selected
+    h, y = gpu.full((routes, hidden + 4), -5.0), gpu.full((routes, channels + 8), -6.0)
+    tsp.planar_moe_routed_m8(gpu, w, gpu.upload(ids.reshape(-1)), gpu.upload(x), tokens, selected, h=h, y=y, x_stride=(channels + 8) * 4,
+                             h_stride=(hidden + 4) * 4, y_stride=(channels + 8) * 4)
+    h, y = h.cpu().numpy(), y.cpu().numpy()
+    ref_h, ref_y = orc.moe_routed_reference(12, dn, gate, up, down, channels, hidden, experts, ids.reshape(-1), tokens, selected,
+                                            np.ascontiguousarray(x[:, :channels]), threads=8)
+    assert nmse(h[:, :hidden], ref_h) <= 1e-6 and nmse(y[:, :channels], ref_y) <= 1e-6
+    assert (h[:, hidden:] == -5.0).all() and (y[:, channels:] == -6.0).all() and gpu.error() == 0
+    if tokens > 2:  # two or more tokens take the same kernels
+        _, pair = tsp.planar_moe_routed_m8(gpu, w, gpu.upload(ids[-2:].reshape(-1)), gpu.upload(np.ascontiguousarray(x[-2:, :channels])), 2, selected)
+        assert np.array_equal(pair.cpu().numpy().view(np.uint32), np.ascontiguousarray(y[-2 * selected:, :channels]).view(np.uint32))

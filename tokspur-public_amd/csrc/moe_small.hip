@@ -5,12 +5,12 @@
 // expert, up to 8 tokens each) let every expert's weights be streamed from HBM once for all the
 // tokens that route to it. f32 decode, f32 accumulate, no narrowing.
 //
-// Fast arms: Q4_K gate/up with K a multiple of 512 (a lane owns one 32-byte nibble pair and keeps
-// the activations of its 64 columns in registers; the two half-waves of a step take the gate row
-// and the up row of the same hidden unit, so SwiGLU needs one cross-lane move), and Q6_K planes
-// for the down projection. Every other planar encoding goes through the generic arm.
+// This file holds the entry points, the choice of a kernel and the per-element arm, which takes any planar encoding, width and
+// alignment. The kernels that stream the weights past the matrix cores are in record_resident.hip, record_stream.hip and
+// skinny.hip.
 #include "decode.hpp"
 #include "record_resident.hpp"
+#include "record_stream.hpp"
 #include "skinny.hpp"
 
 using namespace tsp;
@@ -55,19 +55,6 @@ __device__ __forceinline__ bool load_record(const SmallMoeArgs& a, uint32_t inde
 __device__ __forceinline__ float silu_mul(float g, float u) {
     const float s = sigmoid_stable(g);
     return (g * s) * u;
-}
-
-__device__ __forceinline__ float ubyte(uint32_t w, int i) { return float((w >> (8 * i)) & 0xffu); }
-
-template <int N>
-__device__ __forceinline__ float lanes_sum(float v) {
-    v = dpp_add<0xB1>(v);
-    v = dpp_add<0x4E>(v);
-    v = dpp_add<0x141>(v);
-    if constexpr (N >= 16) v = dpp_add<0x140>(v);
-    if constexpr (N >= 32) v += __shfl_xor(v, 16, kWave);
-    if constexpr (N >= 64) v += __shfl_xor(v, 32, kWave);
-    return v;
 }
 
 // ------------------------------------------------------------------------------------ planar element decode (generic arm)
@@ -169,183 +156,6 @@ __global__ __launch_bounds__(256) void down_generic(SmallMoeArgs a) {
     publish_error(bad, a.error_word);
 }
 
-// ------------------------------------------------------------------------------------ Q4_K gate/up fast arm
-// BPR super-blocks per row (2, 4 or 8). A wave step covers 16 super-blocks = RPS rows; the first
-// RPS/2 are gate rows of hidden units u0.., the others the up rows of the same units. TOK tokens of
-// the record are processed per pass with their activations in registers.
-template <int BPR, int TOK>
-__global__ __launch_bounds__(256) void gate_up_q4k(SmallMoeArgs a) {
-    constexpr int LPR = 4 * BPR, RPS = kWave / LPR, UPS = RPS / 2;  // units per step
-    static_assert(RPS >= 2);
-    Record rec;
-    if (!load_record(a, blockIdx.y, rec)) return;
-    if (rec.expert >= a.experts) {
-        if (threadIdx.x == 0 && blockIdx.x == 0) atomicOr(a.error_word, TSP_ERRBIT_INDEX);
-        return;
-    }
-    const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave, nwaves = blockDim.x / kWave;
-    const uint32_t pair = lane % 4, blk_in_row = (lane / 4) % BPR, row_in_step = lane / LPR;
-    const bool is_up = row_in_step >= UPS;
-    const uint32_t unit_in_step = row_in_step % UPS;
-    const uint8_t* w = pair_base(a, rec.expert) + (is_up ? a.gu.planar_expert_bytes : 0);
-    const uint32_t steps = (a.hidden + UPS - 1) / UPS;
-    const uint32_t passes = (rec.count + TOK - 1) / TOK;
-    uint32_t bad = 0;
-    // work item = (step, pass); consecutive waves take the passes of one step so they share its weights in L1
-    const uint32_t items = steps * passes;
-    uint32_t held_pass = 0xffffffffu;
-    float xa[TOK][32], xb[TOK][32], sxa[TOK], sxb[TOK];
-    for (uint32_t item = blockIdx.x * nwaves + wave; item < items; item += gridDim.x * nwaves) {
-        const uint32_t step = item / passes, pass = item % passes;
-        if (pass != held_pass) {
-            held_pass = pass;
-#pragma unroll
-            for (int t = 0; t < TOK; ++t) {
-                const uint32_t k = pass * TOK + t < rec.count ? pass * TOK + t : rec.count - 1;
-                const float* src = reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(a.x) + rec.token[k] * a.x_stride) +
-                                   blk_in_row * 256 + pair * 64;
-                sxa[t] = 0; sxb[t] = 0;
-#pragma unroll
-                for (int i = 0; i < 32; i += 4) {
-                    const float4 va = *reinterpret_cast<const float4*>(src + i), vb = *reinterpret_cast<const float4*>(src + 32 + i);
-                    xa[t][i] = va.x; xa[t][i + 1] = va.y; xa[t][i + 2] = va.z; xa[t][i + 3] = va.w;
-                    xb[t][i] = vb.x; xb[t][i + 1] = vb.y; xb[t][i + 2] = vb.z; xb[t][i + 3] = vb.w;
-                    sxa[t] += (va.x + va.y) + (va.z + va.w);
-                    sxb[t] += (vb.x + vb.y) + (vb.z + vb.w);
-                }
-            }
-        }
-        const uint32_t unit = step * UPS + unit_in_step;
-        const bool live = unit < a.hidden;
-        const uint64_t blk = uint64_t(live ? unit : a.hidden - 1) * BPR + blk_in_row;
-        const uint8_t* qs = w + a.gu.qs_offset + blk * 128 + pair * 32;
-        const uint4 q0 = *reinterpret_cast<const uint4*>(qs), q1 = *reinterpret_cast<const uint4*>(qs + 16);
-        const uint8_t* sm = w + a.gu.sm_offset + blk * 16 + pair * 2;
-        const uint32_t sc = *reinterpret_cast<const uint16_t*>(sm), mn = *reinterpret_cast<const uint16_t*>(sm + 8);
-        const uint32_t dm = *reinterpret_cast<const uint32_t*>(w + a.gu.dm_offset + blk * 4);
-        const float d = half_bits_to_float(dm & 0xffffu), dmin = half_bits_to_float(dm >> 16);
-        const float dl_a = d * float(sc & 0xffu), dl_b = d * float(sc >> 8);
-        const float ml_a = dmin * float(mn & 0xffu), ml_b = dmin * float(mn >> 8);
-        const uint32_t words[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
-        float dot_a[TOK], dot_b[TOK];
-#pragma unroll
-        for (int t = 0; t < TOK; ++t) { dot_a[t] = 0; dot_b[t] = 0; }
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const uint32_t lo = words[k] & 0x0f0f0f0fu, hi = (words[k] >> 4) & 0x0f0f0f0fu;
-            const float l0 = ubyte(lo, 0), l1 = ubyte(lo, 1), l2 = ubyte(lo, 2), l3 = ubyte(lo, 3);
-            const float h0 = ubyte(hi, 0), h1 = ubyte(hi, 1), h2 = ubyte(hi, 2), h3 = ubyte(hi, 3);
-#pragma unroll
-            for (int t = 0; t < TOK; ++t) {
-                dot_a[t] = __builtin_fmaf(l0, xa[t][4 * k], dot_a[t]);
-                dot_a[t] = __builtin_fmaf(l1, xa[t][4 * k + 1], dot_a[t]);
-                dot_a[t] = __builtin_fmaf(l2, xa[t][4 * k + 2], dot_a[t]);
-                dot_a[t] = __builtin_fmaf(l3, xa[t][4 * k + 3], dot_a[t]);
-                dot_b[t] = __builtin_fmaf(h0, xb[t][4 * k], dot_b[t]);
-                dot_b[t] = __builtin_fmaf(h1, xb[t][4 * k + 1], dot_b[t]);
-                dot_b[t] = __builtin_fmaf(h2, xb[t][4 * k + 2], dot_b[t]);
-                dot_b[t] = __builtin_fmaf(h3, xb[t][4 * k + 3], dot_b[t]);
-            }
-        }
-#pragma unroll
-        for (int t = 0; t < TOK; ++t) {
-            float part = dl_a * dot_a[t] - ml_a * sxa[t];
-            part += dl_b * dot_b[t] - ml_b * sxb[t];
-            const float total = lanes_sum<LPR>(part);
-            // lane of the gate row fetches the up row's total: same unit, UPS rows further on
-            const float other = __shfl(total, (lane + UPS * LPR) % kWave, kWave);
-            const uint32_t k = pass * TOK + t;
-            if (live && !is_up && lane % LPR == 0 && k < rec.count) {
-                const float act = silu_mul(total, other);
-                if (nonfinite(total) || nonfinite(other) || nonfinite(act)) bad = TSP_ERRBIT_NONFINITE;
-                reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(a.h) + rec.route[k] * a.h_stride)[unit] = act;
-            }
-        }
-    }
-    publish_error(bad, a.error_word);
-}
-
-// ------------------------------------------------------------------------------------ Q6_K down fast arm
-// Planes [ql 128][qh 64][sc 16][d 2] per block. A lane owns four byte positions j..j+3 of one
-// 128-weight section: 16 weights (elements j, 32+j, 64+j, 96+j and their three neighbours).
-// 16 lanes per block; BPR = blocks per row (hidden / 256) in {1, 2, 4}.
-template <int BPR, int TOK>
-__global__ __launch_bounds__(256) void down_q6k(SmallMoeArgs a) {
-    constexpr int LPR = 16 * BPR, RPS = kWave / LPR;
-    Record rec;
-    if (!load_record(a, blockIdx.y, rec)) return;
-    if (rec.expert >= a.experts) return;
-    const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave, nwaves = blockDim.x / kWave;
-    const uint32_t jq = lane % 8, sec = (lane / 8) % 2, blk_in_row = (lane / 16) % BPR, row_in_step = lane / LPR;
-    const uint8_t* w = a.down + uint64_t(rec.expert) * a.dn.planar_expert_bytes;
-    const uint32_t steps = (a.channels + RPS - 1) / RPS;
-    const uint32_t passes = (rec.count + TOK - 1) / TOK;
-    const uint32_t items = steps * passes;
-    uint32_t bad = 0, held_pass = 0xffffffffu;
-    float xv[TOK][16], sx[TOK][4];  // [quarter q][i]: element sec*128 + q*32 + jq*4 + i
-    for (uint32_t item = blockIdx.x * nwaves + wave; item < items; item += gridDim.x * nwaves) {
-        const uint32_t step = item / passes, pass = item % passes;
-        if (pass != held_pass) {
-            held_pass = pass;
-#pragma unroll
-            for (int t = 0; t < TOK; ++t) {
-                const uint32_t k = pass * TOK + t < rec.count ? pass * TOK + t : rec.count - 1;
-                const float* src = reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(a.h) + rec.route[k] * a.h_stride) +
-                                   blk_in_row * 256 + sec * 128 + jq * 4;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const float4 v = *reinterpret_cast<const float4*>(src + q * 32);
-                    xv[t][4 * q] = v.x; xv[t][4 * q + 1] = v.y; xv[t][4 * q + 2] = v.z; xv[t][4 * q + 3] = v.w;
-                    sx[t][q] = (v.x + v.y) + (v.z + v.w);
-                }
-            }
-        }
-        const uint32_t row = step * RPS + row_in_step;
-        const bool live = row < a.channels;
-        const uint64_t blk = uint64_t(live ? row : a.channels - 1) * BPR + blk_in_row;
-        const uint8_t* ql = w + a.dn.qs_offset + blk * 128 + sec * 64 + jq * 4;
-        const uint32_t la = *reinterpret_cast<const uint32_t*>(ql), lb = *reinterpret_cast<const uint32_t*>(ql + 32);
-        const uint32_t qh = *reinterpret_cast<const uint32_t*>(w + a.dn.qh_offset + blk * 64 + sec * 32 + jq * 4);
-        const float d = half_bits_to_float(*reinterpret_cast<const uint16_t*>(w + a.dn.dm_offset + blk * 2));
-        // sub-scales of the four 16-weight groups this lane touches: sec*8 + 2*q + (jq*4)/16
-        const uint8_t* scp = w + a.dn.sm_offset + blk * 16 + sec * 8 + jq / 4;
-        // 6-bit codes, four per dword, one dword per quarter q (elements q*32 + jq*4 + 0..3)
-        const uint32_t code[4] = {
-            (la & 0x0f0f0f0fu) | ((qh << 4) & 0x30303030u),
-            (lb & 0x0f0f0f0fu) | ((qh << 2) & 0x30303030u),
-            ((la >> 4) & 0x0f0f0f0fu) | (qh & 0x30303030u),
-            ((lb >> 4) & 0x0f0f0f0fu) | ((qh >> 2) & 0x30303030u),
-        };
-        float part[TOK];
-#pragma unroll
-        for (int t = 0; t < TOK; ++t) part[t] = 0;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const float ds = d * float(int(int8_t(scp[2 * q])));
-            const float c0 = ubyte(code[q], 0), c1 = ubyte(code[q], 1), c2 = ubyte(code[q], 2), c3 = ubyte(code[q], 3);
-#pragma unroll
-            for (int t = 0; t < TOK; ++t) {
-                float dot = -32.0f * sx[t][q];  // sum (c - 32) x = sum c x - 32 sum x
-                dot = __builtin_fmaf(c0, xv[t][4 * q], dot);
-                dot = __builtin_fmaf(c1, xv[t][4 * q + 1], dot);
-                dot = __builtin_fmaf(c2, xv[t][4 * q + 2], dot);
-                dot = __builtin_fmaf(c3, xv[t][4 * q + 3], dot);
-                part[t] = __builtin_fmaf(ds, dot, part[t]);
-            }
-        }
-#pragma unroll
-        for (int t = 0; t < TOK; ++t) {
-            const float total = lanes_sum<LPR>(part[t]);
-            const uint32_t k = pass * TOK + t;
-            if (live && lane % LPR == 0 && k < rec.count) {
-                if (nonfinite(total)) bad = TSP_ERRBIT_NONFINITE;
-                reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(a.y) + rec.route[k] * a.y_stride)[row] = total;
-            }
-        }
-    }
-    publish_error(bad, a.error_word);
-}
-
 // ------------------------------------------------------------------------------------ host side
 bool coloc_pair_kinds(uint32_t gate_kind, uint32_t up_kind, uint32_t* type) {
     if (gate_kind == TSP_KIND_Q4K_COLOC_GATE && up_kind == TSP_KIND_Q4K_COLOC_UP) { *type = 12; return true; }
@@ -420,37 +230,35 @@ SkinnyMoe skinny_view(const SmallMoeArgs& a, const tsp_shared_rows* shared = nul
     return v;
 }
 
-// The record-resident gate/up launch builds the union records itself (and leaves them in `meta` for the down launch): no
-// launch of the union kernel goes before it.
+// Which kernel takes the gate/up product. Q4_K rows of 2048 columns and two or more tokens: the record-resident one (27 us at 8
+// tokens and 512 hidden units where the streaming one takes 34). One token and a row of 1, 2, 4 or 8 super-blocks: one
+// super-block per wave (10.9 against 12.3 us at 2048 x 768, 8.2 against 8.9 at 1024 x 512). Everything else Q4_K up to 2560 columns
+// streams; other encodings, wider rows and rows that 16 bytes do not align go weight by weight.
+enum GateUpArm { GU_GENERIC, GU_RECORD, GU_FLAT, GU_STREAM };
+GateUpArm gate_up_arm(const SmallMoeArgs& a, const tsp_shared_rows* shared) {
+    const SkinnyMoe v = skinny_view(a, shared);
+    if (a.gu.source_type != 12) return GU_GENERIC;
+    if (record_gate_up_takes(v)) return GU_RECORD;
+    const bool flat = flat_gate_up_takes(v);
+    if (a.tokens > 1 || !flat) if (record_stream_gate_up_takes(v)) return GU_STREAM;
+    return flat ? GU_FLAT : GU_GENERIC;
+}
+// The first two build the union records themselves (and leave them in `meta` for the down launch): no launch of the union kernel
+// goes before them.
 bool gate_up_builds_union(const SmallMoeArgs& a, const tsp_shared_rows* shared = nullptr) {
-    return skinny_moe_supported(a.gu.source_type, a.dn.source_type, a.channels, a.hidden, a.x, a.x_stride, a.h, a.h_stride, false) &&
-           record_gate_up_takes(skinny_view(a, shared));
+    const GateUpArm arm = gate_up_arm(a, shared);
+    return arm == GU_RECORD || arm == GU_STREAM;
 }
 
 int launch_gate_up(const SmallMoeArgs& a, hipStream_t s, const tsp_shared_rows* shared = nullptr) {
-    const uint32_t records = record_slots(a);
-    if (skinny_moe_supported(a.gu.source_type, a.dn.source_type, a.channels, a.hidden, a.x, a.x_stride, a.h, a.h_stride, false)) {
-        const SkinnyMoe view = skinny_view(a, shared);
-        return record_gate_up_takes(view) ? launch_record_gate_up(view, s) : skinny_moe_gate_up(view, s);
+    switch (gate_up_arm(a, shared)) {
+    case GU_RECORD: return launch_record_gate_up(skinny_view(a, shared), s);
+    case GU_STREAM: return launch_record_stream_gate_up(skinny_view(a, shared), s);
+    case GU_FLAT: return flat_moe_gate_up(skinny_view(a, shared), s);
+    default: break;
     }
     TSP_REQUIRE(!shared, "the always-on expert rides only on the matrix-core small-row kernels");
-    const bool x_aligned = reinterpret_cast<uintptr_t>(a.x) % 16 == 0 && a.x_stride % 16 == 0;
-    if (a.gu.source_type == 12 && x_aligned && (a.channels == 512 || a.channels == 1024 || a.channels == 2048)) {
-        const uint32_t bpr = a.channels / 256;
-        const uint32_t units_per_step = 64 / (4 * bpr) / 2;
-        const uint32_t steps = (a.hidden + units_per_step - 1) / units_per_step;
-        // tokens == 1: one pass per step; otherwise up to 4 passes of 2 tokens, one per wave of the block
-        const dim3 grid(a.tokens == 1 ? (steps + 3) / 4 : steps, records);
-#define TSP_GU(N)                                                             \
-    if (bpr == N) {                                                           \
-        if (a.tokens == 1) TSP_LAUNCH("gate_up_q4k", s, gate_up_q4k<N, 1><<<grid, 256, 0, s>>>(a));         \
-        else TSP_LAUNCH("gate_up_q4k", s, gate_up_q4k<N, 2><<<grid, 256, 0, s>>>(a));                       \
-        return launch_status("gate_up_q4k");                                  \
-    }
-        TSP_GU(2) TSP_GU(4) TSP_GU(8)
-#undef TSP_GU
-    }
-    const dim3 grid((a.hidden + 3) / 4, records);
+    const dim3 grid((a.hidden + 3) / 4, record_slots(a));
     switch (a.gu.source_type) {
     case 12: TSP_LAUNCH("gate_up_generic", s, gate_up_generic<12><<<grid, 256, 0, s>>>(a)); break;
     case 13: TSP_LAUNCH("gate_up_generic", s, gate_up_generic<13><<<grid, 256, 0, s>>>(a)); break;
@@ -459,29 +267,14 @@ int launch_gate_up(const SmallMoeArgs& a, hipStream_t s, const tsp_shared_rows* 
     return launch_status("gate_up_generic");
 }
 
+// Q6_K rows of 1, 2, 4 or 8 super-blocks keep one super-block per wave (19 us at config 2's 512 hidden units where the
+// streaming kernel takes 23); other widths and the 32-weight blocks stream.
 int launch_down(const SmallMoeArgs& a, hipStream_t s, const tsp_shared_rows* shared = nullptr) {
-    const uint32_t records = record_slots(a);
-    if (a.dn.source_type == 14 && a.hidden % 256 == 0 && a.hidden <= 2048 && reinterpret_cast<uintptr_t>(a.h) % 16 == 0 && a.h_stride % 16 == 0) {
-        const SkinnyMoe view = skinny_view(a, shared);
-        return skinny_moe_down(view, s);
-    }
+    const SkinnyMoe v = skinny_view(a, shared);
+    if (flat_down_takes(v)) return flat_moe_down(v, s);
+    if (record_stream_down_takes(v)) return launch_record_stream_down(v, s);
     TSP_REQUIRE(!shared, "the always-on expert rides only on the matrix-core small-row kernels");
-    const bool h_aligned = reinterpret_cast<uintptr_t>(a.h) % 16 == 0 && a.h_stride % 16 == 0;
-    if (a.dn.source_type == 14 && h_aligned && (a.hidden == 256 || a.hidden == 512 || a.hidden == 1024)) {
-        const uint32_t bpr = a.hidden / 256;
-        const uint32_t rps = 64 / (16 * bpr);
-        const uint32_t steps = (a.channels + rps - 1) / rps;
-        const dim3 grid(a.tokens == 1 ? (steps + 3) / 4 : steps, records);
-#define TSP_DN(N)                                                          \
-    if (bpr == N) {                                                        \
-        if (a.tokens == 1) TSP_LAUNCH("down_q6k", s, down_q6k<N, 1><<<grid, 256, 0, s>>>(a));         \
-        else TSP_LAUNCH("down_q6k", s, down_q6k<N, 2><<<grid, 256, 0, s>>>(a));                       \
-        return launch_status("down_q6k");                                  \
-    }
-        TSP_DN(1) TSP_DN(2) TSP_DN(4)
-#undef TSP_DN
-    }
-    const dim3 grid((a.channels + 3) / 4, records);
+    const dim3 grid((a.channels + 3) / 4, record_slots(a));
     switch (a.dn.source_type) {
     case 7: TSP_LAUNCH("down_generic", s, down_generic<7><<<grid, 256, 0, s>>>(a)); break;
     case 8: TSP_LAUNCH("down_generic", s, down_generic<8><<<grid, 256, 0, s>>>(a)); break;

@@ -26,10 +26,14 @@ struct SkinnyMoe {
     uint64_t shared_h_stride = 0, shared_y_stride = 0;
 };
 
-// Q4_K co-located gate/up (and Q6_K planar down when with_down), columns a multiple of 256 up to 2048, 16-byte aligned rows.
+// The shapes the always-on expert may ride with: Q4_K co-located gate/up (and Q6_K planar down when with_down), columns a
+// multiple of 256 up to 2048, 16-byte aligned rows.
 bool skinny_moe_supported(uint32_t gate_up_type, uint32_t down_type, uint32_t channels, uint32_t hidden, const void* x, uint64_t x_stride,
                           const void* h, uint64_t h_stride, bool with_down);
-int skinny_moe_gate_up(const SkinnyMoe& m, hipStream_t stream);
-int skinny_moe_down(const SkinnyMoe& m, hipStream_t stream);
+// One super-block per wave: rows of 1, 2, 4 or 8 super-blocks.
+bool flat_gate_up_takes(const SkinnyMoe& m);
+bool flat_down_takes(const SkinnyMoe& m);
+int flat_moe_gate_up(const SkinnyMoe& m, hipStream_t stream);
+int flat_moe_down(const SkinnyMoe& m, hipStream_t stream);
 
 }  // namespace tsp
