@@ -301,3 +301,22 @@ def test_gemv_f32_rows(gpu, synth, cols, rows, count):
     want = x.astype(np.float64) @ w.astype(np.float64).T
     scale = np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T
     assert (np.abs(y.cpu().numpy() - want) <= (cols / 64 + 8) * 2.0 ** -24 * scale).all() and gpu.error() == 0
+
+
+@pytest.mark.parametrize("t,cols,rows", [(12, 256, 3), (12, 768, 70), (12, 2560, 513), (12, 6144, 9), (14, 256, 1), (14, 2560, 700), (14, 1280, 5000), (14, 12288, 2),
+                                         (8, 32, 2), (8, 544, 33), (8, 2560, 600), (8, 5120, 17), (8, 1024, 9000)])
+def test_gemv_units(gpu, orc, synth, t, cols, rows):
+    """Rows of any length, 8 to 64 lanes per row, last rounds with idle lanes, more steps than waves. Error bound: activations
+    keep 24 bits of their sub-block's largest value and every product sum is exact per 16 or 32 weights, so 2^-23 of
+    sum |w x| covers rounding the activations and 2^-22 the f32 sums over at most 384 sub-blocks."""
+    w = synth.matrix(t, 2100 + cols, rows, cols)
+    x = synth.activations_f32(2101 + rows, cols)
+    x[cols // 2:] *= np.float32(1e-3)
+    want = orc.reference_gemv(t, w, cols, rows, x)
+    dense = np.abs(orc.dequantize(t, w, rows * cols).reshape(rows, cols)).astype(np.float64)
+    bound = (dense * np.maximum(np.abs(x), np.abs(x.reshape(-1, 32)).max(axis=1).repeat(32))).sum(axis=1) * (2.0 ** -23 + 2.0 ** -22)
+    got = gpu.gemv(t, gpu.upload(w), gpu.upload(x), cols, rows).cpu().numpy().astype(np.float64)
+    assert (np.abs(got - want) <= bound).all() and gpu.error() == 0
+    x[1] = np.nan
+    gpu.gemv(t, gpu.upload(w), gpu.upload(x), cols, rows)
+    assert gpu.error() == 1

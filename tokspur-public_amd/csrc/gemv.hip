@@ -4,14 +4,15 @@
 // nibbles and scales in registers and finishes with DPP reductions inside the wave.
 //
 //  gemv_generic   wave per row, any decodable encoding and any K: the scalar control arm.
-//  gemv_q4k       Q4_K, raw GGUF rows or one planar v3 expert; a lane owns one 32-byte nibble pair
+//  gemv_f32       F32 rows.
+//  gemv_units     Q4_K, Q6_K and Q8_0 raw GGUF rows of any length up to 12 288 columns.
+//  gemv_q4k       Q4_K rows of 2, 4, 8 or 16 super-blocks, raw GGUF rows or one planar v3 expert; a lane owns one 32-byte nibble pair
 //                 (two 32-weight sub-blocks), 4 lanes per super-block. The lane's 64 activations are
 //                 kept as three planes of signed bytes under a per-sub-block scale (24 bits of each
 //                 value), and the nibbles multiply them four at a time with v_dot4_i32_i8: the sums
 //                 of q * x are exact integers, scaled by d * sc in f32 once per sub-block.
-//  gemv_q8        Q8_0 raw rows as a flat dword stream (row bytes are a multiple of 4).
-//  gemv_q6k       Q6_K planar expert planes.
 #include "decode.hpp"
+#include "gemv.hpp"
 
 using namespace tsp;
 
@@ -119,6 +120,63 @@ __device__ __forceinline__ float group_sum(float v) {
     return v;
 }
 
+// One quad of activations as integers, and its share of the sub-block's record in LDS. Per sub-block of 32 one scale brings the
+// largest magnitude to 8 290 000 (just under 127 * 2^16 + 2^15, the most that three signed bytes hold); every value is rounded
+// to the nearest integer of that grid (2^-24 of the sub-block's largest value: the precision of the f32 operand itself for the
+// values that matter) and written as three signed base-256 digits, x = (a 2^16 + b 2^8 + c) / scale with a, b, c in [-128, 127].
+// Four activations' digits share a dword, in the order of the four bytes of a word of codes, so that v_dot4_i32_i8
+// multiplies four weights per instruction and plane. The integer sums are exact; the three of a sub-block recombine in f32.
+// The eight threads of a sub-block are neighbours and agree on its scale with three cross-lane steps.
+// A record: three planes of eight dwords (c, b, a), then 1 / scale, the sum and a flag for values that are not finite; with
+// SUMS also, for each half of sixteen, -32 times the sums of its digits (a, b, c).
+template <uint32_t WORDS, bool SUMS>
+__device__ __forceinline__ void stage_quad(const float4& x4, bool mine, uint32_t quad, uint32_t* planes) {
+    const float v4[4] = {mine ? x4.x : 0.0f, mine ? x4.y : 0.0f, mine ? x4.z : 0.0f, mine ? x4.w : 0.0f};
+    float biggest = fmaxf(fmaxf(fabsf(v4[0]), fabsf(v4[1])), fmaxf(fabsf(v4[2]), fabsf(v4[3])));
+    float sum = (v4[0] + v4[1]) + (v4[2] + v4[3]);
+    uint32_t flag = (nonfinite(v4[0]) || nonfinite(v4[1]) || nonfinite(v4[2]) || nonfinite(v4[3])) ? 1u : 0u;
+    biggest = dpp_max<0xB1>(biggest); biggest = dpp_max<0x4E>(biggest); biggest = dpp_max<0x141>(biggest);
+    sum = octet_sum(sum);
+    flag |= uint32_t(__builtin_amdgcn_update_dpp(0, int(flag), 0xB1, 0xf, 0xf, true));
+    flag |= uint32_t(__builtin_amdgcn_update_dpp(0, int(flag), 0x4E, 0xf, 0xf, true));
+    flag |= uint32_t(__builtin_amdgcn_update_dpp(0, int(flag), 0x141, 0xf, 0xf, true));
+    // a sub-block of zeros, of subnormals only, or with something not finite in it keeps scale 1 (its integers are zeros)
+    const bool usable = biggest >= 1.1754944e-38f && !nonfinite(biggest) && flag == 0;
+    const float scale = usable ? 8290000.0f / biggest : 1.0f;
+    uint32_t w2 = 0, w1 = 0, w0 = 0;
+    int s2 = 0, s1 = 0, s0 = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int xi = usable ? __float2int_rn(v4[e] * scale) : 0;
+        const int c = ((xi + 128) & 255) - 128, upper = (xi - c) >> 8;
+        const int b = ((upper + 128) & 255) - 128, a8 = (upper - b) >> 8;
+        w2 |= uint32_t(a8 & 0xff) << (8 * e);
+        w1 |= uint32_t(b & 0xff) << (8 * e);
+        w0 |= uint32_t(c & 0xff) << (8 * e);
+        if constexpr (SUMS) { s2 += a8; s1 += b; s0 += c; }
+    }
+    uint32_t* sub = planes + (quad / 8) * WORDS;
+    if (mine) {
+        sub[16 + quad % 8] = w2; sub[8 + quad % 8] = w1; sub[quad % 8] = w0;
+        if (quad % 8 == 0) {
+            sub[24] = __float_as_uint(usable ? biggest / 8290000.0f : 1.0f);
+            sub[25] = __float_as_uint(sum);
+            sub[26] = flag;
+        }
+    }
+    if constexpr (SUMS) {
+        auto over_four = [](int v) {
+            v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, true);
+            return v + __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, true);
+        };
+        s2 = over_four(s2); s1 = over_four(s1); s0 = over_four(s0);
+        if (mine && quad % 4 == 0) {
+            uint32_t* half = sub + 28 + quad % 8;
+            half[0] = uint32_t(-32 * s2); half[1] = uint32_t(-32 * s1); half[2] = uint32_t(-32 * s0);
+        }
+    }
+}
+
 // BPR = super-blocks per row (K / 256), one of 2, 4, 8, 16. A wave covers 16 super-blocks per step
 // (16 / BPR rows); lane = (block-in-step, pair) owns 64 weights and keeps their 64 activations in
 // registers for every row it visits.
@@ -176,50 +234,11 @@ __global__ __launch_bounds__(256) void gemv_q4k(GemvArgs a) {
     }
     uint32_t step = blockIdx.x * (blockDim.x / kWave) + wave;
     Raw cur = fetch(step < steps ? step : 0);
-    // The activations become integers, once per workgroup: per sub-block of 32 one scale that brings the largest magnitude to
-    // 8 290 000 (just under 127 * 2^16 + 2^15, the most that three signed bytes hold), every value rounded to the nearest
-    // integer of that grid (2^-24 of the sub-block's largest value: the precision of the f32 operand itself for the values
-    // that matter) and written as three signed base-256 digits, x = (a 2^16 + b 2^8 + c) / scale with a, b, c in [-128, 127].
-    // Four activations' digits share a dword, in the order of the four bytes of a word of nibbles, so that v_dot4_i32_i8
-    // multiplies four weights per instruction and plane: three integer instructions per four weights where the f32 form
-    // spends a conversion and a multiply-add per weight. The integer sums are exact; the three of a sub-block recombine in f32.
-    // A thread turns the quads it loaded into digits; the eight threads of a sub-block are neighbours and agree on its scale
-    // with three cross-lane steps.
+    // the activations become integers, once per workgroup
 #pragma unroll
     for (uint32_t j = 0; j < kMine; ++j) {
         const uint32_t quad = threadIdx.x + j * 256;
-        const bool mine = kQuads % 256 == 0 || quad < kQuads;  // uniform over every group of eight lanes
-        const float v4[4] = {mine ? xv[j].x : 0.0f, mine ? xv[j].y : 0.0f, mine ? xv[j].z : 0.0f, mine ? xv[j].w : 0.0f};
-        float biggest = fmaxf(fmaxf(fabsf(v4[0]), fabsf(v4[1])), fmaxf(fabsf(v4[2]), fabsf(v4[3])));
-        float sum = (v4[0] + v4[1]) + (v4[2] + v4[3]);
-        uint32_t flag = (nonfinite(v4[0]) || nonfinite(v4[1]) || nonfinite(v4[2]) || nonfinite(v4[3])) ? 1u : 0u;
-        biggest = dpp_max<0xB1>(biggest); biggest = dpp_max<0x4E>(biggest); biggest = dpp_max<0x141>(biggest);
-        sum = octet_sum(sum);
-        flag |= uint32_t(__builtin_amdgcn_update_dpp(0, int(flag), 0xB1, 0xf, 0xf, true));
-        flag |= uint32_t(__builtin_amdgcn_update_dpp(0, int(flag), 0x4E, 0xf, 0xf, true));
-        flag |= uint32_t(__builtin_amdgcn_update_dpp(0, int(flag), 0x141, 0xf, 0xf, true));
-        // a sub-block of zeros, of subnormals only, or with something not finite in it keeps scale 1 (its integers are zeros)
-        const bool usable = biggest >= 1.1754944e-38f && !nonfinite(biggest) && flag == 0;
-        const float scale = usable ? 8290000.0f / biggest : 1.0f;
-        uint32_t w2 = 0, w1 = 0, w0 = 0;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int xi = usable ? __float2int_rn(v4[e] * scale) : 0;
-            const int c = ((xi + 128) & 255) - 128, upper = (xi - c) >> 8;
-            const int b = ((upper + 128) & 255) - 128, a8 = (upper - b) >> 8;
-            w2 |= uint32_t(a8 & 0xff) << (8 * e);
-            w1 |= uint32_t(b & 0xff) << (8 * e);
-            w0 |= uint32_t(c & 0xff) << (8 * e);
-        }
-        if (mine) {
-            uint32_t* sub = planes + (quad / 8) * kSubWords;
-            sub[16 + quad % 8] = w2; sub[8 + quad % 8] = w1; sub[quad % 8] = w0;
-            if (quad % 8 == 0) {
-                sub[24] = __float_as_uint(usable ? biggest / 8290000.0f : 1.0f);
-                sub[25] = __float_as_uint(sum);
-                sub[26] = flag;
-            }
-        }
+        stage_quad<kSubWords, false>(xv[j], kQuads % 256 == 0 || quad < kQuads, quad, planes);  // uniform over every group of eight lanes
     }
     __syncthreads();
 
@@ -290,10 +309,217 @@ __global__ __launch_bounds__(256) void gemv_q4k(GemvArgs a) {
     }
 }
 
+// ------------------------------------------------------------------------------------ Q4_K, Q6_K, Q8_0 rows of any length
+// The same arithmetic for rows of any number of super-blocks and for the other two encodings a decode step meets. L lanes share a
+// row; a lane takes every L-th unit of it (64 weights of a K-quant block, one Q8_0 block) and finds its activations' digits in
+// LDS, three reads of 16 bytes per sixteen weights and plane set, instead of keeping those of one place in the row in registers.
+// Bound by memory for large matrices, by one round trip for small ones: the next unit's bytes are requested before the
+// current one is multiplied. Blocks of 34 and 210 bytes are even-aligned only; neighbouring lanes read neighbouring pieces,
+// so the lines are shared all the same. Per-element decoding before: Q6_K 2731 x 2560 9.8 -> 6.0 us, 40 000 x 6144 (202 MB) 46 us
+// now = 4.3 TB/s; Q8_0 16 000 x 2560 21 -> 11 us.
+typedef uint32_t piece16 __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t piece8 __attribute__((ext_vector_type(2), aligned(2)));
+typedef uint32_t quad_words __attribute__((ext_vector_type(4)));
+
+template <uint32_t T> struct UnitBytes;
+template <> struct UnitBytes<12> { quad_words hdr, q0, q1; };
+template <> struct UnitBytes<14> { piece16 la, lb, qh; piece8 sc; uint16_t d; };
+template <> struct UnitBytes<8> { piece16 q0, q1; uint16_t d; };
+
+__device__ __forceinline__ float recombine(int a2, int a1, int a0) {
+    return __builtin_fmaf(float(a2), 65536.0f, __builtin_fmaf(float(a1), 256.0f, float(a0)));
+}
+
+template <uint32_t T, int L>
+__global__ __launch_bounds__(256) void gemv_units(GemvArgs a) {
+    constexpr bool SUMS = T == 14;
+    constexpr uint32_t kWords = SUMS ? 36 : 28, kUnit = T == 8 ? 32 : 64, RPS = kWave / L;
+    extern __shared__ __attribute__((aligned(16))) uint32_t planes[];
+    const uint8_t* w; const float* x; float* y;
+    if (!resolve(a, w, x, y)) return;
+    const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave, in_row = lane % L, row_in_step = lane / L;
+    const uint32_t units = a.columns / kUnit, rounds = (units + L - 1) / L;
+    const uint32_t steps = (a.rows + RPS - 1) / RPS, waves = gridDim.x * (blockDim.x / kWave);
+    const uint64_t row_bytes = uint64_t(a.columns / BlockGeometry<T>::elements) * BlockGeometry<T>::bytes;
+
+    auto fetch = [&](uint32_t step, uint32_t round) {
+        const uint32_t row = step * RPS + row_in_step, u0 = round * L + in_row, u = u0 < units ? u0 : units - 1;
+        const uint8_t* from = w + (row < a.rows ? row : a.rows - 1) * row_bytes;
+        UnitBytes<T> r;
+        if constexpr (T == 12) {
+            const uint8_t* block = from + u / 4 * 144;
+            r.hdr = *reinterpret_cast<const quad_words*>(block);
+            r.q0 = *reinterpret_cast<const quad_words*>(block + 16 + u % 4 * 32);
+            r.q1 = *reinterpret_cast<const quad_words*>(block + 32 + u % 4 * 32);
+        } else if constexpr (T == 14) {  // section u / 2 % 2, the 16-byte half u % 2 of each of its pieces
+            const uint8_t* block = from + u / 4 * 210;
+            const uint32_t sec = u / 2 % 2, half = u % 2;
+            r.la = *reinterpret_cast<const piece16*>(block + sec * 64 + half * 16);
+            r.lb = *reinterpret_cast<const piece16*>(block + sec * 64 + 32 + half * 16);
+            r.qh = *reinterpret_cast<const piece16*>(block + 128 + sec * 32 + half * 16);
+            r.sc = *reinterpret_cast<const piece8*>(block + 192 + sec * 8);
+            r.d = *reinterpret_cast<const uint16_t*>(block + 208);
+        } else {
+            const uint8_t* block = from + u * 34;
+            r.d = *reinterpret_cast<const uint16_t*>(block);
+            r.q0 = *reinterpret_cast<const piece16*>(block + 2);
+            r.q1 = *reinterpret_cast<const piece16*>(block + 18);
+        }
+        return r;
+    };
+
+    // the activations first, the wave's first weight bytes right behind them; the activations are staged while the weights travel
+    const uint32_t quads = a.columns / 4;
+    float4 x0 = make_float4(0, 0, 0, 0);
+    auto load_quad = [&](uint32_t quad) {
+        return quad < quads ? *reinterpret_cast<const float4*>(x + 4 * quad) : make_float4(0, 0, 0, 0);
+    };
+    x0 = load_quad(threadIdx.x);
+    uint32_t step = blockIdx.x * (blockDim.x / kWave) + wave;
+    UnitBytes<T> cur = fetch(step < steps ? step : 0, 0);
+    for (uint32_t quad = threadIdx.x; quad < (quads + 7) / 8 * 8; quad += 256) {
+        const float4 here = x0;
+        x0 = load_quad(quad + 256);
+        stage_quad<kWords, SUMS>(here, quad < quads, quad, planes);
+    }
+    __syncthreads();
+
+    float part = 0;
+    for (uint32_t round = 0; step < steps;) {
+        const UnitBytes<T> now = cur;
+        const uint32_t u0 = round * L + in_row, u = u0 < units ? u0 : units - 1;
+        const bool last = round + 1 == rounds;
+        const uint32_t next_step = last ? (step + waves < steps ? step + waves : step) : step;
+        cur = fetch(next_step, last ? 0 : round + 1);  // the next unit's bytes travel while this one is summed
+        float sum = 0;
+        if constexpr (T == 12) {
+            const uint32_t pair = u % 4;
+            const float d = half_bits_to_float(now.hdr[0] & 0xffffu), dmin = half_bits_to_float(now.hdr[0] >> 16);
+            // sub-blocks 2 pair and 2 pair + 1: two neighbouring bytes of the unpacked scales and minima (mfma_quant.hpp: decode_hdr)
+            const uint32_t sh = (pair & 1u) * 16u;
+            const uint32_t s2 = (now.hdr[1] >> sh) & 0xffffu, m2 = (now.hdr[2] >> sh) & 0xffffu, e2 = (now.hdr[3] >> sh) & 0xffffu;
+            const uint32_t sc = pair < 2 ? s2 & 0x3f3fu : (e2 & 0x0f0fu) | ((s2 >> 2) & 0x3030u);
+            const uint32_t mn = pair < 2 ? m2 & 0x3f3fu : ((e2 >> 4) & 0x0f0fu) | ((m2 >> 2) & 0x3030u);
+            const uint32_t words[8] = {now.q0[0], now.q0[1], now.q0[2], now.q0[3], now.q1[0], now.q1[1], now.q1[2], now.q1[3]};
+            const uint32_t* sub = planes + u * 2 * kWords;
+#pragma unroll
+            for (int h = 0; h < 2; ++h, sub += kWords) {
+                int acc[3] = {0, 0, 0};
+#pragma unroll
+                for (int p = 0; p < 3; ++p)
+#pragma unroll
+                    for (int k = 0; k < 8; k += 4) {
+                        const quad_words digits = *reinterpret_cast<const quad_words*>(sub + p * 8 + k);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) acc[p] = __builtin_amdgcn_sdot4(int((words[k + i] >> (4 * h)) & 0x0f0f0f0fu), int(digits[i]), acc[p], false);
+                    }
+                const quad_words rest = *reinterpret_cast<const quad_words*>(sub + 24);
+                const float dot = recombine(acc[2], acc[1], acc[0]) * __uint_as_float(rest[0]);
+                const float part_h = (d * float((sc >> (8 * h)) & 0xffu)) * dot - (dmin * float((mn >> (8 * h)) & 0xffu)) * __uint_as_float(rest[1]);
+                sum += rest[2] ? __uint_as_float(0x7fc00000u) : part_h;  // a non-finite activation: the row is not a number
+            }
+        } else if constexpr (T == 14) {
+            const uint32_t sec = u / 2 % 2, half = u % 2;
+            const float d = half_bits_to_float(now.d);
+            const uint32_t* sub = planes + (u / 4 * 8 + sec * 4) * kWords;
+#pragma unroll
+            for (int q = 0; q < 4; ++q, sub += kWords) {  // 16 weights of one sub-scale
+                const quad_words bias = *reinterpret_cast<const quad_words*>(sub + 28 + half * 4);  // -32 times the digits' sums
+                int acc[3] = {int(bias[2]), int(bias[1]), int(bias[0])};
+                uint32_t code[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t low = q % 2 ? now.lb[i] : now.la[i], high = now.qh[i] >> (2 * q);
+                    code[i] = ((q < 2 ? low : low >> 4) & 0x0f0f0f0fu) | ((high & 0x03030303u) << 4);
+                }
+#pragma unroll
+                for (int p = 0; p < 3; ++p) {
+                    const quad_words digits = *reinterpret_cast<const quad_words*>(sub + p * 8 + half * 4);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[p] = __builtin_amdgcn_sdot4(int(code[i]), int(digits[i]), acc[p], false);
+                }
+                const quad_words rest = *reinterpret_cast<const quad_words*>(sub + 24);
+                const uint32_t at = 2 * q + half;  // the sub-scale's byte
+                const float ds = d * float(int(int8_t((now.sc[at / 4] >> (at % 4 * 8)) & 0xffu)));
+                const float dot = recombine(acc[2], acc[1], acc[0]) * __uint_as_float(rest[0]);
+                sum += rest[2] ? __uint_as_float(0x7fc00000u) : ds * dot;
+            }
+        } else {
+            const uint32_t words[8] = {now.q0[0], now.q0[1], now.q0[2], now.q0[3], now.q1[0], now.q1[1], now.q1[2], now.q1[3]};
+            const uint32_t* sub = planes + u * kWords;
+            int acc[3] = {0, 0, 0};
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+#pragma unroll
+                for (int k = 0; k < 8; k += 4) {
+                    const quad_words digits = *reinterpret_cast<const quad_words*>(sub + p * 8 + k);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[p] = __builtin_amdgcn_sdot4(int(words[k + i]), int(digits[i]), acc[p], false);
+                }
+            const quad_words rest = *reinterpret_cast<const quad_words*>(sub + 24);
+            sum = half_bits_to_float(now.d) * (recombine(acc[2], acc[1], acc[0]) * __uint_as_float(rest[0]));
+            if (rest[2]) sum = __uint_as_float(0x7fc00000u);
+        }
+        part += u0 < units ? sum : 0.0f;
+        if (!last) { ++round; continue; }
+        const uint32_t row = step * RPS + row_in_step;
+        const float total = group_sum<L>(part);
+        if (row < a.rows && in_row == 0) {
+            if (nonfinite(total)) atomicOr(a.error_word, TSP_ERRBIT_NONFINITE);
+            y[row] = total;
+        }
+        part = 0;
+        round = 0;
+        step += waves;
+    }
+}
+
 // ------------------------------------------------------------------------------------ launch
 uint32_t grid_rows(uint32_t work_items, uint32_t per_block) {
     const uint32_t blocks = (work_items + per_block - 1) / per_block;
     return blocks < 1 ? 1 : blocks > 2048 ? 2048 : blocks;
+}
+
+// Rows whose digits fit LDS, activations in 16-byte pieces, blocks as aligned as their encoding has them.
+bool gemv_units_takes(uint32_t encoding, const GemvArgs& a) {
+    if (encoding != 8 && encoding != 12 && encoding != 14) return false;
+    const uintptr_t step = encoding == 12 ? 16 : 2;
+    return a.columns <= 12288 && reinterpret_cast<uintptr_t>(a.matrix) % step == 0 && a.expert_stride % step == 0 &&
+           reinterpret_cast<uintptr_t>(a.x) % 16 == 0 && a.x_stride % 16 == 0;
+}
+
+template <uint32_t T, int L>
+int launch_units_lanes(const GemvArgs& a, hipStream_t stream) {
+    const uint32_t bytes = a.columns / 32 * (T == 14 ? 36 : 28) * 4;
+    static std::atomic<uint64_t> raised{0};
+    int device = 0;
+    if (bytes > 48 * 1024 && setup_pending(raised, &device)) {
+        TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemv_units<T, L>), hipFuncAttributeMaxDynamicSharedMemorySize, 12288 / 32 * 36 * 4));
+        setup_done(raised, device);
+    }
+    uint32_t blocks = grid_rows((a.rows + kWave / L - 1) / (kWave / L), 4);
+    const uint32_t most = a.count == 1 ? 1024u : 2048u;
+    if (blocks > most) blocks = most;
+    TSP_LAUNCH("gemv_units", stream, gemv_units<T, L><<<dim3(blocks, a.count), 256, bytes, stream>>>(a));
+    return launch_status("gemv_units");
+}
+
+template <uint32_t T>
+int launch_units(const GemvArgs& a, hipStream_t stream) {
+    // Lanes per row: the count that leaves the fewest lanes without a unit in a row's last round (at 16 000 x 2560, 40 units: 8 lanes
+    // 8.0 us, 64 lanes 10.7), sixteen where several leave equally few; more where that would leave the chip with fewer than 512
+    // waves (at 512 x 2560: 64 lanes 4.2 us, 8 lanes 6.0).
+    const uint32_t units = a.columns / (T == 8 ? 32 : 64);
+    uint32_t lanes = 16;
+    auto idle = [&](uint32_t l) { return (units + l - 1) / l * l; };
+    for (const uint32_t l : {32u, 8u, 64u}) if (idle(l) < idle(lanes)) lanes = l;
+    while (lanes < 64 && uint64_t(a.rows) * a.count * lanes / 64 < 512) lanes *= 2;
+    switch (lanes) {
+    case 8: return launch_units_lanes<T, 8>(a, stream);
+    case 16: return launch_units_lanes<T, 16>(a, stream);
+    case 32: return launch_units_lanes<T, 32>(a, stream);
+    default: return launch_units_lanes<T, 64>(a, stream);
+    }
 }
 
 int launch_gemv(uint32_t encoding, uint32_t layout, GemvArgs a, hipStream_t stream) {
@@ -318,6 +544,10 @@ int launch_gemv(uint32_t encoding, uint32_t layout, GemvArgs a, hipStream_t stre
 #undef TSP_Q4K_CASE
     }
     TSP_REQUIRE(layout == TSP_LAYOUT_GGUF, "no GEMV kernel for this layout/encoding/shape");
+    if (gemv_units_takes(encoding, a)) {
+        if (encoding == 12) return launch_units<12>(a, stream);
+        return encoding == 14 ? launch_units<14>(a, stream) : launch_units<8>(a, stream);
+    }
     // 16-byte pieces of every row of either operand
     if (encoding == 0 && aligned && a.columns % 4 == 0 && reinterpret_cast<uintptr_t>(a.x) % 16 == 0 && a.x_stride % 16 == 0) {
         const dim3 grid(grid_rows(a.rows, 2), a.count);
@@ -349,6 +579,17 @@ int check_shape(uint32_t encoding, uint32_t layout, uint64_t matrix_bytes, uint3
 }
 
 }  // namespace
+
+namespace tsp {
+
+int gemv_q8_row(const void* matrix, const float* x, float* y, uint32_t columns, uint32_t rows, uint32_t* error_word, hipStream_t stream, bool* taken) {
+    GemvArgs a{};
+    a.matrix = static_cast<const uint8_t*>(matrix); a.x = x; a.y = y; a.columns = columns; a.rows = rows; a.experts = a.count = 1; a.error_word = error_word;
+    *taken = gemv_units_takes(8, a);
+    return *taken ? launch_units<8>(a, stream) : TSP_OK;
+}
+
+}  // namespace tsp
 
 extern "C" int tsp_gemv_rows(uint32_t encoding, uint32_t layout, const void* matrix, uint64_t matrix_bytes, const float* x,
                              uint64_t x_stride_bytes, float* y, uint64_t y_stride_bytes, uint32_t count, uint32_t columns,

@@ -12,6 +12,7 @@
 //
 // so the four bytes convert with v_cvt_f32_ubyte0..3 and a masked byte (u = 0x80) contributes 0.
 #include "decode.hpp"
+#include "gemv.hpp"
 #include "q8_mfma.hpp"
 
 using namespace tsp;
@@ -182,6 +183,14 @@ extern "C" int tsp_q8_matvec_many(uint32_t layout, const void* matrix, uint64_t 
     TSP_REQUIRE(!ranges_overlap(y, y_span, matrix, matrix_bytes) && !ranges_overlap(y, y_span, x, x_span), "Q8-many output overlaps an input");
     const Q8Args a{static_cast<const uint8_t*>(matrix), x, y, columns, rows, error_word};
     const auto s = static_cast<hipStream_t>(stream);
+    // One row against a matrix of less than 100 MB, or of a width the persistent matrix-core kernel does not take: that kernel's
+    // eight waves per compute unit share out 32-row tiles, of which there are too few (at 4096 x 2048 20.3 us, 5.2 here; at
+    // 60 000 x 2048, 130 MB, 32.2 and 33.6)
+    if (layout == TSP_LAYOUT_GGUF && width == 1 && (matrix_bytes < 100000000 || !q8_mfma_supported(matrix, x, columns, rows))) {
+        bool taken = false;
+        const int rc = gemv_q8_row(matrix, x, y, columns, rows, error_word, s, &taken);
+        if (taken) return rc;
+    }
     if (layout == TSP_LAYOUT_GGUF && q8_mfma_supported(matrix, x, columns, rows)) return q8_mfma(matrix, x, y, columns, rows, width, error_word, s);
     if (layout == TSP_LAYOUT_Q8_LANES_V1 && q8_lanes_mfma_supported(matrix, x, columns, rows))
         return q8_lanes_mfma(matrix, x, y, columns, rows, width, error_word, s);
