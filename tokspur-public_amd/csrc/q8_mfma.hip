@@ -56,8 +56,8 @@ __global__ void clear_rows(float4* out, uint64_t count4) {
 }
 
 // The token rows of a workgroup, [kRows, K] from column k0 on, in chunks of eight columns: chunk i = tid + j * kThreads is columns
-// 8 (i % (K / 8)) .. + 7 of row i / (K / 8). kRows * K / 8 <= 2048 = kMine * kThreads for K <= 2048 (8 rows) or 1024 (16 rows).
-constexpr uint32_t kMine = 4;
+// 8 (i % (K / 8)) .. + 7 of row i / (K / 8). kRows * K / 8 <= 2560 = kMine * kThreads for K <= 2560 (8 rows) or 1280 (16 rows).
+constexpr uint32_t kMine = 5, kMostColumns = kMine * kThreads;
 
 template <int kRows>
 __device__ __forceinline__ void request_token_rows(const Q8MfmaArgs& a, uint32_t K, uint32_t k0, float4 (&xv)[kMine][2]) {
@@ -493,12 +493,12 @@ __global__ __launch_bounds__(kThreads, 1) void q8_lanes_mfma_kernel(Q8MfmaArgs a
 namespace tsp {
 
 bool q8_mfma_supported(const void* matrix, const float* x, uint32_t columns, uint32_t rows) {
-    return columns % 256 == 0 && columns <= 2048 && rows >= 32 && reinterpret_cast<uintptr_t>(matrix) % 16 == 0 &&
+    return columns % 256 == 0 && columns <= kMostColumns && rows >= 32 && reinterpret_cast<uintptr_t>(matrix) % 16 == 0 &&
            reinterpret_cast<uintptr_t>(x) % 16 == 0;
 }
 
 bool q8_mfma_supported_16(const void* matrix, const float* x, const float* y, uint32_t columns, uint32_t rows) {
-    return q8_mfma_supported(matrix, x, columns, rows) && columns % 1024 == 0 && rows >= 64 && rows % 4 == 0 &&
+    return q8_mfma_supported(matrix, x, columns, rows) && columns % 512 == 0 && rows >= 64 && rows % 4 == 0 &&
            reinterpret_cast<uintptr_t>(y) % 16 == 0;
 }
 
@@ -510,9 +510,10 @@ int q8_mfma(const void* matrix, const float* x, float* y, uint32_t columns, uint
     static int units_of[64] = {};
     int device = 0;
     if (setup_pending(raised, &device)) {
-        const int most = int(2 * 8 * 2048 * 2 + kWaves * kTileBytes);
+        const int most = int(2 * 8 * kMostColumns * 2 + kWaves * kTileBytes);
         TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_mfma_kernel<1, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
         TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_mfma_kernel<2, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
+        TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_mfma_kernel<1, 16>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
         TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_mfma_kernel<2, 16>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
         TSP_HIP(hipDeviceGetAttribute(&units_of[device], hipDeviceAttributeMultiprocessorCount, device));
         setup_done(raised, device);
@@ -526,7 +527,8 @@ int q8_mfma(const void* matrix, const float* x, float* y, uint32_t columns, uint
         if (pairs * kWaves > tiles) pairs = (tiles + kWaves - 1) / kWaves;
         const uint64_t count4 = uint64_t(width) * rows / 4;
         TSP_LAUNCH("clear_rows", s, clear_rows<<<uint32_t((count4 + 255) / 256), 256, 0, s>>>(reinterpret_cast<float4*>(y), count4));
-        TSP_LAUNCH("q8_mfma", s, q8_mfma_kernel<2, 16><<<2 * pairs, kThreads, lds_bytes, s>>>(a));
+        if ((columns / 512) % 2 == 0) TSP_LAUNCH("q8_mfma", s, q8_mfma_kernel<2, 16><<<2 * pairs, kThreads, lds_bytes, s>>>(a));
+        else TSP_LAUNCH("q8_mfma", s, q8_mfma_kernel<1, 16><<<2 * pairs, kThreads, lds_bytes, s>>>(a));
         return launch_status("q8_mfma");
     }
     if (grid * kWaves > tiles) grid = (tiles + kWaves - 1) / kWaves;
@@ -537,7 +539,7 @@ int q8_mfma(const void* matrix, const float* x, float* y, uint32_t columns, uint
 }
 
 bool q8_lanes_mfma_supported(const void* matrix, const float* x, uint32_t columns, uint32_t rows) {
-    return columns % 512 == 0 && columns <= 2048 && rows >= 16 && reinterpret_cast<uintptr_t>(matrix) % 16 == 0 &&
+    return columns % 512 == 0 && columns <= kMostColumns && rows >= 16 && reinterpret_cast<uintptr_t>(matrix) % 16 == 0 &&
            reinterpret_cast<uintptr_t>(x) % 16 == 0;
 }
 
@@ -554,7 +556,7 @@ int q8_lanes_mfma(const void* matrix, const float* x, float* y, uint32_t columns
     static int units_of[64] = {};
     int device = 0;
     if (setup_pending(raised, &device)) {
-        const int most = int(2 * 8 * 2048 * 2 + kWaves * kLaneTileBytes);
+        const int most = int(2 * 8 * kMostColumns * 2 + kWaves * kLaneTileBytes);
         TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_lanes_mfma_kernel<1, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
         TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_lanes_mfma_kernel<2, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
         TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_lanes_mfma_kernel<1, 16>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
