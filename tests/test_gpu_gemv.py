@@ -275,6 +275,31 @@ def test_dense_mm_q8_staged(gpu, tsp, orc, synth, tokens, cols, rows):
     gpu.clear_error()
 
 
+@pytest.mark.parametrize("tokens,cols,rows,pad", [(2, 64, 1, 0), (7, 640, 33, 0), (8, 2560, 640, 0), (9, 320, 18, 0), (16, 1088, 47, 12), (5, 2048, 160, 4),
+                                                  (23, 2560, 48, 0), (3, 96, 20, 0), (6, 512, 24640, 0), (15, 512, 14020, 0), (11, 1280, 14001, 0),
+                                                  (7, 2560, 24577, 0), (14, 2560, 14004, 0), (27, 1024, 14004, 0)])
+def test_dense_mm_q8_few_rows(gpu, tsp, orc, synth, tokens, cols, rows, pad):
+    # every kernel that a few raw Q8_0 token rows can go to: 16-row tiles (any multiple of 64 columns, rows any distance apart), the
+    # persistent kernel from 24 576 rows on (14 000 at nine tokens) with eight and sixteen token rows, decoded weights below that
+    w = synth.matrix(8, 2200 + cols, rows, cols)
+    x = synth.activations_f32(2201 + tokens, (tokens, cols + pad))
+    x[0] *= 1e-20
+    x[-1] *= 1e4
+    check = np.unique(np.r_[0:min(rows, 40), max(0, rows - 40):rows])
+    part = np.ascontiguousarray(w.reshape(rows, -1)[check]).reshape(-1)
+    want = np.stack([orc.reference_gemv(8, part, cols, len(check), np.ascontiguousarray(x[t, :cols])) for t in range(tokens)])
+    out = gpu.full((tokens, rows + pad), -5.0)
+    tsp.dense_mm_q8(gpu, tsp.LAYOUT_GGUF, gpu.upload(w), gpu.upload(x), tokens, cols, rows, out=out, x_stride=(cols + pad) * 4, out_stride=(rows + pad) * 4)
+    got = out.cpu().numpy()
+    # against the sum of |w| |x|: 2^-22 for the two halves of an activation, and a few 2^-24 for each rounding on the way through
+    # 32-column sums and their addition; where eight or sixteen rows share one power-of-two scale, 2^-38 of the largest of them all
+    blocks = part.reshape(len(check), -1, 34)
+    weight = np.abs(blocks[:, :, 2:].view(np.int8).astype(np.float64)) * np.ascontiguousarray(blocks[:, :, :2]).view(np.float16).astype(np.float64)
+    weight = weight.reshape(len(check), cols)
+    bound = 2.0 ** -19 * (np.abs(x[:, :cols].astype(np.float64)) @ weight.T) + 2.0 ** -38 * np.abs(x).max() * weight.sum(1)
+    assert (np.abs(got[:, check] - want) <= bound).all() and (got[:, rows:] == -5.0).all() and gpu.error() == 0
+
+
 @pytest.mark.parametrize("width", [1, 2, 4, 8])
 @pytest.mark.parametrize("cols,rows", [(2048, 37), (64, 5), (96, 7), (4096, 9)])
 def test_q8_matvec_many(gpu, tsp, orc, synth, width, cols, rows):

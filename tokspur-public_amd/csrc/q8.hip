@@ -14,6 +14,7 @@
 #include "decode.hpp"
 #include "gemv.hpp"
 #include "q8_mfma.hpp"
+#include "q8_small.hpp"
 
 using namespace tsp;
 
@@ -169,6 +170,15 @@ int launch(uint32_t layout, const Q8Args& a, hipStream_t stream) {
     return launch_status("q8_blocks");
 }
 
+// Two to sixteen token rows against raw rows: a workgroup per 16 matrix rows (q8_small.hip), or the persistent kernel (q8_mfma.hip).
+// The latter's time hardly falls below 24 us (2048 columns; 17 at nine tokens or more) however few the rows, the former's is
+// proportional to them: 15.6 against 24.6 us at 16 000 x 2048, 28.8 against 25.0 at 32 000, at 1024 columns 20 against 16;
+// with nine or more tokens 6.5 against 17.3 at 4096, 21 against 18.6 at 16 000. Widths that the latter refuses all go to the former.
+bool small_rows(const void* matrix, const float* x, uint64_t x_stride_bytes, uint32_t columns, uint32_t rows, uint32_t tokens) {
+    return q8_small_takes(matrix, x, x_stride_bytes, columns, rows) &&
+           (rows < (tokens > 8 ? 14000u : 24576u) || x_stride_bytes != uint64_t(columns) * 4 || !q8_mfma_supported(matrix, x, columns, rows));
+}
+
 }  // namespace
 
 extern "C" int tsp_q8_matvec_many(uint32_t layout, const void* matrix, uint64_t matrix_bytes, const float* x, float* y,
@@ -183,6 +193,8 @@ extern "C" int tsp_q8_matvec_many(uint32_t layout, const void* matrix, uint64_t 
     TSP_REQUIRE(!ranges_overlap(y, y_span, matrix, matrix_bytes) && !ranges_overlap(y, y_span, x, x_span), "Q8-many output overlaps an input");
     const Q8Args a{static_cast<const uint8_t*>(matrix), x, y, columns, rows, error_word};
     const auto s = static_cast<hipStream_t>(stream);
+    if (layout == TSP_LAYOUT_GGUF && width > 1 && small_rows(matrix, x, uint64_t(columns) * 4, columns, rows, width))
+        return q8_small(matrix, x, uint64_t(columns) * 4, y, uint64_t(rows) * 4, columns, rows, width, error_word, s);
     // One row against a matrix of less than 100 MB, or of a width the persistent matrix-core kernel does not take: that kernel's
     // eight waves per compute unit share out 32-row tiles, of which there are too few (at 4096 x 2048 20.3 us, 5.2 here; at
     // 60 000 x 2048, 130 MB, 32.2 and 33.6)
@@ -213,29 +225,36 @@ extern "C" int tsp_dense_mm_q8(uint32_t layout, const void* matrix, uint64_t mat
     const uint64_t out_span = uint64_t(tokens - 1) * output_stride_bytes + uint64_t(rows) * 4;
     TSP_REQUIRE(!ranges_overlap(output, out_span, matrix, matrix_bytes) && !ranges_overlap(output, out_span, input, in_span),
                 "dense Q8_0 GEMM output overlaps an input");
-    // Token rows that lie back to back go eight, four, two, one at a time (each weight decoded once for the group, the
-    // width sequence of src/q8_many.cpp:20-29); rows with padding between them go one by one.
+    // Eight token rows, up to sixteen where a kernel takes them, go through a matrix-core kernel in one pass over the weights;
+    // where none does and the rows lie back to back they go eight, four, two, one at a time (the width sequence of
+    // src/q8_many.cpp:20-29), and one by one where there is padding between them.
     const bool packed = input_stride_bytes == uint64_t(columns) * 4 && output_stride_bytes == uint64_t(rows) * 4;
-    // Nine or more packed rows left: up to sixteen go through the matrix-core kernel in one pass over the weights.
-    const bool whole = packed && matrix && error_word && columns % 32 == 0 && rows <= 1000000 && uint64_t(columns / 32) * rows * 34 == matrix_bytes;
-    const bool lanes = layout == TSP_LAYOUT_Q8_LANES_V1;
-    const bool sixteen = whole && (layout == TSP_LAYOUT_GGUF ? q8_mfma_supported_16(matrix, input, output, columns, rows)
-                                                            : lanes && q8_lanes_mfma_supported_16(matrix, input, output, columns, rows));
+    const bool whole = matrix && error_word && columns && columns % 32 == 0 && rows && rows <= 1000000 && uint64_t(columns / 32) * rows * 34 == matrix_bytes;
+    const bool lanes = layout == TSP_LAYOUT_Q8_LANES_V1, raw = layout == TSP_LAYOUT_GGUF;
+    const bool eight = whole && packed && (raw ? q8_mfma_supported(matrix, input, columns, rows) : lanes && q8_lanes_mfma_supported(matrix, input, columns, rows));
+    const bool sixteen = eight && (raw ? q8_mfma_supported_16(matrix, input, output, columns, rows) : q8_lanes_mfma_supported_16(matrix, input, output, columns, rows));
     for (uint32_t done = 0; done < tokens;) {
-        if (sixteen && tokens - done > 8) {
-            const uint32_t width = tokens - done < 16 ? tokens - done : 16;
-            const int rc = (lanes ? q8_lanes_mfma : q8_mfma)(matrix, input + uint64_t(done) * columns, output + uint64_t(done) * rows, columns, rows, width,
-                                                             error_word, static_cast<hipStream_t>(stream));
+        const uint32_t left = tokens - done;
+        const float* const from = reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(input) + uint64_t(done) * input_stride_bytes);
+        float* const to = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(output) + uint64_t(done) * output_stride_bytes);
+        const auto s = static_cast<hipStream_t>(stream);
+        const uint32_t most = left < 16 ? left : 16;
+        if (left > 1 && whole && raw && small_rows(matrix, input, input_stride_bytes, columns, rows, sixteen || !eight ? most : 8)) {
+            const int rc = q8_small(matrix, from, input_stride_bytes, to, output_stride_bytes, columns, rows, most, error_word, s);
+            if (rc != TSP_OK) return rc;
+            done += most;
+            continue;
+        }
+        if (eight && left > 1) {
+            const uint32_t width = sixteen ? most : left < 8 ? left : 8;
+            const int rc = (lanes ? q8_lanes_mfma : q8_mfma)(matrix, from, to, columns, rows, width, error_word, s);
             if (rc != TSP_OK) return rc;
             done += width;
             continue;
         }
         uint32_t width = 1;
         if (packed) tsp_q8_many_width(tokens - done, &width);
-        const int rc = tsp_q8_matvec_many(layout, matrix, matrix_bytes,
-                                          reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(input) + uint64_t(done) * input_stride_bytes),
-                                          reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(output) + uint64_t(done) * output_stride_bytes),
-                                          columns, rows, width, error_word, stream);
+        const int rc = tsp_q8_matvec_many(layout, matrix, matrix_bytes, from, to, columns, rows, width, error_word, stream);
         if (rc != TSP_OK) return rc;
         done += width;
     }

@@ -130,6 +130,19 @@ __device__ __forceinline__ float wave_largest(float v) {
     return fmaxf(fmaxf(a, b), fmaxf(c, d));
 }
 
+// The largest of each aligned group of 16 lanes, over unsigned values (magnitudes as bits: infinities and NaNs come out on top).
+template <int Ctrl>
+__device__ __forceinline__ uint32_t dpp_max_bits(uint32_t v) {
+    const uint32_t moved = uint32_t(__builtin_amdgcn_update_dpp(0, int(v), Ctrl, 0xf, 0xf, true));
+    return moved > v ? moved : v;
+}
+__device__ __forceinline__ uint32_t row16_largest_bits(uint32_t v) {
+    v = dpp_max_bits<0xB1>(v);
+    v = dpp_max_bits<0x4E>(v);
+    v = dpp_max_bits<0x141>(v);
+    return dpp_max_bits<0x140>(v);
+}
+
 // Sum over aligned groups of 8 lanes; every lane of a group receives the group's sum.
 __device__ __forceinline__ float octet_sum(float v) {
     v = dpp_add<0xB1>(v);
