@@ -49,6 +49,33 @@ def rel_l2(got, ref):
 
 # ---------------------------------------------------------------------------------- dense
 
+# the tile shapes of the raw-row kernel: exact 32 x 64, 64 x 64 and 128 x 128 tiles (the last from 513 tiles of 64 x 64 on), fewer than
+# 256 weight rows at any row count, then rounded 64 x 64, 128 x 128 and 128 x 256 tiles; ragged on both sides, and an odd number of
+# super-blocks where two groups of waves share them out (or one, where the second group has none)
+@pytest.mark.parametrize("tokens,rows,cols", [(32, 64, 256), (31, 65, 768), (9, 1, 512), (33, 63, 1280), (64, 130, 256), (65, 129, 768), (511, 4130, 256),
+                                              (449, 4700, 768), (520, 200, 768), (512, 256, 256), (513, 257, 1280), (600, 4001, 768), (520, 8100, 256)])
+def test_dense_mm_q4k_tiles(gpu, tsp, orc, synth, tokens, rows, cols):
+    w = synth.matrix(12, 2900 + rows, rows, cols)
+    x = synth.round_bf16(synth.activations_f32(2901 + tokens, (tokens, cols)))
+    exact = tokens < 512 or rows < 256
+    want = orc.staged_gemm(12, w, cols, x, nrows=rows, stage_f16=not exact)
+    got = tsp.dense_mm(gpu, 12, tsp.LAYOUT_GGUF, gpu.upload(w), gpu.upload(x), tokens, cols, rows).cpu().numpy()
+    assert gpu.error() == 0
+    if exact:  # f32 sums of exact products
+        assert max_rel_error(got, want) <= 2e-5
+    else:
+        # The reference rounds d * sc * q to f32 before it subtracts, one fused multiply-add does not: 2^-24 of a value whose half has steps of
+        # 2^-11 to 2^-10, so about one weight in 2^20 may round to the other neighbouring half, which moves its row's results by at
+        # most 2^-10 |w| |x|. All others: f32 sums of the same products.
+        scale = np.maximum(np.abs(want), np.sqrt((want ** 2).mean(axis=1, keepdims=True)).clip(1.0))
+        error, other = np.abs(got - want), 2.0 ** -10 * np.abs(orc.dequantize(12, w, rows * cols)).max() * np.abs(x).max()
+        assert (error <= 5e-6 * scale + other).all() and (error > 5e-6 * scale).any(axis=0).sum() <= 1 + rows * cols * 2.0 ** -20
+    out = gpu.full((tokens, rows + 3), 7, "int16")
+    tsp.dense_mm(gpu, 12, tsp.LAYOUT_GGUF, gpu.upload(w), gpu.upload(synth.bf16_bits(x)), tokens, cols, rows, out=out, out_bf16=True, out_stride=(rows + 3) * 2)
+    bits = out.cpu().numpy()
+    assert np.array_equal(bf16_to_f32(bits[:, :rows]), synth.round_bf16(got)) and (bits[:, rows:] == 7).all() and gpu.error() == 0
+
+
 @pytest.mark.parametrize("layout", ["raw", "planar"])
 # GGUF rows of 512, 1024 or 2048 columns against at most 384 rows take 64 x 64 tiles with the columns split over the waves:
 # (33, 96, 512), (128, 256, 2048), (130, 300, 1024), (200, 100, 2048), (384, 132, 1024) and (1, 68, 2048) are its shapes (ragged on either

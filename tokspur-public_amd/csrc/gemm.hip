@@ -24,8 +24,7 @@
 //     two and three steps ahead, into a ring of four slabs; one LDS-only barrier per K step.
 //   * For gate/up the two column tiles of a wave are the gate rows and the up rows of the same 32 hidden
 //     units, so SwiGLU is an element-wise epilogue on accumulator registers.
-#include "dense_ksplit.hpp"
-#include "dense_tall.hpp"
+#include "dense_tile.hpp"
 #include "down_resident.hpp"
 #include "gate_up_resident.hpp"
 #include "grouped_staged.hpp"
@@ -662,23 +661,13 @@ extern "C" int tsp_dense_mm(uint32_t encoding, uint32_t layout, const void* matr
     const auto s = static_cast<hipStream_t>(stream);
     auto* xh = static_cast<_Float16*>(workspace);
     auto* sx = reinterpret_cast<_Float16*>(static_cast<uint8_t*>(workspace) + align256(uint64_t(tokens) * columns * 2));
-    if (encoding == 12 && layout == TSP_LAYOUT_GGUF && dense_tall_takes(tokens, rows, columns, matrix_bytes)) {
-        // a thousand rows and more: tiles 128 or 256 rows high, weights rounded once to half (the engine's arithmetic for this product)
-        int rc = convert_rows(input, input_stride_bytes, input_is_bf16, xh, sx, tokens, columns, error_word, s);  // with the sums come the swapped columns
-        if (rc != TSP_OK) return rc;
-        DenseTallArgs t{};
-        t.a = xh; t.a_stride = columns; t.w = static_cast<const uint8_t*>(matrix); t.m = tokens; t.n = rows; t.k = columns;
-        t.out = output; t.out_stride = output_stride_bytes; t.out_bf16 = output_is_bf16; t.error_word = error_word;
-        return launch_dense_tall(t, s);
-    }
-    int rc = convert_rows(input, input_stride_bytes, input_is_bf16, xh, encoding == 12 ? sx : nullptr, tokens, columns, error_word, s);
+    int rc = convert_rows(input, input_stride_bytes, input_is_bf16, xh, encoding == 12 ? sx : nullptr, tokens, columns, error_word, s);  // with the sums come the swapped columns
     if (rc != TSP_OK) return rc;
-    if (encoding == 12 && layout == TSP_LAYOUT_GGUF && dense_ksplit_takes(tokens, rows, columns)) {
-        // few rows: 64 x 64 tiles with the columns split over a workgroup's waves, so that the chip has tiles enough
-        DenseKsplitArgs t{};
-        t.a = xh; t.sx = sx; t.w = static_cast<const uint8_t*>(matrix); t.m = tokens; t.n = rows; t.k = columns;
+    if (layout == TSP_LAYOUT_GGUF) {
+        DenseTileArgs t{};
+        t.a = xh; t.a_stride = columns; t.sx = sx; t.w = static_cast<const uint8_t*>(matrix); t.m = tokens; t.n = rows; t.k = columns;
         t.out = output; t.out_stride = output_stride_bytes; t.out_bf16 = output_is_bf16; t.error_word = error_word;
-        return launch_dense_ksplit(t, s);
+        return launch_dense_tile(t, s);
     }
     a.a = xh; a.a_stride = columns; a.sx = sx; a.w0 = static_cast<const uint8_t*>(matrix); a.experts = 1;
     a.m = tokens; a.n = rows; a.k = columns; a.out = output; a.out_stride = output_stride_bytes; a.out_scale = 1.0f;
@@ -686,10 +675,8 @@ extern "C" int tsp_dense_mm(uint32_t encoding, uint32_t layout, const void* matr
     const uint32_t col_tiles = (rows + 255) / 256, tasks = (tokens + kTaskRows - 1) / kTaskRows;
     if (encoding == 14) return output_is_bf16 ? launch<B_Q6K_PLANAR, EPI_BF16, ROWS_DENSE>(a, col_tiles, tasks, s)
                                                : launch<B_Q6K_PLANAR, EPI_F32, ROWS_DENSE>(a, col_tiles, tasks, s);
-    if (layout == TSP_LAYOUT_PLANAR_V3) return output_is_bf16 ? launch<B_Q4K_PLANAR, EPI_BF16, ROWS_DENSE>(a, col_tiles, tasks, s)
-                                                               : launch<B_Q4K_PLANAR, EPI_F32, ROWS_DENSE>(a, col_tiles, tasks, s);
-    return output_is_bf16 ? launch<B_Q4K_RAW, EPI_BF16, ROWS_DENSE>(a, col_tiles, tasks, s)
-                          : launch<B_Q4K_RAW, EPI_F32, ROWS_DENSE>(a, col_tiles, tasks, s);
+    return output_is_bf16 ? launch<B_Q4K_PLANAR, EPI_BF16, ROWS_DENSE>(a, col_tiles, tasks, s)
+                          : launch<B_Q4K_PLANAR, EPI_F32, ROWS_DENSE>(a, col_tiles, tasks, s);
 }
 
 // ---------------------------------------------------------------- grouped GEMM over raw GGUF expert stacks
