@@ -275,9 +275,23 @@ def test_dense_mm_q8_staged(gpu, tsp, orc, synth, tokens, cols, rows):
     gpu.clear_error()
 
 
+@pytest.mark.parametrize("tokens,cols,rows", [(33, 2048, 31), (31, 2112, 65), (2, 64, 1), (65, 576, 33), (96, 192, 6400), (97, 64, 6401)])
+def test_dense_mm_q8_staged_tiles(gpu, tsp, synth, tokens, cols, rows):
+    # the columns shared out over eight waves (2048 columns and more) or four, fewer steps than waves, ragged tiles; the last shape is
+    # more tiles than that form takes. A weight and an activation are rounded to halves: 2^-11 each, so 2^-10 of the sum of |w| |x|.
+    w = synth.matrix(8, 2400 + cols, rows, cols)
+    x = synth.activations_f32(2401 + tokens, (tokens, cols))
+    got = tsp.dense_mm_q8_staged(gpu, tsp.LAYOUT_GGUF, gpu.upload(w), gpu.upload(x), tokens, cols, rows).cpu().numpy()
+    blocks = w.reshape(rows, -1, 34)
+    weight = blocks[:, :, 2:].view(np.int8).astype(np.float64) * np.ascontiguousarray(blocks[:, :, :2]).view(np.float16).astype(np.float64)
+    weight = weight.reshape(rows, cols)
+    bound = (2.0 ** -10 + cols * 2.0 ** -24) * (np.abs(x.astype(np.float64)) @ np.abs(weight).T)
+    assert (np.abs(got - x.astype(np.float64) @ weight.T) <= bound).all() and gpu.error() == 0
+
+
 @pytest.mark.parametrize("tokens,cols,rows,pad", [(2, 64, 1, 0), (7, 640, 33, 0), (8, 2560, 640, 0), (9, 320, 18, 0), (16, 1088, 47, 12), (5, 2048, 160, 4),
                                                   (23, 2560, 48, 0), (3, 96, 20, 0), (6, 512, 24640, 0), (15, 512, 14020, 0), (11, 1280, 14001, 0),
-                                                  (7, 2560, 24577, 0), (14, 2560, 14004, 0), (27, 1024, 14004, 0)])
+                                                  (7, 2560, 24577, 0), (14, 2560, 14004, 0), (27, 1024, 14004, 0), (41, 192, 30, 4)])
 def test_dense_mm_q8_few_rows(gpu, tsp, orc, synth, tokens, cols, rows, pad):
     # every kernel that a few raw Q8_0 token rows can go to: 16-row tiles (any multiple of 64 columns, rows any distance apart), the
     # persistent kernel from 24 576 rows on (14 000 at nine tokens) with eight and sixteen token rows, decoded weights below that

@@ -1,13 +1,15 @@
 // Dense Q8_0 GEMM for many token rows (the shared expert of a prefill chunk): out[t, n] = sum_k x[t, k] * d[n, k/32] * q[n, k].
 //
 // The streaming kernels of q8.hip / q8_mfma.hip read the whole matrix once per 8 or 16 token rows: right for decode,
-// hundreds of passes for a 2048-token chunk. Here the matrix is decoded once per call into halves (d * q rounded to
-// nearest: 11 significant bits, what the engine's own kernel stages, include/tokspur/graph.hpp:860 and
-// kernels/grouped_mm.metal:239-243), the token rows are rounded to halves as well, and one matrix-core GEMM with f32
-// accumulation multiplies the two. Both operands are K-contiguous rows, so the GEMM is the "NT" form and both tiles are
-// staged the same way.
+// hundreds of passes for a 2048-token chunk. Here a weight is the half nearest d * q (11 significant bits, what the engine's own
+// kernel stages, include/tokspur/graph.hpp:860 and kernels/grouped_mm.metal:239-243), the token rows are rounded to halves as
+// well, and the matrix cores multiply the two with f32 accumulation.
 //
-// GEMM kernel: a workgroup of four waves owns a 64 x 64 output tile (each wave a 32 x 32 MFMA tile) and walks K in
+// A short chunk goes through one kernel that decodes both operands on their way into the MFMAs (q8_gemm_split, raw rows). With more
+// tokens every operand would be decoded again and again, ten to forty times over, so one launch decodes both into the workspace and
+// f16_gemm_nt multiplies them.
+//
+// f16_gemm_nt: a workgroup of four waves owns a 64 x 64 output tile (each wave a 32 x 32 MFMA tile) and walks K in
 // steps of 64 halfs. Every byte travels global -> LDS directly (16 bytes per lane, no registers in between) into a ring
 // of four stages, three steps ahead of the multiply; chunk c of row r of a slab sits at position r * 8 + (c ^ (r & 7)),
 // which the loads fill linearly by lane and the fragment reads spread over all banks. No other vector-memory operation
@@ -27,6 +29,16 @@ struct F16GemmArgs {
     const _Float16* x;  // [m][k]
     const _Float16* w;  // [n][k]
     float* out;         // rows out_stride bytes apart
+    uint64_t out_stride;
+    uint32_t m, n, k;
+    uint32_t* error_word;
+};
+
+struct Q8GemmArgs {
+    const float* x;  // rows x_stride bytes apart
+    uint64_t x_stride;
+    const uint8_t* w;  // [n][k / 32 blocks of 34 B]
+    float* out;        // rows out_stride bytes apart
     uint64_t out_stride;
     uint32_t m, n, k;
     uint32_t* error_word;
@@ -95,50 +107,168 @@ __global__ __launch_bounds__(256, 2) void f16_gemm_nt(F16GemmArgs a) {
     publish_error(bad, a.error_word);
 }
 
-// Two weights per thread: GGUF rows are 34-byte blocks (f16 d, 32 int8); q8_lanes_v1 rows keep the scales first, then runs
-// of 16 blocks with byte = index * width + block % 16 (src/expert_lanes.cpp:60-119).
-__global__ __launch_bounds__(256) void q8_rows_to_f16(const uint8_t* __restrict__ matrix, uint32_t layout, _Float16* __restrict__ out,
-                                                      uint32_t columns, uint32_t rows) {
-    const uint64_t pair = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (pair >= uint64_t(rows) * (columns / 2)) return;
-    const uint32_t row = uint32_t(pair / (columns / 2)), c = uint32_t(pair % (columns / 2)) * 2;
-    const uint32_t blocks = columns / 32, block = c / 32, index = c % 32;
-    const uint8_t* data = matrix + uint64_t(row) * blocks * 34;
-    float d;
-    int q0, q1;
-    if (layout == TSP_LAYOUT_GGUF) {
-        const uint8_t* b = data + block * 34;
-        d = half_bits_to_float(uint32_t(b[0]) | (uint32_t(b[1]) << 8));
-        q0 = int(int8_t(b[2 + index]));
-        q1 = int(int8_t(b[3 + index]));
-    } else {
-        const uint32_t run = block / 16, width = blocks - run * 16 < 16 ? blocks - run * 16 : 16;
-        const uint8_t* q = data + blocks * 2 + run * 512 + block % 16;
-        d = half_bits_to_float(uint32_t(data[block * 2]) | (uint32_t(data[block * 2 + 1]) << 8));
-        q0 = int(int8_t(q[index * width]));
-        q1 = int(int8_t(q[(index + 1) * width]));
+// A workgroup is one 32 x 32 output tile and its waves take the columns in turns of 64: a chunk of 64 tokens against 640 rows is 40
+// workgroups of eight waves, each wave a chain of five steps. A wave reads a step as it lies (256 bytes of 32 token rows,
+// 17 dwords of 32 weight rows), two steps' requests in flight, and puts it into fragment order through LDS of its own: no barrier
+// until the waves' sums meet, which are added in wave order.
+// Bound by latency: 60 tokens, 2560 -> 640 columns 8.8 us, 640 -> 2560 4.9 (two conversions and a GEMM: 18.7 and 14.4).
+template <int WAVES>
+__global__ __launch_bounds__(WAVES * kWave, 4) void q8_gemm_split(Q8GemmArgs a) {
+    constexpr uint32_t kEdge = 32, kDwords = 17, kWLoads = (kEdge * kDwords + kWave - 1) / kWave, kPitch = kStep + 8;
+    struct WaveLds {
+        _Float16 x[kEdge * kPitch];
+        uint32_t w[kWLoads * kWave];
+    };
+    static_assert(sizeof(WaveLds) >= kEdge * kEdge * 4);
+    __shared__ __attribute__((aligned(16))) WaveLds lds[WAVES];
+    const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid / kWave)));
+    const uint32_t col = lane % 32, khalf = lane / 32;
+    const uint32_t m0 = blockIdx.y * kEdge, n0 = blockIdx.x * kEdge, steps = a.k / kStep, row_bytes = a.k / 32 * 34;
+    const uint8_t* const w_base = a.w + uint64_t(n0) * row_bytes;
+    uint32_t w_at[kWLoads];
+#pragma unroll
+    for (uint32_t q = 0; q < kWLoads; ++q) {
+        const uint32_t id = q * kWave + lane < kEdge * kDwords ? q * kWave + lane : kEdge * kDwords - 1, r = n0 + id / kDwords;
+        w_at[q] = ((r < a.n ? r : a.n - 1) - n0) * row_bytes + id % kDwords * 4;
     }
-    const f16x2 pairs{_Float16(d * float(q0)), _Float16(d * float(q1))};  // d * q is exact in f32: one rounding
-    *reinterpret_cast<f16x2*>(out + uint64_t(row) * columns + c) = pairs;
+    const uint8_t* x_from[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const uint32_t r = m0 + i * 4 + lane / 16;
+        x_from[i] = reinterpret_cast<const uint8_t*>(a.x) + (r < a.m ? r : a.m - 1) * a.x_stride + lane % 16 * 16;
+    }
+    struct Step { f32x4 x[8]; uint32_t w[kWLoads]; };
+    auto fetch = [&](uint32_t s) {
+        Step t;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) t.x[i] = *reinterpret_cast<const f32x4*>(x_from[i] + uint64_t(s) * (kStep * 4));
+#pragma unroll
+        for (uint32_t q = 0; q < kWLoads; ++q) t.w[q] = *reinterpret_cast<const uint32_t*>(w_base + uint64_t(s) * (kDwords * 4) + w_at[q]);
+        return t;
+    };
+    _Float16* const xs = lds[wave].x;
+    uint32_t* const ws = lds[wave].w;
+    uint32_t largest = 0;
+    f32x16 acc{};
+    Step next = fetch(wave < steps ? wave : steps - 1);
+    for (uint32_t s = wave; s < steps; s += WAVES) {
+        const Step now = next;
+        next = fetch(s + WAVES < steps ? s + WAVES : s);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            f16x4 h;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) h[e] = _Float16(now.x[i][e]);
+            const uint2 bits = __builtin_bit_cast(uint2, h);
+            // halves without their signs, two to a word: an exponent of ones carries into the bit above
+            largest |= ((bits.x & 0x7fff7fffu) + 0x04000400u) | ((bits.y & 0x7fff7fffu) + 0x04000400u);
+            *reinterpret_cast<f16x4*>(xs + (i * 4 + lane / 16) * kPitch + lane % 16 * 4) = h;
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < kWLoads; ++q) ws[q * kWave + lane] = now.w[q];
+        __builtin_amdgcn_wave_barrier();
+        const uint32_t* const mine = ws + col * kDwords;
+        const uint32_t d_even = mine[0] & 0xffffu, d_odd = mine[8] >> 16;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            // quants 16 (g % 2) + 8 khalf .. + 7 of block g / 2, which starts at byte 34 (g / 2) of the row's 68 with its scale
+            const uint32_t* const q = mine + (g < 2 ? 0 : 9) + g % 2 * 4 + khalf * 2;
+            uint32_t q0 = q[0], q1 = q[1];
+            if (g < 2) {
+                q0 = __builtin_amdgcn_alignbyte(q1, q0, 2);
+                q1 = __builtin_amdgcn_alignbyte(q[2], q1, 2);
+            }
+            const uint32_t d = g < 2 ? d_even : d_odd;
+            const f16x2 d2 = as_h2(d | d << 16);
+            const f16x8 c = quants8(q0, q1);  // exact, as is d: one packed multiply rounds once
+            const f16x2 p0 = f16x2{c[0], c[1]} * d2, p1 = f16x2{c[2], c[3]} * d2, p2 = f16x2{c[4], c[5]} * d2, p3 = f16x2{c[6], c[7]} * d2;
+            const f16x8 fb{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
+            const f16x8 fa = *reinterpret_cast<const f16x8*>(xs + col * kPitch + g * 16 + khalf * 8);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa, fb, acc, 0, 0, 0);
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+    uint32_t bad = largest & 0x80008000u ? uint32_t(TSP_ERRBIT_NONFINITE) : 0u;
+    // accumulator v: token row 8 (v / 4) + 4 khalf + v % 4 of the tile, weight row `col`; the sums lie over their wave's operands
+    float* const sums = reinterpret_cast<float*>(&lds[wave]);
+#pragma unroll
+    for (int v = 0; v < 16; ++v) sums[(8 * (v / 4) + 4 * khalf + v % 4) * kEdge + col] = acc[v];
+    __syncthreads();
+#pragma unroll
+    for (uint32_t i = tid; i < kEdge * kEdge; i += WAVES * kWave) {
+        float value = 0;
+#pragma unroll
+        for (int q = 0; q < WAVES; ++q) value += reinterpret_cast<const float*>(&lds[q])[i];
+        const uint32_t m = m0 + i / kEdge, n = n0 + i % kEdge;
+        if (m < a.m && n < a.n) {
+            if (nonfinite(value)) bad = TSP_ERRBIT_NONFINITE;
+            reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(a.out) + m * a.out_stride)[n] = value;
+        }
+    }
+    publish_error(bad, a.error_word);
 }
 
-// Eight values per thread; a value that does not fit a half (or is not finite) raises the non-finite bit.
-__global__ __launch_bounds__(256) void f32_rows_to_f16(const float* __restrict__ x, uint64_t stride_bytes, _Float16* __restrict__ out,
-                                                       uint32_t rows, uint32_t columns, uint32_t* error_word) {
-    const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+// Both operands to halves in one launch (two small ones cost more than their work): workgroups below `w_groups` decode the matrix, the
+// others round the token rows.
+// Matrix: sixteen weights per thread, half a block. GGUF rows are 34-byte blocks (f16 d, 32 int8); q8_lanes_v1 rows keep the scales
+// first, then runs of 16 blocks with byte = index * width + block % 16 (src/expert_lanes.cpp:60-119).
+// Token rows: eight values per thread; a value that does not fit a half (or is not finite) raises the non-finite bit.
+struct OperandsArgs {
+    const uint8_t* matrix;
+    const float* x;
+    uint64_t x_stride;  // bytes
+    _Float16 *w16, *x16;
+    uint32_t layout, columns, rows, tokens, w_groups;
+    uint32_t* error_word;
+};
+__global__ __launch_bounds__(256) void q8_operands_to_f16(OperandsArgs a) {
+    if (blockIdx.x < a.w_groups) {
+        const uint64_t at = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+        const uint32_t halves = a.columns / 16, blocks = a.columns / 32;
+        if (at >= uint64_t(a.rows) * halves) return;
+        const uint32_t row = uint32_t(at / halves), part = uint32_t(at % halves), block = part / 2, index = part % 2 * 16;
+        const uint8_t* data = a.matrix + uint64_t(row) * blocks * 34;
+        float d;
+        int q[16];
+        if (a.layout == TSP_LAYOUT_GGUF) {
+            const uint16_t* b = reinterpret_cast<const uint16_t*>(data + block * 34);  // rows and blocks are even byte counts
+            d = half_bits_to_float(b[0]);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t two = b[1 + index / 2 + i];
+                q[2 * i] = int(int8_t(two)); q[2 * i + 1] = int(int8_t(two >> 8));
+            }
+        } else {
+            const uint32_t run = block / 16, width = blocks - run * 16 < 16 ? blocks - run * 16 : 16;
+            const uint8_t* from = data + blocks * 2 + run * 512 + block % 16 + index * width;
+            d = half_bits_to_float(uint32_t(data[block * 2]) | (uint32_t(data[block * 2 + 1]) << 8));
+#pragma unroll
+            for (int i = 0; i < 16; ++i) q[i] = int(int8_t(from[i * width]));
+        }
+        f16x8* const to = reinterpret_cast<f16x8*>(a.w16 + uint64_t(row) * a.columns + part * 16);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            f16x8 w;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) w[e] = _Float16(d * float(q[8 * h + e]));  // d * q is exact in f32: one rounding
+            to[h] = w;
+        }
+        return;
+    }
+    const uint64_t i = uint64_t(blockIdx.x - a.w_groups) * blockDim.x + threadIdx.x;
     uint32_t bad = 0;
-    if (i < uint64_t(rows) * (columns / 8)) {
-        const uint32_t r = uint32_t(i / (columns / 8)), c8 = uint32_t(i % (columns / 8));
-        const float* src = reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(x) + uint64_t(r) * stride_bytes) + c8 * 8;
+    if (i < uint64_t(a.tokens) * (a.columns / 8)) {
+        const uint32_t r = uint32_t(i / (a.columns / 8)), c8 = uint32_t(i % (a.columns / 8));
+        const float* src = reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(a.x) + uint64_t(r) * a.x_stride) + c8 * 8;
         f16x8 h;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             h[e] = _Float16(src[e]);
             if ((__builtin_bit_cast(uint16_t, h[e]) & 0x7c00u) == 0x7c00u) bad = TSP_ERRBIT_NONFINITE;
         }
-        *reinterpret_cast<f16x8*>(out + uint64_t(r) * columns + c8 * 8) = h;
+        *reinterpret_cast<f16x8*>(a.x16 + uint64_t(r) * a.columns + c8 * 8) = h;
     }
-    publish_error(bad, error_word);
+    publish_error(bad, a.error_word);
 }
 
 uint64_t align256(uint64_t v) { return (v + 255) / 256 * 256; }
@@ -170,11 +300,23 @@ extern "C" int tsp_dense_mm_q8_staged(uint32_t layout, const void* matrix, uint6
                     !ranges_overlap(workspace, workspace_bytes, output, out_span),
                 "dense Q8_0 GEMM buffers overlap");
     const auto s = static_cast<hipStream_t>(stream);
+    // Up to 600 tiles of 32 x 32 (two or three rounds over the chip): decoded on the way, else decoded once and multiplied, where a round
+    // costs more than the launch saved (2048 columns x 512 rows: 14.8 against 17.2 us at 400 tiles, 20.7 against 18.1 at 656; 640 x
+    // 2560 8.4 against 9.5 at 560, 12.5 against 11.5 at 1040). f32 rows are read sixteen bytes at a time.
+    const uint64_t tiles = uint64_t((rows + 31) / 32) * ((tokens + 31) / 32);
+    if (layout == TSP_LAYOUT_GGUF && tiles <= 600 && reinterpret_cast<uintptr_t>(input) % 16 == 0 && input_stride_bytes % 16 == 0 &&
+        reinterpret_cast<uintptr_t>(matrix) % 4 == 0) {
+        const Q8GemmArgs a{input, input_stride_bytes, static_cast<const uint8_t*>(matrix), output, output_stride_bytes, tokens, rows, columns, error_word};
+        const dim3 grid((rows + 31) / 32, (tokens + 31) / 32);
+        if (columns >= 2048 && tiles <= 256) TSP_LAUNCH("q8_gemm_split", s, q8_gemm_split<8><<<grid, 512, 0, s>>>(a));
+        else TSP_LAUNCH("q8_gemm_split", s, q8_gemm_split<4><<<grid, 256, 0, s>>>(a));
+        return launch_status("q8_gemm_split");
+    }
     _Float16* const w16 = static_cast<_Float16*>(workspace);
     _Float16* const x16 = reinterpret_cast<_Float16*>(static_cast<uint8_t*>(workspace) + align256(uint64_t(rows) * columns * 2));
-    const uint64_t pairs = uint64_t(rows) * (columns / 2), eights = uint64_t(tokens) * (columns / 8);
-    TSP_LAUNCH("q8_rows_to_f16", s, q8_rows_to_f16<<<uint32_t((pairs + 255) / 256), 256, 0, s>>>(static_cast<const uint8_t*>(matrix), layout, w16, columns, rows));
-    TSP_LAUNCH("f32_rows_to_f16", s, f32_rows_to_f16<<<uint32_t((eights + 255) / 256), 256, 0, s>>>(input, input_stride_bytes, x16, tokens, columns, error_word));
+    const uint64_t w_groups = (uint64_t(rows) * (columns / 16) + 255) / 256, x_groups = (uint64_t(tokens) * (columns / 8) + 255) / 256;
+    const OperandsArgs o{static_cast<const uint8_t*>(matrix), input, input_stride_bytes, w16, x16, layout, columns, rows, tokens, uint32_t(w_groups), error_word};
+    TSP_LAUNCH("q8_operands_to_f16", s, q8_operands_to_f16<<<uint32_t(w_groups + x_groups), 256, 0, s>>>(o));
     const F16GemmArgs a{x16, w16, output, output_stride_bytes, tokens, rows, columns, error_word};
     const dim3 grid((rows + kTile - 1) / kTile, (tokens + kTile - 1) / kTile);
     TSP_LAUNCH("f16_gemm_nt", s, f16_gemm_nt<<<grid, 256, 0, s>>>(a));

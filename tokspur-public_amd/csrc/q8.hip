@@ -240,10 +240,7 @@ extern "C" int tsp_dense_mm_q8(uint32_t layout, const void* matrix, uint64_t mat
         const auto s = static_cast<hipStream_t>(stream);
         const uint32_t most = left < 16 ? left : 16;
         if (left > 1 && whole && raw && small_rows(matrix, input, input_stride_bytes, columns, rows, sixteen || !eight ? most : 8)) {
-            const int rc = q8_small(matrix, from, input_stride_bytes, to, output_stride_bytes, columns, rows, most, error_word, s);
-            if (rc != TSP_OK) return rc;
-            done += most;
-            continue;
+            return q8_small(matrix, from, input_stride_bytes, to, output_stride_bytes, columns, rows, left, error_word, s);  // all that is left
         }
         if (eight && left > 1) {
             const uint32_t width = sixteen ? most : left < 8 ? left : 8;

@@ -44,9 +44,10 @@ __global__ __launch_bounds__(kThreads) void q8_small_kernel(Q8SmallArgs a) {
     };
     __shared__ __attribute__((aligned(16))) WaveLds lds[kWaves];
     const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid / kWave))), n16 = lane % 16, kq = lane / 16;
+    const uint32_t token0 = blockIdx.y * kTokens;  // more token rows than that: the grid's second dimension
     const uint32_t row0 = blockIdx.x * kTile, row_bytes = a.columns / 32 * 34, steps = a.columns / kStep;
     const uint8_t* const w = a.matrix + uint64_t(row0) * row_bytes;
-    const uint8_t* const x = reinterpret_cast<const uint8_t*>(a.x);
+    const uint8_t* const x = reinterpret_cast<const uint8_t*>(a.x) + token0 * a.x_stride;
     uint32_t* const weights = lds[wave].weights;
     _Float16* const tokens = lds[wave].tokens;
     float* const back = lds[wave].back;
@@ -63,8 +64,8 @@ __global__ __launch_bounds__(kThreads) void q8_small_kernel(Q8SmallArgs a) {
     }
 #pragma unroll
     for (uint32_t t = 0; t < kTokenLoads; ++t) {
-        const uint32_t token = t * 4 + kq < a.tokens ? t * 4 + kq : a.tokens - 1;
-        x_at[t] = uint32_t(token * a.x_stride) + n16 * 16;
+        const uint32_t token = token0 + t * 4 + kq < a.tokens ? token0 + t * 4 + kq : a.tokens - 1;
+        x_at[t] = uint32_t((token - token0) * a.x_stride) + n16 * 16;
     }
     struct Piece { uint32_t w[kPieceLoads]; f32x4 x[kTokenLoads]; };
     auto fetch = [&](uint32_t s) {
@@ -143,7 +144,7 @@ __global__ __launch_bounds__(kThreads) void q8_small_kernel(Q8SmallArgs a) {
     __syncthreads();
     constexpr uint32_t kValues = WIDE ? 256 : 128;
     if (tid < kValues) {
-        const uint32_t t = tid / 16, r = row0 + n16;
+        const uint32_t t = token0 + tid / 16, r = row0 + n16;
         float value = 0;
 #pragma unroll
         for (uint32_t q = 0; q < kWaves; ++q) {
@@ -170,7 +171,7 @@ bool q8_small_takes(const void* matrix, const float* x, uint64_t x_stride_bytes,
 int q8_small(const void* matrix, const float* x, uint64_t x_stride_bytes, float* y, uint64_t y_stride_bytes, uint32_t columns, uint32_t rows, uint32_t tokens,
              uint32_t* error_word, hipStream_t s) {
     const Q8SmallArgs a{static_cast<const uint8_t*>(matrix), x, x_stride_bytes, y, y_stride_bytes, columns, rows, tokens, error_word};
-    const uint32_t grid = (rows + kTile - 1) / kTile;
+    const dim3 grid((rows + kTile - 1) / kTile, tokens > 8 ? (tokens + 15) / 16 : 1);
     if (tokens > 8) TSP_LAUNCH("q8_small", s, q8_small_kernel<true><<<grid, kThreads, 0, s>>>(a));
     else TSP_LAUNCH("q8_small", s, q8_small_kernel<false><<<grid, kThreads, 0, s>>>(a));
     return launch_status("q8_small");

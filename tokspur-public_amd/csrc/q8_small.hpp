@@ -4,7 +4,7 @@
 
 namespace tsp {
 
-// y[t, r] = sum_k W[r, k] x[t, k] for 1..16 token rows, raw GGUF rows of a multiple of 128 columns, rows any distance apart that
+// y[t, r] = sum_k W[r, k] x[t, k] for any number of token rows, sixteen (eight) at a time, raw GGUF rows of a multiple of 64 columns, rows any distance apart that
 // 16 bytes (x) resp. 4 bytes (y) divide.
 bool q8_small_takes(const void* matrix, const float* x, uint64_t x_stride_bytes, uint32_t columns, uint32_t rows);
 int q8_small(const void* matrix, const float* x, uint64_t x_stride_bytes, float* y, uint64_t y_stride_bytes, uint32_t columns, uint32_t rows, uint32_t tokens,
