@@ -405,34 +405,25 @@ int launch(DenseTileArgs a, hipStream_t s) {
 
 namespace tsp {
 
-int launch_dense_tile(const DenseTileArgs& whole, hipStream_t s) {
-    const uint64_t row_bytes = uint64_t(whole.k) * 2, rows_at_once = ((1ull << 32) - 1) / row_bytes / 256 * 256;  // rows are addressed with 32-bit offsets
-    const bool exact = whole.m < 512 || whole.n < 256 || whole.m > rows_at_once;
-    auto tiles = [](const DenseTileArgs& a, uint64_t high, uint64_t wide) { return (a.m + high - 1) / high * ((a.n + wide - 1) / wide); };
-    for (uint64_t done = 0; done < whole.m; done += rows_at_once) {
-        DenseTileArgs a = whole;
-        a.m = uint32_t(std::min(whole.m - done, rows_at_once));
-        a.a += done * whole.k;
-        a.sx += done * (whole.k / 256) * 16;
-        a.out = static_cast<uint8_t*>(whole.out) + done * whole.out_stride;
-        int rc;
-        if (exact) {
-            // 64 x 64 tiles while the chip takes them all at once, two to a compute unit: 13 to 24 us at 2560 columns, 41 for twice as many,
-            // where 128 x 128 tiles take 34. Up to 32 rows the lower half of a 64-row tile would be empty.
-            if (a.m <= 32) rc = launch<1, 4, 64, 2, true>(a, s);
-            else if (tiles(a, 64, 64) <= 512) rc = launch<2, 4, 64, 2, true>(a, s);
-            else rc = launch<4, 8, 128, 2, true>(a, s);
-        } else {
-            // The shape whose rounds over the chip end first, a round of each as measured at 2048 columns, in us: two 64 x 64 tiles per
-            // compute unit, or one 128 x 128, 128 x 256 or 256 x 256 tile.
-            const uint64_t cost[4] = {(tiles(a, 64, 64) + 511) / 512 * 17, (tiles(a, 128, 128) + 255) / 256 * 25, (tiles(a, 128, 256) + 255) / 256 * 39,
-                                      (tiles(a, 256, 256) + 255) / 256 * 62};
-            const int best = int(std::min_element(cost, cost + 4) - cost);
-            rc = best == 0 ? launch<2, 4, 64, 2, false>(a, s) : best == 1 ? launch<4, 8, 128, 2, false>(a, s) : best == 2 ? launch<4, 8, 256, 1, false>(a, s) : launch<8, 8, 256, 1, false>(a, s);
-        }
-        if (rc != TSP_OK) return rc;
+int launch_dense_tile(const DenseTileArgs& a, hipStream_t s) {
+    auto tiles = [&](uint64_t high, uint64_t wide) { return (a.m + high - 1) / high * ((a.n + wide - 1) / wide); };
+    if (a.m < 512 || a.n < 256) {
+        // 64 x 64 tiles while the chip takes them all at once, two to a compute unit: 13 to 24 us at 2560 columns, 41 for twice as many,
+        // where 128 x 128 tiles take 34. Up to 32 rows the lower half of a 64-row tile would be empty.
+        if (a.m <= 32) return launch<1, 4, 64, 2, true>(a, s);
+        if (tiles(64, 64) <= 512) return launch<2, 4, 64, 2, true>(a, s);
+        return launch<4, 8, 128, 2, true>(a, s);
     }
-    return TSP_OK;
+    // The shape whose rounds over the chip end first, a round of each as measured at 2048 columns, in us: two 64 x 64 tiles per
+    // compute unit, or one 128 x 128, 128 x 256 or 256 x 256 tile.
+    const uint64_t cost[4] = {(tiles(64, 64) + 511) / 512 * 17, (tiles(128, 128) + 255) / 256 * 25, (tiles(128, 256) + 255) / 256 * 39,
+                              (tiles(256, 256) + 255) / 256 * 62};
+    switch (std::min_element(cost, cost + 4) - cost) {
+        case 0: return launch<2, 4, 64, 2, false>(a, s);
+        case 1: return launch<4, 8, 128, 2, false>(a, s);
+        case 2: return launch<4, 8, 256, 1, false>(a, s);
+        default: return launch<8, 8, 256, 1, false>(a, s);
+    }
 }
 
 }  // namespace tsp

@@ -1,4 +1,5 @@
-// Internal interface of the dense Q4_K GEMM over raw GGUF rows (dense_tile.hip), any number of activation rows.
+// Internal interface of the dense Q4_K GEMM over raw GGUF rows (dense_tile.hip), any number of activation rows whose halves stay
+// under 4 GiB.
 #pragma once
 #include "tsp_common.hpp"
 

@@ -663,7 +663,8 @@ extern "C" int tsp_dense_mm(uint32_t encoding, uint32_t layout, const void* matr
     auto* sx = reinterpret_cast<_Float16*>(static_cast<uint8_t*>(workspace) + align256(uint64_t(tokens) * columns * 2));
     int rc = convert_rows(input, input_stride_bytes, input_is_bf16, xh, encoding == 12 ? sx : nullptr, tokens, columns, error_word, s);  // with the sums come the swapped columns
     if (rc != TSP_OK) return rc;
-    if (layout == TSP_LAYOUT_GGUF) {
+    // Tiles over raw rows address the activations with 32-bit offsets; halves of 4 GiB and more take the task kernel's 64-bit row addresses.
+    if (layout == TSP_LAYOUT_GGUF && uint64_t(tokens) * columns * 2 < (1ull << 32)) {
         DenseTileArgs t{};
         t.a = xh; t.a_stride = columns; t.sx = sx; t.w = static_cast<const uint8_t*>(matrix); t.m = tokens; t.n = rows; t.k = columns;
         t.out = output; t.out_stride = output_stride_bytes; t.out_bf16 = output_is_bf16; t.error_word = error_word;
@@ -675,8 +676,10 @@ extern "C" int tsp_dense_mm(uint32_t encoding, uint32_t layout, const void* matr
     const uint32_t col_tiles = (rows + 255) / 256, tasks = (tokens + kTaskRows - 1) / kTaskRows;
     if (encoding == 14) return output_is_bf16 ? launch<B_Q6K_PLANAR, EPI_BF16, ROWS_DENSE>(a, col_tiles, tasks, s)
                                                : launch<B_Q6K_PLANAR, EPI_F32, ROWS_DENSE>(a, col_tiles, tasks, s);
-    return output_is_bf16 ? launch<B_Q4K_PLANAR, EPI_BF16, ROWS_DENSE>(a, col_tiles, tasks, s)
-                          : launch<B_Q4K_PLANAR, EPI_F32, ROWS_DENSE>(a, col_tiles, tasks, s);
+    if (layout == TSP_LAYOUT_PLANAR_V3) return output_is_bf16 ? launch<B_Q4K_PLANAR, EPI_BF16, ROWS_DENSE>(a, col_tiles, tasks, s)
+                                                               : launch<B_Q4K_PLANAR, EPI_F32, ROWS_DENSE>(a, col_tiles, tasks, s);
+    return output_is_bf16 ? launch<B_Q4K_RAW, EPI_BF16, ROWS_DENSE>(a, col_tiles, tasks, s)
+                          : launch<B_Q4K_RAW, EPI_F32, ROWS_DENSE>(a, col_tiles, tasks, s);
 }
 
 // ---------------------------------------------------------------- grouped GEMM over raw GGUF expert stacks
