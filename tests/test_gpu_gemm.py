@@ -670,6 +670,13 @@ def test_grouped_moe_other_planar_kinds(gpu, tsp, orc, synth, gu_type, dn_type, 
     assert np.array_equal(y.view(np.uint32), again.view(np.uint32))
 
 
+# the down kernel that keeps a task's h rows in LDS: one to six steps of 128 hidden units (six take the requests in two halves), one
+# and three groups of 256 channels, tasks of one and of two row tiles
+@pytest.mark.parametrize("dn_type,channels,hidden", [(8, 256, 128), (7, 768, 128), (7, 256, 384), (8, 768, 384), (8, 256, 768), (7, 768, 768)])
+def test_grouped_moe_down_rows_in_lds(gpu, tsp, orc, synth, dn_type, channels, hidden):
+    test_grouped_moe_other_planar_kinds(gpu, tsp, orc, synth, 12, dn_type, channels, hidden)
+
+
 def test_grouped_moe_sticky_errors(gpu, tsp, synth):
     channels, hidden, experts, selected, n = 256, 256, 4, 2, 40
     gate = synth.matrix(12, 3101, hidden * experts, channels)

@@ -266,10 +266,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                 quarter(std::integral_constant<int, 1>{}, std::integral_constant<int, 2>{});
                 quarter(std::integral_constant<int, 1>{}, std::integral_constant<int, 3>{});
             } else if constexpr (KIND == kQ51) {
-                // Q5_1: element e of a block is nibble e % 16 (low for e < 16, high above) of byte e % 16 with bit e of the
-                // block's fifth-bit word on top; the lane's k-half takes elements 16 khalf .. 16 khalf + 15. A weight is the
-                // half nearest to d * q + m: q exact as a half, one packed fused multiply-add, one rounding (the f32
-                // evaluation rounds the sum to f32 first, which can move the half only when that sum sits on a tie).
                 u32x4 q[8];
 #pragma unroll
                 for (int b = 0; b < 8; ++b) q[b] = *reinterpret_cast<const u32x4*>(st + n * 128 + ((b ^ (n & 7)) * 16));
@@ -285,24 +281,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                 for (int b = 0; b < 8; ++b) {
                     const uint32_t pair = dm[b / 4][b % 4];  // d in the low half, m in the high half
                     const f16x2 d2 = as_h2(__builtin_amdgcn_perm(pair, pair, 0x05040504u)), m2 = as_h2(__builtin_amdgcn_perm(pair, pair, 0x07060706u));
-                    const uint32_t bits = fifth[b / 4][b % 4] >> (16 * khalf);
-                    const f16x2 off = splat(-1024.0f);
                     f16x8 f[2];
-#pragma unroll
-                    for (int ff = 0; ff < 2; ++ff) {
-                        f16x2 p[4];
-#pragma unroll
-                        for (int j = 0; j < 2; ++j) {
-                            const int w = 2 * ff + j;  // bytes 4 w .. 4 w + 3 of the block: elements 16 khalf + 4 w .. + 3
-                            const uint32_t nibbles = (q[b][w] >> (4 * khalf)) & 0x0f0f0f0fu;
-                            // bits 4 w .. 4 w + 3 of the fifth-bit half-word to bit 0 of four bytes: no two partial products share a bit
-                            const uint32_t four = ((bits >> (4 * w)) & 15u) * 0x00204081u & 0x01010101u;
-                            const uint32_t codes = nibbles | (four << 4);
-                            p[2 * j] = fma2(as_h2(spread01(codes, 0x64646464u)) + off, d2, m2);
-                            p[2 * j + 1] = fma2(as_h2(spread23(codes, 0x64646464u)) + off, d2, m2);
-                        }
-                        f[ff] = f16x8{p[0][0], p[0][1], p[1][0], p[1][1], p[2][0], p[2][1], p[3][0], p[3][1]};
-                    }
+                    q51_frags(q[b], fifth[b / 4][b % 4] >> (16 * khalf), d2, m2, khalf, f);
 #pragma unroll
                     for (int ff = 0; ff < 2; ++ff)
 #pragma unroll

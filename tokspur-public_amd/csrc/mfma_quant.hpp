@@ -39,6 +39,17 @@ __device__ __forceinline__ uint32_t lds_address(const void* p) {
 }
 __device__ __forceinline__ void wait_all_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
+// An address that came through LDS says so itself: the compiler would take the generic path, which counts every load among the
+// LDS accesses as well and drains all of them at each wait.
+typedef const uint8_t __attribute__((address_space(1)))* GlobalBytes;
+template <class V> __device__ __forceinline__ V global_at(GlobalBytes base, uint32_t offset) {
+    asm volatile("" : "+v"(offset));  // a scalar base and a lane offset, not a 64-bit address per lane
+    return *reinterpret_cast<const V __attribute__((address_space(1)))*>(base + offset);
+}
+__device__ __forceinline__ GlobalBytes uniform_address(uint32_t lo, uint32_t hi) {
+    return reinterpret_cast<GlobalBytes>(uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(hi))) << 32 | uint32_t(__builtin_amdgcn_readfirstlane(lo)));
+}
+
 __device__ __forceinline__ f16x2 as_h2(uint32_t bits) { return __builtin_bit_cast(f16x2, bits); }
 __device__ __forceinline__ uint32_t as_u32(f16x2 v) { return __builtin_bit_cast(uint32_t, v); }
 __device__ __forceinline__ f16x2 splat(float v) { const _Float16 h = _Float16(v); return f16x2{h, h}; }
@@ -65,6 +76,29 @@ __device__ __forceinline__ f16x8 quants8(uint32_t w0, uint32_t w1) {
     const f16x2 p0 = as_h2(spread01(u0, K)) + off, p1 = as_h2(spread23(u0, K)) + off;
     const f16x2 p2 = as_h2(spread01(u1, K)) + off, p3 = as_h2(spread23(u1, K)) + off;
     return f16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
+}
+
+// Sixteen weights of a Q5_1 block as two fragments. Element e is nibble e % 16 (low for e < 16, high above) of byte e % 16 with bit e
+// of the block's fifth-bit word on top; the lane's k-half takes elements 16 khalf .. 16 khalf + 15. A weight is the half nearest to
+// d * q + m (bits: the k-half's sixteen fifth bits): q exact as a half, one packed fused multiply-add, one rounding (the f32 evaluation rounds the sum to f32 first,
+// which can move the half only when that sum sits on a tie).
+__device__ __forceinline__ void q51_frags(const u32x4& nibble_bytes, uint32_t bits, f16x2 d2, f16x2 m2, uint32_t khalf, f16x8 frag[2]) {
+    const f16x2 off = splat(-1024.0f);
+#pragma unroll
+    for (int ff = 0; ff < 2; ++ff) {
+        f16x2 p[4];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int w = 2 * ff + j;  // bytes 4 w .. 4 w + 3 of the block: elements 16 khalf + 4 w .. + 3
+            const uint32_t nibbles = (nibble_bytes[w] >> (4 * khalf)) & 0x0f0f0f0fu;
+            // bits 4 w .. 4 w + 3 of the fifth-bit half-word to bit 0 of four bytes: no two partial products share a bit
+            const uint32_t four = ((bits >> (4 * w)) & 15u) * 0x00204081u & 0x01010101u;
+            const uint32_t codes = nibbles | (four << 4);
+            p[2 * j] = fma2(as_h2(spread01(codes, 0x64646464u)) + off, d2, m2);
+            p[2 * j + 1] = fma2(as_h2(spread23(codes, 0x64646464u)) + off, d2, m2);
+        }
+        frag[ff] = f16x8{p[0][0], p[0][1], p[1][0], p[1][1], p[2][0], p[2][1], p[3][0], p[3][1]};
+    }
 }
 
 // ---------------------------------------------------------------- Q4_K operands

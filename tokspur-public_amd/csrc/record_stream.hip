@@ -50,17 +50,6 @@ constexpr uint32_t kPartialBytes = 20480;
 static_assert(kUnionScratchWords * 4 <= kPartialBytes, "the union build borrows the partial results' space");
 typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));  // 16 bytes at any even address
 
-// An address that came through LDS says so itself: the compiler would take the generic path, which counts every load among the
-// LDS accesses as well and drains all of them at each wait.
-typedef const uint8_t __attribute__((address_space(1)))* GlobalBytes;
-template <class V> __device__ __forceinline__ V global_at(GlobalBytes base, uint32_t offset) {
-    asm volatile("" : "+v"(offset));  // a scalar base and a lane offset, not a 64-bit address per lane
-    return *reinterpret_cast<const V __attribute__((address_space(1)))*>(base + offset);
-}
-__device__ __forceinline__ GlobalBytes uniform_address(uint32_t lo, uint32_t hi) {
-    return reinterpret_cast<GlobalBytes>(uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(hi))) << 32 | uint32_t(__builtin_amdgcn_readfirstlane(lo)));
-}
-
 enum Kind : int { K_Q4K = 0, K_Q6K = 1, K_Q8 = 2, K_Q51 = 3 };
 
 template <int KIND> struct Traits;
