@@ -21,7 +21,7 @@
 //     parked in wave-private swizzled LDS and read back in MFMA B-fragment order (lane = (row % 32, k-half)); every
 //     weight is unpacked once per task.
 //   * Activations are shared by the four waves: 64 rows x 128 bytes per K step go global -> LDS directly (no registers),
-//     two and three steps ahead, into a ring of four slabs; one LDS-only barrier per K step.
+//     two and three steps ahead, into a ring of four slabs; one LDS-only barrier per two K steps.
 //   * For gate/up the two column tiles of a wave are the gate rows and the up rows of the same 32 hidden
 //     units, so SwiGLU is an element-wise epilogue on accumulator registers.
 #include "dense_tile.hpp"
@@ -314,10 +314,12 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {  // two work
                 constexpr int wbuf = H / 2, ring = H;  // step % RING
                 const uint32_t b = step / 4;
                 // Even steps request the slabs of the steps two and three ahead, as the first loads after their barrier; the
-                // only loads younger than those are the section (6) and, at H == 2, scale (4) loads of the same step, and
-                // for an odd step the two slabs and the loads of the even step before it. Loads complete in order.
+                // only loads younger than those are the section (6) and, at H == 2, scale (4) loads of the same step. Loads complete in
+                // order. One barrier per two steps: the slabs were requested as a pair, and an odd step finds its own already there (its
+                // wait, which also counts the slabs and loads of the even step before it, passes at once).
                 constexpr int W[4] = {6, 0, 10, 0};
-                lds_barrier_after_loads<H % 2 == 0 ? W[(H + 2) % 4] : W[(H + 1) % 4] + 2 * MT + W[(H + 3) % 4]>();  // slab and this wave's section bytes are complete; every wave has left the other buffers
+                if constexpr (H % 2 == 0) lds_barrier_after_loads<W[(H + 2) % 4]>();  // this step's slab, the next one's and this wave's section bytes are complete; every wave has left the other buffers
+                else wait_after_loads<W[(H + 1) % 4] + 2 * MT + W[(H + 3) % 4]>();
                 if (H % 2 == 0) { dma_a(step + 2, (ring + 2) % RING); dma_a(step + 3, (ring + 3) % RING); }
                 if (H % 2 == 0) fetch_w(step / 2 + 1);
                 if (H == 2) { scl_next[0] = load_scales(b + 1, 0); scl_next[1] = load_scales(b + 1, 1); }
@@ -354,8 +356,8 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {  // two work
                 half_step(b * 4 + 3, std::integral_constant<int, 3>{});
             }
         } else {
-            // Q4_K. Quant bytes travel global -> registers -> LDS -> fragment registers, half a super-block (two K steps)
-            // ahead. The global loads are issued row-wise (one instruction = sixteen rows x 64 contiguous bytes, lane = 16-byte
+            // Q4_K. Quant bytes travel global -> registers -> LDS -> fragment registers, half a super-block at a time, four K
+            // steps ahead. The global loads are issued row-wise (one instruction = sixteen rows x 64 contiguous bytes, lane = 16-byte
             // chunk), so cache lines are requested in whole halves by neighbouring lanes. In LDS lane (row, k-half) then picks
             // its 16 bytes of the step. Headers (scales, minima, d, dmin: 16 + 4 bytes per lane) go straight to registers.
             //
@@ -370,40 +372,41 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {  // two work
             const uint32_t wave_row0 = EPI == EPI_SWIGLU ? bx * 128 + wave * 32 : bx * 256 + wave * 64;
             const uint32_t row_bytes = bpr * BLK;
             const uint32_t halves = 2 * bpr;
-            u32x4 wstage[4];
+            u32x4 wstage[2][4];  // odd halves, even halves
             // instruction Q of a half-block: rows 16Q .. 16Q+15 of the wave's 64 (tile Q / 2)
-            auto fetch_w = [&](uint32_t half, auto q_tag) {
+            auto fetch_w = [&](u32x4 (&into)[4], uint32_t half, auto q_tag) {
                 constexpr int Q = decltype(q_tag)::value, J = Q / 2;
                 uint32_t row = wave_row0 + (EPI == EPI_SWIGLU ? (Q % 2) * 16 : Q * 16) + ld_row;
                 row = row < a.n ? row : a.n - 1;
                 // uniform base + 32-bit lane offset (the host refuses matrices whose rows span 4 GiB or more)
                 const uint8_t* base = wbase[J] + (BKIND == B_Q4K_PLANAR ? a.spec.qs_offset : 0) + uint64_t(half / 2) * BLK + QS_AT + (half % 2) * 64;
-                wstage[Q] = *reinterpret_cast<const u32x4*>(base + (row * row_bytes + ld_chunk * 16));
+                into[Q] = *reinterpret_cast<const u32x4*>(base + (row * row_bytes + ld_chunk * 16));
             };
-            auto fetch_w_all = [&](uint32_t half) {
+            auto fetch_w_all = [&](u32x4 (&into)[4], uint32_t half) {
                 half = half < halves ? half : halves - 1;
-                fetch_w(half, std::integral_constant<int, 0>{});
-                fetch_w(half, std::integral_constant<int, 1>{});
-                fetch_w(half, std::integral_constant<int, 2>{});
-                fetch_w(half, std::integral_constant<int, 3>{});
+                fetch_w(into, half, std::integral_constant<int, 0>{});
+                fetch_w(into, half, std::integral_constant<int, 1>{});
+                fetch_w(into, half, std::integral_constant<int, 2>{});
+                fetch_w(into, half, std::integral_constant<int, 3>{});
             };
-            auto store_w = [&](int wbuf) {
+            auto store_w = [&](int wbuf, const u32x4 (&from)[4]) {
     #pragma unroll
-                for (int q = 0; q < 4; ++q) *reinterpret_cast<u32x4*>(my_w + wbuf * 4096 + (q * 64 + lane) * 16) = wstage[q];
+                for (int q = 0; q < 4; ++q) *reinterpret_cast<u32x4*>(my_w + wbuf * 4096 + (q * 64 + lane) * 16) = from[q];
             };
             auto read_w = [&](int wbuf, int j, int p2) {  // row j*32 + col, chunk 2*p2 + khalf
                 return *reinterpret_cast<const u32x4*>(my_w + wbuf * 4096 + ((j * 32 + col) * 4 + ((2 * p2 + khalf) ^ ((col >> 1) & 3))) * 16);
             };
             const Q4Consts q4c = q4_consts();
+            const Q4ScaleConsts q4s = q4_scale_consts();
             HdrQ4 hdr[2];
-            RawHdrQ4 hdr_next[2];  // requested at P == 2, decoded at the end of P == 3: nothing touches the bytes while they travel
+            RawHdrQ4 hdr_next[2];  // requested at P == 0, decoded at the end of P == 3: nothing touches the bytes while they travel
     #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 hdr_next[j] = fetch_hdr_q4k<BKIND>(wbase[j], a.spec, wrow[j], bpr, 0);
                 hdr[j] = decode_hdr_q4k<BKIND>(hdr_next[j]);
             }
-            fetch_w_all(0);
-            store_w(0);
+            fetch_w_all(wstage[1], 0);
+            store_w(0, wstage[1]);
             fetch_sx(0);
             store_sx(0);
             auto pair_step = [&](uint32_t step, auto p_tag) {
@@ -411,26 +414,31 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {  // two work
                 constexpr int wbuf = P / 2, ring = P;  // step % RING
                 const uint32_t b = step / 4;
                 // Even steps request the slabs of the steps two and three ahead, as the first loads after their barrier; the
-                // only loads younger than those are the other loads of the same step (W), and for an odd step the two slabs
-                // and the loads of the even step before it. Loads complete in order.
-                // sums + half-block, -, half-block + headers (planes: scales and d/dmin apart, two loads per tile; GGUF rows: one), -
-                constexpr int W[4] = {5, 0, BKIND == B_Q4K_PLANAR ? 8 : 6, 0};
-                lds_barrier_after_loads<P % 2 == 0 ? W[(P + 2) % 4] : W[(P + 1) % 4] + 2 * MT + W[(P + 3) % 4]>();  // slab, this wave's weight bytes (and at P == 3 lds_sx[b & 1]) are complete; every wave has left the other buffers
+                // only loads younger than those are the other loads of the same step (W). Loads complete in order. One barrier per two
+                // steps: the slabs were requested as a pair, and an odd step finds its own already there (its wait, which also counts
+                // the slabs and loads of the even step before it, passes at once).
+                // sums + headers (planes: scales and d/dmin apart, two loads per tile; GGUF rows: one) + half-block, -, half-block, -.
+                // The half-blocks come last and are parked only in the second step after the one that requested them, behind younger
+                // slabs: loads return in order, and whatever is waited for sooner would bring them along.
+                constexpr int W[4] = {BKIND == B_Q4K_PLANAR ? 9 : 7, 0, 4, 0};
+                if constexpr (P % 2 == 0) lds_barrier_after_loads<W[(P + 2) % 4]>();  // this step's slab, the next one's, this wave's weight bytes and lds_sx[b & 1] are complete; every wave has left the other buffers
+                else wait_after_loads<W[(P + 1) % 4] + 2 * MT + W[(P + 3) % 4]>();
                 if (P % 2 == 0) { dma_a(step + 2, (ring + 2) % RING); dma_a(step + 3, (ring + 3) % RING); }
                 if (P == 0) fetch_sx(b + 1 < bpr ? b + 1 : b);
-                if (P == 0 || P == 2) fetch_w_all(step / 2 + 1);
-                if (P == 2) {
+                if (P == 0) {
     #pragma unroll
                     for (int j = 0; j < 2; ++j) hdr_next[j] = fetch_hdr_q4k<BKIND>(wbase[j], a.spec, wrow[j], bpr, b + 1 < bpr ? b + 1 : b);
                 }
+                if (P == 0 || P == 2) { __builtin_amdgcn_sched_barrier(0); fetch_w_all(wstage[P == 0 ? 1 : 0], step / 2 + 2); }
                 const u32x4 raw0 = read_w(wbuf, 0, P & 1), raw1 = read_w(wbuf, 1, P & 1);
+                const Q4PairScale sc0 = q4_pair_scale<P>(hdr[0].sc[0], hdr[0].sc[1], q4s), sc1 = q4_pair_scale<P>(hdr[1].sc[0], hdr[1].sc[1], q4s);
                 f16x8 f0[2], f1[2];
-                frags_q4k_swapped<P, 0>(raw0, hdr[0], q4c, f0);
-                frags_q4k_swapped<P, 0>(raw1, hdr[1], q4c, f1);
+                frags_q4k_pair(raw0, sc0, 0, q4c, f0);
+                frags_q4k_pair(raw1, sc1, 0, q4c, f1);
                 mfma(ring, 0, f0[0], f1[0], P == 0);
                 mfma(ring, 1, f0[1], f1[1], false);
-                frags_q4k_swapped<P, 1>(raw0, hdr[0], q4c, f0);
-                frags_q4k_swapped<P, 1>(raw1, hdr[1], q4c, f1);
+                frags_q4k_pair(raw0, sc0, 1, q4c, f0);
+                frags_q4k_pair(raw1, sc1, 1, q4c, f1);
                 mfma(ring, 2, f0[0], f1[0], false);
                 mfma(ring, 3, f0[1], f1[1], false);
                 if (P == 3) {
@@ -446,11 +454,12 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {  // two work
                     }
                     fold(-hdr[0].dmin, -hdr[1].dmin);
                 }
-                if (P == 1) store_sx((b + 1) & 1);  // read at P == 3 of the next super-block; the buffer was last read at P == 3 of the one before
-                if (P == 1 || P == 3) store_w(wbuf ^ 1);  // read again two barriers from now; this buffer was last read a step ago
+                if (P == 3) store_sx((b + 1) & 1);  // read at P == 3 of the next super-block; the buffer was last read at P == 3 of the one before
+                if (P == 1 || P == 3) store_w(wbuf ^ 1, wstage[P == 1 ? 0 : 1]);  // read again two barriers from now; this buffer was last read a step ago
                 if (P == 3) { hdr[0] = decode_hdr_q4k<BKIND>(hdr_next[0]); hdr[1] = decode_hdr_q4k<BKIND>(hdr_next[1]); }
             };
             wait_all_loads();  // slabs 0 and 1 (the stores above already waited for younger loads)
+            fetch_w_all(wstage[0], 1);
             for (uint32_t b = 0; b < bpr; ++b) {
                 pair_step(b * 4 + 0, std::integral_constant<int, 0>{});
                 pair_step(b * 4 + 1, std::integral_constant<int, 1>{});

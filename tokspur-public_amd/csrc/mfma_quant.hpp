@@ -24,6 +24,12 @@ __device__ __forceinline__ void lds_barrier_after_loads() {
     static_assert(YOUNGEST >= 0 && YOUNGEST < 64, "vmcnt is a 6-bit counter");
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(YOUNGEST) : "memory");
 }
+// The wait alone, for this wave.
+template <int YOUNGEST>
+__device__ __forceinline__ void wait_after_loads() {
+    static_assert(YOUNGEST >= 0 && YOUNGEST < 64, "vmcnt is a 6-bit counter");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(YOUNGEST) : "memory");
+}
 // 16 bytes per lane from global memory straight into LDS at lds_base + 16 * lane (lds_base uniform over the wave).
 // The compiler does not know this load: it counts in vmcnt like any other, so waits the compiler places for its own
 // loads are only ever longer than needed, and whoever reads the bytes waits for them with lds_barrier_after_loads.
@@ -178,18 +184,10 @@ __device__ __forceinline__ f16x8 scaled8_q4_swapped(uint32_t w0, uint32_t w1, f1
     const f16x2 p2 = fma2(as_h2((w1 & m) | c.bits), sc, bias), p3 = fma2(as_h2(((w1 >> 8) & m) | c.bits), sc, bias);
     return f16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
 }
-template <int P, int HI>
-__device__ __forceinline__ void frags_q4k_swapped(const u32x4& raw, const HdrQ4& h, const Q4Consts& c, f16x8 frag[2]) {
-    const uint32_t sc = (h.sc[P >> 1] >> ((P & 1) * 16 + HI * 8)) & 0xffu;
-    const f16x2 s2 = splat(float(sc) * (HI ? 0.0625f : 1.0f)), bias = splat(float(sc) * (HI ? -64.0f : -1024.0f));
-    frag[0] = scaled8_q4_swapped<HI>(raw[0], raw[1], s2, bias, c);
-    frag[1] = scaled8_q4_swapped<HI>(raw[2], raw[3], s2, bias, c);
-}
-
-// The same unpacking with the scale set-up shared by a pair of sub-blocks: the six-bit scales of sub-blocks 2P and 2P + 1 sit
+// The scale set-up is shared by a pair of sub-blocks: the six-bit scales of sub-blocks 2P and 2P + 1 sit
 // in neighbouring bytes of the header; one byte permute puts them under 0x64 (1024 + sc as halves, side by side), one packed
 // add takes the 1024 off, and two packed multiplies make (sc, sc / 16) and (-1024 sc, -64 sc): the factors and the
-// offsets of the low-nibble and the high-nibble products. Four instructions per pair instead of ten per sub-block.
+// offsets of the low-nibble and the high-nibble products. Four instructions per pair.
 struct Q4ScaleConsts { uint32_t sel[2]; uint32_t k64; f16x2 off, mul, bias; };
 __device__ __forceinline__ Q4ScaleConsts q4_scale_consts() {
     // selector bytes: 0..3 pick a byte of the header word, 4..7 a byte of the constant 0x64646464
