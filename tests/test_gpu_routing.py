@@ -441,3 +441,19 @@ def test_router_f32_batch_sliced(gpu, synth, tokens, columns, experts):
     want = x.astype(np.float64) @ w.astype(np.float64).T
     scale = np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T
     assert (np.abs(got - want) <= 2e-6 * scale).all() and gpu.error() == 0
+
+
+@pytest.mark.parametrize("tokens,columns,experts", [(1, 2048, 512), (2, 2080, 65), (3, 32, 5), (4, 2304, 64), (5, 2592, 333), (8, 96, 1024), (7, 6144, 128)])
+def test_router_f32_batch_pairs(gpu, synth, tokens, columns, experts):
+    """Up to eight tokens: two experts per workgroup (an odd one left over), each number of token rows the kernel is built for and less,
+    columns from less than one wave's piece to several pieces per wave. f32 sums, as for the sliced form."""
+    w = synth.activations_f32(synth.tensor_seed(5, 200 + tokens), (experts, columns))
+    x = synth.activations_f32(synth.tensor_seed(6, 200 + tokens), (tokens, columns))
+    pitch = (experts + 3) // 4 * 4
+    out = gpu.full((tokens + 1, pitch), 7.25)
+    gpu.router_f32_batch(gpu.upload(w), gpu.upload(x), tokens, columns, experts, out=out, out_stride=pitch * 4)
+    got = out.cpu().numpy()
+    want = x.astype(np.float64) @ w.astype(np.float64).T
+    scale = np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T
+    assert (np.abs(got[:tokens, :experts] - want) <= 2e-6 * scale).all() and gpu.error() == 0
+    assert (got[tokens] == 7.25).all() and (got[:, experts:] == 7.25).all()

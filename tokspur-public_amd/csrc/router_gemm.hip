@@ -133,7 +133,7 @@ __global__ __launch_bounds__(512) void router_f32_gemm(RouterArgs a) {
 // row l % 16 of either operand, one column per instruction, so no LDS round trip stands between a wave's requests and its
 // products and all a wave needs is in flight a batch of kUnits steps ahead. Bound by the latency of one trip to memory and the matrix
 // rate of f32 (4 x 32 cycles per 16 columns and tile pair) at eight waves per tile. 512 experts x
-// 2048 columns: 8 tokens 41.8 -> 7.6 us, 203 tokens 42.6 -> 12.8, 400 tokens 42.9 -> 17.2.
+// 2048 columns: 203 tokens 42.6 -> 12.8, 400 tokens 42.9 -> 17.2.
 constexpr uint32_t kSlices = 8;
 typedef float acc4 __attribute__((ext_vector_type(4)));
 
@@ -195,6 +195,64 @@ __global__ __launch_bounds__(512) void router_f32_sliced(RouterArgs a) {
     publish_error(bad, a.error_word);
 }
 
+// A draft's tokens: sixteen rows of tokens would be half empty, and 32 tiles of sixteen experts leave most of the chip idle. A workgroup
+// owns two experts, its eight waves every eighth piece of 256 columns, a lane four columns of every token and both experts: at
+// 2048 columns one trip to memory, all of it requested at once. Bound by that trip and the launch. 512 experts, 8 tokens: 2048 columns
+// 10.1 -> 4.3 us, 2560 columns 11.8 -> 5.8 (5 tokens).
+template <uint32_t TOKENS>
+__global__ __launch_bounds__(512) void router_f32_pairs(RouterArgs a) {
+    constexpr uint32_t E = 2, kPiece = 64, kStep = kSlices * kPiece;
+    __shared__ float sums[kSlices][E * TOKENS];
+    const uint32_t tid = threadIdx.x, lane = tid % 64, wave = tid / 64, expert0 = blockIdx.x * E, quads = a.columns / 4;
+    const acc4* w[E];
+    const acc4* x[TOKENS];
+#pragma unroll
+    for (uint32_t e = 0; e < E; ++e) w[e] = reinterpret_cast<const acc4*>(a.weights + uint64_t(min(expert0 + e, a.experts - 1)) * a.columns);
+#pragma unroll
+    for (uint32_t t = 0; t < TOKENS; ++t) x[t] = reinterpret_cast<const acc4*>(a.input + uint64_t(min(t, a.tokens - 1)) * a.input_stride);
+    acc4 acc[E][TOKENS] = {};
+    for (uint32_t q0 = wave * kPiece; q0 < quads; q0 += kStep) {
+        const uint32_t q = min(q0 + lane, quads - 1);  // past the end: the last piece again, not multiplied
+        acc4 fw[E], fx[TOKENS];
+#pragma unroll
+        for (uint32_t e = 0; e < E; ++e) fw[e] = w[e][q];
+#pragma unroll
+        for (uint32_t t = 0; t < TOKENS; ++t) fx[t] = x[t][q];
+        if (q0 + lane < quads)
+#pragma unroll
+            for (uint32_t t = 0; t < TOKENS; ++t)
+#pragma unroll
+                for (uint32_t e = 0; e < E; ++e)
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) acc[e][t][c] = __builtin_fmaf(fw[e][c], fx[t][c], acc[e][t][c]);
+    }
+#pragma unroll
+    for (uint32_t e = 0; e < E; ++e)
+#pragma unroll
+        for (uint32_t t = 0; t < TOKENS; ++t) {
+            const float sum = wave_sum((acc[e][t][0] + acc[e][t][1]) + (acc[e][t][2] + acc[e][t][3]));
+            if (lane == 0) sums[wave][e * TOKENS + t] = sum;
+        }
+    __syncthreads();
+    uint32_t bad = 0;
+    if (tid < E * TOKENS) {
+        float value = sums[0][tid];
+#pragma unroll
+        for (uint32_t s = 1; s < kSlices; ++s) value += sums[s][tid];
+        const uint32_t token = tid % TOKENS, expert = expert0 + tid / TOKENS;
+        if (token < a.tokens && expert < a.experts) {
+            bad |= nonfinite(value) ? TSP_ERRBIT_NONFINITE : 0u;
+            a.output[uint64_t(token) * a.output_stride + expert] = value;
+        }
+    }
+    publish_error(bad, a.error_word);
+}
+
+template <uint32_t TOKENS>
+void launch_pairs(const RouterArgs& a, hipStream_t s) {
+    TSP_LAUNCH("router_f32_gemm", s, router_f32_pairs<TOKENS><<<(a.experts + 1) / 2, 512, 0, s>>>(a));
+}
+
 template <int ET, int TT>
 void launch_sliced(RouterArgs a, hipStream_t s) {
     a.expert_tiles = (a.experts + ET * 16 - 1) / (ET * 16);
@@ -241,7 +299,9 @@ extern "C" int tsp_router_f32_batch(const float* weights, const float* input, ui
     // that holds: 16 x 16 (9 us a round at 2048 columns), 16 experts x 32 tokens (13 us), 32 x 32 (17 us); two rounds of the
     // largest (35 us, 1024 tokens of 512 experts) still beat the 43 us that the 64 x 64 form takes up to a full round of its own.
     const auto tiles = [&](uint32_t e, uint32_t t) { return uint64_t((experts + e - 1) / e) * ((tokens + t - 1) / t); };
-    if (tiles(16, 16) <= 256) launch_sliced<1, 1>(a, s);
+    // Up to eight tokens: two experts per workgroup, while the chip takes them in two rounds.
+    if (tokens <= 8 && experts <= 1024) tokens <= 2 ? launch_pairs<2>(a, s) : tokens <= 4 ? launch_pairs<4>(a, s) : launch_pairs<8>(a, s);
+    else if (tiles(16, 16) <= 256) launch_sliced<1, 1>(a, s);
     else if (tiles(16, 32) <= 256) launch_sliced<1, 2>(a, s);
     else if (tiles(32, 32) <= 512) launch_sliced<2, 2>(a, s);
     else TSP_LAUNCH("router_f32_gemm", s, router_f32_gemm<<<a.tiles_per_xcd * 8, 512, kLdsBytes, s>>>(a));
