@@ -35,6 +35,18 @@ def test_topk_ties_zeros_nonfinite(gpu, tsp, orc, vocab):
     check_rows(tsp, orc, gpu, x, stride_floats=vocab + 3)
 
 
+# rows without ties, so that both stages bound and rank (but for the third row, whose large values lie in 63 of a tile's 128 sampled groups): around a tile's smallest sampled widths, a narrow last tile, and more partial rows
+# than stage 2 holds in registers (64) and samples (128)
+@pytest.mark.parametrize("vocab", [255, 256, 511, 512, 600, 4096 + 384, 300000, 700000])
+def test_topk_bound_and_rank(gpu, tsp, orc, vocab):
+    x = np.random.default_rng(vocab).normal(size=(3, vocab)).astype(np.float32)
+    x[2, np.arange(vocab) % 1024 < 500] += 20
+    x[1] = -np.abs(x[1])
+    x[1, vocab // 2] = -0.0
+    x[0, [vocab // 3, vocab - 1]] = [np.nan, np.float32(1e-41)]
+    check_rows(tsp, orc, gpu, x, stride_floats=vocab + 1)
+
+
 def test_topk_mostly_nonfinite(gpu, tsp, orc):
     x = np.full((2, 300), np.nan, dtype=np.float32)
     x[0, [5, 17, 299]] = [1.0, -2.0, 1.0]

@@ -2,15 +2,19 @@
 // (value descending, column ascending, -0 == +0), the number found, and the first non-finite and first
 // subnormal column. Rank 0 is the arg-max a greedy sampler needs.
 //
-// Two launches. Stage 1: one workgroup per (4096-column tile, row); each of its sixteen waves keeps the 64 largest keys
-// of its 256 columns in registers, one key per lane, and the sixteen lists are merged pairwise (a tree through LDS) into
-// a partial row. Stage 2: one workgroup per row merges the partial rows' lists the same way and writes the final row. A
-// sort or merge is a chain of dependent cross-lane exchanges, so what shortens it is more waves with shorter chains. Keys are 64 bits: high word
-// = the float mapped to an unsigned integer of the same order (after -0 -> +0), low word = ~column, so that "largest
-// key first" is exactly the ordering above and no two keys are equal. Non-finite logits and padding get key 0, below
-// every finite value's key. A list is sorted with a bitonic network over the wave's lanes; two lists are merged by
-// sorting one of them ascending, taking the lane-wise maximum (the 64 largest of both, a bitonic sequence) and
-// running the last six steps of the network.
+// Two launches. Stage 1: one workgroup per (4096-column tile, row) writes a partial row. Stage 2: one workgroup per row finds the 64
+// largest of the partial rows. Keys are 64 bits: high word = the float mapped to an unsigned integer of the same order (after
+// -0 -> +0), low word = ~column, so that "largest key first" is exactly the ordering above and no two keys are equal. Non-finite
+// logits and padding get key 0, below every finite value's key.
+//
+// Either stage bounds and ranks: the 64th largest of a sample of 128 keys is no larger than the 64th largest key. Stage 1 samples the
+// largest of every 32 columns, stage 2 the first entries of every partial row; of keys spread at random some ninety reach the bound,
+// and every one of those finds its place by counting the larger ones. Bound by the launch and two trips to memory: 4 rows of
+// 151 936: 10.4 us for both stages, where sorting networks over all columns took 17.6 (16 rows: 25 against 44).
+// More than 512 keys at the bound (equal logits by the thousand, most of a row masked out): each of the sixteen waves keeps
+// the 64 largest of its share in registers, one key per lane, by a bitonic network over the wave's lanes, and the sixteen lists
+// are merged pairwise (a tree through LDS); two lists are merged by sorting one of them ascending, taking the lane-wise
+// maximum (the 64 largest of both, a bitonic sequence) and running the last six steps of the network.
 #include "tsp_common.hpp"
 
 using namespace tsp;
@@ -18,7 +22,7 @@ using namespace tsp;
 namespace {
 
 constexpr uint32_t kCapacity = 64, kTileSpan = 4096, kMaxTiles = 256, kNone = 0xffffffffu;
-constexpr uint32_t kWaves = 16, kThreads = kWaves * kWave, kWaveSpan = kTileSpan / kWaves;  // 256 columns per wave of stage 1
+constexpr uint32_t kWaves = 16, kThreads = kWaves * kWave;
 
 struct TopKArgs {
     const float* logits;
@@ -91,15 +95,6 @@ __device__ __forceinline__ uint64_t wave_merge(uint64_t descending, uint64_t asc
     return merge_strides<64, 32, true>(key, lane);
 }
 
-__device__ __forceinline__ uint32_t wave_min(uint32_t v) {
-#pragma unroll
-    for (int m = 1; m < kWave; m <<= 1) {
-        const uint32_t o = __shfl_xor(v, m, kWave);
-        v = o < v ? o : v;
-    }
-    return v;
-}
-
 // Merges the waves' descending lists pairwise through LDS (wave 0 ends with the workgroup's list) and writes the row.
 // Every thread of the workgroup calls it (barriers inside).
 __device__ void merge_waves_and_write(uint64_t top, uint64_t (*lists)[kCapacity], tsp_logit_topk_row* row, const float* logits_row,
@@ -130,61 +125,175 @@ __device__ void merge_waves_and_write(uint64_t top, uint64_t (*lists)[kCapacity]
     }
 }
 
-__global__ __launch_bounds__(kThreads) void topk_stage1(TopKArgs a) {
-    __shared__ uint64_t lists[kWaves][kCapacity];
-    __shared__ uint32_t first_nonfinite, first_subnormal;
-    const uint32_t tile = blockIdx.x, row = blockIdx.y, lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-    const float* logits_row = reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(a.logits) + uint64_t(row) * a.stride_bytes);
-    if (threadIdx.x == 0) { first_nonfinite = kNone; first_subnormal = kNone; }
-    __syncthreads();
-    uint32_t nonfinite = kNone, subnormal = kNone;
-    // 4 batches of 64 columns per wave, two independent running lists so that the exchanges of one hide the other's latency
-    uint64_t top[2] = {0, 0};
-#pragma unroll 1
-    for (uint32_t pair = 0; pair < kWaveSpan / (2 * kWave); ++pair) {
-        uint64_t key[2];
+constexpr uint32_t kSample = 128, kReach = 512;  // keys sampled; keys at or above the bound that are ranked
+struct Shared {
+    union {
+        uint64_t lists[kWaves][kCapacity];
+        struct {
+            uint64_t sample[kSample], reach[kReach];
+            float value[kReach];
+        };
+    };
+    uint64_t bound;
+    uint32_t reached, first_nonfinite, first_subnormal;
+};
+
+// The 64th largest of the sample, or 0 where it has fewer keys. The sample is complete and `bound` is 0 at the barrier before.
+__device__ __forceinline__ void find_bound(Shared& s) {
+    constexpr uint32_t kParts = kThreads / kSample;
+    static_assert(kParts == 8, "eight neighbouring lanes count for one key");
+    const uint32_t part = threadIdx.x % kParts;
+    const uint64_t mine = s.sample[threadIdx.x / kParts];
+    int larger = 0;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const uint32_t column = tile * kTileSpan + wave * kWaveSpan + (pair * 2 + h) * kWave + lane;
-            key[h] = 0;
-            if (column < a.vocabulary) {
-                const float v = logits_row[column];
-                const uint32_t bits = __float_as_uint(v);
-                if ((bits & 0x7f800000u) == 0x7f800000u) nonfinite = nonfinite < column ? nonfinite : column;
-                else if ((bits & 0x7f800000u) == 0 && (bits & 0x007fffffu) != 0) subnormal = subnormal < column ? subnormal : column;
-                key[h] = make_key(v, column);
-            }
+    for (uint32_t j = 0; j < kSample / kParts; ++j) larger += s.sample[j * kParts + part] > mine ? 1 : 0;
+    larger += __builtin_amdgcn_update_dpp(0, larger, 0xB1, 0xf, 0xf, true);
+    larger += __builtin_amdgcn_update_dpp(0, larger, 0x4E, 0xf, 0xf, true);
+    larger += __builtin_amdgcn_update_dpp(0, larger, 0x141, 0xf, 0xf, true);
+    if (part == 0 && larger == int(kCapacity) - 1 && mine != 0) s.bound = mine;
+}
+__device__ __forceinline__ void reach(Shared& s, uint64_t key, float value) {
+    if (key == 0 || key < s.bound) return;
+    const uint32_t at = atomicAdd(&s.reached, 1u);
+    if (at < kReach) { s.reach[at] = key; s.value[at] = value; }
+}
+// The row from the `reached` (at most kReach) keys; the places behind them hold zeros.
+__device__ __forceinline__ void rank_and_write(const Shared& s, tsp_logit_topk_row* row, uint32_t vocabulary) {
+    constexpr uint32_t kParts = 4;  // neighbouring lanes that count for one key
+    const uint32_t n = s.reached, part = threadIdx.x % kParts;
+    for (uint32_t i = threadIdx.x / kParts; i < n; i += kThreads / kParts) {
+        const uint64_t mine = s.reach[i];
+        int larger = 0;
+        for (uint32_t j0 = part; j0 < n; j0 += 8 * kParts) {  // past the end: zeros
+#pragma unroll
+            for (uint32_t j = 0; j < 8; ++j) larger += s.reach[j0 + j * kParts] > mine ? 1 : 0;
         }
-        if (pair == 0) {
-            top[0] = wave_sort<true>(key[0], lane);
-            top[1] = wave_sort<true>(key[1], lane);
-        } else {
-            const uint64_t c0 = wave_sort<false>(key[0], lane), c1 = wave_sort<false>(key[1], lane);
-            top[0] = wave_merge(top[0], c0, lane);
-            top[1] = wave_merge(top[1], c1, lane);
+        larger += __builtin_amdgcn_update_dpp(0, larger, 0xB1, 0xf, 0xf, true);
+        larger += __builtin_amdgcn_update_dpp(0, larger, 0x4E, 0xf, 0xf, true);
+        if (part == 0 && larger < int(kCapacity)) {
+            row->ids[larger] = ~uint32_t(mine);
+            row->logits[larger] = s.value[i];  // the raw value, -0 included
         }
     }
-    const uint64_t mine = wave_merge(top[0], __shfl(top[1], kWave - 1 - lane, kWave), lane);
-    nonfinite = wave_min(nonfinite);
-    subnormal = wave_min(subnormal);
-    if (lane == 0 && nonfinite != kNone) atomicMin(&first_nonfinite, nonfinite);
-    if (lane == 0 && subnormal != kNone) atomicMin(&first_subnormal, subnormal);
-    __syncthreads();
+    if (threadIdx.x < kCapacity && threadIdx.x >= n) {
+        row->ids[threadIdx.x] = 0;
+        row->logits[threadIdx.x] = -__builtin_inff();
+    }
+    if (threadIdx.x == 0) {
+        row->vocabulary = vocabulary;
+        row->count = n < kCapacity ? n : kCapacity;
+        row->first_nonfinite_col = s.first_nonfinite;
+        row->first_subnormal_col = s.first_subnormal;
+    }
+}
+
+__global__ __launch_bounds__(kThreads) void topk_stage1(TopKArgs a) {
+    __shared__ Shared s;
+    const uint32_t tile = blockIdx.x, row = blockIdx.y, lane = threadIdx.x % kWave;
+    const float* logits_row = reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(a.logits) + uint64_t(row) * a.stride_bytes);
+    tsp_logit_topk_row* const out = a.partial + uint64_t(row) * a.tiles + tile;
+    if (threadIdx.x == 0) { s.first_nonfinite = kNone; s.first_subnormal = kNone; s.bound = 0; s.reached = 0; }
     const uint32_t begin = tile * kTileSpan, width = a.vocabulary - begin < kTileSpan ? a.vocabulary - begin : kTileSpan;
-    merge_waves_and_write(mine, lists, a.partial + uint64_t(row) * a.tiles + tile, logits_row, width, first_nonfinite, first_subnormal);
+    constexpr int kBatches = kTileSpan / kThreads;
+    float value[kBatches];
+    uint64_t key[kBatches];
+    uint32_t nonfinite = kNone, subnormal = kNone;
+#pragma unroll
+    for (int b = 0; b < kBatches; ++b) {
+        const uint32_t column = begin + b * kThreads + threadIdx.x;
+        value[b] = logits_row[column < a.vocabulary ? column : a.vocabulary - 1];
+    }
+#pragma unroll
+    for (int b = 0; b < kBatches; ++b) {
+        const uint32_t column = begin + b * kThreads + threadIdx.x, bits = __float_as_uint(value[b]);
+        const bool live = column < a.vocabulary;
+        if (live && (bits & 0x7f800000u) == 0x7f800000u) nonfinite = nonfinite < column ? nonfinite : column;
+        else if (live && (bits & 0x7f800000u) == 0 && (bits & 0x007fffffu) != 0) subnormal = subnormal < column ? subnormal : column;
+        key[b] = live ? make_key(value[b], column) : 0;
+    }
+    // The largest of eight lanes' four columns each, or of four columns in a tile of fewer than 512, which leaves half of the lanes without
+    // one: a tile of 256 columns and more fills 64 of the sample, a smaller one is ranked whole.
+    uint64_t most = key[0];
+#pragma unroll
+    for (int b = 1; b < kBatches; ++b) most = key[b] > most ? key[b] : most;
+    const auto larger_of = [](uint64_t x, uint64_t y) { return x > y ? x : y; };
+    most = larger_of(most, dpp_u64<0xB1>(most));
+    most = larger_of(most, dpp_u64<0x4E>(most));
+    const uint64_t eight = larger_of(most, dpp_u64<0x141>(most));
+    static_assert(kThreads / 8 == kSample);
+    if (width < kSample * 4) {
+        if (lane % 4 == 0 && threadIdx.x < kSample * 4) s.sample[threadIdx.x / 4] = most;
+    } else if (lane % 8 == 0) {
+        s.sample[threadIdx.x / 8] = eight;
+    }
+    if (threadIdx.x < kReach) s.reach[threadIdx.x] = 0;
+    __syncthreads();
+    if (nonfinite != kNone) atomicMin(&s.first_nonfinite, nonfinite);
+    if (subnormal != kNone) atomicMin(&s.first_subnormal, subnormal);
+    find_bound(s);
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < kBatches; ++b) reach(s, key[b], value[b]);
+    __syncthreads();
+    if (s.reached <= kReach) return rank_and_write(s, out, width);
+    // two independent running lists so that the exchanges of one hide the other's latency
+    uint64_t top[2] = {wave_sort<true>(key[0], lane), wave_sort<true>(key[1], lane)};
+    static_assert(kBatches == 4);
+    top[0] = wave_merge(top[0], wave_sort<false>(key[2], lane), lane);
+    top[1] = wave_merge(top[1], wave_sort<false>(key[3], lane), lane);
+    const uint64_t mine = wave_merge(top[0], __shfl(top[1], kWave - 1 - lane, kWave), lane);
+    merge_waves_and_write(mine, s.lists, out, logits_row, width, s.first_nonfinite, s.first_subnormal);
 }
 
 __global__ __launch_bounds__(kThreads) void topk_stage2(TopKArgs a) {
-    __shared__ uint64_t lists[kWaves][kCapacity];
-    __shared__ uint32_t first_nonfinite, first_subnormal;
+    __shared__ Shared s;
     const uint32_t row = blockIdx.x, lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
     const float* logits_row = reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(a.logits) + uint64_t(row) * a.stride_bytes);
     const tsp_logit_topk_row* partial = a.partial + uint64_t(row) * a.tiles;
-    if (threadIdx.x == 0) { first_nonfinite = kNone; first_subnormal = kNone; }
+    if (threadIdx.x == 0) { s.first_nonfinite = kNone; s.first_subnormal = kNone; s.bound = 0; s.reached = 0; }
+    // a partial row is a descending list; an empty slot holds an infinity, which has key 0
+    const auto slot_key = [&](uint32_t tile, uint32_t slot, float* value) -> uint64_t {
+        const float v = partial[tile].logits[slot];
+        *value = v;
+        return make_key(v, partial[tile].ids[slot]);
+    };
+    const uint32_t entries = a.tiles * kCapacity;
+    constexpr uint32_t kHeld = 4;  // entries per thread held in registers
+    uint64_t key[kHeld];
+    float value[kHeld];
+#pragma unroll
+    for (uint32_t h = 0; h < kHeld; ++h) {
+        const uint32_t e = h * kThreads + threadIdx.x, at = e < entries ? e : entries - 1;
+        key[h] = slot_key(at / kCapacity, at % kCapacity, &value[h]);
+        if (e >= entries) key[h] = 0;
+    }
+    if (threadIdx.x < kSample) {  // the first few of every list, at least 64 in all unless there are fewer
+        const uint32_t each = a.tiles < 2 ? kCapacity : kSample / a.tiles ? kSample / a.tiles : 1;
+        const uint32_t tile = threadIdx.x / each, slot = threadIdx.x % each;
+        float unused;
+        s.sample[threadIdx.x] = tile < a.tiles ? slot_key(tile, slot, &unused) : 0;
+    }
+    if (threadIdx.x < kReach) s.reach[threadIdx.x] = 0;
+    uint32_t nonfinite = kNone, subnormal = kNone;
+    if (threadIdx.x < a.tiles) { nonfinite = partial[threadIdx.x].first_nonfinite_col; subnormal = partial[threadIdx.x].first_subnormal_col; }
+    static_assert(kMaxTiles <= kThreads);
     __syncthreads();
-    // a partial row is a descending list (empty slots have key 0); read backwards it is ascending
-    auto list_key = [&](uint32_t tile, uint32_t slot) -> uint64_t {
-        return tile < a.tiles && slot < partial[tile].count ? make_key(partial[tile].logits[slot], partial[tile].ids[slot]) : 0;
+    if (nonfinite != kNone) atomicMin(&s.first_nonfinite, nonfinite);
+    if (subnormal != kNone) atomicMin(&s.first_subnormal, subnormal);
+    find_bound(s);
+    __syncthreads();
+#pragma unroll
+    for (uint32_t h = 0; h < kHeld; ++h) reach(s, key[h], value[h]);
+    for (uint32_t e = kHeld * kThreads + threadIdx.x; e < entries; e += kThreads) {
+        float v;
+        const uint64_t k = slot_key(e / kCapacity, e % kCapacity, &v);
+        reach(s, k, v);
+    }
+    __syncthreads();
+    if (s.reached <= kReach) return rank_and_write(s, a.out + row, a.vocabulary);
+    auto list_key = [&](uint32_t tile, uint32_t slot) -> uint64_t {  // read backwards a list is ascending
+        float unused;
+        return tile < a.tiles ? slot_key(tile, slot, &unused) : 0;
     };
     uint64_t top[2] = {list_key(wave, lane), list_key(wave + kWaves, lane)};
 #pragma unroll 1
@@ -194,12 +303,7 @@ __global__ __launch_bounds__(kThreads) void topk_stage2(TopKArgs a) {
         top[1] = wave_merge(top[1], c1, lane);
     }
     const uint64_t mine = wave_merge(top[0], __shfl(top[1], kWave - 1 - lane, kWave), lane);
-    for (uint32_t tile = threadIdx.x; tile < a.tiles; tile += blockDim.x) {
-        if (partial[tile].first_nonfinite_col != kNone) atomicMin(&first_nonfinite, partial[tile].first_nonfinite_col);
-        if (partial[tile].first_subnormal_col != kNone) atomicMin(&first_subnormal, partial[tile].first_subnormal_col);
-    }
-    __syncthreads();
-    merge_waves_and_write(mine, lists, a.out + row, logits_row, a.vocabulary, first_nonfinite, first_subnormal);
+    merge_waves_and_write(mine, s.lists, a.out + row, logits_row, a.vocabulary, s.first_nonfinite, s.first_subnormal);
 }
 
 uint32_t tiles_for(uint32_t vocabulary) { return (vocabulary + kTileSpan - 1) / kTileSpan; }
