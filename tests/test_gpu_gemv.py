@@ -359,3 +359,19 @@ def test_gemv_units(gpu, orc, synth, t, cols, rows):
     x[1] = np.nan
     gpu.gemv(t, gpu.upload(w), gpu.upload(x), cols, rows)
     assert gpu.error() == 1
+
+
+@pytest.mark.parametrize("t,cols", [(12, 512), (12, 2048), (12, 2560), (14, 512), (14, 2560), (8, 2048), (8, 2560)])
+@pytest.mark.parametrize("exponent", [-70, -103, -110, -124])
+def test_gemv_tiny_activations(gpu, orc, synth, t, cols, exponent):
+    """Activations far below one, down to the smallest floats, multiply like any others. Error bound: as for test_gemv_units, and
+    an f32 operation on subnormals is off by up to 2^-150 whatever its result: a few for each of the row's products."""
+    rows = 65
+    w = synth.matrix(t, 2500 + cols, rows, cols)
+    x = synth.activations_f32(2501, cols) * np.float32(2.0 ** exponent)
+    x[32:64] *= np.float32(2.0 ** -20)  # a sub-block of subnormals among the last exponent's
+    x[64:96] = 0
+    dense = orc.dequantize(t, w, rows * cols).reshape(rows, cols).astype(np.float64)
+    bound = (np.abs(dense) * np.abs(x.astype(np.float64).reshape(-1, 32)).max(axis=1).repeat(32)).sum(axis=1) * (2.0 ** -23 + 2.0 ** -22) + cols * 2.0 ** -147
+    got = gpu.gemv(t, gpu.upload(w), gpu.upload(x), cols, rows).cpu().numpy().astype(np.float64)
+    assert (np.abs(got - dense @ x.astype(np.float64)) <= bound).all() and gpu.error() == 0

@@ -127,8 +127,10 @@ __device__ __forceinline__ float group_sum(float v) {
 // Four activations' digits share a dword, in the order of the four bytes of a word of codes, so that v_dot4_i32_i8
 // multiplies four weights per instruction and plane. The integer sums are exact; the three of a sub-block recombine in f32.
 // The eight threads of a sub-block are neighbours and agree on its scale with three cross-lane steps.
-// A record: three planes of eight dwords (c, b, a), then 1 / scale, the sum and a flag for values that are not finite; with
-// SUMS also, for each half of sixteen, -32 times the sums of its digits (a, b, c).
+// A record: three planes of eight dwords (c, b, a), then 1 / scale, the sum, a flag for values that are not finite and a second factor;
+// with SUMS also, for each half of sixteen, -32 times the sums of its digits (a, b, c).
+// Below 2^-60 a sub-block is first brought up by 2^90 (that is the second factor, 2^-90; else it is 1): the scale itself
+// would leave the range of a float from 2.4e-32 down and its inverse would be subnormal from 1e-31 down.
 template <uint32_t WORDS, bool SUMS>
 __device__ __forceinline__ void stage_quad(const float4& x4, bool mine, uint32_t quad, uint32_t* planes) {
     const float v4[4] = {mine ? x4.x : 0.0f, mine ? x4.y : 0.0f, mine ? x4.z : 0.0f, mine ? x4.w : 0.0f};
@@ -140,14 +142,15 @@ __device__ __forceinline__ void stage_quad(const float4& x4, bool mine, uint32_t
     flag |= uint32_t(__builtin_amdgcn_update_dpp(0, int(flag), 0xB1, 0xf, 0xf, true));
     flag |= uint32_t(__builtin_amdgcn_update_dpp(0, int(flag), 0x4E, 0xf, 0xf, true));
     flag |= uint32_t(__builtin_amdgcn_update_dpp(0, int(flag), 0x141, 0xf, 0xf, true));
-    // a sub-block of zeros, of subnormals only, or with something not finite in it keeps scale 1 (its integers are zeros)
-    const bool usable = biggest >= 1.1754944e-38f && !nonfinite(biggest) && flag == 0;
-    const float scale = usable ? 8290000.0f / biggest : 1.0f;
+    // a sub-block of zeros or with something not finite in it keeps scale 1 (its integers are zeros)
+    const bool usable = biggest > 0 && flag == 0, small = biggest < 0x1p-60f;
+    const float lift = small ? 0x1p90f : 1.0f, lifted = biggest * lift;
+    const float scale = usable ? 8290000.0f / lifted : 1.0f;
     uint32_t w2 = 0, w1 = 0, w0 = 0;
     int s2 = 0, s1 = 0, s0 = 0;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        const int xi = usable ? __float2int_rn(v4[e] * scale) : 0;
+        const int xi = usable ? __float2int_rn((v4[e] * lift) * scale) : 0;
         const int c = ((xi + 128) & 255) - 128, upper = (xi - c) >> 8;
         const int b = ((upper + 128) & 255) - 128, a8 = (upper - b) >> 8;
         w2 |= uint32_t(a8 & 0xff) << (8 * e);
@@ -159,9 +162,10 @@ __device__ __forceinline__ void stage_quad(const float4& x4, bool mine, uint32_t
     if (mine) {
         sub[16 + quad % 8] = w2; sub[8 + quad % 8] = w1; sub[quad % 8] = w0;
         if (quad % 8 == 0) {
-            sub[24] = __float_as_uint(usable ? biggest / 8290000.0f : 1.0f);
+            sub[24] = __float_as_uint(usable ? lifted / 8290000.0f : 1.0f);
             sub[25] = __float_as_uint(sum);
             sub[26] = flag;
+            sub[27] = __float_as_uint(small ? 0x1p-90f : 1.0f);
         }
     }
     if constexpr (SUMS) {
@@ -184,7 +188,7 @@ template <int BPR, bool PLANAR>
 __global__ __launch_bounds__(256) void gemv_q4k(GemvArgs a) {
     constexpr int LPR = 4 * BPR;        // lanes per row
     constexpr int RPS = kWave / LPR;    // rows per wave step
-    // per sub-block of 32 activations: three planes of eight dwords (four signed bytes each), then 1 / scale, the sum, a flag
+    // per sub-block of 32 activations: three planes of eight dwords (four signed bytes each), then 1 / scale, the sum, a flag, the second factor
     constexpr uint32_t kSubWords = 3 * 8 + 4;
     __shared__ __attribute__((aligned(16))) uint32_t planes[BPR * 8 * kSubWords];
     const uint8_t* w; const float* x; float* y;
@@ -243,7 +247,7 @@ __global__ __launch_bounds__(256) void gemv_q4k(GemvArgs a) {
     __syncthreads();
 
     uint32_t pa[3][8], pb[3][8];
-    float sxa, sxb, inv_a, inv_b;
+    float sxa, sxb, inv_a, inv_b, back_a, back_b;
     bool x_bad;
     {
         const uint32_t* sa = planes + (blk_in_row * 8 + pair * 2) * kSubWords;
@@ -255,6 +259,7 @@ __global__ __launch_bounds__(256) void gemv_q4k(GemvArgs a) {
         inv_a = __uint_as_float(sa[24]); sxa = __uint_as_float(sa[25]);
         inv_b = __uint_as_float(sb[24]); sxb = __uint_as_float(sb[25]);
         x_bad = (sa[26] | sb[26]) != 0;
+        back_a = __uint_as_float(sa[27]); back_b = __uint_as_float(sb[27]);
     }
 
     for (; step < steps; step += waves) {
@@ -295,8 +300,8 @@ __global__ __launch_bounds__(256) void gemv_q4k(GemvArgs a) {
             b0 = __builtin_amdgcn_sdot4(hi, int(pb[0][k]), b0, false);
         }
         // each plane's sum is below 2^16 and exact as a float; the three recombine with two roundings to f32
-        const float dot_a = __builtin_fmaf(float(a2), 65536.0f, __builtin_fmaf(float(a1), 256.0f, float(a0))) * inv_a;
-        const float dot_b = __builtin_fmaf(float(b2), 65536.0f, __builtin_fmaf(float(b1), 256.0f, float(b0))) * inv_b;
+        const float dot_a = __builtin_fmaf(float(a2), 65536.0f, __builtin_fmaf(float(a1), 256.0f, float(a0))) * inv_a * back_a;
+        const float dot_b = __builtin_fmaf(float(b2), 65536.0f, __builtin_fmaf(float(b1), 256.0f, float(b0))) * inv_b * back_b;
         // sum_c ((d*sc)*q - dmin*mn) * x = (d*sc) * sum q x - (dmin*mn) * sum x, per sub-block
         float part = (d * float(sc_a)) * dot_a - (dmin * float(mn_a)) * sxa;
         part += (d * float(sc_b)) * dot_b - (dmin * float(mn_b)) * sxb;
@@ -414,7 +419,7 @@ __global__ __launch_bounds__(256) void gemv_units(GemvArgs a) {
                         for (int i = 0; i < 4; ++i) acc[p] = __builtin_amdgcn_sdot4(int((words[k + i] >> (4 * h)) & 0x0f0f0f0fu), int(digits[i]), acc[p], false);
                     }
                 const quad_words rest = *reinterpret_cast<const quad_words*>(sub + 24);
-                const float dot = recombine(acc[2], acc[1], acc[0]) * __uint_as_float(rest[0]);
+                const float dot = recombine(acc[2], acc[1], acc[0]) * __uint_as_float(rest[0]) * __uint_as_float(rest[3]);
                 const float part_h = (d * float((sc >> (8 * h)) & 0xffu)) * dot - (dmin * float((mn >> (8 * h)) & 0xffu)) * __uint_as_float(rest[1]);
                 sum += rest[2] ? __uint_as_float(0x7fc00000u) : part_h;  // a non-finite activation: the row is not a number
             }
@@ -441,7 +446,7 @@ __global__ __launch_bounds__(256) void gemv_units(GemvArgs a) {
                 const quad_words rest = *reinterpret_cast<const quad_words*>(sub + 24);
                 const uint32_t at = 2 * q + half;  // the sub-scale's byte
                 const float ds = d * float(int(int8_t((now.sc[at / 4] >> (at % 4 * 8)) & 0xffu)));
-                const float dot = recombine(acc[2], acc[1], acc[0]) * __uint_as_float(rest[0]);
+                const float dot = recombine(acc[2], acc[1], acc[0]) * __uint_as_float(rest[0]) * __uint_as_float(rest[3]);
                 sum += rest[2] ? __uint_as_float(0x7fc00000u) : ds * dot;
             }
         } else {
@@ -457,7 +462,7 @@ __global__ __launch_bounds__(256) void gemv_units(GemvArgs a) {
                     for (int i = 0; i < 4; ++i) acc[p] = __builtin_amdgcn_sdot4(int(words[k + i]), int(digits[i]), acc[p], false);
                 }
             const quad_words rest = *reinterpret_cast<const quad_words*>(sub + 24);
-            sum = half_bits_to_float(now.d) * (recombine(acc[2], acc[1], acc[0]) * __uint_as_float(rest[0]));
+            sum = half_bits_to_float(now.d) * (recombine(acc[2], acc[1], acc[0]) * __uint_as_float(rest[0]) * __uint_as_float(rest[3]));
             if (rest[2]) sum = __uint_as_float(0x7fc00000u);
         }
         part += u0 < units ? sum : 0.0f;
