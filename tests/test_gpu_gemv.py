@@ -342,20 +342,37 @@ def test_gemv_f32_rows(gpu, synth, cols, rows, count):
     assert (np.abs(y.cpu().numpy() - want) <= (cols / 64 + 8) * 2.0 ** -24 * scale).all() and gpu.error() == 0
 
 
+def zero_columns(t, raw, rows, cols):
+    """Makes the sixth of every 32 weights of a GGUF matrix zero (Q4_K: the minima as well)."""
+    blocks = raw.reshape(rows * cols // (32 if t == 8 else 256), -1)
+    if t == 8:
+        blocks[:, 7] = 0
+    elif t == 12:
+        blocks[:, 2:4] = 0
+        blocks[:, 16 + 5:16 + 128:32] = 0  # both nibbles: the sixth of a pair's first and second 32
+    else:
+        blocks[:, [5, 37, 69, 101]] = 0  # low nibbles of elements 5, 37, 69, 101 of either section; the code 32 is zero
+        blocks[:, [133, 165]] = 0xaa
+
+
 @pytest.mark.parametrize("t,cols,rows", [(12, 256, 3), (12, 768, 70), (12, 2560, 513), (12, 6144, 9), (14, 256, 1), (14, 2560, 700), (14, 1280, 5000), (14, 12288, 2),
                                          (8, 32, 2), (8, 544, 33), (8, 2560, 600), (8, 5120, 17), (8, 1024, 9000)])
 def test_gemv_units(gpu, orc, synth, t, cols, rows):
-    """Rows of any length, 8 to 64 lanes per row, last rounds with idle lanes, more steps than waves. Error bound: activations
-    keep 24 bits of their sub-block's largest value and every product sum is exact per 16 or 32 weights, so 2^-23 of
-    sum |w x| covers rounding the activations and 2^-22 the f32 sums over at most 384 sub-blocks."""
+    """Rows of any length, 8 to 64 lanes per row, last rounds with idle lanes, more steps than waves. Error bound: a weight is rounded
+    once, a product passes at most 16 roundings in its chain, 26 over a row's rounds and 6 across lanes: 2^-18 of sum |w x|.
+    A second row of activations puts 3e4 to 1e30 in front of weights that are zero, one in each 32: nothing may be lost beside them."""
     w = synth.matrix(t, 2100 + cols, rows, cols)
+    zero_columns(t, w, rows, cols)
     x = synth.activations_f32(2101 + rows, cols)
     x[cols // 2:] *= np.float32(1e-3)
-    want = orc.reference_gemv(t, w, cols, rows, x)
-    dense = np.abs(orc.dequantize(t, w, rows * cols).reshape(rows, cols)).astype(np.float64)
-    bound = (dense * np.maximum(np.abs(x), np.abs(x.reshape(-1, 32)).max(axis=1).repeat(32))).sum(axis=1) * (2.0 ** -23 + 2.0 ** -22)
-    got = gpu.gemv(t, gpu.upload(w), gpu.upload(x), cols, rows).cpu().numpy().astype(np.float64)
-    assert (np.abs(got - want) <= bound).all() and gpu.error() == 0
+    dense = orc.dequantize(t, w, rows * cols).reshape(rows, cols).astype(np.float64)
+    assert not dense[:, 5::32].any()
+    beside = x.copy()
+    beside[5::32] = np.resize(np.array([3e4, -1e12, 1e30], dtype=np.float32), cols // 32)
+    for values in (x, beside):
+        bound = (np.abs(dense) @ np.abs(values.astype(np.float64))) * 2.0 ** -18
+        got = gpu.gemv(t, gpu.upload(w), gpu.upload(values), cols, rows).cpu().numpy().astype(np.float64)
+        assert (np.abs(got - dense @ values.astype(np.float64)) <= bound).all() and gpu.error() == 0
     x[1] = np.nan
     gpu.gemv(t, gpu.upload(w), gpu.upload(x), cols, rows)
     assert gpu.error() == 1

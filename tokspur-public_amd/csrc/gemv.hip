@@ -127,11 +127,10 @@ __device__ __forceinline__ float group_sum(float v) {
 // Four activations' digits share a dword, in the order of the four bytes of a word of codes, so that v_dot4_i32_i8
 // multiplies four weights per instruction and plane. The integer sums are exact; the three of a sub-block recombine in f32.
 // The eight threads of a sub-block are neighbours and agree on its scale with three cross-lane steps.
-// A record: three planes of eight dwords (c, b, a), then 1 / scale, the sum, a flag for values that are not finite and a second factor;
-// with SUMS also, for each half of sixteen, -32 times the sums of its digits (a, b, c).
+// A record: three planes of eight dwords (c, b, a), then 1 / scale, the sum, a flag for values that are not finite and a second factor.
 // Below 2^-60 a sub-block is first brought up by 2^90 (that is the second factor, 2^-90; else it is 1): the scale itself
 // would leave the range of a float from 2.4e-32 down and its inverse would be subnormal from 1e-31 down.
-template <uint32_t WORDS, bool SUMS>
+template <uint32_t WORDS>
 __device__ __forceinline__ void stage_quad(const float4& x4, bool mine, uint32_t quad, uint32_t* planes) {
     const float v4[4] = {mine ? x4.x : 0.0f, mine ? x4.y : 0.0f, mine ? x4.z : 0.0f, mine ? x4.w : 0.0f};
     float biggest = fmaxf(fmaxf(fabsf(v4[0]), fabsf(v4[1])), fmaxf(fabsf(v4[2]), fabsf(v4[3])));
@@ -147,7 +146,6 @@ __device__ __forceinline__ void stage_quad(const float4& x4, bool mine, uint32_t
     const float lift = small ? 0x1p90f : 1.0f, lifted = biggest * lift;
     const float scale = usable ? 8290000.0f / lifted : 1.0f;
     uint32_t w2 = 0, w1 = 0, w0 = 0;
-    int s2 = 0, s1 = 0, s0 = 0;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const int xi = usable ? __float2int_rn((v4[e] * lift) * scale) : 0;
@@ -156,7 +154,6 @@ __device__ __forceinline__ void stage_quad(const float4& x4, bool mine, uint32_t
         w2 |= uint32_t(a8 & 0xff) << (8 * e);
         w1 |= uint32_t(b & 0xff) << (8 * e);
         w0 |= uint32_t(c & 0xff) << (8 * e);
-        if constexpr (SUMS) { s2 += a8; s1 += b; s0 += c; }
     }
     uint32_t* sub = planes + (quad / 8) * WORDS;
     if (mine) {
@@ -166,17 +163,6 @@ __device__ __forceinline__ void stage_quad(const float4& x4, bool mine, uint32_t
             sub[25] = __float_as_uint(sum);
             sub[26] = flag;
             sub[27] = __float_as_uint(small ? 0x1p-90f : 1.0f);
-        }
-    }
-    if constexpr (SUMS) {
-        auto over_four = [](int v) {
-            v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, true);
-            return v + __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, true);
-        };
-        s2 = over_four(s2); s1 = over_four(s1); s0 = over_four(s0);
-        if (mine && quad % 4 == 0) {
-            uint32_t* half = sub + 28 + quad % 8;
-            half[0] = uint32_t(-32 * s2); half[1] = uint32_t(-32 * s1); half[2] = uint32_t(-32 * s0);
         }
     }
 }
@@ -242,7 +228,7 @@ __global__ __launch_bounds__(256) void gemv_q4k(GemvArgs a) {
 #pragma unroll
     for (uint32_t j = 0; j < kMine; ++j) {
         const uint32_t quad = threadIdx.x + j * 256;
-        stage_quad<kSubWords, false>(xv[j], kQuads % 256 == 0 || quad < kQuads, quad, planes);  // uniform over every group of eight lanes
+        stage_quad<kSubWords>(xv[j], kQuads % 256 == 0 || quad < kQuads, quad, planes);  // uniform over every group of eight lanes
     }
     __syncthreads();
 
@@ -315,13 +301,16 @@ __global__ __launch_bounds__(256) void gemv_q4k(GemvArgs a) {
 }
 
 // ------------------------------------------------------------------------------------ Q4_K, Q6_K, Q8_0 rows of any length
-// The same arithmetic for rows of any number of super-blocks and for the other two encodings a decode step meets. L lanes share a
-// row; a lane takes every L-th unit of it (64 weights of a K-quant block, one Q8_0 block) and finds its activations' digits in
-// LDS, three reads of 16 bytes per sixteen weights and plane set, instead of keeping those of one place in the row in registers.
-// Bound by memory for large matrices, by one round trip for small ones: the next unit's bytes are requested before the
-// current one is multiplied. Blocks of 34 and 210 bytes are even-aligned only; neighbouring lanes read neighbouring pieces,
-// so the lines are shared all the same. Per-element decoding before: Q6_K 2731 x 2560 9.8 -> 6.0 us, 40 000 x 6144 (202 MB) 46 us
-// now = 4.3 TB/s; Q8_0 16 000 x 2560 21 -> 11 us.
+// Rows of any number of super-blocks, and the other two encodings a decode step meets, in the arithmetic of the per-element kernel:
+// every weight is decoded to the float it stands for (one rounding, where the format needs one) and meets its activation as a float in a
+// fused multiply-add, so one large activation takes no bits from its neighbours. L lanes share a row; a lane takes every L-th unit
+// of it (64 weights of a K-quant block, one Q8_0 block). A unit's activations lie together in LDS, in the order its codes
+// unpack, four floats of padding behind each unit so that neighbouring lanes' reads of 16 bytes fall in different banks.
+// Bound by memory for large matrices (about three and a half instructions per weight take half the time of its bytes), by one round
+// trip for small ones: the next unit's bytes are requested before the current one is multiplied. Blocks of 34 and 210 bytes are
+// even-aligned only; neighbouring lanes read neighbouring pieces, so the lines are shared all the same. The per-element kernel takes
+// 9.8 us at Q6_K 2731 x 2560, this one 4.9; 40 000 x 6144 (202 MB) 48 us = 4.2 TB/s; Q8_0 16 000 x 2560 21 us there, 11 here.
+// (Activations as 24-bit integers under one scale per 32, as gemv_q4k has them: 5.8, 46 and 11 us.)
 typedef uint32_t piece16 __attribute__((ext_vector_type(4), aligned(2)));
 typedef uint32_t piece8 __attribute__((ext_vector_type(2), aligned(2)));
 typedef uint32_t quad_words __attribute__((ext_vector_type(4)));
@@ -331,15 +320,16 @@ template <> struct UnitBytes<12> { quad_words hdr, q0, q1; };
 template <> struct UnitBytes<14> { piece16 la, lb, qh; piece8 sc; uint16_t d; };
 template <> struct UnitBytes<8> { piece16 q0, q1; uint16_t d; };
 
-__device__ __forceinline__ float recombine(int a2, int a1, int a0) {
-    return __builtin_fmaf(float(a2), 65536.0f, __builtin_fmaf(float(a1), 256.0f, float(a0)));
-}
+// Floats of a unit of 64 (32) activations in LDS, padding included, and of a row.
+__host__ __device__ constexpr uint32_t unit_floats(uint32_t type) { return type == 8 ? 36u : 68u; }
+__host__ __device__ constexpr uint32_t units_lds_bytes(uint32_t type, uint32_t columns) { return columns / (type == 8 ? 32 : 64) * unit_floats(type) * 4; }
+
+__device__ __forceinline__ float code_of(uint32_t word, int i) { return float((word >> (8 * i)) & 0xffu); }
 
 template <uint32_t T, int L>
 __global__ __launch_bounds__(256) void gemv_units(GemvArgs a) {
-    constexpr bool SUMS = T == 14;
-    constexpr uint32_t kWords = SUMS ? 36 : 28, kUnit = T == 8 ? 32 : 64, RPS = kWave / L;
-    extern __shared__ __attribute__((aligned(16))) uint32_t planes[];
+    constexpr uint32_t kUnit = T == 8 ? 32 : 64, kFloats = unit_floats(T), RPS = kWave / L;
+    extern __shared__ __attribute__((aligned(16))) float staged[];
     const uint8_t* w; const float* x; float* y;
     if (!resolve(a, w, x, y)) return;
     const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave, in_row = lane % L, row_in_step = lane / L;
@@ -375,17 +365,19 @@ __global__ __launch_bounds__(256) void gemv_units(GemvArgs a) {
 
     // the activations first, the wave's first weight bytes right behind them; the activations are staged while the weights travel
     const uint32_t quads = a.columns / 4;
-    float4 x0 = make_float4(0, 0, 0, 0);
     auto load_quad = [&](uint32_t quad) {
         return quad < quads ? *reinterpret_cast<const float4*>(x + 4 * quad) : make_float4(0, 0, 0, 0);
     };
-    x0 = load_quad(threadIdx.x);
+    float4 x0 = load_quad(threadIdx.x);
     uint32_t step = blockIdx.x * (blockDim.x / kWave) + wave;
     UnitBytes<T> cur = fetch(step < steps ? step : 0, 0);
-    for (uint32_t quad = threadIdx.x; quad < (quads + 7) / 8 * 8; quad += 256) {
+    for (uint32_t quad = threadIdx.x; quad < quads; quad += 256) {
         const float4 here = x0;
         x0 = load_quad(quad + 256);
-        stage_quad<kWords, SUMS>(here, quad < quads, quad, planes);
+        uint32_t at;
+        if constexpr (T == 14) at = (quad / 64 * 4 + quad / 32 % 2 * 2 + quad / 4 % 2) * kFloats + quad / 8 % 4 * 16 + quad % 4 * 4;  // section, half | quarter
+        else at = quad / (kUnit / 4) * kFloats + quad % (kUnit / 4) * 4;
+        *reinterpret_cast<float4*>(staged + at) = here;
     }
     __syncthreads();
 
@@ -396,7 +388,16 @@ __global__ __launch_bounds__(256) void gemv_units(GemvArgs a) {
         const bool last = round + 1 == rounds;
         const uint32_t next_step = last ? (step + waves < steps ? step + waves : step) : step;
         cur = fetch(next_step, last ? 0 : round + 1);  // the next unit's bytes travel while this one is summed
-        float sum = 0;
+        const float* const xs = staged + u * kFloats;
+        float sum[4] = {0, 0, 0, 0};  // four chains
+        // four weights, scale * code + offset each, against the unit's activations 4 i .. 4 i + 3
+        auto four = [&](int i, uint32_t codes, float scale, float offset) {
+            const float4 x4 = *reinterpret_cast<const float4*>(xs + 4 * i);
+            sum[0] = __builtin_fmaf(__builtin_fmaf(code_of(codes, 0), scale, offset), x4.x, sum[0]);
+            sum[1] = __builtin_fmaf(__builtin_fmaf(code_of(codes, 1), scale, offset), x4.y, sum[1]);
+            sum[2] = __builtin_fmaf(__builtin_fmaf(code_of(codes, 2), scale, offset), x4.z, sum[2]);
+            sum[3] = __builtin_fmaf(__builtin_fmaf(code_of(codes, 3), scale, offset), x4.w, sum[3]);
+        };
         if constexpr (T == 12) {
             const uint32_t pair = u % 4;
             const float d = half_bits_to_float(now.hdr[0] & 0xffffu), dmin = half_bits_to_float(now.hdr[0] >> 16);
@@ -405,67 +406,33 @@ __global__ __launch_bounds__(256) void gemv_units(GemvArgs a) {
             const uint32_t s2 = (now.hdr[1] >> sh) & 0xffffu, m2 = (now.hdr[2] >> sh) & 0xffffu, e2 = (now.hdr[3] >> sh) & 0xffffu;
             const uint32_t sc = pair < 2 ? s2 & 0x3f3fu : (e2 & 0x0f0fu) | ((s2 >> 2) & 0x3030u);
             const uint32_t mn = pair < 2 ? m2 & 0x3f3fu : ((e2 >> 4) & 0x0f0fu) | ((m2 >> 2) & 0x3030u);
-            const uint32_t words[8] = {now.q0[0], now.q0[1], now.q0[2], now.q0[3], now.q1[0], now.q1[1], now.q1[2], now.q1[3]};
-            const uint32_t* sub = planes + u * 2 * kWords;
 #pragma unroll
-            for (int h = 0; h < 2; ++h, sub += kWords) {
-                int acc[3] = {0, 0, 0};
+            for (int h = 0; h < 2; ++h) {
+                // both products are exact (11 + 6 bits), so is scale * code: the weight is rounded once, as the decoder rounds it
+                const float scale = d * code_of(sc, h), offset = -(dmin * code_of(mn, h));
 #pragma unroll
-                for (int p = 0; p < 3; ++p)
-#pragma unroll
-                    for (int k = 0; k < 8; k += 4) {
-                        const quad_words digits = *reinterpret_cast<const quad_words*>(sub + p * 8 + k);
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) acc[p] = __builtin_amdgcn_sdot4(int((words[k + i] >> (4 * h)) & 0x0f0f0f0fu), int(digits[i]), acc[p], false);
-                    }
-                const quad_words rest = *reinterpret_cast<const quad_words*>(sub + 24);
-                const float dot = recombine(acc[2], acc[1], acc[0]) * __uint_as_float(rest[0]) * __uint_as_float(rest[3]);
-                const float part_h = (d * float((sc >> (8 * h)) & 0xffu)) * dot - (dmin * float((mn >> (8 * h)) & 0xffu)) * __uint_as_float(rest[1]);
-                sum += rest[2] ? __uint_as_float(0x7fc00000u) : part_h;  // a non-finite activation: the row is not a number
+                for (int i = 0; i < 8; ++i) four(8 * h + i, ((i < 4 ? now.q0[i % 4] : now.q1[i % 4]) >> (4 * h)) & 0x0f0f0f0fu, scale, offset);
             }
         } else if constexpr (T == 14) {
-            const uint32_t sec = u / 2 % 2, half = u % 2;
+            const uint32_t half = u % 2;
             const float d = half_bits_to_float(now.d);
-            const uint32_t* sub = planes + (u / 4 * 8 + sec * 4) * kWords;
 #pragma unroll
-            for (int q = 0; q < 4; ++q, sub += kWords) {  // 16 weights of one sub-scale
-                const quad_words bias = *reinterpret_cast<const quad_words*>(sub + 28 + half * 4);  // -32 times the digits' sums
-                int acc[3] = {int(bias[2]), int(bias[1]), int(bias[0])};
-                uint32_t code[4];
+            for (int q = 0; q < 4; ++q) {  // 16 weights of one sub-scale
+                const uint32_t at = 2 * q + half;  // the sub-scale's byte
+                const float scale = d * float(int(int8_t((now.sc[at / 4] >> (at % 4 * 8)) & 0xffu)));  // exact; scale * (code - 32) is rounded once
+                const float offset = -32.0f * scale;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const uint32_t low = q % 2 ? now.lb[i] : now.la[i], high = now.qh[i] >> (2 * q);
-                    code[i] = ((q < 2 ? low : low >> 4) & 0x0f0f0f0fu) | ((high & 0x03030303u) << 4);
+                    four(4 * q + i, ((q < 2 ? low : low >> 4) & 0x0f0f0f0fu) | ((high & 0x03030303u) << 4), scale, offset);
                 }
-#pragma unroll
-                for (int p = 0; p < 3; ++p) {
-                    const quad_words digits = *reinterpret_cast<const quad_words*>(sub + p * 8 + half * 4);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) acc[p] = __builtin_amdgcn_sdot4(int(code[i]), int(digits[i]), acc[p], false);
-                }
-                const quad_words rest = *reinterpret_cast<const quad_words*>(sub + 24);
-                const uint32_t at = 2 * q + half;  // the sub-scale's byte
-                const float ds = d * float(int(int8_t((now.sc[at / 4] >> (at % 4 * 8)) & 0xffu)));
-                const float dot = recombine(acc[2], acc[1], acc[0]) * __uint_as_float(rest[0]) * __uint_as_float(rest[3]);
-                sum += rest[2] ? __uint_as_float(0x7fc00000u) : ds * dot;
             }
         } else {
-            const uint32_t words[8] = {now.q0[0], now.q0[1], now.q0[2], now.q0[3], now.q1[0], now.q1[1], now.q1[2], now.q1[3]};
-            const uint32_t* sub = planes + u * kWords;
-            int acc[3] = {0, 0, 0};
+            const float d = half_bits_to_float(now.d), offset = -128.0f * d;  // a quant is its code less 128, both products exact
 #pragma unroll
-            for (int p = 0; p < 3; ++p)
-#pragma unroll
-                for (int k = 0; k < 8; k += 4) {
-                    const quad_words digits = *reinterpret_cast<const quad_words*>(sub + p * 8 + k);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) acc[p] = __builtin_amdgcn_sdot4(int(words[k + i]), int(digits[i]), acc[p], false);
-                }
-            const quad_words rest = *reinterpret_cast<const quad_words*>(sub + 24);
-            sum = half_bits_to_float(now.d) * (recombine(acc[2], acc[1], acc[0]) * __uint_as_float(rest[0]) * __uint_as_float(rest[3]));
-            if (rest[2]) sum = __uint_as_float(0x7fc00000u);
+            for (int i = 0; i < 8; ++i) four(i, (i < 4 ? now.q0[i % 4] : now.q1[i % 4]) ^ 0x80808080u, d, offset);
         }
-        part += u0 < units ? sum : 0.0f;
+        part += u0 < units ? (sum[0] + sum[1]) + (sum[2] + sum[3]) : 0.0f;
         if (!last) { ++round; continue; }
         const uint32_t row = step * RPS + row_in_step;
         const float total = group_sum<L>(part);
@@ -485,7 +452,7 @@ uint32_t grid_rows(uint32_t work_items, uint32_t per_block) {
     return blocks < 1 ? 1 : blocks > 2048 ? 2048 : blocks;
 }
 
-// Rows whose digits fit LDS, activations in 16-byte pieces, blocks as aligned as their encoding has them.
+// Rows whose activations fit LDS three times (12 288 columns: 52 KB, three workgroups per compute unit), activations in 16-byte pieces, blocks as aligned as their encoding has them.
 bool gemv_units_takes(uint32_t encoding, const GemvArgs& a) {
     if (encoding != 8 && encoding != 12 && encoding != 14) return false;
     const uintptr_t step = encoding == 12 ? 16 : 2;
@@ -495,11 +462,11 @@ bool gemv_units_takes(uint32_t encoding, const GemvArgs& a) {
 
 template <uint32_t T, int L>
 int launch_units_lanes(const GemvArgs& a, hipStream_t stream) {
-    const uint32_t bytes = a.columns / 32 * (T == 14 ? 36 : 28) * 4;
+    const uint32_t bytes = units_lds_bytes(T, a.columns);
     static std::atomic<uint64_t> raised{0};
     int device = 0;
     if (bytes > 48 * 1024 && setup_pending(raised, &device)) {
-        TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemv_units<T, L>), hipFuncAttributeMaxDynamicSharedMemorySize, 12288 / 32 * 36 * 4));
+        TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemv_units<T, L>), hipFuncAttributeMaxDynamicSharedMemorySize, int(units_lds_bytes(T, 12288))));
         setup_done(raised, device);
     }
     uint32_t blocks = grid_rows((a.rows + kWave / L - 1) / (kWave / L), 4);
@@ -511,9 +478,9 @@ int launch_units_lanes(const GemvArgs& a, hipStream_t stream) {
 
 template <uint32_t T>
 int launch_units(const GemvArgs& a, hipStream_t stream) {
-    // Lanes per row: the count that leaves the fewest lanes without a unit in a row's last round (at 16 000 x 2560, 40 units: 8 lanes
-    // 8.0 us, 64 lanes 10.7), sixteen where several leave equally few; more where that would leave the chip with fewer than 512
-    // waves (at 512 x 2560: 64 lanes 4.2 us, 8 lanes 6.0).
+    // Lanes per row: the count that leaves the fewest lanes without a unit in a row's last round (Q6_K 16 000 x 2560, 40 units: 8
+    // lanes 8.8 us, 64 lanes 10.9), sixteen where several leave equally few; more where that would leave the chip with fewer than 512
+    // waves (at 512 x 2560: 64 lanes 4.7 us, 8 lanes 6.4).
     const uint32_t units = a.columns / (T == 8 ? 32 : 64);
     uint32_t lanes = 16;
     auto idle = [&](uint32_t l) { return (units + l - 1) / l * l; };
