@@ -270,3 +270,64 @@ def test_routed_m8_streamed(gpu, tsp, orc, synth, dn, channels, hidden, experts,
     if tokens > 2:  # two or more tokens take the same kernels
         _, pair = tsp.planar_moe_routed_m8(gpu, w, gpu.upload(ids[-2:].reshape(-1)), gpu.upload(np.ascontiguousarray(x[-2:, :channels])), 2, selected)
         assert np.array_equal(pair.cpu().numpy().view(np.uint32), np.ascontiguousarray(y[-2 * selected:, :channels]).view(np.uint32))
+
+
+@pytest.mark.parametrize("tokens", [1, 4, 5, 6, 8])
+@pytest.mark.parametrize("dn,channels,hidden", [(8, 2560, 640), (7, 2304, 160), (8, 1280, 96), (7, 768, 2560), (14, 256, 2304)])
+def test_routed_m8_streamed_f32(gpu, tsp, orc, synth, dn, channels, hidden, tokens):
+    """Rows of more than 2048 columns, and all rows of Q8_0 and Q5_1, are multiplied as the floats they are, also
+    where every token meets one expert (more rows than one pass has room for): values 1e6 to 1e30 beside ordinary ones, in front
+    of weights that are zero, take nothing from them.
+    Error bound: eight roundings of a block's sums and one for each of at most 80 blocks, of the sum of |scale * code| + |minimum|
+    times |x|, less than 2^-17 of it; the expected values take the rows that the device itself has."""
+    experts, selected = 8, 2
+    gate, up = synth.matrix(12, 61, hidden * experts, channels), synth.matrix(12, 62, hidden * experts, channels)
+    down = synth.matrix(dn, 63, channels * experts, hidden)
+    for raw in (gate, up):  # weight 5 of every 256: a sub-block without minimum, the code zero
+        blocks = raw.reshape(-1, 144)
+        blocks[:, 8] &= 0xC0
+        blocks[:, 16 + 5] &= 0xF0
+    # hidden units 5, 101, 197, ... come out some 2^26 times the others
+    for raw, factor in ((gate, 2.0 ** 6), (up, 2.0 ** 20)):
+        scales = raw.reshape(experts, hidden, channels // 256, 144)[:, 5::96, :, 0:4]
+        scales[:] = np.minimum(np.ascontiguousarray(scales).view(np.float16).astype(np.float64) * factor, 60000).astype(np.float16).view(np.uint8)
+    blocks = down.reshape(-1, 210) if dn == 14 else down.reshape(experts * channels, hidden // 32, -1)[:, ::3]
+    if dn == 14:
+        blocks[:, [5, 37, 69, 101]] = 0
+        blocks[:, [133, 165]] = 0xaa
+    elif dn == 8:
+        blocks[:, :, 2 + 5] = 0
+    else:
+        blocks[:, :, 2:4] = 0
+        blocks[:, :, 4] &= 0xDF  # the fifth bit
+        blocks[:, :, 8 + 5] &= 0xF0
+    w = tsp.PlanarMoeWeights(gpu, 12, dn, channels, hidden, experts, gate, up, down)
+    ids = np.array([[3, (t + 4) % experts] if t != 2 else [3, 1] for t in range(tokens)], dtype=np.uint32).reshape(-1)
+    x = (synth.activations_f32(64 + tokens, (tokens, channels)) * 0.1).astype(np.float32)
+    if channels > 2048:  # up to there a row is two halves under one scale
+        x[:, 5::256] = np.resize(np.array([1e6, -3e12, 1e30], dtype=np.float32), channels // 256)
+    x[tokens // 2] *= np.float32(1e-12)
+    h, y = tsp.planar_moe_routed_m8(gpu, w, gpu.upload(ids), gpu.upload(x), tokens, selected)
+    h, y = h.cpu().numpy().astype(np.float64), y.cpu().numpy().astype(np.float64)
+    assert gpu.error() == 0
+
+    def weights(t, raw, rows, cols):  # the weights of each expert, and |scale * code| + |minimum|
+        value = orc.dequantize(t, raw, experts * rows * cols).astype(np.float64).reshape(experts, rows, cols)
+        if t in (8, 14):
+            return value, np.abs(value)
+        least = raw.copy()
+        b = least.reshape(-1, 144 if t == 12 else 24)
+        b[:, 0:2] = 0  # no scale: the minima alone
+        least = np.abs(orc.dequantize(t, least, value.size).astype(np.float64).reshape(value.shape))
+        return value, np.abs(value) + 2 * least
+
+    (gate_w, gate_a), (up_w, up_a), (down_w, down_a) = weights(12, gate, hidden, channels), weights(12, up, hidden, channels), weights(dn, down, channels, hidden)
+    unit = 2.0 ** -17
+    for r, e in enumerate(ids):
+        row = x[r // selected].astype(np.float64)
+        g, u, dg, du = gate_w[e] @ row, up_w[e] @ row, unit * (gate_a[e] @ np.abs(row)), unit * (up_a[e] @ np.abs(row))
+        s = 1 / (1 + np.exp(-np.clip(g, -700, 700)))
+        bound = 1.1 * dg * (np.abs(u) + du) + np.abs(g * s) * du + 2.0 ** -20 * np.abs(g * s * u) + 1e-36
+        assert (np.abs(h[r] - g * s * u) <= bound).all(), (r, float(np.max(np.abs(h[r] - g * s * u) / bound)))
+        bound = unit * (down_a[e] @ np.abs(h[r])) + 1e-36
+        assert (np.abs(y[r] - down_w[e] @ h[r]) <= bound).all(), (r, float(np.max(np.abs(y[r] - down_w[e] @ h[r]) / bound)))

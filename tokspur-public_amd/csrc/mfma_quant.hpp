@@ -12,6 +12,9 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
 enum BKind : int { B_Q4K_RAW = 0, B_Q4K_PLANAR = 1, B_Q6K_PLANAR = 2 };
 
 // Workgroup barrier that waits for this wave's LDS traffic only. __syncthreads() also drains every outstanding
@@ -82,6 +85,39 @@ __device__ __forceinline__ f16x8 quants8(uint32_t w0, uint32_t w1) {
     const f16x2 p0 = as_h2(spread01(u0, K)) + off, p1 = as_h2(spread23(u0, K)) + off;
     const f16x2 p2 = as_h2(spread01(u1, K)) + off, p3 = as_h2(spread23(u1, K)) + off;
     return f16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
+}
+
+// ---------------------------------------------------------------- f32 operands
+// A float is three bf16 values, its top eight significant bits, the next eight and the last eight: cut off the top, subtract, again.
+// Every step is exact and the pieces have a float's own exponent range, so three products with the same integer weights, summed
+// in f32, are the f32 product whatever else is in the row. (Two halves under a power of two per row carry 22 bits, and fewer for
+// what is far below the row's largest value.) Pieces below 2^-133 are cut off: `row_lift` keeps ordinary rows away from there, and
+// from sums that overflow before the block's scale has been applied. It takes the exponent that a row's largest magnitude has.
+__device__ __forceinline__ float top_bits(float v) { return __uint_as_float(__float_as_uint(v) & 0xffff0000u); }
+struct Pieces { float hi, mid, lo; };  // the upper 16 bits of each
+__device__ __forceinline__ Pieces three_pieces(float v) {
+    const float rest = v - top_bits(v);
+    return Pieces{v, rest, rest - top_bits(rest)};
+}
+__device__ __forceinline__ uint32_t two_tops(float a, float b) { return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u); }
+__device__ __forceinline__ int row_lift(float biggest) { return biggest >= 0x1p64f ? -64 : biggest < 0x1p-40f ? 64 : 0; }
+__device__ __forceinline__ float power_of_two(int e) { return __uint_as_float(uint32_t(127 + e) << 23); }
+
+// Integers of at most eight bits as exact bf16: eight int8 quants, or eight codes 0 .. 255 (one per byte of w0, w1).
+__device__ __forceinline__ bf16x8 quants8_bf16(uint32_t w0, uint32_t w1) {
+    auto f = [](uint32_t w, int i) { return float(int(int8_t(w >> (8 * i)))); };
+    return __builtin_bit_cast(bf16x8, u32x4{two_tops(f(w0, 0), f(w0, 1)), two_tops(f(w0, 2), f(w0, 3)), two_tops(f(w1, 0), f(w1, 1)), two_tops(f(w1, 2), f(w1, 3))});
+}
+__device__ __forceinline__ bf16x8 codes8_bf16(uint32_t w0, uint32_t w1) {
+    auto f = [](uint32_t w, int i) { return float((w >> (8 * i)) & 0xffu); };
+    return __builtin_bit_cast(bf16x8, u32x4{two_tops(f(w0, 0), f(w0, 1)), two_tops(f(w0, 2), f(w0, 3)), two_tops(f(w1, 0), f(w1, 1)), two_tops(f(w1, 2), f(w1, 3))});
+}
+// Eight codes 0 .. 15: as the float8 (e4m3) of the same bits a code q is q 2^-9, subnormal up to 7 and the first binade above, and
+// one conversion turns two of them into bf16 under a power of two.
+__device__ __forceinline__ bf16x8 nibbles8_bf16(uint32_t w0, uint32_t w1) {
+    const bf16x2 p0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 512.0f, false), p1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 512.0f, true);
+    const bf16x2 p2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 512.0f, false), p3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 512.0f, true);
+    return bf16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
 }
 
 // Sixteen weights of a Q5_1 block as two fragments. Element e is nibble e % 16 (low for e < 16, high above) of byte e % 16 with bit e

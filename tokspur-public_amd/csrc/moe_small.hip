@@ -3,7 +3,9 @@
 //   y[rid, c] = Wd[e] h[rid] . c                            down projection
 // with rid = t*selected + slot and e = ids[rid]. HBM-bound: the union records (one per distinct
 // expert, up to 8 tokens each) let every expert's weights be streamed from HBM once for all the
-// tokens that route to it. f32 decode, f32 accumulate, no narrowing.
+// tokens that route to it. f32 sums of exact weights everywhere. The rows are f32, except Q4_K and Q6_K products of up to 2048
+// columns and 16-byte aligned rows: there they are two halves under a power of two, 22 bits below the row's (or the
+// slice's) largest value.
 //
 // This file holds the entry points, the choice of a kernel and the per-element arm, which takes any planar encoding, width and
 // alignment. The kernels that stream the weights past the matrix cores are in record_resident.hip, record_stream.hip and
@@ -233,7 +235,8 @@ SkinnyMoe skinny_view(const SmallMoeArgs& a, const tsp_shared_rows* shared = nul
 // Which kernel takes the gate/up product. Q4_K rows of 2048 columns and two or more tokens: the record-resident one (27 us at 8
 // tokens and 512 hidden units where the streaming one takes 34). One token and a row of 1, 2, 4 or 8 super-blocks: one
 // super-block per wave (10.9 against 12.3 us at 2048 x 768, 8.2 against 8.9 at 1024 x 512). Everything else Q4_K up to 2560 columns
-// streams; other encodings, wider rows and rows that 16 bytes do not align go weight by weight.
+// streams: what a workgroup holds in LDS, and the registers that stage a row, end there. Other encodings, wider rows and rows
+// that 16 bytes do not align go weight by weight.
 enum GateUpArm { GU_GENERIC, GU_RECORD, GU_FLAT, GU_STREAM };
 GateUpArm gate_up_arm(const SmallMoeArgs& a, const tsp_shared_rows* shared) {
     const SkinnyMoe v = skinny_view(a, shared);
@@ -268,7 +271,8 @@ int launch_gate_up(const SmallMoeArgs& a, hipStream_t s, const tsp_shared_rows* 
 }
 
 // Q6_K rows of 1, 2, 4 or 8 super-blocks keep one super-block per wave (19 us at config 2's 512 hidden units where the
-// streaming kernel takes 23); other widths and the 32-weight blocks stream.
+// streaming kernel takes 23); its other widths up to 2048 columns and the 32-weight blocks up to 2560 stream, wider ones go
+// weight by weight.
 int launch_down(const SmallMoeArgs& a, hipStream_t s, const tsp_shared_rows* shared = nullptr) {
     const SkinnyMoe v = skinny_view(a, shared);
     if (flat_down_takes(v)) return flat_moe_down(v, s);

@@ -11,22 +11,29 @@
 //     over the waves whatever tile they fall in; every piece leaves its sums in LDS, and after one barrier the pieces of a row
 //     are added up in column order. No wave waits for another in between, neither an odd number of super-blocks per row nor
 //     one of records leaves waves idle, and a result does not depend on how the launch was cut.
-//   * The rows of the share's records (at most eight, f32) go to LDS once, as an operand of sixteen rows for
-//     v_mfma_f32_16x16x32_f16: under a power of two per row that brings the largest magnitude near 2^14, split into high
-//     halves (operand rows 0..7) and low halves (rows 8..15), 22 significant bits together. One instruction multiplies both with
-//     512 weights, which are exact integers as halves (q for Q8_0 and Q5_1, sc * q for Q4_K, sc * (q - 32) for Q6_K); the block
-//     scales are applied to the f32 sums.
+//   * The rows of the share's records go to LDS once, as an operand of sixteen rows for the 16x16x32 matrix instructions, which
+//     meet 512 weights at a time; the block scales are applied to the f32 sums. Two forms:
+//     f32 rows (Q8_0, Q5_1, and Q4_K above 2048 columns): at most five rows, each as three bf16 pieces that are the float
+//     exactly (mfma_quant.hpp), against the integer codes q; a record of more rows is passed twice.
+//     Rows of 22 bits (Q4_K and Q6_K up to 2048 columns, as the kernels for their other widths have them, skinny.hip): at most eight,
+//     under a power of two per row that brings the largest magnitude near 2^14, as high halves (operand rows 0..7) and low halves
+//     (rows 8..15), against the integers sc * q, resp. sc * (q - 32), which have too many bits for bf16. Half as many scalings, and
+//     eight rows at once: at 1024 x 512, 8 tokens, a sublayer takes 34 us so and 41 in the other form.
 //   * A step's weight bytes are requested three steps ahead, whole 128-byte pieces of rows by neighbouring lanes, into
 //     registers; they turn into fragment order through 2 to 3.5 KB of LDS of the wave's own. (A lane that requests the pieces
 //     of its own row makes the address unit take ~50 cycles per request, more than the memory needs for the bytes.)
 //
-// Measured (events, 2560 channels x 640 hidden units, Q8_0 down, 8 tokens, 69 distinct experts: 131 MB of gate/up, 120 MB of
-// down): 43 + 34 us, where the per-element kernels took 194 + 142. Without the arithmetic the gate/up launch takes 38 us,
-// without the requests 39: of these some 8 are the launch's serial beginning (ids, records, table, first bytes), the rest is
-// a stream at 5 TB/s beside an instruction stream of equal length. Two tiles per step against one read of the operand (a
-// tenth fewer instructions), and the LDS round trip of a step overlapped with the products of the one before, were each
-// built and made no difference. For rows of 1, 2, 4 or 8 super-blocks the kernels that keep a wave's columns in registers
-// (record_resident.hip, skinny.hip) stay the faster ones where they apply: no operand is read from LDS there.
+// Measured (kernel trace, 2560 channels x 640 hidden units, 8 tokens, 69 distinct experts: 131 MB of gate/up, 120 MB of Q8_0 or
+// 85 MB of Q5_1 down): 45 us, 36 and 41, where the per-element kernels took 194 and 142. (With rows of 22 bits 43 and 34: the
+// f32 form costs a scaling per 32 columns in Q4_K, and a Q5_1 block its nearest code.) Some 8 us are the launch's serial
+// beginning (ids, records, table, first bytes), the rest is a stream at 5 TB/s beside an instruction stream of equal length.
+// Two tiles per step against one read of the operand (a tenth fewer instructions), and the LDS round trip of a step overlapped
+// with the products of the one before, were each built and made no difference. For rows of 1, 2, 4 or 8 super-blocks the
+// kernels that keep a wave's columns in registers (record_resident.hip, skinny.hip) stay the faster ones where they apply: no
+// operand is read from LDS there.
+//
+// Error against sums in 64 bits (2-norm, per row of 16 experts, normal rows): gate/up at 2560 x 640 1.35e-7 of h (per element in f32
+// 2.1e-7, rows of 22 bits 2.0e-7), Q8_0 down 8.0e-8 (8.8e-8, 9.2e-8), Q5_1 down 7.6e-8 (6.6e-8, 9.7e-8).
 #include "record_stream.hpp"
 
 #include <type_traits>
@@ -40,7 +47,7 @@ namespace {
 
 constexpr uint32_t kWaves = 8, kThreads = kWaves * kWave;
 constexpr uint32_t kTile = 16;        // weight rows per tile
-constexpr uint32_t kSlots = 8;        // activation rows held at a time
+constexpr uint32_t kMostRows = 8;     // rows of a record
 constexpr uint32_t kMaxTiles = 64;    // tiles per pass over the waves, if their pieces' sums fit
 constexpr uint32_t kPiece = 2;        // steps per piece
 constexpr uint32_t kMaxColumns = 2560;
@@ -50,13 +57,21 @@ constexpr uint32_t kPartialBytes = 20480;
 static_assert(kUnionScratchWords * 4 <= kPartialBytes, "the union build borrows the partial results' space");
 typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));  // 16 bytes at any even address
 
-enum Kind : int { K_Q4K = 0, K_Q6K = 1, K_Q8 = 2, K_Q51 = 3 };
+enum Kind : int { K_Q4K = 0, K_Q6K = 1, K_Q8 = 2, K_Q51 = 3, K_Q4K_F32 = 4 };
+constexpr bool is_q4(int kind) { return kind == K_Q4K || kind == K_Q4K_F32; }
 
+// slots: activation rows held at a time. Of f32 rows slot s < 4 has its three pieces in operand rows s, 4 + s and 12 + s, slot 4 in
+// rows 8, 9 and 10: the sums of a row's pieces meet across the lane quarters, resp. in the third quarter's own registers, the two
+// small ones first (sum_bytes: a slot's sums of a super-block, eight of each half, resp. of each piece). The minima are added up with the second pieces: apart from the largest sums, so that a block costs those one rounding.
 template <int KIND> struct Traits;
-template <> struct Traits<K_Q4K> { static constexpr uint32_t step = 256, block = 256, bytes = 128, stage = 2048 + 512; };
-template <> struct Traits<K_Q6K> { static constexpr uint32_t step = 256, block = 256, bytes = 128, stage = 2048 + 1024 + 512; };
-template <> struct Traits<K_Q8> { static constexpr uint32_t step = 128, block = 32, bytes = 32, stage = 2048 + 256; };
-template <> struct Traits<K_Q51> { static constexpr uint32_t step = 128, block = 32, bytes = 16, stage = 1024 + 256 + 512; };
+template <> struct Traits<K_Q4K> { static constexpr uint32_t step = 256, block = 256, bytes = 128, stage = 2048 + 512, slots = 8, sum_bytes = 32; };
+template <> struct Traits<K_Q4K_F32> { static constexpr uint32_t step = 256, block = 256, bytes = 128, stage = 2048 + 512, slots = 5, sum_bytes = 48; };
+template <> struct Traits<K_Q6K> { static constexpr uint32_t step = 256, block = 256, bytes = 128, stage = 2048 + 1024 + 512, slots = 8; };
+template <> struct Traits<K_Q8> { static constexpr uint32_t step = 128, block = 32, bytes = 32, stage = 2048 + 256, slots = 5; };
+template <> struct Traits<K_Q51> { static constexpr uint32_t step = 128, block = 32, bytes = 16, stage = 1024 + 256 + 768, slots = 5; };
+constexpr uint32_t kQ51SumBytes = 32;  // the slots' sums of a block: slots 0..3, zero, slot 4, two zeros
+
+template <int KIND> constexpr uint32_t q4_sum_bytes() { if constexpr (is_q4(KIND)) return Traits<KIND>::sum_bytes; else return 0; }
 
 struct StreamArgs {
     const float* x;            // rows of the product: tokens (gate/up) or routes (down), x_stride bytes apart
@@ -80,9 +95,9 @@ struct StreamArgs {
 
 // What a pass works on, worked out by the first wave and read by all.
 struct PassTable {
-    uint32_t item1, rows, tiles, pad;
-    uint64_t src[kSlots], dst[kSlots];  // a row's operand and result rows
-    float back[kSlots];                 // the power of two that takes a row's scaling off again
+    uint32_t item1, rows, tiles, next_row;  // next_row: where the pass after this one goes on in the same record, 0: with the next items
+    uint64_t src[kMostRows], dst[kMostRows];  // a row's operand and result rows
+    float back[kMostRows];                    // the power of two that takes a row's scaling off again
     u32x4 tile[kMaxTiles];              // expert's base (two words), first block, first slot | rows << 8 | tile within the expert << 16
 };
 
@@ -95,7 +110,7 @@ __host__ __device__ Layout layout_of(uint32_t columns) {
     Layout l;
     l.row_bytes = padded * 2 + 16;
     l.sums = 16 * l.row_bytes;
-    l.zero = l.sums + (KIND == K_Q4K ? kSlots * (padded / 256) * 32 : KIND == K_Q51 ? padded / 32 * kSlots * 4 : 0);
+    l.zero = l.sums + (is_q4(KIND) ? Traits<KIND>::slots * (padded / 256) * q4_sum_bytes<KIND>() : KIND == K_Q51 ? padded / 32 * kQ51SumBytes : 0);
     l.block = l.zero + 128;
     l.table = l.block + kBlockWords * 4;
     l.partial = l.table + sizeof(PassTable);
@@ -108,6 +123,8 @@ __host__ __device__ Layout layout_of(uint32_t columns) {
 template <int KIND, bool SWIGLU, uint32_t PIECES>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void record_stream(StreamArgs a) {
     using T = Traits<KIND>;
+    constexpr bool F32 = KIND != K_Q6K && KIND != K_Q4K, Q4 = is_q4(KIND);
+    constexpr uint32_t kSlots = T::slots;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const Layout at = layout_of<KIND>(a.k);
     const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -149,12 +166,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 
     // Lane l of the first wave looks after record k0 + l, then row slot l, then tile l. A record that does not check out has no
     // rows and reads expert 0: the batch is refused.
-    auto plan_pass = [&](uint32_t item0) {
+    // A record of more rows than slots makes passes of its own, over the same items with the rows from row0 on.
+    auto plan_pass = [&](uint32_t item0, uint32_t row0) {
         const uint32_t k0 = item0 / units, k = k0 + lane, index = k < 128 ? k : 0;
         const bool shared = a.shared_w0 != nullptr && k == live;
         uint32_t expert = shared ? 0 : block[8 + index], count = shared ? a.tokens : block[136 + index];
         if (k >= records) count = 0;
-        else if (count > kSlots || expert >= a.experts) { count = 0; expert = 0; bad |= TSP_ERRBIT_INDEX; }
+        else if (count > kMostRows || expert >= a.experts) { count = 0; expert = 0; bad |= TSP_ERRBIT_INDEX; }
+        const uint32_t first = __builtin_amdgcn_readlane(count, 0);
+        const bool split = first > kSlots;
         uint32_t upto = count;
 #pragma unroll
         for (uint32_t d = 1; d < kWave; d <<= 1) {
@@ -165,15 +185,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         const uint64_t fits = __builtin_amdgcn_ballot_w64(k * units < item1 && (lane == 0 || upto <= kSlots));
         const uint32_t taken = __builtin_ctzll(~fits);  // records of this pass: nearly always all of the share's
         if ((k0 + taken) * units < item1) item1 = (k0 + taken) * units;
-        const uint32_t rows = __builtin_amdgcn_readlane(upto, taken - 1);
-        const uint32_t room = kPartialBytes / 4 / ((rows ? rows : 1) * kTile * ppt * kMats);
+        const uint32_t whole = __builtin_amdgcn_readlane(upto, taken - 1), rows = !split ? whole : first - row0 < kSlots ? first - row0 : kSlots;
+        const uint32_t room = kPartialBytes / 4 / ((split ? kSlots : rows ? rows : 1) * kTile * ppt * kMats);  // the same for a record's passes
         if (item1 - item0 > room) item1 = item0 + room;
         const uint32_t tiles = (item1 - item0) * kMats;
-        if (lane == 0) { pass.item1 = item1; pass.rows = rows; pass.tiles = tiles; }
+        if (lane == 0) { pass.item1 = item1; pass.rows = rows; pass.tiles = tiles; pass.next_row = split && row0 + rows < first ? row0 + rows : 0; }
         // slot `lane` is row `in` of record k0 + q
         uint32_t q = 0;
         for (uint32_t i = 0; i < taken; ++i) q += uint32_t(__builtin_amdgcn_readlane(upto, i)) <= lane ? 1 : 0;
-        const uint32_t in = lane - (__shfl(upto, q, kWave) - __shfl(count, q, kWave));
+        const uint32_t in = lane - (__shfl(upto, q, kWave) - __shfl(count, q, kWave)) + row0;
         if (lane < kSlots && lane >= rows) pass.src[lane] = reinterpret_cast<uint64_t>(a.x);  // read and not used
         if (lane < rows) {
             const uint32_t rk = k0 + q, ri = rk < 128 ? rk : 0;
@@ -192,7 +212,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             base = (te < half_e ? a.w0 : a.w1) + (uint64_t(te < half_e ? te : te - half_e) * 2 + mat) * a.spec.planar_expert_bytes;
         } else base = a.w0 + uint64_t(te) * a.spec.planar_expert_bytes;
         const uint64_t bits = reinterpret_cast<uint64_t>(base);
-        if (lane < tiles) pass.tile[lane] = u32x4{uint32_t(bits), uint32_t(bits >> 32), unit * kTile * bpr, (tu - tc) | tc << 8 | unit << 16};
+        if (lane < tiles) pass.tile[lane] = u32x4{uint32_t(bits), uint32_t(bits >> 32), unit * kTile * bpr, (tu - tc) | (split ? rows : tc) << 8 | unit << 16};
     };
 
     // ---- request addresses: a uniform base per step plus these lane parts.
@@ -211,10 +231,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         }
         if constexpr (KIND == K_Q6K) q_lane[2] = uint32_t(a.spec.qh_offset) + lane / 4 * bpr * 64 + ((lane % 4) ^ (lane / 16)) * 16;
     }
-    if constexpr (KIND == K_Q4K || KIND == K_Q6K) {
+    if constexpr (Q4 || KIND == K_Q6K) {
         // lanes 0..15 (and 32..47) a row's scales, 16 bytes; the others the 16 bytes that END with its d (so that the last one
         // stays inside the expert)
-        constexpr uint32_t d_bytes = KIND == K_Q4K ? 4 : 2;
+        constexpr uint32_t d_bytes = Q4 ? 4 : 2;
         hdr_lane = lane & 16 ? uint32_t(a.spec.dm_offset) + (n16 * bpr + 1) * d_bytes - 16 : uint32_t(a.spec.sm_offset) + n16 * bpr * 16;
         hdr_step = lane & 16 ? d_bytes : 16;
     } else {
@@ -223,19 +243,27 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     // ---- fragment addresses (LDS): the lane's columns of operand row n16, and of the sums
     const uint32_t a_lane = n16 * at.row_bytes + (KIND == K_Q4K ? kq * 128 : KIND == K_Q6K ? kq / 2 * 256 + kq % 2 * 32 : kq * 16);
     uint32_t s_lane = at.zero, s_step = 0;
-    if constexpr (KIND == K_Q4K) {
-        if (n16 < 8 && kq < 2) { s_lane = at.sums + n16 * ((at.row_bytes - 16) / 512) * 32 + kq * 16; s_step = 32; }
+    if constexpr (KIND == K_Q4K) {  // the high-half rows; the others get zeros
+        if (n16 < 8 && kq < 2) { s_lane = at.sums + n16 * ((at.row_bytes - 16) / 512) * T::sum_bytes + kq * 16; s_step = T::sum_bytes; }
+    } else if constexpr (KIND == K_Q4K_F32) {  // the rows of the second pieces
+        if (kq < 3 && ((n16 >= 4 && n16 < 8) || n16 == 9)) {
+            s_lane = at.sums + (n16 < 8 ? n16 - 4 : 4) * ((at.row_bytes - 16) / 512) * T::sum_bytes + kq * 16;
+            s_step = T::sum_bytes;
+        }
     } else if constexpr (KIND == K_Q51) {
-        if (kq < 2) { s_lane = at.sums + kq * 16; s_step = 4 * kSlots * 4; }
+        if (kq == 1 || kq == 2) { s_lane = at.sums + (kq - 1) * 16; s_step = 4 * kQ51SumBytes; }
     }
+
     const Q4Consts q4c = q4_consts();
     Q4ScaleConsts q4s = q4_scale_consts();
     const uint32_t q4_sel = kq & 1 ? 0x04030402u : 0x04010400u;
 
+    uint32_t row0 = 0;
     for (uint32_t item0 = items * blockIdx.x / gridDim.x; item0 < share1;) {
-        if (wave == 0) plan_pass(item0);
+        if (wave == 0) plan_pass(item0, row0);
         lds_barrier();
         const uint32_t item1 = __builtin_amdgcn_readfirstlane(pass.item1), rows = __builtin_amdgcn_readfirstlane(pass.rows), tiles = __builtin_amdgcn_readfirstlane(pass.tiles);
+        row0 = __builtin_amdgcn_readfirstlane(pass.next_row);  // of the next pass
         const uint32_t stride = rows * kTile, pieces = tiles * ppt, each = (pieces + kWaves - 1) / kWaves;
         const uint32_t p0 = wave * each < pieces ? wave * each : pieces, p1 = p0 + each < pieces ? p0 + each : pieces;
         const uint32_t tile0 = p0 / ppt, tile1 = p1 / ppt;
@@ -266,7 +294,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             st.q[0] = global_at<u32x4>(q, q_lane[0]);
             if constexpr (KIND != K_Q51) st.q[1] = global_at<u32x4>(q, q_lane[1]);
             if constexpr (KIND == K_Q6K) st.q[2] = global_at<u32x4>(f_base + uint64_t(b) * 64, q_lane[2]);
-            if constexpr (KIND == K_Q4K || KIND == K_Q6K) {
+            if constexpr (Q4 || KIND == K_Q6K) {
                 st.hdr = global_at<u32x4_any>(f_base, hdr_lane + b * hdr_step);
             } else {
                 uint32_t e = hdr_lane + b;
@@ -290,7 +318,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         for (uint32_t i = 0; i < kDepth; ++i) fetch(st[i]);
         __builtin_amdgcn_sched_barrier(0);  // everything is requested before the first wait
 
-        // ---- the row becomes an operand row of high halves and one of low halves
+        // ---- the row becomes its operand rows
         if (wave < rows) {
             float biggest = 0;
 #pragma unroll
@@ -300,46 +328,60 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                 biggest = fmaxf(biggest, fmaxf(fmaxf(fabsf(row[j].x), fabsf(row[j].y)), fmaxf(fabsf(row[j].z), fabsf(row[j].w))));
             }
             biggest = wave_largest(biggest);
-            // scale = 2^(13 - exponent(biggest)): the largest |x * scale| is below 2^14, the sub-block sums / 32 as well
-            float scale = 1.0f, inv_scale = 1.0f;
-            if (biggest > 0 && !nonfinite(biggest)) {
-                int shift = 13 - (int((__float_as_uint(biggest) >> 23) & 0xffu) - 127);
+            int shift = 0;
+            if constexpr (F32) {
+                shift = row_lift(biggest);
+            } else if (biggest > 0 && !nonfinite(biggest)) {  // the largest |x * scale| comes to just below 2^14
+                shift = 13 - (int((__float_as_uint(biggest) >> 23) & 0xffu) - 127);
                 shift = shift > 100 ? 100 : shift < -100 ? -100 : shift;
-                scale = __uint_as_float(uint32_t(127 + shift) << 23);
-                inv_scale = __uint_as_float(uint32_t(127 - shift) << 23);
             }
-            if (lane == 0) pass.back[wave] = inv_scale;
-            uint8_t* const hi_at = lds + wave * at.row_bytes + lane * 8;
-            uint8_t* const lo_at = hi_at + 8 * at.row_bytes;
+            const float scale = power_of_two(shift);
+            if (lane == 0) pass.back[wave] = power_of_two(-shift);
+            uint8_t* const at0 = lds + (!F32 || wave < 4 ? wave : 8) * at.row_bytes + lane * 8;  // of the first piece; the others follow at
+            const uint32_t second = (!F32 ? 8 : wave < 4 ? 4 : 1) * at.row_bytes, third = (wave < 4 ? 12 : 2) * at.row_bytes;
 #pragma unroll
             for (uint32_t j = 0; j < PIECES; ++j) {
                 if (j * 256 >= a.k) break;
                 const float s4[4] = {row[j].x * scale, row[j].y * scale, row[j].z * scale, row[j].w * scale};
-                _Float16 hi[4], lo[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) { hi[e] = _Float16(s4[e]); lo[e] = _Float16(s4[e] - float(hi[e])); }
-                if constexpr (KIND == K_Q4K) {  // the order in which a dword of nibbles unpacks
-                    *reinterpret_cast<f16x4*>(hi_at + j * 512) = f16x4{hi[0], hi[2], hi[1], hi[3]};
-                    *reinterpret_cast<f16x4*>(lo_at + j * 512) = f16x4{lo[0], lo[2], lo[1], lo[3]};
+                uint8_t* const here = at0 + j * 512;
+                if constexpr (F32) {
+                    const Pieces p[4] = {three_pieces(s4[0]), three_pieces(s4[1]), three_pieces(s4[2]), three_pieces(s4[3])};
+                    *reinterpret_cast<uint2*>(here) = uint2{two_tops(p[0].hi, p[1].hi), two_tops(p[2].hi, p[3].hi)};
+                    *reinterpret_cast<uint2*>(here + second) = uint2{two_tops(p[0].mid, p[1].mid), two_tops(p[2].mid, p[3].mid)};
+                    *reinterpret_cast<uint2*>(here + third) = uint2{two_tops(p[0].lo, p[1].lo), two_tops(p[2].lo, p[3].lo)};
                 } else {
-                    *reinterpret_cast<f16x4*>(hi_at + j * 512) = f16x4{hi[0], hi[1], hi[2], hi[3]};
-                    *reinterpret_cast<f16x4*>(lo_at + j * 512) = f16x4{lo[0], lo[1], lo[2], lo[3]};
+                    _Float16 hi[4], lo[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) { hi[e] = _Float16(s4[e]); lo[e] = _Float16(s4[e] - float(hi[e])); }
+                    constexpr int I1 = KIND == K_Q4K ? 2 : 1, I2 = 3 - I1;  // Q4_K: the order in which a dword of nibbles unpacks
+                    *reinterpret_cast<f16x4*>(here) = f16x4{hi[0], hi[I1], hi[I2], hi[3]};
+                    *reinterpret_cast<f16x4*>(here + second) = f16x4{lo[0], lo[I1], lo[I2], lo[3]};
                 }
-                if constexpr (KIND == K_Q4K || KIND == K_Q51) {
+                if constexpr (Q4 || KIND == K_Q51) {
                     const float sum = octet_sum((s4[0] + s4[1]) + (s4[2] + s4[3]));  // eight lanes hold 32 columns
                     if (lane % 8 == 0) {
-                        if constexpr (KIND == K_Q4K) {
-                            _Float16* o = reinterpret_cast<_Float16*>(lds + at.sums) + (wave * ((at.row_bytes - 16) / 512) + j) * 16 + lane / 8;
-                            const float s32 = sum * 0.03125f;
-                            const _Float16 h = _Float16(s32);
-                            o[0] = h;
-                            o[8] = _Float16(s32 - float(h));
+                        if constexpr (Q4) {
+                            uint16_t* o = reinterpret_cast<uint16_t*>(lds + at.sums + (wave * ((at.row_bytes - 16) / 512) + j) * T::sum_bytes) + lane / 8;
+                            if constexpr (F32) {
+                                const Pieces p = three_pieces(sum);
+                                o[0] = uint16_t(__float_as_uint(p.hi) >> 16);
+                                o[8] = uint16_t(__float_as_uint(p.mid) >> 16);
+                                o[16] = uint16_t(__float_as_uint(p.lo) >> 16);
+                            } else {
+                                const float s32 = sum * 0.03125f;
+                                const _Float16 high = _Float16(s32);
+                                o[0] = __builtin_bit_cast(uint16_t, high);
+                                o[8] = __builtin_bit_cast(uint16_t, _Float16(s32 - float(high)));
+                            }
                         } else {
-                            reinterpret_cast<float*>(lds + at.sums)[(j * 8 + lane / 8) * kSlots + wave] = sum;
+                            *reinterpret_cast<float*>(lds + at.sums + (j * 8 + lane / 8) * kQ51SumBytes + (wave < 4 ? wave : 5) * 4) = sum;
                         }
                     }
                 }
             }
+        } else if (KIND == K_Q51 && wave >= kSlots) {  // the first and third piece of slot 4 and the row after them
+            const uint32_t none = wave == kSlots ? 4 : wave;
+            for (uint32_t i = lane; i < (at.zero - at.sums) / kQ51SumBytes; i += kWave) *reinterpret_cast<float*>(lds + at.sums + i * kQ51SumBytes + none * 4) = 0;
         }
         lds_barrier();
 
@@ -347,22 +389,36 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         uint32_t c_step = s0 - tile0 * spt;
         uint32_t a_at = a_lane + c_step * (T::step * 2), s_at = s_lane + c_step * s_step;
         f32x4 acc{};
-        float* out = partial + p0 * stride + kq * 4 * kTile + n16;
-        auto leave_piece = [&]() {  // low-half rows 8..15 (lanes 32..63) join the high-half rows; then lanes 0..31 hold rows 4 kq + v of column n16
+        float* out = partial + p0 * stride + (F32 ? 0 : kq * 4 * kTile) + n16;
+        auto leave_piece = [&]() {
+            auto halves_sum = [](float v) {  // over lanes l and l ^ 32
+                const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+                return __uint_as_float(both[0]) + __uint_as_float(both[1]);
+            };
+            if constexpr (F32) {
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const uint32_t bits = __float_as_uint(acc[v]);
-                const auto halves = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
-                const float both = __uint_as_float(halves[0]) + __uint_as_float(halves[1]);
-                if (lane < 32 && kq * 4 + v < rows) out[v * kTile] = both;
+                for (int v = 0; v < 4; ++v) {  // slot v: lanes 0..15 get first + (second + third)
+                    const float outer = halves_sum(kq == 2 ? 0.0f : acc[v]);
+                    const auto quarters = __builtin_amdgcn_permlane16_swap(__float_as_uint(outer), __float_as_uint(outer), false, false);
+                    const float all = __uint_as_float(quarters[0]) + __uint_as_float(quarters[1]);
+                    if (kq == 0 && v < rows) out[v * kTile] = all;
+                }
+                if (kq == 2 && rows > 4) out[4 * kTile] = acc[0] + (acc[1] + acc[2]);  // in the same order
+            } else {  // low-half rows 8..15 (lanes 32..63) join the high-half rows; then lanes 0..31 hold rows 4 kq + v of column n16
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const float both = halves_sum(acc[v]);
+                    if (lane < 32 && kq * 4 + v < rows) out[v * kTile] = both;
+                }
             }
             acc = f32x4{};
             out += stride;
         };
         auto operand = [&](uint32_t bytes) { return *reinterpret_cast<const f16x8*>(lds + a_at + bytes); };
+        auto exact_operand = [&](uint32_t bytes) { return *reinterpret_cast<const bf16x8*>(lds + a_at + bytes); };
         auto body = [&](Stage& cur) {
-            // registers -> LDS, and the stage is free for the step kDepth ahead
-            if constexpr (KIND == K_Q4K || KIND == K_Q6K) {
+            // registers -> LDS, and the stage is free for the step kDepth ahead (past the row's end the scales are another row's, and stay out)
+            if constexpr (Q4 || KIND == K_Q6K) {
                 *reinterpret_cast<u32x4*>(stage_lds + lane * 16) = cur.q[0];
                 *reinterpret_cast<u32x4*>(stage_lds + 1024 + lane * 16) = cur.q[1];
                 if constexpr (KIND == K_Q6K) *reinterpret_cast<u32x4*>(stage_lds + 2048 + lane * 16) = cur.q[2];
@@ -370,12 +426,18 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             } else if constexpr (KIND == K_Q8) {
                 *reinterpret_cast<u32x4*>(stage_lds + lane * 16) = cur.q[0];
                 *reinterpret_cast<u32x4*>(stage_lds + 1024 + lane * 16) = cur.q[1];
-                *reinterpret_cast<float*>(stage_lds + 2048 + (n16 * 4 + kq) * 4) = half_bits_to_float(cur.hdr[0]);
+                *reinterpret_cast<float*>(stage_lds + 2048 + (n16 * 4 + kq) * 4) = c_step * 4 + kq < bpr ? half_bits_to_float(cur.hdr[0]) : 0.0f;
             } else {
                 *reinterpret_cast<u32x4*>(stage_lds + lane * 16) = cur.q[0];
                 *reinterpret_cast<uint32_t*>(stage_lds + 1024 + (n16 * 4 + kq) * 4) = cur.hdr[0];
-                *reinterpret_cast<float*>(stage_lds + 1280 + (n16 * 4 + kq) * 4) = half_bits_to_float(cur.hdr[1] & 0xffffu);
-                *reinterpret_cast<float*>(stage_lds + 1536 + (n16 * 4 + kq) * 4) = half_bits_to_float(cur.hdr[1] >> 16);
+                // d q + m = d (q - c) + (m + c d) with the code c that comes nearest to zero: neither part is larger than the weight by
+                // more than d / 2, so the two sums lose no more than the weights' own would
+                const float d = half_bits_to_float(cur.hdr[1] & 0xffffu), least = half_bits_to_float(cur.hdr[1] >> 16);
+                const float c = fminf(fmaxf(__builtin_rintf(-least * __builtin_amdgcn_rcpf(d)), 0.0f), 31.0f);
+                const bool inside = c_step * 4 + kq < bpr;
+                *reinterpret_cast<float*>(stage_lds + 1280 + (n16 * 4 + kq) * 4) = inside ? d : 0.0f;
+                *reinterpret_cast<float*>(stage_lds + 1536 + (n16 * 4 + kq) * 4) = inside ? __builtin_fmaf(c, d, least) : 0.0f;
+                *reinterpret_cast<uint32_t*>(stage_lds + 1792 + (n16 * 4 + kq) * 4) = uint32_t(c) * 0x01010101u;
             }
             fetch(cur);
             const f32x4 zero{};
@@ -409,6 +471,27 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                 const float d = half_bits_to_float(dm & 0xffffu), dmin = -32.0f * half_bits_to_float(dm >> 16);
 #pragma unroll
                 for (int v = 0; v < 4; ++v) acc[v] = __builtin_fmaf(dmin, mins[v], __builtin_fmaf(d, blk[v], acc[v]));
+            } else if constexpr (KIND == K_Q4K_F32) {
+                const uint32_t swz = n16 / 2;
+                const u32x4 sm = *reinterpret_cast<const u32x4*>(stage_lds + 2048 + n16 * 16);
+                const uint32_t dm = *reinterpret_cast<const uint32_t*>(stage_lds + 2048 + 256 + n16 * 16 + 12);
+                const float d = half_bits_to_float(dm & 0xffffu), dmin = -half_bits_to_float(dm >> 16);
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {  // sub-blocks 2 p (low nibbles) and 2 p + 1: lane kq has weights 8 kq .. 8 kq + 7 of each
+                    const uint2 q = *reinterpret_cast<const uint2*>(stage_lds + n16 * 128 + ((2 * p + kq / 2) ^ swz) * 16 + kq % 2 * 8);
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const bf16x8 f = nibbles8_bf16((q.x >> (4 * h)) & 0x0f0f0f0fu, (q.y >> (4 * h)) & 0x0f0f0f0fu);
+                        const f32x4 sub = __builtin_amdgcn_mfma_f32_16x16x32_bf16(exact_operand((2 * p + h) * 64), f, zero, 0, 0, 0);
+                        const float scale = d * float((sm[p / 2] >> (p % 2 * 16 + h * 8)) & 0xffu);
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) acc[v] = __builtin_fmaf(scale, sub[v], acc[v]);
+                    }
+                }
+                // minima: operand columns 8 i .. 8 i + 7 are the i-th pieces of the sums, the last eight and all other rows zero
+                const f32x4 mins = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(lds + s_at), codes8_bf16(sm[2], sm[3]), zero, 0, 0, 0);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[v] = __builtin_fmaf(dmin, mins[v], acc[v]);
             } else if constexpr (KIND == K_Q6K) {
                 const uint32_t sec = kq / 2, half = kq % 2, swz = n16 / 2;
                 RawQ6 raw;
@@ -438,29 +521,27 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {  // a block is one instruction: lane kq has quants 8 kq .. 8 kq + 7
                     const uint2 q = *reinterpret_cast<const uint2*>(stage_lds + n16 * 128 + ((2 * j + kq / 2) ^ swz) * 16 + kq % 2 * 8);
-                    const f32x4 blk = __builtin_amdgcn_mfma_f32_16x16x32_f16(operand(j * 64), quants8(q.x, q.y), zero, 0, 0, 0);
+                    const f32x4 blk = __builtin_amdgcn_mfma_f32_16x16x32_bf16(exact_operand(j * 64), quants8_bf16(q.x, q.y), zero, 0, 0, 0);
 #pragma unroll
                     for (int v = 0; v < 4; ++v) acc[v] = __builtin_fmaf(d[j], blk[v], acc[v]);
                 }
             } else {
                 const u32x4 qh = *reinterpret_cast<const u32x4*>(stage_lds + 1024 + n16 * 16);
                 const f32x4 d = *reinterpret_cast<const f32x4*>(stage_lds + 1280 + n16 * 16), m = *reinterpret_cast<const f32x4*>(stage_lds + 1536 + n16 * 16);
+                const u32x4 nearest = *reinterpret_cast<const u32x4*>(stage_lds + 1792 + n16 * 16);
                 const uint32_t swz = n16 / 4;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     // lane kq has weights 8 kq .. 8 kq + 7: low nibbles of the first or second eight bytes for kq < 2, then the high ones
                     const uint2 q = *reinterpret_cast<const uint2*>(stage_lds + n16 * 64 + (j ^ swz) * 16 + kq % 2 * 8);
                     const uint32_t fifth = qh[j] >> (8 * kq);
-                    // bit i of the eight goes to bit 4 of byte i % 4
+                    // bit i of the eight goes to bit 4 of byte i % 4; a byte's code is then 128 more until c is off it
                     const uint32_t f0 = ((fifth & 15u) * 0x00204081u & 0x01010101u) << 4, f1 = ((fifth >> 4 & 15u) * 0x00204081u & 0x01010101u) << 4;
-                    const uint32_t w0 = (q.x >> (kq / 2 * 4) & 0x0f0f0f0fu) | f0, w1 = (q.y >> (kq / 2 * 4) & 0x0f0f0f0fu) | f1;
-                    constexpr uint32_t K = 0x64646464u;  // 1024 + code
-                    const f16x2 off = splat(-1024.0f);
-                    const f16x2 c0 = as_h2(spread01(w0, K)) + off, c1 = as_h2(spread23(w0, K)) + off, c2 = as_h2(spread01(w1, K)) + off, c3 = as_h2(spread23(w1, K)) + off;
-                    const f16x8 f{c0[0], c0[1], c1[0], c1[1], c2[0], c2[1], c3[0], c3[1]};
-                    const f32x4 blk = __builtin_amdgcn_mfma_f32_16x16x32_f16(operand(j * 64), f, zero, 0, 0, 0);
-                    // the block's minimum times its rows' sums: the high-half rows only (the low-half rows read zeros)
-                    const f32x4 s = *reinterpret_cast<const f32x4*>(lds + s_at + j * (kSlots * 4));
+                    const uint32_t w0 = (((q.x >> (kq / 2 * 4) & 0x0f0f0f0fu) | f0 | 0x80808080u) - nearest[j]) ^ 0x80808080u;
+                    const uint32_t w1 = (((q.y >> (kq / 2 * 4) & 0x0f0f0f0fu) | f1 | 0x80808080u) - nearest[j]) ^ 0x80808080u;
+                    const f32x4 blk = __builtin_amdgcn_mfma_f32_16x16x32_bf16(exact_operand(j * 64), quants8_bf16(w0, w1), zero, 0, 0, 0);
+                    // the block's minimum times its rows' sums: once per row (the operand rows of the other pieces read zeros)
+                    const f32x4 s = *reinterpret_cast<const f32x4*>(lds + s_at + j * kQ51SumBytes);
 #pragma unroll
                     for (int v = 0; v < 4; ++v) acc[v] = __builtin_fmaf(m[j], s[v], __builtin_fmaf(d[j], blk[v], acc[v]));
                 }
@@ -501,7 +582,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             }
             reinterpret_cast<float __attribute__((address_space(1)))*>(pass.dst[slot])[n] = value;
         }
-        item0 = item1;
+        if (row0 == 0) item0 = item1;
         if (item0 < share1) __syncthreads();  // the table, the rows and the partial results are taken over by the next pass
     }
     publish_error(bad, a.error_word);
@@ -538,9 +619,12 @@ int launch_pieces(const char* name, const StreamArgs& a, hipStream_t s) {
 
 template <int KIND, bool SWIGLU>
 int launch(const char* name, const StreamArgs& a, hipStream_t s) {
-    if (a.k <= 4 * 256) return launch_pieces<KIND, SWIGLU, 4>(name, a, s);
-    if (a.k <= 8 * 256) return launch_pieces<KIND, SWIGLU, 8>(name, a, s);
-    return launch_pieces<KIND, SWIGLU, kMaxColumns / 256>(name, a, s);
+    constexpr bool narrow = KIND != K_Q4K_F32, wide = KIND != K_Q4K && KIND != K_Q6K;  // up to 2048 columns, beyond
+    if constexpr (narrow) {
+        if (a.k <= 4 * 256) return launch_pieces<KIND, SWIGLU, 4>(name, a, s);
+        if (!wide || a.k <= 8 * 256) return launch_pieces<KIND, SWIGLU, 8>(name, a, s);
+    }
+    if constexpr (wide) return launch_pieces<KIND, SWIGLU, kMaxColumns / 256>(name, a, s);
 }
 
 bool aligned16(const void* p, uint64_t stride) { return reinterpret_cast<uintptr_t>(p) % 16 == 0 && stride % 16 == 0; }
@@ -550,7 +634,7 @@ bool aligned16(const void* p, uint64_t stride) { return reinterpret_cast<uintptr
 namespace tsp {
 
 bool record_stream_gate_up_takes(const SkinnyMoe& m) {
-    return m.gu.source_type == 12 && m.channels <= kMaxColumns && m.gu.planar_expert_bytes < (1ull << 32) && aligned16(m.x, m.x_stride) && m.tokens <= kSlots && m.hidden % kTile == 0;
+    return m.gu.source_type == 12 && m.channels <= kMaxColumns && m.gu.planar_expert_bytes < (1ull << 32) && aligned16(m.x, m.x_stride) && m.tokens <= kMostRows && m.hidden % kTile == 0;
 }
 
 int launch_record_stream_gate_up(const SkinnyMoe& m, hipStream_t s) {
@@ -562,12 +646,14 @@ int launch_record_stream_gate_up(const SkinnyMoe& m, hipStream_t s) {
         a.shared_w0 = m.shared_gate; a.shared_w1 = m.shared_up; a.shared_x = m.x; a.shared_x_stride = m.x_stride;
         a.shared_out = m.shared_h; a.shared_out_stride = m.shared_h_stride;
     }
-    return launch<K_Q4K, true>("record_gate_up_swiglu", a, s);
+    // Q4_K rows of more columns than the kernels in halves take keep f32 rows
+    return m.channels > 2048 ? launch<K_Q4K_F32, true>("record_gate_up_swiglu", a, s) : launch<K_Q4K, true>("record_gate_up_swiglu", a, s);
 }
 
 bool record_stream_down_takes(const SkinnyMoe& m) {
-    return (m.dn.source_type == 8 || m.dn.source_type == 7 || m.dn.source_type == 14) && m.hidden <= kMaxColumns && m.dn.planar_expert_bytes < (1ull << 32) &&
-           aligned16(m.h, m.h_stride) && m.tokens <= kSlots && m.channels % kTile == 0;
+    // Q6_K in halves only as far as its other widths are (skinny.hip): beyond, the per-element kernel keeps the rows in f32
+    return (m.dn.source_type == 8 || m.dn.source_type == 7 || (m.dn.source_type == 14 && m.hidden <= 2048)) && m.hidden <= kMaxColumns && m.dn.planar_expert_bytes < (1ull << 32) &&
+           aligned16(m.h, m.h_stride) && m.tokens <= kMostRows && m.channels % kTile == 0;
 }
 
 int launch_record_stream_down(const SkinnyMoe& m, hipStream_t s) {
