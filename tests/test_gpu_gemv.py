@@ -293,8 +293,8 @@ def test_dense_mm_q8_staged_tiles(gpu, tsp, synth, tokens, cols, rows):
                                                   (23, 2560, 48, 0), (3, 96, 20, 0), (6, 512, 24640, 0), (15, 512, 14020, 0), (11, 1280, 14001, 0),
                                                   (7, 2560, 24577, 0), (14, 2560, 14004, 0), (27, 1024, 14004, 0), (41, 192, 30, 4)])
 def test_dense_mm_q8_few_rows(gpu, tsp, orc, synth, tokens, cols, rows, pad):
-    # every kernel that a few raw Q8_0 token rows can go to: 16-row tiles (any multiple of 64 columns, rows any distance apart), the
-    # persistent kernel from 24 576 rows on (14 000 at nine tokens) with eight and sixteen token rows, decoded weights below that
+    # every kernel that a few raw Q8_0 token rows can go to: 16-row tiles (any multiple of 64 columns, rows any distance apart), up to 2048
+    # columns the persistent kernel from 24 576 rows on (14 000 at nine tokens) with eight and sixteen token rows
     w = synth.matrix(8, 2200 + cols, rows, cols)
     x = synth.activations_f32(2201 + tokens, (tokens, cols + pad))
     x[0] *= 1e-20
@@ -392,3 +392,32 @@ def test_gemv_tiny_activations(gpu, orc, synth, t, cols, exponent):
     bound = (np.abs(dense) * np.abs(x.astype(np.float64).reshape(-1, 32)).max(axis=1).repeat(32)).sum(axis=1) * (2.0 ** -23 + 2.0 ** -22) + cols * 2.0 ** -147
     got = gpu.gemv(t, gpu.upload(w), gpu.upload(x), cols, rows).cpu().numpy().astype(np.float64)
     assert (np.abs(got - dense @ x.astype(np.float64)) <= bound).all() and gpu.error() == 0
+
+
+@pytest.mark.parametrize("lanes,tokens,cols,rows,pad", [(False, 2, 64, 1, 0), (False, 7, 640, 33, 0), (False, 8, 2560, 640, 0), (False, 9, 320, 18, 0), (False, 16, 1088, 47, 12),
+                                                        (False, 5, 2048, 160, 4), (False, 21, 512, 30, 4), (False, 1, 2560, 40004, 0), (False, 5, 2560, 60001, 0),
+                                                        (False, 8, 2560, 60000, 0), (False, 16, 2560, 25000, 0), (False, 13, 2304, 60000, 0), (True, 1, 2560, 16, 0), (True, 5, 2560, 1003, 0),
+                                                        (True, 8, 2560, 4100, 0), (True, 16, 2560, 512, 0)])
+def test_dense_mm_q8_f32_rows(gpu, tsp, orc, synth, lanes, tokens, cols, rows, pad):
+    """Few token rows of up to 16 rows' tiles, and any of more than 2048 columns, are multiplied as the floats they are: 3e4 to 1e30 in front
+    of weights that are zero, one in each 32, take nothing from the values beside them, nor does one row from another. Error
+    bound: a block's sum in at most 12 roundings, 80 blocks or waves' sums one each: less than 2^-17 of sum |w x|."""
+    w = synth.matrix(8, 2600 + cols, rows, cols)
+    zero_columns(8, w, rows, cols)
+    x = synth.activations_f32(2601 + tokens, (tokens, cols + pad))
+    x[:, 5:cols:32] = np.resize(np.array([3e4, -1e12, 1e30], dtype=np.float32), (tokens, cols // 32))
+    x[0] *= np.float32(1e-37) if tokens > 1 else np.float32(1)
+    matrix = tsp.q8_lanes_pack_rows(cols, w) if lanes else w
+    check = np.unique(np.r_[0:min(rows, 300), max(0, rows - 40):rows])
+    dense = orc.dequantize(8, np.ascontiguousarray(w.reshape(rows, -1)[check]).reshape(-1), len(check) * cols).reshape(len(check), cols).astype(np.float64)
+    out = gpu.full((tokens, rows + pad), -5.0)
+    tsp.dense_mm_q8(gpu, tsp.LAYOUT_Q8_LANES_V1 if lanes else tsp.LAYOUT_GGUF, gpu.upload(matrix), gpu.upload(x), tokens, cols, rows, out=out,
+                    x_stride=(cols + pad) * 4, out_stride=(rows + pad) * 4)
+    got, x = out.cpu().numpy(), x[:, :cols].astype(np.float64)
+    bound = 2.0 ** -17 * (np.abs(x) @ np.abs(dense).T) + cols * 2.0 ** -149
+    assert gpu.error() == 0 and (got[:, rows:] == -5.0).all()
+    assert (np.abs(got[:, check] - x @ dense.T) <= bound).all(), float(np.max(np.abs(got[:, check] - x @ dense.T) / bound))
+    x = np.ascontiguousarray(x, dtype=np.float32)
+    x[tokens // 2, cols - 1] = np.nan
+    tsp.dense_mm_q8(gpu, tsp.LAYOUT_Q8_LANES_V1 if lanes else tsp.LAYOUT_GGUF, gpu.upload(matrix), gpu.upload(x), tokens, cols, rows)
+    assert gpu.error() == tsp.ERRBIT_NONFINITE

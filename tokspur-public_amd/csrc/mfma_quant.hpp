@@ -91,8 +91,9 @@ __device__ __forceinline__ f16x8 quants8(uint32_t w0, uint32_t w1) {
 // A float is three bf16 values, its top eight significant bits, the next eight and the last eight: cut off the top, subtract, again.
 // Every step is exact and the pieces have a float's own exponent range, so three products with the same integer weights, summed
 // in f32, are the f32 product whatever else is in the row. (Two halves under a power of two per row carry 22 bits, and fewer for
-// what is far below the row's largest value.) Pieces below 2^-133 are cut off: `row_lift` keeps ordinary rows away from there, and
-// from sums that overflow before the block's scale has been applied. It takes the exponent that a row's largest magnitude has.
+// what is far below the row's largest value.) Pieces below 2^-133 are cut off: `row_lift` is the power of two that brings a row's largest
+// magnitude to 2^80 (by 120 binades at most, which is enough for subnormals), so that only what is 2^-189 of it loses bits, and
+// sums that the blocks' scales, up to 2^22, have yet to meet stay finite.
 __device__ __forceinline__ float top_bits(float v) { return __uint_as_float(__float_as_uint(v) & 0xffff0000u); }
 struct Pieces { float hi, mid, lo; };  // the upper 16 bits of each
 __device__ __forceinline__ Pieces three_pieces(float v) {
@@ -100,7 +101,10 @@ __device__ __forceinline__ Pieces three_pieces(float v) {
     return Pieces{v, rest, rest - top_bits(rest)};
 }
 __device__ __forceinline__ uint32_t two_tops(float a, float b) { return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u); }
-__device__ __forceinline__ int row_lift(float biggest) { return biggest >= 0x1p64f ? -64 : biggest < 0x1p-40f ? 64 : 0; }
+__device__ __forceinline__ int row_lift(float biggest) {
+    const int up = 80 + 127 - int((__float_as_uint(biggest) >> 23) & 0xffu);
+    return up > 120 ? 120 : up;
+}
 __device__ __forceinline__ float power_of_two(int e) { return __uint_as_float(uint32_t(127 + e) << 23); }
 
 // Integers of at most eight bits as exact bf16: eight int8 quants, or eight codes 0 .. 255 (one per byte of w0, w1).

@@ -171,12 +171,18 @@ int launch(uint32_t layout, const Q8Args& a, hipStream_t stream) {
 }
 
 // Two to sixteen token rows against raw rows: a workgroup per 16 matrix rows (q8_small.hip), or the persistent kernel (q8_mfma.hip).
-// The latter's time hardly falls below 24 us (2048 columns; 17 at nine tokens or more) however few the rows, the former's is
-// proportional to them: 15.6 against 24.6 us at 16 000 x 2048, 28.8 against 25.0 at 32 000, at 1024 columns 20 against 16;
-// with nine or more tokens 6.5 against 17.3 at 4096, 21 against 18.6 at 16 000. Widths that the latter refuses all go to the former.
+// The latter's time hardly falls below a floor however few the rows, 25 us at 2048 columns and 14 at 1024 (17 and 12 at nine tokens
+// or more), the former's is proportional to them: 16.1 us at 16 000 x 2048, 24.5 against 25.0 at 24 576, 31 against 25 at 32 000; at
+// 1024 columns 11.2 us at 16 000, 16 against 16 at 24 576; with nine or more tokens 17 at 12 000 x 2048, 24 against 18 at 16 000. Of more
+// than 2048 columns the persistent kernel takes ten token rows a pass (2560 columns) or five: 27 us against 35 at 24 576 x 2560, 37
+// against 36 at 32 000; two passes for sixteen tokens 56 against 75 at 32 000, 78 against 80 at 40 000, 124 against 88 at 64 000.
+// Widths that it refuses all go to the former.
 bool small_rows(const void* matrix, const float* x, uint64_t x_stride_bytes, uint32_t columns, uint32_t rows, uint32_t tokens) {
-    return q8_small_takes(matrix, x, x_stride_bytes, columns, rows) &&
-           (rows < (tokens > 8 ? 14000u : 24576u) || x_stride_bytes != uint64_t(columns) * 4 || !q8_mfma_supported(matrix, x, columns, rows));
+    if (!q8_small_takes(matrix, x, x_stride_bytes, columns, rows)) return false;
+    if (x_stride_bytes != uint64_t(columns) * 4 || !q8_mfma_supported(matrix, x, columns, rows)) return true;
+    if (columns <= 2048) return rows < (tokens > 8 ? 14000u : 24576u);
+    const uint32_t at_once = columns % 512 == 0 && rows % 4 == 0 ? 10 : 5;
+    return rows < (tokens > 8 ? 22000u : 31000u) * ((tokens + at_once - 1) / at_once);
 }
 
 }  // namespace
@@ -196,7 +202,7 @@ extern "C" int tsp_q8_matvec_many(uint32_t layout, const void* matrix, uint64_t 
     if (layout == TSP_LAYOUT_GGUF && width > 1 && small_rows(matrix, x, uint64_t(columns) * 4, columns, rows, width))
         return q8_small(matrix, x, uint64_t(columns) * 4, y, uint64_t(rows) * 4, columns, rows, width, error_word, s);
     // One row against a matrix of less than 100 MB, or of a width the persistent matrix-core kernel does not take: that kernel's
-    // eight waves per compute unit share out 32-row tiles, of which there are too few (at 4096 x 2048 20.3 us, 5.2 here; at
+    // eight waves per compute unit share out 32-row tiles, of which there are too few (at 4096 x 2048 20.3 us, 4.4 here; at
     // 60 000 x 2048, 130 MB, 32.2 and 33.6)
     if (layout == TSP_LAYOUT_GGUF && width == 1 && (matrix_bytes < 100000000 || !q8_mfma_supported(matrix, x, columns, rows))) {
         bool taken = false;

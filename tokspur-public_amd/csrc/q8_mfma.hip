@@ -6,7 +6,9 @@
 // of them repeated when there are only eight). The block's scale multiplies the f32 result once (4 fused multiply-adds per
 // lane and 16 weight rows). The activations are scaled by a power of two and split into hi + lo halves, staged once in
 // LDS for all of K, so the result carries 22 significant bits of x: this is the f32 GEMV of the engine to within f32
-// accumulation error, at ~1.3 VALU operations per weight byte whatever the number of token rows.
+// accumulation error, at ~1.3 VALU operations per weight byte whatever the number of token rows. Rows of more than 2048
+// columns are staged as the floats they are, three bf16 pieces each (mfma_quant.hpp): fifteen operand rows for up to five
+// token rows, in the same LDS, or for up to ten where a workgroup can take half of the columns; more take more passes.
 //
 // Raw rows are only 2-byte aligned inside, so the bytes travel global -> registers -> LDS -> registers: a wave reads
 // its 32 weight rows x 8 blocks (272 contiguous bytes per row, 16-byte aligned because 8 blocks = 17 x 16 bytes) with
@@ -56,8 +58,11 @@ __global__ void clear_rows(float4* out, uint64_t count4) {
 }
 
 // The token rows of a workgroup, [kRows, K] from column k0 on, in chunks of eight columns: chunk i = tid + j * kThreads is columns
-// 8 (i % (K / 8)) .. + 7 of row i / (K / 8). kRows * K / 8 <= 2560 = kMine * kThreads for K <= 2560 (8 rows) or 1280 (16 rows).
-constexpr uint32_t kMine = 5, kMostColumns = kMine * kThreads;
+// 8 (i % (K / 8)) .. + 7 of row i / (K / 8). kRows * K / 8 <= 2048 = kMine * kThreads for K <= 2048 (8 rows) or 1024 (16 rows).
+// Five rows in f32: chunk tid of row j (LDS has room for 2560 columns); ten rows, K = 1280 columns: chunk tid % 256 of row j for the first
+// four waves, of row 5 + j for the others.
+constexpr uint32_t kMine = 4, kHalvesColumns = kMine * kThreads, kMostColumns = 2560;
+constexpr int kF32Rows = 5;
 
 template <int kRows>
 __device__ __forceinline__ void request_token_rows(const Q8MfmaArgs& a, uint32_t K, uint32_t k0, float4 (&xv)[kMine][2]) {
@@ -124,14 +129,94 @@ __device__ __forceinline__ float stage_token_rows(const float4 (&xv)[kMine][2], 
     return inv_scale;
 }
 
+// The same for SETS times five rows in f32: xv[j] is row 5 set + j of the thread's set.
+template <int SETS>
+__device__ __forceinline__ void request_f32_rows(const Q8MfmaArgs& a, uint32_t K, uint32_t k0, float4 (&xv)[kF32Rows][2]) {
+    const uint32_t chunk = threadIdx.x % (kThreads / SETS), set = threadIdx.x / (kThreads / SETS);
+#pragma unroll
+    for (uint32_t j = 0; j < kF32Rows; ++j) {
+        xv[j][0] = xv[j][1] = float4{0, 0, 0, 0};
+        if (chunk < K / 8 && set * kF32Rows + j < a.m) {
+            const float4* src = reinterpret_cast<const float4*>(a.x + uint64_t(set * kF32Rows + j) * a.columns + k0 + chunk * 8);
+            xv[j][0] = src[0];
+            xv[j][1] = src[1];
+        }
+    }
+}
+
+// Row s < 4 of a set becomes operand rows s, 4 + s and 12 + s (its pieces from the largest down), row 4 operand rows 8, 9 and 10; a set's
+// sixteen operand rows follow the other's. `back` gets what undoes each row's scale. Ends with a barrier.
+template <int SETS>
+__device__ __forceinline__ void stage_f32_rows(const float4 (&xv)[kF32Rows][2], uint32_t K, __bf16* rows, float (*wave_max)[kWaves], float (&back)[SETS][kF32Rows],
+                                               uint32_t& bad) {
+    constexpr uint32_t kSetWaves = kWaves / SETS;
+    const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave, chunks = K / 8, chunk = tid % (kThreads / SETS), set = tid / (kThreads / SETS);
+#pragma unroll
+    for (int j = 0; j < kF32Rows; ++j) {
+        float biggest = 0;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const float4 v = xv[j][h];
+            if (nonfinite(v.x) || nonfinite(v.y) || nonfinite(v.z) || nonfinite(v.w)) bad = TSP_ERRBIT_NONFINITE;
+            biggest = fmaxf(biggest, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+        }
+        biggest = wave_largest(biggest);
+        if (lane == 0) wave_max[j][wave] = biggest;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kF32Rows; ++j) {
+        float scale = 1.0f;
+#pragma unroll
+        for (uint32_t q = 0; q < SETS; ++q) {
+            float biggest = wave_max[j][q * kSetWaves];
+#pragma unroll
+            for (uint32_t w = 1; w < kSetWaves; ++w) biggest = fmaxf(biggest, wave_max[j][q * kSetWaves + w]);
+            const int shift = row_lift(biggest);
+            if (q == set) scale = power_of_two(shift);
+            back[q][j] = power_of_two(-shift);
+        }
+        if (chunk < chunks) {
+            const float v[8] = {xv[j][0].x, xv[j][0].y, xv[j][0].z, xv[j][0].w, xv[j][1].x, xv[j][1].y, xv[j][1].z, xv[j][1].w};
+            Pieces p[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) p[e] = three_pieces(v[e] * scale);
+            auto put = [&](uint32_t row, u32x4 eight) { *reinterpret_cast<u32x4*>(rows + ((set * 16 + row) * chunks + (chunk ^ row)) * 8) = eight; };
+            const uint32_t first = j < 4 ? j : 8, second = j < 4 ? 4 + j : 9, third = j < 4 ? 12 + j : 10;
+            put(first, u32x4{two_tops(p[0].hi, p[1].hi), two_tops(p[2].hi, p[3].hi), two_tops(p[4].hi, p[5].hi), two_tops(p[6].hi, p[7].hi)});
+            put(second, u32x4{two_tops(p[0].mid, p[1].mid), two_tops(p[2].mid, p[3].mid), two_tops(p[4].mid, p[5].mid), two_tops(p[6].mid, p[7].mid)});
+            put(third, u32x4{two_tops(p[0].lo, p[1].lo), two_tops(p[2].lo, p[3].lo), two_tops(p[4].lo, p[5].lo), two_tops(p[6].lo, p[7].lo)});
+        }
+    }
+    __syncthreads();
+}
+
+// The sums of five rows in f32 out of the accumulators of their fifteen operand rows (row 4 kq + v in acc[v]) for the weight row of
+// lane n16: store(token row, sum) in the lanes that hold one. The small pieces first.
+template <class Store>
+__device__ __forceinline__ void f32_row_sums(const float (&acc)[4], uint32_t kq, const float (&back)[kF32Rows], Store store) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const uint32_t mine = __float_as_uint(kq == 2 ? 0.0f : acc[v]);
+        const auto halves = __builtin_amdgcn_permlane32_swap(mine, mine, false, false);  // lanes l and l ^ 32
+        const uint32_t outer = __float_as_uint(__uint_as_float(halves[0]) + __uint_as_float(halves[1]));
+        const auto quarters = __builtin_amdgcn_permlane16_swap(outer, outer, false, false);  // l and l ^ 16
+        const float sum = __uint_as_float(quarters[0]) + __uint_as_float(quarters[1]);
+        if (kq == 0) store(uint32_t(v), sum * back[v]);
+    }
+    if (kq == 2) store(4u, (acc[0] + (acc[1] + acc[2])) * back[4]);
+}
+
 // DEPTH = (tile, group) items whose bytes are on their way while one is multiplied (1, 2 or 4; it divides the number of groups
-// of a workgroup). ROWS = token rows staged (8: all of K per workgroup; 16: half of K per workgroup, sums added into y).
+// of a workgroup). ROWS = token rows staged (8: all of K per workgroup; 16: half of K per workgroup, sums added into y; 5
+// and 10: the same in f32).
 template <int DEPTH, int ROWS>
 __global__ __launch_bounds__(kThreads, 1) void q8_mfma_kernel(Q8MfmaArgs a) {
-    constexpr int kRows = ROWS;
-    constexpr uint32_t KSPLIT = ROWS / 8;
+    constexpr bool F32 = ROWS % kF32Rows == 0;
+    constexpr int SETS = F32 ? ROWS / kF32Rows : 1, kRows = F32 ? 8 * SETS : ROWS;  // kRows: of each of two operand planes; as much LDS in f32
+    constexpr uint32_t KSPLIT = kRows / 8;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // [hi plane][lo plane][8 weight tiles]
-    __shared__ float wave_max[kWaves];
+    __shared__ float wave_max[kF32Rows][kWaves];
     __shared__ uint32_t next_tile;
 
     const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
@@ -149,8 +234,9 @@ __global__ __launch_bounds__(kThreads, 1) void q8_mfma_kernel(Q8MfmaArgs a) {
     // ---- the token rows: this lane's 16-byte chunks are requested first (they come from cache and return first), then the
     // wave's first weight bytes, and only then the arithmetic. The weights travel while the rows are staged.
     uint32_t bad = 0;
-    float4 xv[kMine][2];
-    request_token_rows<kRows>(a, K, k0, xv);
+    float4 xv[F32 ? kF32Rows : kMine][2];
+    if constexpr (F32) request_f32_rows<SETS>(a, K, k0, xv);
+    else request_token_rows<kRows>(a, K, k0, xv);
     // chunk `id` of a group tile: row id / 17 of the wave's 32, bytes (id % 17) * 16 of that row's 272. The byte offsets from
     // the tile's first row and the group's first byte never change, so a request is a uniform address plus a lane offset.
     uint32_t chunk_at[kStageLoads];
@@ -198,13 +284,16 @@ __global__ __launch_bounds__(kThreads, 1) void q8_mfma_kernel(Q8MfmaArgs a) {
         }
     }
     __builtin_amdgcn_sched_barrier(0);  // every request above is out before the first wait below
-    const float inv_scale = stage_token_rows<kRows>(xv, K, a_hi, a_lo, wave_max, bad);
+    float inv_scale = 1.0f, back[SETS][kF32Rows];
+    if constexpr (F32) stage_f32_rows<SETS>(xv, K, reinterpret_cast<__bf16*>(lds), wave_max, back, bad);
+    else inv_scale = stage_token_rows<kRows>(xv, K, a_hi, a_lo, wave_max[0], bad);
 
     // The activation chunk of block B of group g, columns 8 kq .. 8 kq + 7, is chunk g * 32 + B * 4 + kq of row `arow`, kept at
     // position chunk ^ arow. arow < kRows only flips the low bits, which B % kVariants and kq decide: the lane keeps one
     // address per variant and the rest of the chunk index is an offset known when the code is compiled (B) or uniform (g).
-    const uint32_t arow = n16 & (kRows - 1);
-    constexpr uint32_t kVariants = kRows / 4;
+    constexpr uint32_t kOperandRows = F32 ? 16 : kRows;
+    const uint32_t arow = n16 & (kOperandRows - 1);
+    constexpr uint32_t kVariants = kOperandRows / 4;
     uint32_t a_at[kVariants];  // in halves, from the start of a plane
 #pragma unroll
     for (uint32_t v = 0; v < kVariants; ++v) a_at[v] = (arow * chunks + ((v * 4 + kq) ^ arow)) * 8;
@@ -221,7 +310,7 @@ __global__ __launch_bounds__(kThreads, 1) void q8_mfma_kernel(Q8MfmaArgs a) {
 
     for (; t < share_end; t = t_next, t_next = take_tile()) {
         const uint32_t row0 = t * 32;
-        float acc[2][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}};  // [16-row half of the tile][token row 4 kq + v]
+        float acc[SETS][2][4] = {};  // [set][16-row half of the tile][token row 4 kq + v]
         // one item: its bytes go registers -> LDS tile, the item DEPTH ahead is requested into the freed registers, then the
         // tile is multiplied.
         auto item = [&](uint32_t g, auto set_tag) {
@@ -234,12 +323,14 @@ __global__ __launch_bounds__(kThreads, 1) void q8_mfma_kernel(Q8MfmaArgs a) {
             const uint32_t group = !wraps ? ahead : more ? ahead - groups : g;
             fetch_group(following * 32, group, set_tag);
             const uint8_t* mine = tile + n16 * kTileStride + kq * 8;
+            float group_sum[SETS][2][4] = {};  // in f32 a group's blocks are added up by themselves: a tenth as many roundings of the whole sum
+            auto& sums = F32 ? group_sum : acc;
             auto block = [&](auto b_tag) {
                 constexpr int B = decltype(b_tag)::value;
                 // the lane's eight quants of the block, for rows n16 and n16 + 16 of the tile: bytes 34 B + 2 + 8 kq .. + 8 of the
                 // row, dword aligned for odd B, 2 bytes past a dword for even B
                 constexpr uint32_t Q_AT = 34 * B + 2, ALIGNED = Q_AT & ~3u;
-                f16x8 b_frag[2];
+                std::conditional_t<F32, bf16x8, f16x8> b_frag[2];
                 float scale_d[2];
 #pragma unroll
                 for (int nt = 0; nt < 2; ++nt) {
@@ -255,20 +346,30 @@ __global__ __launch_bounds__(kThreads, 1) void q8_mfma_kernel(Q8MfmaArgs a) {
                         w[0] = __builtin_amdgcn_alignbyte(d[1], d[0], 2);
                         w[1] = __builtin_amdgcn_alignbyte(d[2], d[1], 2);
                     }
-                    b_frag[nt] = quants8(w[0], w[1]);
+                    if constexpr (F32) b_frag[nt] = quants8_bf16(w[0], w[1]);
+                    else b_frag[nt] = quants8(w[0], w[1]);
                     scale_d[nt] = half_bits_to_float(*reinterpret_cast<const uint16_t*>(tile + (nt * 16 + n16) * kTileStride + 34 * B));
                 }
                 // columns g * 256 + B * 32 + 8 kq of the lane's token row
                 const uint32_t at = a_at[B % kVariants] + (g * 32 + (B / kVariants) * kVariants * 4) * 8;
-                const f16x8 ah = *reinterpret_cast<const f16x8*>(a_hi + at), al = *reinterpret_cast<const f16x8*>(a_lo + at);
                 const f32x4 zero{};
 #pragma unroll
                 for (int nt = 0; nt < 2; ++nt) {
-                    // the lo halves of the rows first, the hi halves on top of them: one f32 result per block to scale
-                    const f32x4 part_lo = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, b_frag[nt], zero, 0, 0, 0);
-                    const f32x4 part = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, b_frag[nt], part_lo, 0, 0, 0);
+                    f32x4 part;
+                    if constexpr (F32) {
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) acc[nt][v] = __builtin_fmaf(scale_d[nt], part[v], acc[nt][v]);  // rows 4 kq + v
+                        for (int set = 1; set < SETS; ++set) {
+                            part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(a_hi + set * 16 * K + at), b_frag[nt], zero, 0, 0, 0);
+#pragma unroll
+                            for (int v = 0; v < 4; ++v) sums[set][nt][v] = __builtin_fmaf(scale_d[nt], part[v], sums[set][nt][v]);
+                        }
+                        part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(a_hi + at), b_frag[nt], zero, 0, 0, 0);
+                    } else {  // the lo halves of the rows first, the hi halves on top of them: one f32 result per block to scale
+                        part = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const f16x8*>(a_lo + at), b_frag[nt], zero, 0, 0, 0);
+                        part = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const f16x8*>(a_hi + at), b_frag[nt], part, 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) sums[0][nt][v] = __builtin_fmaf(scale_d[nt], part[v], sums[0][nt][v]);  // rows 4 kq + v
                 }
             };
             block(std::integral_constant<int, 0>{});
@@ -279,6 +380,14 @@ __global__ __launch_bounds__(kThreads, 1) void q8_mfma_kernel(Q8MfmaArgs a) {
             block(std::integral_constant<int, 5>{});
             block(std::integral_constant<int, 6>{});
             block(std::integral_constant<int, 7>{});
+            if constexpr (F32) {
+#pragma unroll
+                for (int set = 0; set < SETS; ++set)
+#pragma unroll
+                    for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) acc[set][nt][v] += group_sum[set][nt][v];
+            }
         };
         for (uint32_t g = 0; g < groups; g += DEPTH) {  // the host picks a DEPTH that divides the number of groups
             item(g, std::integral_constant<int, 0>{});
@@ -291,11 +400,24 @@ __global__ __launch_bounds__(kThreads, 1) void q8_mfma_kernel(Q8MfmaArgs a) {
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt) {
             const uint32_t r = row0 + nt * 16 + n16;
+            if constexpr (F32) {
+#pragma unroll
+                for (int set = 0; set < SETS; ++set) {
+                    f32_row_sums(acc[set][nt], kq, back[set], [&](uint32_t row, float val) {
+                        const uint32_t m = set * kF32Rows + row;
+                        if (m >= a.m || r >= a.rows) return;
+                        if (nonfinite(val)) bad = TSP_ERRBIT_NONFINITE;
+                        if constexpr (KSPLIT == 1) a.y[uint64_t(m) * a.rows + r] = val;
+                        else unsafeAtomicAdd(a.y + uint64_t(m) * a.rows + r, val);
+                    });
+                }
+                continue;
+            }
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const uint32_t m = 4 * kq + v;  // lanes with 4 kq >= kRows hold repeats of rows 0 .. kRows - 1
                 if (m < kRows && m < a.m && r < a.rows) {
-                    const float val = acc[nt][v] * inv_scale;
+                    const float val = acc[0][nt][v] * inv_scale;
                     if (nonfinite(val)) bad = TSP_ERRBIT_NONFINITE;
                     if constexpr (KSPLIT == 1) a.y[uint64_t(m) * a.rows + r] = val;
                     else unsafeAtomicAdd(a.y + uint64_t(m) * a.rows + r, val);
@@ -323,10 +445,11 @@ constexpr uint32_t kLaneLoads = (kLaneRows * kRunChunks + kWave - 1) / kWave;  /
 // each pair over its share of the tiles, both adding their f32 sums into an output the host cleared: the matrix is read once).
 template <int DEPTH, int ROWS>
 __global__ __launch_bounds__(kThreads, 1) void q8_lanes_mfma_kernel(Q8MfmaArgs a) {
-    constexpr int kRows = ROWS;
-    constexpr uint32_t KSPLIT = ROWS / 8;
+    constexpr bool F32 = ROWS % kF32Rows == 0;
+    constexpr int SETS = F32 ? ROWS / kF32Rows : 1, kRows = F32 ? 8 * SETS : ROWS;  // kRows: of each of two operand planes; as much LDS in f32
+    constexpr uint32_t KSPLIT = kRows / 8;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // [hi plane][lo plane][8 weight tiles]
-    __shared__ float wave_max[kWaves];
+    __shared__ float wave_max[kF32Rows][kWaves];
     __shared__ uint32_t next_tile;
 
     const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
@@ -343,8 +466,9 @@ __global__ __launch_bounds__(kThreads, 1) void q8_lanes_mfma_kernel(Q8MfmaArgs a
     uint8_t* const tile = lds + 2 * kRows * K * 2 + wave * kLaneTileBytes;
 
     uint32_t bad = 0;
-    float4 xv[kMine][2];
-    request_token_rows<kRows>(a, K, run0 * (kRunBlocks * 32), xv);
+    float4 xv[F32 ? kF32Rows : kMine][2];
+    if constexpr (F32) request_f32_rows<SETS>(a, K, run0 * (kRunBlocks * 32), xv);
+    else request_token_rows<kRows>(a, K, run0 * (kRunBlocks * 32), xv);
 
     // chunk `id` of a tile: row id / 34 of the wave's 16, piece id % 34 of that row's run: pieces 0 and 1 are the run's scales
     // (32 bytes per run from the row's start), pieces 2 .. 33 its quants (512 bytes per run after all the scales).
@@ -390,12 +514,15 @@ __global__ __launch_bounds__(kThreads, 1) void q8_lanes_mfma_kernel(Q8MfmaArgs a
         if constexpr (DEPTH >= 2) fetch_run(t * kLaneRows, 1, std::integral_constant<int, 1 % DEPTH>{});
     }
     __builtin_amdgcn_sched_barrier(0);  // every request above is out before the first wait below
-    const float inv_scale = stage_token_rows<kRows>(xv, K, a_hi, a_lo, wave_max, bad);
+    float inv_scale = 1.0f, back[SETS][kF32Rows];
+    if constexpr (F32) stage_f32_rows<SETS>(xv, K, reinterpret_cast<__bf16*>(lds), wave_max, back, bad);
+    else inv_scale = stage_token_rows<kRows>(xv, K, a_hi, a_lo, wave_max[0], bad);
 
     // the activation chunk of block B of run g, columns 8 kq .. 8 kq + 7: chunk g * 64 + B * 4 + kq of row `arow`, kept at
     // chunk ^ arow; arow < kRows flips the three or four low bits, which B % kVariants and kq decide
-    const uint32_t arow = n16 & (kRows - 1);
-    constexpr uint32_t kVariants = kRows / 4;
+    constexpr uint32_t kOperandRows = F32 ? 16 : kRows;
+    const uint32_t arow = n16 & (kOperandRows - 1);
+    constexpr uint32_t kVariants = kOperandRows / 4;
     uint32_t a_at[kVariants];
 #pragma unroll
     for (uint32_t v = 0; v < kVariants; ++v) a_at[v] = (arow * chunks + ((v * 4 + kq) ^ arow)) * 8;
@@ -428,6 +555,8 @@ __global__ __launch_bounds__(kThreads, 1) void q8_lanes_mfma_kernel(Q8MfmaArgs a
             uint4 q[8];  // q[j]: quant 8 kq + j of the run's sixteen blocks, one byte per block
 #pragma unroll
             for (int j = 0; j < 8; ++j) q[j] = *reinterpret_cast<const uint4*>(mine + 32 + (8 * kq + j) * 16);
+            float run_sum[4] = {0, 0, 0, 0};  // in f32 a run's blocks are added up by themselves
+            auto& sums = F32 ? run_sum : acc;
             auto quad = [&](auto m_tag) {  // blocks 4 M .. 4 M + 3 of the run
                 constexpr int M = decltype(m_tag)::value;
                 uint32_t d[8];
@@ -453,27 +582,43 @@ __global__ __launch_bounds__(kThreads, 1) void q8_lanes_mfma_kernel(Q8MfmaArgs a
                 for (int b = 0; b < 4; ++b) {
                     constexpr int kBase = 4 * M;
                     const int B = kBase + b;
-                    const f16x8 b_frag = quants8(w[b][0], w[b][1]);
                     const float scale_d = half_bits_to_float((scales[B / 2] >> (16 * (B % 2))) & 0xffffu);
                     const uint32_t at = a_at[B % kVariants] + (g * 64 + (B / kVariants) * kVariants * 4) * 8;  // columns g * 512 + B * 32 + 8 kq of the lane's token row
-                    const f16x8 ah = *reinterpret_cast<const f16x8*>(a_hi + at), al = *reinterpret_cast<const f16x8*>(a_lo + at);
                     const f32x4 zero{};
-                    const f32x4 part_lo = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, b_frag, zero, 0, 0, 0);
-                    const f32x4 part = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, b_frag, part_lo, 0, 0, 0);
+                    f32x4 part;
+                    if constexpr (F32) {
+                        part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(a_hi + at), quants8_bf16(w[b][0], w[b][1]), zero, 0, 0, 0);
+                    } else {
+                        const f16x8 b_frag = quants8(w[b][0], w[b][1]);
+                        part = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const f16x8*>(a_lo + at), b_frag, zero, 0, 0, 0);
+                        part = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const f16x8*>(a_hi + at), b_frag, part, 0, 0, 0);
+                    }
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) acc[v] = __builtin_fmaf(scale_d, part[v], acc[v]);
+                    for (int v = 0; v < 4; ++v) sums[v] = __builtin_fmaf(scale_d, part[v], sums[v]);
                 }
             };
             quad(std::integral_constant<int, 0>{});
             quad(std::integral_constant<int, 1>{});
             quad(std::integral_constant<int, 2>{});
             quad(std::integral_constant<int, 3>{});
+            if constexpr (F32) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[v] += run_sum[v];
+            }
         };
         for (uint32_t g = 0; g < runs; g += DEPTH) {  // the host picks a DEPTH that divides the number of runs
             item(g, std::integral_constant<int, 0>{});
             if constexpr (DEPTH >= 2) item(g + 1, std::integral_constant<int, 1 % DEPTH>{});
         }
         const uint32_t r = row0 + n16;
+        if constexpr (F32) {
+            f32_row_sums(acc, kq, back[0], [&](uint32_t m, float val) {
+                if (m >= a.m || r >= a.rows) return;
+                if (nonfinite(val)) bad = TSP_ERRBIT_NONFINITE;
+                a.y[uint64_t(m) * a.rows + r] = val;
+            });
+            continue;
+        }
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const uint32_t m = 4 * kq + v;  // with eight token rows the lanes with kq >= 2 hold repeats of rows 0 .. 7
@@ -488,6 +633,20 @@ __global__ __launch_bounds__(kThreads, 1) void q8_lanes_mfma_kernel(Q8MfmaArgs a
     publish_error(bad, a.error_word);
 }
 
+// At most `most` token rows at a time, evenly.
+template <class Launch>
+void for_f32_passes(const Q8MfmaArgs& all, uint32_t most, Launch launch) {
+    const uint32_t passes = (all.m + most - 1) / most;
+    for (uint32_t p = 0, done = 0; p < passes; ++p) {
+        Q8MfmaArgs a = all;
+        a.m = (all.m - done + (passes - p) - 1) / (passes - p);
+        a.x += uint64_t(done) * all.columns;
+        a.y += uint64_t(done) * all.rows;
+        launch(a);
+        done += a.m;
+    }
+}
+
 }  // namespace
 
 namespace tsp {
@@ -498,6 +657,7 @@ bool q8_mfma_supported(const void* matrix, const float* x, uint32_t columns, uin
 }
 
 bool q8_mfma_supported_16(const void* matrix, const float* x, const float* y, uint32_t columns, uint32_t rows) {
+    if (columns > kHalvesColumns) return q8_mfma_supported(matrix, x, columns, rows);  // in passes of its own
     return q8_mfma_supported(matrix, x, columns, rows) && columns % 512 == 0 && rows >= 64 && rows % 4 == 0 &&
            reinterpret_cast<uintptr_t>(y) % 16 == 0;
 }
@@ -515,23 +675,45 @@ int q8_mfma(const void* matrix, const float* x, float* y, uint32_t columns, uint
         TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_mfma_kernel<2, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
         TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_mfma_kernel<1, 16>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
         TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_mfma_kernel<2, 16>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
+        TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_mfma_kernel<1, kF32Rows>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
+        TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_mfma_kernel<2, kF32Rows>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
+        TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_mfma_kernel<1, 2 * kF32Rows>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
         TSP_HIP(hipDeviceGetAttribute(&units_of[device], hipDeviceAttributeMultiprocessorCount, device));
         setup_done(raised, device);
     }
     const int compute_units = units_of[device];
     const uint32_t tiles = (rows + 31) / 32;
     uint32_t grid = uint32_t(compute_units > 0 ? compute_units : 256);
-    if (width > 8) {
-        // two workgroups (one per half of the columns) share each run of tiles; the output starts at zero
-        uint32_t pairs = grid / 2 ? grid / 2 : 1;
-        if (pairs * kWaves > tiles) pairs = (tiles + kWaves - 1) / kWaves;
-        const uint64_t count4 = uint64_t(width) * rows / 4;
-        TSP_LAUNCH("clear_rows", s, clear_rows<<<uint32_t((count4 + 255) / 256), 256, 0, s>>>(reinterpret_cast<float4*>(y), count4));
+    // two workgroups (one per half of the columns) share each run of tiles; the output starts at zero
+    uint32_t pairs = grid / 2 ? grid / 2 : 1;
+    if (pairs * kWaves > tiles) pairs = (tiles + kWaves - 1) / kWaves;
+    auto clear = [&](float* out, uint32_t token_rows) {
+        const uint64_t count4 = uint64_t(token_rows) * rows / 4;
+        TSP_LAUNCH("clear_rows", s, clear_rows<<<uint32_t((count4 + 255) / 256), 256, 0, s>>>(reinterpret_cast<float4*>(out), count4));
+    };
+    if (columns > kHalvesColumns && width > kF32Rows && columns % 512 == 0 && rows % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0) {
+        // 2560 columns, five groups to a half: one pass for 8 token rows and two for 16, where five at a time would take two and four
+        // (151 936 rows, 8 token rows: 96 us against 166)
+        for_f32_passes(a, 2 * kF32Rows, [&](const Q8MfmaArgs& pass) {
+            clear(pass.y, pass.m);
+            TSP_LAUNCH("q8_mfma", s, q8_mfma_kernel<1, 2 * kF32Rows><<<2 * pairs, kThreads, lds_bytes, s>>>(pass));
+        });
+        return launch_status("q8_mfma");
+    }
+    if (width > 8 && columns <= kHalvesColumns) {
+        clear(y, width);
         if ((columns / 512) % 2 == 0) TSP_LAUNCH("q8_mfma", s, q8_mfma_kernel<2, 16><<<2 * pairs, kThreads, lds_bytes, s>>>(a));
         else TSP_LAUNCH("q8_mfma", s, q8_mfma_kernel<1, 16><<<2 * pairs, kThreads, lds_bytes, s>>>(a));
         return launch_status("q8_mfma");
     }
     if (grid * kWaves > tiles) grid = (tiles + kWaves - 1) / kWaves;
+    if (columns > kHalvesColumns) {
+        for_f32_passes(a, kF32Rows, [&](const Q8MfmaArgs& pass) {
+            if ((columns / 256) % 2 == 0) TSP_LAUNCH("q8_mfma", s, q8_mfma_kernel<2, kF32Rows><<<grid, kThreads, lds_bytes, s>>>(pass));
+            else TSP_LAUNCH("q8_mfma", s, q8_mfma_kernel<1, kF32Rows><<<grid, kThreads, lds_bytes, s>>>(pass));
+        });
+        return launch_status("q8_mfma");
+    }
     // two items in flight measured best on MI355X (one: 72 us, two: 69 us, four: 75 us at 151 936 x 2048)
     if ((columns / 256) % 2 == 0) TSP_LAUNCH("q8_mfma", s, q8_mfma_kernel<2, 8><<<grid, kThreads, lds_bytes, s>>>(a));
     else TSP_LAUNCH("q8_mfma", s, q8_mfma_kernel<1, 8><<<grid, kThreads, lds_bytes, s>>>(a));
@@ -544,6 +726,7 @@ bool q8_lanes_mfma_supported(const void* matrix, const float* x, uint32_t column
 }
 
 bool q8_lanes_mfma_supported_16(const void* matrix, const float* x, const float* y, uint32_t columns, uint32_t rows) {
+    if (columns > kHalvesColumns) return q8_lanes_mfma_supported(matrix, x, columns, rows);
     return q8_lanes_mfma_supported(matrix, x, columns, rows) && columns % 1024 == 0 && rows >= 32 && rows % 4 == 0 &&
            reinterpret_cast<uintptr_t>(y) % 16 == 0;
 }
@@ -561,13 +744,14 @@ int q8_lanes_mfma(const void* matrix, const float* x, float* y, uint32_t columns
         TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_lanes_mfma_kernel<2, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
         TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_lanes_mfma_kernel<1, 16>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
         TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_lanes_mfma_kernel<2, 16>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
+        TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_lanes_mfma_kernel<1, kF32Rows>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
         TSP_HIP(hipDeviceGetAttribute(&units_of[device], hipDeviceAttributeMultiprocessorCount, device));
         setup_done(raised, device);
     }
     const int compute_units = units_of[device];
     const uint32_t tiles = (rows + kLaneRows - 1) / kLaneRows;
     uint32_t grid = uint32_t(compute_units > 0 ? compute_units : 256);
-    if (width > 8) {
+    if (width > 8 && columns <= kHalvesColumns) {
         // two workgroups (one per half of a row's runs) share each stretch of tiles; the output starts at zero
         uint32_t pairs = grid / 2 ? grid / 2 : 1;
         if (pairs * kWaves > tiles) pairs = (tiles + kWaves - 1) / kWaves;
@@ -578,6 +762,12 @@ int q8_lanes_mfma(const void* matrix, const float* x, float* y, uint32_t columns
         return launch_status("q8_lanes_mfma");
     }
     if (grid * kWaves > tiles) grid = (tiles + kWaves - 1) / kWaves;
+    if (columns > kHalvesColumns) {  // 2560: five runs
+        for_f32_passes(a, kF32Rows, [&](const Q8MfmaArgs& pass) {
+            TSP_LAUNCH("q8_lanes_mfma", s, q8_lanes_mfma_kernel<1, kF32Rows><<<grid, kThreads, lds_bytes, s>>>(pass));
+        });
+        return launch_status("q8_lanes_mfma");
+    }
     if ((columns / 512) % 2 == 0) TSP_LAUNCH("q8_lanes_mfma", s, q8_lanes_mfma_kernel<2, 8><<<grid, kThreads, lds_bytes, s>>>(a));
     else TSP_LAUNCH("q8_lanes_mfma", s, q8_lanes_mfma_kernel<1, 8><<<grid, kThreads, lds_bytes, s>>>(a));
     return launch_status("q8_lanes_mfma");

@@ -6,9 +6,9 @@
 // columns in turns of 64, so that 640 x 2560 is 640 waves that each ask for at most three pieces. A piece is read as it lies (17
 // dwords of each weight row, 256 bytes of each token row, neighbouring lanes at neighbouring addresses: asking for fragments
 // directly, sixteen rows by 8 bytes at a time, took 12 us where this takes 5.4) and put into fragment order through LDS that belongs
-// to the wave alone, so no barrier stands between a piece's arrival and its multiplication. Each token row's part of a piece is scaled by
-// a power of two of its own and split into high and low halves (22 significant bits). The waves' sums meet in LDS in wave order. Bound by
-// latency: launch, one round trip to memory, the sum.
+// to the wave alone, so no barrier stands between a piece's arrival and its multiplication. A token row is three bf16 pieces that are the
+// float exactly (mfma_quant.hpp), each against the same quants. The waves' sums meet in LDS in wave order. Bound by latency: launch,
+// one round trip to memory, the sum.
 #include "q8_small.hpp"
 
 #include "mfma_quant.hpp"
@@ -20,7 +20,7 @@ namespace {
 constexpr uint32_t kWaves = 16, kThreads = kWaves * kWave, kTile = 16, kBlocks = 2, kStep = kBlocks * 32;
 constexpr uint32_t kPieceDwords = kBlocks * 34 / 4;                             // 17: odd, so sixteen rows start in different banks
 constexpr uint32_t kPieceLoads = (kTile * kPieceDwords + kWave - 1) / kWave;    // 5, the last a quarter used
-constexpr uint32_t kHalfStride = kStep + 8;                                     // halves between operand rows: 36 dwords
+constexpr uint32_t kRowStride = kStep + 8;                                      // bf16 values between operand rows: 36 dwords
 
 struct Q8SmallArgs {
     const uint8_t* matrix;
@@ -32,15 +32,15 @@ struct Q8SmallArgs {
     uint32_t* error_word;
 };
 
-// WIDE: nine to sixteen token rows, one operand of sixteen high halves and one of low halves; else one operand whose rows 0..7 are
-// the high halves and 8..15 the low halves of up to eight token rows.
+// WIDE: nine to sixteen token rows, an operand each of their first, second and third pieces; else one operand whose rows 0..7 are the
+// first pieces and 8..15 the second pieces of up to eight token rows, and one with the third pieces and eight rows of zeros.
 template <bool WIDE>
 __global__ __launch_bounds__(kThreads) void q8_small_kernel(Q8SmallArgs a) {
-    constexpr uint32_t kTokens = WIDE ? 16 : 8, kOperandRows = WIDE ? 32 : 16, kTokenLoads = kTokens / 4;
+    constexpr uint32_t kTokens = WIDE ? 16 : 8, kOperandRows = 3 * kTokens + (WIDE ? 0 : 1), kTokenLoads = kTokens / 4;
     struct WaveLds {
         float back[kTokens];  // what undoes the scale of a token row's part of the piece at hand
         uint32_t weights[kPieceLoads * kWave];
-        _Float16 tokens[kOperandRows * kHalfStride];  // kTokens rows of high halves, kTokens of low ones
+        __bf16 tokens[kOperandRows * kRowStride];  // kTokens rows each of first, second and third pieces, a row of zeros
     };
     __shared__ __attribute__((aligned(16))) WaveLds lds[kWaves];
     const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid / kWave))), n16 = lane % 16, kq = lane / 16;
@@ -49,9 +49,11 @@ __global__ __launch_bounds__(kThreads) void q8_small_kernel(Q8SmallArgs a) {
     const uint8_t* const w = a.matrix + uint64_t(row0) * row_bytes;
     const uint8_t* const x = reinterpret_cast<const uint8_t*>(a.x) + token0 * a.x_stride;
     uint32_t* const weights = lds[wave].weights;
-    _Float16* const tokens = lds[wave].tokens;
+    __bf16* const tokens = lds[wave].tokens;
     float* const back = lds[wave].back;
     uint32_t bad = 0;
+    if (!WIDE && lane < kStep / 4) *reinterpret_cast<uint2*>(tokens + 3 * kTokens * kRowStride + lane * 4) = uint2{0, 0};
+    const uint32_t third_row = WIDE ? 32 + n16 : n16 < 8 ? 16 + n16 : 24;
 
     // rows past the end repeat the last one, lanes past the piece its last dword
     uint32_t w_at[kPieceLoads], x_at[kTokenLoads];
@@ -84,7 +86,7 @@ __global__ __launch_bounds__(kThreads) void q8_small_kernel(Q8SmallArgs a) {
         next = fetch(s + kWaves < steps ? s + kWaves : s);
 #pragma unroll
         for (uint32_t t = 0; t < kTokenLoads; ++t) {
-            // sixteen lanes hold a row's 64 columns; its largest magnitude comes to just below 2^14
+            // sixteen lanes hold a row's 64 columns
             uint32_t largest = 0;  // as bits, where infinities and NaNs come out on top
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -93,20 +95,14 @@ __global__ __launch_bounds__(kThreads) void q8_small_kernel(Q8SmallArgs a) {
             }
             largest = row16_largest_bits(largest);
             if (largest >= 0x7f800000u) bad = TSP_ERRBIT_NONFINITE;
-            int shift = 140 - int(largest >> 23);
-            shift = shift > 100 ? 100 : shift < -100 ? -100 : shift;
-            const float scale = __uint_as_float(uint32_t(127 + shift) << 23);
-            f16x4 hi, lo;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float v = now.x[t][e] * scale;
-                hi[e] = _Float16(v);
-                lo[e] = _Float16(v - float(hi[e]));
-            }
-            _Float16* at = tokens + (t * 4 + kq) * kHalfStride + n16 * 4;
-            *reinterpret_cast<f16x4*>(at) = hi;
-            *reinterpret_cast<f16x4*>(at + kTokens * kHalfStride) = lo;
-            back[t * 4 + kq] = __uint_as_float(uint32_t(127 - shift) << 23);
+            const int shift = row_lift(__uint_as_float(largest));
+            const float scale = power_of_two(shift);
+            const Pieces p[4] = {three_pieces(now.x[t][0] * scale), three_pieces(now.x[t][1] * scale), three_pieces(now.x[t][2] * scale), three_pieces(now.x[t][3] * scale)};
+            __bf16* at = tokens + (t * 4 + kq) * kRowStride + n16 * 4;
+            *reinterpret_cast<uint2*>(at) = uint2{two_tops(p[0].hi, p[1].hi), two_tops(p[2].hi, p[3].hi)};
+            *reinterpret_cast<uint2*>(at + kTokens * kRowStride) = uint2{two_tops(p[0].mid, p[1].mid), two_tops(p[2].mid, p[3].mid)};
+            *reinterpret_cast<uint2*>(at + 2 * kTokens * kRowStride) = uint2{two_tops(p[0].lo, p[1].lo), two_tops(p[2].lo, p[3].lo)};
+            back[t * 4 + kq] = power_of_two(-shift);
         }
 #pragma unroll
         for (uint32_t t = 0; t < kPieceLoads; ++t) weights[t * kWave + lane] = now.w[t];
@@ -127,11 +123,12 @@ __global__ __launch_bounds__(kThreads) void q8_small_kernel(Q8SmallArgs a) {
             } else {
                 d = half_bits_to_float(uint16_t(mine[34 * b / 4] >> 16));
             }
-            const f16x8 quants = quants8(w0, w1);
+            const bf16x8 quants = quants8_bf16(w0, w1);
+            auto operand = [&](uint32_t row) { return *reinterpret_cast<const bf16x8*>(tokens + row * kRowStride + b * 32 + kq * 8); };
             f32x4 part{};
-            if constexpr (WIDE)
-                part = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const f16x8*>(tokens + (16 + n16) * kHalfStride + b * 32 + kq * 8), quants, part, 0, 0, 0);
-            part = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const f16x8*>(tokens + n16 * kHalfStride + b * 32 + kq * 8), quants, part, 0, 0, 0);
+            part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(operand(third_row), quants, part, 0, 0, 0);
+            if constexpr (WIDE) part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(operand(16 + n16), quants, part, 0, 0, 0);
+            part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(operand(n16), quants, part, 0, 0, 0);
 #pragma unroll
             for (int v = 0; v < 4; ++v) acc[v] = __builtin_fmaf(d * undo[v], part[v], acc[v]);
         }
