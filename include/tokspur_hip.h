@@ -90,10 +90,6 @@ int tsp_profile_end(tsp_kernel_time* rows, uint32_t capacity, uint32_t* count);
  * it give the factor by which to scale the same counters read for the other kernels. */
 int tsp_calibration_copy(void* dst, const void* src, uint64_t bytes, void* stream);
 
-/* Measurement aid with no counterpart in the reference: keeps `stream` busy for about `microseconds` (at most 1000) with one idle wave,
- * so that what is enqueued meanwhile runs back to back and the time between two events is the device's, not the caller's. */
-int tsp_stream_pause(uint32_t microseconds, void* stream);
-
 /* ------------------------------------------------------------------ host: formats and layouts */
 
 /* src/gguf.cpp:21-32, 157-160 `encoding()`: block geometry of a GGUF type. */

@@ -8,22 +8,7 @@ namespace {
 __global__ __launch_bounds__(256) void calibration_copy(const uint4* __restrict__ src, uint4* __restrict__ dst, uint64_t chunks) {
     for (uint64_t i = blockIdx.x * uint64_t(blockDim.x) + threadIdx.x; i < chunks; i += uint64_t(gridDim.x) * blockDim.x) dst[i] = src[i];
 }
-// One wave asleep until the device's constant-rate clock has advanced by `ticks`; the number of naps is bounded as well.
-__global__ void stream_pause(uint64_t ticks, uint32_t naps) {
-    const uint64_t start = wall_clock64();
-    for (uint32_t i = 0; i < naps && uint64_t(wall_clock64()) - start < ticks; ++i) __builtin_amdgcn_s_sleep(8);  // 512 cycles
-}
 }  // namespace
-
-extern "C" int tsp_stream_pause(uint32_t microseconds, void* stream) {
-    TSP_REQUIRE(microseconds && microseconds <= 1000, "stream pause length");
-    int device = 0, kilohertz = 0;
-    TSP_HIP(hipGetDevice(&device));
-    TSP_HIP(hipDeviceGetAttribute(&kilohertz, hipDeviceAttributeWallClockRate, device));
-    const auto s = static_cast<hipStream_t>(stream);
-    TSP_LAUNCH("stream_pause", s, stream_pause<<<1, kWave, 0, s>>>(uint64_t(microseconds) * uint64_t(kilohertz) / 1000, microseconds * 8));
-    return launch_status("stream_pause");
-}
 
 extern "C" int tsp_calibration_copy(void* dst, const void* src, uint64_t bytes, void* stream) {
     TSP_REQUIRE(dst && src && bytes && bytes % 16 == 0, "calibration copy takes a non-empty multiple of 16 bytes");

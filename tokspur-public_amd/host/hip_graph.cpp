@@ -460,9 +460,6 @@ void HipGraph::begin() {
     // with a profile asked for, the GPU's clock and the host's start the batch together: the stream is idle here, so the wait is short
     if (impl_->profile_capacity) hip(hipEventSynchronize(impl_->started), "hipEventSynchronize");
     impl_->wall_start = std::chrono::steady_clock::now();
-    // and the host gets a lead: an operator of a few microseconds is over before the next one is enqueued, and the boundary after it would
-    // be stamped when the host came to record it
-    if (impl_->profile_capacity) check(tsp_stream_pause(100, impl_->stream));
 }
 
 void HipGraph::abort() {
