@@ -181,6 +181,22 @@ def test_routed_m8_sticky_errors_and_refusals(gpu, tsp, orc, synth):
         tsp.planar_moe_routed_m8(gpu, w, good, xd, 2, selected, y=xd)
 
 
+def test_routed_m8_through_ctypes(gpu, tsp, orc):
+    """A program that binds the C ABI with ctypes and the exported structures gets the compiled binding's bits."""
+    import ctypes
+    channels, hidden, experts, selected, tokens = 256, 64, 8, 4, 3
+    w = build(tsp, gpu, orc, 12, 7, channels, hidden, experts)[3]
+    ids = gpu.upload(np.array([[0, 3, 5, 7], [1, 0, 2, 4], [6, 5, 0, 1]], dtype=np.uint32).reshape(-1))
+    x = gpu.upload(lcg_inputs(77, tokens * channels).reshape(tokens, channels))
+    h, y = tsp.planar_moe_routed_m8(gpu, w, ids, x, tokens, selected)
+    h2, y2 = gpu.zeros(h.shape), gpu.zeros(y.shape)
+    m = tsp.SmallMoe(w.pair_lo.data_ptr(), w.pair_hi.data_ptr(), w.down.data_ptr(), *tsp.COLOC_KINDS[12], tsp.DOWN_KINDS[7], channels, hidden, experts, selected,
+                     tokens, ids.data_ptr(), x.data_ptr(), channels * 4, h2.data_ptr(), hidden * 4, y2.data_ptr(), channels * 4, w.union_meta.data_ptr(),
+                     gpu.err.data_ptr())
+    assert tsp.dll().tsp_planar_moe_routed_m8(ctypes.byref(m), gpu.stream()) == tsp.OK and gpu.error() == 0
+    assert np.array_equal(h2.cpu().numpy(), h.cpu().numpy()) and np.array_equal(y2.cpu().numpy(), y.cpu().numpy())
+
+
 def test_config2_moe_verify(gpu, tsp, orc, synth):
     """BASELINE config 2 at full size: T = 8, hidden 2048, 512 experts, top-10 renormalised softmax routing,
     gate+up Q4_K [2x512, 2048], down Q6_K [2048, 512]; router -> routed experts -> weighted combine with an

@@ -163,6 +163,27 @@ def test_missing_library_fails_loudly(tsp, monkeypatch, tmp_path):
         tsp.dll()
 
 
+def test_operand_descriptions_of_the_c_abi(tsp):
+    """The structures a program calling the C ABI through ctypes fills in: as large as the header's (pointers and 64-bit sizes
+    at 8 bytes), and an empty one is refused on the host."""
+    import ctypes
+    assert [ctypes.sizeof(t) for t in (tsp.SmallMoe, tsp.SharedRows, tsp.GroupedMoe, tsp.SharedExpert)] == [128, 56, 144, 40]
+    lib = tsp.dll()
+    for entry, args in ((lib.tsp_planar_moe_routed_m8, (tsp.SmallMoe(),)), (lib.tsp_planar_moe_routed_m8_shared, (tsp.SmallMoe(), tsp.SharedRows())),
+                        (lib.tsp_planar_nax_grouped_moe, (tsp.GroupedMoe(),)), (lib.tsp_planar_nax_grouped_moe_shared, (tsp.GroupedMoe(), tsp.SharedExpert()))):
+        assert entry(*(ctypes.byref(a) for a in args), None) == tsp.ERR_FORMAT
+
+
+def test_compiled_binding_belongs_to_this_interpreter(tsp, monkeypatch, tmp_path):
+    import sysconfig
+    module = tsp.native()
+    assert module.__file__.endswith("_native" + sysconfig.get_config_var("EXT_SUFFIX"))
+    monkeypatch.setattr(tsp, "_module", None)
+    monkeypatch.setattr(tsp, "HERE", str(tmp_path))
+    with pytest.raises(RuntimeError, match="missing"):
+        tsp.native()
+
+
 def test_host_class_library_exports_graph_operators():
     """libtokspur_graph.so (tokspur::HipGraph, the C++ mirror of the engine's graph class) carries every operator of the path."""
     import subprocess

@@ -13,7 +13,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libtokspur_hip.so")
 HOST_LIB = os.path.join(HERE, "libtokspur_graph.so")
-BINDING = os.path.join(HERE, "_native.so")
+BINDING = os.path.join(HERE, "_native" + sysconfig.get_config_var("EXT_SUFFIX"))  # for this interpreter
 
 HIP_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++20", "-fPIC", "-ffp-contract=off", "-fno-gpu-rdc",
@@ -55,7 +55,7 @@ def build(verbose=False, jobs=8):
 
 
 def build_binding():
-    """The CPython module over the C ABI that capi.Device calls through: binding.cpp -> _native.so, next to the library it links."""
+    """The CPython module over the C ABI that capi.Device calls through: binding.cpp -> _native.<interpreter's tag>.so, next to the library it links."""
     cmd = ["g++", "-std=c++20", "-O2", "-fPIC", "-shared", "-Wall", os.path.join(HERE, "binding.cpp"), "-I", sysconfig.get_path("include"),
            "-L", HERE, "-ltokspur_hip", "-Wl,-rpath,$ORIGIN", "-Wl,--allow-shlib-undefined", "-o", BINDING]
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)

@@ -4,11 +4,13 @@ The library must have been built (python -m build step or __graft_entry__.build(
 loudly when libtokspur_hip.so is missing — there is no fallback path of any kind. `Device` wraps
 torch tensors as device buffers and calls every device entry point on torch's current stream. Host
 functions go through ctypes, device entry points through the compiled module `_native` (binding.cpp),
-which costs a fifth of it per call.
+which costs a fifth of it per call. `SmallMoe`, `SharedRows`, `GroupedMoe` and `SharedExpert` are the C ABI's
+descriptions of MoE operands for programs that call it through ctypes themselves.
 """
 import ctypes as C
 import importlib
 import os
+import sysconfig
 
 import numpy as np
 
@@ -66,8 +68,9 @@ def native():
     global _module
     if _module is None:
         dll()
-        if not os.path.exists(os.path.join(HERE, "_native.so")):
-            raise RuntimeError(f"{HERE}/_native.so is missing: build it with __graft_entry__.build() — there is no fallback")
+        path = os.path.join(HERE, "_native" + sysconfig.get_config_var("EXT_SUFFIX"))
+        if not os.path.exists(path):
+            raise RuntimeError(f"{path} is missing: build it with __graft_entry__.build() under this interpreter — there is no fallback")
         _module = importlib.import_module("._native", __package__)
     return _module
 
@@ -219,6 +222,35 @@ def q8_many_chunks(rows):
     return w.value
 
 
+# ------------------------------------------------------------------ descriptions of MoE operands
+
+class SmallMoe(C.Structure):
+    _fields_ = [("pair_lo", C.c_void_p), ("pair_hi", C.c_void_p), ("down", C.c_void_p),
+                ("gate_kind", C.c_uint32), ("up_kind", C.c_uint32), ("down_kind", C.c_uint32),
+                ("channels", C.c_uint32), ("hidden", C.c_uint32), ("experts", C.c_uint32), ("selected", C.c_uint32),
+                ("tokens", C.c_uint32), ("ids", C.c_void_p), ("x", C.c_void_p), ("x_stride_bytes", C.c_uint64),
+                ("h", C.c_void_p), ("h_stride_bytes", C.c_uint64), ("y", C.c_void_p), ("y_stride_bytes", C.c_uint64),
+                ("union_meta", C.c_void_p), ("error_word", C.c_void_p)]
+
+
+class SharedRows(C.Structure):
+    _fields_ = [("gate", C.c_void_p), ("up", C.c_void_p), ("down", C.c_void_p), ("h", C.c_void_p), ("h_stride_bytes", C.c_uint64),
+                ("y", C.c_void_p), ("y_stride_bytes", C.c_uint64)]
+
+
+class GroupedMoe(C.Structure):
+    _fields_ = [("pair_lo", C.c_void_p), ("pair_hi", C.c_void_p), ("down", C.c_void_p),
+                ("gate_kind", C.c_uint32), ("up_kind", C.c_uint32), ("down_kind", C.c_uint32),
+                ("channels", C.c_uint32), ("hidden", C.c_uint32), ("experts", C.c_uint32), ("selected", C.c_uint32),
+                ("tokens", C.c_uint32), ("ids", C.c_void_p), ("x", C.c_void_p), ("x_stride_bytes", C.c_uint64),
+                ("y", C.c_void_p), ("y_stride_bytes", C.c_uint64), ("token_map", C.c_void_p), ("counts", C.c_void_p),
+                ("tasks", C.c_void_p), ("workspace", C.c_void_p), ("workspace_bytes", C.c_uint64), ("error_word", C.c_void_p)]
+
+
+class SharedExpert(C.Structure):
+    _fields_ = [("gate", C.c_void_p), ("up", C.c_void_p), ("down", C.c_void_p), ("y", C.c_void_p), ("y_stride_bytes", C.c_uint64)]
+
+
 # ------------------------------------------------------------------ device side
 
 class Device:
@@ -232,8 +264,9 @@ class Device:
         self.dev = torch.device("cuda", torch.cuda.current_device())
         self.err = torch.zeros(1, dtype=torch.int32, device=self.dev)
         self.native = native()
-        # the handle of the current device's current stream; torch's stream object costs 2.7 us to make, these two calls 0.15
-        self._raw_stream, self._current_device = torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice
+        # the handle of the current device's current stream; torch's stream object costs 2.7 us to make, these two calls 0.15. They are
+        # not part of torch's public interface: a torch without them is asked for the object.
+        self._raw_stream, self._current_device = getattr(torch._C, "_cuda_getCurrentRawStream", None), getattr(torch._C, "_cuda_getDevice", None)
 
     # -- memory
     def upload(self, a):
@@ -264,6 +297,8 @@ class Device:
         return t.numel() * t.element_size()
 
     def _stream(self):
+        if self._raw_stream is None or self._current_device is None:
+            return self.torch.cuda.current_stream().cuda_stream
         return self._raw_stream(self._current_device())
 
     def stream(self):
