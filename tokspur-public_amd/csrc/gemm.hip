@@ -455,7 +455,7 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {  // two work
                     fold(-hdr[0].dmin, -hdr[1].dmin);
                 }
                 if (P == 3) store_sx((b + 1) & 1);  // read at P == 3 of the next super-block; the buffer was last read at P == 3 of the one before
-                if (P == 1 || P == 3) store_w(wbuf ^ 1, wstage[P == 1 ? 0 : 1]);  // read again two barriers from now; this buffer was last read a step ago
+                if (P == 1 || P == 3) store_w(wbuf ^ 1, wstage[P == 1 ? 0 : 1]);  // the wave's own bytes: read from the next step on, last read two steps ago
                 if (P == 3) { hdr[0] = decode_hdr_q4k<BKIND>(hdr_next[0]); hdr[1] = decode_hdr_q4k<BKIND>(hdr_next[1]); }
             };
             wait_all_loads();  // slabs 0 and 1 (the stores above already waited for younger loads)
