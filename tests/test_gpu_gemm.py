@@ -77,9 +77,8 @@ def test_dense_mm_q4k_tiles(gpu, tsp, orc, synth, tokens, rows, cols):
 
 
 @pytest.mark.parametrize("layout", ["raw", "planar"])
-# GGUF rows of 512, 1024 or 2048 columns against at most 384 rows take 64 x 64 tiles with the columns split over the waves:
-# (33, 96, 512), (128, 256, 2048), (130, 300, 1024), (200, 100, 2048), (384, 132, 1024) and (1, 68, 2048) are its shapes (ragged on either
-# side, one to three rounds of tiles); (385, 64, 2048) and (257, 512, 768) stay with the general kernel
+# GGUF rows take the exact forms of the tile kernel, 32 x 64 tiles for one row and 64 x 64 for the others, their columns shared out over
+# two groups of waves; planar ones the task kernel
 @pytest.mark.parametrize("tokens,rows,cols", [(1, 64, 256), (33, 96, 512), (128, 256, 2048), (130, 300, 1024), (257, 512, 768),
                                               (200, 100, 2048), (384, 132, 1024), (1, 68, 2048), (385, 64, 2048)])
 def test_dense_mm_q4k(gpu, tsp, orc, synth, layout, tokens, rows, cols):
@@ -102,12 +101,12 @@ def test_dense_mm_q4k(gpu, tsp, orc, synth, layout, tokens, rows, cols):
     assert np.array_equal(got_b, synth.round_bf16(got)) and gpu.error() == 0
 
 
-# the last shape is 240 tiles of 256 rows, ragged on both sides: the one-wave-per-SIMD form of the kernel on a 256-unit GPU
-# (512, 300, 256), (600, 1000, 512) and (1000, 256, 1024): fewer than 1024 rows take 128 x 128 tiles, ragged on both sides
+# (2000, 7500, 256): 256 x 256 tiles, ragged on both sides; the others are fewer tiles than the chip takes at once and get 64 x 64
+# (128 x 128 and 128 x 256: test_dense_mm_q4k_tiles)
 @pytest.mark.parametrize("tokens,rows,cols", [(1024, 256, 256), (1100, 300, 512), (1300, 777, 1024), (2000, 7500, 256),
                                               (512, 300, 256), (600, 1000, 512), (1000, 256, 1024)])
 def test_dense_mm_q4k_many_rows(gpu, tsp, orc, synth, tokens, rows, cols):
-    """Raw GGUF Q4_K rows against 512 and more activation rows: the kernel with tiles 128 or 256 rows high, ragged on
+    """Raw GGUF Q4_K rows against 512 and more activation rows: the rounding forms of the tile kernel, ragged on
     both sides. Its arithmetic is the engine's (weights rounded once to half, bf16 activations, f32 accumulation): the
     half-staged reference is met to accumulation accuracy; strided rows and padding stay."""
     w = synth.matrix(12, 2300 + rows, rows, cols)
@@ -128,6 +127,27 @@ def test_dense_mm_q4k_many_rows(gpu, tsp, orc, synth, tokens, rows, cols):
     bad[tokens - 1, 5] = np.nan
     tsp.dense_mm(gpu, 12, tsp.LAYOUT_GGUF, dw, gpu.upload(bad), tokens, cols, rows, x_stride=(cols + 8) * 4)
     assert gpu.error() & tsp.ERRBIT_NONFINITE
+
+
+@pytest.mark.parametrize("rows,out_bf16", [(264, False), (40, True)])
+def test_dense_mm_q4k_activations_of_4_gib(gpu, tsp, orc, synth, rows, out_bf16):
+    """Raw Q4_K rows against 65 536 x 32 768 activations, whose halves are 4 GiB: the kernel with 64-bit row addresses. Error bound:
+    weights and bf16 activations are exact there, so f32 sums of 128 super-blocks over their 256 columns: 2^-15 of sum |w x|; a
+    bf16 result adds 2^-8 of itself."""
+    tokens, cols = 65536, 32768
+    w = synth.matrix(12, 2950 + rows, rows, cols)
+    x = gpu.torch.randn(tokens, cols, dtype=gpu.torch.bfloat16, device=gpu.dev, generator=gpu.torch.Generator(device=gpu.dev).manual_seed(5))
+    out = tsp.dense_mm(gpu, 12, tsp.LAYOUT_GGUF, gpu.upload(w), x, tokens, cols, rows, out_bf16=out_bf16)
+    assert gpu.error() == 0
+    check = [0, 1, 63, 64, 32767, 32768, 65471, 65535]
+    got = (out[check].view(gpu.torch.bfloat16) if out_bf16 else out[check]).double().cpu().numpy()
+    some = x[check].double().cpu().numpy()
+    del out, x
+    gpu.torch.cuda.empty_cache()
+    dense = orc.dequantize(12, w, rows * cols).reshape(rows, cols).astype(np.float64)
+    want = some @ dense.T
+    bound = 2.0 ** -15 * (np.abs(some) @ np.abs(dense).T) + (2.0 ** -8 * np.abs(want) if out_bf16 else 0)
+    assert (np.abs(got - want) <= bound).all()
 
 
 def test_dense_mm_q6k_planar(gpu, tsp, orc, synth):
@@ -675,6 +695,41 @@ def test_grouped_moe_other_planar_kinds(gpu, tsp, orc, synth, gu_type, dn_type, 
 @pytest.mark.parametrize("dn_type,channels,hidden", [(8, 256, 128), (7, 768, 128), (7, 256, 384), (8, 768, 384), (8, 256, 768), (7, 768, 768)])
 def test_grouped_moe_down_rows_in_lds(gpu, tsp, orc, synth, dn_type, channels, hidden):
     test_grouped_moe_other_planar_kinds(gpu, tsp, orc, synth, 12, dn_type, channels, hidden)
+
+
+@pytest.mark.parametrize("dn_type,hidden", [(8, 640), (7, 384)])
+def test_grouped_moe_down_rows_in_lds_errors(gpu, tsp, synth, dn_type, hidden):
+    """The same kernel: an infinite scale in one block of the weights spoils that channel of that expert's routes and nothing else;
+    values that are not finite and expert ids out of range are reported, and the next batch is clean."""
+    channels, experts, selected, n = 768, 4, 2, 90
+    gate, up = synth.matrix(12, 3111, hidden * experts, channels), synth.matrix(12, 3112, hidden * experts, channels)
+    w = tsp.PlanarMoeWeights(gpu, 12, dn_type, channels, hidden, experts, gate, up, synth.matrix(dn_type, 3113, channels * experts, hidden))
+    scratch = tsp.GroupedScratch(gpu, n, selected, experts, channels, hidden)
+    x = (synth.activations_f32(3114, (n, channels)) * 0.1).astype(np.float32)
+    ids = np.array([[0 if t < 70 else 3, 1 + t % 2] for t in range(n)], dtype=np.uint32).reshape(-1)
+    good_ids, good_x = gpu.upload(ids), gpu.upload(x)
+    want = tsp.planar_nax_grouped_moe(gpu, w, good_ids, good_x, n, selected, scratch).cpu().numpy()
+    assert gpu.error() == 0 and np.isfinite(want).all()
+    size, row, expert = (4 if dn_type == 7 else 2), 300, 0
+    at = expert * w.dn_spec.planar_expert_bytes + w.dn_spec.dm_offset + (row * w.dn_spec.blocks_per_row + 3) * size
+    kept = w.down[at:at + 2].clone()
+    w.down[at:at + 2] = gpu.upload(np.array([0x00, 0x7C], dtype=np.uint8))
+    y = tsp.planar_nax_grouped_moe(gpu, w, good_ids, good_x, n, selected, scratch).cpu().numpy()
+    w.down[at:at + 2] = kept
+    assert gpu.error() == tsp.ERRBIT_NONFINITE and not np.isfinite(y[ids == expert, row]).any()
+    y[ids == expert, row] = want[ids == expert, row]
+    assert np.array_equal(y, want)
+    for value in (np.inf, np.nan):
+        bad = x.copy()
+        bad[77, 0] = value
+        tsp.planar_nax_grouped_moe(gpu, w, good_ids, gpu.upload(bad), n, selected, scratch)
+        assert gpu.error() & tsp.ERRBIT_NONFINITE
+    poisoned = ids.copy()
+    poisoned[5] = experts
+    tsp.planar_nax_grouped_moe(gpu, w, gpu.upload(poisoned), good_x, n, selected, scratch)
+    assert gpu.error() & tsp.ERRBIT_INDEX
+    y = tsp.planar_nax_grouped_moe(gpu, w, good_ids, good_x, n, selected, scratch).cpu().numpy()
+    assert gpu.error() == 0 and np.array_equal(y, want)
 
 
 def test_grouped_moe_sticky_errors(gpu, tsp, synth):

@@ -280,8 +280,10 @@ def test_routed_m8_streamed(gpu, tsp, orc, synth, dn, channels, hidden, experts,
                              h_stride=(hidden + 4) * 4, y_stride=(channels + 8) * 4)
     h, y = h.cpu().numpy(), y.cpu().numpy()
     ref_h, ref_y = orc.moe_routed_reference(12, dn, gate, up, down, channels, hidden, experts, ids.reshape(-1), tokens, selected,
-                                            np.ascontiguousarray(x[:, :channels]), threads=8)
-    assert nmse(h[:, :hidden], ref_h) <= 1e-6 and nmse(y[:, :channels], ref_y) <= 1e-6
+                                            np.ascontiguousarray(x[:, :channels]), stage=8 if dn == 14 else 0, threads=8)
+    # a row of two halves has 22 bits of its largest value, 2^-22 of the row or 6e-14 here; one half alone is 4e-8. (Stage bit 8: a Q6_K
+    # product sc * (q - 32) above 2048 loses its lowest bit as a half, which is 1.8e-8 against the exact weights.)
+    assert nmse(h[:, :hidden], ref_h) <= 1e-12 and nmse(y[:, :channels], ref_y) <= 1e-12
     assert (h[:, hidden:] == -5.0).all() and (y[:, channels:] == -6.0).all() and gpu.error() == 0
     if tokens > 2:  # two or more tokens take the same kernels
         _, pair = tsp.planar_moe_routed_m8(gpu, w, gpu.upload(ids[-2:].reshape(-1)), gpu.upload(np.ascontiguousarray(x[-2:, :channels])), 2, selected)
@@ -347,3 +349,49 @@ def test_routed_m8_streamed_f32(gpu, tsp, orc, synth, dn, channels, hidden, toke
         assert (np.abs(h[r] - g * s * u) <= bound).all(), (r, float(np.max(np.abs(h[r] - g * s * u) / bound)))
         bound = unit * (down_a[e] @ np.abs(h[r])) + 1e-36
         assert (np.abs(y[r] - down_w[e] @ h[r]) <= bound).all(), (r, float(np.max(np.abs(y[r] - down_w[e] @ h[r]) / bound)))
+
+
+@pytest.mark.parametrize("tokens", [1, 3, 7])
+@pytest.mark.parametrize("dn,channels,hidden", [(8, 2560, 96), (7, 2304, 160), (14, 1280, 768), (8, 768, 640)])
+def test_routed_m8_streamed_errors(gpu, tsp, synth, dn, channels, hidden, tokens):
+    """The streaming kernels: a value that is not finite in a row, an infinite scale in a block of the down weights and an expert id
+    out of range are reported, the rows of other weights and experts keep their bits (also the row before the infinite block, where a
+    step of 128 columns reads across), and the next batch is clean."""
+    experts, selected = 6, 2
+    gate, up = synth.matrix(12, 71, hidden * experts, channels), synth.matrix(12, 72, hidden * experts, channels)
+    w = tsp.PlanarMoeWeights(gpu, 12, dn, channels, hidden, experts, gate, up, synth.matrix(dn, 73, channels * experts, hidden))
+    ids = np.array([[2, t % 2 * 3 + 1] for t in range(tokens)], dtype=np.uint32).reshape(-1)
+    x = (synth.activations_f32(74, (tokens, channels)) * 0.1).astype(np.float32)
+    good_ids, good_x, routes = gpu.upload(ids), gpu.upload(x), tokens * selected
+
+    def run(d_ids, d_x):
+        h, y = gpu.full((routes, hidden), -3.0), gpu.full((routes, channels), -4.0)
+        tsp.planar_moe_routed_m8(gpu, w, d_ids, d_x, tokens, selected, h=h, y=y)
+        return gpu.error(), y.cpu().numpy()
+
+    status, want = run(good_ids, good_x)
+    assert status == 0 and np.isfinite(want).all()
+    for value in (np.inf, np.nan):
+        bad = x.copy()
+        bad[tokens - 1, channels - 1] = value
+        status, y = run(good_ids, gpu.upload(bad))
+        assert status == tsp.ERRBIT_NONFINITE and np.array_equal(y[:routes - selected], want[:routes - selected])
+    size, row, expert = (4 if dn == 7 else 2), 17, 2
+    at = expert * w.dn_spec.planar_expert_bytes + w.dn_spec.dm_offset + row * w.dn_spec.blocks_per_row * size
+    kept = w.down[at:at + 2].clone()
+    w.down[at:at + 2] = gpu.upload(np.array([0x00, 0x7C], dtype=np.uint8))
+    status, y = run(good_ids, good_x)
+    w.down[at:at + 2] = kept
+    assert status == tsp.ERRBIT_NONFINITE and not np.isfinite(y[ids == expert, row]).any()
+    y[ids == expert, row] = want[ids == expert, row]
+    assert np.array_equal(y, want)
+    poisoned = ids.copy()
+    poisoned[routes - 1] = experts
+    status, y = run(gpu.upload(poisoned), good_x)
+    assert status == tsp.ERRBIT_INDEX
+    if tokens > 1:
+        assert (y == -4.0).all()  # no record of the batch stands
+    else:
+        assert np.array_equal(y[0], want[0]) and (y[1] == -4.0).all()
+    status, y = run(good_ids, good_x)
+    assert status == 0 and np.array_equal(y, want)

@@ -3,9 +3,9 @@
 //   y[rid, c] = Wd[e] h[rid] . c                            down projection
 // with rid = t*selected + slot and e = ids[rid]. HBM-bound: the union records (one per distinct
 // expert, up to 8 tokens each) let every expert's weights be streamed from HBM once for all the
-// tokens that route to it. f32 sums of exact weights everywhere. The rows are f32, except Q4_K and Q6_K products of up to 2048
-// columns and 16-byte aligned rows: there they are two halves under a power of two, 22 bits below the row's (or the
-// slice's) largest value.
+// tokens that route to it. The sums are f32 everywhere, and so are weights and rows, except in Q4_K and Q6_K products of up to 2048
+// columns and 16-byte aligned rows: there a row is two halves under a power of two, 22 bits below its (or its slice's) largest
+// value, and the integer part of a Q6_K weight, sc * (q - 32), a half (above 2048 it loses its lowest bit).
 //
 // This file holds the entry points, the choice of a kernel and the per-element arm, which takes any planar encoding, width and
 // alignment. The kernels that stream the weights past the matrix cores are in record_resident.hip, record_stream.hip and

@@ -17,8 +17,9 @@
 //     exactly (mfma_quant.hpp), against the integer codes q; a record of more rows is passed twice.
 //     Rows of 22 bits (Q4_K and Q6_K up to 2048 columns, as the kernels for their other widths have them, skinny.hip): at most eight,
 //     under a power of two per row that brings the largest magnitude near 2^14, as high halves (operand rows 0..7) and low halves
-//     (rows 8..15), against the integers sc * q, resp. sc * (q - 32), which have too many bits for bf16. Half as many scalings, and
-//     eight rows at once: at 1024 x 512, 8 tokens, a sublayer takes 34 us so and 41 in the other form.
+//     (rows 8..15), against the integers sc * q, resp. sc * (q - 32) (above 2048 without their lowest bit), which have too many
+//     bits for bf16. Half as many scalings, and eight rows at once: at 1024 x 512, 8 tokens, a sublayer takes 34 us so and 41 in
+//     the other form.
 //   * A step's weight bytes are requested three steps ahead, whole 128-byte pieces of rows by neighbouring lanes, into
 //     registers; they turn into fragment order through 2 to 3.5 KB of LDS of the wave's own. (A lane that requests the pieces
 //     of its own row makes the address unit take ~50 cycles per request, more than the memory needs for the bytes.)
