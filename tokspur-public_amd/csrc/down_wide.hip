@@ -285,6 +285,7 @@ int launch_kind(const ResidentDownArgs& a, uint32_t hidden, int groups, hipStrea
 
 namespace tsp {
 
+// The rows of 1024 hidden units (132 KB) would leave no LDS for the waves' stages; 896 are not built.
 bool wide_down_takes(uint32_t source_type, uint32_t channels, uint32_t hidden) {
     return (source_type == kQ8 || source_type == kQ51) && hidden >= 128 && hidden <= 768 && hidden % 128 == 0 && hidden != 512 && channels >= 256 && channels % 256 == 0;
 }

@@ -520,9 +520,9 @@ int launch_gemv(uint32_t encoding, uint32_t layout, GemvArgs a, hipStream_t stre
         if (encoding == 12) return launch_units<12>(a, stream);
         return encoding == 14 ? launch_units<14>(a, stream) : launch_units<8>(a, stream);
     }
-    // 16-byte pieces of every row of either operand, for the routers' sizes (512 x 2560: 5 MB). Above 16 MB the per-element kernel stays: an
-    // operator's boundaries in a profile scatter by up to 10 us here, and the profile's test of its order counts on the 16 us that
-    // kernel takes for 32 MB (7 us in pieces came out shorter than the activation after it now and then).
+    // 16-byte pieces of every row of either operand, for the routers' sizes (512 x 2560: 5 MB). Above 16 MB the per-element kernel stays,
+    // although pieces are faster there as well (4096 x 2048, 32 MB: 7 us against 16): an operator's boundaries in a profile scatter by up
+    // to 10 us, and a 32 MB product is what the profile's test orders against an activation. No matrix of a sublayer is that large.
     if (encoding == 0 && uint64_t(a.columns) * a.rows <= (4u << 20) && aligned && a.columns % 4 == 0 && reinterpret_cast<uintptr_t>(a.x) % 16 == 0 && a.x_stride % 16 == 0) {
         const dim3 grid(grid_rows(a.rows, 2), a.count);
         TSP_LAUNCH("gemv_f32", stream, gemv_f32<<<grid, 128, 0, stream>>>(a));

@@ -1,4 +1,4 @@
-// Internal interface of the integer-digit GEMV (gemv.hip) for the Q8_0 entry points.
+// Internal interface of the any-length GEMV (gemv.hip) for the Q8_0 entry points.
 #pragma once
 #include "tsp_common.hpp"
 
