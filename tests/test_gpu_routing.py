@@ -443,6 +443,33 @@ def test_router_f32_batch_sliced(gpu, synth, tokens, columns, experts):
     assert (np.abs(got - want) <= 2e-6 * scale).all() and gpu.error() == 0
 
 
+@pytest.mark.parametrize("tokens,columns,experts", [(520, 2080, 512), (1025, 64, 512), (300, 32, 931), (577, 288, 500), (2048, 2560, 512)])
+def test_router_f32_batch_pieces(gpu, synth, tokens, columns, experts):
+    """The 64 x 64 form on bf16 pieces: waves with no columns at all, ragged edges, and the rows that pieces cannot carry. What six of nine
+    products of pieces leave out is 2 x 2^-23 of a product at most, under the bound of f32 sums that the other forms keep; an infinite
+    activation gives the infinities of plain f32 arithmetic, rows of subnormals and near them the bound that f32 sums have, zeros zeros."""
+    w = synth.activations_f32(synth.tensor_seed(5, 300 + tokens), (experts, columns))
+    x = synth.activations_f32(synth.tensor_seed(6, 300 + tokens), (tokens, columns))
+    x[3] *= np.float32(2.0 ** -118)
+    x[tokens - 2] *= np.float32(2.0 ** 60)
+    x[7] = 0
+    pitch = (experts + 3) // 4 * 4
+    out = gpu.full((tokens + 1, pitch), 7.25)
+    gpu.router_f32_batch(gpu.upload(w), gpu.upload(x), tokens, columns, experts, out=out, out_stride=pitch * 4)
+    got = out.cpu().numpy()
+    want = x.astype(np.float64) @ w.astype(np.float64).T
+    scale = np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T
+    assert (np.abs(got[:tokens, :experts] - want) <= 2e-6 * scale).all() and gpu.error() == 0
+    assert (got[7, :experts] == 0).all() and (got[tokens] == 7.25).all() and (got[:, experts:] == 7.25).all()
+    x[tokens - 1, columns - 1] = np.inf
+    gpu.router_f32_batch(gpu.upload(w), gpu.upload(x), tokens, columns, experts, out=out, out_stride=pitch * 4)
+    again = out.cpu().numpy()
+    assert np.array_equal(again[:tokens - 1].view(np.uint32), got[:tokens - 1].view(np.uint32)) and gpu.error() != 0
+    gpu.clear_error()
+    last = w[:, columns - 1]
+    assert np.array_equal(again[tokens - 1, :experts], np.where(last == 0, np.nan, np.copysign(np.inf, last)).astype(np.float32), equal_nan=True)
+
+
 @pytest.mark.parametrize("tokens,columns,experts", [(1, 2048, 512), (2, 2080, 65), (3, 32, 5), (4, 2304, 64), (5, 2592, 333), (8, 96, 1024), (7, 6144, 128)])
 def test_router_f32_batch_pairs(gpu, synth, tokens, columns, experts):
     """Up to eight tokens: two experts per workgroup (an odd one left over), each number of token rows the kernel is built for and less,

@@ -2,27 +2,36 @@
 //
 // Replaces the engine's `graph_moe_router_f32_batch` (kernels/moe_router_f32_batch.metal:13-50: 32x32x32 f32 tiles,
 // full-precision multiply-accumulate, operands never narrowed) and its windowed sibling for up to 2048 tokens.
-// Both operands stay f32 from memory to the accumulator: the products run on the f32 matrix-core instruction
-// (v_mfma_f32_32x32x2_f32), which rounds once per fused multiply-add like the scalar code does.
+// Both operands stay whole floats from memory to the accumulator. Few tokens run on the f32 matrix instructions or the vector ALUs.
 //
-// Many tokens: one workgroup of eight waves owns a 64 token x 64 expert tile. Per 64-column step both 64 x 64 operand tiles go
-// global -> registers -> LDS (rows padded to 68 floats so that the 16-byte fragment reads of a wave spread over all
-// banks), double buffered with one barrier per step; waves 0-3 multiply the first 32 columns of the step, waves 4-7 the
-// last 32, so every SIMD holds two waves that hide each other's LDS latency. The two halves are added in a fixed order
-// at the end (deterministic). Consecutive tiles of one token block go to one XCD so that its L2 serves the x rows.
-#include "tsp_common.hpp"
+// Many tokens: a workgroup of eight waves owns 64 tokens x 64 experts, each wave an eighth of the columns; the partial tiles are added in
+// LDS in wave order (deterministic). A float is its three bf16 pieces (mfma_quant.hpp) and a product of two floats the sum of
+// six products of pieces, all exact, in f32 accumulators: v_mfma_f32_32x32x16_bf16 does in 6 x 32 cycles what v_mfma_f32_32x32x2_f32
+// does in 512, and the accumulator is rounded 6 times per sixteen columns instead of 8 (error against 64-bit sums, 2-norm, 2048 x 2560 by 512
+// experts: 2.9e-7, 6.5e-7 with f32 products in two column halves). What is left out is 2^-22 of a product and less. Bound by the matrix pipe
+// (31 k of 56 k cycles) and the splitting (5.5 vector instructions a float, in every tile anew) beside it. 512 experts, 2048
+// tokens: 2560 columns 59 -> 34 us, 2048 columns 46 -> 28.
+#include "mfma_quant.hpp"
+
+#include <type_traits>
 
 using namespace tsp;
 
 namespace {
 
 constexpr uint32_t kTile = 64;                          // tokens and experts per workgroup
-constexpr uint32_t kStep = 64;                          // columns per LDS stage
-constexpr uint32_t kPitch = 68;                         // floats per LDS row
-constexpr uint32_t kStageFloats = 2 * kTile * kPitch;   // x tile, then W tile
-constexpr uint32_t kLdsBytes = 2 * kStageFloats * 4;    // 69 632
+constexpr uint32_t kLdsBytes = 8 * kTile * kTile * 4;    // the eight waves' partial tiles
 
-typedef float acc16 __attribute__((ext_vector_type(16)));
+// Eight floats as three fragments of bf16 pieces (mfma_quant.hpp)
+__device__ __forceinline__ void pieces8(const f32x4 (&v)[2], bf16x8 (&out)[3]) {
+    u32x4 hi, mid, lo;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const Pieces p = three_pieces(v[i / 2][2 * (i % 2)]), q = three_pieces(v[i / 2][2 * (i % 2) + 1]);
+        hi[i] = two_tops(p.hi, q.hi); mid[i] = two_tops(p.mid, q.mid); lo[i] = two_tops(p.lo, q.lo);
+    }
+    out[0] = __builtin_bit_cast(bf16x8, hi); out[1] = __builtin_bit_cast(bf16x8, mid); out[2] = __builtin_bit_cast(bf16x8, lo);
+}
 
 struct RouterArgs {
     const float* weights;
@@ -34,97 +43,133 @@ struct RouterArgs {
     uint32_t* error_word;
 };
 
-__global__ __launch_bounds__(512) void router_f32_gemm(RouterArgs a) {
+// What f32 arithmetic makes of one product of rows, for results that the pieces cannot give: sums that are not finite, and
+// operands so small that a piece of theirs falls below bf16 (a float under 2^-109 loses bits of its last piece).
+__device__ __noinline__ float plain_dot(const float* w, const float* x, uint32_t columns) {
+    float sum = 0.0f;
+    for (uint32_t k = 0; k < columns; ++k) sum = __builtin_fmaf(w[k], x[k], sum);
+    return sum;
+}
+
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void router_f32_gemm(RouterArgs a) {
     extern __shared__ __align__(16) float lds[];
     // blockIdx % 8 names the XCD; each XCD takes a contiguous run of tiles (all expert tiles of a token block together)
     const uint32_t tile = (blockIdx.x % 8) * a.tiles_per_xcd + blockIdx.x / 8;
     if (tile >= a.tiles || blockIdx.x / 8 >= a.tiles_per_xcd) return;
     const uint32_t token0 = (tile / a.expert_tiles) * kTile, expert0 = (tile % a.expert_tiles) * kTile;
-    const uint32_t tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
-    const uint32_t half = wave / 4, wt = (wave % 4) / 2, we = wave % 2;
-
-    // staging: thread t moves float4 number t and t + 512 of each 64 x 64 tile (row = n / 16, 16-byte column = n % 16)
-    const float* xrow[2];
-    const float* wrow[2];
-    uint32_t slot[2];
+    const uint32_t tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    // Requests, 32 columns of the tile's 64 + 64 rows at a time into 16 KB of LDS of the wave's own (nobody else's: no barrier):
+    // instruction q takes rows 8 q .. 8 q + 7, eight neighbouring lanes one whole line, and position p of row r holds the row's 16-byte
+    // chunk p ^ (r / 2) % 8, so that sixteen consecutive lanes of the reads below touch every bank once.
+    const uint8_t* const x0 = reinterpret_cast<const uint8_t*>(a.input + uint64_t(token0) * a.input_stride);
+    const uint8_t* const w0 = reinterpret_cast<const uint8_t*>(a.weights + uint64_t(expert0) * a.columns);
+    uint32_t xat[8], wat[8];  // the launch has checked that 64 rows of either span less than 4 GiB
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const uint32_t n = tid + i * 512, row = n / 16, c4 = n % 16;
-        const uint32_t token = min(token0 + row, a.tokens - 1), expert = min(expert0 + row, a.experts - 1);  // tails re-read a valid row
-        xrow[i] = a.input + uint64_t(token) * a.input_stride + c4 * 4;
-        wrow[i] = a.weights + uint64_t(expert) * a.columns + c4 * 4;
-        slot[i] = row * kPitch + c4 * 4;
+    for (uint32_t q = 0; q < 8; ++q) {  // tails re-read a valid row
+        const uint32_t chunk = ((lane % 8) ^ (4 * (q % 2) + lane / 16)) * 16;
+        xat[q] = min(q * 8 + lane / 8, a.tokens - 1 - token0) * uint32_t(a.input_stride * 4) + chunk;
+        wat[q] = min(q * 8 + lane / 8, a.experts - 1 - expert0) * (a.columns * 4) + chunk;
     }
-    const uint32_t c4 = tid % 16;
-    float4 rx[2], rw[2];
-    auto fetch = [&](uint32_t step) {
-        const uint32_t k = step * kStep;
-        const bool inside = k + c4 * 4 < a.columns;  // columns is a multiple of 32: a last half step reads zeros
+    uint8_t* const mine = reinterpret_cast<uint8_t*>(lds) + wave * 16384;
+    const uint32_t mine_lds = __builtin_amdgcn_readfirstlane(lds_address(mine));
+    const uint32_t n = lane % 32, khalf = lane / 32;
+    f32x16 acc[2][2] = {};  // [expert half][token half]
+    // 32-column units of this wave's slice, two groups of sixteen columns each
+    const uint32_t units = a.columns / 32, first = uint32_t(uint64_t(units) * wave / 8), last = uint32_t(uint64_t(units) * (wave + 1) / 8);
+    auto request = [&](uint32_t unit) {
+        unit = min(unit, last - 1);  // every request unconditional: past the end the last unit again, unused
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            rx[i] = inside ? *reinterpret_cast<const float4*>(xrow[i] + k) : float4{0, 0, 0, 0};
-            rw[i] = inside ? *reinterpret_cast<const float4*>(wrow[i] + k) : float4{0, 0, 0, 0};
+        for (uint32_t q = 0; q < 8; ++q) load_to_lds_16(x0 + uint64_t(unit) * 128, xat[q], mine_lds + q * 1024);
+#pragma unroll
+        for (uint32_t q = 0; q < 8; ++q) load_to_lds_16(w0 + uint64_t(unit) * 128, wat[q], mine_lds + 8192 + q * 1024);
+    };
+    struct Operands { bf16x8 x[2][3], w[2][3]; };
+    struct Rows { f32x4 v[4][2]; };  // x rows 0..31, 32..63, w rows 0..31, 32..63
+    auto read_rows = [&](uint32_t group) {  // a lane's eight columns of a fragment: chunks 4 group + 2 khalf and the next of row n
+        Rows r;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (uint32_t j = 0; j < 2; ++j) r.v[i][j] = *reinterpret_cast<const f32x4*>(mine + i * 4096 + n * 128 + (((4 * group + 2 * khalf + j) ^ (n / 2 % 8)) * 16));
+        return r;
+    };
+    auto split = [&](const Rows& r, Operands& o) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) { pieces8(r.v[i], o.x[i]); pieces8(r.v[2 + i], o.w[i]); }
+    };
+    // One group: its products, and between them the next group's pieces (a 32 x 32 product leaves half of its cycles to the vector ALUs,
+    // a 16 x 16 one none).
+    auto group_of = [&](uint32_t unit, auto parity, const Operands& now, Operands& next) {
+        constexpr uint32_t P = decltype(parity)::value;
+        __builtin_amdgcn_sched_barrier(0);
+        if (P == 1) wait_all_loads();  // the next unit's rows
+        const Rows rows = read_rows(P ^ 1);
+        __builtin_amdgcn_sched_barrier(0);
+        auto add = [&](int i, int j) {
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) acc[e][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(now.x[t][i], now.w[e][j], acc[e][t], 0, 0, 0);
+        };
+        // the small products first; those of 2^-22 of the whole and less (middle with last, last with last) are left out
+        add(2, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (P == 0) {  // the whole unit is in registers: the next one goes there
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            request(unit + 1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        split(rows, next);
+        add(1, 1); add(0, 2); add(1, 0); add(0, 1); add(0, 0);
+#pragma unroll
+        for (int g = 0; g < 20; ++g) {
+            __builtin_amdgcn_sched_group_barrier(0x2, 9, 0);  // nine vector instructions
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);  // and a matrix instruction in turn
         }
     };
-    auto stash = [&](uint32_t stage) {
-        float* base = lds + stage * kStageFloats;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            *reinterpret_cast<float4*>(base + slot[i]) = rx[i];
-            *reinterpret_cast<float4*>(base + kTile * kPitch + slot[i]) = rw[i];
+    if (first < last) {
+        Operands even, odd;
+        request(first);
+        wait_all_loads();
+        split(read_rows(0), even);
+        for (uint32_t u = first; u < last; ++u) {
+            group_of(u, std::integral_constant<uint32_t, 0>{}, even, odd);
+            group_of(u, std::integral_constant<uint32_t, 1>{}, odd, even);
         }
-    };
-
-    // fragments of v_mfma_f32_32x32x2_f32: lane holds A[lane % 32][lane / 32] and B[lane / 32][lane % 32]. A 16-byte read
-    // gives a lane four columns; the same four go to A and B, so the order in which columns meet does not matter.
-    const uint32_t frag_x = (wt * 32 + lane % 32) * kPitch + half * 32 + (lane / 32) * 4;
-    const uint32_t frag_w = kTile * kPitch + (we * 32 + lane % 32) * kPitch + half * 32 + (lane / 32) * 4;
-    acc16 acc = {};
-    const uint32_t steps = (a.columns + kStep - 1) / kStep;
-    fetch(0);
-    stash(0);
-    if (steps > 1) fetch(1);
-    __syncthreads();
-    for (uint32_t s = 0; s < steps; ++s) {
-        const float* base = lds + (s & 1) * kStageFloats;
-        float4 fx[4], fw[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            fx[q] = *reinterpret_cast<const float4*>(base + frag_x + q * 8);
-            fw[q] = *reinterpret_cast<const float4*>(base + frag_w + q * 8);
-        }
-        if (s + 1 < steps) stash((s + 1) & 1);   // the other stage: every wave left it before the last barrier
-        if (s + 2 < steps) fetch(s + 2);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fx[q].x, fw[q].x, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fx[q].y, fw[q].y, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fx[q].z, fw[q].z, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fx[q].w, fw[q].w, acc, 0, 0, 0);
-        }
-        __syncthreads();
-    }
-    // second column half -> LDS -> added by the wave that owns the same 32 x 32 block
-    float* sums = lds + (wave % 4) * 1024;
-    if (half == 1) {
-#pragma unroll
-        for (int v = 0; v < 16; ++v) sums[v * 64 + lane] = acc[v];
+        wait_all_loads();  // requests that nobody reads: they must have landed before the stages are reused
     }
     __syncthreads();
-    if (half == 0) {
-        uint32_t bad = 0;
-        const uint32_t expert = expert0 + we * 32 + lane % 32;
+    // the eight slices, added in wave order
+    f32x4* const sums = reinterpret_cast<f32x4*>(lds);
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const float value = acc[v] + sums[v * 64 + lane];
-            const uint32_t token = token0 + wt * 32 + (v / 4) * 8 + (lane / 32) * 4 + v % 4;  // D[i][j]: j = lane % 32
+    for (int i = 0; i < 16; ++i) {
+        f32x4 quad;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) quad[r] = acc[i / 8][i / 4 % 2][i % 4 * 4 + r];
+        sums[(wave * 16 + i) * 64 + lane] = quad;
+    }
+    __syncthreads();
+    uint32_t bad = 0;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const uint32_t i = tid + j * 512, l = i % 64, b = i / 64 % 4, t = i / 256 % 2, e = i / 512;  // registers 4 b .. 4 b + 3 of lane l of tile (e, t)
+        f32x4 value = sums[i];
+#pragma unroll
+        for (int s = 1; s < 8; ++s) value += sums[s * 1024 + i];
+        const uint32_t expert = expert0 + e * 32 + l % 32;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const uint32_t token = token0 + t * 32 + b * 8 + (l / 32) * 4 + r;  // D[i][j]: j = lane % 32
             if (token < a.tokens && expert < a.experts) {
-                bad |= nonfinite(value) ? TSP_ERRBIT_NONFINITE : 0u;
-                a.output[uint64_t(token) * a.output_stride + expert] = value;
+                float v = value[r];
+                if (nonfinite(v) || (v != 0.0f && fabsf(v) < 0x1p-64f))
+                    v = plain_dot(a.weights + uint64_t(expert) * a.columns, a.input + uint64_t(token) * a.input_stride, a.columns);
+                bad |= nonfinite(v) ? TSP_ERRBIT_NONFINITE : 0u;
+                a.output[uint64_t(token) * a.output_stride + expert] = v;
             }
         }
-        publish_error(bad, a.error_word);
     }
+    publish_error(bad, a.error_word);
 }
 
 // Fewer tokens than fill the chip with 64 x 64 tiles (eight of them for a draft's tokens): a workgroup owns ET * 16 experts x
@@ -296,14 +341,15 @@ extern "C" int tsp_router_f32_batch(const float* weights, const float* input, ui
     a.error_word = error_word;
     const auto s = static_cast<hipStream_t>(stream);
     // The sliced form as long as one round of its tiles (256 compute units) covers the product, on the smallest tile for which
-    // that holds: 16 x 16 (9 us a round at 2048 columns), 16 experts x 32 tokens (13 us), 32 x 32 (17 us); two rounds of the
-    // largest (35 us, 1024 tokens of 512 experts) still beat the 43 us that the 64 x 64 form takes up to a full round of its own.
+    // that holds: 16 x 16 (9 us a round at 2048 columns), 16 experts x 32 tokens (13 us), 32 x 32 (18 us; two rounds of it take 36 us, the
+    // 64 x 64 form 24 at 1024 tokens of 512 experts and 29 for a full round of its own). Rows so far apart that 64 of them span 4 GiB stay with the sliced form's 64-bit addresses.
+    const bool near = 64 * input_stride_bytes < (1ull << 32);
     const auto tiles = [&](uint32_t e, uint32_t t) { return uint64_t((experts + e - 1) / e) * ((tokens + t - 1) / t); };
     // Up to eight tokens: two experts per workgroup, while the chip takes them in two rounds.
     if (tokens <= 8 && experts <= 1024) tokens <= 2 ? launch_pairs<2>(a, s) : tokens <= 4 ? launch_pairs<4>(a, s) : launch_pairs<8>(a, s);
     else if (tiles(16, 16) <= 256) launch_sliced<1, 1>(a, s);
     else if (tiles(16, 32) <= 256) launch_sliced<1, 2>(a, s);
-    else if (tiles(32, 32) <= 512) launch_sliced<2, 2>(a, s);
+    else if (tiles(32, 32) <= 256 || !near) launch_sliced<2, 2>(a, s);
     else TSP_LAUNCH("router_f32_gemm", s, router_f32_gemm<<<a.tiles_per_xcd * 8, 512, kLdsBytes, s>>>(a));
     return launch_status("router_f32_gemm");
 }
