@@ -690,6 +690,44 @@ def test_grouped_moe_other_planar_kinds(gpu, tsp, orc, synth, gu_type, dn_type, 
     assert np.array_equal(y.view(np.uint32), again.view(np.uint32))
 
 
+# the streaming gate/up kernel: one super-block of columns, less than a set of four headers, sets that end in the middle; waves past the last
+# hidden units; tasks of one and of two row tiles
+@pytest.mark.parametrize("channels,hidden", [(256, 160), (768, 96), (1024, 160), (1280, 224), (2304, 96), (3328, 128)])
+def test_grouped_moe_gate_up_stream(gpu, tsp, orc, synth, channels, hidden):
+    test_grouped_moe_other_planar_kinds(gpu, tsp, orc, synth, 12, 8, channels, hidden)
+
+
+@pytest.mark.parametrize("n,hidden,experts,selected", [(20, 256, 32, 4), (90, 512, 64, 4), (95, 256, 64, 4), (96, 256, 64, 4)])
+def test_grouped_moe_2048_columns_few_rows(gpu, tsp, orc, synth, n, hidden, experts, selected):
+    """Either side of six rows per expert, where 2048-column experts change from the resident to the streaming gate/up kernel: loads of none, a
+    few, more than 32 and more than 64 rows, the bounds of the larger cases, and what is reported."""
+    channels = 2048
+    gate, up, down = synth.matrix(12, 3421, hidden * experts, channels), synth.matrix(12, 3422, hidden * experts, channels), synth.matrix(14, 3423, channels * experts, hidden)
+    w = tsp.PlanarMoeWeights(gpu, 12, 14, channels, hidden, experts, gate, up, down)
+    rng = np.random.default_rng(n)
+    ids = np.stack([3 + rng.permutation(experts - 3)[:selected] for _ in range(n)]).astype(np.uint32)  # expert 2 stays empty
+    ids[:n * 3 // 4, 0] = 0
+    ids[n // 2:, 1] = 1
+    x = synth.round_bf16(synth.activations_f32(3424 + n, (n, channels)))
+    scratch = tsp.GroupedScratch(gpu, n, selected, experts, channels, hidden)
+    d_x = gpu.upload(x)
+    y = tsp.planar_nax_grouped_moe(gpu, w, gpu.upload(ids.reshape(-1)), d_x, n, selected, scratch).cpu().numpy()
+    assert gpu.error() == 0
+    _, declared = orc.moe_routed_reference(12, 14, gate, up, down, channels, hidden, experts, ids.reshape(-1), n, selected, x, stage=12, threads=8)
+    scale = np.maximum(1.0, np.sqrt((declared ** 2).mean(axis=1, keepdims=True)))
+    err = np.abs(y - declared) / np.maximum(scale, np.abs(declared))
+    # as for the larger cases above: f32 accumulation, and now and then a carried half that falls the other way
+    assert float(np.median(err)) <= 2e-5 and float(err.max()) <= 4e-3 and nmse(y, declared) <= 1e-7
+    broken = ids.copy()
+    broken[n // 2, 2] = broken[n // 2, 0]
+    for poisoned in (broken, np.where(ids == 5, experts, ids)):
+        tsp.planar_nax_grouped_moe(gpu, w, gpu.upload(poisoned.astype(np.uint32).reshape(-1)), d_x, n, selected, scratch)
+        assert gpu.error() & tsp.ERRBIT_INDEX
+    x[n - 1, 2047] = np.inf
+    tsp.planar_nax_grouped_moe(gpu, w, gpu.upload(ids.reshape(-1)), gpu.upload(x), n, selected, scratch)
+    assert gpu.error() & tsp.ERRBIT_NONFINITE
+
+
 # the down kernel that keeps a task's h rows in LDS: one to six steps of 128 hidden units (six take the requests in two halves), one
 # and three groups of 256 channels, tasks of one and of two row tiles
 @pytest.mark.parametrize("dn_type,channels,hidden", [(8, 256, 128), (7, 768, 128), (7, 256, 384), (8, 768, 384), (8, 256, 768), (7, 768, 768)])

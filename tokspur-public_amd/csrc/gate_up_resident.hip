@@ -1,4 +1,4 @@
-// Grouped gate/up GEMM with fused SwiGLU for 2048-column Q4_K experts, activations resident in registers.
+// Grouped gate/up GEMM with fused SwiGLU for 2048-column Q4_K experts that have few rows each, activations resident in registers.
 //
 // The ragged grouped product is bound by the expert weights streaming in from HBM, so the kernel is built around that
 // stream and keeps everything else off the memory pipeline:

@@ -22,8 +22,6 @@
 //     weight is unpacked once per task.
 //   * Activations are shared by the four waves: 64 rows x 128 bytes per K step go global -> LDS directly (no registers),
 //     two and three steps ahead, into a ring of four slabs; one LDS-only barrier per two K steps.
-//   * For gate/up the two column tiles of a wave are the gate rows and the up rows of the same 32 hidden
-//     units, so SwiGLU is an element-wise epilogue on accumulator registers.
 #include "dense_tile.hpp"
 #include "down_resident.hpp"
 #include "gate_up_resident.hpp"
@@ -38,8 +36,8 @@ using namespace tsp;
 
 namespace {
 
-enum Epilogue : int { EPI_F32 = 0, EPI_BF16 = 1, EPI_SWIGLU = 2 };
-enum Rows : int { ROWS_DENSE = 0, ROWS_GATHER_TOKENS = 1, ROWS_TASK_SLOTS = 2, ROWS_ROUTES = 3 };
+enum Epilogue : int { EPI_F32 = 0, EPI_BF16 = 1 };
+enum Rows : int { ROWS_DENSE = 0, ROWS_TASK_SLOTS = 1, ROWS_ROUTES = 2 };
 
 constexpr int kTaskRows = 64;
 constexpr int kRowTiles = kTaskRows / 32;
@@ -48,8 +46,7 @@ struct GemmArgs {
     const _Float16* a;        // activation rows, a_stride halfs apart
     uint64_t a_stride;
     const _Float16* sx;       // per row, per super-block: 8 sub-block sums (hi) + 8 residuals (lo); Q4_K only
-    const uint8_t* w0;        // dense matrix / pair_lo / down experts
-    const uint8_t* w1;        // pair_hi
+    const uint8_t* w0;        // dense matrix / experts
     tsp_planar_spec spec;     // planar layouts (per expert)
     uint32_t experts;
     const uint32_t* tasks;    // grouped: [2 + 2*bound] with kTaskRows-row tiles
@@ -57,7 +54,7 @@ struct GemmArgs {
     const uint32_t* token_map;
     const uint32_t* ids;
     uint32_t tokens, selected;
-    uint32_t m, n, k;         // dense rows; weight rows (or hidden units for SwiGLU); columns
+    uint32_t m, n, k;         // dense rows; weight rows; columns
     void* out;
     uint64_t out_stride;      // bytes
     float out_scale;
@@ -66,9 +63,8 @@ struct GemmArgs {
     uint32_t broadcast;              // ROWS_ROUTES: one input row per token instead of one per route
     uint32_t col_tiles, task_slots;  // logical grid: column tiles x tasks, launched as one linear grid
     // an always-on expert riding in the same launch: tasks whose expert id is `experts` take every token as their rows,
-    // these weights (gate / up halves, or the down matrix) and, for the down product, these output rows
+    // this down matrix and these output rows
     const uint8_t* shared_w0;
-    const uint8_t* shared_w1;
     void* shared_out;
     uint64_t shared_out_stride;
 };
@@ -154,13 +150,11 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {  // two work
                 rid = a.token_map[uint64_t(expert) * a.tokens + start + (tid < nrows ? tid : 0)];
                 if (rid >= a.tokens * a.selected || a.ids[rid] != expert) { rid = 0xffffffffu; task_bad = 1; }
             }
-            // activation row: the route's token (gate/up, broadcast grouped GEMM), the route itself (grouped GEMM with one input
-            // row per route) or the task's slot in the intermediate buffer (down); output row: task slot or route
+            // activation row: the route's token (broadcast grouped GEMM), the route itself (grouped GEMM with one input
+            // row per route) or the task's slot in the intermediate buffer (down); output row: the route
             const uint32_t safe = rid == 0xffffffffu ? 0 : rid;
-            row_src[tid] = ROWS == ROWS_GATHER_TOKENS ? safe / a.selected
-                         : ROWS == ROWS_ROUTES       ? (a.broadcast ? safe / a.selected : safe)
-                                                     : task * kTaskRows + (tid < nrows ? tid : 0);
-            my_dst = ROWS == ROWS_GATHER_TOKENS ? task * kTaskRows + tid : shared ? rid / a.selected : rid;
+            row_src[tid] = ROWS == ROWS_ROUTES ? (a.broadcast ? safe / a.selected : safe) : task * kTaskRows + (tid < nrows ? tid : 0);
+            my_dst = shared ? rid / a.selected : rid;
         }
     }
     __syncthreads();
@@ -172,24 +166,13 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {  // two work
     uint64_t wrow[2];
     uint32_t out_col[2];
     bool col_live[2];
-    if constexpr (EPI == EPI_SWIGLU) {
-        const uint32_t unit = bx * 128 + wave * 32 + col;
-        const uint32_t half_e = a.experts / 2;
-        const uint8_t* pair = (expert < half_e ? a.w0 : a.w1) + uint64_t(expert < half_e ? expert : expert - half_e) * 2 * a.spec.planar_expert_bytes;
-        wbase[0] = shared ? a.shared_w0 : pair;
-        wbase[1] = shared ? a.shared_w1 : pair + a.spec.planar_expert_bytes;
-        col_live[0] = col_live[1] = unit < a.n;
-        wrow[0] = wrow[1] = col_live[0] ? unit : a.n - 1;
-        out_col[0] = out_col[1] = unit;
-    } else {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const uint32_t n = bx * 256 + wave * 64 + j * 32 + col;
-            col_live[j] = n < a.n;
-            wrow[j] = col_live[j] ? n : a.n - 1;
-            out_col[j] = n;
-            wbase[j] = shared ? a.shared_w0 : a.w0 + uint64_t(expert) * (BKIND == B_Q4K_RAW ? a.raw_expert_bytes : a.spec.planar_expert_bytes);
-        }
+    for (int j = 0; j < 2; ++j) {
+        const uint32_t n = bx * 256 + wave * 64 + j * 32 + col;
+        col_live[j] = n < a.n;
+        wrow[j] = col_live[j] ? n : a.n - 1;
+        out_col[j] = n;
+        wbase[j] = shared ? a.shared_w0 : a.w0 + uint64_t(expert) * (BKIND == B_Q4K_RAW ? a.raw_expert_bytes : a.spec.planar_expert_bytes);
     }
     const uint32_t bpr = a.k / 256;
     const uint32_t ksteps = a.k / KSTEP;
@@ -369,14 +352,14 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {  // two work
             constexpr uint32_t BLK = BKIND == B_Q4K_PLANAR ? 128 : 144, QS_AT = BKIND == B_Q4K_PLANAR ? 0 : 16;
             uint8_t* const my_w = lds_w + wave * (2 * 64 * 64);  // [2 buffers][64 rows][4 chunks of 16 B]
             const uint32_t ld_row = lane / 4, ld_chunk = (lane % 4) ^ ((lane / 8) & 3);  // chunk c of row r sits at position c ^ ((r >> 1) & 3)
-            const uint32_t wave_row0 = EPI == EPI_SWIGLU ? bx * 128 + wave * 32 : bx * 256 + wave * 64;
+            const uint32_t wave_row0 = bx * 256 + wave * 64;
             const uint32_t row_bytes = bpr * BLK;
             const uint32_t halves = 2 * bpr;
             u32x4 wstage[2][4];  // odd halves, even halves
             // instruction Q of a half-block: rows 16Q .. 16Q+15 of the wave's 64 (tile Q / 2)
             auto fetch_w = [&](u32x4 (&into)[4], uint32_t half, auto q_tag) {
                 constexpr int Q = decltype(q_tag)::value, J = Q / 2;
-                uint32_t row = wave_row0 + (EPI == EPI_SWIGLU ? (Q % 2) * 16 : Q * 16) + ld_row;
+                uint32_t row = wave_row0 + Q * 16 + ld_row;
                 row = row < a.n ? row : a.n - 1;
                 // uniform base + 32-bit lane offset (the host refuses matrices whose rows span 4 GiB or more)
                 const uint8_t* base = wbase[J] + (BKIND == B_Q4K_PLANAR ? a.spec.qs_offset : 0) + uint64_t(half / 2) * BLK + QS_AT + (half % 2) * 64;
@@ -486,30 +469,18 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {  // two work
             if (r >= nrows) continue;
             const uint32_t dst = row_dst[r];
             if (dst == 0xffffffffu) continue;
-            if constexpr (EPI == EPI_SWIGLU) {
-                if (!col_live[0]) continue;
-                const float g = acc[i][0][v], u = acc[i][1][v];
-                const float sg = sigmoid_stable(g);
-                const float h = (g * sg) * u;
-                // h is carried between the two GEMMs as the half nearest to h * 2^-8: 11 significant bits for
-                // 0.016 <= |h| < 1.6e7, an absolute step of 2^-16 below that
-                const _Float16 carried = _Float16(h * 0.00390625f);
-                if (nonfinite(g) || nonfinite(u) || nonfinite(h) || (__builtin_bit_cast(uint16_t, carried) & 0x7c00u) == 0x7c00u) bad = TSP_ERRBIT_NONFINITE;
-                reinterpret_cast<_Float16*>(a.out)[uint64_t(dst) * a.n + out_col[0]] = carried;
-            } else {
 #pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    if (!col_live[j]) continue;
-                    const float val = acc[i][j][v] * a.out_scale;
-                    if (nonfinite(val)) bad = TSP_ERRBIT_NONFINITE;
-                    uint8_t* orow = shared && ROWS == ROWS_TASK_SLOTS ? static_cast<uint8_t*>(a.shared_out) + uint64_t(dst) * a.shared_out_stride
-                                                                      : static_cast<uint8_t*>(a.out) + uint64_t(dst) * a.out_stride;
-                    if constexpr (EPI == EPI_F32) {
-                        reinterpret_cast<float*>(orow)[out_col[j]] = val;
-                    } else {
-                        const uint32_t vb = __float_as_uint(val);
-                        reinterpret_cast<uint16_t*>(orow)[out_col[j]] = uint16_t((vb + 0x7fffu + ((vb >> 16) & 1u)) >> 16);
-                    }
+            for (int j = 0; j < 2; ++j) {
+                if (!col_live[j]) continue;
+                const float val = acc[i][j][v] * a.out_scale;
+                if (nonfinite(val)) bad = TSP_ERRBIT_NONFINITE;
+                uint8_t* orow = shared && ROWS == ROWS_TASK_SLOTS ? static_cast<uint8_t*>(a.shared_out) + uint64_t(dst) * a.shared_out_stride
+                                                                  : static_cast<uint8_t*>(a.out) + uint64_t(dst) * a.out_stride;
+                if constexpr (EPI == EPI_F32) {
+                    reinterpret_cast<float*>(orow)[out_col[j]] = val;
+                } else {
+                    const uint32_t vb = __float_as_uint(val);
+                    reinterpret_cast<uint16_t*>(orow)[out_col[j]] = uint16_t((vb + 0x7fffu + ((vb >> 16) & 1u)) >> 16);
                 }
             }
         }
@@ -599,7 +570,7 @@ __global__ __launch_bounds__(512) void tasks_and_rows(TaskLists t, const void* _
 
 template <int BKIND, int EPI, int ROWS>
 int launch(const GemmArgs& a, uint32_t col_tiles, uint32_t tasks, hipStream_t s) {
-    constexpr const char* name = EPI == EPI_SWIGLU ? "gemm_gate_up_swiglu" : ROWS == ROWS_TASK_SLOTS ? "gemm_down" : ROWS == ROWS_ROUTES ? "gemm_grouped" : "gemm_dense";
+    constexpr const char* name = ROWS == ROWS_TASK_SLOTS ? "gemm_down" : ROWS == ROWS_ROUTES ? "gemm_grouped" : "gemm_dense";
     GemmArgs g = a;
     g.col_tiles = col_tiles;
     g.task_slots = tasks;
@@ -939,23 +910,21 @@ int grouped_moe(const tsp_grouped_moe* m, const tsp_shared_expert* shared, void*
     staged.task_list = task_list; staged.task_slots = l.bound; staged.counts = m->counts; staged.token_map = m->token_map; staged.ids = m->ids;
     staged.hbuf = hbuf; staged.y = m->y; staged.y_stride = m->y_stride_bytes; staged.error_word = m->error_word;
 
-    GemmArgs g{};
-    g.a = xh; g.a_stride = m->channels; g.sx = sx; g.w0 = static_cast<const uint8_t*>(m->pair_lo); g.w1 = static_cast<const uint8_t*>(m->pair_hi);
-    g.spec = gu; g.experts = m->experts; g.tasks = task_list; g.counts = m->counts; g.token_map = m->token_map; g.ids = m->ids;
-    g.tokens = m->tokens; g.selected = m->selected; g.n = m->hidden; g.k = m->channels; g.out = hbuf; g.out_scale = 1.0f;
-    g.error_word = m->error_word;
-    if (shared) { g.shared_w0 = static_cast<const uint8_t*>(shared->gate); g.shared_w1 = static_cast<const uint8_t*>(shared->up); }
     if (!fast_gate_up) {
         rc = launch_planar_staged_gate_up(staged, s);
-    } else if (resident_gate_up_takes(m->channels, m->hidden)) {
+    } else {
         ResidentGateUpArgs r{};
-        r.xh = xh; r.sx = sx; r.pair_lo = g.w0; r.pair_hi = g.w1; r.shared_gate = g.shared_w0; r.shared_up = g.shared_w1; r.spec = gu;
-        r.experts = m->experts; r.tokens = m->tokens; r.selected = m->selected; r.hidden = m->hidden;
+        r.xh = xh; r.sx = sx; r.pair_lo = static_cast<const uint8_t*>(m->pair_lo); r.pair_hi = static_cast<const uint8_t*>(m->pair_hi);
+        if (shared) { r.shared_gate = static_cast<const uint8_t*>(shared->gate); r.shared_up = static_cast<const uint8_t*>(shared->up); }
+        r.spec = gu; r.experts = m->experts; r.tokens = m->tokens; r.selected = m->selected; r.channels = m->channels; r.hidden = m->hidden;
         r.tasks = task_list; r.classes = reinterpret_cast<const uint32_t*>(ws + l.classes); r.counts = m->counts; r.token_map = m->token_map; r.ids = m->ids; r.task_slots = l.bound;
         r.hbuf = hbuf; r.error_word = m->error_word;
-        rc = launch_resident_gate_up(r, s);
-    } else {
-        rc = launch<B_Q4K_PLANAR, EPI_SWIGLU, ROWS_GATHER_TOKENS>(g, (m->hidden + 127) / 128, l.bound, s);
+        // Few rows per expert: the launch is bound by HBM, and the resident kernel's shares of 32 units leave no compute unit waiting for
+        // another (a sublayer of 2048 x 512, 512 experts: 20 tokens 102 us against 114, 100 tokens 216 against 220; 400 tokens 302 against 295, 2048
+        // tokens 478 against 449; 2048 x 768, 128 experts: 50 tokens 143 against 145, 100 tokens 152 against 151, 2048 tokens 408 against 383).
+        // The two add a row's super-blocks up in the same order but not with the same roundings.
+        const bool few = routes < 6 * m->experts;
+        rc = few && resident_gate_up_takes(m->channels, m->hidden) ? launch_resident_gate_up(r, s) : launch_stream_gate_up(r, s);
     }
     if (rc != TSP_OK) return rc;
     const uint64_t shared_span = shared ? uint64_t(m->tokens) * shared->y_stride_bytes : 0;

@@ -1,4 +1,4 @@
-// Shared by the two resident grouped GEMMs (gate_up_resident.hip, down_resident.hip): how a persistent workgroup learns about
+// Shared by the grouped GEMMs that keep a task's rows on the chip (gate_up_resident.hip, gate_up_stream.hip, down_resident.hip, down_wide.hip): how a persistent workgroup learns about
 // the tasks of its share. A task is an entry of the grouped GEMMs' 64-row task list, (expert, first row); the always-on
 // expert's tasks carry expert id == experts and take the tokens themselves as their rows.
 #pragma once
