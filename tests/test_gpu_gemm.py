@@ -76,6 +76,13 @@ def test_dense_mm_q4k_tiles(gpu, tsp, orc, synth, tokens, rows, cols):
     assert np.array_equal(bf16_to_f32(bits[:, :rows]), synth.round_bf16(got)) and (bits[:, rows:] == 7).all() and gpu.error() == 0
 
 
+# the forms for few tiles: 32 x 32 up to a full round, one tile more, super-blocks that do not divide among four groups and fewer than groups, then
+# 64 x 32, and 32 rows of more tiles than a round
+@pytest.mark.parametrize("tokens,rows,cols", [(64, 4096, 256), (32, 8193, 512), (3, 33, 1536), (70, 97, 2560), (40, 4200, 768), (33, 8170, 1280), (97, 4064, 2304)])
+def test_dense_mm_q4k_few_tiles(gpu, tsp, orc, synth, tokens, rows, cols):
+    test_dense_mm_q4k_tiles(gpu, tsp, orc, synth, tokens, rows, cols)
+
+
 @pytest.mark.parametrize("layout", ["raw", "planar"])
 # GGUF rows take the exact forms of the tile kernel, 32 x 64 tiles for one row and 64 x 64 for the others, their columns shared out over
 # two groups of waves; planar ones the task kernel

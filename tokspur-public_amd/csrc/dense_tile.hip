@@ -64,18 +64,32 @@ constexpr int kStepK = 64, kRing = 3;
 
 // TN: weight rows of a tile (TN / 32 waves side by side).
 template <int RT, int WAVES, int TN, int GROUPS, bool EXACT>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void dense_tile_kernel(DenseTileArgs a) {
-    constexpr int kGroupWaves = WAVES / GROUPS, kThreadsT = 64 * kGroupWaves, WN = TN / 32, WM = kGroupWaves / WN, kTileM = WM * RT * 32;
-    constexpr int kSlabBytes = kTileM * kStepK * 2, kSxBytes = EXACT ? kTileM * 32 : 0;
+struct Shape {
+    static constexpr int kGroupWaves = WAVES / GROUPS, kThreadsT = 64 * kGroupWaves, WN = TN / 32, WM = kGroupWaves / WN, kTileM = WM * RT * 32;
+    static constexpr int kSlabBytes = kTileM * kStepK * 2, kSxBytes = EXACT ? kTileM * 32 : 0;
     static_assert(WM >= 1 && WN * WM * GROUPS == WAVES && (RT % GROUPS == 0 || GROUPS % RT == 0));
-    constexpr int kSlabPieces = kSlabBytes / (kThreadsT * 16), kSxPieces = (kSxBytes + kThreadsT * 16 - 1) / (kThreadsT * 16);
+    static constexpr int kSlabPieces = kSlabBytes / (kThreadsT * 16), kSxPieces = (kSxBytes + kThreadsT * 16 - 1) / (kThreadsT * 16);
     static_assert(kSlabBytes % (kThreadsT * 16) == 0);
-    constexpr int kChunks = TN * 9, kWPieces = (kChunks + kThreadsT - 1) / kThreadsT;  // 16-byte pieces of a super-block of the tile's weight rows
-    constexpr int kWAt = kRing * kSlabBytes, kSxAt = kWAt + kWPieces * kThreadsT * 16, kGroupBytes = kSxAt + 2 * kSxBytes;
-    constexpr int kOwn = RT >= GROUPS ? RT / GROUPS : 1, kShares = RT / kOwn;  // row tiles of the wave's results that a group stores, and groups that store
-    constexpr int kParts = GROUPS == 1 ? 0 : GROUPS * kShares * kThreadsT * kOwn * 64, kRegion = 12 * 1024;
-    __shared__ __attribute__((aligned(16))) uint8_t lds_all[std::max(GROUPS * kGroupBytes, std::max(kParts, WAVES * kRegion))];
-    static_assert(sizeof(lds_all) * (8 / WAVES) <= 160 * 1024, "the workgroups of a compute unit share 160 KB");
+    static constexpr int kChunks = TN * 9, kWPieces = (kChunks + kThreadsT - 1) / kThreadsT;  // 16-byte pieces of a super-block of the tile's weight rows
+    static constexpr int kWAt = kRing * kSlabBytes, kSxAt = kWAt + kWPieces * kThreadsT * 16, kGroupBytes = kSxAt + 2 * kSxBytes;
+    static constexpr int kOwn = RT >= GROUPS ? RT / GROUPS : 1, kShares = RT / kOwn;  // row tiles of the wave's results that a group stores, and groups that store
+    static constexpr int kParts = GROUPS == 1 ? 0 : GROUPS * kShares * kThreadsT * kOwn * 64, kRegion = 12 * 1024;
+    static constexpr int kLds = std::max(GROUPS * kGroupBytes, std::max(kParts, WAVES * kRegion));
+    // Where one workgroup of four waves fills a compute unit the LDS is sized at the launch: knowing its size the compiler would keep sums in
+    // accumulator registers and move them out again to scale them.
+    static constexpr bool kAtLaunch = WAVES == 4 && kLds > 80 * 1024;
+    static_assert(kLds * (kAtLaunch ? 1 : 8 / WAVES) <= 160 * 1024, "the workgroups of a compute unit share 160 KB");
+};
+
+template <int RT, int WAVES, int TN, int GROUPS, bool EXACT>
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void dense_tile_kernel(DenseTileArgs a) {
+    using S = Shape<RT, WAVES, TN, GROUPS, EXACT>;
+    constexpr int kGroupWaves = S::kGroupWaves, kThreadsT = S::kThreadsT, WN = S::WN, kTileM = S::kTileM, kSlabBytes = S::kSlabBytes, kSxBytes = S::kSxBytes;
+    constexpr int kSlabPieces = S::kSlabPieces, kSxPieces = S::kSxPieces, kChunks = S::kChunks, kWPieces = S::kWPieces, kWAt = S::kWAt, kSxAt = S::kSxAt;
+    constexpr int kGroupBytes = S::kGroupBytes, kOwn = S::kOwn, kShares = S::kShares, kRegion = S::kRegion;
+    __shared__ __attribute__((aligned(16))) uint8_t lds_sized[S::kAtLaunch ? 16 : S::kLds];
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds_at_launch[];
+    uint8_t* const lds_all = S::kAtLaunch ? lds_at_launch : lds_sized;
 
     const uint32_t group = GROUPS == 1 ? 0 : uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x / kThreadsT)));
     uint8_t* const lds_raw = lds_all + group * kGroupBytes;
@@ -288,7 +302,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
         // group g stores row tiles g * kOwn .. of the tile: every group leaves the others' parts in LDS, and the parts of a result
         // are added in the order of the columns, its own among them
         constexpr int kPart = kOwn * 16;  // floats of a lane in one group's share
-        static_assert(GROUPS * kShares * kThreadsT * kPart * 4 <= int(sizeof(lds_all)));
+        static_assert(GROUPS * kShares * kThreadsT * kPart * 4 <= S::kLds);
         float* const parts = reinterpret_cast<float*>(lds_all);  // [group][share][wave][kPart / 4][lane][4]
         auto at = [&](uint32_t from, uint32_t share, int piece) { return parts + (((from * kShares + share) * kGroupWaves + wave) * kPart + piece * 4) * kWave + lane * 4; };
 #pragma unroll
@@ -317,7 +331,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
         // more than the row keeps the column-wise writes and the row-wise reads off each other's banks). A lane storing
         // its own 2- or 4-byte results one by one, 128 stores, took a fifth of the kernel's time.
         uint8_t* const mine = lds_all + (group * kGroupWaves + wave) * kRegion;
-        static_assert(WAVES * kRegion <= int(sizeof(lds_all)));
+        static_assert(WAVES * kRegion <= S::kLds);
         // four row tiles at a time as bf16, two as f32 (with two column tiles per wave; twice that with four, and four and two with one),
         // or as many as there are
         constexpr int kTilesB = std::min(kOwn, 4), kTilesF = std::min(kOwn, 2);
@@ -387,6 +401,15 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
 
 template <int RT, int WAVES, int TN, int GROUPS, bool EXACT>
 int launch(DenseTileArgs a, hipStream_t s) {
+    using S = Shape<RT, WAVES, TN, GROUPS, EXACT>;
+    if constexpr (S::kAtLaunch) {
+        static std::atomic<uint64_t> raised{0};
+        int device = 0;
+        if (setup_pending(raised, &device)) {
+            TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&dense_tile_kernel<RT, WAVES, TN, GROUPS, EXACT>), hipFuncAttributeMaxDynamicSharedMemorySize, S::kLds));
+            setup_done(raised, device);
+        }
+    }
     constexpr uint32_t TM = WAVES / GROUPS / (TN / 32) * RT * 32;
     const uint32_t m_tiles = (a.m + TM - 1) / TM, n_tiles = (a.n + TN - 1) / TN, tiles = m_tiles * n_tiles;
     // Each XCD fetches the activation rows and the weight rows that its run of tiles touches into an L2 of its own: the band that makes
@@ -397,7 +420,7 @@ int launch(DenseTileArgs a, hipStream_t s) {
         const uint64_t bytes = uint64_t(high) * TM * 32 + uint64_t(wide) * TN * 9;
         if (bytes < least) { least = bytes; a.band = band; }
     }
-    TSP_LAUNCH("gemm_dense_tile", s, (dense_tile_kernel<RT, WAVES, TN, GROUPS, EXACT><<<(tiles + 7) / 8 * 8, WAVES * 64, 0, s>>>(a)));
+    TSP_LAUNCH("gemm_dense_tile", s, (dense_tile_kernel<RT, WAVES, TN, GROUPS, EXACT><<<(tiles + 7) / 8 * 8, WAVES * 64, S::kAtLaunch ? S::kLds : 0, s>>>(a)));
     return launch_status("dense_tile");
 }
 
@@ -408,9 +431,16 @@ namespace tsp {
 int launch_dense_tile(const DenseTileArgs& a, hipStream_t s) {
     auto tiles = [&](uint64_t high, uint64_t wide) { return (a.m + high - 1) / high * ((a.n + wide - 1) / wide); };
     if (a.m < 512 || a.n < 256) {
-        // 64 x 64 tiles while the chip takes them all at once, two to a compute unit: 13 to 24 us at 2560 columns, 41 for twice as many,
-        // where 128 x 128 tiles take 34. Up to 32 rows the lower half of a 64-row tile would be empty.
+        // A wave alone on its SIMD issues an instruction every eight cycles, and few tiles are waves that stand alone: as long as the chip takes
+        // the smallest tiles at once, one to a compute unit, they share out the super-blocks four ways (2560 columns, up to 4096 rows: 12.5 to 13.8 us with
+        // two groups of 64-row tiles, 10.1 to 10.7 so; 2048 columns 11.4 to 12.2, now 8.7 to 9.2; 512 columns 8.4, 7.3). With two such tiles to a
+        // compute unit nothing is left of that, with five or eight groups 0.6 us less of it. Then tiles of 64 x 32 (37 rows: 2048 x 8192 12.0
+        // and 10.6, 2560 x 6100 14.3 and 13.6), which need three super-blocks to have work for the groups.
+        if (tiles(32, 32) <= 256) return launch<1, 4, 32, 4, true>(a, s);
         if (a.m <= 32) return launch<1, 4, 64, 2, true>(a, s);
+        if (tiles(64, 32) <= 256 && a.k > 512) return launch<2, 4, 32, 4, true>(a, s);
+        // 64 x 64 tiles while the chip takes them all at once, two to a compute unit: 13 to 24 us at 2560 columns, 41 for twice as many,
+        // where 128 x 128 tiles take 34.
         if (tiles(64, 64) <= 512) return launch<2, 4, 64, 2, true>(a, s);
         return launch<4, 8, 128, 2, true>(a, s);
     }
