@@ -26,8 +26,8 @@
 //
 // Measured (kernel trace, 2560 channels x 640 hidden units, 8 tokens, 69 distinct experts: 131 MB of gate/up, 120 MB of Q8_0 or
 // 85 MB of Q5_1 down): 45 us, 36 and 41, where the per-element kernels took 194 and 142. (With rows of 22 bits 43 and 34: the
-// f32 form costs a scaling per 32 columns in Q4_K, and a Q5_1 block its nearest code.) Some 8 us are the launch's serial
-// beginning (ids, records, table, first bytes), the rest is a stream at 5 TB/s beside an instruction stream of equal length.
+// f32 form costs a scaling per 32 columns in Q4_K, and a Q5_1 block its nearest code.) Some 7 us are the launch's serial
+// beginning (ids, records, table, first bytes; a microsecond more with divisions in the table's planning, 5 tokens 30.0 -> 28.6 us), the rest is a stream at 5 TB/s beside an instruction stream of equal length.
 // Two tiles per step against one read of the operand (a tenth fewer instructions), and the LDS round trip of a step overlapped
 // with the products of the one before, were each built and made no difference. For rows of 1, 2, 4 or 8 super-blocks the
 // kernels that keep a wave's columns in registers (record_resident.hip, skinny.hip) stay the faster ones where they apply: no
@@ -74,6 +74,11 @@ constexpr uint32_t kQ51SumBytes = 32;  // the slots' sums of a block: slots 0..3
 
 template <int KIND> constexpr uint32_t q4_sum_bytes() { if constexpr (is_q4(KIND)) return Traits<KIND>::sum_bytes; else return 0; }
 
+// n / d as one multiplication: magic = 2^32 / d rounded up is off by less than d / 2^32 per unit, so the quotient is exact for n * d < 2^32.
+struct Divisor { uint32_t d, magic; };
+__device__ __forceinline__ uint32_t operator/(uint32_t n, const Divisor& v) { return v.d == 1 ? n : __umulhi(n, v.magic); }
+Divisor divisor(uint32_t d) { return Divisor{d, d == 1 ? 0 : uint32_t((1ull << 32) / d + ((1ull << 32) % d != 0))}; }
+
 struct StreamArgs {
     const float* x;            // rows of the product: tokens (gate/up) or routes (down), x_stride bytes apart
     uint64_t x_stride;
@@ -91,6 +96,8 @@ struct StreamArgs {
     float* shared_out;         // rows by token
     uint64_t shared_out_stride;
     uint32_t experts, tokens, selected, n, k;  // n: weight rows (hidden units | channels); k: columns
+    Divisor units, ppt;                        // tiles of a record, pieces of a tile
+    uint32_t per_group;                        // 2^32 / workgroups, rounded down
     uint32_t* error_word;
 };
 
@@ -160,16 +167,19 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     const uint32_t limit = a.tokens * a.selected < 128 ? a.tokens * a.selected : 128;
     const uint32_t listed = __builtin_amdgcn_readfirstlane(block[6]), live = listed < limit ? listed : limit;
     const uint32_t units = a.n / kTile, records = live + (a.shared_w0 ? 1 : 0), items = records * units;  // at most 129 x 4096
-    const uint32_t share1 = items * (blockIdx.x + 1) / gridDim.x;
+    // Where share b begins: any monotone cut will do, and this one is a multiplication (a division is some thirty dependent instructions of a
+    // wave that is alone, and they all stand before the first byte is requested).
+    auto share_at = [&](uint32_t b) { return b == gridDim.x ? items : __umulhi(items * b, a.per_group); };
+    const uint32_t share1 = share_at(blockIdx.x + 1);
     const uint32_t bpr = a.k / T::block, last_block = a.n * bpr - 1;
-    const uint32_t spt = (a.k + T::step - 1) / T::step, ppt = (spt + kPiece - 1) / kPiece;  // steps and pieces per tile
+    const uint32_t spt = (a.k + T::step - 1) / T::step, ppt = a.ppt.d;  // steps and pieces per tile
     if (listed > limit) bad |= TSP_ERRBIT_INDEX;
 
     // Lane l of the first wave looks after record k0 + l, then row slot l, then tile l. A record that does not check out has no
     // rows and reads expert 0: the batch is refused.
     // A record of more rows than slots makes passes of its own, over the same items with the rows from row0 on.
     auto plan_pass = [&](uint32_t item0, uint32_t row0) {
-        const uint32_t k0 = item0 / units, k = k0 + lane, index = k < 128 ? k : 0;
+        const uint32_t k0 = item0 / a.units, k = k0 + lane, index = k < 128 ? k : 0;
         const bool shared = a.shared_w0 != nullptr && k == live;
         uint32_t expert = shared ? 0 : block[8 + index], count = shared ? a.tokens : block[136 + index];
         if (k >= records) count = 0;
@@ -177,17 +187,19 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         const uint32_t first = __builtin_amdgcn_readlane(count, 0);
         const bool split = first > kSlots;
         uint32_t upto = count;
-#pragma unroll
-        for (uint32_t d = 1; d < kWave; d <<= 1) {
-            const uint32_t before = __shfl_up(upto, d, kWave);
-            if (lane >= d) upto += before;
-        }
+        // sums over the first sixteen lanes: more records than slots are never taken
+        auto add_shifted = [&](auto control) { upto += uint32_t(__builtin_amdgcn_update_dpp(0, int(upto), decltype(control)::value, 0xf, 0xf, true)); };
+        add_shifted(std::integral_constant<int, 0x111>{});
+        add_shifted(std::integral_constant<int, 0x112>{});
+        add_shifted(std::integral_constant<int, 0x114>{});
+        add_shifted(std::integral_constant<int, 0x118>{});
         uint32_t item1 = share1 - item0 > kMaxTiles / kMats ? item0 + kMaxTiles / kMats : share1;
-        const uint64_t fits = __builtin_amdgcn_ballot_w64(k * units < item1 && (lane == 0 || upto <= kSlots));
+        const uint64_t fits = __builtin_amdgcn_ballot_w64(lane < 16 && k * units < item1 && (lane == 0 || upto <= kSlots));
         const uint32_t taken = __builtin_ctzll(~fits);  // records of this pass: nearly always all of the share's
         if ((k0 + taken) * units < item1) item1 = (k0 + taken) * units;
         const uint32_t whole = __builtin_amdgcn_readlane(upto, taken - 1), rows = !split ? whole : first - row0 < kSlots ? first - row0 : kSlots;
-        const uint32_t room = kPartialBytes / 4 / ((split ? kSlots : rows ? rows : 1) * kTile * ppt * kMats);  // the same for a record's passes
+        // kPartialBytes / 4 / (rows * kTile * ppt * kMats), the same for a record's passes; quotients of small numbers, at least 1 / 128 apart from a whole one
+        const uint32_t room = uint32_t(float(kPartialBytes / 4 / (kTile * kMats)) * __builtin_amdgcn_rcpf(float((split ? kSlots : rows ? rows : 1) * ppt)) + 0.001f);
         if (item1 - item0 > room) item1 = item0 + room;
         const uint32_t tiles = (item1 - item0) * kMats;
         if (lane == 0) { pass.item1 = item1; pass.rows = rows; pass.tiles = tiles; pass.next_row = split && row0 + rows < first ? row0 + rows : 0; }
@@ -204,7 +216,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             pass.src[lane] = reinterpret_cast<uint64_t>(rs ? a.shared_x : a.x) + uint64_t(SWIGLU ? token : route) * (rs ? a.shared_x_stride : a.x_stride);
             pass.dst[lane] = reinterpret_cast<uint64_t>(rs ? a.shared_out : a.out) + uint64_t(route) * (rs ? a.shared_out_stride : a.out_stride);
         }
-        const uint32_t tile = lane < tiles ? lane : 0, item = item0 + tile / kMats, mat = tile % kMats, tk = item / units - k0;
+        const uint32_t tile = lane < tiles ? lane : 0, item = item0 + tile / kMats, mat = tile % kMats, tk = item / a.units - k0;
         const uint32_t te = __shfl(expert, tk, kWave), tc = __shfl(count, tk, kWave), tu = __shfl(upto, tk, kWave), unit = item - (tk + k0) * units;
         const uint8_t* base;
         if (a.shared_w0 != nullptr && tk + k0 == live) base = mat ? a.shared_w1 : a.shared_w0;
@@ -260,14 +272,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     const uint32_t q4_sel = kq & 1 ? 0x04030402u : 0x04010400u;
 
     uint32_t row0 = 0;
-    for (uint32_t item0 = items * blockIdx.x / gridDim.x; item0 < share1;) {
+    for (uint32_t item0 = share_at(blockIdx.x); item0 < share1;) {
         if (wave == 0) plan_pass(item0, row0);
         lds_barrier();
         const uint32_t item1 = __builtin_amdgcn_readfirstlane(pass.item1), rows = __builtin_amdgcn_readfirstlane(pass.rows), tiles = __builtin_amdgcn_readfirstlane(pass.tiles);
         row0 = __builtin_amdgcn_readfirstlane(pass.next_row);  // of the next pass
         const uint32_t stride = rows * kTile, pieces = tiles * ppt, each = (pieces + kWaves - 1) / kWaves;
         const uint32_t p0 = wave * each < pieces ? wave * each : pieces, p1 = p0 + each < pieces ? p0 + each : pieces;
-        const uint32_t tile0 = p0 / ppt, tile1 = p1 / ppt;
+        const uint32_t tile0 = p0 / a.ppt, tile1 = p1 / a.ppt;
         const uint32_t s0 = tile0 * spt + (p0 - tile0 * ppt) * kPiece, s1 = tile1 * spt + (p1 - tile1 * ppt) * kPiece;
 
         // ---- this wave's row, requested first: loads come back in the order they were asked for
@@ -614,7 +626,12 @@ int launch_pieces(const char* name, const StreamArgs& a, hipStream_t s) {
     }
     const int rc = compute_units(&cus);
     if (rc != TSP_OK) return rc;
-    TSP_LAUNCH(name, s, record_stream<KIND, SWIGLU, PIECES><<<cus, kThreads, layout_of<KIND>(a.k).total, s>>>(a));
+    StreamArgs g = a;
+    const uint32_t spt = (a.k + Traits<KIND>::step - 1) / Traits<KIND>::step;
+    g.units = divisor(a.n / kTile);
+    g.ppt = divisor((spt + kPiece - 1) / kPiece);
+    g.per_group = uint32_t((1ull << 32) / (cus > 1 ? cus : 2));
+    TSP_LAUNCH(name, s, record_stream<KIND, SWIGLU, PIECES><<<cus > 1 ? cus : 2, kThreads, layout_of<KIND>(a.k).total, s>>>(g));
     return launch_status(name);
 }
 
