@@ -11,9 +11,12 @@
 //
 // f16_gemm_nt: a workgroup of four waves owns a 64 x 64 output tile (each wave a 32 x 32 MFMA tile) and walks K in
 // steps of 64 halfs. Every byte travels global -> LDS directly (16 bytes per lane, no registers in between) into a ring
-// of four stages, three steps ahead of the multiply; chunk c of row r of a slab sits at position r * 8 + (c ^ (r & 7)),
-// which the loads fill linearly by lane and the fragment reads spread over all banks. No other vector-memory operation
-// exists in the loop, so the wait before a step's barrier is simply "all but the two younger stages have landed".
+// of four stages, three steps ahead of the multiply; chunk c of row r of a slab sits at position r * 8 + (c ^ (r / 2 % 8)),
+// which the loads fill linearly by lane and sixteen consecutive lanes of the fragment reads find in all banks. No other vector-memory operation
+// exists in the loop, so the wait before a step's barrier is simply "all but the two younger stages have landed". Bound by the way from
+// L2 into LDS: 210 MB in 18 us at 2048 tokens, 2560 columns, 640 rows. Tiles of an XCD side by side, its fragments read ahead: a call with its
+// conversion 31.0 -> 27.3 us there, 24.6 -> 24.2 at 640 columns x 2560 rows, 20.0 -> 19.2 at 2048 x 512 (128 x 64 tiles 27.1, 26.0 and 21.5,
+// 128 x 128 33.7, 26.7 and 27.9: half and a quarter of the compute units without a tile).
 #include "mfma_quant.hpp"
 
 using namespace tsp;
@@ -48,16 +51,21 @@ __global__ __launch_bounds__(256, 2) void f16_gemm_nt(F16GemmArgs a) {
     __shared__ __attribute__((aligned(16))) uint8_t lds[kRing * kStageBytes];  // 64 KB: two workgroups per CU
     const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
     const uint32_t col = lane % 32, khalf = lane / 32;
-    const uint32_t m0 = blockIdx.y * kTile, n0 = blockIdx.x * kTile;
+    // an XCD (workgroup id % 8) takes a run of tiles and with it an eighth of the larger operand and all of the smaller one into its L2
+    const uint32_t n_tiles = (a.n + kTile - 1) / kTile, m_tiles = (a.m + kTile - 1) / kTile, tiles = n_tiles * m_tiles, per_xcd = (tiles + 7) / 8;
+    const uint32_t tile = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+    if (blockIdx.x / 8 >= per_xcd || tile >= tiles) return;
+    const bool tall = a.m >= a.n;
+    const uint32_t m0 = (tall ? tile / n_tiles : tile % m_tiles) * kTile, n0 = (tall ? tile % n_tiles : tile / m_tiles) * kTile;
     const uint32_t steps = a.k / kStep;
 
     // piece p = i * 256 + tid of a stage (1024 pieces of 16 bytes): slab p / 512, LDS position q = p % 512 -> row q / 8,
-    // chunk (q % 8) ^ (row & 7). Rows past the matrix re-read its last row (never stored).
+    // chunk (q % 8) ^ (row / 2 % 8). Rows past the matrix re-read its last row (never stored).
     const uint8_t* src[4];
     uint32_t lds_at[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const uint32_t p = i * 256 + tid, slab = p / 512, q = p % 512, r = q / 8, c = (q % 8) ^ (r & 7);
+        const uint32_t p = i * 256 + tid, slab = p / 512, q = p % 512, r = q / 8, c = (q % 8) ^ (r / 2 % 8);
         uint32_t row = (slab ? n0 : m0) + r;
         const uint32_t limit = slab ? a.n : a.m;
         row = row < limit ? row : limit - 1;
@@ -73,23 +81,27 @@ __global__ __launch_bounds__(256, 2) void f16_gemm_nt(F16GemmArgs a) {
     f32x16 acc;
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
-    const uint32_t arow = (wave / 2) * 32 + col, brow = (wave % 2) * 32 + col;
+    // chunk 2 kc + khalf of the wave's row
+    const uint32_t at = col * 128 + ((khalf ^ (col / 2 % 8)) * 16), x_at = (wave / 2) * 4096 + at, w_at = kSlabBytes + (wave % 2) * 4096 + at;
     request(0, 0);
     request(1, 1);
     request(2, 2);
     for (uint32_t s = 0; s < steps; ++s) {
         const uint32_t slot = s % kRing;
         lds_barrier_after_loads<8>();  // stage s has landed (the two younger stages may be on their way); every wave has left slot (s + 3) % 4
+        // every fragment is read before the first product: a read right before its product is its latency four times a step
+        f16x8 fa[4], fb[4];
+        auto read = [&](uint32_t kc) {
+            fa[kc] = *reinterpret_cast<const f16x8*>(lds + slot * kStageBytes + (x_at ^ (kc * 32)));
+            fb[kc] = *reinterpret_cast<const f16x8*>(lds + slot * kStageBytes + (w_at ^ (kc * 32)));
+        };
+        read(0);
+        read(1);
         request(s + 3, (s + 3) % kRing);
-        const uint8_t* xs = lds + slot * kStageBytes;
-        const uint8_t* ws = xs + kSlabBytes;
+        read(2);
+        read(3);
 #pragma unroll
-        for (int kc = 0; kc < 4; ++kc) {
-            const uint32_t c = kc * 2 + khalf;
-            const f16x8 fa = *reinterpret_cast<const f16x8*>(xs + (arow * 8 + (c ^ (arow & 7))) * 16);
-            const f16x8 fb = *reinterpret_cast<const f16x8*>(ws + (brow * 8 + (c ^ (brow & 7))) * 16);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa, fb, acc, 0, 0, 0);
-        }
+        for (int kc = 0; kc < 4; ++kc) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[kc], fb[kc], acc, 0, 0, 0);
     }
     wait_all_loads();  // the last requests land in slots nobody reads: they must be done before this LDS is given away
 
@@ -318,7 +330,7 @@ extern "C" int tsp_dense_mm_q8_staged(uint32_t layout, const void* matrix, uint6
     const OperandsArgs o{static_cast<const uint8_t*>(matrix), input, input_stride_bytes, w16, x16, layout, columns, rows, tokens, uint32_t(w_groups), error_word};
     TSP_LAUNCH("q8_operands_to_f16", s, q8_operands_to_f16<<<uint32_t(w_groups + x_groups), 256, 0, s>>>(o));
     const F16GemmArgs a{x16, w16, output, output_stride_bytes, tokens, rows, columns, error_word};
-    const dim3 grid((rows + kTile - 1) / kTile, (tokens + kTile - 1) / kTile);
-    TSP_LAUNCH("f16_gemm_nt", s, f16_gemm_nt<<<grid, 256, 0, s>>>(a));
+    const uint64_t f16_tiles = uint64_t((rows + kTile - 1) / kTile) * ((tokens + kTile - 1) / kTile);
+    TSP_LAUNCH("f16_gemm_nt", s, f16_gemm_nt<<<uint32_t((f16_tiles + 7) / 8 * 8), 256, 0, s>>>(a));
     return launch_status("f16_gemm_nt");
 }
