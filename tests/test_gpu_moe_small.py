@@ -395,3 +395,26 @@ def test_routed_m8_streamed_errors(gpu, tsp, synth, dn, channels, hidden, tokens
         assert np.array_equal(y[0], want[0]) and (y[1] == -4.0).all()
     status, y = run(good_ids, good_x)
     assert status == 0 and np.array_equal(y, want)
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("dn,channels,hidden", [(14, 3072, 1024), (14, 1024, 512), (14, 2048, 768), (14, 512, 256), (8, 2048, 1024), (8, 2304, 544),
+                                                (7, 1280, 736), (7, 1024, 992), (7, 256, 512)])
+def test_routed_m8_one_token(gpu, tsp, orc, synth, dn, channels, hidden, offset):
+    """One token: every split of a row over lanes and units, full and with a tail, the widest rows these kernels take, a token row and
+    route rows that only floats align (offset 1). Sums of f32 products: a rounding or two of 2^-24 per value and partial sum, an
+    error of less than 2^-20 of the row's size, 1e-12 of its square. (Stage bit 8: a Q6_K product sc * (q - 32) is a half.)"""
+    experts, selected = 6, 4
+    gate, up = synth.matrix(12, 91, hidden * experts, channels), synth.matrix(12, 92, hidden * experts, channels)
+    down = synth.matrix(dn, 93, channels * experts, hidden)
+    w = tsp.PlanarMoeWeights(gpu, 12, dn, channels, hidden, experts, gate, up, down)
+    ids = np.array([5, 0, 3, 2], dtype=np.uint32)
+    x = (synth.activations_f32(94, (1, channels)) * 0.1).astype(np.float32)
+    d_x = gpu.upload(np.concatenate([np.zeros((1, offset), dtype=np.float32), x], axis=1))[:, offset:]
+    h, y = gpu.full((selected, hidden + 4 + offset), -5.0), gpu.full((selected, channels + 4), -6.0)
+    tsp.planar_moe_routed_m8(gpu, w, gpu.upload(ids), d_x, 1, selected, h=h, y=y, x_stride=(channels + offset) * 4,
+                             h_stride=(hidden + 4 + offset) * 4, y_stride=(channels + 4) * 4)
+    h, y = h.cpu().numpy(), y.cpu().numpy()
+    ref_h, ref_y = orc.moe_routed_reference(12, dn, gate, up, down, channels, hidden, experts, ids, 1, selected, x, stage=8 if dn == 14 else 0, threads=8)
+    assert nmse(h[:, :hidden], ref_h) <= 1e-12 and nmse(y[:, :channels], ref_y) <= 1e-12
+    assert (h[:, hidden:] == -5.0).all() and (y[:, channels:] == -6.0).all() and gpu.error() == 0

@@ -3,14 +3,15 @@
 //   y[rid, c] = Wd[e] h[rid] . c                            down projection
 // with rid = t*selected + slot and e = ids[rid]. HBM-bound: the union records (one per distinct
 // expert, up to 8 tokens each) let every expert's weights be streamed from HBM once for all the
-// tokens that route to it. The sums are f32 everywhere, and so are weights and rows, except in Q4_K and Q6_K products of up to 2048
-// columns and 16-byte aligned rows: there a row is two halves under a power of two, 22 bits below its (or its slice's) largest
+// tokens that route to it. The sums are f32 everywhere, and so are weights and rows, except in Q4_K and Q6_K products of two or more tokens,
+// up to 2048 columns and 16-byte aligned rows: there a row is two halves under a power of two, 22 bits below its (or its slice's) largest
 // value, and the integer part of a Q6_K weight, sc * (q - 32), a half (above 2048 it loses its lowest bit).
 //
 // This file holds the entry points, the choice of a kernel and the per-element arm, which takes any planar encoding, width and
 // alignment. The kernels that stream the weights past the matrix cores are in record_resident.hip, record_stream.hip and
-// skinny.hip.
+// skinny.hip; those for one token, matrix-vector products in f32, in moe_one.hip.
 #include "decode.hpp"
+#include "moe_one.hpp"
 #include "record_resident.hpp"
 #include "record_stream.hpp"
 #include "skinny.hpp"
@@ -232,21 +233,22 @@ SkinnyMoe skinny_view(const SmallMoeArgs& a, const tsp_shared_rows* shared = nul
     return v;
 }
 
-// Which kernel takes the gate/up product. Q4_K rows of 2048 columns and two or more tokens: the record-resident one (27 us at 8
-// tokens and 512 hidden units where the streaming one takes 34). One token and a row of 1, 2, 4 or 8 super-blocks: one
-// super-block per wave (10.9 against 12.3 us at 2048 x 768, 8.2 against 8.9 at 1024 x 512). Everything else Q4_K up to 2560 columns
-// streams: what a workgroup holds in LDS, and the registers that stage a row, end there. Other encodings, wider rows and rows
-// that 16 bytes do not align go weight by weight.
-enum GateUpArm { GU_GENERIC, GU_RECORD, GU_FLAT, GU_STREAM };
+// Which kernel takes the gate/up product. One token: matrix-vector products up to 3072 columns (kernel times at 2048 x 512, 1024 x 512
+// and 2560 x 640: 6.3, 4.1 and 9.2 us; one super-block per wave takes 9.5 at the first, streaming 14.6 at the last). More tokens,
+// Q4_K rows of 2048 columns: the record-resident one (27 us at 8 tokens and 512 hidden units where the streaming one takes 34).
+// Everything else Q4_K up to 2560 columns streams: what a workgroup holds in LDS, and the registers that stage a row, end there.
+// Hidden widths that are no multiple of 16, in rows of 1, 2, 4 or 8 super-blocks: one super-block per wave. Other encodings, wider
+// rows and rows of several tokens that 16 bytes do not align go weight by weight.
+enum GateUpArm { GU_GENERIC, GU_ONE, GU_RECORD, GU_FLAT, GU_STREAM };
 GateUpArm gate_up_arm(const SmallMoeArgs& a, const tsp_shared_rows* shared) {
     const SkinnyMoe v = skinny_view(a, shared);
     if (a.gu.source_type != 12) return GU_GENERIC;
+    if (one_gate_up_takes(v)) return GU_ONE;
     if (record_gate_up_takes(v)) return GU_RECORD;
-    const bool flat = flat_gate_up_takes(v);
-    if (a.tokens > 1 || !flat) if (record_stream_gate_up_takes(v)) return GU_STREAM;
-    return flat ? GU_FLAT : GU_GENERIC;
+    if (record_stream_gate_up_takes(v)) return GU_STREAM;
+    return flat_gate_up_takes(v) ? GU_FLAT : GU_GENERIC;
 }
-// The first two build the union records themselves (and leave them in `meta` for the down launch): no launch of the union kernel
+// The record-resident and the streaming kernel build the union records themselves (and leave them in `meta` for the down launch): no launch of the union kernel
 // goes before them.
 bool gate_up_builds_union(const SmallMoeArgs& a, const tsp_shared_rows* shared = nullptr) {
     const GateUpArm arm = gate_up_arm(a, shared);
@@ -255,6 +257,7 @@ bool gate_up_builds_union(const SmallMoeArgs& a, const tsp_shared_rows* shared =
 
 int launch_gate_up(const SmallMoeArgs& a, hipStream_t s, const tsp_shared_rows* shared = nullptr) {
     switch (gate_up_arm(a, shared)) {
+    case GU_ONE: return launch_one_gate_up(skinny_view(a, shared), s);
     case GU_RECORD: return launch_record_gate_up(skinny_view(a, shared), s);
     case GU_STREAM: return launch_record_stream_gate_up(skinny_view(a, shared), s);
     case GU_FLAT: return flat_moe_gate_up(skinny_view(a, shared), s);
@@ -270,11 +273,13 @@ int launch_gate_up(const SmallMoeArgs& a, hipStream_t s, const tsp_shared_rows* 
     return launch_status("gate_up_generic");
 }
 
-// Q6_K rows of 1, 2, 4 or 8 super-blocks keep one super-block per wave (19 us at config 2's 512 hidden units where the
-// streaming kernel takes 23); its other widths up to 2048 columns and the 32-weight blocks up to 2560 stream, wider ones go
-// weight by weight.
+// One token: matrix-vector products up to 1024 columns (5.2 us at 512 -> 2048 Q6_K, one super-block per wave 6.6; 5.6 at 640 -> 2560
+// Q8_0, streaming 9.2). Q6_K rows of 1, 2, 4 or 8 super-blocks keep one super-block per wave (19 us at 512 hidden units and eight
+// tokens where the streaming kernel takes 23); its other widths up to 2048 columns and the 32-weight blocks up to 2560 stream,
+// wider ones go weight by weight.
 int launch_down(const SmallMoeArgs& a, hipStream_t s, const tsp_shared_rows* shared = nullptr) {
     const SkinnyMoe v = skinny_view(a, shared);
+    if (one_down_takes(v)) return launch_one_down(v, s);
     if (flat_down_takes(v)) return flat_moe_down(v, s);
     if (record_stream_down_takes(v)) return launch_record_stream_down(v, s);
     TSP_REQUIRE(!shared, "the always-on expert rides only on the matrix-core small-row kernels");
