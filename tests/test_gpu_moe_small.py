@@ -418,3 +418,64 @@ def test_routed_m8_one_token(gpu, tsp, orc, synth, dn, channels, hidden, offset)
     ref_h, ref_y = orc.moe_routed_reference(12, dn, gate, up, down, channels, hidden, experts, ids, 1, selected, x, stage=8 if dn == 14 else 0, threads=8)
     assert nmse(h[:, :hidden], ref_h) <= 1e-12 and nmse(y[:, :channels], ref_y) <= 1e-12
     assert (h[:, hidden:] == -5.0).all() and (y[:, channels:] == -6.0).all() and gpu.error() == 0
+
+
+@pytest.mark.parametrize("dn,channels,hidden,experts,selected,tokens", [(8, 256, 1280, 20, 16, 8), (14, 512, 1280, 6, 6, 5), (7, 3328, 96, 4, 1, 3),
+                                                                        (14, 2048, 512, 64, 10, 8), (8, 3328, 640, 8, 2, 1), (7, 512, 1056, 8, 3, 2)])
+def test_routed_m8_few_tokens(gpu, tsp, orc, synth, dn, channels, hidden, experts, selected, tokens):
+    """Experts met by one, two and many tokens, routes on both sides of the sixty-fourth, a token with the same expert twice, the splits of
+    wide rows over lanes, rows that only floats align; and the union block that the call leaves for its caller. A row's bits don't depend on
+    the tokens beside it. Sums of f32 products: see the test of one token."""
+    gate, up = synth.matrix(12, 95, hidden * experts, channels), synth.matrix(12, 96, hidden * experts, channels)
+    down = synth.matrix(dn, 97, channels * experts, hidden)
+    w = tsp.PlanarMoeWeights(gpu, 12, dn, channels, hidden, experts, gate, up, down)
+    rng = np.random.default_rng(channels + tokens)
+    ids = np.stack([rng.permutation(experts)[:selected] for _ in range(tokens)]).astype(np.uint32)
+    ids[0, -1] = ids[0, 0]
+    x = (synth.activations_f32(98, (tokens, channels + 1)) * 0.1).astype(np.float32)
+    routes = tokens * selected
+    w.union_meta.fill_(-1)
+
+    def run(rows, x_rows):
+        h, y = gpu.full((rows.size, hidden + 1), -5.0), gpu.full((rows.size, channels + 4), -6.0)
+        tsp.planar_moe_routed_m8(gpu, w, gpu.upload(rows.reshape(-1)), gpu.upload(x_rows)[:, 1:], len(rows), selected, h=h, y=y, x_stride=(channels + 1) * 4,
+                                 h_stride=(hidden + 1) * 4, y_stride=(channels + 4) * 4)
+        return h.cpu().numpy(), y.cpu().numpy()
+
+    h, y = run(ids, x)
+    if tokens > 1:
+        want, _ = orc.union_metadata(experts, selected, tokens, hidden, channels, ids.reshape(-1).tolist(), poison=0xFFFFFFFF)
+        assert np.array_equal(w.union_meta.cpu().numpy().view(np.uint32), np.asarray(want, dtype=np.uint32))
+    ref_h, ref_y = orc.moe_routed_reference(12, dn, gate, up, down, channels, hidden, experts, ids.reshape(-1), tokens, selected,
+                                            np.ascontiguousarray(x[:, 1:]), stage=8 if dn == 14 else 0, threads=8)
+    assert nmse(h[:, :hidden], ref_h) <= 1e-12 and nmse(y[:, :channels], ref_y) <= 1e-12
+    assert (h[:, hidden:] == -5.0).all() and (y[:, channels:] == -6.0).all() and gpu.error() == 0
+    if tokens > 2:
+        part_h, part_y = run(ids[-2:], np.ascontiguousarray(x[-2:]))
+        assert np.array_equal(part_h, h[routes - 2 * selected:]) and np.array_equal(part_y, y[routes - 2 * selected:])
+
+
+@pytest.mark.parametrize("tokens", [1, 2, 3])
+def test_routed_m8_largest_rows(gpu, tsp, orc, synth, tokens):
+    """Rows near the largest float, whose sums with the codes pass it before the block scales bring them back: finite results, no error. The
+    gates are all minima, below -1e30, and close; only the always-on sum of the up product has to hold."""
+    channels, hidden, experts = 2048, 64, 4
+    gate, up = synth.matrix(12, 99, hidden * experts, channels), synth.matrix(12, 100, hidden * experts, channels)
+    tiny = np.array([2.0 ** -24], dtype=np.float16).view(np.uint8)
+    gate.reshape(-1, 144)[:, 0:2] = 0
+    gate.reshape(-1, 144)[:, 2:4] = tiny
+    up.reshape(-1, 144)[:, 0:2] = tiny
+    up.reshape(-1, 144)[:, 2:4] = 0
+    w = tsp.PlanarMoeWeights(gpu, 12, 8, channels, hidden, experts, gate, up, synth.matrix(8, 101, channels * experts, hidden))
+    x = np.full((tokens, channels), 3e37, dtype=np.float32)
+    x[-1] = 1.0  # an ordinary row beside them
+    x[0, 7] = 1e37
+    if tokens == 1:
+        x[0] = 3e37
+    h, y = tsp.planar_moe_routed_m8(gpu, w, gpu.upload(np.array([[1, 2]] * tokens, dtype=np.uint32).reshape(-1)), gpu.upload(x), tokens, 2)
+    h, y = h.cpu().numpy(), y.cpu().numpy()
+    assert gpu.error() == 0 and np.isfinite(h).all() and np.isfinite(y).all()
+    if tokens > 1:
+        ref_h, _ = orc.moe_routed_reference(12, 8, gate, up, synth.matrix(8, 101, channels * experts, hidden), channels, hidden, experts,
+                                            np.array([1, 2], dtype=np.uint32), 1, 2, x[-1:], threads=4)
+        assert nmse(h[-2:], ref_h) <= 1e-12

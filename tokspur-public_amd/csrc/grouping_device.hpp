@@ -1,4 +1,4 @@
-// Device code shared by grouping.hip, gemm.hip and record_resident.hip: the task list of the grouped GEMMs and the union
+// Device code shared by grouping.hip, gemm.hip and moe_few.hip: the task list of the grouped GEMMs and the union
 // records of a step of at most eight tokens.
 #pragma once
 #include "tsp_common.hpp"

@@ -12,7 +12,6 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 enum BKind : int { B_Q4K_RAW = 0, B_Q4K_PLANAR = 1, B_Q6K_PLANAR = 2 };
@@ -69,14 +68,6 @@ __device__ __forceinline__ f16x2 fma2(f16x2 a, f16x2 b, f16x2 c) { return __buil
 __device__ __forceinline__ uint32_t spread01(uint32_t codes, uint32_t hi) { return __builtin_amdgcn_perm(hi, codes, 0x04010400u); }
 __device__ __forceinline__ uint32_t spread23(uint32_t codes, uint32_t hi) { return __builtin_amdgcn_perm(hi, codes, 0x04030402u); }
 
-// Eight codes 0..15 (one per byte of c0, c1) times the integer scale: (1024 + q) * sc - 1024 * sc, exact in f16.
-__device__ __forceinline__ f16x8 scaled8_q4(uint32_t c0, uint32_t c1, f16x2 sc, f16x2 bias) {
-    constexpr uint32_t K = 0x64646464u;  // 0x64xx = 1024 + xx
-    const f16x2 p0 = fma2(as_h2(spread01(c0, K)), sc, bias), p1 = fma2(as_h2(spread23(c0, K)), sc, bias);
-    const f16x2 p2 = fma2(as_h2(spread01(c1, K)), sc, bias), p3 = fma2(as_h2(spread23(c1, K)), sc, bias);
-    return f16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
-}
-
 // Eight int8 quants (two dwords) as exact halves: q ^ 0x80 = q + 128 in 0..255, 0x6400 | u = 1024 + u, minus 1152.
 __device__ __forceinline__ f16x8 quants8(uint32_t w0, uint32_t w1) {
     constexpr uint32_t K = 0x64646464u;
@@ -112,18 +103,6 @@ __device__ __forceinline__ bf16x8 quants8_bf16(uint32_t w0, uint32_t w1) {
     auto f = [](uint32_t w, int i) { return float(int(int8_t(w >> (8 * i)))); };
     return __builtin_bit_cast(bf16x8, u32x4{two_tops(f(w0, 0), f(w0, 1)), two_tops(f(w0, 2), f(w0, 3)), two_tops(f(w1, 0), f(w1, 1)), two_tops(f(w1, 2), f(w1, 3))});
 }
-__device__ __forceinline__ bf16x8 codes8_bf16(uint32_t w0, uint32_t w1) {
-    auto f = [](uint32_t w, int i) { return float((w >> (8 * i)) & 0xffu); };
-    return __builtin_bit_cast(bf16x8, u32x4{two_tops(f(w0, 0), f(w0, 1)), two_tops(f(w0, 2), f(w0, 3)), two_tops(f(w1, 0), f(w1, 1)), two_tops(f(w1, 2), f(w1, 3))});
-}
-// Eight codes 0 .. 15: as the float8 (e4m3) of the same bits a code q is q 2^-9, subnormal up to 7 and the first binade above, and
-// one conversion turns two of them into bf16 under a power of two.
-__device__ __forceinline__ bf16x8 nibbles8_bf16(uint32_t w0, uint32_t w1) {
-    const bf16x2 p0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 512.0f, false), p1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 512.0f, true);
-    const bf16x2 p2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 512.0f, false), p3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 512.0f, true);
-    return bf16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
-}
-
 // Sixteen weights of a Q5_1 block as two fragments. Element e is nibble e % 16 (low for e < 16, high above) of byte e % 16 with bit e
 // of the block's fifth-bit word on top; the lane's k-half takes elements 16 khalf .. 16 khalf + 15. A weight is the half nearest to
 // d * q + m (bits: the k-half's sixteen fifth bits): q exact as a half, one packed fused multiply-add, one rounding (the f32 evaluation rounds the sum to f32 first,
@@ -189,25 +168,10 @@ __device__ __forceinline__ HdrQ4 decode_hdr_q4k(const RawHdrQ4& r) {
     return h;
 }
 
-template <int BKIND>
-__device__ __forceinline__ HdrQ4 load_hdr_q4k(const uint8_t* base, const tsp_planar_spec& s, uint64_t row, uint32_t bpr, uint32_t b) {
-    return decode_hdr_q4k<BKIND>(fetch_hdr_q4k<BKIND>(base, s, row, bpr, b));
-}
-
 // Fragments of pair P: bytes 16h..16h+15 of the 32-byte pair; low nibbles (HI = 0) are sub-block 2P, high nibbles
 // sub-block 2P+1. Fragment f of a half covers activation columns HI*32 + 16h + f*8 .. +8 of the 64-column slab.
-template <int P, int HI>
-__device__ __forceinline__ void frags_q4k(const u32x4& raw, const HdrQ4& h, f16x8 frag[2]) {
-    constexpr uint32_t M4 = 0x0f0f0f0fu;
-    const uint32_t sc = (h.sc[P >> 1] >> ((P & 1) * 16 + HI * 8)) & 0xffu;
-    const f16x2 s2 = splat(float(sc)), bias = s2 * splat(-1024.0f);
-    frag[0] = scaled8_q4((raw[0] >> (4 * HI)) & M4, (raw[1] >> (4 * HI)) & M4, s2, bias);
-    frag[1] = scaled8_q4((raw[2] >> (4 * HI)) & M4, (raw[3] >> (4 * HI)) & M4, s2, bias);
-}
-
-// The same fragments with the columns of every eight in the order (0, 2, 1, 3, 4, 6, 5, 7), for activations stored in
-// that order: one mask-or per pair of weights instead of a mask and two byte permutes per four. Low nibbles become
-// 1024 + q, high nibbles stay in place as 1024 + 16 q and take the scale sc / 16 (exact: sc < 64).
+// The columns of every eight come in the order (0, 2, 1, 3, 4, 6, 5, 7), for activations stored in that order: one mask-or per pair
+// of weights instead of a mask and two byte permutes per four. Low nibbles become 1024 + q, high nibbles stay in place as 1024 + 16 q and take the scale sc / 16 (exact: sc < 64).
 // (w & mask) | bits is one instruction (v_and_or_b32) only when the constants sit in registers: a VOP3 instruction of
 // this target takes no literal, and with two literals the compiler emits an and plus an or. The kernel therefore pins
 // the three constants to registers once and hands them to the unpacking.

@@ -1,20 +1,14 @@
 // Routed MoE for 1..8 token rows (decode and speculative verify) on Pack v3 planar experts:
 //   h[rid, r] = silu(Wg[e] x_t . r) * (Wu[e] x_t . r)      gate + up + SwiGLU, one kernel
 //   y[rid, c] = Wd[e] h[rid] . c                            down projection
-// with rid = t*selected + slot and e = ids[rid]. HBM-bound: the union records (one per distinct
-// expert, up to 8 tokens each) let every expert's weights be streamed from HBM once for all the
-// tokens that route to it. The sums are f32 everywhere, and so are weights and rows, except in Q4_K and Q6_K products of two or more tokens,
-// up to 2048 columns and 16-byte aligned rows: there a row is two halves under a power of two, 22 bits below its (or its slice's) largest
-// value, and the integer part of a Q6_K weight, sc * (q - 32), a half (above 2048 it loses its lowest bit).
+// with rid = t*selected + slot and e = ids[rid]. HBM-bound. Rows, sums and weights are f32 or more, but for the integer part of a
+// Q6_K weight up to 2048 columns, sc * (q - 32), which is a half (above 2048 in size it loses its lowest bit).
 //
 // This file holds the entry points, the choice of a kernel and the per-element arm, which takes any planar encoding, width and
-// alignment. The kernels that stream the weights past the matrix cores are in record_resident.hip, record_stream.hip and
-// skinny.hip; those for one token, matrix-vector products in f32, in moe_one.hip.
+// alignment on the union records (one per distinct expert, up to 8 tokens each). The kernels for Q4_K gate/up and for down rows
+// that fit in LDS are in moe_few.hip.
 #include "decode.hpp"
-#include "moe_one.hpp"
-#include "record_resident.hpp"
-#include "record_stream.hpp"
-#include "skinny.hpp"
+#include "moe_few.hpp"
 
 using namespace tsp;
 
@@ -222,9 +216,9 @@ uint32_t record_slots(const SmallMoeArgs& a) {
     return routes < 128 ? routes : 128;
 }
 
-SkinnyMoe skinny_view(const SmallMoeArgs& a, const tsp_shared_rows* shared = nullptr) {
-    SkinnyMoe v{a.pair_lo, a.pair_hi, a.down, a.ids, a.meta, a.x, a.h, a.y, a.x_stride, a.h_stride, a.y_stride,
-                a.channels, a.hidden, a.experts, a.selected, a.tokens, record_slots(a), a.gu, a.dn, a.error_word};
+FewMoe few_view(const SmallMoeArgs& a, const tsp_shared_rows* shared = nullptr) {
+    FewMoe v{a.pair_lo, a.pair_hi, a.down, a.ids, a.meta, a.x, a.h, a.y, a.x_stride, a.h_stride, a.y_stride,
+             a.channels, a.hidden, a.experts, a.selected, a.tokens, a.gu, a.dn, a.error_word};
     if (shared) {
         v.shared_gate = static_cast<const uint8_t*>(shared->gate); v.shared_up = static_cast<const uint8_t*>(shared->up);
         v.shared_down = static_cast<const uint8_t*>(shared->down);
@@ -233,37 +227,23 @@ SkinnyMoe skinny_view(const SmallMoeArgs& a, const tsp_shared_rows* shared = nul
     return v;
 }
 
-// Which kernel takes the gate/up product. One token: matrix-vector products up to 3072 columns (kernel times at 2048 x 512, 1024 x 512
-// and 2560 x 640: 6.3, 4.1 and 9.2 us; one super-block per wave takes 9.5 at the first, streaming 14.6 at the last). More tokens,
-// Q4_K rows of 2048 columns: the record-resident one (27 us at 8 tokens and 512 hidden units where the streaming one takes 34).
-// Everything else Q4_K up to 2560 columns streams: what a workgroup holds in LDS, and the registers that stage a row, end there.
-// Hidden widths that are no multiple of 16, in rows of 1, 2, 4 or 8 super-blocks: one super-block per wave. Other encodings, wider
-// rows and rows of several tokens that 16 bytes do not align go weight by weight.
-enum GateUpArm { GU_GENERIC, GU_ONE, GU_RECORD, GU_FLAT, GU_STREAM };
-GateUpArm gate_up_arm(const SmallMoeArgs& a, const tsp_shared_rows* shared) {
-    const SkinnyMoe v = skinny_view(a, shared);
-    if (a.gu.source_type != 12) return GU_GENERIC;
-    if (one_gate_up_takes(v)) return GU_ONE;
-    if (record_gate_up_takes(v)) return GU_RECORD;
-    if (record_stream_gate_up_takes(v)) return GU_STREAM;
-    return flat_gate_up_takes(v) ? GU_FLAT : GU_GENERIC;
-}
-// The record-resident and the streaming kernel build the union records themselves (and leave them in `meta` for the down launch): no launch of the union kernel
-// goes before them.
-bool gate_up_builds_union(const SmallMoeArgs& a, const tsp_shared_rows* shared = nullptr) {
-    const GateUpArm arm = gate_up_arm(a, shared);
-    return arm == GU_RECORD || arm == GU_STREAM;
+// The shapes the always-on expert may ride with: Q4_K co-located gate/up and Q6_K planes down, columns a multiple of 256 up to 2048,
+// 16-byte aligned rows.
+bool shared_may_ride(const SmallMoeArgs& a) {
+    auto aligned16 = [](const void* p, uint64_t stride) { return reinterpret_cast<uintptr_t>(p) % 16 == 0 && stride % 16 == 0; };
+    return a.gu.source_type == 12 && a.dn.source_type == 14 && a.channels % 256 == 0 && a.channels <= 2048 && a.hidden % 256 == 0 && a.hidden <= 2048 &&
+           aligned16(a.x, a.x_stride) && aligned16(a.h, a.h_stride);
 }
 
+// Q4_K experts take the kernels of moe_few.hip, which build the union records themselves (and leave them in `meta` for the down launch
+// and the caller): no launch of the union kernel goes before them. Other encodings, and rows so wide that two of them don't fit in
+// LDS, go weight by weight.
+bool gate_up_builds_union(const SmallMoeArgs& a) { return few_gate_up_takes(few_view(a)); }
+
 int launch_gate_up(const SmallMoeArgs& a, hipStream_t s, const tsp_shared_rows* shared = nullptr) {
-    switch (gate_up_arm(a, shared)) {
-    case GU_ONE: return launch_one_gate_up(skinny_view(a, shared), s);
-    case GU_RECORD: return launch_record_gate_up(skinny_view(a, shared), s);
-    case GU_STREAM: return launch_record_stream_gate_up(skinny_view(a, shared), s);
-    case GU_FLAT: return flat_moe_gate_up(skinny_view(a, shared), s);
-    default: break;
-    }
-    TSP_REQUIRE(!shared, "the always-on expert rides only on the matrix-core small-row kernels");
+    const FewMoe v = few_view(a, shared);
+    if (few_gate_up_takes(v)) return launch_few_gate_up(v, s);
+    TSP_REQUIRE(!shared, "the always-on expert rides only on the kernels for few tokens");
     const dim3 grid((a.hidden + 3) / 4, record_slots(a));
     switch (a.gu.source_type) {
     case 12: TSP_LAUNCH("gate_up_generic", s, gate_up_generic<12><<<grid, 256, 0, s>>>(a)); break;
@@ -273,16 +253,10 @@ int launch_gate_up(const SmallMoeArgs& a, hipStream_t s, const tsp_shared_rows* 
     return launch_status("gate_up_generic");
 }
 
-// One token: matrix-vector products up to 1024 columns (5.2 us at 512 -> 2048 Q6_K, one super-block per wave 6.6; 5.6 at 640 -> 2560
-// Q8_0, streaming 9.2). Q6_K rows of 1, 2, 4 or 8 super-blocks keep one super-block per wave (19 us at 512 hidden units and eight
-// tokens where the streaming kernel takes 23); its other widths up to 2048 columns and the 32-weight blocks up to 2560 stream,
-// wider ones go weight by weight.
 int launch_down(const SmallMoeArgs& a, hipStream_t s, const tsp_shared_rows* shared = nullptr) {
-    const SkinnyMoe v = skinny_view(a, shared);
-    if (one_down_takes(v)) return launch_one_down(v, s);
-    if (flat_down_takes(v)) return flat_moe_down(v, s);
-    if (record_stream_down_takes(v)) return launch_record_stream_down(v, s);
-    TSP_REQUIRE(!shared, "the always-on expert rides only on the matrix-core small-row kernels");
+    const FewMoe v = few_view(a, shared);
+    if (few_down_takes(v)) return launch_few_down(v, s);
+    TSP_REQUIRE(!shared, "the always-on expert rides only on the kernels for few tokens");
     const dim3 grid((a.channels + 3) / 4, record_slots(a));
     switch (a.dn.source_type) {
     case 7: TSP_LAUNCH("down_generic", s, down_generic<7><<<grid, 256, 0, s>>>(a)); break;
@@ -326,8 +300,7 @@ extern "C" int tsp_planar_moe_routed_m8_shared(const tsp_small_moe* m, const tsp
     int rc = fill_common(m, &a, true);
     if (rc != TSP_OK) return rc;
     TSP_REQUIRE(shared->gate && shared->up && shared->down && shared->h && shared->y, "null device pointer");
-    TSP_REQUIRE(skinny_moe_supported(a.gu.source_type, a.dn.source_type, a.channels, a.hidden, a.x, a.x_stride, a.h, a.h_stride, true) &&
-                    a.gu.source_type == 12 && a.dn.source_type == 14,
+    TSP_REQUIRE(shared_may_ride(a),
                 "the always-on expert rides only with Q4_K co-located gate/up and Q6_K planes down, 16-byte aligned rows");
     TSP_REQUIRE(reinterpret_cast<uintptr_t>(shared->gate) % 16 == 0 && reinterpret_cast<uintptr_t>(shared->up) % 16 == 0 &&
                     reinterpret_cast<uintptr_t>(shared->down) % 16 == 0 && reinterpret_cast<uintptr_t>(shared->h) % 16 == 0 &&
@@ -346,7 +319,7 @@ extern "C" int tsp_planar_moe_routed_m8_shared(const tsp_small_moe* m, const tsp
                     "planar v3 small MoE outputs overlap inputs");
     TSP_REQUIRE(!ranges_overlap(shared->h, h_span, shared->y, y_span), "planar v3 small MoE outputs overlap inputs");
     const auto s = static_cast<hipStream_t>(stream);
-    if (m->tokens > 1 && !gate_up_builds_union(a, shared)) {
+    if (m->tokens > 1 && !gate_up_builds_union(a)) {
         rc = tsp_planar_union_build(m->ids, m->union_meta, m->experts, m->selected, m->tokens, m->hidden, m->channels, m->error_word, stream);
         if (rc != TSP_OK) return rc;
     }
