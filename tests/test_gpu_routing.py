@@ -484,3 +484,19 @@ def test_router_f32_batch_pairs(gpu, synth, tokens, columns, experts):
     scale = np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T
     assert (np.abs(got[:tokens, :experts] - want) <= 2e-6 * scale).all() and gpu.error() == 0
     assert (got[tokens] == 7.25).all() and (got[:, experts:] == 7.25).all()
+
+
+@pytest.mark.parametrize("tokens,columns,experts", [(90, 64, 17), (700, 288, 40), (1400, 2048, 128), (33, 544, 32), (9, 32, 9)])
+def test_router_f32_batch_more_tokens_than_experts(gpu, synth, tokens, columns, experts):
+    """The sliced form with its tiles in runs per XCD (their number no multiple of eight), and about as many tokens as experts; waves
+    with fewer units than they keep in flight, and with none; rows apart. f32 sums, as above."""
+    w = synth.activations_f32(synth.tensor_seed(5, 400 + tokens), (experts, columns))
+    x = synth.activations_f32(synth.tensor_seed(6, 400 + tokens), (tokens, columns + 4))
+    pitch = (experts + 3) // 4 * 4
+    out = gpu.full((tokens + 1, pitch), 7.25)
+    gpu.router_f32_batch(gpu.upload(w), gpu.upload(x), tokens, columns, experts, x_stride=(columns + 4) * 4, out=out, out_stride=pitch * 4)
+    got, x = out.cpu().numpy(), x[:, :columns]
+    want = x.astype(np.float64) @ w.astype(np.float64).T
+    scale = np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T
+    assert (np.abs(got[:tokens, :experts] - want) <= 2e-6 * scale).all() and gpu.error() == 0
+    assert (got[tokens] == 7.25).all() and (got[:, experts:] == 7.25).all()

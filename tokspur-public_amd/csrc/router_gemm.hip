@@ -174,52 +174,79 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
 // Fewer tokens than fill the chip with 64 x 64 tiles (eight of them for a draft's tokens): a workgroup owns ET * 16 experts x
 // TT * 16 tokens, its eight waves a slice of the columns each, and the eight partial tiles are added in LDS in wave order.
-// Operands go straight from memory into the fragments of v_mfma_f32_16x16x4_f32: lane l holds four consecutive columns of
-// row l % 16 of either operand, one column per instruction, so no LDS round trip stands between a wave's requests and its
-// products and all a wave needs is in flight a batch of kUnits steps ahead. Bound by the latency of one trip to memory and the matrix
-// rate of f32 (4 x 32 cycles per 16 columns and tile pair) at eight waves per tile. 512 experts x
-// 2048 columns: 203 tokens 42.6 -> 12.8, 400 tokens 42.9 -> 17.2.
+// Operands come in whole lines, 32 columns of the tile's rows at a time, into LDS of the wave's own (nobody else's: no barrier in the
+// loop), two to four such units ahead, and are read as the fragments of v_mfma_f32_16x16x4_f32: lane l holds four consecutive
+// columns of row l % 16 of either operand, one column per instruction. (Loaded from memory in that order every request touches 64
+// separate pieces and keeps the address unit busy for some 70 cycles, three times as long as whole lines do, which is what bound this
+// form.) Bound by the matrix rate of f32 (4 x 32 cycles per 16 columns and tile pair) and, at 32 x 32, by what the unit's lines
+// take beside it. 2048 columns, 512 experts: 9 tokens 7.8 -> 5.7 us, 100 9.4 -> 6.2, 203 13.0 -> 8.8, 400 18.2 -> 14.2; 128 experts:
+// 300 tokens 9.6 -> 6.1, 1400 18.9 -> 13.9.
 constexpr uint32_t kSlices = 8;
 typedef float acc4 __attribute__((ext_vector_type(4)));
 
+// Units of 32 columns in flight per wave: what 144 KB of LDS hold for eight waves.
+constexpr int sliced_depth(int et, int tt) { return 9 / (et + tt); }
+constexpr uint32_t sliced_lds(int et, int tt) { return kSlices * sliced_depth(et, tt) * (et + tt) * 2048; }
+
 template <int ET, int TT>
 __global__ __launch_bounds__(512) void router_f32_sliced(RouterArgs a) {
-    __shared__ __attribute__((aligned(16))) float sums[kSlices * ET * TT * 256];
-    const uint32_t token0 = (blockIdx.x / a.expert_tiles) * (TT * 16), expert0 = (blockIdx.x % a.expert_tiles) * (ET * 16);
-    const uint32_t tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
+    constexpr int kTiles = ET + TT, kDepth = sliced_depth(ET, TT);
+    constexpr uint32_t kUnitBytes = kTiles * 2048;
+    extern __shared__ __attribute__((aligned(16))) float sums[];  // [wave][unit in flight][tile][16 rows][128 bytes], then the partial tiles
+    // more tokens than experts: an XCD (blockIdx % 8) takes a run of token blocks with all their experts, so that the tokens pass one
+    // L2 each (1024 columns, 64 experts, 2048 tokens: 7.6 -> 5.8 us)
+    const uint32_t tile = a.tokens > a.experts ? (blockIdx.x % 8) * a.tiles_per_xcd + blockIdx.x / 8 : blockIdx.x;
+    if (tile >= a.tiles) return;
+    const uint32_t token0 = (tile / a.expert_tiles) * (TT * 16), expert0 = (tile % a.expert_tiles) * (ET * 16);
+    const uint32_t tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
     const uint32_t r16 = lane % 16, k4 = lane / 16;
-    const float* xrow[TT];
-    const float* wrow[ET];
+    uint8_t* const mine = reinterpret_cast<uint8_t*>(sums) + wave * (kDepth * kUnitBytes);
+    const uint32_t mine_lds = __builtin_amdgcn_readfirstlane(lds_address(mine));
+    // request q takes rows 8 q .. 8 q + 7 of the tiles (tokens first), eight neighbouring lanes a whole line; position p of row r holds chunk
+    // p ^ (r / 2) % 8. Tails re-read a valid row.
+    const float* from[2 * kTiles];
 #pragma unroll
-    for (int t = 0; t < TT; ++t) xrow[t] = a.input + uint64_t(min(token0 + t * 16 + r16, a.tokens - 1)) * a.input_stride + k4 * 4;
-#pragma unroll
-    for (int e = 0; e < ET; ++e) wrow[e] = a.weights + uint64_t(min(expert0 + e * 16 + r16, a.experts - 1)) * a.columns + k4 * 4;
-    acc4 acc[ET][TT] = {};
-    // 16-column units of this wave's slice
-    const uint32_t units = a.columns / 16, per_wave = (units + kSlices - 1) / kSlices;
-    const uint32_t first = wave * per_wave, last = min(first + per_wave, units);
-    constexpr uint32_t kUnits = 8 / (ET * TT > 2 ? 2 : 1);
-    for (uint32_t u0 = first; u0 < last; u0 += kUnits) {
-        acc4 fx[kUnits][TT], fw[kUnits][ET];
-#pragma unroll
-        for (uint32_t j = 0; j < kUnits; ++j) {
-            const uint32_t k = min(u0 + j, last - 1) * 16;  // past the slice: its last unit again, not multiplied
-#pragma unroll
-            for (int t = 0; t < TT; ++t) fx[j][t] = *reinterpret_cast<const acc4*>(xrow[t] + k);
-#pragma unroll
-            for (int e = 0; e < ET; ++e) fw[j][e] = *reinterpret_cast<const acc4*>(wrow[e] + k);
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < kUnits; ++j) {
-            if (u0 + j >= last) break;  // uniform over the wave
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-#pragma unroll
-                for (int e = 0; e < ET; ++e)
-#pragma unroll
-                    for (int t = 0; t < TT; ++t) acc[e][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(fx[j][t][c], fw[j][e][c], acc[e][t], 0, 0, 0);
-        }
+    for (uint32_t q = 0; q < 2 * kTiles; ++q) {
+        const uint32_t row = q * 8 + lane / 8, chunk = (lane % 8) ^ (4 * (q % 2) + lane / 16);
+        from[q] = (q < 2 * TT ? a.input + uint64_t(min(token0 + row, a.tokens - 1)) * a.input_stride
+                              : a.weights + uint64_t(min(expert0 + row - 16 * TT, a.experts - 1)) * a.columns) + chunk * 4;
     }
+    acc4 acc[ET][TT] = {};
+    // 32-column units of this wave's slice
+    const uint32_t units = a.columns / 32, per_wave = (units + kSlices - 1) / kSlices;
+    const uint32_t first = min(wave * per_wave, units), last = min(first + per_wave, units);
+    auto request = [&](uint32_t unit, uint32_t slot) {  // every request unconditional: past the end the last unit again, unused
+        const uint32_t column = min(unit, last - 1) * 32;
+#pragma unroll
+        for (uint32_t q = 0; q < 2 * kTiles; ++q) load_to_lds_16(from[q] + column, mine_lds + slot * kUnitBytes + q * 1024);
+    };
+    if (first < last) {
+#pragma unroll
+        for (uint32_t d = 0; d < kDepth; ++d) request(first + d, d);
+        uint32_t slot = 0;
+        for (uint32_t u = first; u < last; ++u) {
+            wait_after_loads<2 * kTiles * (kDepth - 1)>();
+            acc4 f[2][kTiles];
+#pragma unroll
+            for (uint32_t g = 0; g < 2; ++g)
+#pragma unroll
+                for (uint32_t i = 0; i < kTiles; ++i)
+                    f[g][i] = *reinterpret_cast<const acc4*>(mine + slot * kUnitBytes + i * 2048 + r16 * 128 + (((4 * g + k4) ^ (r16 / 2)) * 16));
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the unit is in registers: another one goes there
+            request(u + kDepth, slot);
+            slot = slot + 1 == kDepth ? 0 : slot + 1;
+#pragma unroll
+            for (int g = 0; g < 2; ++g)
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+#pragma unroll
+                    for (int e = 0; e < ET; ++e)
+#pragma unroll
+                        for (int t = 0; t < TT; ++t) acc[e][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[g][t][c], f[g][TT + e][c], acc[e][t], 0, 0, 0);
+        }
+        wait_all_loads();  // requests that nobody reads: they must have landed before the stages are reused
+    }
+    __syncthreads();
 #pragma unroll
     for (int e = 0; e < ET; ++e)
 #pragma unroll
@@ -301,8 +328,9 @@ void launch_pairs(const RouterArgs& a, hipStream_t s) {
 template <int ET, int TT>
 void launch_sliced(RouterArgs a, hipStream_t s) {
     a.expert_tiles = (a.experts + ET * 16 - 1) / (ET * 16);
-    const uint32_t tiles = a.expert_tiles * ((a.tokens + TT * 16 - 1) / (TT * 16));
-    TSP_LAUNCH("router_f32_gemm", s, router_f32_sliced<ET, TT><<<tiles, 512, 0, s>>>(a));
+    a.tiles = a.expert_tiles * ((a.tokens + TT * 16 - 1) / (TT * 16));
+    a.tiles_per_xcd = (a.tiles + 7) / 8;
+    TSP_LAUNCH("router_f32_gemm", s, router_f32_sliced<ET, TT><<<a.tiles_per_xcd * 8, 512, sliced_lds(ET, TT), s>>>(a));
 }
 
 std::atomic<uint64_t> g_lds_raised{0};
@@ -329,6 +357,9 @@ extern "C" int tsp_router_f32_batch(const float* weights, const float* input, ui
     int device = 0;
     if (setup_pending(g_lds_raised, &device)) {
         TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(router_f32_gemm), hipFuncAttributeMaxDynamicSharedMemorySize, int(kLdsBytes)));
+        TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&router_f32_sliced<1, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, int(sliced_lds(1, 1))));
+        TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&router_f32_sliced<1, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, int(sliced_lds(1, 2))));
+        TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&router_f32_sliced<2, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, int(sliced_lds(2, 2))));
         setup_done(g_lds_raised, device);
     }
     RouterArgs a{};
@@ -341,8 +372,9 @@ extern "C" int tsp_router_f32_batch(const float* weights, const float* input, ui
     a.error_word = error_word;
     const auto s = static_cast<hipStream_t>(stream);
     // The sliced form as long as one round of its tiles (256 compute units) covers the product, on the smallest tile for which
-    // that holds: 16 x 16 (9 us a round at 2048 columns), 16 experts x 32 tokens (13 us), 32 x 32 (18 us; two rounds of it take 36 us, the
-    // 64 x 64 form 24 at 1024 tokens of 512 experts and 29 for a full round of its own). Rows so far apart that 64 of them span 4 GiB stay with the sliced form's 64-bit addresses.
+    // that holds: 16 x 16 (6 us a round at 2048 columns), 16 experts x 32 tokens (9 us), 32 x 32 (14 us; two rounds of it would take
+    // 28 us, the 64 x 64 form takes 21 at 600 tokens of 512 experts and 28 for a full round of its own). Rows so far apart that 64 of
+    // them span 4 GiB stay with the sliced form's 64-bit addresses.
     const bool near = 64 * input_stride_bytes < (1ull << 32);
     const auto tiles = [&](uint32_t e, uint32_t t) { return uint64_t((experts + e - 1) / e) * ((tokens + t - 1) / t); };
     // Up to eight tokens: two experts per workgroup, while the chip takes them in two rounds.
