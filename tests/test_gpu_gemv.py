@@ -421,3 +421,11 @@ def test_dense_mm_q8_f32_rows(gpu, tsp, orc, synth, lanes, tokens, cols, rows, p
     x[tokens // 2, cols - 1] = np.nan
     tsp.dense_mm_q8(gpu, tsp.LAYOUT_Q8_LANES_V1 if lanes else tsp.LAYOUT_GGUF, gpu.upload(matrix), gpu.upload(x), tokens, cols, rows)
     assert gpu.error() == tsp.ERRBIT_NONFINITE
+
+
+@pytest.mark.parametrize("tokens,rows", [(6, 20), (7, 1002), (10, 1008), (11, 16), (15, 4112)])
+def test_dense_mm_q8_lanes_half_rows(gpu, tsp, orc, synth, tokens, rows):
+    """Six to ten rows of 2560 columns in one pass, two workgroups to a row with its middle run shared, a last tile of four rows, a number
+    of rows that the cleared output does not take (five at a time), two passes of eight. The bound of the test above: one more addition."""
+    test_dense_mm_q8_f32_rows(gpu, tsp, orc, synth, True, tokens, 2560, rows, 0)
+

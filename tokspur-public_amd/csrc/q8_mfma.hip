@@ -8,7 +8,7 @@
 // LDS for all of K, so the result carries 22 significant bits of x: this is the f32 GEMV of the engine to within f32
 // accumulation error, at ~1.3 VALU operations per weight byte whatever the number of token rows. Rows of more than 2048
 // columns are staged as the floats they are, three bf16 pieces each (mfma_quant.hpp): fifteen operand rows for up to five
-// token rows, in the same LDS, or for up to ten where a workgroup can take half of the columns; more take more passes.
+// token rows, in the same LDS, or for up to ten where a workgroup takes half of the columns; more take more passes.
 //
 // Raw rows are only 2-byte aligned inside, so the bytes travel global -> registers -> LDS -> registers: a wave reads
 // its 32 weight rows x 8 blocks (272 contiguous bytes per row, 16-byte aligned because 8 blocks = 17 x 16 bytes) with
@@ -442,7 +442,9 @@ constexpr uint32_t kLaneRows = 16, kLaneStride = 560, kLaneTileBytes = kLaneRows
 constexpr uint32_t kLaneLoads = (kLaneRows * kRunChunks + kWave - 1) / kWave;  // 9 chunk loads per lane and run (the last half used)
 
 // ROWS = token rows staged: 8 (all of K per workgroup) or 16 (even workgroups the first half of a row's runs, odd ones the second,
-// each pair over its share of the tiles, both adding their f32 sums into an output the host cleared: the matrix is read once).
+// each pair over its share of the tiles, both adding their f32 sums into an output the host cleared: the matrix is read once); 5 and
+// 10: the same in f32, ten on rows of five runs only: either workgroup takes two and a half of them, and both read the third, which
+// costs less than the second pass over the matrix that five rows at a time take (151 936 rows, six tokens: 168 us of kernels, now 96).
 template <int DEPTH, int ROWS>
 __global__ __launch_bounds__(kThreads, 1) void q8_lanes_mfma_kernel(Q8MfmaArgs a) {
     constexpr bool F32 = ROWS % kF32Rows == 0;
@@ -455,8 +457,10 @@ __global__ __launch_bounds__(kThreads, 1) void q8_lanes_mfma_kernel(Q8MfmaArgs a
     const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
     const uint32_t n16 = lane % 16, kq = lane / 16;
     // K: the columns this workgroup multiplies, runs run0 .. run0 + runs - 1 of every row
-    const uint32_t K = a.columns / KSPLIT, chunks = K / 8, blocks = a.columns / 32, runs = blocks / kRunBlocks / KSPLIT, row_bytes = blocks * 34;
-    const uint32_t run0 = (blockIdx.x % KSPLIT) * runs;
+    constexpr bool kShared = F32 && KSPLIT == 2;  // the middle run is both workgroups'
+    const uint32_t part = blockIdx.x % KSPLIT, all_runs = a.columns / 32 / kRunBlocks;
+    const uint32_t K = a.columns / KSPLIT, chunks = K / 8, blocks = a.columns / 32, runs = (all_runs + (kShared ? 1 : 0)) / KSPLIT, row_bytes = blocks * 34;
+    const uint32_t run0 = part * (all_runs - runs);
     const uint32_t sharer = blockIdx.x / KSPLIT, sharers = gridDim.x / KSPLIT;  // the host launches a multiple of KSPLIT
     const uint32_t tiles = (a.rows + kLaneRows - 1) / kLaneRows;
     if (tid == 0) next_tile = 0;
@@ -467,7 +471,7 @@ __global__ __launch_bounds__(kThreads, 1) void q8_lanes_mfma_kernel(Q8MfmaArgs a
 
     uint32_t bad = 0;
     float4 xv[F32 ? kF32Rows : kMine][2];
-    if constexpr (F32) request_f32_rows<SETS>(a, K, run0 * (kRunBlocks * 32), xv);
+    if constexpr (F32) request_f32_rows<SETS>(a, K, part * K, xv);
     else request_token_rows<kRows>(a, K, run0 * (kRunBlocks * 32), xv);
 
     // chunk `id` of a tile: row id / 34 of the wave's 16, piece id % 34 of that row's run: pieces 0 and 1 are the run's scales
@@ -539,7 +543,7 @@ __global__ __launch_bounds__(kThreads, 1) void q8_lanes_mfma_kernel(Q8MfmaArgs a
 
     for (; t < share_end; t = t_next, t_next = take_tile()) {
         const uint32_t row0 = t * kLaneRows;
-        float acc[4] = {0, 0, 0, 0};  // token row 4 kq + v
+        float acc[SETS][4] = {};  // [set][token row 4 kq + v]
         auto item = [&](uint32_t g, auto set_tag) {
             store_run(set_tag);  // the previous item's reads were issued before this point; LDS serves a wave in order
             const uint32_t ahead = g + DEPTH;
@@ -555,7 +559,8 @@ __global__ __launch_bounds__(kThreads, 1) void q8_lanes_mfma_kernel(Q8MfmaArgs a
             uint4 q[8];  // q[j]: quant 8 kq + j of the run's sixteen blocks, one byte per block
 #pragma unroll
             for (int j = 0; j < 8; ++j) q[j] = *reinterpret_cast<const uint4*>(mine + 32 + (8 * kq + j) * 16);
-            float run_sum[4] = {0, 0, 0, 0};  // in f32 a run's blocks are added up by themselves
+            float run_sum[SETS][4] = {};  // in f32 a run's blocks are added up by themselves
+            const uint32_t columns_at = g * 64 * 8 - (kShared && part ? kRunBlocks / 2 * 4 * 8 : 0);  // of the run, in the staged rows
             auto& sums = F32 ? run_sum : acc;
             auto quad = [&](auto m_tag) {  // blocks 4 M .. 4 M + 3 of the run
                 constexpr int M = decltype(m_tag)::value;
@@ -583,27 +588,40 @@ __global__ __launch_bounds__(kThreads, 1) void q8_lanes_mfma_kernel(Q8MfmaArgs a
                     constexpr int kBase = 4 * M;
                     const int B = kBase + b;
                     const float scale_d = half_bits_to_float((scales[B / 2] >> (16 * (B % 2))) & 0xffffu);
-                    const uint32_t at = a_at[B % kVariants] + (g * 64 + (B / kVariants) * kVariants * 4) * 8;  // columns g * 512 + B * 32 + 8 kq of the lane's token row
+                    const uint32_t at = a_at[B % kVariants] + columns_at + (B / kVariants) * kVariants * 4 * 8;  // columns g * 512 + B * 32 + 8 kq of the lane's token row
                     const f32x4 zero{};
-                    f32x4 part;
+                    f32x4 product;
                     if constexpr (F32) {
-                        part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(a_hi + at), quants8_bf16(w[b][0], w[b][1]), zero, 0, 0, 0);
+                        const bf16x8 b_frag = quants8_bf16(w[b][0], w[b][1]);
+#pragma unroll
+                        for (int set = 0; set < SETS; ++set) {
+                            product = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(a_hi + set * 16 * K + at), b_frag, zero, 0, 0, 0);
+#pragma unroll
+                            for (int v = 0; v < 4; ++v) sums[set][v] = __builtin_fmaf(scale_d, product[v], sums[set][v]);
+                        }
                     } else {
                         const f16x8 b_frag = quants8(w[b][0], w[b][1]);
-                        part = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const f16x8*>(a_lo + at), b_frag, zero, 0, 0, 0);
-                        part = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const f16x8*>(a_hi + at), b_frag, part, 0, 0, 0);
-                    }
+                        product = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const f16x8*>(a_lo + at), b_frag, zero, 0, 0, 0);
+                        product = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const f16x8*>(a_hi + at), b_frag, product, 0, 0, 0);
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) sums[v] = __builtin_fmaf(scale_d, part[v], sums[v]);
+                        for (int v = 0; v < 4; ++v) sums[0][v] = __builtin_fmaf(scale_d, product[v], sums[0][v]);
+                    }
                 }
             };
-            quad(std::integral_constant<int, 0>{});
-            quad(std::integral_constant<int, 1>{});
-            quad(std::integral_constant<int, 2>{});
-            quad(std::integral_constant<int, 3>{});
+            // of the middle run the first workgroup takes the first half, the second the second: uniform
+            if (!kShared || part == 0 || g != 0) {
+                quad(std::integral_constant<int, 0>{});
+                quad(std::integral_constant<int, 1>{});
+            }
+            if (!kShared || part != 0 || g + 1 != runs) {
+                quad(std::integral_constant<int, 2>{});
+                quad(std::integral_constant<int, 3>{});
+            }
             if constexpr (F32) {
 #pragma unroll
-                for (int v = 0; v < 4; ++v) acc[v] += run_sum[v];
+                for (int set = 0; set < SETS; ++set)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) acc[set][v] += run_sum[set][v];
             }
         };
         for (uint32_t g = 0; g < runs; g += DEPTH) {  // the host picks a DEPTH that divides the number of runs
@@ -612,18 +630,23 @@ __global__ __launch_bounds__(kThreads, 1) void q8_lanes_mfma_kernel(Q8MfmaArgs a
         }
         const uint32_t r = row0 + n16;
         if constexpr (F32) {
-            f32_row_sums(acc, kq, back[0], [&](uint32_t m, float val) {
-                if (m >= a.m || r >= a.rows) return;
-                if (nonfinite(val)) bad = TSP_ERRBIT_NONFINITE;
-                a.y[uint64_t(m) * a.rows + r] = val;
-            });
+#pragma unroll
+            for (int set = 0; set < SETS; ++set) {
+                f32_row_sums(acc[set], kq, back[set], [&](uint32_t row, float val) {
+                    const uint32_t m = set * kF32Rows + row;
+                    if (m >= a.m || r >= a.rows) return;
+                    if (nonfinite(val)) bad = TSP_ERRBIT_NONFINITE;
+                    if constexpr (KSPLIT == 1) a.y[uint64_t(m) * a.rows + r] = val;
+                    else unsafeAtomicAdd(a.y + uint64_t(m) * a.rows + r, val);
+                });
+            }
             continue;
         }
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const uint32_t m = 4 * kq + v;  // with eight token rows the lanes with kq >= 2 hold repeats of rows 0 .. 7
             if (m < kRows && m < a.m && r < a.rows) {
-                const float val = acc[v] * inv_scale;
+                const float val = acc[0][v] * inv_scale;
                 if (nonfinite(val)) bad = TSP_ERRBIT_NONFINITE;
                 if constexpr (KSPLIT == 1) a.y[uint64_t(m) * a.rows + r] = val;
                 else unsafeAtomicAdd(a.y + uint64_t(m) * a.rows + r, val);
@@ -745,18 +768,31 @@ int q8_lanes_mfma(const void* matrix, const float* x, float* y, uint32_t columns
         TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_lanes_mfma_kernel<1, 16>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
         TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_lanes_mfma_kernel<2, 16>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
         TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_lanes_mfma_kernel<1, kF32Rows>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
+        TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_lanes_mfma_kernel<1, 2 * kF32Rows>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
         TSP_HIP(hipDeviceGetAttribute(&units_of[device], hipDeviceAttributeMultiprocessorCount, device));
         setup_done(raised, device);
     }
     const int compute_units = units_of[device];
     const uint32_t tiles = (rows + kLaneRows - 1) / kLaneRows;
     uint32_t grid = uint32_t(compute_units > 0 ? compute_units : 256);
+    // two workgroups (one per half of a row's runs) share each stretch of tiles; the output starts at zero
+    uint32_t pairs = grid / 2 ? grid / 2 : 1;
+    if (pairs * kWaves > tiles) pairs = (tiles + kWaves - 1) / kWaves;
+    auto clear = [&](float* out, uint32_t token_rows) {
+        const uint64_t count4 = uint64_t(token_rows) * rows / 4;
+        TSP_LAUNCH("clear_rows", s, clear_rows<<<uint32_t((count4 + 255) / 256), 256, 0, s>>>(reinterpret_cast<float4*>(out), count4));
+    };
+    if (columns > kHalvesColumns && width > kF32Rows && rows % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0) {
+        // 2560 columns: one pass for up to ten token rows and two for 16, where five at a time take two and four (151 936 rows with the
+        // top-64 behind: six rows 183 -> 111 us, 12 271 -> 212, 16 357 -> 217)
+        for_f32_passes(a, 2 * kF32Rows, [&](const Q8MfmaArgs& pass) {
+            clear(pass.y, pass.m);
+            TSP_LAUNCH("q8_lanes_mfma", s, q8_lanes_mfma_kernel<1, 2 * kF32Rows><<<2 * pairs, kThreads, lds_bytes, s>>>(pass));
+        });
+        return launch_status("q8_lanes_mfma");
+    }
     if (width > 8 && columns <= kHalvesColumns) {
-        // two workgroups (one per half of a row's runs) share each stretch of tiles; the output starts at zero
-        uint32_t pairs = grid / 2 ? grid / 2 : 1;
-        if (pairs * kWaves > tiles) pairs = (tiles + kWaves - 1) / kWaves;
-        const uint64_t count4 = uint64_t(width) * rows / 4;
-        TSP_LAUNCH("clear_rows", s, clear_rows<<<uint32_t((count4 + 255) / 256), 256, 0, s>>>(reinterpret_cast<float4*>(y), count4));
+        clear(y, width);
         if ((columns / 1024) % 2 == 0) TSP_LAUNCH("q8_lanes_mfma", s, q8_lanes_mfma_kernel<2, 16><<<2 * pairs, kThreads, lds_bytes, s>>>(a));
         else TSP_LAUNCH("q8_lanes_mfma", s, q8_lanes_mfma_kernel<1, 16><<<2 * pairs, kThreads, lds_bytes, s>>>(a));
         return launch_status("q8_lanes_mfma");
