@@ -429,3 +429,25 @@ def test_dense_mm_q8_lanes_half_rows(gpu, tsp, orc, synth, tokens, rows):
     of rows that the cleared output does not take (five at a time), two passes of eight. The bound of the test above: one more addition."""
     test_dense_mm_q8_f32_rows(gpu, tsp, orc, synth, True, tokens, 2560, rows, 0)
 
+
+@pytest.mark.parametrize("lanes,tokens,cols,rows", [(False, 9, 512, 14003), (False, 16, 1024, 14002), (False, 7, 2560, 31001), (True, 13, 1024, 37), (True, 16, 2048, 515),
+                                                    (True, 9, 2560, 1001)])
+def test_dense_mm_q8_odd_rows(gpu, tsp, orc, synth, lanes, tokens, cols, rows):
+    """Two workgroups to a matrix row whose sums meet in an output that starts on any float and whose rows end on any: all of it is cleared
+    and nothing around it. Rows of two halves keep 22 bits of their largest value, and f32 sums 2^-18 of sum |w x|."""
+    w = synth.matrix(8, 2700 + cols, rows, cols)
+    x = synth.activations_f32(2701 + tokens, (tokens, cols))
+    matrix = tsp.q8_lanes_pack_rows(cols, w) if lanes else w
+    whole = gpu.full((tokens * rows + 8,), -5.0)
+    for start in (1, 2, 4):
+        whole.fill_(-5.0)
+        out = whole[start:start + tokens * rows].view(tokens, rows)
+        tsp.dense_mm_q8(gpu, tsp.LAYOUT_Q8_LANES_V1 if lanes else tsp.LAYOUT_GGUF, gpu.upload(matrix), gpu.upload(x), tokens, cols, rows, out=out)
+        got = whole.cpu().numpy()
+        assert (got[:start] == -5.0).all() and (got[start + tokens * rows:] == -5.0).all() and gpu.error() == 0
+        got = got[start:start + tokens * rows].reshape(tokens, rows)
+        check = np.unique(np.r_[0:min(rows, 200), max(0, rows - 40):rows])
+        dense = orc.dequantize(8, np.ascontiguousarray(w.reshape(rows, -1)[check]).reshape(-1), len(check) * cols).reshape(len(check), cols).astype(np.float64)
+        x64 = x.astype(np.float64)
+        bound = 2.0 ** -18 * (np.abs(x64) @ np.abs(dense).T) + 2.0 ** -22 * np.abs(x64).max() * np.abs(dense).sum(axis=1)
+        assert (np.abs(got[:, check] - x64 @ dense.T) <= bound).all()

@@ -181,7 +181,7 @@ bool small_rows(const void* matrix, const float* x, uint64_t x_stride_bytes, uin
     if (!q8_small_takes(matrix, x, x_stride_bytes, columns, rows)) return false;
     if (x_stride_bytes != uint64_t(columns) * 4 || !q8_mfma_supported(matrix, x, columns, rows)) return true;
     if (columns <= 2048) return rows < (tokens > 8 ? 14000u : 24576u);
-    const uint32_t at_once = columns % 512 == 0 && rows % 4 == 0 ? 10 : 5;
+    const uint32_t at_once = columns % 512 == 0 ? 10 : 5;
     return rows < (tokens > 8 ? 22000u : 31000u) * ((tokens + at_once - 1) / at_once);
 }
 
@@ -238,7 +238,7 @@ extern "C" int tsp_dense_mm_q8(uint32_t layout, const void* matrix, uint64_t mat
     const bool whole = matrix && error_word && columns && columns % 32 == 0 && rows && rows <= 1000000 && uint64_t(columns / 32) * rows * 34 == matrix_bytes;
     const bool lanes = layout == TSP_LAYOUT_Q8_LANES_V1, raw = layout == TSP_LAYOUT_GGUF;
     const bool eight = whole && packed && (raw ? q8_mfma_supported(matrix, input, columns, rows) : lanes && q8_lanes_mfma_supported(matrix, input, columns, rows));
-    const bool sixteen = eight && (raw ? q8_mfma_supported_16(matrix, input, output, columns, rows) : q8_lanes_mfma_supported_16(matrix, input, output, columns, rows));
+    const bool sixteen = eight && (raw ? q8_mfma_supported_16(matrix, input, columns, rows) : q8_lanes_mfma_supported_16(matrix, input, columns, rows));
     for (uint32_t done = 0; done < tokens;) {
         const uint32_t left = tokens - done;
         const float* const from = reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(input) + uint64_t(done) * input_stride_bytes);

@@ -52,9 +52,17 @@ struct Q8MfmaArgs {
     uint32_t* error_word;
 };
 
-__global__ void clear_rows(float4* out, uint64_t count4) {
+// Any number of floats at any float's address: whole 16-byte pieces but for the ends. (For numbers of weight rows that four does not
+// divide: nine to sixteen token rows took two passes over the matrix there, ten by 151 934 x 2048 145 us where this way takes 86.)
+__global__ void clear_rows(float* out, uint64_t count) {
     const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < count4) out[i] = float4{0, 0, 0, 0};
+    const uint64_t ahead = (16 - reinterpret_cast<uintptr_t>(out) % 16) % 16 / 4, head = ahead < count ? ahead : count, pieces = (count - head) / 4;
+    if (i < pieces) reinterpret_cast<float4*>(out + head)[i] = float4{0, 0, 0, 0};
+    if (i < head) out[i] = 0;
+    if (i < count - head - 4 * pieces) out[head + 4 * pieces + i] = 0;
+}
+void clear_output(float* out, uint64_t count, hipStream_t s) {
+    TSP_LAUNCH("clear_rows", s, clear_rows<<<uint32_t((count / 4 + 3 + 255) / 256), 256, 0, s>>>(out, count));
 }
 
 // The token rows of a workgroup, [kRows, K] from column k0 on, in chunks of eight columns: chunk i = tid + j * kThreads is columns
@@ -679,10 +687,9 @@ bool q8_mfma_supported(const void* matrix, const float* x, uint32_t columns, uin
            reinterpret_cast<uintptr_t>(x) % 16 == 0;
 }
 
-bool q8_mfma_supported_16(const void* matrix, const float* x, const float* y, uint32_t columns, uint32_t rows) {
+bool q8_mfma_supported_16(const void* matrix, const float* x, uint32_t columns, uint32_t rows) {
     if (columns > kHalvesColumns) return q8_mfma_supported(matrix, x, columns, rows);  // in passes of its own
-    return q8_mfma_supported(matrix, x, columns, rows) && columns % 512 == 0 && rows >= 64 && rows % 4 == 0 &&
-           reinterpret_cast<uintptr_t>(y) % 16 == 0;
+    return q8_mfma_supported(matrix, x, columns, rows) && columns % 512 == 0 && rows >= 64;
 }
 
 int q8_mfma(const void* matrix, const float* x, float* y, uint32_t columns, uint32_t rows, uint32_t width, uint32_t* error_word, hipStream_t s) {
@@ -710,21 +717,17 @@ int q8_mfma(const void* matrix, const float* x, float* y, uint32_t columns, uint
     // two workgroups (one per half of the columns) share each run of tiles; the output starts at zero
     uint32_t pairs = grid / 2 ? grid / 2 : 1;
     if (pairs * kWaves > tiles) pairs = (tiles + kWaves - 1) / kWaves;
-    auto clear = [&](float* out, uint32_t token_rows) {
-        const uint64_t count4 = uint64_t(token_rows) * rows / 4;
-        TSP_LAUNCH("clear_rows", s, clear_rows<<<uint32_t((count4 + 255) / 256), 256, 0, s>>>(reinterpret_cast<float4*>(out), count4));
-    };
-    if (columns > kHalvesColumns && width > kF32Rows && columns % 512 == 0 && rows % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0) {
+    if (columns > kHalvesColumns && width > kF32Rows && columns % 512 == 0) {
         // 2560 columns, five groups to a half: one pass for 8 token rows and two for 16, where five at a time would take two and four
         // (151 936 rows, 8 token rows: 96 us against 166)
         for_f32_passes(a, 2 * kF32Rows, [&](const Q8MfmaArgs& pass) {
-            clear(pass.y, pass.m);
+            clear_output(pass.y, uint64_t(pass.m) * rows, s);
             TSP_LAUNCH("q8_mfma", s, q8_mfma_kernel<1, 2 * kF32Rows><<<2 * pairs, kThreads, lds_bytes, s>>>(pass));
         });
         return launch_status("q8_mfma");
     }
     if (width > 8 && columns <= kHalvesColumns) {
-        clear(y, width);
+        clear_output(y, uint64_t(width) * rows, s);
         if ((columns / 512) % 2 == 0) TSP_LAUNCH("q8_mfma", s, q8_mfma_kernel<2, 16><<<2 * pairs, kThreads, lds_bytes, s>>>(a));
         else TSP_LAUNCH("q8_mfma", s, q8_mfma_kernel<1, 16><<<2 * pairs, kThreads, lds_bytes, s>>>(a));
         return launch_status("q8_mfma");
@@ -748,10 +751,9 @@ bool q8_lanes_mfma_supported(const void* matrix, const float* x, uint32_t column
            reinterpret_cast<uintptr_t>(x) % 16 == 0;
 }
 
-bool q8_lanes_mfma_supported_16(const void* matrix, const float* x, const float* y, uint32_t columns, uint32_t rows) {
+bool q8_lanes_mfma_supported_16(const void* matrix, const float* x, uint32_t columns, uint32_t rows) {
     if (columns > kHalvesColumns) return q8_lanes_mfma_supported(matrix, x, columns, rows);
-    return q8_lanes_mfma_supported(matrix, x, columns, rows) && columns % 1024 == 0 && rows >= 32 && rows % 4 == 0 &&
-           reinterpret_cast<uintptr_t>(y) % 16 == 0;
+    return q8_lanes_mfma_supported(matrix, x, columns, rows) && columns % 1024 == 0 && rows >= 32;
 }
 
 int q8_lanes_mfma(const void* matrix, const float* x, float* y, uint32_t columns, uint32_t rows, uint32_t width, uint32_t* error_word,
@@ -778,21 +780,17 @@ int q8_lanes_mfma(const void* matrix, const float* x, float* y, uint32_t columns
     // two workgroups (one per half of a row's runs) share each stretch of tiles; the output starts at zero
     uint32_t pairs = grid / 2 ? grid / 2 : 1;
     if (pairs * kWaves > tiles) pairs = (tiles + kWaves - 1) / kWaves;
-    auto clear = [&](float* out, uint32_t token_rows) {
-        const uint64_t count4 = uint64_t(token_rows) * rows / 4;
-        TSP_LAUNCH("clear_rows", s, clear_rows<<<uint32_t((count4 + 255) / 256), 256, 0, s>>>(reinterpret_cast<float4*>(out), count4));
-    };
-    if (columns > kHalvesColumns && width > kF32Rows && rows % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0) {
+    if (columns > kHalvesColumns && width > kF32Rows) {
         // 2560 columns: one pass for up to ten token rows and two for 16, where five at a time take two and four (151 936 rows with the
         // top-64 behind: six rows 183 -> 111 us, 12 271 -> 212, 16 357 -> 217)
         for_f32_passes(a, 2 * kF32Rows, [&](const Q8MfmaArgs& pass) {
-            clear(pass.y, pass.m);
+            clear_output(pass.y, uint64_t(pass.m) * rows, s);
             TSP_LAUNCH("q8_lanes_mfma", s, q8_lanes_mfma_kernel<1, 2 * kF32Rows><<<2 * pairs, kThreads, lds_bytes, s>>>(pass));
         });
         return launch_status("q8_lanes_mfma");
     }
     if (width > 8 && columns <= kHalvesColumns) {
-        clear(y, width);
+        clear_output(y, uint64_t(width) * rows, s);
         if ((columns / 1024) % 2 == 0) TSP_LAUNCH("q8_lanes_mfma", s, q8_lanes_mfma_kernel<2, 16><<<2 * pairs, kThreads, lds_bytes, s>>>(a));
         else TSP_LAUNCH("q8_lanes_mfma", s, q8_lanes_mfma_kernel<1, 16><<<2 * pairs, kThreads, lds_bytes, s>>>(a));
         return launch_status("q8_lanes_mfma");
