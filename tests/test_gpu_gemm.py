@@ -906,3 +906,11 @@ def test_config3_moe_grouped_prefill(gpu, tsp, orc, synth):
         want = orc.mixture_reference(yh[t].astype(np.float64), wh[t].astype(np.float64), ysh[t].astype(np.float64), float(lh[t]))
         assert max_rel_error(out2[t], want) <= 1e-5
     assert gpu.error() == 0
+
+
+# Q6_K down of 512 hidden units either side of eight items of 128 channels to a compute unit, where a workgroup per item gives way to the
+# resident kernel: loads of none, a few, more than 32 and more than 64 rows
+@pytest.mark.parametrize("experts", [126, 128])
+def test_grouped_moe_q6_down_items(gpu, tsp, orc, synth, experts):
+    test_grouped_moe_2048_columns_few_rows(gpu, tsp, orc, synth, 90, 512, experts, 4)
+

@@ -929,7 +929,11 @@ int grouped_moe(const tsp_grouped_moe* m, const tsp_shared_expert* shared, void*
     if (rc != TSP_OK) return rc;
     const uint64_t shared_span = shared ? uint64_t(m->tokens) * shared->y_stride_bytes : 0;
     // At 512 columns the h rows fit the waves' registers (2048 x 512, 512 experts, Q5_1, 400 tokens: 319 us a sublayer against 325 with the rows in LDS).
-    const bool resident = resident_down_takes(down_type, m->channels, m->hidden) && uint64_t(routes) * m->y_stride_bytes < (1ull << 32) && shared_span < (1ull << 32);
+    // Q6_K with fewer than eight items of 128 channels to a compute unit: the resident kernel's start (tables, rows, the first tiles) weighs more than
+    // its stream, and a workgroup per item is through sooner (64 experts of 1024 x 512: 64 tokens 39 us a sublayer against 46, 700 tokens 54
+    // against 61, 5.7 items 80 against 82; 128 experts, 7.7 items 93 against 97; 128 experts of 2048, 8.2 items 59 against 54).
+    const bool brief = fast_down && uint64_t(l.bound) * m->channels < 8 * 256 * 128;
+    const bool resident = !brief && resident_down_takes(down_type, m->channels, m->hidden) && uint64_t(routes) * m->y_stride_bytes < (1ull << 32) && shared_span < (1ull << 32);
     const bool wide = !resident && wide_down_takes(down_type, m->channels, m->hidden) && y_span <= 0xffff0000u;
     if (resident || wide) {
         ResidentDownArgs r{};
