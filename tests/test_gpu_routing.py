@@ -66,6 +66,18 @@ def test_route_batch_ids_bit_exact(gpu, orc, synth, tokens, experts, selected):
     assert np.allclose(w.sum(axis=1), 1.0, rtol=1e-5)
 
 
+@pytest.mark.parametrize("experts", [1, 63, 65, 512, 513, 1025, 4095, 4096])
+def test_route_row_ends(gpu, orc, experts):
+    """The row's last, partly empty slots: the largest logits sit at its end, and what stands behind the row is larger still."""
+    selected = min(experts, 5)
+    logits = np.linspace(-3, 3, experts, dtype=np.float32)
+    padded = gpu.upload(np.concatenate([logits, np.full(4096, 50, dtype=np.float32)]))
+    ids, w = gpu.route(padded[:experts], selected, 0, True)
+    want_ids, want_w = orc.route_reference(logits.astype(np.float64), selected, 0, True)
+    assert np.array_equal(u32(ids)[0], want_ids)
+    assert np.allclose(w.cpu().numpy()[0], want_w, rtol=2e-5, atol=1e-9) and gpu.error() == 0  # the bound of the batch test above
+
+
 def lcg_values(state, count):
     """`count` draws of the 32-bit generator x -> 1664525 x + 1013904223 as float(int(x % 1993) - 996) / 997, and the state."""
     out = np.empty(count, dtype=np.float64)
