@@ -403,7 +403,8 @@ def test_routed_m8_streamed_errors(gpu, tsp, synth, dn, channels, hidden, tokens
 def test_routed_m8_one_token(gpu, tsp, orc, synth, dn, channels, hidden, offset):
     """One token: every split of a row over lanes and units, full and with a tail, the widest rows these kernels take, a token row and
     route rows that only floats align (offset 1). Sums of f32 products: a rounding or two of 2^-24 per value and partial sum, an
-    error of less than 2^-20 of the row's size, 1e-12 of its square. (Stage bit 8: a Q6_K product sc * (q - 32) is a half.)"""
+    error of less than 2^-20 of the row's size, 1e-12 of its square. (Stage bit 8: a Q6_K product sc * (q - 32) is a half, of route rows that
+    16 bytes align; of others every weight is the float that it decodes to.)"""
     experts, selected = 6, 4
     gate, up = synth.matrix(12, 91, hidden * experts, channels), synth.matrix(12, 92, hidden * experts, channels)
     down = synth.matrix(dn, 93, channels * experts, hidden)
@@ -415,7 +416,7 @@ def test_routed_m8_one_token(gpu, tsp, orc, synth, dn, channels, hidden, offset)
     tsp.planar_moe_routed_m8(gpu, w, gpu.upload(ids), d_x, 1, selected, h=h, y=y, x_stride=(channels + offset) * 4,
                              h_stride=(hidden + 4 + offset) * 4, y_stride=(channels + 4) * 4)
     h, y = h.cpu().numpy(), y.cpu().numpy()
-    ref_h, ref_y = orc.moe_routed_reference(12, dn, gate, up, down, channels, hidden, experts, ids, 1, selected, x, stage=8 if dn == 14 else 0, threads=8)
+    ref_h, ref_y = orc.moe_routed_reference(12, dn, gate, up, down, channels, hidden, experts, ids, 1, selected, x, stage=8 if dn == 14 and offset == 0 else 0, threads=8)
     assert nmse(h[:, :hidden], ref_h) <= 1e-12 and nmse(y[:, :channels], ref_y) <= 1e-12
     assert (h[:, hidden:] == -5.0).all() and (y[:, channels:] == -6.0).all() and gpu.error() == 0
 
@@ -425,7 +426,7 @@ def test_routed_m8_one_token(gpu, tsp, orc, synth, dn, channels, hidden, offset)
 def test_routed_m8_few_tokens(gpu, tsp, orc, synth, dn, channels, hidden, experts, selected, tokens):
     """Experts met by one, two and many tokens, routes on both sides of the sixty-fourth, a token with the same expert twice, the splits of
     wide rows over lanes, rows that only floats align; and the union block that the call leaves for its caller. A row's bits don't depend on
-    the tokens beside it. Sums of f32 products: see the test of one token."""
+    the tokens beside it. Sums of f32 products: see the test of one token. (Q6_K down rows: a second call with route rows that 16 bytes align.)"""
     gate, up = synth.matrix(12, 95, hidden * experts, channels), synth.matrix(12, 96, hidden * experts, channels)
     down = synth.matrix(dn, 97, channels * experts, hidden)
     w = tsp.PlanarMoeWeights(gpu, 12, dn, channels, hidden, experts, gate, up, down)
@@ -436,10 +437,10 @@ def test_routed_m8_few_tokens(gpu, tsp, orc, synth, dn, channels, hidden, expert
     routes = tokens * selected
     w.union_meta.fill_(-1)
 
-    def run(rows, x_rows):
-        h, y = gpu.full((rows.size, hidden + 1), -5.0), gpu.full((rows.size, channels + 4), -6.0)
+    def run(rows, x_rows, pad=1):
+        h, y = gpu.full((rows.size, hidden + pad), -5.0), gpu.full((rows.size, channels + 4), -6.0)
         tsp.planar_moe_routed_m8(gpu, w, gpu.upload(rows.reshape(-1)), gpu.upload(x_rows)[:, 1:], len(rows), selected, h=h, y=y, x_stride=(channels + 1) * 4,
-                                 h_stride=(hidden + 1) * 4, y_stride=(channels + 4) * 4)
+                                 h_stride=(hidden + pad) * 4, y_stride=(channels + 4) * 4)
         return h.cpu().numpy(), y.cpu().numpy()
 
     h, y = run(ids, x)
@@ -447,12 +448,18 @@ def test_routed_m8_few_tokens(gpu, tsp, orc, synth, dn, channels, hidden, expert
         want, _ = orc.union_metadata(experts, selected, tokens, hidden, channels, ids.reshape(-1).tolist(), poison=0xFFFFFFFF)
         assert np.array_equal(w.union_meta.cpu().numpy().view(np.uint32), np.asarray(want, dtype=np.uint32))
     ref_h, ref_y = orc.moe_routed_reference(12, dn, gate, up, down, channels, hidden, experts, ids.reshape(-1), tokens, selected,
-                                            np.ascontiguousarray(x[:, 1:]), stage=8 if dn == 14 else 0, threads=8)
+                                            np.ascontiguousarray(x[:, 1:]), stage=0, threads=8)
     assert nmse(h[:, :hidden], ref_h) <= 1e-12 and nmse(y[:, :channels], ref_y) <= 1e-12
     assert (h[:, hidden:] == -5.0).all() and (y[:, channels:] == -6.0).all() and gpu.error() == 0
-    if tokens > 2:
-        part_h, part_y = run(ids[-2:], np.ascontiguousarray(x[-2:]))
-        assert np.array_equal(part_h, h[routes - 2 * selected:]) and np.array_equal(part_y, y[routes - 2 * selected:])
+    for pad in (1, 4) if dn == 14 else (1,):
+        if pad != 1:
+            h, y = run(ids, x, pad)
+            _, ref_y = orc.moe_routed_reference(12, dn, gate, up, down, channels, hidden, experts, ids.reshape(-1), tokens, selected,
+                                                np.ascontiguousarray(x[:, 1:]), stage=8, threads=8)
+            assert nmse(h[:, :hidden], ref_h) <= 1e-12 and nmse(y[:, :channels], ref_y) <= 1e-12 and gpu.error() == 0
+        if tokens > 2:
+            part_h, part_y = run(ids[-2:], np.ascontiguousarray(x[-2:]), pad)
+            assert np.array_equal(part_h, h[routes - 2 * selected:]) and np.array_equal(part_y, y[routes - 2 * selected:])
 
 
 @pytest.mark.parametrize("tokens", [1, 2, 3])

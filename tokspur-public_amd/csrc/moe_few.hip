@@ -596,7 +596,8 @@ int launch(const char* name, const OneArgs& a, hipStream_t s) {
     return launch_status(name);
 }
 
-// Q6_K rows up to here have sc * (q - 32) as a half, wider ones the weight as it decodes: the per-element kernel.
+// Q6_K rows up to here, and aligned to 16 bytes, have sc * (q - 32) as a half; wider and other ones the weight as it decodes: the
+// per-element kernel, since nobody has asked for fewer bits there.
 constexpr uint32_t kMostHalves = 2048;
 // What few_rows stages of two activation rows at most, and the widest row whose loads one_row keeps all in flight.
 constexpr uint32_t kMostLds = 64 * 1024, kOneGateUp = 3072, kOneDown = 1024;
@@ -611,7 +612,8 @@ static bool few_fits(uint32_t type, uint32_t columns, uint64_t expert_bytes) {
 bool few_gate_up_takes(const FewMoe& m) { return m.gu.source_type == 12 && few_fits(12, m.channels, m.gu.planar_expert_bytes); }
 bool few_down_takes(const FewMoe& m) {
     const uint32_t type = m.dn.source_type;
-    return (type == 7 || type == 8 || (type == 14 && m.hidden <= kMostHalves)) && few_fits(type, m.hidden, m.dn.planar_expert_bytes);
+    const bool aligned = reinterpret_cast<uintptr_t>(m.h) % 16 == 0 && m.h_stride % 16 == 0;
+    return (type == 7 || type == 8 || (type == 14 && m.hidden <= kMostHalves && aligned)) && few_fits(type, m.hidden, m.dn.planar_expert_bytes);
 }
 
 static FewArgs few_args(const FewMoe& m, const OneArgs& a) {

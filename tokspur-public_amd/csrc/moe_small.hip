@@ -2,7 +2,7 @@
 //   h[rid, r] = silu(Wg[e] x_t . r) * (Wu[e] x_t . r)      gate + up + SwiGLU, one kernel
 //   y[rid, c] = Wd[e] h[rid] . c                            down projection
 // with rid = t*selected + slot and e = ids[rid]. HBM-bound. Rows, sums and weights are f32 or more, but for the integer part of a
-// Q6_K weight up to 2048 columns, sc * (q - 32), which is a half (above 2048 in size it loses its lowest bit).
+// Q6_K weight of up to 2048 columns against h rows that 16 bytes align: sc * (q - 32) is a half there (above 2048 in size it loses its lowest bit).
 //
 // This file holds the entry points, the choice of a kernel and the per-element arm, which takes any planar encoding, width and
 // alignment on the union records (one per distinct expert, up to 8 tokens each). The kernels for Q4_K gate/up and for down rows
@@ -236,8 +236,8 @@ bool shared_may_ride(const SmallMoeArgs& a) {
 }
 
 // Q4_K experts take the kernels of moe_few.hip, which build the union records themselves (and leave them in `meta` for the down launch
-// and the caller): no launch of the union kernel goes before them. Other encodings, and rows so wide that two of them don't fit in
-// LDS, go weight by weight.
+// and the caller): no launch of the union kernel goes before them. Other encodings, rows so wide that two of them don't fit in LDS, and
+// Q6_K down rows whose weights are to stay floats, go weight by weight.
 bool gate_up_builds_union(const SmallMoeArgs& a) { return few_gate_up_takes(few_view(a)); }
 
 int launch_gate_up(const SmallMoeArgs& a, hipStream_t s, const tsp_shared_rows* shared = nullptr) {
