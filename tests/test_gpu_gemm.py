@@ -914,3 +914,32 @@ def test_config3_moe_grouped_prefill(gpu, tsp, orc, synth):
 def test_grouped_moe_q6_down_items(gpu, tsp, orc, synth, experts):
     test_grouped_moe_2048_columns_few_rows(gpu, tsp, orc, synth, 90, 512, experts, 4)
 
+
+# loads on either side of six rows per expert, where 2048-column experts change their gate/up kernel, and of eight items of 128 channels to a
+# compute unit, where 512 hidden units change their down kernel
+@pytest.mark.parametrize("n,hidden", [(20, 256), (250, 256), (20, 512), (250, 512)])
+def test_grouped_moe_rows_whatever_company(gpu, tsp, synth, n, hidden):
+    """The always-on expert's rows have the bits of a separate call, whose two experts and one route a token choose other kernels than the 128
+    experts that it rides with, and a token's rows have the bits that they have in a chunk of half the size."""
+    channels, experts, selected = 2048, 128, 4
+    w = tsp.PlanarMoeWeights(gpu, 12, 14, channels, hidden, experts, synth.matrix(12, 3431, hidden * experts, channels), synth.matrix(12, 3432, hidden * experts, channels),
+                             synth.matrix(14, 3433, channels * experts, hidden))
+    rng = np.random.default_rng(n)
+    ids = np.stack([rng.permutation(experts)[:selected] for _ in range(n)]).astype(np.uint32)
+    ids[:, 0] = 0  # one expert of many rows
+    ids[:, 1:][ids[:, 1:] == 0] = 1
+    x = gpu.upload(synth.round_bf16(synth.activations_f32(3434 + n, (n, channels))))
+    sg, su, sd = synth.matrix(12, 3435, hidden, channels), synth.matrix(12, 3436, hidden, channels), synth.matrix(14, 3437, channels, hidden)
+    shared = tsp.PlanarSharedExpert(gpu, channels, hidden, sg, su, sd)
+
+    def routed(weights, chosen, tokens, per_token, **always_on):
+        scratch = tsp.GroupedScratch(gpu, tokens, per_token, weights.experts, channels, hidden, with_shared=bool(always_on))
+        return tsp.planar_nax_grouped_moe(gpu, weights, gpu.upload(np.ascontiguousarray(chosen).reshape(-1)), x, tokens, per_token, scratch, **always_on)
+
+    y, riding = routed(w, ids, n, selected, shared=shared)
+    alone = tsp.PlanarMoeWeights(gpu, 12, 14, channels, hidden, 2, np.concatenate([sg, sg]), np.concatenate([su, su]), np.concatenate([sd, sd]))
+    separate = routed(alone, np.zeros(n, dtype=np.uint32), n, 1)
+    part = routed(w, ids[:n // 2], n // 2, selected)
+    assert gpu.error() == 0 and bool(gpu.torch.isfinite(y).all())
+    assert gpu.torch.equal(riding, separate)
+    assert gpu.torch.equal(part, y[:n // 2 * selected])

@@ -42,6 +42,10 @@ __device__ __forceinline__ void load_to_lds_4(const void* uniform_base, uint32_t
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds_base), "v"(lane_offset), "s"(uniform_base) : "memory", "m0");
 }
 
+// BY_BLOCKS: super-blocks are summed by themselves and then added up, in order, as the resident kernel's waves do, and with its roundings: a row's
+// bits may not tell which of the two has had it, since that goes by the rows of the whole call. Else the two products of a super-block go
+// straight to the sum, an instruction less for each.
+template <bool BY_BLOCKS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gate_up_stream_kernel(ResidentGateUpArgs a) {
     __shared__ __attribute__((aligned(16))) uint8_t lds[kLdsBytes];
     const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -229,7 +233,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                         const f32x16 zero{};
                         const f32x16 m = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums, mn[j], zero, 0, 0, 0);
 #pragma unroll
-                        for (int v = 0; v < 16; ++v) acc[i][j][v] = __builtin_fmaf(-dmin[j], m[v], __builtin_fmaf(d[j], blk[i][j][v], acc[i][j][v]));
+                        for (int v = 0; v < 16; ++v) {
+                            if constexpr (BY_BLOCKS) acc[i][j][v] += __builtin_fmaf(-dmin[j], m[v], d[j] * blk[i][j][v]);
+                            else acc[i][j][v] = __builtin_fmaf(-dmin[j], m[v], __builtin_fmaf(d[j], blk[i][j][v], acc[i][j][v]));
+                        }
                     }
                 }
                 sm[0] = sm_next[0]; sm[1] = sm_next[1]; dm[0] = dm_next[0]; dm[1] = dm_next[1];
@@ -290,7 +297,8 @@ namespace tsp {
 
 int launch_stream_gate_up(const ResidentGateUpArgs& a, hipStream_t s) {
     const uint32_t groups = (a.task_slots * ((a.hidden + kUnits - 1) / kUnits) + 7) / 8 * 8;
-    TSP_LAUNCH("gemm_gate_up_swiglu", s, gate_up_stream_kernel<<<groups, 256, 0, s>>>(a));
+    if (resident_gate_up_takes(a.channels, a.hidden)) TSP_LAUNCH("gemm_gate_up_swiglu", s, gate_up_stream_kernel<true><<<groups, 256, 0, s>>>(a));
+    else TSP_LAUNCH("gemm_gate_up_swiglu", s, gate_up_stream_kernel<false><<<groups, 256, 0, s>>>(a));
     return launch_status("gate_up_stream");
 }
 

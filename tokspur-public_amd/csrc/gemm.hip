@@ -922,7 +922,7 @@ int grouped_moe(const tsp_grouped_moe* m, const tsp_shared_expert* shared, void*
         // Few rows per expert: the launch is bound by HBM, and the resident kernel's shares of 32 units leave no compute unit waiting for
         // another (a sublayer of 2048 x 512, 512 experts: 20 tokens 102 us against 114, 100 tokens 216 against 220; 400 tokens 302 against 295, 2048
         // tokens 478 against 449; 2048 x 768, 128 experts: 50 tokens 143 against 145, 100 tokens 152 against 151, 2048 tokens 408 against 383).
-        // The two add a row's super-blocks up in the same order but not with the same roundings.
+        // The two add a row's super-blocks up in the same order and with the same roundings.
         const bool few = routes < 6 * m->experts;
         rc = few && resident_gate_up_takes(m->channels, m->hidden) ? launch_resident_gate_up(r, s) : launch_stream_gate_up(r, s);
     }
