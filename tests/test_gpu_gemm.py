@@ -943,3 +943,34 @@ def test_grouped_moe_rows_whatever_company(gpu, tsp, synth, n, hidden):
     assert gpu.error() == 0 and bool(gpu.torch.isfinite(y).all())
     assert gpu.torch.equal(riding, separate)
     assert gpu.torch.equal(part, y[:n // 2 * selected])
+
+
+def test_grouped_moe_sigmoid_bits(gpu, tsp, synth):
+    """Gate sums from -34 to -21, exact in any order, behind a down matrix that passes h through: SwiGLU is good to an f32's last places also
+    where the exponential is all that is left of it. An error of 2^-22 moves a carried half, whose steps are 2^-11 of its value and more, for one
+    value in 2^11 at most; an exponential whose argument has 24 bits alone is off by 2^-20 there and moves more than twice as many."""
+    channels, hidden, experts, n = 768, 128, 2, 900
+    # a row's weight is its code times d (and 63) in one column, nothing in the others
+    gate = np.zeros((experts, hidden, channels // 256, 144), dtype=np.uint8)
+    up = gate.copy()
+    gate_codes, up_codes = 12 + np.arange(hidden) % 4, 1 + np.arange(hidden) // 4 % 15
+    gate[:, :, 0, 0:2], up[:, :, 0, 0:2] = (np.array([v], dtype=np.float16).view(np.uint8) for v in (-0.125, 32768.0))
+    gate[:, :, 0, 4], up[:, :, 0, 4] = 1, 63
+    gate[:, :, 0, 16], up[:, :, 0, 17] = gate_codes, up_codes
+    down = np.zeros((experts, channels, hidden // 32, 34), dtype=np.uint8)
+    down[..., 0:2] = np.array([1.0], dtype=np.float16).view(np.uint8)
+    for c in range(hidden):
+        down[:, c, c // 32, 2 + c % 32] = 1
+    w = tsp.PlanarMoeWeights(gpu, 12, 8, channels, hidden, experts, gate.reshape(-1), up.reshape(-1), down.reshape(-1))
+    x = np.zeros((n, channels), dtype=np.float32)
+    x[:, 0], x[:, 1] = 14.5 + np.arange(n) % 55 / 16, 256 * (128 + np.arange(n) % 128)
+    x = synth.round_bf16(x)
+    scratch = tsp.GroupedScratch(gpu, n, 1, experts, channels, hidden)
+    y = tsp.planar_nax_grouped_moe(gpu, w, gpu.upload(np.zeros(n, dtype=np.uint32)), gpu.upload(x), n, 1, scratch).cpu().numpy()[:, :hidden]
+    assert gpu.error() == 0
+    g, u = x[:, :1].astype(np.float64) * (-0.125 * gate_codes), x[:, 1:2].astype(np.float64) * (63 * 32768.0 * up_codes)
+    h = g / (1 + np.exp(-g)) * u
+    held = np.abs(h / 256) > 2.0 ** -14  # whole halves
+    moved = int((y != (h / 256).astype(np.float16).astype(np.float64) * 256)[held].sum())
+    print(f"{moved} of {int(held.sum())} carried halves moved")
+    assert held.sum() > 100000 and moved <= held.sum() / 2048

@@ -270,13 +270,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         wait_all_loads();  // the last requests fetched what nobody reads: they must have landed before the LDS is given away
 
         // accumulator v of tile (i, j): row i*32 + 8*(v/4) + 4*khalf + v%4, hidden unit col. h travels to the down product as the half
-        // nearest to h * 2^-8; a sum that is not finite, or a product too large for a half, leaves an infinity or a NaN there.
+        // nearest to h * 2^-8; a sum that is not finite, or a product too large for a half, leaves an infinity or a NaN there. The sigmoid is
+        // the resident kernel's short one only where rows share that kernel's bits; at other widths it is good to its last places (2560 x 640,
+        // 2048 tokens: 740 us a sublayer with the short one, 749).
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const uint32_t r = i * 32 + 8 * (v / 4) + 4 * khalf + (v % 4);
-                const float g = acc[i][0][v], h = (g * sigmoid_fast(g)) * acc[i][1][v];
+                const float g = acc[i][0][v], h = (g * (BY_BLOCKS ? sigmoid_fast(g) : sigmoid_stable(g))) * acc[i][1][v];
                 const _Float16 carried = _Float16(h * 0.00390625f);
                 if (r < t.nrows && unit0 < a.hidden) {
                     const uint32_t magnitude = __builtin_bit_cast(uint16_t, carried) & 0x7fffu;
