@@ -451,3 +451,34 @@ def test_dense_mm_q8_odd_rows(gpu, tsp, orc, synth, lanes, tokens, cols, rows):
         x64 = x.astype(np.float64)
         bound = 2.0 ** -18 * (np.abs(x64) @ np.abs(dense).T) + 2.0 ** -22 * np.abs(x64).max() * np.abs(dense).sum(axis=1)
         assert (np.abs(got[:, check] - x64 @ dense.T) <= bound).all()
+
+
+@pytest.mark.parametrize("lanes,tokens,cols,rows", [(False, 9, 1024, 14003), (False, 16, 2048, 24576), (False, 10, 2560, 40001), (True, 13, 1024, 37), (True, 16, 2048, 512),
+                                                    (True, 7, 2560, 1001), (True, 12, 2560, 64)])
+def test_dense_mm_q8_sums_that_overflow_at_the_join(gpu, tsp, lanes, tokens, cols, rows):
+    """Two workgroups to a matrix row, either half of whose sum is finite: a sum that passes the largest float is reported, wherever in the matrix
+    it is, and halves of which one is nearly as large and the other takes it back are not."""
+    blocks = np.zeros((rows, cols // 32, 34), dtype=np.uint8)
+    blocks[:, :, 0:2] = np.array([4096.0], dtype=np.float16).view(np.uint8)
+    blocks[:, 0, 2] = 1      # the first column and the last one
+    blocks[:, -1, 33] = 1
+    x = np.zeros((tokens, cols), dtype=np.float32)
+    x[:, 0], x[:, -1] = 1.0 / 4096, 2.0 / 4096
+    layout = tsp.LAYOUT_Q8_LANES_V1 if lanes else tsp.LAYOUT_GGUF
+
+    def run(raw, token_rows):
+        flat = np.ascontiguousarray(raw).reshape(-1)
+        out = tsp.dense_mm_q8(gpu, layout, gpu.upload(tsp.q8_lanes_pack_rows(cols, flat) if lanes else flat), gpu.upload(token_rows), tokens, cols, rows)
+        return gpu.error(), out.cpu().numpy()
+
+    status, got = run(blocks, x)
+    assert status == 0 and (got == 3.0).all()
+    x[tokens - 1, 0], x[tokens - 1, -1] = 3.0 * 2.0 ** 114, -1.5 * 2.0 ** 114
+    status, got = run(blocks, x)
+    assert status == 0 and (got[tokens - 1] == np.float32(1.5 * 2.0 ** 126)).all()
+    for row in (0, rows // 2, rows - 1):  # this row alone has the sum's second half with the sign turned round
+        turned = blocks.copy()
+        turned[row, -1, 33] = 255
+        status, got = run(turned, x)
+        assert np.isinf(got[tokens - 1, row]) and np.isfinite(np.delete(got, row, axis=1)).all()
+        assert status == tsp.ERRBIT_NONFINITE

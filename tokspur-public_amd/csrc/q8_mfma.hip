@@ -215,6 +215,21 @@ __device__ __forceinline__ void f32_row_sums(const float (&acc)[4], uint32_t kq,
     if (kq == 2) store(4u, (acc[0] + (acc[1] + acc[2])) * back[4]);
 }
 
+// Two workgroups whose halves of a sum meet in an output that starts at zero: the halves may be finite and the sum not, which only the one
+// that adds last can see. What an addition found there is kept until the next tile's additions, by when it has long come back.
+struct Joined { float mine = 0, found = 0; };
+__device__ __forceinline__ Joined join(float* y, uint32_t at, float half) {  // sixteen rows of 1 000 000 at most: 32-bit offsets
+    return {half, unsafeAtomicAdd(reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(y) + at * 4), half)};
+}
+template <int N>
+__device__ __forceinline__ void check_joined(Joined (&all)[N], uint32_t& bad) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        if (nonfinite(all[i].found + all[i].mine)) bad = TSP_ERRBIT_NONFINITE;
+        all[i] = Joined{};
+    }
+}
+
 // DEPTH = (tile, group) items whose bytes are on their way while one is multiplied (1, 2 or 4; it divides the number of groups
 // of a workgroup). ROWS = token rows staged (8: all of K per workgroup; 16: half of K per workgroup, sums added into y; 5
 // and 10: the same in f32).
@@ -316,6 +331,7 @@ __global__ __launch_bounds__(kThreads, 1) void q8_mfma_kernel(Q8MfmaArgs a) {
         }
     };
 
+    Joined joined[KSPLIT == 2 ? SETS * 8 : 1];
     for (; t < share_end; t = t_next, t_next = take_tile()) {
         const uint32_t row0 = t * 32;
         float acc[SETS][2][4] = {};  // [set][16-row half of the tile][token row 4 kq + v]
@@ -397,14 +413,16 @@ __global__ __launch_bounds__(kThreads, 1) void q8_mfma_kernel(Q8MfmaArgs a) {
                         for (int v = 0; v < 4; ++v) acc[set][nt][v] += group_sum[set][nt][v];
             }
         };
-        for (uint32_t g = 0; g < groups; g += DEPTH) {  // the host picks a DEPTH that divides the number of groups
+        uint32_t g = 0;
+        do {  // the host picks a DEPTH that divides the number of groups; there is at least one, and the compiler has to know it to count what is in flight
             item(g, std::integral_constant<int, 0>{});
             if constexpr (DEPTH >= 2) item(g + 1, std::integral_constant<int, 1 % DEPTH>{});
             if constexpr (DEPTH >= 4) {
                 item(g + 2, std::integral_constant<int, 2 % DEPTH>{});
                 item(g + 3, std::integral_constant<int, 3 % DEPTH>{});
             }
-        }
+        } while ((g += DEPTH) < groups);
+        if constexpr (KSPLIT == 2) check_joined(joined, bad);
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt) {
             const uint32_t r = row0 + nt * 16 + n16;
@@ -416,7 +434,7 @@ __global__ __launch_bounds__(kThreads, 1) void q8_mfma_kernel(Q8MfmaArgs a) {
                         if (m >= a.m || r >= a.rows) return;
                         if (nonfinite(val)) bad = TSP_ERRBIT_NONFINITE;
                         if constexpr (KSPLIT == 1) a.y[uint64_t(m) * a.rows + r] = val;
-                        else unsafeAtomicAdd(a.y + uint64_t(m) * a.rows + r, val);
+                        else joined[(set * 2 + nt) * 4 + row % 4] = join(a.y, m * a.rows + r, val);  // (row 4 is in other lanes than row 0)
                     });
                 }
                 continue;
@@ -428,11 +446,12 @@ __global__ __launch_bounds__(kThreads, 1) void q8_mfma_kernel(Q8MfmaArgs a) {
                     const float val = acc[0][nt][v] * inv_scale;
                     if (nonfinite(val)) bad = TSP_ERRBIT_NONFINITE;
                     if constexpr (KSPLIT == 1) a.y[uint64_t(m) * a.rows + r] = val;
-                    else unsafeAtomicAdd(a.y + uint64_t(m) * a.rows + r, val);
+                    else joined[nt * 4 + v] = join(a.y, m * a.rows + r, val);
                 }
             }
         }
     }
+    if constexpr (KSPLIT == 2) check_joined(joined, bad);
     publish_error(bad, a.error_word);
 }
 
@@ -549,6 +568,7 @@ __global__ __launch_bounds__(kThreads, 1) void q8_lanes_mfma_kernel(Q8MfmaArgs a
         }
     };
 
+    Joined joined[KSPLIT == 2 ? SETS * 4 : 1];
     for (; t < share_end; t = t_next, t_next = take_tile()) {
         const uint32_t row0 = t * kLaneRows;
         float acc[SETS][4] = {};  // [set][token row 4 kq + v]
@@ -632,11 +652,13 @@ __global__ __launch_bounds__(kThreads, 1) void q8_lanes_mfma_kernel(Q8MfmaArgs a
                     for (int v = 0; v < 4; ++v) acc[set][v] += run_sum[set][v];
             }
         };
-        for (uint32_t g = 0; g < runs; g += DEPTH) {  // the host picks a DEPTH that divides the number of runs
+        uint32_t g = 0;
+        do {  // the host picks a DEPTH that divides the number of runs; there is at least one
             item(g, std::integral_constant<int, 0>{});
             if constexpr (DEPTH >= 2) item(g + 1, std::integral_constant<int, 1 % DEPTH>{});
-        }
+        } while ((g += DEPTH) < runs);
         const uint32_t r = row0 + n16;
+        if constexpr (KSPLIT == 2) check_joined(joined, bad);
         if constexpr (F32) {
 #pragma unroll
             for (int set = 0; set < SETS; ++set) {
@@ -645,7 +667,7 @@ __global__ __launch_bounds__(kThreads, 1) void q8_lanes_mfma_kernel(Q8MfmaArgs a
                     if (m >= a.m || r >= a.rows) return;
                     if (nonfinite(val)) bad = TSP_ERRBIT_NONFINITE;
                     if constexpr (KSPLIT == 1) a.y[uint64_t(m) * a.rows + r] = val;
-                    else unsafeAtomicAdd(a.y + uint64_t(m) * a.rows + r, val);
+                    else joined[set * 4 + row % 4] = join(a.y, m * a.rows + r, val);
                 });
             }
             continue;
@@ -657,10 +679,11 @@ __global__ __launch_bounds__(kThreads, 1) void q8_lanes_mfma_kernel(Q8MfmaArgs a
                 const float val = acc[0][v] * inv_scale;
                 if (nonfinite(val)) bad = TSP_ERRBIT_NONFINITE;
                 if constexpr (KSPLIT == 1) a.y[uint64_t(m) * a.rows + r] = val;
-                else unsafeAtomicAdd(a.y + uint64_t(m) * a.rows + r, val);
+                else joined[v] = join(a.y, m * a.rows + r, val);
             }
         }
     }
+    if constexpr (KSPLIT == 2) check_joined(joined, bad);
     publish_error(bad, a.error_word);
 }
 
