@@ -457,8 +457,8 @@ def test_router_f32_batch_sliced(gpu, synth, tokens, columns, experts):
 
 @pytest.mark.parametrize("tokens,columns,experts", [(520, 2080, 512), (1025, 64, 512), (300, 32, 931), (577, 288, 500), (2048, 2560, 512)])
 def test_router_f32_batch_pieces(gpu, synth, tokens, columns, experts):
-    """The 64 x 64 form on bf16 pieces: waves with no columns at all, ragged edges, and the rows that pieces cannot carry. What six of nine
-    products of pieces leave out is 2 x 2^-23 of a product at most, under the bound of f32 sums that the other forms keep; an infinite
+    """The 64 x 64 form on bf16 pieces: waves with no columns at all, ragged edges, and the rows that pieces cannot carry. What eight of nine
+    products of pieces leave out is 2^-30 of a product at most, under the bound of f32 sums that the other forms keep; an infinite
     activation gives the infinities of plain f32 arithmetic, rows of subnormals and near them the bound that f32 sums have, zeros zeros."""
     w = synth.activations_f32(synth.tensor_seed(5, 300 + tokens), (experts, columns))
     x = synth.activations_f32(synth.tensor_seed(6, 300 + tokens), (tokens, columns))
@@ -512,3 +512,18 @@ def test_router_f32_batch_more_tokens_than_experts(gpu, synth, tokens, columns, 
     scale = np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T
     assert (np.abs(got[:tokens, :experts] - want) <= 2e-6 * scale).all() and gpu.error() == 0
     assert (got[tokens] == 7.25).all() and (got[:, experts:] == 7.25).all()
+
+
+def test_router_f32_batch_one_product(gpu):
+    """The 64 x 64 form where one product is the whole logit: two floats of 24 bits each, multiplied as f32 arithmetic does, to half a unit of
+    the result's last place (2^-24 of it), with 2^-29 for what pieces may leave out."""
+    tokens, columns, experts = 640, 128, 512
+    rng = np.random.default_rng(3)
+    w = ((1 + rng.random((experts, columns))) * rng.choice([-1, 1], (experts, columns))).astype(np.float32)
+    x = np.zeros((tokens, columns), dtype=np.float32)
+    at = rng.integers(0, columns, tokens)
+    x[np.arange(tokens), at] = (1 + rng.random(tokens)).astype(np.float32) * 2.0 ** rng.integers(-20, 20, tokens)
+    got = gpu.router_f32_batch(gpu.upload(w), gpu.upload(x), tokens, columns, experts).cpu().numpy()
+    want = x[np.arange(tokens), at].astype(np.float64)[:, None] * w[:, at].astype(np.float64).T
+    error = np.abs(got - want) / np.abs(want)
+    assert gpu.error() == 0 and error.max() <= 2.0 ** -24 + 2.0 ** -29, float(error.max() * 2 ** 24)

@@ -2,15 +2,17 @@
 //
 // Replaces the engine's `graph_moe_router_f32_batch` (kernels/moe_router_f32_batch.metal:13-50: 32x32x32 f32 tiles,
 // full-precision multiply-accumulate, operands never narrowed) and its windowed sibling for up to 2048 tokens.
-// Both operands stay whole floats from memory to the accumulator. Few tokens run on the f32 matrix instructions or the vector ALUs.
+// Few tokens run on the f32 matrix instructions or the vector ALUs, with operands that stay whole floats from memory to the accumulator.
 //
 // Many tokens: a workgroup of eight waves owns 64 tokens x 64 experts, each wave an eighth of the columns; the partial tiles are added in
 // LDS in wave order (deterministic). A float is its three bf16 pieces (mfma_quant.hpp) and a product of two floats the sum of
-// six products of pieces, all exact, in f32 accumulators: v_mfma_f32_32x32x16_bf16 does in 6 x 32 cycles what v_mfma_f32_32x32x2_f32
-// does in 512, and the accumulator is rounded 6 times per sixteen columns instead of 8 (error against 64-bit sums, 2-norm, 2048 x 2560 by 512
-// experts: 2.9e-7, 6.5e-7 with f32 products in two column halves). What is left out is 2^-22 of a product and less. Bound by the matrix pipe
-// (31 k of 56 k cycles) and the splitting (5.5 vector instructions a float, in every tile anew) beside it. 512 experts, 2048
-// tokens: 2560 columns 59 -> 34 us, 2048 columns 46 -> 28.
+// eight products of pieces, all exact, in f32 accumulators: v_mfma_f32_32x32x16_bf16 does in 8 x 32 cycles what v_mfma_f32_32x32x2_f32
+// does in 512. What is left out, last piece by last piece, is 2^-30 of a product and less. The matrix instruction cuts its sum off where an f32 addition
+// rounds, so the products of two first pieces, sixteen bits each, have an accumulator of their own and meet the others in one rounding: a
+// logit that is one product is that product rounded once, as in f32 arithmetic (one accumulator and six products: off by 2^-21). Error against 64-bit
+// sums, 2-norm, 2048 x 2560 by 512 experts: 1.1e-7 (one accumulator 2.8e-7, f32 products in two column halves 6.5e-7). Bound by the matrix pipe and
+// the splitting (5.5 vector instructions a float, in every tile anew) beside it. 512 experts, 2048 tokens: 2560 columns 59 us with f32 products, 40 now
+// (34 with six products in one accumulator), 2048 columns 46 and 33 (28).
 #include "mfma_quant.hpp"
 
 #include <type_traits>
@@ -73,7 +75,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     uint8_t* const mine = reinterpret_cast<uint8_t*>(lds) + wave * 16384;
     const uint32_t mine_lds = __builtin_amdgcn_readfirstlane(lds_address(mine));
     const uint32_t n = lane % 32, khalf = lane / 32;
-    f32x16 acc[2][2] = {};  // [expert half][token half]
+    f32x16 acc[2][2] = {}, small[2][2] = {};  // [expert half][token half]: the products of two first pieces, and the others
     // 32-column units of this wave's slice, two groups of sixteen columns each
     const uint32_t units = a.columns / 32, first = uint32_t(uint64_t(units) * wave / 8), last = uint32_t(uint64_t(units) * (wave + 1) / 8);
     auto request = [&](uint32_t unit) {
@@ -106,13 +108,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         const Rows rows = read_rows(P ^ 1);
         __builtin_amdgcn_sched_barrier(0);
         auto add = [&](int i, int j) {
+            auto& sum = i + j ? small : acc;
 #pragma unroll
             for (int e = 0; e < 2; ++e)
 #pragma unroll
-                for (int t = 0; t < 2; ++t) acc[e][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(now.x[t][i], now.w[e][j], acc[e][t], 0, 0, 0);
+                for (int t = 0; t < 2; ++t) sum[e][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(now.x[t][i], now.w[e][j], sum[e][t], 0, 0, 0);
         };
-        // the small products first; those of 2^-22 of the whole and less (middle with last, last with last) are left out
-        add(2, 0);
+        // the small products first; that of the two last pieces, below 2^-30 of the whole, is left out
+        add(2, 1); add(1, 2);
         __builtin_amdgcn_sched_barrier(0);
         if (P == 0) {  // the whole unit is in registers: the next one goes there
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -120,10 +123,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             __builtin_amdgcn_sched_barrier(0);
         }
         split(rows, next);
-        add(1, 1); add(0, 2); add(1, 0); add(0, 1); add(0, 0);
+        add(2, 0); add(1, 1); add(0, 2); add(1, 0); add(0, 1); add(0, 0);
 #pragma unroll
-        for (int g = 0; g < 20; ++g) {
-            __builtin_amdgcn_sched_group_barrier(0x2, 9, 0);  // nine vector instructions
+        for (int g = 0; g < 24; ++g) {
+            __builtin_amdgcn_sched_group_barrier(0x2, 8, 0);  // eight vector instructions
             __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);  // and a matrix instruction in turn
         }
     };
@@ -145,7 +148,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int i = 0; i < 16; ++i) {
         f32x4 quad;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) quad[r] = acc[i / 8][i / 4 % 2][i % 4 * 4 + r];
+        for (int r = 0; r < 4; ++r) quad[r] = acc[i / 8][i / 4 % 2][i % 4 * 4 + r] + small[i / 8][i / 4 % 2][i % 4 * 4 + r];
         sums[(wave * 16 + i) * 64 + lane] = quad;
     }
     __syncthreads();
