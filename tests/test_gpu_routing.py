@@ -527,3 +527,25 @@ def test_router_f32_batch_one_product(gpu):
     want = x[np.arange(tokens), at].astype(np.float64)[:, None] * w[:, at].astype(np.float64).T
     error = np.abs(got - want) / np.abs(want)
     assert gpu.error() == 0 and error.max() <= 2.0 ** -24 + 2.0 ** -29, float(error.max() * 2 ** 24)
+
+
+@pytest.mark.parametrize("weight_exponent,row_exponent", [(60, -116), (-116, 60), (120, -125), (100, -149), (30, -112)])
+def test_router_f32_batch_pieces_far_apart(gpu, synth, weight_exponent, row_exponent):
+    """The 64 x 64 form with operands whose last pieces are below bf16 against ones large enough that the logit is not small: the f32 bound
+    holds for those rows, whichever operand it is, and the bits of every other logit do not change."""
+    tokens, columns, experts = 577, 288, 500
+    w = synth.activations_f32(synth.tensor_seed(5, 500), (experts, columns))
+    x = synth.activations_f32(synth.tensor_seed(6, 500), (tokens, columns))
+    usual = gpu.router_f32_batch(gpu.upload(w), gpu.upload(x), tokens, columns, experts, out_stride=experts * 4).cpu().numpy()
+    w[70] *= np.float32(2.0 ** (weight_exponent // 2))
+    w[70] *= np.float32(2.0 ** (weight_exponent - weight_exponent // 2))
+    x[130] *= np.float32(2.0 ** (row_exponent // 2))
+    x[130] *= np.float32(2.0 ** (row_exponent - row_exponent // 2))
+    got = gpu.router_f32_batch(gpu.upload(w), gpu.upload(x), tokens, columns, experts, out_stride=experts * 4).cpu().numpy()
+    want = float(x[130].astype(np.float64) @ w[70].astype(np.float64))
+    scale = float(np.abs(x[130]).astype(np.float64) @ np.abs(w[70]).astype(np.float64))
+    assert gpu.error() == 0
+    assert abs(float(got[130, 70]) - want) <= 2e-6 * scale, abs(float(got[130, 70]) - want) / scale
+    others = np.ones(got.shape, dtype=bool)
+    others[130], others[:, 70] = False, False
+    assert np.array_equal(got[others], usual[others])

@@ -11,7 +11,7 @@
 // rounds, so the products of two first pieces, sixteen bits each, have an accumulator of their own and meet the others in one rounding: a
 // logit that is one product is that product rounded once, as in f32 arithmetic (one accumulator and six products: off by 2^-21). Error against 64-bit
 // sums, 2-norm, 2048 x 2560 by 512 experts: 1.1e-7 (one accumulator 2.8e-7, f32 products in two column halves 6.5e-7). Bound by the matrix pipe and
-// the splitting (5.5 vector instructions a float, in every tile anew) beside it. 512 experts, 2048 tokens: 2560 columns 59 us with f32 products, 40 now
+// the splitting (6.5 vector instructions a float, in every tile anew) beside it. 512 experts, 2048 tokens: 2560 columns 59 us with f32 products, 40 now
 // (34 with six products in one accumulator), 2048 columns 46 and 33 (28).
 #include "mfma_quant.hpp"
 
@@ -24,12 +24,16 @@ namespace {
 constexpr uint32_t kTile = 64;                          // tokens and experts per workgroup
 constexpr uint32_t kLdsBytes = 8 * kTile * kTile * 4;    // the eight waves' partial tiles
 
+// Operands are split 2^24 times their size: a float below 2^-109 would lose bits of its last piece, the smallest one all of it, and against a large
+// operand on the other side that shows. Nothing is lost so; products come out 2^48 times theirs.
+constexpr float kLift = 0x1p24f, kLower = 0x1p-48f;
+
 // Eight floats as three fragments of bf16 pieces (mfma_quant.hpp)
 __device__ __forceinline__ void pieces8(const f32x4 (&v)[2], bf16x8 (&out)[3]) {
     u32x4 hi, mid, lo;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const Pieces p = three_pieces(v[i / 2][2 * (i % 2)]), q = three_pieces(v[i / 2][2 * (i % 2) + 1]);
+        const Pieces p = three_pieces(v[i / 2][2 * (i % 2)] * kLift), q = three_pieces(v[i / 2][2 * (i % 2) + 1] * kLift);
         hi[i] = two_tops(p.hi, q.hi); mid[i] = two_tops(p.mid, q.mid); lo[i] = two_tops(p.lo, q.lo);
     }
     out[0] = __builtin_bit_cast(bf16x8, hi); out[1] = __builtin_bit_cast(bf16x8, mid); out[2] = __builtin_bit_cast(bf16x8, lo);
@@ -45,12 +49,16 @@ struct RouterArgs {
     uint32_t* error_word;
 };
 
-// What f32 arithmetic makes of one product of rows, for results that the pieces cannot give: sums that are not finite, and
-// operands so small that a piece of theirs falls below bf16 (a float under 2^-109 loses bits of its last piece).
+// What f32 arithmetic makes of one product of rows, for results that the pieces cannot give: those that are not finite (an operand of 2^104 or a sum
+// of 2^80 is too large once lifted), and those so small that products of pieces may have vanished beside them. By a whole wave.
 __device__ __noinline__ float plain_dot(const float* w, const float* x, uint32_t columns) {
-    float sum = 0.0f;
-    for (uint32_t k = 0; k < columns; ++k) sum = __builtin_fmaf(w[k], x[k], sum);
-    return sum;
+    f32x4 sum{};
+    for (uint32_t k = threadIdx.x % kWave * 4; k < columns; k += kWave * 4) {
+        const f32x4 a = *reinterpret_cast<const f32x4*>(w + k), b = *reinterpret_cast<const f32x4*>(x + k);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) sum[c] = __builtin_fmaf(a[c], b[c], sum[c]);
+    }
+    return wave_sum((sum[0] + sum[1]) + (sum[2] + sum[3]));
 }
 
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void router_f32_gemm(RouterArgs a) {
@@ -115,7 +123,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 for (int t = 0; t < 2; ++t) sum[e][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(now.x[t][i], now.w[e][j], sum[e][t], 0, 0, 0);
         };
         // the small products first; that of the two last pieces, below 2^-30 of the whole, is left out
-        add(2, 1); add(1, 2);
+        add(2, 1);
         __builtin_amdgcn_sched_barrier(0);
         if (P == 0) {  // the whole unit is in registers: the next one goes there
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -123,9 +131,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             __builtin_amdgcn_sched_barrier(0);
         }
         split(rows, next);
-        add(2, 0); add(1, 1); add(0, 2); add(1, 0); add(0, 1); add(0, 0);
+        add(1, 2); add(2, 0); add(1, 1); add(0, 2); add(1, 0); add(0, 1); add(0, 0);
 #pragma unroll
-        for (int g = 0; g < 24; ++g) {
+        for (int g = 0; g < 28; ++g) {
             __builtin_amdgcn_sched_group_barrier(0x2, 8, 0);  // eight vector instructions
             __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);  // and a matrix instruction in turn
         }
@@ -163,10 +171,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const uint32_t token = token0 + t * 32 + b * 8 + (l / 32) * 4 + r;  // D[i][j]: j = lane % 32
-            if (token < a.tokens && expert < a.experts) {
-                float v = value[r];
-                if (nonfinite(v) || (v != 0.0f && fabsf(v) < 0x1p-64f))
-                    v = plain_dot(a.weights + uint64_t(expert) * a.columns, a.input + uint64_t(token) * a.input_stride, a.columns);
+            const bool live = token < a.tokens && expert < a.experts;
+            float v = value[r] * kLower;
+            for (uint64_t again = __builtin_amdgcn_ballot_w64(live && (nonfinite(v) || (v != 0.0f && fabsf(v) < 0x1p-64f))); again; again &= again - 1) {
+                const uint32_t which = __builtin_ctzll(again);
+                const uint32_t row = __builtin_amdgcn_readlane(expert, which), column = __builtin_amdgcn_readlane(token, which);
+                const float plain = plain_dot(a.weights + uint64_t(row) * a.columns, a.input + uint64_t(column) * a.input_stride, a.columns);
+                if (lane == which) v = plain;
+            }
+            if (live) {
                 bad |= nonfinite(v) ? TSP_ERRBIT_NONFINITE : 0u;
                 a.output[uint64_t(token) * a.output_stride + expert] = v;
             }
