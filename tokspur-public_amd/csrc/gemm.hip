@@ -37,7 +37,7 @@ using namespace tsp;
 namespace {
 
 enum Epilogue : int { EPI_F32 = 0, EPI_BF16 = 1 };
-enum Rows : int { ROWS_DENSE = 0, ROWS_TASK_SLOTS = 1, ROWS_ROUTES = 2, ROWS_TOKENS = 3 };  // the last two: routes with an input row each, or one per token
+enum Rows : int { ROWS_DENSE = 0, ROWS_TASK_SLOTS = 1, ROWS_ROUTES = 2 };
 
 constexpr int kTaskRows = 64;
 constexpr int kRowTiles = kTaskRows / 32;
@@ -60,6 +60,7 @@ struct GemmArgs {
     float out_scale;
     uint32_t* error_word;
     uint64_t raw_expert_bytes;       // raw GGUF expert stacks: bytes between experts (0 for one dense matrix)
+    uint32_t broadcast;              // ROWS_ROUTES: one input row per token instead of one per route
     uint32_t col_tiles, task_slots;  // logical grid: column tiles x tasks, launched as one linear grid
     // an always-on expert riding in the same launch: tasks whose expert id is `experts` take every token as their rows,
     // this down matrix and these output rows
@@ -152,7 +153,7 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {  // two work
             // activation row: the route's token (broadcast grouped GEMM), the route itself (grouped GEMM with one input
             // row per route) or the task's slot in the intermediate buffer (down); output row: the route
             const uint32_t safe = rid == 0xffffffffu ? 0 : rid;
-            row_src[tid] = ROWS == ROWS_TOKENS ? safe / a.selected : ROWS == ROWS_ROUTES ? safe : task * kTaskRows + (tid < nrows ? tid : 0);
+            row_src[tid] = ROWS == ROWS_ROUTES ? (a.broadcast ? safe / a.selected : safe) : task * kTaskRows + (tid < nrows ? tid : 0);
             my_dst = shared ? rid / a.selected : rid;
         }
     }
@@ -569,7 +570,7 @@ __global__ __launch_bounds__(512) void tasks_and_rows(TaskLists t, const void* _
 
 template <int BKIND, int EPI, int ROWS>
 int launch(const GemmArgs& a, uint32_t col_tiles, uint32_t tasks, hipStream_t s) {
-    constexpr const char* name = ROWS == ROWS_TASK_SLOTS ? "gemm_down" : ROWS == ROWS_ROUTES || ROWS == ROWS_TOKENS ? "gemm_grouped" : "gemm_dense";
+    constexpr const char* name = ROWS == ROWS_TASK_SLOTS ? "gemm_down" : ROWS == ROWS_ROUTES ? "gemm_grouped" : "gemm_dense";
     GemmArgs g = a;
     g.col_tiles = col_tiles;
     g.task_slots = tasks;
@@ -750,10 +751,9 @@ extern "C" int tsp_grouped_mm(uint32_t encoding, uint32_t layout, const void* ma
     GemmArgs a{};
     a.a = xh; a.a_stride = columns; a.sx = sx; a.w0 = static_cast<const uint8_t*>(matrices); a.raw_expert_bytes = expert_bytes;
     a.experts = experts; a.tasks = task_list; a.counts = counts; a.token_map = token_map; a.ids = ids; a.tokens = tokens; a.selected = selected;
-    a.n = rows; a.k = columns; a.out = output; a.out_stride = output_stride_bytes; a.out_scale = 1.0f;
+    a.broadcast = broadcast ? 1 : 0; a.n = rows; a.k = columns; a.out = output; a.out_stride = output_stride_bytes; a.out_scale = 1.0f;
     a.error_word = error_word;
-    return broadcast ? launch<B_Q4K_RAW, EPI_F32, ROWS_TOKENS>(a, (rows + 255) / 256, l.bound, s)
-                     : launch<B_Q4K_RAW, EPI_F32, ROWS_ROUTES>(a, (rows + 255) / 256, l.bound, s);
+    return launch<B_Q4K_RAW, EPI_F32, ROWS_ROUTES>(a, (rows + 255) / 256, l.bound, s);
 }
 
 // ---------------------------------------------------------------- grouped MoE
