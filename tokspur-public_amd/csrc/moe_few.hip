@@ -7,24 +7,29 @@
 // and 5.0e-8 to 5.7e-8 of y's (Q8_0, Q5_1). (Rows as two halves or three bf16 pieces on the matrix cores: 1.8e-7 to 3.2e-7, 6.7e-8
 // to 7.3e-8.)
 //
-// Matrix cores are not needed for it: two and a half instructions per weight and row are half of the time its bytes take, while
-// their operand order gathers 16 bytes from 64 places per request, or takes a plan over the step's records first, and both cost more.
+// Matrix cores are not needed for it: two and a half instructions per weight and row are in the end a quarter of the time where experts meet one
+// row each, while their operand order gathers 16 bytes from 64 places per request, or takes a plan over the step's records first, and both cost more.
 // L lanes share a weight row and read neighbouring pieces of it; a lane owns every L-th unit of 64 (32) weights of TWO rows, the
 // gate and up rows of a hidden unit or two rows of down, so that an activation read from LDS serves two weights.
 //
 //  one_row   one token. Bound by one trip to memory, the launch and the issue of its instructions, in about equal parts: a wave
 //            asks for everything it will ever need before it waits, R units of each row.
 //  few_rows  more tokens, and one token's rows that are too wide for that. Bound by memory with a head of one trip and a tail of one
-//            unit's arithmetic: the next unit's bytes travel while one is multiplied, three or four waves per SIMD.
+//            unit's arithmetic: the next unit's bytes travel while one is multiplied, three or four waves per SIMD. Both activation rows are
+//            asked for whole, ahead of the first weights: piece by piece as they are staged they were three more trips (eight tokens, gate/up
+//            2048 x 512, 24.4 -> 23.3 us).
 //
 // Kernel times, before -> now (ten of 512 experts; the kernels before were one super-block per wave, rows kept in registers, or a
 // stream over the records, each on the matrix cores):
 //   one token     gate/up 2048 x 512 9.5 -> 6.3 us, 2560 x 640 14.6 -> 9.0; down 512 -> 2048 Q6_K 6.6 -> 5.2, 640 -> 2560 Q8_0 9.2 -> 5.6
 //   three tokens  gate/up 2048 x 512 16.4 -> 13.0, down 512 -> 2048 Q8_0 13.4 -> 8.0
-//   five tokens   gate/up 2560 x 640 30.8 -> 24.3 (88 MB: 18 us at the rate of a copy), down Q8_0 26.0 -> 18.2
-//   eight tokens  gate/up 2048 x 512 26.8 -> 25.4, down Q6_K 19.6 -> 18.4; eight of 128, down 768 -> 2048 Q5_1 31.4 -> 18.2
-// A whole call, four sets of experts for eight tokens (2048 x 512, Q6_K): 32.9 -> 30 us. Only where all eight tokens take the same
-// ten experts does it lose, 20 -> 26 us, to the matrix cores' rows that come for nothing.
+//   five tokens   gate/up 2560 x 640 30.8 -> 23.1 (88 MB: 18 us at the rate of a copy), down Q8_0 26.0 -> 17.6
+//   eight tokens  gate/up 2048 x 512 26.8 -> 23.3, down Q6_K 19.6 -> 17.0; eight of 128, down 768 -> 2048 Q5_1 31.4 -> 18.2
+// Tokens that agree, a whole call of eight at 2048 x 512 with Q6_K, against the kernels with records on the matrix cores before (us): eight sets of
+// experts 45.6 -> 39.9, four 34.5 -> 29.5, two 27.5 -> 27.4, all on the same ten 21.0 -> 27.3; five on the same ten 20.7 -> 21.3, four 20.4, both, three
+// 18.6 -> 17.2. Wider and larger layers gain throughout (eight on the same eight of 4096 x 1536, Q8_0: 539 -> 90). What the last of the eight lose is
+// arithmetic, 2.75 waves a SIMD of it: rows that come for nothing on the matrix cores. v_mfma_f32_4x4x1 gives the bits of these multiply-adds, but
+// not beside vector instructions (10 cycles, and 20 with one conversion between).
 #include "moe_few.hpp"
 
 #include <type_traits>
@@ -394,7 +399,7 @@ __global__ __launch_bounds__(kThreads) void one_row(OneArgs a) {
 
 // ---------------------------------------------------------------- two to eight tokens
 // A task is an expert and one or two of its routes: every workgroup reads the step's ids, finds the routes of its own route's
-// expert with two ballots and leaves if its own is the second, fourth ... of them. Nothing is planned or written first; one workgroup of the
+// expert with two ballots and leaves if its own is in their second half. Nothing is planned or written first; one workgroup of the
 // gate/up launch writes the union block that the call promises. The always-on expert's tasks are its tokens by twos.
 // JOINT: a second row uses the first one's converted codes, at the price of registers (165 against 122 at Q4_K, a wave per SIMD
 // less); else the codes are converted again. Up to 2048 columns joint: 25.4 against 24.3 us for eight tokens on even experts,
@@ -407,7 +412,7 @@ struct FewArgs {
     uint32_t hidden, channels;
 };
 
-template <uint32_t T, bool PAIR, int L, bool JOINT>
+template <uint32_t T, bool PAIR, int L, int Q, bool JOINT>
 __global__ __launch_bounds__(kThreads) void few_rows(FewArgs f) {
     const OneArgs& a = f.one;
     constexpr uint32_t kUnit = unit_weights(T), kFloats = unit_floats(T), kGroups = kWave / L, kRows = kGroups * (PAIR ? 1 : 2);
@@ -438,20 +443,26 @@ __global__ __launch_bounds__(kThreads) void few_rows(FewArgs f) {
     } else {
         const uint32_t route = blockIdx.y - f.shared_tasks;
         expert = uint32_t(__builtin_amdgcn_readlane(int(route < kWave ? id_low : id_high), int(route % kWave)));
-        // the routes of this expert: the first, third ... of them take the next one along, the others have been taken
+        // the routes of this expert: each of the first half of them takes one of the second half along, so that workgroups with nothing to do come
+        // behind those that have something (with neighbours in pairs, eight tokens on the same ten experts: 16.9 us of gate/up, 16.2 so)
         const uint64_t low = __builtin_amdgcn_ballot_w64(lane < a.routes && id_low == expert);
         const uint64_t high = __builtin_amdgcn_ballot_w64(kWave + lane < a.routes && id_high == expert);
         if (expert >= a.experts) {  // one token: the other routes do
             if (tid == 0 && blockIdx.x == 0) atomicOr(a.error_word, TSP_ERRBIT_INDEX);
             return;
         }
-        const uint64_t bit = 1ull << (route % kWave);
-        const uint32_t before = route < kWave ? __builtin_popcountll(low & (bit - 1)) : __builtin_popcountll(low) + __builtin_popcountll(high & (bit - 1));
-        if (before % 2) return;
-        const uint64_t above_low = route < kWave ? low & ~(bit | (bit - 1)) : 0, above_high = route < kWave ? high : high & ~(bit | (bit - 1));
+        const uint32_t in_low = __builtin_popcountll(low), all = in_low + __builtin_popcountll(high), half = (all + 1) / 2;
+        const uint64_t below = (1ull << (route % kWave)) - 1;
+        const uint32_t before = route < kWave ? __builtin_popcountll(low & below) : in_low + __builtin_popcountll(high & below);
+        if (before >= half) return;
         uint32_t next = route;
-        if (above_low) { next = __builtin_ctzll(above_low); count = 2; }
-        else if (above_high) { next = kWave + __builtin_ctzll(above_high); count = 2; }
+        if (before + half < all) {
+            uint32_t n = before + half;
+            uint64_t left = n < in_low ? low : high;
+            for (n = n < in_low ? n : n - in_low; n; --n) left &= left - 1;
+            next = (before + half < in_low ? 0 : kWave) + __builtin_ctzll(left);
+            count = 2;
+        }
         row_out[0] = route; row_out[1] = next;
         row_in[0] = PAIR ? route / f.selected : route;
         row_in[1] = PAIR ? next / f.selected : next;
@@ -464,7 +475,12 @@ __global__ __launch_bounds__(kThreads) void few_rows(FewArgs f) {
         if (reinterpret_cast<uintptr_t>(from) % 16 == 0) return reinterpret_cast<const float4*>(from)[quad];
         return make_float4(from[4 * quad], from[4 * quad + 1], from[4 * quad + 2], from[4 * quad + 3]);
     };
-    float4 x0 = load(x[0], tid);
+    float4 held[2][Q];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+            if (uint32_t(j) < count) held[j][q] = load(x[j], tid + q * kThreads);
 
     const uint32_t first = (blockIdx.x * (kThreads / kWave) + wave) * kRows + group;
     const uint8_t* w[2];
@@ -491,13 +507,18 @@ __global__ __launch_bounds__(kThreads) void few_rows(FewArgs f) {
     ask(0, next);
     __builtin_amdgcn_sched_barrier(0);
     const uint32_t rounded = (quads + kThreads - 1) / kThreads * kThreads;
-    for (uint32_t j = 0; j < count; ++j) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        if (uint32_t(j) >= count) break;
         uint32_t largest = 0;
-        for (uint32_t quad = tid; quad < rounded; quad += kThreads) {
-            const float4 here = j == 0 && quad == tid ? x0 : load(x[j], quad);
+        auto take = [&](const float4& here, uint32_t quad) {
             largest = max(largest, largest_bits(here));
             stage<T>(staged + j * row_floats, quad, here, quad < quads);
-        }
+        };
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+            if (q * kThreads < quads) take(held[j][q], tid + q * kThreads);
+        for (uint32_t quad = tid + Q * kThreads; quad < rounded; quad += kThreads) take(load(x[j], quad), quad);
         const bool over = __builtin_amdgcn_ballot_w64(largest >= kHuge) != 0;
         if (lane == 0) huge[j][wave] = over;
     }
@@ -578,13 +599,13 @@ __global__ __launch_bounds__(kThreads) void few_rows(FewArgs f) {
     publish_error(bad, a.error_word);
 }
 
-template <uint32_t T, bool PAIR, int L, bool JOINT>
+template <uint32_t T, bool PAIR, int L, int Q, bool JOINT>
 int launch_few(const char* name, const FewArgs& f, hipStream_t s) {
     constexpr uint32_t per_group = kThreads / L * (PAIR ? 1 : 2);
     const dim3 grid((f.one.n + per_group - 1) / per_group, f.shared_tasks + f.one.routes + (PAIR && f.meta ? 1 : 0));
     uint32_t lds = 2 * (f.one.k / unit_weights(T)) * unit_floats(T) * 4;
     if (PAIR && lds < kUnionScratchWords * 4) lds = kUnionScratchWords * 4;
-    TSP_LAUNCH(name, s, few_rows<T, PAIR, L, JOINT><<<grid, kThreads, lds, s>>>(f));
+    TSP_LAUNCH(name, s, few_rows<T, PAIR, L, Q, JOINT><<<grid, kThreads, lds, s>>>(f));
     return launch_status(name);
 }
 
@@ -626,7 +647,7 @@ int launch_few_gate_up(const FewMoe& m, hipStream_t s) {
     if (m.tokens > 1 || m.channels > kOneGateUp) {
         FewArgs f = few_args(m, a);
         f.one.x_stride = f.shared_x_stride = m.x_stride; f.shared_out_stride = m.shared_h_stride; f.one.routes = m.tokens * m.selected;
-        return m.channels <= 2048 ? launch_few<12, true, 8, true>("few_gate_up", f, s) : launch_few<12, true, 8, false>("few_gate_up", f, s);
+        return m.channels <= 2048 ? launch_few<12, true, 8, 2, true>("few_gate_up", f, s) : launch_few<12, true, 8, 3, false>("few_gate_up", f, s);
     }
     // 2048 columns with 32, 16 and 8 lanes to a row: 6.3, 7.2, 7.7 us; 2560 columns 9.8, 9.2, 10.1 (24 of 64, 8 of 48 and no lanes
     // idle, against fewer and longer waves)
@@ -654,9 +675,9 @@ int launch_few_down(const FewMoe& m, hipStream_t s) {
         // round (640 -> 2560 Q8_0, five tokens: 18.2 and, with eight lanes, 18.8).
         const bool wide = m.hidden > kOneDown;
         switch (m.dn.source_type) {
-        case 7: return wide ? launch_few<7, false, 16, true>("few_down", f, s) : launch_few<7, false, 8, true>("few_down", f, s);
-        case 8: return wide ? launch_few<8, false, 16, false>("few_down", f, s) : launch_few<8, false, 4, false>("few_down", f, s);
-        default: return wide ? launch_few<14, false, 8, true>("few_down", f, s) : launch_few<14, false, 4, true>("few_down", f, s);
+        case 7: return wide ? launch_few<7, false, 16, 2, true>("few_down", f, s) : launch_few<7, false, 8, 1, true>("few_down", f, s);
+        case 8: return wide ? launch_few<8, false, 16, 2, false>("few_down", f, s) : launch_few<8, false, 4, 1, false>("few_down", f, s);
+        default: return wide ? launch_few<14, false, 8, 2, true>("few_down", f, s) : launch_few<14, false, 4, 1, true>("few_down", f, s);
         }
     }
     switch (m.dn.source_type) {
