@@ -29,7 +29,8 @@
 // experts 45.6 -> 39.9, four 34.5 -> 29.5, two 27.5 -> 27.4, all on the same ten 21.0 -> 27.3; five on the same ten 20.7 -> 21.3, four 20.4, both, three
 // 18.6 -> 17.2. Wider and larger layers gain throughout (eight on the same eight of 4096 x 1536, Q8_0: 539 -> 90). What the last of the eight lose is
 // arithmetic, 2.75 waves a SIMD of it: rows that come for nothing on the matrix cores. v_mfma_f32_4x4x1 gives the bits of these multiply-adds, but
-// not beside vector instructions (10 cycles, and 20 with one conversion between).
+// not beside vector instructions (10 cycles, and 20 with one conversion between); up to four rows to a task share a conversion more, in 244
+// registers where three waves a SIMD have 168 (gate/up 16 -> 50 us with what that spills).
 #include "moe_few.hpp"
 
 #include <type_traits>
