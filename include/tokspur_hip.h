@@ -185,8 +185,10 @@ int tsp_q8_matvec_many(uint32_t layout, const void* matrix, uint64_t matrix_byte
 /* include/tokspur/graph.hpp:860 `dense_mm_q8` (kernels/grouped_mm.metal:239-243; planner src/grouped_mm.cpp:48-54):
  * out[t, :] = W in[t, :] for a dense Q8_0 matrix in GGUF rows (layout 0) or q8_lanes_v1 rows (layout 1), f32 rows in
  * and out with byte strides. Decoded and accumulated in f32 (the engine stages halves); token rows that lie back to
- * back share each weight read eight at a time, and up to sixteen at a time for rows of 1024 or 2048 columns in either
- * layout (16-byte aligned buffers, at least 64 matrix rows, 32 for the lanes layout, in multiples of 4). */
+ * back share each weight read eight at a time; up to sixteen at a time for rows of up to 2048 columns in multiples of 512 (1024 in
+ * the lanes layout; matrix and token rows 16-byte aligned, at least 64 matrix rows, 32 for the lanes layout), up to ten for 2560
+ * columns, where more than eight (five) of them add two halves of a sum into the output: any number of matrix rows, any float's
+ * address, and a sum that overflows there is reported like any other; and all of them for small matrices in GGUF rows. */
 int tsp_dense_mm_q8(uint32_t layout, const void* matrix, uint64_t matrix_bytes, const float* input, uint64_t input_stride_bytes,
                     float* output, uint64_t output_stride_bytes, uint32_t tokens, uint32_t columns, uint32_t rows,
                     uint32_t* error_word, void* stream);
