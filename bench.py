@@ -334,8 +334,8 @@ def main():
         del w8
         # NOT a BASELINE configuration: the engine's own expert shape (2560 channels, 640 hidden units: src/moe_mm_many_plan.cpp:7,31)
         # with its kinds, Q4_K co-located gate/up and Q8_0 planes down, 2048 tokens, 512 experts, top-10, uniform router. Neither
-        # resident kernel takes this shape (they want 2048 columns resp. 512 hidden units): gate/up runs on the general
-        # integer-factor kernel, down on the staged kernel. 64 synthetic experts repeated eight times.
+        # resident kernel takes this shape (they want 2048 columns resp. 512 hidden units): gate/up runs on the streaming
+        # kernel, down on the one that keeps a task's rows in LDS. 64 synthetic experts repeated eight times.
         Ce, He = 2560, 640
         rep = E // 64
         ge = np.tile(synth.matrix(12, synth.tensor_seed(3, 30), He * 64, Ce), rep)

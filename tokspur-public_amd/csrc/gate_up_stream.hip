@@ -17,11 +17,12 @@
 //     barrier per step stands before the step's last group: by then every wave has the whole slab in registers, so the
 //     barrier frees it and publishes the next.
 //   * Every request is unconditional (past the end the last one again), so each wave waits with an exact count.
-// 2048 tokens, 512 experts of 2560 x 640: 340 -> 270 us a launch (half lines through registers, a fragment read from LDS right before its product
-// before); 2048 x 512: 224 -> 192 (the resident kernel). 1.39 GB are fetched at 5.2 TB/s: 944 MB of planes, heavy experts' once per task, the
-// headers' lines more than once, 0.1 GB of rows. With the nibbles' lines in L2 242 us are left, with the headers' 245, without unpacking 260: bound
-// by the lines' way in and by instruction issue (66 % of the cycles) at once. Tried: persistent workgroups that request the next item's bytes during
-// the last steps of this one (298), tasks of more than 32 rows first (280), nibbles' lines as non-temporal (285).
+// 2048 tokens, 512 experts of 2560 x 640: 340 -> 278 us a launch (half lines through registers, a fragment read from LDS right before its product
+// before; 8 us of it are the sigmoid); 2048 x 512: 224 -> 196 (the resident kernel; 4 us are sums by super-block). At 2560 x 640 with the short
+// sigmoid, 270 us: 1.39 GB are fetched at 5.2 TB/s: 944 MB of planes, heavy experts' once per task, the headers' lines more than once, 0.1 GB
+// of rows. With the nibbles' lines in L2 242 us are left, with the headers' 245, without unpacking 260: bound by the lines' way in and by
+// instruction issue (66 % of the cycles) at once. Tried: persistent workgroups that request the next item's bytes during the last steps of this
+// one (298), tasks of more than 32 rows first (280), nibbles' lines as non-temporal (285).
 #include "gate_up_resident.hpp"
 #include "mfma_quant.hpp"
 #include "resident_tasks.hpp"

@@ -22,9 +22,9 @@
 // Kernel times, before -> now (ten of 512 experts; the kernels before were one super-block per wave, rows kept in registers, or a
 // stream over the records, each on the matrix cores):
 //   one token     gate/up 2048 x 512 9.5 -> 6.3 us, 2560 x 640 14.6 -> 9.0; down 512 -> 2048 Q6_K 6.6 -> 5.2, 640 -> 2560 Q8_0 9.2 -> 5.6
-//   three tokens  gate/up 2048 x 512 16.4 -> 13.0, down 512 -> 2048 Q8_0 13.4 -> 8.0
-//   five tokens   gate/up 2560 x 640 30.8 -> 23.1 (88 MB: 18 us at the rate of a copy), down Q8_0 26.0 -> 17.6
-//   eight tokens  gate/up 2048 x 512 26.8 -> 23.3, down Q6_K 19.6 -> 17.0; eight of 128, down 768 -> 2048 Q5_1 31.4 -> 18.2
+//   three tokens  gate/up 2048 x 512 15.7 -> 11.6, down 512 -> 2048 Q8_0 13.4 -> 7.4
+//   five tokens   gate/up 2560 x 640 30.8 -> 22.8 (88 MB: 18 us at the rate of a copy), down Q8_0 26.0 -> 17.6
+//   eight tokens  gate/up 2048 x 512 27.1 -> 23.1, down Q6_K 19.6 -> 17.1; eight of 128, down 768 -> 2048 Q5_1 31.4 -> 17.2
 // Tokens that agree, a whole call of eight at 2048 x 512 with Q6_K, against the kernels with records on the matrix cores before (us): eight sets of
 // experts 45.6 -> 39.9, four 34.5 -> 29.5, two 27.5 -> 27.4, all on the same ten 21.0 -> 27.3; five on the same ten 20.7 -> 21.3, four 20.4, both, three
 // 18.6 -> 17.2. Wider and larger layers gain throughout (eight on the same eight of 4096 x 1536, Q8_0: 539 -> 90). What the last of the eight lose is
@@ -403,8 +403,8 @@ __global__ __launch_bounds__(kThreads) void one_row(OneArgs a) {
 // expert with two ballots and leaves if its own is in their second half. Nothing is planned or written first; one workgroup of the
 // gate/up launch writes the union block that the call promises. The always-on expert's tasks are its tokens by twos.
 // JOINT: a second row uses the first one's converted codes, at the price of registers (165 against 122 at Q4_K, a wave per SIMD
-// less); else the codes are converted again. Up to 2048 columns joint: 25.4 against 24.3 us for eight tokens on even experts,
-// 26 against 34 for the call where all take the same. 2560 columns: 26.3 and 24.3 us for five tokens; Q8_0 down 20.9 and 18.2.
+// less); else the codes are converted again. Up to 2048 columns joint: 23.8 against 24.6 us for eight tokens on even experts,
+// 27.6 against 30.0 for the call where all take the same. 2560 columns: 25.0 and 23.2 us for five tokens; Q8_0 down 21.0 and 17.7.
 struct FewArgs {
     OneArgs one;              // x_stride: between the token rows (gate/up) or route rows (down)
     uint32_t tokens, selected, shared_tasks;
