@@ -49,9 +49,9 @@ def rel_l2(got, ref):
 
 # ---------------------------------------------------------------------------------- dense
 
-# the tile shapes of the raw-row kernel: exact 32 x 64, 64 x 64 and 128 x 128 tiles (the last from 513 tiles of 64 x 64 on), fewer than
-# 256 weight rows at any row count, then rounded 64 x 64, 128 x 128 and 128 x 256 tiles; ragged on both sides, and an odd number of
-# super-blocks where two groups of waves share them out (or one, where the second group has none)
+# the kernels of raw rows: up to 704 tiles of 32 x 32 in fragment order, then exact 64 x 64 and 128 x 128 tiles (the last from 513 tiles of
+# 64 x 64 on), fewer than 256 weight rows at any row count, and rounded 64 x 64, 128 x 128 and 128 x 256 tiles; ragged on both sides, and an odd number
+# of super-blocks where waves or groups of waves share them out
 @pytest.mark.parametrize("tokens,rows,cols", [(32, 64, 256), (31, 65, 768), (9, 1, 512), (33, 63, 1280), (64, 130, 256), (65, 129, 768), (511, 4130, 256),
                                               (449, 4700, 768), (520, 200, 768), (512, 256, 256), (513, 257, 1280), (600, 4001, 768), (520, 8100, 256)])
 def test_dense_mm_q4k_tiles(gpu, tsp, orc, synth, tokens, rows, cols):
@@ -76,16 +76,22 @@ def test_dense_mm_q4k_tiles(gpu, tsp, orc, synth, tokens, rows, cols):
     assert np.array_equal(bf16_to_f32(bits[:, :rows]), synth.round_bf16(got)) and (bits[:, rows:] == 7).all() and gpu.error() == 0
 
 
-# the forms for few tiles: 32 x 32 up to a full round, one tile more, super-blocks that do not divide among four groups and fewer than groups, then
-# 64 x 32, and 32 rows of more tiles than a round
+# few tiles: up to a round of workgroups, one tile more, super-blocks that do not divide among four waves and fewer than waves
 @pytest.mark.parametrize("tokens,rows,cols", [(64, 4096, 256), (32, 8193, 512), (3, 33, 1536), (70, 97, 2560), (40, 4200, 768), (33, 8170, 1280), (97, 4064, 2304)])
 def test_dense_mm_q4k_few_tiles(gpu, tsp, orc, synth, tokens, rows, cols):
     test_dense_mm_q4k_tiles(gpu, tsp, orc, synth, tokens, rows, cols)
 
 
+# the smallest there is, whole tiles and one row or weight row more, one to five super-blocks; 704 tiles and more, exact (rows of more than 704 tiles:
+# 32 x 64, with one super-block for two groups 64 x 64) and rounded
+@pytest.mark.parametrize("tokens,rows,cols", [(1, 1, 256), (32, 32, 512), (33, 33, 768), (63, 31, 1024), (5, 64, 1280), (64, 11264, 256), (64, 11265, 256), (9, 22600, 512),
+                                              (200, 3300, 768), (1024, 704, 512), (1025, 704, 512)])
+def test_dense_mm_q4k_fragments(gpu, tsp, orc, synth, tokens, rows, cols):
+    test_dense_mm_q4k_tiles(gpu, tsp, orc, synth, tokens, rows, cols)
+
+
 @pytest.mark.parametrize("layout", ["raw", "planar"])
-# GGUF rows take the exact forms of the tile kernel, 32 x 64 tiles for one row and 64 x 64 for the others, their columns shared out over
-# two groups of waves; planar ones the task kernel
+# GGUF rows take the kernel for few tiles; planar ones the task kernel
 @pytest.mark.parametrize("tokens,rows,cols", [(1, 64, 256), (33, 96, 512), (128, 256, 2048), (130, 300, 1024), (257, 512, 768),
                                               (200, 100, 2048), (384, 132, 1024), (1, 68, 2048), (385, 64, 2048)])
 def test_dense_mm_q4k(gpu, tsp, orc, synth, layout, tokens, rows, cols):
@@ -108,7 +114,7 @@ def test_dense_mm_q4k(gpu, tsp, orc, synth, layout, tokens, rows, cols):
     assert np.array_equal(got_b, synth.round_bf16(got)) and gpu.error() == 0
 
 
-# (2000, 7500, 256): 256 x 256 tiles, ragged on both sides; the others are fewer tiles than the chip takes at once and get 64 x 64
+# (2000, 7500, 256): 256 x 256 tiles, ragged on both sides; (1300, 777, 1024): 64 x 64; the others are few enough for fragment order
 # (128 x 128 and 128 x 256: test_dense_mm_q4k_tiles)
 @pytest.mark.parametrize("tokens,rows,cols", [(1024, 256, 256), (1100, 300, 512), (1300, 777, 1024), (2000, 7500, 256),
                                               (512, 300, 256), (600, 1000, 512), (1000, 256, 1024)])

@@ -40,20 +40,6 @@ __device__ __forceinline__ const uint8_t* uniform_pointer(const uint8_t* p) {
     return reinterpret_cast<const uint8_t*>(uint64_t(hi) << 32 | lo);
 }
 
-// Byte N of a word as a float: one v_cvt_f32_ubyteN.
-template <int N>
-__device__ __forceinline__ float byte_as_float(uint32_t word) { return float((word >> (8 * N)) & 0xffu); }
-
-// Two weights from two codes sitting in the mantissas of two halves (q or q << 4 per half, everything else zero): each is scale *
-// code + offset evaluated as one f32 fused multiply-add whose result is rounded to half (v_fma_mix widens the half operand
-// inside the instruction, subnormals included). With scale = d * sc * 2^24 (2^20) and offset = -dmin * mn this is the f32 value
-// d * sc * q - dmin * mn exactly, then rounded once.
-__device__ __forceinline__ uint32_t two_weights(uint32_t codes, float scale, float offset) {
-    const f16x2 c = as_h2(codes);
-    const _Float16 lo = _Float16(__builtin_fmaf(float(c[0]), scale, offset)), hi = _Float16(__builtin_fmaf(float(c[1]), scale, offset));
-    return as_u32(f16x2{lo, hi});
-}
-
 // 16 bytes per lane from base + lane_offset to LDS at lds_base + AT (uniform) + 16 * lane
 template <int AT>
 __device__ __forceinline__ void to_lds(const uint8_t* base, uint32_t lane_offset, uint32_t lds_base) {
@@ -205,14 +191,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
                 w = hi ? scaled8_q4_swapped<1>(raw[P][2 * ff], raw[P][2 * ff + 1], f16x2{ps.mul[1], ps.mul[1]}, f16x2{ps.bias[1], ps.bias[1]}, q4c)
                        : scaled8_q4_swapped<0>(raw[P][2 * ff], raw[P][2 * ff + 1], f16x2{ps.mul[0], ps.mul[0]}, f16x2{ps.bias[0], ps.bias[0]}, q4c);
             } else {
-                u32x4 packed;
-#pragma unroll
-                for (int q = 0; q < 2; ++q) {
-                    const uint32_t word = raw[P][2 * ff + q], mask = hi == 0 ? kc.low : kc.high;
-                    packed[2 * q] = two_weights(word & mask, scale[hi], offset[hi]);
-                    packed[2 * q + 1] = two_weights((word >> 8) & mask, scale[hi], offset[hi]);
-                }
-                w = __builtin_bit_cast(f16x8, packed);
+                w = weights8_q4_swapped(raw[P][2 * ff], raw[P][2 * ff + 1], hi == 0 ? kc.low : kc.high, scale[hi], offset[hi]);
             }
             if (g == 3 && P == 3) read_header(b + 1);
             uint32_t from = a_at[(g + 1) % 4] + (g < 3 ? slot_now : slot_next);
@@ -412,14 +391,7 @@ int launch(DenseTileArgs a, hipStream_t s) {
     }
     constexpr uint32_t TM = WAVES / GROUPS / (TN / 32) * RT * 32;
     const uint32_t m_tiles = (a.m + TM - 1) / TM, n_tiles = (a.n + TN - 1) / TN, tiles = m_tiles * n_tiles;
-    // Each XCD fetches the activation rows and the weight rows that its run of tiles touches into an L2 of its own: the band that makes
-    // the run touch the fewest bytes.
-    uint64_t least = ~0ull;
-    for (uint32_t band = 1; band <= m_tiles; ++band) {
-        const uint32_t run = (tiles + 7) / 8, wide = std::min(n_tiles, (run + band - 1) / band), high = band * std::max(1u, run / (band * n_tiles));
-        const uint64_t bytes = uint64_t(high) * TM * 32 + uint64_t(wide) * TN * 9;
-        if (bytes < least) { least = bytes; a.band = band; }
-    }
+    a.band = dense_band(m_tiles, n_tiles, TM, TN);
     TSP_LAUNCH("gemm_dense_tile", s, (dense_tile_kernel<RT, WAVES, TN, GROUPS, EXACT><<<(tiles + 7) / 8 * 8, WAVES * 64, S::kAtLaunch ? S::kLds : 0, s>>>(a)));
     return launch_status("dense_tile");
 }
@@ -430,15 +402,9 @@ namespace tsp {
 
 int launch_dense_tile(const DenseTileArgs& a, hipStream_t s) {
     auto tiles = [&](uint64_t high, uint64_t wide) { return (a.m + high - 1) / high * ((a.n + wide - 1) / wide); };
-    if (a.m < 512 || a.n < 256) {
-        // A wave alone on its SIMD issues an instruction every eight cycles, and few tiles are waves that stand alone: as long as the chip takes
-        // the smallest tiles at once, one to a compute unit, they share out the super-blocks four ways (2560 columns, up to 4096 rows: 12.5 to 13.8 us with
-        // two groups of 64-row tiles, 10.1 to 10.7 so; 2048 columns 11.4 to 12.2, now 8.7 to 9.2; 512 columns 8.4, 7.3). With two such tiles to a
-        // compute unit nothing is left of that, with five or eight groups 0.6 us less of it. Then tiles of 64 x 32 (37 rows: 2048 x 8192 12.0
-        // and 10.6, 2560 x 6100 14.3 and 13.6), which need three super-blocks to have work for the groups.
-        if (tiles(32, 32) <= 256) return launch<1, 4, 32, 4, true>(a, s);
+    if (dense_exact(a.m, a.n)) {
+        // Few tiles are dense_fragments.hip's.
         if (a.m <= 32) return launch<1, 4, 64, 2, true>(a, s);
-        if (tiles(64, 32) <= 256 && a.k > 512) return launch<2, 4, 32, 4, true>(a, s);
         // 64 x 64 tiles while the chip takes them all at once, two to a compute unit: 13 to 24 us at 2560 columns, 41 for twice as many,
         // where 128 x 128 tiles take 34.
         if (tiles(64, 64) <= 512) return launch<2, 4, 64, 2, true>(a, s);

@@ -499,46 +499,75 @@ typedef float f32_piece __attribute__((ext_vector_type(4), aligned(4)));
 constexpr uint32_t kWaveColumns = 8 * kWave;
 __host__ __device__ constexpr uint32_t column_waves(uint32_t columns) { return (columns + kWaveColumns - 1) / kWaveColumns; }
 
+// Eight columns, their sum over the four lanes of a sub-block, and the largest half's bits without the sign: what is not finite, or too large for a
+// half, shows there.
+struct EightHalves { f16x8 v; float sum; uint32_t most; };
+template <bool FROM_BF16>
+__device__ __forceinline__ EightHalves eight_halves(const uint8_t* __restrict__ from) {
+    float v[8];
+    if constexpr (FROM_BF16) {
+        const bf16_piece w = *reinterpret_cast<const bf16_piece*>(from);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { v[2 * e] = __uint_as_float(w[e] << 16); v[2 * e + 1] = __uint_as_float(w[e] & 0xffff0000u); }
+    } else {
+        const f32_piece w0 = *reinterpret_cast<const f32_piece*>(from), w1 = *reinterpret_cast<const f32_piece*>(from + 16);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { v[e] = float(__bf16(w0[e])); v[4 + e] = float(__bf16(w1[e])); }
+    }
+    EightHalves h{};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        h.v[e] = _Float16(v[e]);
+        const uint32_t magnitude = __builtin_bit_cast(uint16_t, _Float16(h.v[e])) & 0x7fffu;
+        h.most = h.most > magnitude ? h.most : magnitude;
+        h.sum += float(h.v[e]);
+    }
+    h.sum = dpp_add<0x4E>(dpp_add<0xB1>(h.sum));
+    return h;
+}
+// Q4_K consumers (the ones that ask for sums) unpack a dword of nibbles into the column pairs (0, 2), (1, 3):
+// their activations are stored in that order, columns 1 <-> 2 and 5 <-> 6 of every eight swapped
+__device__ __forceinline__ f16x8 swapped_columns(f16x8 v) { return f16x8{v[0], v[2], v[1], v[3], v[4], v[6], v[5], v[7]}; }
+
 template <bool FROM_BF16>
 __device__ __forceinline__ void to_f16_row_part(const void* __restrict__ src, uint64_t src_stride_bytes, _Float16* __restrict__ dst,
                                                 _Float16* __restrict__ sx, uint32_t row, uint32_t part, uint32_t columns, uint32_t* error_word) {
     const uint32_t lane = threadIdx.x % kWave, c8 = part * kWave + lane;
     if (c8 * 8 >= columns) return;  // groups of four lanes leave together: a row is a multiple of 32 columns
-    const uint8_t* const from = static_cast<const uint8_t*>(src) + row * src_stride_bytes;
-    float v[8];
-    if constexpr (FROM_BF16) {
-        const bf16_piece w = *reinterpret_cast<const bf16_piece*>(from + c8 * 16);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) { v[2 * e] = __uint_as_float(w[e] << 16); v[2 * e + 1] = __uint_as_float(w[e] & 0xffff0000u); }
-    } else {
-        const f32_piece w0 = *reinterpret_cast<const f32_piece*>(from + c8 * 32), w1 = *reinterpret_cast<const f32_piece*>(from + c8 * 32 + 16);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) { v[e] = float(__bf16(w0[e])); v[4 + e] = float(__bf16(w1[e])); }
-    }
-    float sum = 0;
-    f16x8 out;
-    uint32_t most = 0;  // the largest half's bits without the sign: what is not finite, or too large for a half, shows there
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        out[e] = _Float16(v[e]);
-        const uint32_t magnitude = __builtin_bit_cast(uint16_t, _Float16(out[e])) & 0x7fffu;
-        most = most > magnitude ? most : magnitude;
-        sum += float(out[e]);
-    }
-    sum = dpp_add<0x4E>(dpp_add<0xB1>(sum));
-    // Q4_K consumers (the ones that ask for sums) unpack a dword of nibbles into the column pairs (0, 2), (1, 3):
-    // their activations are stored in that order, columns 1 <-> 2 and 5 <-> 6 of every eight swapped
-    if (sx) out = f16x8{out[0], out[2], out[1], out[3], out[4], out[6], out[5], out[7]};
-    *reinterpret_cast<f16x8*>(dst + uint64_t(row) * columns + c8 * 8) = out;
+    EightHalves h = eight_halves<FROM_BF16>(static_cast<const uint8_t*>(src) + row * src_stride_bytes + c8 * (FROM_BF16 ? 16 : 32));
+    *reinterpret_cast<f16x8*>(dst + uint64_t(row) * columns + c8 * 8) = sx ? swapped_columns(h.v) : h.v;
     if (sx && (c8 & 3) == 0) {
-        const _Float16 hi = _Float16(sum), lo = _Float16(sum - float(hi));
+        const _Float16 hi = _Float16(h.sum), lo = _Float16(h.sum - float(hi));
         const uint32_t magnitude = __builtin_bit_cast(uint16_t, hi) & 0x7fffu;
-        most = most > magnitude ? most : magnitude;
+        h.most = h.most > magnitude ? h.most : magnitude;
         _Float16* o = sx + (uint64_t(row) * (columns / 256) + c8 / 32) * 16 + c8 / 4 % 8;
         o[0] = hi;
         o[8] = lo;
     }
-    publish_error(most >= 0x7c00u ? uint32_t(TSP_ERRBIT_NONFINITE) : 0u, error_word);
+    publish_error(h.most >= 0x7c00u ? uint32_t(TSP_ERRBIT_NONFINITE) : 0u, error_word);
+}
+
+// The same into fragment order (dense_tile.hpp). Workgroup (x, y): super-block x of rows 8 y .. 8 y + 7, a wave 64 columns of them: 256 (128) bytes of a row by
+// neighbouring lanes, and out as eight rows' pieces of one fragment side by side.
+template <bool FROM_BF16>
+__global__ __launch_bounds__(256) void to_f16_fragments(const void* __restrict__ src, uint64_t src_stride_bytes, _Float16* __restrict__ dst,
+                                                        _Float16* __restrict__ sx, uint32_t rows, uint32_t columns, uint32_t* error_word) {
+    const uint32_t lane = threadIdx.x % kWave, step = threadIdx.x / kWave, c8 = lane % 8, row = blockIdx.y * 8 + lane / 8;
+    if (row >= rows) return;
+    EightHalves h = eight_halves<FROM_BF16>(static_cast<const uint8_t*>(src) + row * src_stride_bytes + ((blockIdx.x * 4 + step) * 8 + c8) * (FROM_BF16 ? 16 : 32));
+    const uint32_t block = row / 32, height = rows - block * 32 < 32 ? rows - block * 32 : 32;
+    // chunk 4 (g / 2) + 2 khalf + g % 2 of 64 columns is k-half khalf of fragment g
+    const uint32_t fragment = (blockIdx.x * 4 + step) * 4 + c8 / 4 * 2 + c8 % 2, khalf = c8 / 2 % 2;
+    *reinterpret_cast<f16x8*>(dst + uint64_t(block) * 32 * columns + ((fragment * 2 + khalf) * height + row % 32) * 8) = swapped_columns(h.v);
+    if (c8 % 4 == 0) {
+        const _Float16 hi = _Float16(h.sum), lo = _Float16(h.sum - float(hi));
+        const uint32_t magnitude = __builtin_bit_cast(uint16_t, hi) & 0x7fffu;
+        h.most = h.most > magnitude ? h.most : magnitude;
+        _Float16* o = sx + uint64_t(block) * 32 * (columns / 16) + (blockIdx.x * 2 * height + row % 32) * 8 + step * 2 + c8 / 4;
+        o[0] = hi;
+        o[height * 8] = lo;
+    }
+    publish_error(h.most >= 0x7c00u ? uint32_t(TSP_ERRBIT_NONFINITE) : 0u, error_word);
 }
 
 // Workgroup (x, y): rows 4 y .. 4 y + 3, one to a wave, columns 512 x on.
@@ -589,6 +618,14 @@ int convert_rows(const void* src, uint64_t stride, int from_bf16, _Float16* dst,
     if (from_bf16) TSP_LAUNCH("to_f16_rows", s, to_f16_rows<true><<<grid, 256, 0, s>>>(src, stride, dst, sx, rows, columns, err));
     else TSP_LAUNCH("to_f16_rows", s, to_f16_rows<false><<<grid, 256, 0, s>>>(src, stride, dst, sx, rows, columns, err));
     return launch_status("to_f16_rows");
+}
+
+// The same in fragment order: columns in whole super-blocks.
+int convert_fragments(const void* src, uint64_t stride, int from_bf16, _Float16* dst, _Float16* sx, uint32_t rows, uint32_t columns, uint32_t* err, hipStream_t s) {
+    const dim3 grid(columns / 256, (rows + 7) / 8);
+    if (from_bf16) TSP_LAUNCH("to_f16_fragments", s, to_f16_fragments<true><<<grid, 256, 0, s>>>(src, stride, dst, sx, rows, columns, err));
+    else TSP_LAUNCH("to_f16_fragments", s, to_f16_fragments<false><<<grid, 256, 0, s>>>(src, stride, dst, sx, rows, columns, err));
+    return launch_status("to_f16_fragments");
 }
 
 // f32 rows only; the caller has checked the task geometry (experts <= 512, tiles <= 256)
@@ -643,14 +680,17 @@ extern "C" int tsp_dense_mm(uint32_t encoding, uint32_t layout, const void* matr
     const auto s = static_cast<hipStream_t>(stream);
     auto* xh = static_cast<_Float16*>(workspace);
     auto* sx = reinterpret_cast<_Float16*>(static_cast<uint8_t*>(workspace) + align256(uint64_t(tokens) * columns * 2));
-    int rc = convert_rows(input, input_stride_bytes, input_is_bf16, xh, encoding == 12 ? sx : nullptr, tokens, columns, error_word, s);  // with the sums come the swapped columns
-    if (rc != TSP_OK) return rc;
     // Tiles over raw rows address the activations with 32-bit offsets; halves of 4 GiB and more take the task kernel's 64-bit row addresses.
-    if (layout == TSP_LAYOUT_GGUF && uint64_t(tokens) * columns * 2 < (1ull << 32)) {
+    const bool tiled = layout == TSP_LAYOUT_GGUF && uint64_t(tokens) * columns * 2 < (1ull << 32);
+    const uint32_t fragment_waves = tiled ? dense_fragments_waves(tokens, rows, columns) : 0;
+    int rc = fragment_waves ? convert_fragments(input, input_stride_bytes, input_is_bf16, xh, sx, tokens, columns, error_word, s)
+                            : convert_rows(input, input_stride_bytes, input_is_bf16, xh, encoding == 12 ? sx : nullptr, tokens, columns, error_word, s);  // with the sums come the swapped columns
+    if (rc != TSP_OK) return rc;
+    if (tiled) {
         DenseTileArgs t{};
         t.a = xh; t.a_stride = columns; t.sx = sx; t.w = static_cast<const uint8_t*>(matrix); t.m = tokens; t.n = rows; t.k = columns;
         t.out = output; t.out_stride = output_stride_bytes; t.out_bf16 = output_is_bf16; t.error_word = error_word;
-        return launch_dense_tile(t, s);
+        return fragment_waves ? launch_dense_fragments(t, fragment_waves, s) : launch_dense_tile(t, s);
     }
     a.a = xh; a.a_stride = columns; a.sx = sx; a.w0 = static_cast<const uint8_t*>(matrix); a.experts = 1;
     a.m = tokens; a.n = rows; a.k = columns; a.out = output; a.out_stride = output_stride_bytes; a.out_scale = 1.0f;

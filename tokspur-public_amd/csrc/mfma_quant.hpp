@@ -188,6 +188,24 @@ __device__ __forceinline__ f16x8 scaled8_q4_swapped(uint32_t w0, uint32_t w1, f1
     const f16x2 p2 = fma2(as_h2((w1 & m) | c.bits), sc, bias), p3 = fma2(as_h2(((w1 >> 8) & m) | c.bits), sc, bias);
     return f16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
 }
+// Byte N of a word as a float: one v_cvt_f32_ubyteN.
+template <int N>
+__device__ __forceinline__ float byte_as_float(uint32_t word) { return float((word >> (8 * N)) & 0xffu); }
+
+// Two weights from two codes sitting in the mantissas of two halves (q or q << 4 per half, everything else zero): each is scale *
+// code + offset evaluated as one f32 fused multiply-add whose result is rounded to half (v_fma_mix widens the half operand
+// inside the instruction, subnormals included). With scale = d * sc * 2^24 (2^20) and offset = -dmin * mn this is the f32 value
+// d * sc * q - dmin * mn exactly, then rounded once.
+__device__ __forceinline__ uint32_t two_weights(uint32_t codes, float scale, float offset) {
+    const f16x2 c = as_h2(codes);
+    const _Float16 lo = _Float16(__builtin_fmaf(float(c[0]), scale, offset)), hi = _Float16(__builtin_fmaf(float(c[1]), scale, offset));
+    return as_u32(f16x2{lo, hi});
+}
+// Eight weights from two words of nibbles, in the swapped order; mask: where the codes sit.
+__device__ __forceinline__ f16x8 weights8_q4_swapped(uint32_t w0, uint32_t w1, uint32_t mask, float scale, float offset) {
+    return __builtin_bit_cast(f16x8, u32x4{two_weights(w0 & mask, scale, offset), two_weights((w0 >> 8) & mask, scale, offset), two_weights(w1 & mask, scale, offset),
+                                           two_weights((w1 >> 8) & mask, scale, offset)});
+}
 // The scale set-up is shared by a pair of sub-blocks: the six-bit scales of sub-blocks 2P and 2P + 1 sit
 // in neighbouring bytes of the header; one byte permute puts them under 0x64 (1024 + sc as halves, side by side), one packed
 // add takes the 1024 off, and two packed multiplies make (sc, sc / 16) and (-1024 sc, -64 sc): the factors and the
