@@ -56,24 +56,27 @@ __global__ __launch_bounds__(64 * kMostWaves) __attribute__((amdgpu_waves_per_eu
 
     u32x4 staged[kWPieces];
     f16x8 af[16], sums;
-    // what is requested past the wave's last super-block comes from buffers without bytes: nothing travels
-    struct Sources { __amdgpu_buffer_rsrc_t w, a, s; };
-    auto sources = [&](bool live) {
-        return Sources{buffer(a.w, live ? uint64_t(a.n) * bpr * 144 : 0), buffer(a.a, live ? uint64_t(a.m) * a.k * 2 : 0), buffer(a.sx, live ? uint64_t(a.m) * bpr * 32 : 0)};
+    // What is requested past the wave's last super-block comes from the beginning of buffers without bytes: nothing travels. (From the beginning: whether
+    // a scalar offset counts when the hardware compares with a buffer's size is nothing to rely on.)
+    struct Sources { __amdgpu_buffer_rsrc_t w, a, s; uint32_t w_at, a_at, a_step, s_at; };
+    auto sources = [&](uint32_t b) {
+        const bool live = b < end;
+        return Sources{buffer(a.w, live ? uint64_t(a.n) * bpr * 144 : 0), buffer(a.a, live ? uint64_t(a.m) * a.k * 2 : 0), buffer(a.sx, live ? uint64_t(a.m) * bpr * 32 : 0),
+                       live ? b * 144 : 0, live ? a_base + b * 16 * a_pitch : 0, live ? a_pitch : 0, live ? s_base + b * a_pitch : 0};
     };
-    auto request_weights = [&](const Sources& s, uint32_t b) {
+    auto request_weights = [&](const Sources& s) {
 #pragma unroll
-        for (uint32_t q = 0; q < kWPieces; ++q) staged[q] = load(s.w, w_lane[q], b * 144);
+        for (uint32_t q = 0; q < kWPieces; ++q) staged[q] = load(s.w, w_lane[q], s.w_at);
     };
-    auto request_rows = [&](const Sources& s, uint32_t b, int f) { af[f] = __builtin_bit_cast(f16x8, load(s.a, a_lane, a_base + (b * 16 + f) * a_pitch)); };
-    auto request_sums = [&](const Sources& s, uint32_t b) { sums = __builtin_bit_cast(f16x8, load(s.s, a_lane, s_base + b * a_pitch)); };
+    auto request_rows = [&](const Sources& s, int f) { af[f] = __builtin_bit_cast(f16x8, load(s.a, a_lane, s.a_at + f * s.a_step)); };
+    auto request_sums = [&](const Sources& s) { sums = __builtin_bit_cast(f16x8, load(s.s, a_lane, s.s_at)); };
 
     {
-        const Sources s = sources(first < end);
-        request_weights(s, first);
+        const Sources s = sources(first);
+        request_weights(s);
 #pragma unroll
-        for (int f = 0; f < 16; ++f) request_rows(s, first, f);
-        if constexpr (EXACT) request_sums(s, first);
+        for (int f = 0; f < 16; ++f) request_rows(s, f);
+        if constexpr (EXACT) request_sums(s);
     }
     __builtin_amdgcn_sched_barrier(0);
 
@@ -81,11 +84,11 @@ __global__ __launch_bounds__(64 * kMostWaves) __attribute__((amdgpu_waves_per_eu
     const Q4Consts q4c = q4_consts();
     const Q4ScaleConsts q4s = q4_scale_consts();
     for (uint32_t b = first; b < end; ++b) {
-        const Sources next = sources(b + 1 < end);
+        const Sources next = sources(b + 1);
 #pragma unroll
         for (uint32_t q = 0; q < kWPieces; ++q) *reinterpret_cast<u32x4*>(stage + (q * kWave + lane) * 16) = staged[q];
         __builtin_amdgcn_sched_barrier(0);
-        request_weights(next, b + 1);
+        request_weights(next);
         __builtin_amdgcn_wave_barrier();  // the wave's own LDS, served in order
         RawHdrQ4 words;
         words.words = *reinterpret_cast<const uint4*>(mine);
@@ -119,7 +122,7 @@ __global__ __launch_bounds__(64 * kMostWaves) __attribute__((amdgpu_waves_per_eu
                     w = weights8_q4_swapped(raw[2 * ff], raw[2 * ff + 1], hi ? q4c.hi_mask : q4c.lo_mask, scale[hi], offset[hi]);
                     acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[f], w, acc, 0, 0, 0);
                 }
-                request_rows(next, b + 1, f);
+                request_rows(next, f);
             }
         };
         step(std::integral_constant<int, 0>{});
@@ -131,7 +134,7 @@ __global__ __launch_bounds__(64 * kMostWaves) __attribute__((amdgpu_waves_per_eu
             __builtin_amdgcn_sched_barrier(0);
             const f32x16 zero{};
             const f32x16 low = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums, minima_frag(hdr), zero, 0, 0, 0);
-            request_sums(next, b + 1);
+            request_sums(next);
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[v] = __builtin_fmaf(-hdr.dmin, low[v], __builtin_fmaf(hdr.d, blk[v], acc[v]));
         }
