@@ -170,19 +170,19 @@ int launch(uint32_t layout, const Q8Args& a, hipStream_t stream) {
     return launch_status("q8_blocks");
 }
 
-// Two to sixteen token rows against raw rows: a workgroup per 16 matrix rows (q8_small.hip), or the persistent kernel (q8_mfma.hip).
-// The latter's time hardly falls below a floor however few the rows, 25 us at 2048 columns and 14 at 1024 (17 and 12 at nine tokens
-// or more), the former's is proportional to them: 16.1 us at 16 000 x 2048, 24.5 against 25.0 at 24 576, 31 against 25 at 32 000; at
-// 1024 columns 11.2 us at 16 000, 16 against 16 at 24 576; with nine or more tokens 17 at 12 000 x 2048, 24 against 18 at 16 000. Of more
-// than 2048 columns the persistent kernel takes ten token rows a pass (2560 columns) or five: 27 us against 35 at 24 576 x 2560, 37
-// against 36 at 32 000; two passes for sixteen tokens 56 against 75 at 32 000, 78 against 80 at 40 000, 124 against 88 at 64 000.
-// Widths that it refuses all go to the former.
+// Two to sixteen token rows against raw rows: a workgroup per 16 matrix rows (q8_small.hip), or a persistent kernel (q8_resident.hip; q8_mfma.hip for up to
+// ten token rows of more than 2048 columns). The latter starts slowly, with five to ten microseconds whatever the rows, the former's time is
+// proportional to them, and to the token rows beyond eight. Small, then persistent, us a call: eight token rows 8000 x 2048 9.0 and 9.2, 12 000 12.8 and
+// 12.7, 16 000 16.7 and 14.1; 12 000 x 1024 9.1 and 8.7, x 256 5.7 and 5.6; nine 4000 x 2048 6.9 and 9.0, 6000 11.8 and 8.9, 16 000 22.6 and 14.0; 6000 x
+// 512 6.0 and 5.3, x 256 5.0 and 5.2. Of more than 2048 columns up to ten token rows (five where columns are no two halves) 27 and 35 at 24 576 x 2560, 37
+// and 36 at 32 000; more, all in registers, sixteen 12 000 x 2560 21.8 and 23.5, 16 000 28.2 and 24.8.
+// Widths that the persistent kernels refuse all go to the former.
 bool small_rows(const void* matrix, const float* x, uint64_t x_stride_bytes, uint32_t columns, uint32_t rows, uint32_t tokens) {
     if (!q8_small_takes(matrix, x, x_stride_bytes, columns, rows)) return false;
     if (x_stride_bytes != uint64_t(columns) * 4 || !q8_mfma_supported(matrix, x, columns, rows)) return true;
-    if (columns <= 2048) return rows < (tokens > 8 ? 14000u : 24576u);
-    const uint32_t at_once = columns % 512 == 0 ? 10 : 5;
-    return rows < (tokens > 8 ? 22000u : 31000u) * ((tokens + at_once - 1) / at_once);
+    if (columns <= 2048) return rows < (tokens > 8 ? 6000u : 12000u);
+    if (tokens > (columns % 512 == 0 ? 10u : 5u)) return rows < (tokens > 8 ? 13000u : 16000u);
+    return rows < (tokens > 8 ? 22000u : 31000u);
 }
 
 }  // namespace

@@ -1,14 +1,15 @@
-// Q8_0 GEMV for up to sixteen token rows on the matrix cores (LM head, verify): y[m, r] = sum_k d[r, k/32] * q[r, k] * x[m, k].
+// Q8_0 GEMV for up to sixteen token rows on the matrix cores (LM head, verify): y[m, r] = sum_k d[r, k/32] * q[r, k] * x[m, k]. Raw rows of more than 2048 columns
+// with up to ten token rows, and q8_lanes_v1 rows; the other raw rows are q8_resident.hip's.
 //
-// A Q8_0 row is a run of 34-byte blocks (f16 scale + 32 int8). The int8 quants are exact halves, so a block is one
+// A Q8_0 row is a run of 34-byte blocks (f16 scale + 32 int8). The int8 quants are exact halves and bf16, so a block is one
 // 16x16x32 MFMA step per 16 weight rows: the block's 32 columns are the instruction's whole K, a lane (n, kq) supplies the
 // eight quants 8 kq .. 8 kq + 7 of weight row n, and the sixteen operand rows on the other side are the token rows (eight
 // of them repeated when there are only eight). The block's scale multiplies the f32 result once (4 fused multiply-adds per
-// lane and 16 weight rows). The activations are scaled by a power of two and split into hi + lo halves, staged once in
+// lane and 16 weight rows). Up to 2048 columns the activations are scaled by a power of two and split into hi + lo halves, staged once in
 // LDS for all of K, so the result carries 22 significant bits of x: this is the f32 GEMV of the engine to within f32
 // accumulation error, at ~1.3 VALU operations per weight byte whatever the number of token rows. Rows of more than 2048
 // columns are staged as the floats they are, three bf16 pieces each (mfma_quant.hpp): fifteen operand rows for up to five
-// token rows, in the same LDS, or for up to ten where a workgroup takes half of the columns; more take more passes.
+// token rows, in the same LDS, or for up to ten where a workgroup takes half of the columns.
 //
 // Raw rows are only 2-byte aligned inside, so the bytes travel global -> registers -> LDS -> registers: a wave reads
 // its 32 weight rows x 8 blocks (272 contiguous bytes per row, 16-byte aligned because 8 blocks = 17 x 16 bytes) with
@@ -17,16 +18,17 @@
 // aligned dword reads and a byte funnel shift. The next group of 8 blocks is in flight while the current one is multiplied.
 //
 // Workgroups are persistent (one per compute unit, 8 waves): the activations are staged once per workgroup, which owns
-// every n-th of the matrix's 32-row tiles (n workgroups: at any moment the grid reads one stretch of the matrix, 1 us
+// every n-th of the matrix's tiles (n workgroups: at any moment the grid reads one stretch of the matrix, 1 us
 // faster at 151 936 x 2048 than a contiguous share per workgroup); its waves take the workgroup's tiles through a counter in LDS. A
 // lane asks for its share of the token rows first and for its wave's first weight bytes second, and stages the rows
 // while the weights travel. Every address inside the loop is a uniform base plus a lane offset fixed before the loop.
 //
-// Nine to sixteen token rows do not fit LDS for all of K beside the weight tiles, so that variant splits K in two:
+// Token rows that do not fit LDS for all of K beside the weight tiles (more than eight, in f32 five) split K in two:
 // even workgroups take the first half of the columns, odd ones the second, each over its share of the tiles, and both
 // add their f32 partial sums into an output the host cleared before the launch (two addends onto zero: the sum does
 // not depend on which arrives first). The matrix is still read once.
 #include "q8_mfma.hpp"
+#include "q8_resident.hpp"
 
 #include <type_traits>
 
@@ -230,15 +232,13 @@ __device__ __forceinline__ void check_joined(Joined (&all)[N], uint32_t& bad) {
     }
 }
 
-// DEPTH = (tile, group) items whose bytes are on their way while one is multiplied (1, 2 or 4; it divides the number of groups
-// of a workgroup). ROWS = token rows staged (8: all of K per workgroup; 16: half of K per workgroup, sums added into y; 5
-// and 10: the same in f32).
+// DEPTH = (tile, group) items whose bytes are on their way while one is multiplied (1 or 2; it divides the number of groups
+// of a workgroup). ROWS = token rows staged, in f32 (5: all of K per workgroup; 10: half of K per workgroup, sums added into y).
 template <int DEPTH, int ROWS>
 __global__ __launch_bounds__(kThreads, 1) void q8_mfma_kernel(Q8MfmaArgs a) {
-    constexpr bool F32 = ROWS % kF32Rows == 0;
-    constexpr int SETS = F32 ? ROWS / kF32Rows : 1, kRows = F32 ? 8 * SETS : ROWS;  // kRows: of each of two operand planes; as much LDS in f32
-    constexpr uint32_t KSPLIT = kRows / 8;
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // [hi plane][lo plane][8 weight tiles]
+    constexpr int SETS = ROWS / kF32Rows;
+    constexpr uint32_t KSPLIT = SETS;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // [sets of sixteen operand rows][8 weight tiles]
     __shared__ float wave_max[kF32Rows][kWaves];
     __shared__ uint32_t next_tile;
 
@@ -250,16 +250,14 @@ __global__ __launch_bounds__(kThreads, 1) void q8_mfma_kernel(Q8MfmaArgs a) {
     const uint32_t sharer = blockIdx.x / KSPLIT, sharers = gridDim.x / KSPLIT;  // the host launches a multiple of KSPLIT
     if (tid == 0) next_tile = 0;
     __syncthreads();  // the tile counter is set before any wave takes from it
-    _Float16* const a_hi = reinterpret_cast<_Float16*>(lds);
-    _Float16* const a_lo = a_hi + kRows * K;
-    uint8_t* const tile = lds + 2 * kRows * K * 2 + wave * kTileBytes;
+    __bf16* const operands = reinterpret_cast<__bf16*>(lds);
+    uint8_t* const tile = lds + SETS * 16 * K * 2 + wave * kTileBytes;
 
     // ---- the token rows: this lane's 16-byte chunks are requested first (they come from cache and return first), then the
     // wave's first weight bytes, and only then the arithmetic. The weights travel while the rows are staged.
     uint32_t bad = 0;
-    float4 xv[F32 ? kF32Rows : kMine][2];
-    if constexpr (F32) request_f32_rows<SETS>(a, K, k0, xv);
-    else request_token_rows<kRows>(a, K, k0, xv);
+    float4 xv[kF32Rows][2];
+    request_f32_rows<SETS>(a, K, k0, xv);
     // chunk `id` of a group tile: row id / 17 of the wave's 32, bytes (id % 17) * 16 of that row's 272. The byte offsets from
     // the tile's first row and the group's first byte never change, so a request is a uniform address plus a lane offset.
     uint32_t chunk_at[kStageLoads];
@@ -301,23 +299,17 @@ __global__ __launch_bounds__(kThreads, 1) void q8_mfma_kernel(Q8MfmaArgs a) {
     if (t < share_end) {
         fetch_group(t * 32, 0, std::integral_constant<int, 0>{});
         if constexpr (DEPTH >= 2) fetch_group(t * 32, 1, std::integral_constant<int, 1 % DEPTH>{});
-        if constexpr (DEPTH >= 4) {
-            fetch_group(t * 32, 2, std::integral_constant<int, 2 % DEPTH>{});
-            fetch_group(t * 32, 3, std::integral_constant<int, 3 % DEPTH>{});
-        }
     }
     __builtin_amdgcn_sched_barrier(0);  // every request above is out before the first wait below
-    float inv_scale = 1.0f, back[SETS][kF32Rows];
-    if constexpr (F32) stage_f32_rows<SETS>(xv, K, reinterpret_cast<__bf16*>(lds), wave_max, back, bad);
-    else inv_scale = stage_token_rows<kRows>(xv, K, a_hi, a_lo, wave_max[0], bad);
+    float back[SETS][kF32Rows];
+    stage_f32_rows<SETS>(xv, K, operands, wave_max, back, bad);
 
     // The activation chunk of block B of group g, columns 8 kq .. 8 kq + 7, is chunk g * 32 + B * 4 + kq of row `arow`, kept at
-    // position chunk ^ arow. arow < kRows only flips the low bits, which B % kVariants and kq decide: the lane keeps one
+    // position chunk ^ arow. arow only flips the four low bits, which B % kVariants and kq decide: the lane keeps one
     // address per variant and the rest of the chunk index is an offset known when the code is compiled (B) or uniform (g).
-    constexpr uint32_t kOperandRows = F32 ? 16 : kRows;
-    const uint32_t arow = n16 & (kOperandRows - 1);
-    constexpr uint32_t kVariants = kOperandRows / 4;
-    uint32_t a_at[kVariants];  // in halves, from the start of a plane
+    const uint32_t arow = n16;
+    constexpr uint32_t kVariants = 4;
+    uint32_t a_at[kVariants];  // in bf16s, from the start of a set
 #pragma unroll
     for (uint32_t v = 0; v < kVariants; ++v) a_at[v] = (arow * chunks + ((v * 4 + kq) ^ arow)) * 8;
     auto store_group = [&](auto set_tag) {
@@ -347,14 +339,13 @@ __global__ __launch_bounds__(kThreads, 1) void q8_mfma_kernel(Q8MfmaArgs a) {
             const uint32_t group = !wraps ? ahead : more ? ahead - groups : g;
             fetch_group(following * 32, group, set_tag);
             const uint8_t* mine = tile + n16 * kTileStride + kq * 8;
-            float group_sum[SETS][2][4] = {};  // in f32 a group's blocks are added up by themselves: a tenth as many roundings of the whole sum
-            auto& sums = F32 ? group_sum : acc;
+            float sums[SETS][2][4] = {};  // a group's blocks are added up by themselves: a tenth as many roundings of the whole sum
             auto block = [&](auto b_tag) {
                 constexpr int B = decltype(b_tag)::value;
                 // the lane's eight quants of the block, for rows n16 and n16 + 16 of the tile: bytes 34 B + 2 + 8 kq .. + 8 of the
                 // row, dword aligned for odd B, 2 bytes past a dword for even B
                 constexpr uint32_t Q_AT = 34 * B + 2, ALIGNED = Q_AT & ~3u;
-                std::conditional_t<F32, bf16x8, f16x8> b_frag[2];
+                bf16x8 b_frag[2];
                 float scale_d[2];
 #pragma unroll
                 for (int nt = 0; nt < 2; ++nt) {
@@ -370,31 +361,20 @@ __global__ __launch_bounds__(kThreads, 1) void q8_mfma_kernel(Q8MfmaArgs a) {
                         w[0] = __builtin_amdgcn_alignbyte(d[1], d[0], 2);
                         w[1] = __builtin_amdgcn_alignbyte(d[2], d[1], 2);
                     }
-                    if constexpr (F32) b_frag[nt] = quants8_bf16(w[0], w[1]);
-                    else b_frag[nt] = quants8(w[0], w[1]);
+                    b_frag[nt] = quants8_bf16(w[0], w[1]);
                     scale_d[nt] = half_bits_to_float(*reinterpret_cast<const uint16_t*>(tile + (nt * 16 + n16) * kTileStride + 34 * B));
                 }
                 // columns g * 256 + B * 32 + 8 kq of the lane's token row
                 const uint32_t at = a_at[B % kVariants] + (g * 32 + (B / kVariants) * kVariants * 4) * 8;
                 const f32x4 zero{};
 #pragma unroll
-                for (int nt = 0; nt < 2; ++nt) {
-                    f32x4 part;
-                    if constexpr (F32) {
+                for (int nt = 0; nt < 2; ++nt)
 #pragma unroll
-                        for (int set = 1; set < SETS; ++set) {
-                            part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(a_hi + set * 16 * K + at), b_frag[nt], zero, 0, 0, 0);
+                    for (int set = SETS - 1; set >= 0; --set) {
+                        const f32x4 part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(operands + set * 16 * K + at), b_frag[nt], zero, 0, 0, 0);
 #pragma unroll
-                            for (int v = 0; v < 4; ++v) sums[set][nt][v] = __builtin_fmaf(scale_d[nt], part[v], sums[set][nt][v]);
-                        }
-                        part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(a_hi + at), b_frag[nt], zero, 0, 0, 0);
-                    } else {  // the lo halves of the rows first, the hi halves on top of them: one f32 result per block to scale
-                        part = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const f16x8*>(a_lo + at), b_frag[nt], zero, 0, 0, 0);
-                        part = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const f16x8*>(a_hi + at), b_frag[nt], part, 0, 0, 0);
+                        for (int v = 0; v < 4; ++v) sums[set][nt][v] = __builtin_fmaf(scale_d[nt], part[v], sums[set][nt][v]);
                     }
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) sums[0][nt][v] = __builtin_fmaf(scale_d[nt], part[v], sums[0][nt][v]);  // rows 4 kq + v
-                }
             };
             block(std::integral_constant<int, 0>{});
             block(std::integral_constant<int, 1>{});
@@ -404,50 +384,31 @@ __global__ __launch_bounds__(kThreads, 1) void q8_mfma_kernel(Q8MfmaArgs a) {
             block(std::integral_constant<int, 5>{});
             block(std::integral_constant<int, 6>{});
             block(std::integral_constant<int, 7>{});
-            if constexpr (F32) {
 #pragma unroll
-                for (int set = 0; set < SETS; ++set)
+            for (int set = 0; set < SETS; ++set)
 #pragma unroll
-                    for (int nt = 0; nt < 2; ++nt)
+                for (int nt = 0; nt < 2; ++nt)
 #pragma unroll
-                        for (int v = 0; v < 4; ++v) acc[set][nt][v] += group_sum[set][nt][v];
-            }
+                    for (int v = 0; v < 4; ++v) acc[set][nt][v] += sums[set][nt][v];
         };
         uint32_t g = 0;
         do {  // the host picks a DEPTH that divides the number of groups; there is at least one, and the compiler has to know it to count what is in flight
             item(g, std::integral_constant<int, 0>{});
             if constexpr (DEPTH >= 2) item(g + 1, std::integral_constant<int, 1 % DEPTH>{});
-            if constexpr (DEPTH >= 4) {
-                item(g + 2, std::integral_constant<int, 2 % DEPTH>{});
-                item(g + 3, std::integral_constant<int, 3 % DEPTH>{});
-            }
         } while ((g += DEPTH) < groups);
         if constexpr (KSPLIT == 2) check_joined(joined, bad);
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt) {
             const uint32_t r = row0 + nt * 16 + n16;
-            if constexpr (F32) {
 #pragma unroll
-                for (int set = 0; set < SETS; ++set) {
-                    f32_row_sums(acc[set][nt], kq, back[set], [&](uint32_t row, float val) {
-                        const uint32_t m = set * kF32Rows + row;
-                        if (m >= a.m || r >= a.rows) return;
-                        if (nonfinite(val)) bad = TSP_ERRBIT_NONFINITE;
-                        if constexpr (KSPLIT == 1) a.y[uint64_t(m) * a.rows + r] = val;
-                        else joined[(set * 2 + nt) * 4 + row % 4] = join(a.y, m * a.rows + r, val);  // (row 4 is in other lanes than row 0)
-                    });
-                }
-                continue;
-            }
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const uint32_t m = 4 * kq + v;  // lanes with 4 kq >= kRows hold repeats of rows 0 .. kRows - 1
-                if (m < kRows && m < a.m && r < a.rows) {
-                    const float val = acc[0][nt][v] * inv_scale;
+            for (int set = 0; set < SETS; ++set) {
+                f32_row_sums(acc[set][nt], kq, back[set], [&](uint32_t row, float val) {
+                    const uint32_t m = set * kF32Rows + row;
+                    if (m >= a.m || r >= a.rows) return;
                     if (nonfinite(val)) bad = TSP_ERRBIT_NONFINITE;
                     if constexpr (KSPLIT == 1) a.y[uint64_t(m) * a.rows + r] = val;
-                    else joined[nt * 4 + v] = join(a.y, m * a.rows + r, val);
-                }
+                    else joined[(set * 2 + nt) * 4 + row % 4] = join(a.y, m * a.rows + r, val);  // (row 4 is in other lanes than row 0)
+                });
             }
         }
     }
@@ -687,20 +648,6 @@ __global__ __launch_bounds__(kThreads, 1) void q8_lanes_mfma_kernel(Q8MfmaArgs a
     publish_error(bad, a.error_word);
 }
 
-// At most `most` token rows at a time, evenly.
-template <class Launch>
-void for_f32_passes(const Q8MfmaArgs& all, uint32_t most, Launch launch) {
-    const uint32_t passes = (all.m + most - 1) / most;
-    for (uint32_t p = 0, done = 0; p < passes; ++p) {
-        Q8MfmaArgs a = all;
-        a.m = (all.m - done + (passes - p) - 1) / (passes - p);
-        a.x += uint64_t(done) * all.columns;
-        a.y += uint64_t(done) * all.rows;
-        launch(a);
-        done += a.m;
-    }
-}
-
 }  // namespace
 
 namespace tsp {
@@ -710,24 +657,23 @@ bool q8_mfma_supported(const void* matrix, const float* x, uint32_t columns, uin
            reinterpret_cast<uintptr_t>(x) % 16 == 0;
 }
 
-bool q8_mfma_supported_16(const void* matrix, const float* x, uint32_t columns, uint32_t rows) {
-    if (columns > kHalvesColumns) return q8_mfma_supported(matrix, x, columns, rows);  // in passes of its own
-    return q8_mfma_supported(matrix, x, columns, rows) && columns % 512 == 0 && rows >= 64;
-}
+bool q8_mfma_supported_16(const void* matrix, const float* x, uint32_t columns, uint32_t rows) { return q8_mfma_supported(matrix, x, columns, rows); }
 
 int q8_mfma(const void* matrix, const float* x, float* y, uint32_t columns, uint32_t rows, uint32_t width, uint32_t* error_word, hipStream_t s) {
+    // Up to ten token rows of 2560 columns (five where the columns are no two halves) are one pass here, with fewer matrix instructions than pieces by themselves
+    // take: 2560 columns, eight token rows by 64 001 55.7 us with the top-64 behind, 63.3 the other way; sixteen, two passes, 109.7 against 71.7.
+    const uint32_t at_once = columns % 512 == 0 ? 2 * kF32Rows : kF32Rows;
+    // Up to 2048 columns a small matrix is multiplied by floats in three pieces, at no cost there; two halves, which the large ones take, are 2 to 3 % faster
+    // (eight token rows by 151 936 x 2048 82.9 us with the top-64 behind, 85.3 in three pieces).
+    if (columns <= kHalvesColumns || width > at_once) return q8_resident(false, rows < (width > 8 ? 14000u : 24576u), matrix, x, y, columns, rows, width, error_word, s);
     const Q8MfmaArgs a{static_cast<const uint8_t*>(matrix), x, y, columns, rows, width, error_word};
-    // 8 rows x all columns and 16 rows x half the columns stage the same number of bytes
+    // five rows x all columns and ten rows x half the columns stage the same number of bytes
     const uint32_t lds_bytes = 2 * 8 * columns * 2 + kWaves * kTileBytes;
     static std::atomic<uint64_t> raised{0};
     static int units_of[64] = {};
     int device = 0;
     if (setup_pending(raised, &device)) {
         const int most = int(2 * 8 * kMostColumns * 2 + kWaves * kTileBytes);
-        TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_mfma_kernel<1, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
-        TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_mfma_kernel<2, 8>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
-        TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_mfma_kernel<1, 16>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
-        TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_mfma_kernel<2, 16>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
         TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_mfma_kernel<1, kF32Rows>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
         TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_mfma_kernel<2, kF32Rows>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
         TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_mfma_kernel<1, 2 * kF32Rows>), hipFuncAttributeMaxDynamicSharedMemorySize, most));
@@ -737,35 +683,16 @@ int q8_mfma(const void* matrix, const float* x, float* y, uint32_t columns, uint
     const int compute_units = units_of[device];
     const uint32_t tiles = (rows + 31) / 32;
     uint32_t grid = uint32_t(compute_units > 0 ? compute_units : 256);
-    // two workgroups (one per half of the columns) share each run of tiles; the output starts at zero
-    uint32_t pairs = grid / 2 ? grid / 2 : 1;
-    if (pairs * kWaves > tiles) pairs = (tiles + kWaves - 1) / kWaves;
-    if (columns > kHalvesColumns && width > kF32Rows && columns % 512 == 0) {
-        // 2560 columns, five groups to a half: one pass for 8 token rows and two for 16, where five at a time would take two and four
-        // (151 936 rows, 8 token rows: 96 us against 166)
-        for_f32_passes(a, 2 * kF32Rows, [&](const Q8MfmaArgs& pass) {
-            clear_output(pass.y, uint64_t(pass.m) * rows, s);
-            TSP_LAUNCH("q8_mfma", s, q8_mfma_kernel<1, 2 * kF32Rows><<<2 * pairs, kThreads, lds_bytes, s>>>(pass));
-        });
-        return launch_status("q8_mfma");
-    }
-    if (width > 8 && columns <= kHalvesColumns) {
+    if (width > kF32Rows) {  // two workgroups (one per half of the columns) share each run of tiles; the output starts at zero
+        uint32_t pairs = grid / 2 ? grid / 2 : 1;
+        if (pairs * kWaves > tiles) pairs = (tiles + kWaves - 1) / kWaves;
         clear_output(y, uint64_t(width) * rows, s);
-        if ((columns / 512) % 2 == 0) TSP_LAUNCH("q8_mfma", s, q8_mfma_kernel<2, 16><<<2 * pairs, kThreads, lds_bytes, s>>>(a));
-        else TSP_LAUNCH("q8_mfma", s, q8_mfma_kernel<1, 16><<<2 * pairs, kThreads, lds_bytes, s>>>(a));
+        TSP_LAUNCH("q8_mfma", s, q8_mfma_kernel<1, 2 * kF32Rows><<<2 * pairs, kThreads, lds_bytes, s>>>(a));
         return launch_status("q8_mfma");
     }
     if (grid * kWaves > tiles) grid = (tiles + kWaves - 1) / kWaves;
-    if (columns > kHalvesColumns) {
-        for_f32_passes(a, kF32Rows, [&](const Q8MfmaArgs& pass) {
-            if ((columns / 256) % 2 == 0) TSP_LAUNCH("q8_mfma", s, q8_mfma_kernel<2, kF32Rows><<<grid, kThreads, lds_bytes, s>>>(pass));
-            else TSP_LAUNCH("q8_mfma", s, q8_mfma_kernel<1, kF32Rows><<<grid, kThreads, lds_bytes, s>>>(pass));
-        });
-        return launch_status("q8_mfma");
-    }
-    // two items in flight measured best on MI355X (one: 72 us, two: 69 us, four: 75 us at 151 936 x 2048)
-    if ((columns / 256) % 2 == 0) TSP_LAUNCH("q8_mfma", s, q8_mfma_kernel<2, 8><<<grid, kThreads, lds_bytes, s>>>(a));
-    else TSP_LAUNCH("q8_mfma", s, q8_mfma_kernel<1, 8><<<grid, kThreads, lds_bytes, s>>>(a));
+    if ((columns / 256) % 2 == 0) TSP_LAUNCH("q8_mfma", s, q8_mfma_kernel<2, kF32Rows><<<grid, kThreads, lds_bytes, s>>>(a));
+    else TSP_LAUNCH("q8_mfma", s, q8_mfma_kernel<1, kF32Rows><<<grid, kThreads, lds_bytes, s>>>(a));
     return launch_status("q8_mfma");
 }
 
@@ -781,6 +708,9 @@ bool q8_lanes_mfma_supported_16(const void* matrix, const float* x, uint32_t col
 
 int q8_lanes_mfma(const void* matrix, const float* x, float* y, uint32_t columns, uint32_t rows, uint32_t width, uint32_t* error_word,
                   hipStream_t s) {
+    // In one pass instead of two, though a wave's 256 columns are half a run there: 2560 columns, 16 token rows by 151 936 215 -> 157 us with the top-64 behind,
+    // twelve by 33 000 71 -> 52. Where one pass is enough here it is the faster one (2048 columns, four token rows by 151 936 79 against 88).
+    if (columns > kHalvesColumns && width > 2 * kF32Rows) return q8_resident(true, true, matrix, x, y, columns, rows, width, error_word, s);
     const Q8MfmaArgs a{static_cast<const uint8_t*>(matrix), x, y, columns, rows, width, error_word};
     const uint32_t lds_bytes = 2 * 8 * columns * 2 + kWaves * kLaneTileBytes;
     static std::atomic<uint64_t> raised{0};
@@ -804,12 +734,9 @@ int q8_lanes_mfma(const void* matrix, const float* x, float* y, uint32_t columns
     uint32_t pairs = grid / 2 ? grid / 2 : 1;
     if (pairs * kWaves > tiles) pairs = (tiles + kWaves - 1) / kWaves;
     if (columns > kHalvesColumns && width > kF32Rows) {
-        // 2560 columns: one pass for up to ten token rows and two for 16, where five at a time take two and four (151 936 rows with the
-        // top-64 behind: six rows 183 -> 111 us, 12 271 -> 212, 16 357 -> 217)
-        for_f32_passes(a, 2 * kF32Rows, [&](const Q8MfmaArgs& pass) {
-            clear_output(pass.y, uint64_t(pass.m) * rows, s);
-            TSP_LAUNCH("q8_lanes_mfma", s, q8_lanes_mfma_kernel<1, 2 * kF32Rows><<<2 * pairs, kThreads, lds_bytes, s>>>(pass));
-        });
+        // 2560 columns: one pass for up to ten token rows, where five at a time take two (151 936 rows, six token rows with the top-64 behind: 183 -> 111 us)
+        clear_output(y, uint64_t(width) * rows, s);
+        TSP_LAUNCH("q8_lanes_mfma", s, q8_lanes_mfma_kernel<1, 2 * kF32Rows><<<2 * pairs, kThreads, lds_bytes, s>>>(a));
         return launch_status("q8_lanes_mfma");
     }
     if (width > 8 && columns <= kHalvesColumns) {
@@ -820,9 +747,7 @@ int q8_lanes_mfma(const void* matrix, const float* x, float* y, uint32_t columns
     }
     if (grid * kWaves > tiles) grid = (tiles + kWaves - 1) / kWaves;
     if (columns > kHalvesColumns) {  // 2560: five runs
-        for_f32_passes(a, kF32Rows, [&](const Q8MfmaArgs& pass) {
-            TSP_LAUNCH("q8_lanes_mfma", s, q8_lanes_mfma_kernel<1, kF32Rows><<<grid, kThreads, lds_bytes, s>>>(pass));
-        });
+        TSP_LAUNCH("q8_lanes_mfma", s, q8_lanes_mfma_kernel<1, kF32Rows><<<grid, kThreads, lds_bytes, s>>>(a));
         return launch_status("q8_lanes_mfma");
     }
     if ((columns / 512) % 2 == 0) TSP_LAUNCH("q8_lanes_mfma", s, q8_lanes_mfma_kernel<2, 8><<<grid, kThreads, lds_bytes, s>>>(a));
