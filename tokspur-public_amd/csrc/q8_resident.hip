@@ -247,10 +247,10 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(W
                 float part[WAVES];
 #pragma unroll
                 for (uint32_t w = 0; w < WAVES; ++w) part[w] = set[(d * WAVES + w) * (kSumBytes / 4) + from];  // all on their way at once
-                float sum = part[0];
+                double total = part[0];  // rounded once: the pieces of a block's product, which meet in one accumulator, are rounded once more than by themselves
 #pragma unroll
-                for (uint32_t w = 1; w < WAVES; ++w) sum += part[w];
-                sum *= largest[0][m];
+                for (uint32_t w = 1; w < WAVES; ++w) total += part[w];
+                const float sum = float(total) * largest[0][m];
                 const uint32_t row = (tile + d * step) * kTileRows + r;
                 const bool there = u < kTileRows * a.m && row < a.rows;
                 if (there && nonfinite(sum)) bad = TSP_ERRBIT_NONFINITE;
