@@ -783,6 +783,13 @@ def test_grouped_moe_down_rows_in_lds_errors(gpu, tsp, synth, dn_type, hidden):
     assert gpu.error() == 0 and np.array_equal(y, want)
 
 
+@pytest.mark.parametrize("dn_type", [8, 7])
+def test_grouped_moe_down_rows_in_lds_of_512(gpu, tsp, orc, synth, dn_type):
+    """Four steps, from one route an expert on where the register-resident kernel has the width otherwise: results and reports."""
+    test_grouped_moe_other_planar_kinds(gpu, tsp, orc, synth, 12, dn_type, 512, 512)
+    test_grouped_moe_down_rows_in_lds_errors(gpu, tsp, synth, dn_type, 512)
+
+
 def test_grouped_moe_sticky_errors(gpu, tsp, synth):
     channels, hidden, experts, selected, n = 256, 256, 4, 2, 40
     gate = synth.matrix(12, 3101, hidden * experts, channels)

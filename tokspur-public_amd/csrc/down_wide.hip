@@ -1,5 +1,5 @@
 // Grouped down GEMM for experts in Q8_0 planes (quants / d) or Q5_1 planes (nibbles / fifth bits / d, m) of 128 to 768 hidden units
-// in multiples of 128 except 512 (down_resident.hip), the task's h rows in LDS: y[route, channel] = 256 * sum_k h[slot, k] / 256 * w[channel, k].
+// in multiples of 128 (512: where down_resident.hip is not the faster one), the task's h rows in LDS: y[route, channel] = 256 * sum_k h[slot, k] / 256 * w[channel, k].
 //
 // The launch is a stream of expert weights from HBM and of f32 results back to it; what it costs is how many requests are on
 // their way. Hence:
@@ -276,6 +276,7 @@ int launch_kind(const ResidentDownArgs& a, uint32_t hidden, int groups, hipStrea
         case 1: return launch_steps<KIND, 1>(a, groups, s);
         case 2: return launch_steps<KIND, 2>(a, groups, s);
         case 3: return launch_steps<KIND, 3>(a, groups, s);
+        case 4: return launch_steps<KIND, 4>(a, groups, s);
         case 5: return launch_steps<KIND, 5>(a, groups, s);
         default: return launch_steps<KIND, 6>(a, groups, s);
     }
@@ -287,7 +288,7 @@ namespace tsp {
 
 // The rows of 1024 hidden units (132 KB) would leave no LDS for the waves' stages; 896 are not built.
 bool wide_down_takes(uint32_t source_type, uint32_t channels, uint32_t hidden) {
-    return (source_type == kQ8 || source_type == kQ51) && hidden >= 128 && hidden <= 768 && hidden % 128 == 0 && hidden != 512 && channels >= 256 && channels % 256 == 0;
+    return (source_type == kQ8 || source_type == kQ51) && hidden >= 128 && hidden <= 768 && hidden % 128 == 0 && channels >= 256 && channels % 256 == 0;
 }
 
 int launch_wide_down(const ResidentDownArgs& a, uint32_t hidden, hipStream_t s) {

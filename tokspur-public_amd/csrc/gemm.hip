@@ -970,13 +970,19 @@ int grouped_moe(const tsp_grouped_moe* m, const tsp_shared_expert* shared, void*
     }
     if (rc != TSP_OK) return rc;
     const uint64_t shared_span = shared ? uint64_t(m->tokens) * shared->y_stride_bytes : 0;
-    // At 512 columns the h rows fit the waves' registers (2048 x 512, 512 experts, Q5_1, 400 tokens: 319 us a sublayer against 325 with the rows in LDS).
+    // At 512 columns the h rows fit the waves' registers.
     // Q6_K with fewer than eight items of 128 channels to a compute unit: the resident kernel's start (tables, rows, the first tiles) weighs more than
     // its stream, and a workgroup per item is through sooner (64 experts of 1024 x 512: 64 tokens 39 us a sublayer against 46, 700 tokens 54
     // against 61, 5.7 items 80 against 82; 128 experts, 7.7 items 93 against 97; 128 experts of 2048, 8.2 items 59 against 54).
-    const bool brief = fast_down && uint64_t(l.bound) * m->channels < 8 * 256 * 128;
-    const bool resident = !brief && resident_down_takes(down_type, m->channels, m->hidden) && uint64_t(routes) * m->y_stride_bytes < (1ull << 32) && shared_span < (1ull << 32);
-    const bool wide = !resident && wide_down_takes(down_type, m->channels, m->hidden) && y_span <= 0xffff0000u;
+    const bool small = uint64_t(l.bound) * m->channels < 8 * 256 * 128, brief = fast_down && small;
+    // Q8_0 and Q5_1 planes of 512 hidden units in such layers: a share of the resident kernel's that changes its task now and then loads registers anew each
+    // time, the wide one's next rows travel beside the last products. Kernels alone, 64 experts of 1024 x 512: 762 tokens Q8_0 33.2 -> 23.7 us, Q5_1 33.0 -> 24.6,
+    // 2048 41.0 -> 32.4 and 41.4 -> 33.3, 16 11.2 -> 9.8 and 11.4 -> 10.6; below a route an expert 12 tokens 8.4 and 9.4. With many items they are even (512
+    // experts of 2048, a sublayer of 600 tokens 396 and 391 us, of 2048 528 and 540).
+    const bool wide_fits = wide_down_takes(down_type, m->channels, m->hidden) && y_span <= 0xffff0000u;
+    const bool wide_first = wide_fits && small && routes >= m->experts;
+    const bool resident = !brief && !wide_first && resident_down_takes(down_type, m->channels, m->hidden) && uint64_t(routes) * m->y_stride_bytes < (1ull << 32) && shared_span < (1ull << 32);
+    const bool wide = !resident && wide_fits;
     if (resident || wide) {
         ResidentDownArgs r{};
         r.hbuf = hbuf; r.down = static_cast<const uint8_t*>(m->down); r.shared_down = shared ? static_cast<const uint8_t*>(shared->down) : nullptr;
