@@ -549,3 +549,41 @@ def test_router_f32_batch_pieces_far_apart(gpu, synth, weight_exponent, row_expo
     others = np.ones(got.shape, dtype=bool)
     others[130], others[:, 70] = False, False
     assert np.array_equal(got[others], usual[others])
+
+
+@pytest.mark.parametrize("tokens,selected,experts", [(1, 1, 2), (9, 3, 8), (511, 2, 64), (513, 7, 32), (1025, 16, 16), (1536, 5, 130), (2048, 10, 512), (2048, 15, 512)])
+def test_grouped_products_prepare_routes_and_lists(gpu, tsp, orc, synth, tokens, selected, experts):
+    """The launch that a grouped product starts with: its routes, counts and tasks against the oracle's, either side of the 512 tokens that go in one launch, ids whose
+    rows 8 bytes align and ids whose rows they do not; and with ids out of range, or twice in a token, what the entry points of their own make of them."""
+    channels, hidden = 256, 32
+    w = tsp.PlanarMoeWeights(gpu, 12, 8, channels, hidden, experts, synth.matrix(12, 71, hidden * experts, channels), synth.matrix(12, 72, hidden * experts, channels),
+                             synth.matrix(8, 73, channels * experts, hidden))
+    ids = random_ids(np.random.default_rng(tokens + selected), tokens, selected, experts, skew=selected == 10)
+    x = gpu.upload(synth.activations_f32(74, (tokens, channels)))
+    scratch = tsp.GroupedScratch(gpu, tokens, selected, experts, channels, hidden)
+
+    def prepared(ids, words_before):
+        room = gpu.upload(np.concatenate([np.zeros(words_before, np.uint32), ids]))
+        for buffer in (scratch.token_map, scratch.counts, scratch.tasks):
+            buffer.zero_()
+        tsp.planar_nax_grouped_moe(gpu, w, room[words_before:], x, tokens, selected, scratch)
+        return u32(scratch.token_map).reshape(experts, tokens), u32(scratch.counts), u32(scratch.tasks)
+
+    want_map, want_counts, _ = orc.grouped_routes(ids, experts, selected, tokens)
+    want_map = want_map.reshape(experts, tokens)
+    for words_before in (0, 1):
+        token_map, counts, tasks = prepared(ids, words_before)
+        assert gpu.error() == 0 and np.array_equal(counts, want_counts)
+        assert all(np.array_equal(token_map[e, :counts[e]], want_map[e, :counts[e]]) for e in range(experts))
+        assert np.array_equal(tasks, orc.grouped_tasks(want_counts, experts, selected, tokens, 32)[0])
+    for at, value in [(tokens * selected - 1, experts), (0, 0xffffffff)] + [(tokens // 2 * selected + selected - 1, int(ids[tokens // 2 * selected]))] * (selected > 1):
+        wrong = ids.copy()
+        wrong[at] = value
+        token_map, counts, tasks = prepared(wrong, 0)
+        assert gpu.error() == tsp.ERRBIT_INDEX
+        alone_map, alone_counts = gpu.grouped_routes(gpu.upload(wrong), experts, selected, tokens)
+        alone_tasks = gpu.grouped_tasks(alone_counts, experts, selected, tokens, 32)
+        assert gpu.error() == tsp.ERRBIT_INDEX
+        alone_map, alone_counts = u32(alone_map).reshape(experts, tokens), u32(alone_counts)
+        assert alone_counts.sum() < tokens * selected and np.array_equal(counts, alone_counts) and np.array_equal(tasks, u32(alone_tasks))
+        assert all(np.array_equal(token_map[e, :counts[e]], alone_map[e, :counts[e]]) for e in range(experts))

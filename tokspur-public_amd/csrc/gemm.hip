@@ -578,25 +578,34 @@ __global__ __launch_bounds__(256) void to_f16_rows(const void* __restrict__ src,
     if (row < rows) to_f16_row_part<FROM_BF16>(src, src_stride_bytes, dst, sx, row, blockIdx.x, columns, error_word);
 }
 
-// The two task lists of a grouped product (workgroups 0 and 1) and the row conversion (all other workgroups) in one launch:
-// neither needs the other, both need only what the route permutation before them wrote or nothing at all, and a launch of
-// its own costs each of these small kernels more than its work.
+// What a grouped product needs before its first matrix instruction: the two task lists (workgroups 0 and 1), each expert's routes (ROUTES: the next
+// `experts` workgroups; else they are there) and the row conversion (all others) in one launch: a launch of its own costs each of these small kernels
+// more than its work. With ROUTES the lists' workgroups count the ids for themselves.
 struct TaskLists {
-    const uint32_t* counts; uint32_t* tasks0; uint32_t tile0; uint32_t* tasks1; uint32_t tile1; uint32_t experts, selected, tokens;
+    const uint32_t* ids; uint32_t *token_map, *counts;
+    uint32_t* tasks0; uint32_t tile0; uint32_t* tasks1; uint32_t tile1; uint32_t experts, selected, tokens;
     bool every_token1;  // list 1 also holds the always-on expert's tasks
     uint32_t* classes1;  // list 1 is a 64-row list: its tasks by number of rows (task_class_lists_block), or null
 };
+template <bool ROUTES>
 __global__ __launch_bounds__(512) void tasks_and_rows(TaskLists t, const void* __restrict__ src, uint64_t src_stride_bytes, _Float16* __restrict__ dst,
                                                       _Float16* __restrict__ sx, uint32_t rows, uint32_t columns, uint32_t* error_word) {
-    __shared__ uint32_t tiles_scan[512];
-    __shared__ uint32_t routes_scan[512];
-    __shared__ uint32_t third_scan[512];
+    __shared__ __attribute__((aligned(16))) uint32_t counted[ROUTES ? 2048 : 4];
+    __shared__ uint32_t totals[24];
+    const uint32_t others = 2 + (ROUTES ? t.experts : 0);
     if (blockIdx.x < 2) {
-        grouped_tasks_block(t.counts, blockIdx.x == 0 ? t.tasks0 : t.tasks1, blockIdx.x == 0 ? t.tile0 : t.tile1, t.experts, t.selected, t.tokens,
-                            error_word, tiles_scan, routes_scan, blockIdx.x == 1 && t.every_token1);
-        if (blockIdx.x == 1 && t.classes1) task_class_lists_block(t.counts, t.classes1, t.experts, t.selected, t.tokens, t.every_token1, tiles_scan, routes_scan, third_scan);
+        const uint32_t* counts = t.counts;
+        if constexpr (ROUTES) {
+            count_routes_block(t.ids, t.experts, t.selected, t.tokens, counted);
+            counts = counted;
+        }
+        grouped_tasks_block(counts, blockIdx.x == 0 ? t.tasks0 : t.tasks1, blockIdx.x == 0 ? t.tile0 : t.tile1, t.experts, t.selected, t.tokens,
+                            error_word, totals, blockIdx.x == 1 && t.every_token1);
+        if (blockIdx.x == 1 && t.classes1) task_class_lists_block(counts, t.classes1, t.experts, t.selected, t.tokens, t.every_token1, totals);
+    } else if (ROUTES && blockIdx.x < others) {
+        expert_routes_block<512>(t.ids, t.token_map, t.counts, blockIdx.x - 2, t.experts, t.selected, t.tokens, error_word, totals);
     } else {
-        const uint32_t parts = column_waves(columns), block = blockIdx.x - 2, row = block / parts * 8 + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+        const uint32_t parts = column_waves(columns), block = blockIdx.x - others, row = block / parts * 8 + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
         if (row < rows) to_f16_row_part<false>(src, src_stride_bytes, dst, sx, row, block % parts, columns, error_word);
     }
 }
@@ -628,11 +637,19 @@ int convert_fragments(const void* src, uint64_t stride, int from_bf16, _Float16*
     return launch_status("to_f16_fragments");
 }
 
-// f32 rows only; the caller has checked the task geometry (experts <= 512, tiles <= 256)
-int lists_and_rows(const TaskLists& t, const void* src, uint64_t stride, _Float16* dst, _Float16* sx, uint32_t rows, uint32_t columns,
-                   uint32_t* err, hipStream_t s) {
-    const uint32_t grid = 2 + (rows + 7) / 8 * column_waves(columns);
-    TSP_LAUNCH("tasks_and_rows", s, tasks_and_rows<<<grid, 512, 0, s>>>(t, src, stride, dst, sx, rows, columns, err));
+// Routes, task lists and rows (f32 only); the caller has checked the geometry of the routes (tsp_grouped_routes) and of the tasks (experts <= 512, tiles <= 256).
+// Up to 512 tokens, a thread each in the lists' workgroups, in one launch: 16 tokens of 64 experts 6.5 -> 4.6 us, 203 of 512 9.8 -> 6.6, 500 of 512 9.9 ->
+// 6.4, and no gap between two. With more their counting takes as long as the launch that it saves, or longer (600 tokens 10.0 us, 2048 16.4 against 9.9 and 17.4
+// in two, and the rows come later).
+int prepare_grouped(const TaskLists& t, const void* src, uint64_t stride, _Float16* dst, _Float16* sx, uint32_t rows, uint32_t columns, uint32_t* err, hipStream_t s) {
+    const uint32_t row_groups = (rows + 7) / 8 * column_waves(columns);
+    if (t.tokens <= 512) {
+        TSP_LAUNCH("tasks_and_rows", s, tasks_and_rows<true><<<2 + t.experts + row_groups, 512, 0, s>>>(t, src, stride, dst, sx, rows, columns, err));
+        return launch_status("tasks_and_rows");
+    }
+    const int rc = tsp_grouped_routes(t.ids, t.token_map, t.counts, t.experts, t.selected, t.tokens, err, s);
+    if (rc != TSP_OK) return rc;
+    TSP_LAUNCH("tasks_and_rows", s, tasks_and_rows<false><<<2 + row_groups, 512, 0, s>>>(t, src, stride, dst, sx, rows, columns, err));
     return launch_status("tasks_and_rows");
 }
 
@@ -786,9 +803,8 @@ extern "C" int tsp_grouped_mm(uint32_t encoding, uint32_t layout, const void* ma
     auto* xh = reinterpret_cast<_Float16*>(ws);
     auto* sx = reinterpret_cast<_Float16*>(ws + l.sx);
     auto* task_list = reinterpret_cast<uint32_t*>(ws + l.tasks);
-    int rc = tsp_grouped_routes(ids, token_map, counts, experts, selected, tokens, error_word, stream);
-    if (rc == TSP_OK) rc = lists_and_rows(TaskLists{counts, tasks, 32, task_list, kTaskRows, experts, selected, tokens, false, nullptr}, input, input_stride_bytes, xh, sx,
-                                          l.in_rows, columns, error_word, s);
+    const int rc = prepare_grouped(TaskLists{ids, token_map, counts, tasks, 32, task_list, kTaskRows, experts, selected, tokens, false, nullptr}, input, input_stride_bytes, xh, sx,
+                                   l.in_rows, columns, error_word, s);
     if (rc != TSP_OK) return rc;
     GemmArgs a{};
     a.a = xh; a.a_stride = columns; a.sx = sx; a.w0 = static_cast<const uint8_t*>(matrices); a.raw_expert_bytes = expert_bytes;
@@ -939,10 +955,10 @@ int grouped_moe(const tsp_grouped_moe* m, const tsp_shared_expert* shared, void*
     auto* task_list = reinterpret_cast<uint32_t*>(ws + l.tasks);
     auto* hbuf = reinterpret_cast<_Float16*>(ws + l.hbuf);
 
-    rc = tsp_grouped_routes(m->ids, m->token_map, m->counts, m->experts, m->selected, m->tokens, m->error_word, stream);
     // only the Q4_K gate/up kernels want the activation sums and the column order that goes with them
-    if (rc == TSP_OK) rc = lists_and_rows(TaskLists{m->counts, m->tasks, 32, task_list, kTaskRows, m->experts, m->selected, m->tokens, shared != nullptr, reinterpret_cast<uint32_t*>(ws + l.classes)}, m->x,
-                                          m->x_stride_bytes, xh, fast_gate_up ? sx : nullptr, m->tokens, m->channels, m->error_word, s);
+    rc = prepare_grouped(TaskLists{m->ids, m->token_map, m->counts, m->tasks, 32, task_list, kTaskRows, m->experts, m->selected, m->tokens, shared != nullptr,
+                                   reinterpret_cast<uint32_t*>(ws + l.classes)},
+                         m->x, m->x_stride_bytes, xh, fast_gate_up ? sx : nullptr, m->tokens, m->channels, m->error_word, s);
     if (rc != TSP_OK) return rc;
 
     PlanarStagedArgs staged{};

@@ -20,52 +20,15 @@ __global__ __launch_bounds__(kRouteThreads) void grouped_routes_kernel(const uin
                                                              uint32_t* __restrict__ counts, uint32_t experts, uint32_t selected,
                                                              uint32_t tokens, uint32_t* error_word) {
     __shared__ uint32_t wave_totals[kRouteThreads / kWave];
-    const uint32_t expert = blockIdx.x, tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-    uint32_t accumulated = 0, bad = 0;
-    for (uint32_t base = 0; base < tokens; base += kRouteThreads) {
-        const uint32_t token = base + tid;
-        uint32_t slot = 0xffffffffu, matches = 0;
-        if (token < tokens) {
-            const uint32_t* row = ids + uint64_t(token) * selected;
-            if (selected % 2 == 0 && reinterpret_cast<uintptr_t>(ids) % 8 == 0) {  // 8-byte aligned rows of an even number of ids: half as many loads
-                for (uint32_t i = 0; i < selected; i += 2) {
-                    const uint2 pair = *reinterpret_cast<const uint2*>(row + i);
-                    if (pair.x >= experts || pair.y >= experts) bad = TSP_ERRBIT_INDEX;
-                    if (pair.x == expert) { slot = i; ++matches; }
-                    if (pair.y == expert) { slot = i + 1; ++matches; }
-                }
-            } else {
-                for (uint32_t i = 0; i < selected; ++i) {
-                    const uint32_t id = row[i];
-                    if (id >= experts) bad = TSP_ERRBIT_INDEX;
-                    if (id == expert) { slot = i; ++matches; }
-                }
-            }
-        }
-        if (matches > 1) bad = TSP_ERRBIT_INDEX;
-        const bool found = matches == 1;
-        const uint64_t mask = __builtin_amdgcn_ballot_w64(found);
-        const uint32_t prefix = __builtin_popcountll(mask & ((1ull << lane) - 1ull));
-        if (lane == 0) wave_totals[wave] = __builtin_popcountll(mask);
-        __syncthreads();
-        uint32_t before = 0, chunk = 0;
-        for (uint32_t w = 0; w < kRouteThreads / kWave; ++w) { if (w < wave) before += wave_totals[w]; chunk += wave_totals[w]; }
-        if (found) token_map[uint64_t(expert) * tokens + accumulated + before + prefix] = token * selected + slot;
-        accumulated += chunk;
-        __syncthreads();
-    }
-    if (tid == 0) counts[expert] = accumulated;
-    publish_error(bad, error_word);
+    expert_routes_block<kRouteThreads>(ids, token_map, counts, blockIdx.x, experts, selected, tokens, error_word, wave_totals);
 }
 
 // Block b writes list b: the same counts tiled two ways in one launch (tasks1 may be null with a grid of one).
 __global__ __launch_bounds__(512) void grouped_tasks_kernel(const uint32_t* __restrict__ counts, uint32_t* __restrict__ tasks0, uint32_t tile0,
                                                             uint32_t* __restrict__ tasks1, uint32_t tile1, uint32_t experts, uint32_t selected,
                                                             uint32_t tokens, uint32_t* error_word) {
-    __shared__ uint32_t tiles_scan[512];
-    __shared__ uint32_t routes_scan[512];
-    grouped_tasks_block(counts, blockIdx.x == 0 ? tasks0 : tasks1, blockIdx.x == 0 ? tile0 : tile1, experts, selected, tokens, error_word,
-                        tiles_scan, routes_scan);
+    __shared__ uint32_t totals[16];
+    grouped_tasks_block(counts, blockIdx.x == 0 ? tasks0 : tasks1, blockIdx.x == 0 ? tile0 : tile1, experts, selected, tokens, error_word, totals);
 }
 
 // 128 threads, one per flat route (T*S <= 128); the block's layout and arithmetic: union_block (grouping_device.hpp).

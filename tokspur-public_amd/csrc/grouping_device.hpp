@@ -1,5 +1,5 @@
-// Device code shared by grouping.hip, gemm.hip and moe_few.hip: the task list of the grouped GEMMs and the union
-// records of a step of at most eight tokens.
+// Device code shared by grouping.hip, gemm.hip and moe_few.hip: an expert's routes, the task list of the grouped GEMMs and the
+// union records of a step of at most eight tokens.
 #pragma once
 #include "tsp_common.hpp"
 
@@ -35,14 +35,111 @@ __device__ __forceinline__ void scan512(uint32_t (&v)[N], uint32_t (&grand)[N], 
     }
 }
 
+// A workgroup of THREADS threads writes one expert's routes: token_map[e*T + k] = t*S + slot for the k-th token (ascending) that names e once,
+// counts[e] = how many do. `wave_totals`: a word of LDS per wave.
+template <uint32_t THREADS>
+__device__ __forceinline__ void expert_routes_block(const uint32_t* __restrict__ ids, uint32_t* __restrict__ token_map, uint32_t* __restrict__ counts, uint32_t expert,
+                                                    uint32_t experts, uint32_t selected, uint32_t tokens, uint32_t* error_word, uint32_t* wave_totals) {
+    const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+    uint32_t accumulated = 0, bad = 0;
+    for (uint32_t base = 0; base < tokens; base += THREADS) {
+        const uint32_t token = base + tid;
+        uint32_t slot = 0xffffffffu, matches = 0;
+        if (token < tokens) {
+            const uint32_t* row = ids + uint64_t(token) * selected;
+            if (selected % 2 == 0 && reinterpret_cast<uintptr_t>(ids) % 8 == 0) {  // 8-byte aligned rows of an even number of ids: half as many loads
+                for (uint32_t i = 0; i < selected; i += 2) {
+                    const uint2 pair = *reinterpret_cast<const uint2*>(row + i);
+                    if (pair.x >= experts || pair.y >= experts) bad = TSP_ERRBIT_INDEX;
+                    if (pair.x == expert) { slot = i; ++matches; }
+                    if (pair.y == expert) { slot = i + 1; ++matches; }
+                }
+            } else {
+                for (uint32_t i = 0; i < selected; ++i) {
+                    const uint32_t id = row[i];
+                    if (id >= experts) bad = TSP_ERRBIT_INDEX;
+                    if (id == expert) { slot = i; ++matches; }
+                }
+            }
+        }
+        if (matches > 1) bad = TSP_ERRBIT_INDEX;
+        const bool found = matches == 1;
+        const uint64_t mask = __builtin_amdgcn_ballot_w64(found);
+        const uint32_t prefix = __builtin_popcountll(mask & ((1ull << lane) - 1ull));
+        if (lane == 0) wave_totals[wave] = __builtin_popcountll(mask);
+        __syncthreads();
+        uint32_t before = 0, chunk = 0;
+        for (uint32_t w = 0; w < THREADS / kWave; ++w) { if (w < wave) before += wave_totals[w]; chunk += wave_totals[w]; }
+        if (found) token_map[uint64_t(expert) * tokens + accumulated + before + prefix] = token * selected + slot;
+        accumulated += chunk;
+        __syncthreads();
+    }
+    if (tid == 0) counts[expert] = accumulated;
+    publish_error(bad, error_word);
+}
+
+// The same counts of at most 512 tokens, for all experts, by one workgroup of 512 threads, which then need not wait for the experts' workgroups. What is
+// wrong with the ids is theirs to report. `counted`: 2048 words of LDS, 16-byte aligned, the counts in the first 512; an expert has four
+// counters, by lane, since lanes that add to the same one take turns.
+__device__ __forceinline__ void count_routes_block(const uint32_t* __restrict__ ids, uint32_t experts, uint32_t selected, uint32_t tokens, uint32_t* counted) {
+    const uint32_t tid = threadIdx.x;
+    reinterpret_cast<uint4*>(counted)[tid] = uint4{0, 0, 0, 0};
+    uint32_t id[16];
+    if (tid < tokens) {
+        const uint32_t* const row = ids + tid * selected;
+        const bool pairs = selected % 2 == 0 && reinterpret_cast<uintptr_t>(ids) % 8 == 0;
+#pragma unroll
+        for (uint32_t i = 0; i < 16; i += 2) {
+            if (i < selected && pairs) {
+                const uint2 two = *reinterpret_cast<const uint2*>(row + i);
+                id[i] = two.x; id[i + 1] = two.y;
+            } else {
+                if (i < selected) id[i] = row[i];
+                if (i + 1 < selected) id[i + 1] = row[i + 1];
+            }
+        }
+    }
+    __syncthreads();
+    if (tid < tokens) {
+        bool wrong = id[0] >= experts;
+#pragma unroll
+        for (uint32_t i = 1; i < 16; ++i)
+            if (i < selected) {
+                wrong |= id[i] >= experts;
+#pragma unroll
+                for (uint32_t j = 0; j < i; ++j) wrong |= id[i] == id[j];
+            }
+        auto count = [&](uint32_t e) { atomicAdd(&counted[e * 4 + tid % 4], 1u); };
+        if (!__builtin_amdgcn_ballot_w64(wrong)) {
+#pragma unroll
+            for (uint32_t i = 0; i < 16; ++i)
+                if (i < selected) count(id[i]);
+        } else {  // an id counts if it is an expert's and no other of the token's
+#pragma unroll 1
+            for (uint32_t i = 0; i < selected; ++i) {
+                const uint32_t mine = ids[tid * selected + i];
+                uint32_t alike = 0;
+#pragma unroll 1
+                for (uint32_t j = 0; j < selected; ++j) alike += ids[tid * selected + j] == mine ? 1 : 0;
+                if (mine < experts && alike == 1) count(mine);
+            }
+        }
+    }
+    __syncthreads();
+    const uint4 four = reinterpret_cast<const uint4*>(counted)[tid];
+    __syncthreads();
+    counted[tid] = (four.x + four.y) + (four.z + four.w);
+    __syncthreads();
+}
+
 // One block of 512 threads writes one list; experts <= 512. tiles(e) = ceil(min(counts[e], T) / tile), exclusive scan over
-// the experts, task i of expert e is (e, i * tile); unused slots up to the bound are 0xFFFFFFFF. The two scan arrays (512
-// words each) are the caller's LDS.
+// the experts, task i of expert e is (e, i * tile); unused slots up to the bound are 0xFFFFFFFF. `totals`: LDS of
+// the scans, eight words for each of two (three in the class lists).
 // `every_token` appends ceil(tokens / tile) tasks (experts, i * tile) after the experts' own: an always-on expert whose rows
 // are the tokens themselves (the bound grows by that many slots).
 __device__ __forceinline__ void grouped_tasks_block(const uint32_t* __restrict__ counts, uint32_t* __restrict__ tasks, uint32_t tile,
                                                     uint32_t experts, uint32_t selected, uint32_t tokens, uint32_t* error_word,
-                                                    uint32_t* tiles_scan, uint32_t* routes_scan, bool every_token = false) {
+                                                    uint32_t* totals, bool every_token = false) {
     const uint32_t tid = threadIdx.x;
     const uint32_t extra = every_token ? (tokens + tile - 1) / tile : 0;
     const uint32_t bound = tokens * selected / tile + experts + extra;
@@ -51,12 +148,10 @@ __device__ __forceinline__ void grouped_tasks_block(const uint32_t* __restrict__
     if (count > tokens) bad = TSP_ERRBIT_INDEX;
     const uint32_t n = ((count < tokens ? count : tokens) + tile - 1) / tile;
     uint32_t scans[2] = {n, count}, sums[2];
-    scan512(scans, sums, tiles_scan);
-    (void)routes_scan;
+    scan512(scans, sums, totals);
     const uint32_t total = sums[0], routes = sums[1];
     const uint32_t offset = scans[0] - n;
-    for (uint32_t i = tid; i < bound; i += 512) { tasks[2 + 2 * i] = 0xffffffffu; tasks[3 + 2 * i] = 0xffffffffu; }
-    __syncthreads();
+    for (uint32_t i = total + extra + tid; i < bound; i += 512) { tasks[2 + 2 * i] = 0xffffffffu; tasks[3 + 2 * i] = 0xffffffffu; }
     if (tid < experts)
         for (uint32_t i = 0; i < n; ++i)
             if (offset + i < bound) { tasks[2 + 2 * (offset + i)] = tid; tasks[3 + 2 * (offset + i)] = i * tile; }
@@ -75,8 +170,7 @@ __device__ __forceinline__ void grouped_tasks_block(const uint32_t* __restrict__
 // second kind's. Of an expert's tasks only the last can have fewer than 64 rows, so the lists follow from the counts alone:
 // the same block of 512 threads that wrote the task list writes them, from three more scans (experts <= 512).
 __device__ __forceinline__ void task_class_lists_block(const uint32_t* __restrict__ counts, uint32_t* __restrict__ out, uint32_t experts,
-                                                       uint32_t selected, uint32_t tokens, bool every_token, uint32_t* scan_all,
-                                                       uint32_t* scan_small, uint32_t* scan_large) {
+                                                       uint32_t selected, uint32_t tokens, bool every_token, uint32_t* totals) {
     constexpr uint32_t tile = 64;
     const uint32_t tid = threadIdx.x;
     const uint32_t extra = every_token ? (tokens + tile - 1) / tile : 0;
@@ -85,8 +179,7 @@ __device__ __forceinline__ void task_class_lists_block(const uint32_t* __restric
     const uint32_t n = (count + tile - 1) / tile;
     const uint32_t small = n && count - (n - 1) * tile <= 32 ? 1 : 0;  // the last task is a small one
     uint32_t scans[3] = {n, small, n - small}, sums[3];
-    scan512(scans, sums, scan_all);
-    (void)scan_small; (void)scan_large;
+    scan512(scans, sums, totals);
     const uint32_t total = sums[0], total_small = sums[1], total_large = sums[2];
     const uint32_t first = scans[0] - n, first_small = scans[1] - small, first_large = scans[2] - (n - small);
     uint32_t* list_small = out + 2;
