@@ -240,7 +240,7 @@ def test_dense_mm_q8(gpu, tsp, orc, synth, tokens, cols, rows):
         tsp.dense_mm_q8(gpu, tsp.LAYOUT_PLANAR_V3, gpu.upload(w), gpu.upload(x), tokens, cols, rows, x_stride=(cols + 4) * 4)
 
 
-@pytest.mark.parametrize("tokens,cols,rows", [(1, 64, 5), (70, 128, 33), (200, 2048, 512), (129, 512, 2048), (64, 4096, 64)])
+@pytest.mark.parametrize("tokens,cols,rows", [(1, 64, 5), (70, 128, 33), (200, 2048, 512), (129, 512, 2048), (64, 4096, 64), (45, 1088, 30)])
 def test_dense_mm_q8_staged(gpu, tsp, orc, synth, tokens, cols, rows):
     # the many-row form of graph.hpp:860 `dense_mm_q8`: matrix and rows as halves, one matrix-core GEMM. Both layouts, rows with
     # padding on both sides (canaries stay), tiles that overhang the matrix on either edge, and agreement with the streaming

@@ -220,66 +220,59 @@ __global__ __launch_bounds__(WAVES * kWave, 4) void q8_gemm_split(Q8GemmArgs a) 
     publish_error(bad, a.error_word);
 }
 
-// Both operands to halves in one launch (two small ones cost more than their work): workgroups below `w_groups` decode the matrix, the
-// others round the token rows.
-// Matrix: sixteen weights per thread, half a block. GGUF rows are 34-byte blocks (f16 d, 32 int8); q8_lanes_v1 rows keep the scales
-// first, then runs of 16 blocks with byte = index * width + block % 16 (src/expert_lanes.cpp:60-119).
-// Token rows: eight values per thread; a value that does not fit a half (or is not finite) raises the non-finite bit.
+// Both operands to halves in one launch (two small ones cost more than their work): the first `rows` rows of the grid are the matrix's, the others
+// the token rows. Workgroup (x, y): rows 4 x .. 4 x + 3, one to a wave, columns 512 y on, eight to a lane, with no division left to the lanes.
+// GGUF rows are 34-byte blocks (f16 d, 32 int8); q8_lanes_v1 rows keep the scales first, then runs of 16 blocks with byte = index * width +
+// block % 16 (src/expert_lanes.cpp:60-119). A token's value that does not fit a half (or is not finite) raises the non-finite bit.
+// Bound by memory from some 1000 rows on, below by a trip there. A flat index divided by the row's length in 64 bits, element-wise loads and sixteen weights
+// to a lane before: 2048 x 2560 with 640 matrix rows 9.6 -> 8.2 us, 2048 x 2048 with 512 8.8 -> 7.9, 2048 x 512 with 1024 4.4 -> 4.0.
 struct OperandsArgs {
     const uint8_t* matrix;
     const float* x;
     uint64_t x_stride;  // bytes
     _Float16 *w16, *x16;
-    uint32_t layout, columns, rows, tokens, w_groups;
+    uint32_t layout, columns, rows, tokens;
     uint32_t* error_word;
 };
+using four_floats = f32x4 __attribute__((aligned(4)));
+using four_quants = uint32_t __attribute__((aligned(2)));  // rows and blocks are even byte counts
 __global__ __launch_bounds__(256) void q8_operands_to_f16(OperandsArgs a) {
-    if (blockIdx.x < a.w_groups) {
-        const uint64_t at = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-        const uint32_t halves = a.columns / 16, blocks = a.columns / 32;
-        if (at >= uint64_t(a.rows) * halves) return;
-        const uint32_t row = uint32_t(at / halves), part = uint32_t(at % halves), block = part / 2, index = part % 2 * 16;
-        const uint8_t* data = a.matrix + uint64_t(row) * blocks * 34;
+    const uint32_t lane = threadIdx.x % kWave, row = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), c8 = blockIdx.y * kWave + lane;
+    if (row >= a.rows + a.tokens || c8 * 8 >= a.columns) return;
+    f16x8 h;
+    if (row < a.rows) {
+        const uint32_t blocks = a.columns / 32, block = c8 / 4, index = c8 % 4 * 8;
+        const uint8_t* const data = a.matrix + uint64_t(row) * blocks * 34;
         float d;
-        int q[16];
+        uint32_t q[2];
         if (a.layout == TSP_LAYOUT_GGUF) {
-            const uint16_t* b = reinterpret_cast<const uint16_t*>(data + block * 34);  // rows and blocks are even byte counts
-            d = half_bits_to_float(b[0]);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const uint32_t two = b[1 + index / 2 + i];
-                q[2 * i] = int(int8_t(two)); q[2 * i + 1] = int(int8_t(two >> 8));
-            }
+            const uint8_t* const b = data + block * 34;
+            d = half_bits_to_float(*reinterpret_cast<const uint16_t*>(b));
+            const four_quants* const from = reinterpret_cast<const four_quants*>(b + 2 + index);
+            q[0] = from[0]; q[1] = from[1];
         } else {
             const uint32_t run = block / 16, width = blocks - run * 16 < 16 ? blocks - run * 16 : 16;
-            const uint8_t* from = data + blocks * 2 + run * 512 + block % 16 + index * width;
+            const uint8_t* const from = data + blocks * 2 + run * 512 + block % 16 + index * width;
             d = half_bits_to_float(uint32_t(data[block * 2]) | (uint32_t(data[block * 2 + 1]) << 8));
+            q[0] = q[1] = 0;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) q[i] = int(int8_t(from[i * width]));
+            for (int i = 0; i < 8; ++i) q[i / 4] |= uint32_t(from[i * width]) << (i % 4 * 8);
         }
-        f16x8* const to = reinterpret_cast<f16x8*>(a.w16 + uint64_t(row) * a.columns + part * 16);
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            f16x8 w;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) w[e] = _Float16(d * float(q[8 * h + e]));  // d * q is exact in f32: one rounding
-            to[h] = w;
-        }
+        for (int e = 0; e < 8; ++e) h[e] = _Float16(d * float(int8_t(q[e / 4] >> (e % 4 * 8))));  // d * q is exact in f32: one rounding
+        *reinterpret_cast<f16x8*>(a.w16 + uint64_t(row) * a.columns + c8 * 8) = h;
         return;
     }
-    const uint64_t i = uint64_t(blockIdx.x - a.w_groups) * blockDim.x + threadIdx.x;
+    const uint32_t token = row - a.rows;
+    const four_floats* const from = reinterpret_cast<const four_floats*>(reinterpret_cast<const uint8_t*>(a.x) + token * a.x_stride + c8 * 32);
+    const f32x4 v0 = from[0], v1 = from[1];
     uint32_t bad = 0;
-    if (i < uint64_t(a.tokens) * (a.columns / 8)) {
-        const uint32_t r = uint32_t(i / (a.columns / 8)), c8 = uint32_t(i % (a.columns / 8));
-        const float* src = reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(a.x) + uint64_t(r) * a.x_stride) + c8 * 8;
-        f16x8 h;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            h[e] = _Float16(src[e]);
-            if ((__builtin_bit_cast(uint16_t, h[e]) & 0x7c00u) == 0x7c00u) bad = TSP_ERRBIT_NONFINITE;
-        }
-        *reinterpret_cast<f16x8*>(a.x16 + uint64_t(r) * a.columns + c8 * 8) = h;
+    for (int e = 0; e < 8; ++e) {
+        h[e] = _Float16(e < 4 ? v0[e % 4] : v1[e % 4]);
+        if ((__builtin_bit_cast(uint16_t, _Float16(h[e])) & 0x7c00u) == 0x7c00u) bad = TSP_ERRBIT_NONFINITE;
     }
+    *reinterpret_cast<f16x8*>(a.x16 + uint64_t(token) * a.columns + c8 * 8) = h;
     publish_error(bad, a.error_word);
 }
 
@@ -326,9 +319,8 @@ extern "C" int tsp_dense_mm_q8_staged(uint32_t layout, const void* matrix, uint6
     }
     _Float16* const w16 = static_cast<_Float16*>(workspace);
     _Float16* const x16 = reinterpret_cast<_Float16*>(static_cast<uint8_t*>(workspace) + align256(uint64_t(rows) * columns * 2));
-    const uint64_t w_groups = (uint64_t(rows) * (columns / 16) + 255) / 256, x_groups = (uint64_t(tokens) * (columns / 8) + 255) / 256;
-    const OperandsArgs o{static_cast<const uint8_t*>(matrix), input, input_stride_bytes, w16, x16, layout, columns, rows, tokens, uint32_t(w_groups), error_word};
-    TSP_LAUNCH("q8_operands_to_f16", s, q8_operands_to_f16<<<uint32_t(w_groups + x_groups), 256, 0, s>>>(o));
+    const OperandsArgs o{static_cast<const uint8_t*>(matrix), input, input_stride_bytes, w16, x16, layout, columns, rows, tokens, error_word};
+    TSP_LAUNCH("q8_operands_to_f16", s, q8_operands_to_f16<<<dim3((rows + tokens + 3) / 4, (columns + 511) / 512), 256, 0, s>>>(o));
     const F16GemmArgs a{x16, w16, output, output_stride_bytes, tokens, rows, columns, error_word};
     const uint64_t f16_tiles = uint64_t((rows + kTile - 1) / kTile) * ((tokens + kTile - 1) / kTile);
     TSP_LAUNCH("f16_gemm_nt", s, f16_gemm_nt<<<uint32_t((f16_tiles + 7) / 8 * 8), 256, 0, s>>>(a));
