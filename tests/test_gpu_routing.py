@@ -551,7 +551,7 @@ def test_router_f32_batch_pieces_far_apart(gpu, synth, weight_exponent, row_expo
     assert np.array_equal(got[others], usual[others])
 
 
-@pytest.mark.parametrize("tokens,selected,experts", [(1, 1, 2), (9, 3, 8), (511, 2, 64), (513, 7, 32), (1025, 16, 16), (1536, 5, 130), (2048, 10, 512), (2048, 15, 512)])
+@pytest.mark.parametrize("tokens,selected,experts", [(1, 1, 2), (9, 3, 8), (511, 2, 64), (512, 16, 512), (513, 7, 32), (1025, 16, 16), (1536, 5, 130), (2048, 10, 512), (2048, 15, 512)])
 def test_grouped_products_prepare_routes_and_lists(gpu, tsp, orc, synth, tokens, selected, experts):
     """The launch that a grouped product starts with: its routes, counts and tasks against the oracle's, either side of the 512 tokens that go in one launch, ids whose
     rows 8 bytes align and ids whose rows they do not; and with ids out of range, or twice in a token, what the entry points of their own make of them."""
