@@ -433,13 +433,14 @@ def test_dense_mm_q8_lanes_half_rows(gpu, tsp, orc, synth, tokens, rows):
 # one wave to ten, just past the sizes that a workgroup per sixteen rows takes; one tile more than whole rounds and a last tile of one row
 @pytest.mark.parametrize("lanes,tokens,cols,rows", [(False, 2, 256, 12001), (False, 9, 512, 6001), (False, 16, 768, 6017), (False, 8, 1024, 16385), (False, 11, 1280, 8193),
                                                     (False, 16, 1536, 6001), (False, 10, 1792, 6016), (False, 5, 2048, 12033), (False, 7, 2304, 16001), (False, 16, 2560, 13003),
-                                                    (True, 11, 2560, 17), (True, 16, 2560, 8193)])
+                                                    (True, 11, 2560, 17), (True, 16, 2560, 8193), (False, 9, 1792, 14016), (False, 16, 768, 14001), (False, 11, 1280, 20003),
+                                                    (False, 13, 256, 24575)])
 def test_dense_mm_q8_resident_rows(gpu, tsp, orc, synth, lanes, tokens, cols, rows):
     """Token rows in registers, a wave per 256 columns, as the floats they are: the bound of the tests above, ten waves' sums one addition each."""
     test_dense_mm_q8_f32_rows(gpu, tsp, orc, synth, lanes, tokens, cols, rows, 0)
 
 
-@pytest.mark.parametrize("tokens,cols,rows", [(2, 256, 24577), (16, 768, 14001), (7, 1280, 24610), (9, 1792, 14016), (16, 2048, 16385)])
+@pytest.mark.parametrize("tokens,cols,rows", [(2, 256, 24577), (16, 768, 24577), (7, 1280, 24610), (9, 1792, 24600), (16, 2048, 16385)])
 def test_dense_mm_q8_resident_halves(gpu, tsp, orc, synth, tokens, cols, rows):
     """The same of large matrices, in two halves under one power of two: the bound and the canaries of the test below."""
     test_dense_mm_q8_odd_rows(gpu, tsp, orc, synth, False, tokens, cols, rows)

@@ -664,8 +664,10 @@ int q8_mfma(const void* matrix, const float* x, float* y, uint32_t columns, uint
     // take: 2560 columns, eight token rows by 64 001 55.7 us with the top-64 behind, 63.3 the other way; sixteen, two passes, 109.7 against 71.7.
     const uint32_t at_once = columns % 512 == 0 ? 2 * kF32Rows : kF32Rows;
     // Up to 2048 columns a small matrix is multiplied by floats in three pieces, at no cost there; two halves, which the large ones take, are 2 to 3 % faster
-    // (eight token rows by 151 936 x 2048 82.9 us with the top-64 behind, 85.3 in three pieces).
-    if (columns <= kHalvesColumns || width > at_once) return q8_resident(false, rows < (width > 8 ? 14000u : 24576u), matrix, x, y, columns, rows, width, error_word, s);
+    // (eight token rows by 151 936 x 2048 82.9 us with the top-64 behind, 85.3 in three pieces). Large: 24 576 rows, 14 000 with nine token rows or more of whole
+    // 512 columns. What is below has never had fewer bits than the floats it is given.
+    const bool floats = rows < (width > 8 && columns % 512 == 0 ? 14000u : 24576u);
+    if (columns <= kHalvesColumns || width > at_once) return q8_resident(false, floats, matrix, x, y, columns, rows, width, error_word, s);
     const Q8MfmaArgs a{static_cast<const uint8_t*>(matrix), x, y, columns, rows, width, error_word};
     // five rows x all columns and ten rows x half the columns stage the same number of bytes
     const uint32_t lds_bytes = 2 * 8 * columns * 2 + kWaves * kTileBytes;
