@@ -7,7 +7,7 @@
 //
 // A Q8_0 block is one 16x16x32 matrix instruction per 16 weight rows and piece of the activations: lane (n, kq) supplies the eight quants 8 kq .. 8 kq + 7 of
 // weight row n, exact bf16 or halves, on the other side are the token rows; the block's scale multiplies the f32 result. F32: each activation as its three bf16 pieces
-// (mfma_quant.hpp: the f32 product, whatever else is in the row); else hi + lo halves under one power of two, 22 significant bits of the largest.
+// (mfma_quant.hpp: the f32 product, whatever else is in the row); else hi + lo halves under a power of two per token row, 22 significant bits of the row's largest.
 //
 // Bound by the matrix's bytes from some 60 000 rows on (151 936 x 2048: 65 us, 5.1 TB/s), below that by the first bytes' trip as well. What it replaced gave a wave all of a tile's
 // columns, so that few tiles were few waves, and nine token rows half of the columns at a time, sums meeting by atomic additions in an output cleared by
@@ -114,7 +114,6 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(W
     __syncthreads();
     float biggest = 0;  // of token row n16
     for (uint32_t w = 0; w < WAVES; ++w) biggest = fmaxf(biggest, largest[w][n16]);
-    if constexpr (!F32) biggest = wave_largest(biggest);  // one scale for all of them
     const int exponent = int((__float_as_uint(biggest) >> 23) & 0xffu) - 127;
     const int shift = F32 ? row_lift(biggest) : !(biggest > 0) || nonfinite(biggest) ? 0 : exponent < -87 ? 100 : 13 - exponent;
     const float scale = power_of_two(shift);
