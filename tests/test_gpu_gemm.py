@@ -790,6 +790,22 @@ def test_grouped_moe_down_rows_in_lds_of_512(gpu, tsp, orc, synth, dn_type):
     test_grouped_moe_down_rows_in_lds_errors(gpu, tsp, synth, dn_type, 512)
 
 
+@pytest.mark.parametrize("dn_type", [8, 7])
+def test_grouped_moe_down_of_512_either_side_of_a_route_an_expert(gpu, tsp, synth, dn_type):
+    """63 routes of 64 experts go to the register-resident kernel, 64 to the one with the rows in LDS: a token's rows are the same bits in either company."""
+    channels, hidden, experts = 1024, 512, 64
+    gate, up = synth.matrix(12, 3121, hidden * experts, channels), synth.matrix(12, 3122, hidden * experts, channels)
+    w = tsp.PlanarMoeWeights(gpu, 12, dn_type, channels, hidden, experts, gate, up, synth.matrix(dn_type, 3123, channels * experts, hidden))
+    ids = np.random.default_rng(17).permutation(experts).astype(np.uint32)
+    x = synth.activations_f32(3124, (experts, channels))
+    rows = []
+    for tokens in (experts - 1, experts):
+        scratch = tsp.GroupedScratch(gpu, tokens, 1, experts, channels, hidden)
+        rows.append(tsp.planar_nax_grouped_moe(gpu, w, gpu.upload(ids[:tokens]), gpu.upload(x[:tokens]), tokens, 1, scratch).cpu().numpy())
+        assert gpu.error() == 0
+    assert np.array_equal(rows[0].view(np.uint32), rows[1][:-1].view(np.uint32))
+
+
 def test_grouped_moe_sticky_errors(gpu, tsp, synth):
     channels, hidden, experts, selected, n = 256, 256, 4, 2, 40
     gate = synth.matrix(12, 3101, hidden * experts, channels)

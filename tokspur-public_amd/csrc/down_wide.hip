@@ -46,6 +46,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     constexpr uint32_t kPitch = kColumns * 2 + 16;  // sixteen lanes reading 16 bytes of sixteen rows touch all banks once
     constexpr uint32_t kStageBytes = KIND == kQ8 ? 4096 : 2048;
     constexpr int kDepth = STEPS == 6 ? 3 : STEPS;  // steps requested ahead
+    constexpr bool kHalves = STEPS == 4;  // two sums of 256 columns, added: the bits of down_resident.hip, which takes the same calls with fewer routes
     constexpr uint32_t kRowAt = kTaskRows * kPitch, kInfoAt = kRowAt + kTaskRows * 4, kStagesAt = kInfoAt + 2 * kInfoSlots * 16;
     __shared__ __attribute__((aligned(16))) uint8_t lds_raw[kStagesAt + kWaves * kStageBytes];
     static_assert(sizeof(lds_raw) <= 160 * 1024, "one workgroup per compute unit");
@@ -133,7 +134,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         for (int s = 0; s < kDepth; ++s) fetch(st[s], s);
         __builtin_amdgcn_sched_barrier(0);
 
-        f32x16 blk[MT];
+        f32x16 blk[MT], first[kHalves ? MT : 1];
 #pragma unroll
         for (int i = 0; i < MT; ++i) blk[i] = f32x16{};
         auto store_tile = [&](uint32_t tile, bool live) {
@@ -158,6 +159,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         auto step = [&](auto s_tag) {
             constexpr int S = decltype(s_tag)::value;
             Stage<KIND>& cur = st[S % kDepth];
+            constexpr bool kFresh = S == 0 || (kHalves && S == STEPS / 2);  // sums begin here
+            if constexpr (kFresh && S > 0)
+#pragma unroll
+                for (int i = 0; i < MT; ++i) first[i] = blk[i];
 #pragma unroll
             for (int i = 0; i < int(kStageBytes / 1024); ++i) *reinterpret_cast<u32x4*>(stage + i * 1024 + lane * 16) = cur.q[i];
             // everything a stage holds is used up before it is requested again: a value carried over would be moved at the end of
@@ -201,9 +206,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                     for (int i = 0; i < MT; ++i) {
                         const f16x8 rows = *reinterpret_cast<const f16x8*>(lds_raw + a_lane + i * 32 * kPitch + S * 256 + b * 64 + ff * 16);
                         const f32x16 zero{};
-                        blk[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(rows, f[ff], S == 0 && b == 0 && ff == 0 ? zero : blk[i], 0, 0, 0);
+                        blk[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(rows, f[ff], kFresh && b == 0 && ff == 0 ? zero : blk[i], 0, 0, 0);
                     }
             }
+            if constexpr (kHalves && S == STEPS - 1)
+#pragma unroll
+                for (int i = 0; i < MT; ++i) blk[i] = first[i] + blk[i];
         };
 
         // ---- a task's rows: requested before the last results of the task before go out, put down when every wave has left that task

@@ -994,7 +994,7 @@ int grouped_moe(const tsp_grouped_moe* m, const tsp_shared_expert* shared, void*
     // Q8_0 and Q5_1 planes of 512 hidden units in such layers: a share of the resident kernel's that changes its task now and then loads registers anew each
     // time, the wide one's next rows travel beside the last products. Kernels alone, 64 experts of 1024 x 512: 762 tokens Q8_0 33.2 -> 23.7 us, Q5_1 33.0 -> 24.6,
     // 2048 41.0 -> 32.4 and 41.4 -> 33.3, 16 11.2 -> 9.8 and 11.4 -> 10.6; below a route an expert 12 tokens 8.4 and 9.4. With many items they are even (512
-    // experts of 2048, a sublayer of 600 tokens 396 and 391 us, of 2048 528 and 540).
+    // experts of 2048, a sublayer of 600 tokens 396 and 391 us, of 2048 528 and 540). A row's bits are the same from either.
     const bool wide_fits = wide_down_takes(down_type, m->channels, m->hidden) && y_span <= 0xffff0000u;
     const bool wide_first = wide_fits && small && routes >= m->experts;
     const bool resident = !brief && !wide_first && resident_down_takes(down_type, m->channels, m->hidden) && uint64_t(routes) * m->y_stride_bytes < (1ull << 32) && shared_span < (1ull << 32);
