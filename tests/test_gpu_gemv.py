@@ -446,8 +446,9 @@ def test_dense_mm_q8_resident_halves(gpu, tsp, orc, synth, tokens, cols, rows):
     test_dense_mm_q8_odd_rows(gpu, tsp, orc, synth, False, tokens, cols, rows)
 
 
-@pytest.mark.parametrize("tokens,cols,rows", [(2, 256, 24577), (16, 768, 24577), (7, 1280, 24610), (9, 1792, 24600), (16, 2048, 16385), (8, 2048, 24600)])
-def test_dense_mm_q8_resident_halves_far_apart(gpu, tsp, orc, synth, tokens, cols, rows):
+@pytest.mark.parametrize("lanes,tokens,cols,rows", [(False, 2, 256, 24577), (False, 16, 768, 24577), (False, 7, 1280, 24610), (False, 9, 1792, 24600), (False, 16, 2048, 16385),
+                                                    (False, 8, 2048, 24600), (True, 5, 512, 1001), (True, 16, 1024, 1000), (True, 8, 1536, 403), (True, 11, 2048, 1001)])
+def test_dense_mm_q8_halves_far_apart(gpu, tsp, orc, synth, lanes, tokens, cols, rows):
     """Token rows in two halves each have a power of two of their own: rows of 1e-20 and 1e4 beside one another keep their bits. Error bound: as above for
     sums, and 22 bits of the row's largest value, or less where a half is subnormal: 2^-22 of each |x| and 2^-37 of the row's largest, in front of sum |w|."""
     w = synth.matrix(8, 2800 + cols, rows, cols)
@@ -456,7 +457,8 @@ def test_dense_mm_q8_resident_halves_far_apart(gpu, tsp, orc, synth, tokens, col
     x[-1] *= np.float32(1e4)
     check = np.unique(np.r_[0:200, rows // 2:rows // 2 + 40, rows - 40:rows])
     dense = orc.dequantize(8, np.ascontiguousarray(w.reshape(rows, -1)[check]).reshape(-1), len(check) * cols).reshape(len(check), cols).astype(np.float64)
-    got = tsp.dense_mm_q8(gpu, tsp.LAYOUT_GGUF, gpu.upload(w), gpu.upload(x), tokens, cols, rows).cpu().numpy()
+    matrix, layout = (tsp.q8_lanes_pack_rows(cols, w), tsp.LAYOUT_Q8_LANES_V1) if lanes else (w, tsp.LAYOUT_GGUF)
+    got = tsp.dense_mm_q8(gpu, layout, gpu.upload(matrix), gpu.upload(x), tokens, cols, rows).cpu().numpy()
     x64 = x.astype(np.float64)
     bound = (2.0 ** -18 + 2.0 ** -22) * (np.abs(x64) @ np.abs(dense).T) + 2.0 ** -37 * np.abs(x64).max(axis=1, keepdims=True) * np.abs(dense).sum(axis=1)
     assert gpu.error() == 0 and (np.abs(got[:, check] - x64 @ dense.T) <= bound).all()

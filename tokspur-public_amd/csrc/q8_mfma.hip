@@ -5,8 +5,8 @@
 // 16x16x32 MFMA step per 16 weight rows: the block's 32 columns are the instruction's whole K, a lane (n, kq) supplies the
 // eight quants 8 kq .. 8 kq + 7 of weight row n, and the sixteen operand rows on the other side are the token rows (eight
 // of them repeated when there are only eight). The block's scale multiplies the f32 result once (4 fused multiply-adds per
-// lane and 16 weight rows). Up to 2048 columns the activations are scaled by a power of two and split into hi + lo halves, staged once in
-// LDS for all of K, so the result carries 22 significant bits of x: this is the f32 GEMV of the engine to within f32
+// lane and 16 weight rows). Up to 2048 columns the activations are scaled by a power of two per token row and split into hi + lo halves, staged once in
+// LDS for all of K, so the result carries 22 significant bits of the row's largest x: this is the f32 GEMV of the engine to within f32
 // accumulation error, at ~1.3 VALU operations per weight byte whatever the number of token rows. Rows of more than 2048
 // columns are staged as the floats they are, three bf16 pieces each (mfma_quant.hpp): fifteen operand rows for up to five
 // token rows, in the same LDS, or for up to ten where a workgroup takes half of the columns.
@@ -89,40 +89,32 @@ __device__ __forceinline__ void request_token_rows(const Q8MfmaArgs& a, uint32_t
     }
 }
 
-// Largest magnitude of the workgroup's rows -> power-of-two scale -> hi + lo halves in LDS, the 16-byte chunks of a row swizzled
-// by the row's index (chunk c of row r sits at c ^ r). Returns the factor that undoes the scale; ends with a barrier.
+// Largest magnitude of each row, as bits in `largest` (zeros before), -> power-of-two scale -> hi + lo halves in LDS, the 16-byte chunks of a row swizzled
+// by the row's index (chunk c of row r sits at c ^ r). Ends with a barrier.
+__device__ __forceinline__ int halves_shift(uint32_t largest) {  // the largest to 2^13; a row that is not finite stays as it is
+    const int up = 13 + 127 - int(largest >> 23);
+    return largest == 0 || largest >= 0x7f800000u ? 0 : up > 100 ? 100 : up;
+}
 template <int kRows>
-__device__ __forceinline__ float stage_token_rows(const float4 (&xv)[kMine][2], uint32_t K, _Float16* a_hi, _Float16* a_lo, float* wave_max,
-                                                  uint32_t& bad) {
-    const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave, chunks = K / 8;
-    float biggest = 0;
+__device__ __forceinline__ void stage_token_rows(const float4 (&xv)[kMine][2], uint32_t K, _Float16* a_hi, _Float16* a_lo, uint32_t* largest, uint32_t& bad) {
+    const uint32_t tid = threadIdx.x, chunks = K / 8;
 #pragma unroll
     for (uint32_t j = 0; j < kMine; ++j) {
+        uint32_t bits = 0;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const float4 v = xv[j][h];
-            if (nonfinite(v.x) || nonfinite(v.y) || nonfinite(v.z) || nonfinite(v.w)) bad = TSP_ERRBIT_NONFINITE;
-            biggest = fmaxf(biggest, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-        }
+        for (int h = 0; h < 2; ++h)
+            for (const float v : {xv[j][h].x, xv[j][h].y, xv[j][h].z, xv[j][h].w}) bits = max(bits, __float_as_uint(v) & 0x7fffffffu);
+        if (bits >= 0x7f800000u) bad = TSP_ERRBIT_NONFINITE;
+        bits = row16_largest_bits(bits);  // sixteen lanes are of one row: a row's chunks are a multiple of sixteen
+        const uint32_t i = tid + j * kThreads;
+        if (tid % 16 == 0 && i < kRows * chunks) atomicMax(&largest[i / chunks], bits);
     }
-    biggest = wave_largest(biggest);
-    if (lane == 0) wave_max[wave] = biggest;
     __syncthreads();
-    biggest = wave_max[0];
-#pragma unroll
-    for (uint32_t w = 1; w < kWaves; ++w) biggest = fmaxf(biggest, wave_max[w]);
-    float scale = 1.0f, inv_scale = 1.0f;
-    if (biggest > 0 && !nonfinite(biggest)) {
-        const int e = int((__float_as_uint(biggest) >> 23) & 0xffu) - 127;
-        int shift = 13 - e;
-        shift = shift > 100 ? 100 : shift < -100 ? -100 : shift;
-        scale = __uint_as_float(uint32_t(127 + shift) << 23);
-        inv_scale = __uint_as_float(uint32_t(127 - shift) << 23);
-    }
 #pragma unroll
     for (uint32_t j = 0; j < kMine; ++j) {
         const uint32_t i = tid + j * kThreads, r = i / chunks, c = i % chunks;
         if (i >= kRows * chunks) break;
+        const float scale = power_of_two(halves_shift(largest[r]));
         const float v[8] = {xv[j][0].x, xv[j][0].y, xv[j][0].z, xv[j][0].w, xv[j][1].x, xv[j][1].y, xv[j][1].z, xv[j][1].w};
         f16x8 hi, lo;  // zeros for the rows past a.m
 #pragma unroll
@@ -136,7 +128,12 @@ __device__ __forceinline__ float stage_token_rows(const float4 (&xv)[kMine][2], 
         *reinterpret_cast<f16x8*>(a_lo + at) = lo;
     }
     __syncthreads();
-    return inv_scale;
+}
+// What undoes the scales of the token rows that a lane's accumulators belong to.
+template <int kRows>
+__device__ __forceinline__ void halves_back(const uint32_t* largest, uint32_t kq, float (&back)[4]) {
+#pragma unroll
+    for (uint32_t v = 0; v < 4; ++v) back[v] = power_of_two(-halves_shift(largest[(4 * kq + v) % kRows]));
 }
 
 // The same for SETS times five rows in f32: xv[j] is row 5 set + j of the thread's set.
@@ -440,6 +437,7 @@ __global__ __launch_bounds__(kThreads, 1) void q8_lanes_mfma_kernel(Q8MfmaArgs a
     constexpr uint32_t KSPLIT = kRows / 8;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // [hi plane][lo plane][8 weight tiles]
     __shared__ float wave_max[kF32Rows][kWaves];
+    __shared__ uint32_t largest[16];
     __shared__ uint32_t next_tile;
 
     const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
@@ -452,6 +450,7 @@ __global__ __launch_bounds__(kThreads, 1) void q8_lanes_mfma_kernel(Q8MfmaArgs a
     const uint32_t sharer = blockIdx.x / KSPLIT, sharers = gridDim.x / KSPLIT;  // the host launches a multiple of KSPLIT
     const uint32_t tiles = (a.rows + kLaneRows - 1) / kLaneRows;
     if (tid == 0) next_tile = 0;
+    if (!F32 && tid < 16) largest[tid] = 0;
     __syncthreads();
     _Float16* const a_hi = reinterpret_cast<_Float16*>(lds);
     _Float16* const a_lo = a_hi + kRows * K;
@@ -506,9 +505,13 @@ __global__ __launch_bounds__(kThreads, 1) void q8_lanes_mfma_kernel(Q8MfmaArgs a
         if constexpr (DEPTH >= 2) fetch_run(t * kLaneRows, 1, std::integral_constant<int, 1 % DEPTH>{});
     }
     __builtin_amdgcn_sched_barrier(0);  // every request above is out before the first wait below
-    float inv_scale = 1.0f, back[SETS][kF32Rows];
-    if constexpr (F32) stage_f32_rows<SETS>(xv, K, reinterpret_cast<__bf16*>(lds), wave_max, back, bad);
-    else inv_scale = stage_token_rows<kRows>(xv, K, a_hi, a_lo, wave_max[0], bad);
+    float back[SETS][F32 ? kF32Rows : 4];
+    if constexpr (F32) {
+        stage_f32_rows<SETS>(xv, K, reinterpret_cast<__bf16*>(lds), wave_max, back, bad);
+    } else {
+        stage_token_rows<kRows>(xv, K, a_hi, a_lo, largest, bad);
+        halves_back<kRows>(largest, kq, back[0]);
+    }
 
     // the activation chunk of block B of run g, columns 8 kq .. 8 kq + 7: chunk g * 64 + B * 4 + kq of row `arow`, kept at
     // chunk ^ arow; arow < kRows flips the three or four low bits, which B % kVariants and kq decide
@@ -637,7 +640,7 @@ __global__ __launch_bounds__(kThreads, 1) void q8_lanes_mfma_kernel(Q8MfmaArgs a
         for (int v = 0; v < 4; ++v) {
             const uint32_t m = 4 * kq + v;  // with eight token rows the lanes with kq >= 2 hold repeats of rows 0 .. 7
             if (m < kRows && m < a.m && r < a.rows) {
-                const float val = acc[0][v] * inv_scale;
+                const float val = acc[0][v] * back[0][v];
                 if (nonfinite(val)) bad = TSP_ERRBIT_NONFINITE;
                 if constexpr (KSPLIT == 1) a.y[uint64_t(m) * a.rows + r] = val;
                 else joined[v] = join(a.y, m * a.rows + r, val);
