@@ -464,6 +464,30 @@ def test_dense_mm_q8_halves_far_apart(gpu, tsp, orc, synth, lanes, tokens, cols,
     assert gpu.error() == 0 and (np.abs(got[:, check] - x64 @ dense.T) <= bound).all()
 
 
+# a wave with whole matrix rows: one group of columns to eight, one item in flight and two, rounds of 2048 tiles with a last one of one row
+@pytest.mark.parametrize("tokens,cols,rows", [(8, 256, 40001), (2, 256, 131073), (3, 1280, 72001), (1, 1280, 100000), (8, 1792, 72033), (6, 1536, 65569), (4, 2048, 65537), (7, 2048, 131105)])
+def test_dense_mm_q8_rows_by_waves(gpu, tsp, orc, synth, tokens, cols, rows):
+    """Some large matrices go to another kernel with up to eight token rows: the bits are those that the rows have in the company of others (twelve, which the
+    other kernel takes), the bound that of the test above, and a value that is not finite is reported and spoils its own token's row alone."""
+    w = synth.matrix(8, 2900 + cols, rows, cols)
+    x = synth.activations_f32(2901 + tokens, (12, cols))
+    x[0] *= np.float32(1e-20)
+    x[tokens - 1, cols // 2:] *= np.float32(1e4)
+    matrix = gpu.upload(w)
+    few = lambda rows_of_x: tsp.dense_mm_q8(gpu, tsp.LAYOUT_GGUF, matrix, gpu.upload(rows_of_x), len(rows_of_x), cols, rows).cpu().numpy()
+    got = few(x[:tokens])
+    assert gpu.error() == 0
+    assert np.array_equal(got.view(np.uint32), few(x)[:tokens].view(np.uint32)) and gpu.error() == 0
+    check = np.unique(np.r_[0:200, rows // 2:rows // 2 + 40, rows - 40:rows])
+    dense = orc.dequantize(8, np.ascontiguousarray(w.reshape(rows, -1)[check]).reshape(-1), len(check) * cols).reshape(len(check), cols).astype(np.float64)
+    x64 = x[:tokens].astype(np.float64)
+    bound = (2.0 ** -18 + 2.0 ** -22) * (np.abs(x64) @ np.abs(dense).T) + 2.0 ** -37 * np.abs(x64).max(axis=1, keepdims=True) * np.abs(dense).sum(axis=1)
+    assert (np.abs(got[:, check] - x64 @ dense.T) <= bound).all()
+    x[tokens - 1, cols - 1] = np.nan
+    spoilt = few(x[:tokens])
+    assert gpu.error() == tsp.ERRBIT_NONFINITE and np.array_equal(spoilt[:-1].view(np.uint32), got[:-1].view(np.uint32))
+
+
 @pytest.mark.parametrize("lanes,tokens,cols,rows", [(False, 9, 512, 14003), (False, 16, 1024, 14002), (False, 7, 2560, 31001), (True, 13, 1024, 37), (True, 16, 2048, 515),
                                                     (True, 9, 2560, 1001)])
 def test_dense_mm_q8_odd_rows(gpu, tsp, orc, synth, lanes, tokens, cols, rows):

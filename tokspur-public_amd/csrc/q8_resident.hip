@@ -11,8 +11,8 @@
 //
 // Bound by the matrix's bytes from some 60 000 rows on (151 936 x 2048: 65 us, 5.1 TB/s), below that by the first bytes' trip as well. What it replaced gave a wave all of a tile's
 // columns, so that few tiles were few waves, and nine token rows half of the columns at a time, sums meeting by atomic additions in an output cleared by
-// a launch of its own. Calls with the top-64 behind, before and now, by 2048 columns: eight token rows x 32 000 34.2 -> 28.9 us, 45 000 36.9 -> 35.1, 64 001 42.5 -> 43.5, 90 000
-// 56.5 -> 54.7; sixteen x 64 001 49.5 -> 45.9, 151 936 94.0 -> 89.0; by 1024, twelve x 64 001 36.0 -> 28.9; by 2560, twelve x 33 000 69 -> 46, 151 936 200 -> 118 (two
+// a launch of its own. Calls with the top-64 behind, before and now, by 2048 columns: eight token rows x 32 000 34.2 -> 28.9 us, 45 000 36.9 -> 35.1, 90 000
+// 56.5 -> 54.7 (64 001 42.5 and 43.5: where it is the slower way such calls stay, rows_by_waves in q8_mfma.hip); sixteen x 64 001 49.5 -> 45.9, 151 936 94.0 -> 89.0; by 1024, twelve x 64 001 36.0 -> 28.9; by 2560, twelve x 33 000 69 -> 46, 151 936 200 -> 118 (two
 // passes before). Without the top-64: nine x 16 000 x 2048 22.6 -> 14.0 (a workgroup per sixteen rows before), eight 16.7 -> 14.1.
 // Of q8_lanes_v1 rows a wave has half of each run, 8 bytes of every 16, so two waves fetch each line: only where it saves a pass.
 #include "q8_resident.hpp"
