@@ -291,10 +291,11 @@ def test_dense_mm_q8_staged_tiles(gpu, tsp, synth, tokens, cols, rows):
 
 @pytest.mark.parametrize("tokens,cols,rows,pad", [(2, 64, 1, 0), (7, 640, 33, 0), (8, 2560, 640, 0), (9, 320, 18, 0), (16, 1088, 47, 12), (5, 2048, 160, 4),
                                                   (23, 2560, 48, 0), (3, 96, 20, 0), (6, 512, 24640, 0), (15, 512, 14020, 0), (11, 1280, 14001, 0),
-                                                  (7, 2560, 24577, 0), (14, 2560, 14004, 0), (27, 1024, 14004, 0), (41, 192, 30, 4)])
+                                                  (7, 2560, 24577, 0), (14, 2560, 14004, 0), (27, 1024, 14004, 0), (41, 192, 30, 4),
+                                                  (18, 768, 6144, 0), (18, 768, 6145, 0), (64, 2048, 7000, 0), (64, 2048, 8200, 0), (8, 1536, 12288, 0), (37, 512, 10300, 0)])
 def test_dense_mm_q8_few_rows(gpu, tsp, orc, synth, tokens, cols, rows, pad):
-    # every kernel that a few raw Q8_0 token rows can go to: 16-row tiles (any multiple of 64 columns, rows any distance apart), up to 2048
-    # columns the persistent kernel from 24 576 rows on (14 000 at nine tokens) with eight and sixteen token rows
+    # every kernel that a few raw Q8_0 token rows can go to: 16-row tiles (any multiple of 64 columns, rows any distance apart), or, up to sixteen at a time,
+    # the persistent ones, from 6000 to 31 000 rows on; either side of where a pass of those and what is left over take the place of the tiles
     w = synth.matrix(8, 2200 + cols, rows, cols)
     x = synth.activations_f32(2201 + tokens, (tokens, cols + pad))
     x[0] *= 1e-20
@@ -306,11 +307,11 @@ def test_dense_mm_q8_few_rows(gpu, tsp, orc, synth, tokens, cols, rows, pad):
     tsp.dense_mm_q8(gpu, tsp.LAYOUT_GGUF, gpu.upload(w), gpu.upload(x), tokens, cols, rows, out=out, x_stride=(cols + pad) * 4, out_stride=(rows + pad) * 4)
     got = out.cpu().numpy()
     # against the sum of |w| |x|: 2^-22 for the two halves of an activation, and a few 2^-24 for each rounding on the way through
-    # 32-column sums and their addition; where eight or sixteen rows share one power-of-two scale, 2^-38 of the largest of them all
+    # 32-column sums and their addition; where halves are subnormal under the row's power of two, 2^-38 of its largest
     blocks = part.reshape(len(check), -1, 34)
     weight = np.abs(blocks[:, :, 2:].view(np.int8).astype(np.float64)) * np.ascontiguousarray(blocks[:, :, :2]).view(np.float16).astype(np.float64)
     weight = weight.reshape(len(check), cols)
-    bound = 2.0 ** -19 * (np.abs(x[:, :cols].astype(np.float64)) @ weight.T) + 2.0 ** -38 * np.abs(x).max() * weight.sum(1)
+    bound = 2.0 ** -19 * (np.abs(x[:, :cols].astype(np.float64)) @ weight.T) + 2.0 ** -38 * np.abs(x).max(axis=1, keepdims=True) * weight.sum(1)
     assert (np.abs(got[:, check] - want) <= bound).all() and (got[:, rows:] == -5.0).all() and gpu.error() == 0
 
 
@@ -431,8 +432,8 @@ def test_dense_mm_q8_lanes_half_rows(gpu, tsp, orc, synth, tokens, rows):
 
 
 # one wave to ten, just past the sizes that a workgroup per sixteen rows takes; one tile more than whole rounds and a last tile of one row
-@pytest.mark.parametrize("lanes,tokens,cols,rows", [(False, 2, 256, 12001), (False, 9, 512, 6001), (False, 16, 768, 6017), (False, 8, 1024, 16385), (False, 11, 1280, 8193),
-                                                    (False, 16, 1536, 6001), (False, 10, 1792, 6016), (False, 5, 2048, 12033), (False, 7, 2304, 16001), (False, 16, 2560, 13003),
+@pytest.mark.parametrize("lanes,tokens,cols,rows", [(False, 2, 256, 12289), (False, 9, 512, 6001), (False, 16, 768, 6017), (False, 8, 1024, 16385), (False, 11, 1280, 8193),
+                                                    (False, 16, 1536, 6001), (False, 10, 1792, 6016), (False, 5, 2048, 12321), (False, 7, 2304, 20481), (False, 16, 2560, 13003),
                                                     (True, 11, 2560, 17), (True, 16, 2560, 8193), (False, 9, 1792, 14016), (False, 16, 768, 14001), (False, 11, 1280, 20003),
                                                     (False, 13, 256, 24575)])
 def test_dense_mm_q8_resident_rows(gpu, tsp, orc, synth, lanes, tokens, cols, rows):

@@ -170,19 +170,30 @@ int launch(uint32_t layout, const Q8Args& a, hipStream_t stream) {
     return launch_status("q8_blocks");
 }
 
-// Two to sixteen token rows against raw rows: a workgroup per 16 matrix rows (q8_small.hip), or a persistent kernel (q8_resident.hip; q8_mfma.hip for up to
-// ten token rows of more than 2048 columns). The latter starts slowly, with five to ten microseconds whatever the rows, the former's time is
-// proportional to them, and to the token rows beyond eight. Small, then persistent, us a call: eight token rows 8000 x 2048 9.0 and 9.2, 12 000 12.8 and
-// 12.7, 16 000 16.7 and 14.1; 12 000 x 1024 9.1 and 8.7, x 256 5.7 and 5.6; nine 4000 x 2048 6.9 and 9.0, 6000 11.8 and 8.9, 16 000 22.6 and 14.0; 6000 x
-// 512 6.0 and 5.3, x 256 5.0 and 5.2. Of more than 2048 columns up to ten token rows (five where columns are no two halves) 27 and 35 at 24 576 x 2560, 37
-// and 36 at 32 000; more, all in registers, sixteen 12 000 x 2560 21.8 and 23.5, 16 000 28.2 and 24.8.
+// Two and more token rows against raw rows: workgroups of 16 matrix rows and 16 token rows (q8_small.hip), all in one launch, or up to sixteen at a time a persistent
+// kernel (q8_resident.hip; q8_mfma.hip for up to ten token rows of more than 2048 columns). The latter starts slowly, with five to ten microseconds whatever the
+// rows; the former goes up by a step for every 4096 matrix rows, with nine to sixteen token rows a larger one, as many workgroups as there are compute units. us a call,
+// small and persistent:
+//   up to eight token rows: on either side of three steps. Eight by 12 001 x 2048 12.8 and 13.4, 13 000 16.3 and 13.6; x 1280 10.0 and 11.7, 12.5 and 11.9; x 256 7.5 and 7.5.
+//   nine to sixteen: nine by 6001 x 2048 11.9 and 10.3, 9000 17.0 and 13.3; sixteen by 7000 x 1792 11.1 and 11.4, 9000 15.8 and 13.9; 6001 x 512 7.5 and 7.6.
+//   more: passes of the persistent kernel against steps. A step and a half for each sixteen token rows where a pass of few is left over (18 by 6001 x 1536 14.3 and
+//   17.6, 6700 18.4 and 17.8), else two and a half (64 by 10 200 x 768 33.8 and 39.1, 12 200 39.7 and 39.2; 200 by 10 200 x 1792 166 and 168), less than two at 2048 columns (40 by
+//   6700 28.5 and 31.6, 7400 33.3 and 31.8; 200 by 7400 130 and 142, 10 200 182 and 174), two and a half or three up to 512 (24 by 10 200 x 512 13.9 and 15.2, 12 200 16.5 and 16.0; 200 98 and 108, 13 900 112 and 108).
+//   more than 2048 columns: up to ten token rows (five where columns are no two halves) 27 and 35 at 24 576 x 2560, 37 and 36 at 32 000; more, all in
+//   registers, eight by 20 000 x 2304 24.1 and 25.2, 22 000 29.2 and 26.4; sixteen by 12 000 x 2560 21.8 and 23.5, 16 000 28.2 and 24.8.
 // Widths that the persistent kernels refuse all go to the former.
 bool small_rows(const void* matrix, const float* x, uint64_t x_stride_bytes, uint32_t columns, uint32_t rows, uint32_t tokens) {
     if (!q8_small_takes(matrix, x, x_stride_bytes, columns, rows)) return false;
     if (x_stride_bytes != uint64_t(columns) * 4 || !q8_mfma_supported(matrix, x, columns, rows)) return true;
-    if (columns <= 2048) return rows < (tokens > 8 ? 6000u : 12000u);
-    if (tokens > (columns % 512 == 0 ? 10u : 5u)) return rows < (tokens > 8 ? 13000u : 16000u);
-    return rows < (tokens > 8 ? 22000u : 31000u);
+    if (columns > 2048) {
+        if (tokens > (columns % 512 == 0 ? 10u : 5u)) return tokens > 8 ? rows < 13000 : rows <= 20480;
+        return rows < (tokens > 8 ? 22000u : 31000u);
+    }
+    if (tokens <= 8) return rows <= 12288;
+    if (tokens <= 16 || rows < 6000) return rows < 6000;
+    const uint32_t tiles = (tokens + 15) / 16, steps = ((rows + 15) / 16 * tiles + 255) / 256;
+    const uint32_t halves = columns <= 512 ? (tiles > 2 ? 6 : 5) : tokens <= 24 ? 3 : columns <= 1792 ? 5 : 4;  // of a step, for a tile
+    return 2 * steps + (columns > 1792 ? 1 : 0) <= halves * tiles;
 }
 
 }  // namespace
@@ -245,7 +256,7 @@ extern "C" int tsp_dense_mm_q8(uint32_t layout, const void* matrix, uint64_t mat
         float* const to = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(output) + uint64_t(done) * output_stride_bytes);
         const auto s = static_cast<hipStream_t>(stream);
         const uint32_t most = left < 16 ? left : 16;
-        if (left > 1 && whole && raw && small_rows(matrix, input, input_stride_bytes, columns, rows, sixteen || !eight ? most : 8)) {
+        if (left > 1 && whole && raw && small_rows(matrix, input, input_stride_bytes, columns, rows, left)) {
             return q8_small(matrix, from, input_stride_bytes, to, output_stride_bytes, columns, rows, left, error_word, s);  // all that is left
         }
         if (eight && left > 1) {
