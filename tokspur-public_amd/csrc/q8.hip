@@ -212,9 +212,8 @@ extern "C" int tsp_q8_matvec_many(uint32_t layout, const void* matrix, uint64_t 
     const auto s = static_cast<hipStream_t>(stream);
     if (layout == TSP_LAYOUT_GGUF && width > 1 && small_rows(matrix, x, uint64_t(columns) * 4, columns, rows, width))
         return q8_small(matrix, x, uint64_t(columns) * 4, y, uint64_t(rows) * 4, columns, rows, width, error_word, s);
-    // One row against a matrix of less than 100 MB, or of a width the persistent matrix-core kernel does not take: that kernel's
-    // eight waves per compute unit share out 32-row tiles, of which there are too few (at 4096 x 2048 20.3 us, 4.4 here; at
-    // 60 000 x 2048, 130 MB, 32.2 and 33.6)
+    // One row against a matrix of less than 100 MB, or of a width the persistent matrix-core kernels do not take: those start slowly, and this one by and by has too few
+    // bytes on their way (46 000 x 2048, 100 MB, 27.5 us here and 25.8 there; 92 000 x 1024 25.8 and 24.3; 36 770 x 2560 26.9 and 37.7)
     if (layout == TSP_LAYOUT_GGUF && width == 1 && (matrix_bytes < 100000000 || !q8_mfma_supported(matrix, x, columns, rows))) {
         bool taken = false;
         const int rc = gemv_q8_row(matrix, x, y, columns, rows, error_word, s, &taken);

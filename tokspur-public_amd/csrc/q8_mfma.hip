@@ -691,14 +691,15 @@ namespace tsp {
 //   33.4, x 1536 30.7 and 32.5; one 34.8 and 40.5. With an odd number of token rows this kernel is some 3 us slower in the first range (five by 68 000
 //   x 2048 37.0 and 38.5): why is not known.
 //   1280 and 1792: five and seven waves there, one such workgroup a compute unit, are too few bytes on their way: eight by 64 000 x 1792 33.1 and 32.9,
-//   72 000 37.0 and 34.9, 128 000 58.8 and 52.4, x 1280 44.3 and 39.4; two by 72 000 x 1280 27.0 and 29.1, 88 000 31.2 and 30.2.
-//   256: a workgroup of one wave there: eight by 32 000 7.7 and 7.7, 48 000 8.7 and 7.7, 151 936 14.0 and 12.3; one 9.4 and 9.3.
+//   72 000 37.0 and 34.9, 128 000 58.8 and 52.4, x 1280 44.3 and 39.4; two by 72 000 x 1280 27.0 and 29.1, 88 000 31.2 and 30.2; one by 52 530 x 1792 (fewer
+//   are gemv.hip's) 28.6 and 25.7, 72 000 34.6 and 37.7.
+//   256: a workgroup of one wave there: eight by 32 000 7.7 and 7.7, 48 000 8.7 and 7.7, 151 936 14.0 and 12.3; one by 367 650 24.9 and 23.7.
 //   512 to 1024: never slower there by more than half a microsecond (eight by 64 001 x 1024 20.0 and 19.8, 100 000 26.7 and 31.1).
 static bool rows_by_waves(uint32_t columns, uint32_t rows, uint32_t width) {
     if (width > 8) return false;
     switch (columns / 256) {
-    case 1: return width > 1 && rows >= 40000;
-    case 5: case 7: return rows >= (width > 2 ? 72000u : 90000u);
+    case 1: return rows >= 40000;
+    case 5: case 7: return rows >= (width > 2 ? 72000u : 90000u) || (width == 1 && rows < 66000);
     case 6: case 8: return width >= 4 && (rows >= 116000 || (rows >= 52000 && rows < 84000 && width % 2 == 0 && (width > 4 || columns == 2048)));
     default: return false;
     }
