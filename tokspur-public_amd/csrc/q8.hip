@@ -241,14 +241,14 @@ extern "C" int tsp_dense_mm_q8(uint32_t layout, const void* matrix, uint64_t mat
     const uint64_t out_span = uint64_t(tokens - 1) * output_stride_bytes + uint64_t(rows) * 4;
     TSP_REQUIRE(!ranges_overlap(output, out_span, matrix, matrix_bytes) && !ranges_overlap(output, out_span, input, in_span),
                 "dense Q8_0 GEMM output overlaps an input");
-    // Eight token rows, up to sixteen where a kernel takes them, go through a matrix-core kernel in one pass over the weights;
+    // Sixteen token rows, of some q8_lanes_v1 matrices eight, go through a matrix-core kernel in one pass over the weights;
     // where none does and the rows lie back to back they go eight, four, two, one at a time (the width sequence of
     // src/q8_many.cpp:20-29), and one by one where there is padding between them.
     const bool packed = input_stride_bytes == uint64_t(columns) * 4 && output_stride_bytes == uint64_t(rows) * 4;
     const bool whole = matrix && error_word && columns && columns % 32 == 0 && rows && rows <= 1000000 && uint64_t(columns / 32) * rows * 34 == matrix_bytes;
     const bool lanes = layout == TSP_LAYOUT_Q8_LANES_V1, raw = layout == TSP_LAYOUT_GGUF;
     const bool eight = whole && packed && (raw ? q8_mfma_supported(matrix, input, columns, rows) : lanes && q8_lanes_mfma_supported(matrix, input, columns, rows));
-    const bool sixteen = eight && (raw ? q8_mfma_supported_16(matrix, input, columns, rows) : q8_lanes_mfma_supported_16(matrix, input, columns, rows));
+    const bool sixteen = eight && (raw || q8_lanes_mfma_supported_16(matrix, input, columns, rows));
     for (uint32_t done = 0; done < tokens;) {
         const uint32_t left = tokens - done;
         const float* const from = reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(input) + uint64_t(done) * input_stride_bytes);

@@ -710,8 +710,6 @@ bool q8_mfma_supported(const void* matrix, const float* x, uint32_t columns, uin
            reinterpret_cast<uintptr_t>(x) % 16 == 0;
 }
 
-bool q8_mfma_supported_16(const void* matrix, const float* x, uint32_t columns, uint32_t rows) { return q8_mfma_supported(matrix, x, columns, rows); }
-
 int q8_mfma(const void* matrix, const float* x, float* y, uint32_t columns, uint32_t rows, uint32_t width, uint32_t* error_word, hipStream_t s) {
     // Up to ten token rows of 2560 columns (five where the columns are no two halves) are one pass here, with fewer matrix instructions than pieces by themselves
     // take: 2560 columns, eight token rows by 64 001 55.7 us with the top-64 behind, 63.3 the other way; sixteen, two passes, 109.7 against 71.7.
