@@ -657,15 +657,15 @@ def test_grouped_moe_exact_when_products_fit_half(gpu, tsp, orc, synth):
                                                              (13, 8, 2048, 512), (12, 7, 256, 512), (8, 7, 768, 512),
                                                              (12, 7, 2048, 160), (12, 8, 2048, 96),
                                                              (12, 8, 2560, 640), (12, 7, 2560, 640), (13, 8, 2560, 640), (8, 7, 2560, 640)])
-def test_grouped_moe_other_planar_kinds(gpu, tsp, orc, synth, gu_type, dn_type, channels, hidden):
+def test_grouped_moe_other_planar_kinds(gpu, tsp, orc, synth, gu_type, dn_type, channels, hidden, experts=6):
     """The planar kinds of include/tokspur/moe.hpp:27-29 beside Q4_K gate/up and Q6_K down (Q5_K / Q8_0 gate and up, Q5_1 / Q8_0
     down) run on the matrix cores as well, their weights decoded to halves on the fly; any gate/up kind combines with any down
-    kind (experts of 512 hidden units with Q8_0 planes down take the kernel that keeps a task's h rows in registers). Same
-    token_map / counts / tasks; expert_down rows against the reference with the declared staging: activations as
+    kind (of experts of 512 hidden units the ones with 384 channels take the kernel that keeps a task's h rows in registers, the others, few and small, the one
+    with the rows in LDS). Same token_map / counts / tasks; expert_down rows against the reference with the declared staging: activations as
     bf16 values, h as 256 * half(h / 256), weights of the staged kinds rounded to half (Q4_K / Q6_K keep their integer factors).
     The last four shapes are the engine's own expert, 2560 channels and 640 hidden units (native/src/moe_mm_many_plan.cpp:7,31),
     with each of its gate/up and down kinds."""
-    experts, selected, n = 6, 3, 75  # an expert with more than 64 routes, one with more than 32, ragged tails
+    selected, n = 3, 75  # of six, an expert with more than 64 routes, one with more than 32, ragged tails
     gate = synth.matrix(gu_type, 3301, hidden * experts, channels)
     up = synth.matrix(gu_type, 3302, hidden * experts, channels)
     down = synth.matrix(dn_type, 3303, channels * experts, hidden)
@@ -749,12 +749,12 @@ def test_grouped_moe_down_rows_in_lds(gpu, tsp, orc, synth, dn_type, channels, h
 
 
 @pytest.mark.parametrize("dn_type,hidden", [(8, 640), (7, 384)])
-def test_grouped_moe_down_rows_in_lds_errors(gpu, tsp, synth, dn_type, hidden):
+def test_grouped_moe_down_rows_in_lds_errors(gpu, tsp, synth, dn_type, hidden, gu_type=12, channels=768):
     """The same kernel: an infinite scale in one block of the weights spoils that channel of that expert's routes and nothing else;
     values that are not finite and expert ids out of range are reported, and the next batch is clean."""
-    channels, experts, selected, n = 768, 4, 2, 90
-    gate, up = synth.matrix(12, 3111, hidden * experts, channels), synth.matrix(12, 3112, hidden * experts, channels)
-    w = tsp.PlanarMoeWeights(gpu, 12, dn_type, channels, hidden, experts, gate, up, synth.matrix(dn_type, 3113, channels * experts, hidden))
+    experts, selected, n = 4, 2, 90
+    gate, up = synth.matrix(gu_type, 3111, hidden * experts, channels), synth.matrix(gu_type, 3112, hidden * experts, channels)
+    w = tsp.PlanarMoeWeights(gpu, gu_type, dn_type, channels, hidden, experts, gate, up, synth.matrix(dn_type, 3113, channels * experts, hidden))
     scratch = tsp.GroupedScratch(gpu, n, selected, experts, channels, hidden)
     x = (synth.activations_f32(3114, (n, channels)) * 0.1).astype(np.float32)
     ids = np.array([[0 if t < 70 else 3, 1 + t % 2] for t in range(n)], dtype=np.uint32).reshape(-1)
@@ -788,6 +788,15 @@ def test_grouped_moe_down_rows_in_lds_of_512(gpu, tsp, orc, synth, dn_type):
     """Four steps, from one route an expert on where the register-resident kernel has the width otherwise: results and reports."""
     test_grouped_moe_other_planar_kinds(gpu, tsp, orc, synth, 12, dn_type, 512, 512)
     test_grouped_moe_down_rows_in_lds_errors(gpu, tsp, synth, dn_type, 512)
+
+
+# the register-resident kernel: channels that are no multiple of 256, fewer routes than experts, and a layer of many items
+@pytest.mark.parametrize("gu_type,channels,experts", [(8, 384, 6), (8, 640, 6), (12, 512, 256), (12, 2048, 128)])
+@pytest.mark.parametrize("dn_type", [8, 7])
+def test_grouped_moe_down_of_512_in_registers(gpu, tsp, orc, synth, gu_type, dn_type, channels, experts):
+    test_grouped_moe_other_planar_kinds(gpu, tsp, orc, synth, gu_type, dn_type, channels, 512, experts)
+    if channels % 256:
+        test_grouped_moe_down_rows_in_lds_errors(gpu, tsp, synth, dn_type, 512, gu_type, channels)
 
 
 @pytest.mark.parametrize("dn_type", [8, 7])

@@ -409,7 +409,7 @@ def test_dense_mm_q8_f32_rows(gpu, tsp, orc, synth, lanes, tokens, cols, rows, p
     x[:, 5:cols:32] = np.resize(np.array([3e4, -1e12, 1e30], dtype=np.float32), (tokens, cols // 32))
     x[0] *= np.float32(1e-37) if tokens > 1 else np.float32(1)
     matrix = tsp.q8_lanes_pack_rows(cols, w) if lanes else w
-    check = np.unique(np.r_[0:min(rows, 300), max(0, rows - 40):rows])
+    check = np.unique(np.r_[0:min(rows, 300), np.linspace(0, rows - 1, 500).astype(int), max(0, rows - 40):rows])
     dense = orc.dequantize(8, np.ascontiguousarray(w.reshape(rows, -1)[check]).reshape(-1), len(check) * cols).reshape(len(check), cols).astype(np.float64)
     out = gpu.full((tokens, rows + pad), -5.0)
     tsp.dense_mm_q8(gpu, tsp.LAYOUT_Q8_LANES_V1 if lanes else tsp.LAYOUT_GGUF, gpu.upload(matrix), gpu.upload(x), tokens, cols, rows, out=out,
@@ -426,12 +426,13 @@ def test_dense_mm_q8_f32_rows(gpu, tsp, orc, synth, lanes, tokens, cols, rows, p
 
 @pytest.mark.parametrize("tokens,rows", [(6, 20), (7, 1002), (10, 1008), (11, 16), (15, 4112)])
 def test_dense_mm_q8_lanes_half_rows(gpu, tsp, orc, synth, tokens, rows):
-    """Six to ten rows of 2560 columns in one pass, two workgroups to a row with its middle run shared, a last tile of four rows, a number
-    of rows that the cleared output does not take (five at a time), two passes of eight. The bound of the test above: one more addition."""
+    """Six to ten rows of 2560 columns, two workgroups to a matrix row with its middle run shared, a last tile of four rows, an output whose length is no
+    multiple of four; more than ten, ten waves to a matrix row. The bound of the test above: one more addition."""
     test_dense_mm_q8_f32_rows(gpu, tsp, orc, synth, True, tokens, 2560, rows, 0)
 
 
-# one wave to ten, just past the sizes that a workgroup per sixteen rows takes; one tile more than whole rounds and a last tile of one row
+# one wave to ten, just past the sizes that a workgroup per sixteen rows takes and up to the last of floats; from five waves on some workgroups have a second
+# tile or more, and most last tiles are of one row or a few (rounds of tiles: test_dense_mm_q8_resident_rounds)
 @pytest.mark.parametrize("lanes,tokens,cols,rows", [(False, 2, 256, 12289), (False, 9, 512, 6001), (False, 16, 768, 6017), (False, 8, 1024, 16385), (False, 11, 1280, 8193),
                                                     (False, 16, 1536, 6001), (False, 10, 1792, 6016), (False, 5, 2048, 12321), (False, 7, 2304, 20481), (False, 16, 2560, 13003),
                                                     (True, 11, 2560, 17), (True, 16, 2560, 8193), (False, 9, 1792, 14016), (False, 16, 768, 14001), (False, 11, 1280, 20003),
@@ -456,13 +457,26 @@ def test_dense_mm_q8_halves_far_apart(gpu, tsp, orc, synth, lanes, tokens, cols,
     x = synth.activations_f32(2801 + tokens, (tokens, cols))
     x[0] *= np.float32(1e-20)
     x[-1] *= np.float32(1e4)
-    check = np.unique(np.r_[0:200, rows // 2:rows // 2 + 40, rows - 40:rows])
+    check = np.unique(np.r_[0:200, np.linspace(0, rows - 1, 500).astype(int), rows // 2:rows // 2 + 40, rows - 40:rows])
     dense = orc.dequantize(8, np.ascontiguousarray(w.reshape(rows, -1)[check]).reshape(-1), len(check) * cols).reshape(len(check), cols).astype(np.float64)
     matrix, layout = (tsp.q8_lanes_pack_rows(cols, w), tsp.LAYOUT_Q8_LANES_V1) if lanes else (w, tsp.LAYOUT_GGUF)
     got = tsp.dense_mm_q8(gpu, layout, gpu.upload(matrix), gpu.upload(x), tokens, cols, rows).cpu().numpy()
     x64 = x.astype(np.float64)
     bound = (2.0 ** -18 + 2.0 ** -22) * (np.abs(x64) @ np.abs(dense).T) + 2.0 ** -37 * np.abs(x64).max(axis=1, keepdims=True) * np.abs(dense).sum(axis=1)
     assert gpu.error() == 0 and (np.abs(got[:, check] - x64 @ dense.T) <= bound).all()
+
+
+# Token rows in registers, tile after tile: the sums have two places in turn, and the first is written again in a workgroup's third round (two tiles a round; one from
+# nine waves on). Rounds of 131 072 matrix rows with one wave, 65 536 with two, 32 768 with three and four, 16 384 with five to eight, 8192 with nine and ten:
+# into the second and into the third of each, the last round whole, of one tile, of one row, and with one tile of two
+@pytest.mark.parametrize("lanes,tokens,cols,rows", [(False, 16, 256, 140001), (False, 9, 256, 270001), (False, 12, 512, 70001), (False, 9, 512, 131073), (False, 16, 768, 65600), (False, 8, 1024, 65600),
+                                                    (False, 16, 1024, 100001), (False, 13, 1280, 40960), (False, 16, 1536, 32769), (False, 9, 1792, 41001), (False, 7, 2048, 49152),
+                                                    (False, 16, 2048, 33001), (False, 7, 2304, 24576), (False, 12, 2560, 16417), (True, 12, 2560, 16417), (True, 16, 2560, 40001)])
+def test_dense_mm_q8_resident_rounds(gpu, tsp, orc, synth, lanes, tokens, cols, rows):
+    if cols > 2048:  # floats
+        test_dense_mm_q8_f32_rows(gpu, tsp, orc, synth, lanes, tokens, cols, rows, 0)
+    else:
+        test_dense_mm_q8_halves_far_apart(gpu, tsp, orc, synth, lanes, tokens, cols, rows)
 
 
 # a wave with whole matrix rows: one group of columns to eight, one item in flight and two, rounds of 2048 tiles with a last one of one row
@@ -490,10 +504,11 @@ def test_dense_mm_q8_rows_by_waves(gpu, tsp, orc, synth, tokens, cols, rows):
 
 
 @pytest.mark.parametrize("lanes,tokens,cols,rows", [(False, 9, 512, 14003), (False, 16, 1024, 14002), (False, 7, 2560, 31001), (True, 13, 1024, 37), (True, 16, 2048, 515),
-                                                    (True, 9, 2560, 1001)])
+                                                    (True, 9, 2560, 1001), (False, 6, 2560, 33003), (False, 10, 2560, 22001)])
 def test_dense_mm_q8_odd_rows(gpu, tsp, orc, synth, lanes, tokens, cols, rows):
-    """Two workgroups to a matrix row whose sums meet in an output that starts on any float and whose rows end on any: all of it is cleared
-    and nothing around it. Rows of two halves keep 22 bits of their largest value, and f32 sums 2^-18 of sum |w x|."""
+    """An output that starts on any float and whose rows end on any: all of it is written and nothing around it, also where two workgroups to a matrix row add into
+    one that was cleared before (2560 columns with six to ten token rows, q8_lanes_v1 rows with nine and more). Rows of two halves keep 22 bits of their
+    largest value, and f32 sums 2^-18 of sum |w x|."""
     w = synth.matrix(8, 2700 + cols, rows, cols)
     x = synth.activations_f32(2701 + tokens, (tokens, cols))
     matrix = tsp.q8_lanes_pack_rows(cols, w) if lanes else w
@@ -513,10 +528,11 @@ def test_dense_mm_q8_odd_rows(gpu, tsp, orc, synth, lanes, tokens, cols, rows):
 
 
 @pytest.mark.parametrize("lanes,tokens,cols,rows", [(False, 9, 1024, 14003), (False, 16, 2048, 24576), (False, 10, 2560, 40001), (True, 13, 1024, 37), (True, 16, 2048, 512),
-                                                    (True, 7, 2560, 1001), (True, 12, 2560, 64)])
+                                                    (True, 7, 2560, 1001), (True, 12, 2560, 64), (False, 6, 2560, 31003), (False, 9, 2560, 22001)])
 def test_dense_mm_q8_sums_that_overflow_at_the_join(gpu, tsp, lanes, tokens, cols, rows):
-    """Two workgroups to a matrix row, either half of whose sum is finite: a sum that passes the largest float is reported, wherever in the matrix
-    it is, and halves of which one is nearly as large and the other takes it back are not."""
+    """Two workgroups to a matrix row (2560 columns with six to ten token rows, q8_lanes_v1 rows of up to 2048 with nine and more) or, the others, two waves to it, either
+    half of whose sum is finite: a sum that passes the largest float is reported, wherever in the matrix it is, and halves of which one is nearly as
+    large and the other takes it back are not."""
     blocks = np.zeros((rows, cols // 32, 34), dtype=np.uint8)
     blocks[:, :, 0:2] = np.array([4096.0], dtype=np.float16).view(np.uint8)
     blocks[:, 0, 2] = 1      # the first column and the last one
