@@ -292,7 +292,8 @@ def test_dense_mm_q8_staged_tiles(gpu, tsp, synth, tokens, cols, rows):
 @pytest.mark.parametrize("tokens,cols,rows,pad", [(2, 64, 1, 0), (7, 640, 33, 0), (8, 2560, 640, 0), (9, 320, 18, 0), (16, 1088, 47, 12), (5, 2048, 160, 4),
                                                   (23, 2560, 48, 0), (3, 96, 20, 0), (6, 512, 24640, 0), (15, 512, 14020, 0), (11, 1280, 14001, 0),
                                                   (7, 2560, 24577, 0), (14, 2560, 14004, 0), (27, 1024, 14004, 0), (41, 192, 30, 4),
-                                                  (18, 768, 6144, 0), (18, 768, 6145, 0), (64, 2048, 7000, 0), (64, 2048, 8200, 0), (8, 1536, 12288, 0), (37, 512, 10300, 0)])
+                                                  (18, 768, 6144, 0), (18, 768, 6145, 0), (64, 2048, 7000, 0), (64, 2048, 8200, 0), (8, 1536, 12288, 0), (37, 512, 10300, 0),
+                                                  (18, 768, 12288, 0), (18, 768, 12289, 0), (64, 2048, 7200, 0), (64, 2048, 9217, 0), (40, 1280, 11400, 0), (33, 2304, 17000, 0)])
 def test_dense_mm_q8_few_rows(gpu, tsp, orc, synth, tokens, cols, rows, pad):
     # every kernel that a few raw Q8_0 token rows can go to: 16-row tiles (any multiple of 64 columns, rows any distance apart), or, up to sixteen at a time,
     # the persistent ones, from 6000 to 31 000 rows on; either side of where a pass of those and what is left over take the place of the tiles
@@ -470,7 +471,7 @@ def test_dense_mm_q8_halves_far_apart(gpu, tsp, orc, synth, lanes, tokens, cols,
 # nine waves on). Rounds of 131 072 matrix rows with one wave, 65 536 with two, 32 768 with three and four, 16 384 with five to eight, 8192 with nine and ten:
 # into the second and into the third of each, the last round whole, of one tile, of one row, and with one tile of two
 @pytest.mark.parametrize("lanes,tokens,cols,rows", [(False, 16, 256, 140001), (False, 9, 256, 270001), (False, 12, 512, 70001), (False, 9, 512, 131073), (False, 16, 768, 65600), (False, 8, 1024, 65600),
-                                                    (False, 16, 1024, 100001), (False, 13, 1280, 40960), (False, 16, 1536, 32769), (False, 9, 1792, 41001), (False, 7, 2048, 49152),
+                                                    (False, 16, 1024, 100001), (False, 13, 1280, 40960), (False, 16, 1536, 32769), (False, 9, 1792, 41001), (False, 11, 2048, 49152),
                                                     (False, 16, 2048, 33001), (False, 7, 2304, 24576), (False, 12, 2560, 16417), (True, 12, 2560, 16417), (True, 16, 2560, 40001)])
 def test_dense_mm_q8_resident_rounds(gpu, tsp, orc, synth, lanes, tokens, cols, rows):
     if cols > 2048:  # floats
@@ -480,7 +481,8 @@ def test_dense_mm_q8_resident_rounds(gpu, tsp, orc, synth, lanes, tokens, cols, 
 
 
 # a wave with whole matrix rows: one group of columns to eight, one item in flight and two, rounds of 2048 tiles with a last one of one row
-@pytest.mark.parametrize("tokens,cols,rows", [(8, 256, 40001), (2, 256, 131073), (3, 1280, 72001), (1, 1280, 100000), (1, 1792, 52600), (8, 1792, 72033), (6, 1536, 65569), (4, 2048, 65537), (7, 2048, 131105)])
+@pytest.mark.parametrize("tokens,cols,rows", [(8, 256, 40001), (2, 256, 131073), (3, 1280, 72001), (1, 1280, 100000), (1, 1792, 52600), (8, 1792, 72033), (6, 1536, 65569), (4, 2048, 65537), (7, 2048, 131105),
+                                              (8, 512, 65569), (8, 1024, 57345), (3, 2048, 57377), (2, 2048, 155649), (1, 1536, 204801)])
 def test_dense_mm_q8_rows_by_waves(gpu, tsp, orc, synth, tokens, cols, rows):
     """Some large matrices go to another kernel with up to eight token rows: the bits are those that the rows have in the company of others (twelve, which the
     other kernel takes), the bound that of the test above, and a value that is not finite is reported and spoils its own token's row alone."""

@@ -176,24 +176,26 @@ int launch(uint32_t layout, const Q8Args& a, hipStream_t stream) {
 // small and persistent:
 //   up to eight token rows: on either side of three steps. Eight by 12 001 x 2048 12.8 and 13.4, 13 000 16.3 and 13.6; x 1280 10.0 and 11.7, 12.5 and 11.9; x 256 7.5 and 7.5.
 //   nine to sixteen: nine by 6001 x 2048 11.9 and 10.3, 9000 17.0 and 13.3; sixteen by 7000 x 1792 11.1 and 11.4, 9000 15.8 and 13.9; 6001 x 512 7.5 and 7.6.
-//   more: passes of the persistent kernel against steps. A step and a half for each sixteen token rows where a pass of few is left over (18 by 6001 x 1536 14.3 and
-//   17.6, 6700 18.4 and 17.8), else two and a half (64 by 10 200 x 768 33.8 and 39.1, 12 200 39.7 and 39.2; 200 by 10 200 x 1792 166 and 168), less than two at 2048 columns (40 by
-//   6700 28.5 and 31.6, 7400 33.3 and 31.8; 200 by 7400 130 and 142, 10 200 182 and 174), two and a half or three up to 512 (24 by 10 200 x 512 13.9 and 15.2, 12 200 16.5 and 16.0; 200 98 and 108, 13 900 112 and 108).
+//   more: passes of the persistent kernel, each of which goes up with every 8192 matrix rows, against all steps together. 64 by 8100 x 1536 37.4 and 40.6, 9400 45.6 and 49.5, 11 350 54.4
+//   and 50.3; 200 by 8100 113.0 and 129.8, 11 350 158.2 and 158.5, 12 650 175.5 and 159.3. At 2048 columns passes are cheaper (32 by 6150 23.4 and 22.9; 200 by 7450 131.3 and 144.8,
+//   8100 142.5 and 145.1, 9400 163.5 and 174.6, 11 350 199.2 and 177.3), up to 768 dearer (64 by 11 350 x 512 30.4 and 32.8, 200 by 12 500 97.8 and 105.7, 13 950 106.7 and 105.8), above
+//   2048 dearer still (64 by 9400 x 2560 66.5 and 89.9, 13 900 91.2 and 95.4, 17 850 119.8 and 114.9; 32 by 12 500 47.3 and 51.8).
 //   more than 2048 columns: up to ten token rows (five where columns are no two halves) 27 and 35 at 24 576 x 2560, 37 and 36 at 32 000; more, all in
 //   registers, eight by 20 000 x 2304 24.1 and 25.2, 22 000 29.2 and 26.4; sixteen by 12 000 x 2560 21.8 and 23.5, 16 000 28.2 and 24.8.
 // Widths that the persistent kernels refuse all go to the former.
 bool small_rows(const void* matrix, const float* x, uint64_t x_stride_bytes, uint32_t columns, uint32_t rows, uint32_t tokens) {
     if (!q8_small_takes(matrix, x, x_stride_bytes, columns, rows)) return false;
     if (x_stride_bytes != uint64_t(columns) * 4 || !q8_mfma_supported(matrix, x, columns, rows)) return true;
+    if (tokens > 16) {
+        const uint32_t tiles = (tokens + 15) / 16, steps = ((rows + 15) / 16 * tiles + 255) / 256, stretches = (rows + 8191) / 8192;
+        const uint32_t pass = columns > 2048 ? 17 + 9 * stretches : columns == 2048 ? 14 + 5 * stretches : columns > 768 ? 12 + 8 * stretches : 11 + 10 * stretches;  // tenths of a step
+        return 10 * steps <= pass * tiles;
+    }
     if (columns > 2048) {
         if (tokens > (columns % 512 == 0 ? 10u : 5u)) return tokens > 8 ? rows < 13000 : rows <= 20480;
         return rows < (tokens > 8 ? 22000u : 31000u);
     }
-    if (tokens <= 8) return rows <= 12288;
-    if (tokens <= 16 || rows < 6000) return rows < 6000;
-    const uint32_t tiles = (tokens + 15) / 16, steps = ((rows + 15) / 16 * tiles + 255) / 256;
-    const uint32_t halves = columns <= 512 ? (tiles > 2 ? 6 : 5) : tokens <= 24 ? 3 : columns <= 1792 ? 5 : 4;  // of a step, for a tile
-    return 2 * steps + (columns > 1792 ? 1 : 0) <= halves * tiles;
+    return tokens > 8 ? rows < 6000 : rows <= 12288;
 }
 
 }  // namespace

@@ -685,22 +685,28 @@ __global__ __launch_bounds__(kThreads, 1) void q8_lanes_mfma_kernel(Q8MfmaArgs a
 namespace tsp {
 
 // Up to eight token rows in halves against a large matrix, where a wave with whole matrix rows is through before q8_resident.hip's workgroups (the bits are the
-// same). us a call, there and here:
-//   1536 and 2048 columns, four token rows on: the 65 536 rows that the waves take at once, give or take, and from two such rounds on: eight by 48 000 x 2048 27.4 and
-//   29.0, 60 000 33.8 and 31.2, 68 000 37.0 and 34.2, 80 000 41.2 and 40.6, 92 000 45.7 and 48.5, 124 000 59.4 and 58.3, 152 000 71.2 and 69.7; four by 68 000 37.1 and
-//   33.4, x 1536 30.7 and 32.5; one 34.8 and 40.5. With an odd number of token rows this kernel is some 3 us slower in the first range (five by 68 000
-//   x 2048 37.0 and 38.5): why is not known.
-//   1280 and 1792: five and seven waves there, one such workgroup a compute unit, are too few bytes on their way: eight by 64 000 x 1792 33.1 and 32.9,
-//   72 000 37.0 and 34.9, 128 000 58.8 and 52.4, x 1280 44.3 and 39.4; two by 72 000 x 1280 27.0 and 29.1, 88 000 31.2 and 30.2; one by 52 530 x 1792 (fewer
-//   are gemv.hip's) 28.6 and 25.7, 72 000 34.6 and 37.7.
-//   256: a workgroup of one wave there: eight by 32 000 7.7 and 7.7, 48 000 8.7 and 7.7, 151 936 14.0 and 12.3; one by 367 650 24.9 and 23.7.
-//   512 to 1024: never slower there by more than half a microsecond (eight by 64 001 x 1024 20.0 and 19.8, 100 000 26.7 and 31.1).
+// same). `tiles`: of 32 rows, for each of 256 compute units; eight are as many as its waves here. us a call, there and here:
+//   1536 and 2048 columns: where the tiles nearly fill a round of these waves, or fall short of half of the next one, and beyond the second round, where there is little
+//   between them: eight by 48 100 x 2048 27.1 and 28.6, 58 000 32.6 and 29.8, 71 200 37.5 and 34.7, 97 600 46.6 and 46.1, 100 900 49.4 and 53.2, 124 000 58.9 and 57.6; four by
+//   84 400 42.3 and 40.7; with five only from ten tiles on (67 900 36.3 and 39.1, 84 400 42.4 and 41.6), with one and three in one stretch (three by 58 000 31.2 and 30.5), with two
+//   nowhere (58 000 31.1 and 32.2) but behind half of a round there (157 200 66.0 and 63.2); by 1536 columns eight by
+//   51 400 25.6 and 24.2, 97 600 38.7 and 38.4; five by 67 900 30.6 and 28.7, three by 84 400 34.8 and 34.4, 206 300 70.8 and 65.4.
+//   1280 and 1792: five and seven waves there, one such workgroup a compute unit, are too few bytes on their way: eight by 58 000 x 1792 31.5 and 29.7, 71 200 36.5
+//   and 32.8, 153 700 67.7 and 61.6, x 1280 49.9 and 46.3; with few token rows there is less to do beside them: two by 67 900 x 1792 34.4 and 34.6, 84 400 40.1 and 37.7; one by
+//   54 700 (fewer are gemv.hip's) 28.3 and 26.1, 67 900 34.1 and 37.1, 91 000 41.4 and 39.1.
+//   256: a workgroup of one wave there: eight by 31 600 6.7 and 6.9, 34 900 8.3 and 7.1, 150 400 14.7 and 13.6; one by 367 650 24.9 and 23.7.
+//   512 to 1024: with eight, half a microsecond in a stretch each (77 800 x 512 16.3 and 15.7, 58 000 x 1024 19.4 and 18.8), else never (100 900 x 1024 27.1 and 31.8).
 static bool rows_by_waves(uint32_t columns, uint32_t rows, uint32_t width) {
+    const uint32_t tiles = rows / 8192;
     if (width > 8) return false;
     switch (columns / 256) {
-    case 1: return rows >= 40000;
-    case 5: case 7: return rows >= (width > 2 ? 72000u : 90000u) || (width == 1 && rows < 66000);
-    case 6: case 8: return width >= 4 && (rows >= 116000 || (rows >= 52000 && rows < 84000 && width % 2 == 0 && (width > 4 || columns == 2048)));
+    case 1: return tiles >= 4;
+    case 2: return width == 8 && tiles >= 8 && tiles < 11;
+    case 4: return width == 8 && tiles == 7;
+    case 5: return tiles >= (width > 5 ? 7 : width > 2 ? 8 : width == 2 ? 10 : 12);
+    case 6: return tiles >= 25 || (tiles >= 14 ? width >= 4 : width >= 5 ? tiles >= (width == 8 ? 6 : 8) && tiles < 12 : width == 3 && tiles == 10);
+    case 7: return (width == 1 && tiles < 8) || tiles >= (width > 6 ? 7 : width > 3 ? 8 : 10);
+    case 8: return tiles >= 14 ? width >= 5 || tiles == 19 : width == 4 || width >= 6 ? tiles >= 6 && tiles < 12 : width == 5 ? tiles >= 10 && tiles < 12 : width != 2 && tiles == 7;
     default: return false;
     }
 }
