@@ -28,7 +28,7 @@ struct ResidentDownArgs {
 bool resident_down_takes(uint32_t source_type, uint32_t channels, uint32_t hidden);  // source_type: 14 (Q6_K planes), 8 (Q8_0 planes) or 7 (Q5_1 planes)
 int launch_resident_down(const ResidentDownArgs& args, hipStream_t stream);
 
-// down_wide.hip: Q8_0 and Q5_1 planes, `hidden` columns (not 512), no always-on expert; the output spans at most 0xffff0000 bytes
+// down_wide.hip: Q8_0 and Q5_1 planes, `hidden` columns, no always-on expert; the output spans at most 0xffff0000 bytes
 bool wide_down_takes(uint32_t source_type, uint32_t channels, uint32_t hidden);
 int launch_wide_down(const ResidentDownArgs& args, uint32_t hidden, hipStream_t stream);
 

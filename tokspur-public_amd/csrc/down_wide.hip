@@ -1,5 +1,5 @@
 // Grouped down GEMM for experts in Q8_0 planes (quants / d) or Q5_1 planes (nibbles / fifth bits / d, m) of 128 to 768 hidden units
-// in multiples of 128 (512: where down_resident.hip is not the faster one), the task's h rows in LDS: y[route, channel] = 256 * sum_k h[slot, k] / 256 * w[channel, k].
+// in multiples of 128 (512: small layers with a route an expert and more, gemm.hip), the task's h rows in LDS: y[route, channel] = 256 * sum_k h[slot, k] / 256 * w[channel, k].
 //
 // The launch is a stream of expert weights from HBM and of f32 results back to it; what it costs is how many requests are on
 // their way. Hence:
@@ -18,7 +18,8 @@
 //
 // Measured (2048 tokens, 512 experts of 2560 x 640, ten selected, 615 tasks; 891 MB of Q8_0 weights and 210 MB of results): 250 us,
 // where the staged kernel's short-lived workgroups took 495 (planar_staged.hip, which stays for other widths). Bound by the
-// stream: 4.9 TB/s counting the rows of heavy experts that are read once per task.
+// stream: 4.9 TB/s counting the rows of heavy experts that are read once per task. Q8_0 at 640 hidden units takes all 256 registers and five
+// in scratch, read again where the task changes.
 #include "down_resident.hpp"
 #include "mfma_quant.hpp"
 #include "resident_tasks.hpp"

@@ -493,7 +493,7 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {  // two work
 // neighbouring lanes share one sub-block. Values outside the f16 range are flagged.
 // A wave takes 512 columns of one row: row and base addresses are scalars and nothing is divided per lane (a flat index divided by the
 // row's length, in 64 bits, and element-wise loads before). Bound by a trip to memory and back for small chunks, by memory from some 1000 rows
-// on. Products with their conversion: 37 x 6100 x 2560 f32 13.0 -> 12.4 us, 450 x 8192 x 2560 bf16 32.1 -> 31.6, 2048 x 8192 x 2048 69.2 -> 68.1.
+// on. Products with their conversion: 37 x 6100 x 2560 f32 13.0 -> 12.4 us; 450 x 8192 x 2560 bf16 and 2048 x 8192 x 2048 no more than runs differ (1 to 2 %).
 typedef uint32_t bf16_piece __attribute__((ext_vector_type(4), aligned(2)));  // rows are as aligned as their elements
 typedef float f32_piece __attribute__((ext_vector_type(4), aligned(4)));
 constexpr uint32_t kWaveColumns = 8 * kWave;

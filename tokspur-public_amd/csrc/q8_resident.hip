@@ -42,7 +42,8 @@ template <bool LANES, uint32_t WAVES, bool F32, int DEPTH>
 __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(WAVES > 8 ? 3 : 2, WAVES > 8 ? 3 : 2))) void q8_resident_kernel(Q8ResidentArgs a) {
     using Frag = std::conditional_t<F32, bf16x8, f16x8>;
     constexpr int PIECES = F32 ? 3 : 2;
-    constexpr bool kTight = WAVES > 8;  // three waves to a SIMD: 168 registers
+    // three waves to a SIMD: 168 registers, and eleven more in scratch (40 bytes a lane), which raw rows use before and behind the tile loop only; of q8_lanes_v1 rows four are read again for each tile
+    constexpr bool kTight = WAVES > 8;
     constexpr uint32_t kRounds = (kTileRows * kMostTokens + WAVES * kWave - 1) / (WAVES * kWave);
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // the waves' stages, then two sets of DEPTH tiles' sums [wave][16-row half][lane][4]
     __shared__ float largest[WAVES][kMostTokens];
@@ -122,7 +123,7 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(W
     Frag act[8][PIECES];  // the smallest pieces first
 #pragma unroll
     for (int b = 0; b < 8; ++b) {
-        if constexpr (kTight) {  // asked for again: beside the pieces and a tile's bytes they would not fit the registers
+        if constexpr (kTight) {  // asked for again: beside the pieces and a tile's bytes still more would not fit the registers
             asm volatile("" ::: "memory");
             __builtin_amdgcn_sched_barrier(0);
             xv[b] = token_piece(b);

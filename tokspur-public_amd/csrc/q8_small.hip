@@ -1,9 +1,8 @@
 // A Q8_0 matrix of a few megabytes against up to sixteen token rows (a sublayer's shared expert at draft verify, a short prompt):
 // y[t, r] = sum over blocks b of d[r, b] * sum_{k in b} q[r, k] * x[t, k].
 //
-// The persistent kernel (q8_mfma.hip) gives a wave all of K for 32 matrix rows, which leaves a matrix of 640 rows with twenty waves
-// on the whole chip, each a chain of ten round trips. Here a workgroup is ONE tile of 16 matrix rows and its sixteen waves take the
-// columns in turns of 64, so that 640 x 2560 is 640 waves that each ask for at most three pieces. A piece is read as it lies (17
+// The persistent kernel (q8_resident.hip) has tiles of 32 matrix rows for its workgroups, so a matrix of 640 rows is twenty of them on the
+// whole chip. Here a workgroup is ONE tile of 16 matrix rows and its sixteen waves take the columns in turns of 64, so that 640 x 2560 is 640 waves that each ask for at most three pieces. A piece is read as it lies (17
 // dwords of each weight row, 256 bytes of each token row, neighbouring lanes at neighbouring addresses: asking for fragments
 // directly, sixteen rows by 8 bytes at a time, took 12 us where this takes 5.4) and put into fragment order through LDS that belongs
 // to the wave alone, so no barrier stands between a piece's arrival and its multiplication. A token row is three bf16 pieces that are the
