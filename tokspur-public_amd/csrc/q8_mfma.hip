@@ -686,11 +686,12 @@ namespace tsp {
 
 // Up to eight token rows in halves against a large matrix, where a wave with whole matrix rows is through before q8_resident.hip's workgroups (the bits are the
 // same). `tiles`: of 32 rows, for each of 256 compute units; eight are as many as its waves here. us a call, there and here:
-//   1536 and 2048 columns: where the tiles nearly fill a round of these waves, or fall short of half of the next one, and beyond the second round, where there is little
-//   between them: eight by 48 100 x 2048 27.1 and 28.6, 58 000 32.6 and 29.8, 71 200 37.5 and 34.7, 97 600 46.6 and 46.1, 100 900 49.4 and 53.2, 124 000 58.9 and 57.6; four by
-//   84 400 42.3 and 40.7; with five only from ten tiles on (67 900 36.3 and 39.1, 84 400 42.4 and 41.6), with one and three in one stretch (three by 58 000 31.2 and 30.5), with two
-//   nowhere (58 000 31.1 and 32.2) but behind half of a round there (157 200 66.0 and 63.2); by 1536 columns eight by
-//   51 400 25.6 and 24.2, 97 600 38.7 and 38.4; five by 67 900 30.6 and 28.7, three by 84 400 34.8 and 34.4, 206 300 70.8 and 65.4.
+//   1536 and 2048 columns: where the tiles nearly fill a round of these waves, or fall short of half of the next one, and those of the second round and half of the third, where
+//   there is little between them: eight by 48 100 x 2048 27.1 and 28.6, 58 000 32.6 and 29.8, 71 200 37.5 and 34.7, 97 600 46.6 and 46.1, 100 900 49.4 and 53.2, 124 000 58.9 and
+//   57.6, 151 936 70.0 and 69.3, 168 000 76.2 and 80.7; four by 84 400 42.3 and 40.7, 151 936 66.6 and 67.1; with five only from ten tiles on (67 900 36.3 and 39.1, 84 400 42.4 and
+//   41.6), with one and three in one stretch (three by 58 000 31.2 and 30.5), with two nowhere (58 000 31.1 and 32.2); by 1536 columns eight by 51 400 25.6 and 24.2, 97 600
+//   38.7 and 38.4; five by 67 900 30.6 and 28.7, three by 84 400 34.8 and 34.4. (Matrices in rotation. Called with one matrix over and over, a good part of which the last-level
+//   cache then keeps, this kernel is the faster one from 143 900 rows on: one by 151 936 62.3 and 60.1.)
 //   1280 and 1792: five and seven waves there, one such workgroup a compute unit, are too few bytes on their way: eight by 58 000 x 1792 31.5 and 29.7, 71 200 36.5
 //   and 32.8, 153 700 67.7 and 61.6, x 1280 49.9 and 46.3; with few token rows there is less to do beside them: two by 67 900 x 1792 34.4 and 34.6, 84 400 40.1 and 37.7; one by
 //   54 700 (fewer are gemv.hip's) 28.3 and 26.1, 67 900 34.1 and 37.1, 91 000 41.4 and 39.1.
@@ -704,9 +705,9 @@ static bool rows_by_waves(uint32_t columns, uint32_t rows, uint32_t width) {
     case 2: return width == 8 && tiles >= 8 && tiles < 11;
     case 4: return width == 8 && tiles == 7;
     case 5: return tiles >= (width > 5 ? 7 : width > 2 ? 8 : width == 2 ? 10 : 12);
-    case 6: return tiles >= 25 || (tiles >= 14 ? width >= 4 : width >= 5 ? tiles >= (width == 8 ? 6 : 8) && tiles < 12 : width == 3 && tiles == 10);
+    case 6: return width >= 5 ? (tiles >= (width == 8 ? 6 : 8) && tiles < 12) || (tiles >= 14 && tiles < 20) : width == 3 && tiles == 10;
     case 7: return (width == 1 && tiles < 8) || tiles >= (width > 6 ? 7 : width > 3 ? 8 : 10);
-    case 8: return tiles >= 14 ? width >= 5 || tiles == 19 : width == 4 || width >= 6 ? tiles >= 6 && tiles < 12 : width == 5 ? tiles >= 10 && tiles < 12 : width != 2 && tiles == 7;
+    case 8: return width >= 4 && tiles < 12 ? tiles >= (width == 5 ? 10 : 6) : width >= 5 ? tiles >= 14 && tiles < 20 : width != 2 && width != 4 && tiles == 7;
     default: return false;
     }
 }
