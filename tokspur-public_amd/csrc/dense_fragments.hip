@@ -81,7 +81,7 @@ __global__ __launch_bounds__(64 * kMostWaves) __attribute__((amdgpu_waves_per_eu
     __builtin_amdgcn_sched_barrier(0);
 
     f32x16 acc{}, blk;
-    const Q4Consts q4c = q4_consts();
+    const Q4Masks masks = q4_masks();
     const Q4ScaleConsts q4s = q4_scale_consts();
     for (uint32_t b = first; b < end; ++b) {
         const Sources next = sources(b + 1);
@@ -97,7 +97,7 @@ __global__ __launch_bounds__(64 * kMostWaves) __attribute__((amdgpu_waves_per_eu
         auto step = [&](auto p_tag) {
             constexpr int P = decltype(p_tag)::value;
             const u32x4 raw = *reinterpret_cast<const u32x4*>(mine + 16 + P * 32 + khalf * 16);
-            Q4PairScale ps;
+            f16x2 ps;
             float scale[2], offset[2];
             if constexpr (EXACT) {
                 ps = q4_pair_scale<P>(hdr.sc[0], hdr.sc[1], q4s);
@@ -114,12 +114,12 @@ __global__ __launch_bounds__(64 * kMostWaves) __attribute__((amdgpu_waves_per_eu
                 __builtin_amdgcn_sched_barrier(0);  // fragments unpacked ahead of their products would not fit the registers
                 f16x8 w;
                 if constexpr (EXACT) {
-                    w = hi ? scaled8_q4_swapped<1>(raw[2 * ff], raw[2 * ff + 1], f16x2{ps.mul[1], ps.mul[1]}, f16x2{ps.bias[1], ps.bias[1]}, q4c)
-                           : scaled8_q4_swapped<0>(raw[2 * ff], raw[2 * ff + 1], f16x2{ps.mul[0], ps.mul[0]}, f16x2{ps.bias[0], ps.bias[0]}, q4c);
+                    w = hi ? scaled8_q4_swapped<1>(raw[2 * ff], raw[2 * ff + 1], f16x2{ps[1], ps[1]}, masks)
+                           : scaled8_q4_swapped<0>(raw[2 * ff], raw[2 * ff + 1], f16x2{ps[0], ps[0]}, masks);
                     const f32x16 zero{};
                     blk = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[f], w, f == 0 ? zero : blk, 0, 0, 0);
                 } else {
-                    w = weights8_q4_swapped(raw[2 * ff], raw[2 * ff + 1], hi ? q4c.hi_mask : q4c.lo_mask, scale[hi], offset[hi]);
+                    w = weights8_q4_swapped(raw[2 * ff], raw[2 * ff + 1], hi ? masks.hi : masks.lo, scale[hi], offset[hi]);
                     acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[f], w, acc, 0, 0, 0);
                 }
                 request_rows(next, f);
@@ -133,10 +133,12 @@ __global__ __launch_bounds__(64 * kMostWaves) __attribute__((amdgpu_waves_per_eu
             // acc += d * blk - dmin * sum_s Sx(hi + lo)[m, s] * mn[n, s]
             __builtin_amdgcn_sched_barrier(0);
             const f32x16 zero{};
+            float d = hdr.d * kQ4Lift, dmin = hdr.dmin;
+            asm volatile("" : "+v"(d), "+v"(dmin));  // as floats in registers: as halves they make every multiply-add a mixed-precision one, half as fast
             const f32x16 low = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums, minima_frag(hdr), zero, 0, 0, 0);
             request_sums(next);
 #pragma unroll
-            for (int v = 0; v < 16; ++v) acc[v] = __builtin_fmaf(-hdr.dmin, low[v], __builtin_fmaf(hdr.d, blk[v], acc[v]));
+            for (int v = 0; v < 16; ++v) acc[v] = __builtin_fmaf(-dmin, low[v], __builtin_fmaf(d, blk[v], acc[v]));
         }
     }
 

@@ -143,10 +143,8 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
     const uint32_t w_at = kWAt + w_r * 144;
     const uint32_t sx_at = kSxAt + (wm * (RT * 32) + col) * 32 + khalf * 16;
 
-    const Q4Consts q4c = q4_consts();
+    const Q4Masks masks = q4_masks();
     const Q4ScaleConsts q4s = q4_scale_consts();
-    struct { uint32_t low, high; } kc{0x000f000fu, 0x00f000f0u};
-    asm volatile("" : "+s"(kc.low), "+s"(kc.high));
     HdrQ4 hdr{};   // of the super-block at hand: a lane holds one weight row
     u32x4 raw[4];  // the lane's nibbles of the super-block's four steps
     f16x8 af[RT];  // a fragment serves one MFMA, and its register is refilled for the next group right behind it
@@ -164,9 +162,9 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
     uint32_t slot_now = 0, slot_next = kSlabBytes, slot_last = 2 * kSlabBytes;  // of the step at hand and the two after it
     auto step_fn = [&]<int P>(uint32_t b, const uint8_t* a_now, const uint8_t* a_next, const uint8_t* w_next, const uint8_t* sx_next, std::integral_constant<int, P>) {
         const uint8_t* const a_from = P == 0 ? a_now + 3 * 128 : a_next + (P - 1) * 128;
-        Q4PairScale ps;
+        f16x2 ps;
         float scale[2], offset[2];
-        const float fold_d = hdr.d, fold_dmin = hdr.dmin;
+        const float fold_d = hdr.d * kQ4Lift, fold_dmin = hdr.dmin;
         f16x8 minima;
         if constexpr (EXACT) {
             ps = q4_pair_scale<P>(hdr.sc[0], hdr.sc[1], q4s);
@@ -188,10 +186,10 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
             }
             f16x8 w;
             if constexpr (EXACT) {
-                w = hi ? scaled8_q4_swapped<1>(raw[P][2 * ff], raw[P][2 * ff + 1], f16x2{ps.mul[1], ps.mul[1]}, f16x2{ps.bias[1], ps.bias[1]}, q4c)
-                       : scaled8_q4_swapped<0>(raw[P][2 * ff], raw[P][2 * ff + 1], f16x2{ps.mul[0], ps.mul[0]}, f16x2{ps.bias[0], ps.bias[0]}, q4c);
+                w = hi ? scaled8_q4_swapped<1>(raw[P][2 * ff], raw[P][2 * ff + 1], f16x2{ps[1], ps[1]}, masks)
+                       : scaled8_q4_swapped<0>(raw[P][2 * ff], raw[P][2 * ff + 1], f16x2{ps[0], ps[0]}, masks);
             } else {
-                w = weights8_q4_swapped(raw[P][2 * ff], raw[P][2 * ff + 1], hi == 0 ? kc.low : kc.high, scale[hi], offset[hi]);
+                w = weights8_q4_swapped(raw[P][2 * ff], raw[P][2 * ff + 1], hi ? masks.hi : masks.lo, scale[hi], offset[hi]);
             }
             if (g == 3 && P == 3) read_header(b + 1);
             uint32_t from = a_at[(g + 1) % 4] + (g < 3 ? slot_now : slot_next);

@@ -95,7 +95,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 
     uint32_t bad = 0, phase = 0;
     uint32_t biggest = 0;  // the largest carried half's bits without the sign: anything not finite shows at the end
-    const Q4Consts q4c = q4_consts();
+    const Q4Masks masks = q4_masks();
     const Q4ScaleConsts q4s = q4_scale_consts();
 
     // The tasks come in two kinds, those of at most 32 rows (one row tile: 64 registers of activations) and those of 33..64
@@ -213,18 +213,18 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             // the stage is free again: the tile two ahead goes there
             request_next();
             stage = stage + kStageBytes == kStages * kStageBytes ? 0 : stage + kStageBytes;
-            float d = half_bits_to_float(dm & 0xffffu), dmin = half_bits_to_float(dm >> 16);
+            float d = half_bits_to_float(dm & 0xffffu) * kQ4Lift, dmin = half_bits_to_float(dm >> 16);
             asm volatile("" : "+v"(d), "+v"(dmin));  // as floats in registers: folded into the arithmetic as halves they make every multiply-add a mixed-precision one
 
             f32x16 blk[MT];
             auto steps = [&](auto p_tag) {
                 constexpr int P = decltype(p_tag)::value;
                 // the scales of sub-blocks 2P (low nibbles) and 2P + 1 (high nibbles, in place as 16 q: scale / 16) as one pair
-                const Q4PairScale sc = q4_pair_scale<P>(sm.x, sm.y, q4s);
+                const f16x2 sc = q4_pair_scale<P>(sm.x, sm.y, q4s);
 #pragma unroll
                 for (int hi = 0; hi < 2; ++hi) {
                     f16x8 f[2];
-                    frags_q4k_pair(raw[P], sc, hi, q4c, f);
+                    frags_q4k_pair(raw[P], sc, hi, masks, f);
 #pragma unroll
                     for (int ff = 0; ff < 2; ++ff)
 #pragma unroll

@@ -130,7 +130,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
     // ---- fragment addresses: chunk 4 (q / 2) + 2 khalf + q % 2 of row col in a slab, chunk 2 P + khalf of row col in a wave's lines
     const uint32_t a_at = col * 128 + (((2 * khalf) ^ (col / 2 % 8)) * 16), w_at = col * 128 + ((khalf ^ (col / 2 % 8)) * 16);
-    const Q4Consts q4c = q4_consts();
+    const Q4Masks masks = q4_masks();
     const Q4ScaleConsts q4s = q4_scale_consts();
     uint32_t biggest = 0;  // the largest carried half's bits without the sign: anything not finite shows at the end
 
@@ -152,7 +152,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         f32x16 acc[MT][2] = {}, blk[MT][2];
         f16x8 rows[MT], w[2];    // the present group's fragments
         u32x4 raw[4][2];  // the present super-block's nibbles by step
-        Q4PairScale scale[2];
+        f16x2 scale[2];
         uint4 sm[2], sm_next[2];
         uint32_t dm[2], dm_next[2];
         auto read_rows = [&](uint32_t from, int q, f16x8 (&into)[MT]) {
@@ -179,8 +179,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 if (G == 0) scale[j] = q4_pair_scale<P>(s[j].x, s[j].y, q4s);
-                const f16x2 s2 = f16x2{scale[j].mul[G / 2], scale[j].mul[G / 2]}, bias = f16x2{scale[j].bias[G / 2], scale[j].bias[G / 2]};
-                into[j] = scaled8_q4_swapped<G / 2>(raw[P][j][2 * (G % 2)], raw[P][j][2 * (G % 2) + 1], s2, bias, q4c);
+                into[j] = scaled8_q4_swapped<G / 2>(raw[P][j][2 * (G % 2)], raw[P][j][2 * (G % 2) + 1], f16x2{scale[j][G / 2], scale[j][G / 2]}, masks);
             }
         };
         // Group G (sixteen columns) of step P of super-block b
@@ -223,7 +222,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                     HdrQ4 h;
                     h.mn[0] = sm[j].z; h.mn[1] = sm[j].w;
                     mn[j] = minima_frag(h);
-                    d[j] = half_bits_to_float(dm[j] & 0xffffu); dmin[j] = half_bits_to_float(dm[j] >> 16);
+                    d[j] = half_bits_to_float(dm[j] & 0xffffu) * kQ4Lift; dmin[j] = half_bits_to_float(dm[j] >> 16);
                     asm volatile("" : "+v"(d[j]), "+v"(dmin[j]));  // as floats in registers: as halves they make every multiply-add a mixed-precision one
                 }
 #pragma unroll

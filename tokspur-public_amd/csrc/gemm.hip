@@ -379,7 +379,7 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {  // two work
             auto read_w = [&](int wbuf, int j, int p2) {  // row j*32 + col, chunk 2*p2 + khalf
                 return *reinterpret_cast<const u32x4*>(my_w + wbuf * 4096 + ((j * 32 + col) * 4 + ((2 * p2 + khalf) ^ ((col >> 1) & 3))) * 16);
             };
-            const Q4Consts q4c = q4_consts();
+            const Q4Masks masks = q4_masks();
             const Q4ScaleConsts q4s = q4_scale_consts();
             HdrQ4 hdr[2];
             RawHdrQ4 hdr_next[2];  // requested at P == 0, decoded at the end of P == 3: nothing touches the bytes while they travel
@@ -414,18 +414,18 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {  // two work
                 }
                 if (P == 0 || P == 2) { __builtin_amdgcn_sched_barrier(0); fetch_w_all(wstage[P == 0 ? 1 : 0], step / 2 + 2); }
                 const u32x4 raw0 = read_w(wbuf, 0, P & 1), raw1 = read_w(wbuf, 1, P & 1);
-                const Q4PairScale sc0 = q4_pair_scale<P>(hdr[0].sc[0], hdr[0].sc[1], q4s), sc1 = q4_pair_scale<P>(hdr[1].sc[0], hdr[1].sc[1], q4s);
+                const f16x2 sc0 = q4_pair_scale<P>(hdr[0].sc[0], hdr[0].sc[1], q4s), sc1 = q4_pair_scale<P>(hdr[1].sc[0], hdr[1].sc[1], q4s);
                 f16x8 f0[2], f1[2];
-                frags_q4k_pair(raw0, sc0, 0, q4c, f0);
-                frags_q4k_pair(raw1, sc1, 0, q4c, f1);
+                frags_q4k_pair(raw0, sc0, 0, masks, f0);
+                frags_q4k_pair(raw1, sc1, 0, masks, f1);
                 mfma(ring, 0, f0[0], f1[0], P == 0);
                 mfma(ring, 1, f0[1], f1[1], false);
-                frags_q4k_pair(raw0, sc0, 1, q4c, f0);
-                frags_q4k_pair(raw1, sc1, 1, q4c, f1);
+                frags_q4k_pair(raw0, sc0, 1, masks, f0);
+                frags_q4k_pair(raw1, sc1, 1, masks, f1);
                 mfma(ring, 2, f0[0], f1[0], false);
                 mfma(ring, 3, f0[1], f1[1], false);
                 if (P == 3) {
-                    fold(hdr[0].d, hdr[1].d);
+                    fold(hdr[0].d * kQ4Lift, hdr[1].d * kQ4Lift);
                     // minima: acc -= dmin * sum_s Sx(hi + lo)[m, s] * mn[n, s]
                     const f16x8 m0 = minima_frag(hdr[0]), m1 = minima_frag(hdr[1]);
     #pragma unroll

@@ -170,24 +170,25 @@ __device__ __forceinline__ HdrQ4 decode_hdr_q4k(const RawHdrQ4& r) {
 
 // Fragments of pair P: bytes 16h..16h+15 of the 32-byte pair; low nibbles (HI = 0) are sub-block 2P, high nibbles
 // sub-block 2P+1. Fragment f of a half covers activation columns HI*32 + 16h + f*8 .. +8 of the 64-column slab.
-// The columns of every eight come in the order (0, 2, 1, 3, 4, 6, 5, 7), for activations stored in that order: one mask-or per pair
-// of weights instead of a mask and two byte permutes per four. Low nibbles become 1024 + q, high nibbles stay in place as 1024 + 16 q and take the scale sc / 16 (exact: sc < 64).
-// (w & mask) | bits is one instruction (v_and_or_b32) only when the constants sit in registers: a VOP3 instruction of
-// this target takes no literal, and with two literals the compiler emits an and plus an or. The kernel therefore pins
-// the three constants to registers once and hands them to the unpacking.
-struct Q4Consts { uint32_t lo_mask, hi_mask, bits; };
-__device__ __forceinline__ Q4Consts q4_consts() {
-    Q4Consts c{0x000f000fu, 0x00f000f0u, 0x64006400u};
-    asm volatile("" : "+s"(c.lo_mask), "+s"(c.hi_mask), "+v"(c.bits));
-    return c;
+// The columns of every eight come in the order (0, 2, 1, 3, 4, 6, 5, 7), for activations stored in that order: one mask per pair of weights
+// instead of a mask and two byte permutes per four. A masked pair of nibbles is two subnormal halves, q * 2^-24 or, where the high ones sit, 16 q * 2^-24;
+// times 2^8 sc or 2^4 sc that is sc * q * 2^-16, as exact as sc * q itself (a scale byte of 255 still fits), in two instructions for two
+// weights, and the block's d makes up for the power of two (kQ4Lift). An and of two vector registers issues at twice the rate of an and-or, or of an and
+// with a scalar register, when two waves share a SIMD (1.0 against 1.9 ns an instruction): hence no bits to be or'ed in, and the masks in vector registers.
+struct Q4Masks { uint32_t lo, hi; };
+__device__ __forceinline__ Q4Masks q4_masks() {
+    Q4Masks m{0x000f000fu, 0x00f000f0u};
+    asm volatile("" : "+v"(m.lo), "+v"(m.hi));
+    return m;
 }
 template <int HI>
-__device__ __forceinline__ f16x8 scaled8_q4_swapped(uint32_t w0, uint32_t w1, f16x2 sc, f16x2 bias, const Q4Consts& c) {
-    const uint32_t m = HI ? c.hi_mask : c.lo_mask;
-    const f16x2 p0 = fma2(as_h2((w0 & m) | c.bits), sc, bias), p1 = fma2(as_h2(((w0 >> 8) & m) | c.bits), sc, bias);
-    const f16x2 p2 = fma2(as_h2((w1 & m) | c.bits), sc, bias), p3 = fma2(as_h2(((w1 >> 8) & m) | c.bits), sc, bias);
+__device__ __forceinline__ f16x8 scaled8_q4_swapped(uint32_t w0, uint32_t w1, f16x2 sc, const Q4Masks& masks) {
+    const uint32_t m = HI ? masks.hi : masks.lo;
+    const f16x2 p0 = as_h2(w0 & m) * sc, p1 = as_h2((w0 >> 8) & m) * sc;
+    const f16x2 p2 = as_h2(w1 & m) * sc, p3 = as_h2((w1 >> 8) & m) * sc;
     return f16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
 }
+constexpr float kQ4Lift = 65536.0f;
 // Byte N of a word as a float: one v_cvt_f32_ubyteN.
 template <int N>
 __device__ __forceinline__ float byte_as_float(uint32_t word) { return float((word >> (8 * N)) & 0xffu); }
@@ -206,34 +207,29 @@ __device__ __forceinline__ f16x8 weights8_q4_swapped(uint32_t w0, uint32_t w1, u
     return __builtin_bit_cast(f16x8, u32x4{two_weights(w0 & mask, scale, offset), two_weights((w0 >> 8) & mask, scale, offset), two_weights(w1 & mask, scale, offset),
                                            two_weights((w1 >> 8) & mask, scale, offset)});
 }
-// The scale set-up is shared by a pair of sub-blocks: the six-bit scales of sub-blocks 2P and 2P + 1 sit
-// in neighbouring bytes of the header; one byte permute puts them under 0x64 (1024 + sc as halves, side by side), one packed
-// add takes the 1024 off, and two packed multiplies make (sc, sc / 16) and (-1024 sc, -64 sc): the factors and the
-// offsets of the low-nibble and the high-nibble products. Four instructions per pair.
-struct Q4ScaleConsts { uint32_t sel[2]; uint32_t k64; f16x2 off, mul, bias; };
+// The scale set-up is shared by a pair of sub-blocks: the six-bit scales of sub-blocks 2P and 2P + 1 sit in neighbouring bytes of the
+// header; one byte permute puts them under 0x64 (1024 + sc as halves, side by side), one packed add takes the 1024 off, and one
+// packed multiply makes (2^8 sc, 2^4 sc): the factors of the low-nibble and of the high-nibble codes. Three instructions per pair.
+struct Q4ScaleConsts { uint32_t sel[2]; uint32_t k64; f16x2 off, mul; };
 __device__ __forceinline__ Q4ScaleConsts q4_scale_consts() {
     // selector bytes: 0..3 pick a byte of the header word, 4..7 a byte of the constant 0x64646464
-    Q4ScaleConsts c{{0x04010400u, 0x04030402u}, 0x64646464u, f16x2{_Float16(-1024.0f), _Float16(-1024.0f)},
-                    f16x2{_Float16(1.0f), _Float16(0.0625f)}, f16x2{_Float16(-1024.0f), _Float16(-64.0f)}};
+    Q4ScaleConsts c{{0x04010400u, 0x04030402u}, 0x64646464u, f16x2{_Float16(-1024.0f), _Float16(-1024.0f)}, f16x2{_Float16(256.0f), _Float16(16.0f)}};
     asm volatile("" : "+s"(c.sel[0]), "+s"(c.sel[1]), "+v"(c.k64));
     return c;
 }
-struct Q4PairScale { f16x2 mul, bias; };  // [0]: low nibbles (sub-block 2P), [1]: high nibbles (sub-block 2P + 1)
 template <int P>
-__device__ __forceinline__ Q4PairScale q4_pair_scale(uint32_t sc_lo4, uint32_t sc_hi4, const Q4ScaleConsts& c) {
+__device__ __forceinline__ f16x2 q4_pair_scale(uint32_t sc_lo4, uint32_t sc_hi4, const Q4ScaleConsts& c) {
     const uint32_t word = P < 2 ? sc_lo4 : sc_hi4;  // scales 0..3 | 4..7, one per byte
-    const f16x2 sc = as_h2(__builtin_amdgcn_perm(c.k64, word, c.sel[P & 1])) + c.off;  // (sc[2P], sc[2P + 1])
-    return Q4PairScale{sc * c.mul, sc * c.bias};
+    return (as_h2(__builtin_amdgcn_perm(c.k64, word, c.sel[P & 1])) + c.off) * c.mul;
 }
-__device__ __forceinline__ void frags_q4k_pair(const u32x4& raw, const Q4PairScale& s, int hi, const Q4Consts& c, f16x8 frag[2]) {
-    const f16x2 s2 = hi ? f16x2{s.mul[1], s.mul[1]} : f16x2{s.mul[0], s.mul[0]};
-    const f16x2 bias = hi ? f16x2{s.bias[1], s.bias[1]} : f16x2{s.bias[0], s.bias[0]};
+__device__ __forceinline__ void frags_q4k_pair(const u32x4& raw, f16x2 scale, int hi, const Q4Masks& masks, f16x8 frag[2]) {
+    const f16x2 s2 = hi ? f16x2{scale[1], scale[1]} : f16x2{scale[0], scale[0]};
     if (hi) {
-        frag[0] = scaled8_q4_swapped<1>(raw[0], raw[1], s2, bias, c);
-        frag[1] = scaled8_q4_swapped<1>(raw[2], raw[3], s2, bias, c);
+        frag[0] = scaled8_q4_swapped<1>(raw[0], raw[1], s2, masks);
+        frag[1] = scaled8_q4_swapped<1>(raw[2], raw[3], s2, masks);
     } else {
-        frag[0] = scaled8_q4_swapped<0>(raw[0], raw[1], s2, bias, c);
-        frag[1] = scaled8_q4_swapped<0>(raw[2], raw[3], s2, bias, c);
+        frag[0] = scaled8_q4_swapped<0>(raw[0], raw[1], s2, masks);
+        frag[1] = scaled8_q4_swapped<0>(raw[2], raw[3], s2, masks);
     }
 }
 
