@@ -710,6 +710,34 @@ def test_grouped_moe_gate_up_stream(gpu, tsp, orc, synth, channels, hidden):
     test_grouped_moe_other_planar_kinds(gpu, tsp, orc, synth, 12, 8, channels, hidden)
 
 
+# eight runs of places, small tasks among large ones: none or one of either kind, fewer tasks than runs, loads on either side of 32 and 64 rows, ends of
+# runs that are all tail, the most tasks there can be
+@pytest.mark.parametrize("loads", [[1, 0], [33, 0], [0, 2048], [1] * 512, [33] * 62, [32, 33, 64, 65, 31, 1, 0, 97, 96, 128, 129, 2], [70, 3] * 20 + [40] * 13 + [5],
+                                   [4] * 500 + [0, 0, 0, 0, 8, 3, 5, 1, 1, 30, 0, 0]], ids=len)
+@pytest.mark.parametrize("always_on", [False, True])
+def test_grouped_moe_order_of_tasks(gpu, tsp, orc, synth, loads, always_on):
+    channels, hidden, experts, n = 256, 256, len(loads), sum(loads)
+    gate, up, down = synth.matrix(12, 3441, hidden * experts, channels), synth.matrix(12, 3442, hidden * experts, channels), synth.matrix(14, 3443, channels * experts, hidden)
+    w = tsp.PlanarMoeWeights(gpu, 12, 14, channels, hidden, experts, gate, up, down)
+    ids = np.random.default_rng(n).permutation(np.repeat(np.arange(experts), loads)).astype(np.uint32)
+    x = synth.round_bf16(synth.activations_f32(3444 + n, (n, channels)))
+    shared = {}
+    if always_on:
+        sg, su, sd = synth.matrix(12, 3445, hidden, channels), synth.matrix(12, 3446, hidden, channels), synth.matrix(14, 3447, channels, hidden)
+        shared = {"shared": tsp.PlanarSharedExpert(gpu, channels, hidden, sg, su, sd)}
+    out = tsp.planar_nax_grouped_moe(gpu, w, gpu.upload(ids), gpu.upload(x), n, 1, tsp.GroupedScratch(gpu, n, 1, experts, channels, hidden, with_shared=always_on),
+                                     y=gpu.full((n, channels), np.nan), **shared)
+    assert gpu.error() == 0
+    wanted = [(out[0] if always_on else out, orc.moe_routed_reference(12, 14, gate, up, down, channels, hidden, experts, ids, n, 1, x, stage=12, threads=8)[1])]
+    if always_on:
+        wanted.append((out[1], orc.moe_routed_reference(12, 14, sg, su, sd, channels, hidden, 1, np.zeros(n, dtype=np.uint32), n, 1, x, stage=12, threads=8)[1]))
+    for got, declared in wanted:  # the bounds of the larger cases
+        got = got.cpu().numpy()
+        scale = np.maximum(1.0, np.sqrt((declared ** 2).mean(axis=1, keepdims=True)))
+        err = np.abs(got - declared) / np.maximum(scale, np.abs(declared))
+        assert float(np.median(err)) <= 2e-5 and float(err.max()) <= 4e-3 and nmse(got, declared) <= 1e-7
+
+
 @pytest.mark.parametrize("n,hidden,experts,selected", [(20, 256, 32, 4), (90, 512, 64, 4), (95, 256, 64, 4), (96, 256, 64, 4)])
 def test_grouped_moe_2048_columns_few_rows(gpu, tsp, orc, synth, n, hidden, experts, selected):
     """Either side of six rows per expert, where 2048-column experts change from the resident to the streaming gate/up kernel: loads of none, a

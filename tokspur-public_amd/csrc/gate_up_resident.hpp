@@ -1,7 +1,7 @@
 // Launch interface of the two grouped gate/up kernels: activations resident in registers (gate_up_resident.hip, 2048 channels), weights
 // and activations both streaming through LDS (gate_up_stream.hip, any multiple of 256).
 #pragma once
-#include "tsp_common.hpp"
+#include "grouping_device.hpp"
 
 namespace tsp {
 
@@ -20,12 +20,14 @@ struct ResidentGateUpArgs {
     const uint32_t* token_map;
     const uint32_t* ids;
     uint32_t task_slots;
+    const OrderedTask* order;  // the streaming kernel's: the same tasks as it takes them (task_order_block)
     _Float16* hbuf;           // [task_slots * 64][hidden]: SwiGLU output rows by task slot, as halves of h / 256
     uint32_t* error_word;
 };
 
 bool resident_gate_up_takes(uint32_t channels, uint32_t hidden);
 int launch_resident_gate_up(const ResidentGateUpArgs& args, hipStream_t stream);
+uint32_t stream_gate_up_tail(uint32_t hidden);  // task_order_block's tail for it
 int launch_stream_gate_up(const ResidentGateUpArgs& args, hipStream_t stream);  // hidden units in 32s
 
 }  // namespace tsp

@@ -17,12 +17,16 @@
 //     barrier per step stands before the step's last group: by then every wave has the whole slab in registers, so the
 //     barrier frees it and publishes the next.
 //   * Every request is unconditional (past the end the last one again), so each wave waits with an exact count.
+//   * A workgroup finds its task in one word pair at a place that its id names, and asks for the routes ahead of everything else: two trips
+//     stand before the rows' request where there were five. The places are filled so that the XCDs' runs are alike and end on light tasks (task_order_block).
 // 2048 tokens, 512 experts of 2560 x 640: 340 -> 278 us a launch (half lines through registers, a fragment read from LDS right before its product
-// before; 8 us of it are the sigmoid); 2048 x 512: 224 -> 196 (the resident kernel; 4 us are sums by super-block). At 2560 x 640 with the short
-// sigmoid, 270 us: 1.39 GB are fetched at 5.2 TB/s: 944 MB of planes, heavy experts' once per task, the headers' lines more than once, 0.1 GB
-// of rows. With the nibbles' lines in L2 242 us are left, with the headers' 245, without unpacking 260: bound by the lines' way in and by
-// instruction issue (66 % of the cycles) at once. Tried: persistent workgroups that request the next item's bytes during the last steps of this
-// one (298), tasks of more than 32 rows first (280), nibbles' lines as non-temporal (285).
+// before; 8 us of it are the sigmoid); 2048 x 512: 224 -> 196 (the resident kernel; 4 us are sums by super-block). With places and routes first, measured
+// in turn on another box: 203 -> 191 (2048 x 512), 290 -> 281. Bound by what it fetches and by its instructions at once (2048 x 512 and 2560 x 640): 0.91 and 1.36 GB,
+// the planes once per task, the headers' lines twice, 0.1 GB of rows, in 167 and 250 us without any arithmetic (5.4 TB/s); the arithmetic alone
+// takes 158 and 215 with nothing to wait for, 40 and 46 of it where a super-block's sums are scaled and added. Barriers and reads of rows from LDS are free.
+// Tried: persistent workgroups that request the next item's bytes during the last steps of this
+// one (298 for 270), tasks of more than 32 rows first (280), nibbles' lines as non-temporal (285), an expert's tasks on one column tile side by side (they do not
+// meet in L2 either: as many bytes).
 #include "gate_up_resident.hpp"
 #include "mfma_quant.hpp"
 #include "resident_tasks.hpp"
@@ -53,21 +57,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const uint32_t col = lane % 32, khalf = lane / 32;
     const uint32_t bpr = a.channels / 256, steps = 4 * bpr, col_tiles = (a.hidden + kUnits - 1) / kUnits;
 
-    // ---- (task, units) from the workgroup id: ids go to the eight XCDs in turn, and each XCD takes an eighth of the live pairs in order,
-    // so that the units of a task, and the tasks of an expert, meet in one L2
-    const uint32_t listed = a.tasks[0];
-    if (listed > a.task_slots || a.tasks[1] != a.tokens * a.selected) {
-        if (tid == 0 && blockIdx.x == 0) atomicOr(a.error_word, TSP_ERRBIT_INDEX);
-        return;
-    }
-    const uint32_t live = listed * col_tiles, per_xcd = (live + 7) / 8, logical = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-    if (blockIdx.x / 8 >= per_xcd || logical >= live) return;
-    const uint32_t unit0 = (logical % col_tiles) * kUnits + wave * 32;
-    const ResidentTask t = resolve_resident_task(a.tasks, a.counts, logical / col_tiles, listed, a.experts, a.tokens, a.shared_gate != nullptr);
-    if (!t.ok) {
-        if (tid == 0) atomicOr(a.error_word, TSP_ERRBIT_INDEX);
-        return;
-    }
+    // ---- (task, units) from the workgroup id: ids go to the eight XCDs in turn, and the units of a task meet in one L2
+    const uint32_t place = blockIdx.x / 8;
+    const OrderedTask mine = a.order[(blockIdx.x % 8) * order_pitch(a.task_slots) + place / col_tiles];
+    if (!(mine.what >> 31)) return;
+    ResidentTask t;
+    t.task = mine.task; t.expert = mine.what & 1023u; t.start = (mine.what >> 10 & 63u) * kTaskRows; t.nrows = mine.what >> 16 & 127u;
+    t.shared = t.expert == a.experts;
+    const uint32_t unit0 = (place % col_tiles) * kUnits + wave * 32;
     const uint32_t half_e = a.experts / 2;
     const uint8_t* const pair = (t.expert < half_e ? a.pair_lo : a.pair_hi) + uint64_t(t.expert < half_e ? t.expert : t.expert - half_e) * 2 * a.spec.planar_expert_bytes;
     const uint8_t* const gate = t.shared ? a.shared_gate : pair;
@@ -99,33 +96,38 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
     };
     const uint32_t gate_at = my_lines, up_at = gate_at + kLines;
+    // The task's routes first, each wave its own copy: their answer alone has to be there before the rows can be asked for (a table of the
+    // workgroup's behind the weights, with the expert's id of each route looked up before its row is, was three more trips one after the other).
+    const uint32_t my_routes = kSumsAt + wave * 512;
+    if (!t.shared) load_to_lds_4(a.token_map + uint64_t(t.expert) * a.tokens + t.start, (lane < t.nrows ? lane : 0) * 4, lds_at + my_routes);
     request_lines(gate, 0, gate_at);
     request_lines(up, 0, up_at);
     request_headers(0);
 
-    // ---- the task's rows: a row past the end repeats the first one and is not stored, a route that is not the expert's stands for token 0 and
-    // the batch is refused
-    uint32_t* const row_src = reinterpret_cast<uint32_t*>(lds + kSumsAt);
+    // ---- the task's rows: a row past the end repeats the first one and is not stored; a route that is not the expert's shows behind the first wait,
+    // and the batch is refused. Activations: instruction i covers rows 8 wave + 32 i .. + 7, eight lanes per row; sums: 16 bytes each of 64 rows x 32, sixteen rows per wave.
     uint32_t bad = 0;
-    if (tid < kTaskRows) {
-        const uint32_t r = t.start + (tid < t.nrows ? tid : 0);
-        uint32_t token = r;
-        if (!t.shared) {
-            const uint32_t rid = a.token_map[uint64_t(t.expert) * a.tokens + r];
-            const bool fits = rid < a.tokens * a.selected && a.ids[rid] == t.expert;
-            if (!fits) bad = TSP_ERRBIT_INDEX;
-            token = fits ? rid / a.selected : 0;
+    const uint32_t my_rows[3] = {wave * 8 + lane / 8, wave * 8 + lane / 8 + 32, wave * 16 + col / 2};
+    uint32_t token[3], named[2] = {t.expert, t.expert};  // the experts that the first two rows' routes name
+    if (t.shared) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) token[i] = t.start + (my_rows[i] < t.nrows ? my_rows[i] : 0);
+    } else {
+        wait_after_loads<16>();  // all but the requests for weights
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            uint32_t rid = *reinterpret_cast<const uint32_t*>(lds + my_routes + my_rows[i] * 4);
+            if (rid >= a.tokens * a.selected) { bad = TSP_ERRBIT_INDEX; rid = 0; }
+            token[i] = rid / a.selected;
+            if (i < 2) named[i] = a.ids[rid];
         }
-        row_src[tid] = token;
     }
-    __syncthreads();
-    // activations: instruction i covers rows 8 wave + 32 i .. + 7, eight lanes per row; chunk c of row n sits at position c ^ (n / 2) % 8
+    // chunk c of row n sits at position c ^ (n / 2) % 8
     const uint32_t a_chunk = ((lane % 8) ^ ((4 * wave + lane / 16) % 8)) * 16;
     uint32_t a_lane[2];  // byte offsets: 2048 tokens of 65536 channels at most
 #pragma unroll
-    for (uint32_t i = 0; i < 2; ++i) a_lane[i] = row_src[wave * 8 + lane / 8 + i * 32] * (a.channels * 2) + a_chunk;
-    // sums: 16 bytes each of 64 rows x 32, sixteen rows per wave
-    const uint32_t s_lane = row_src[wave * 16 + col / 2] * (bpr * 32) + (col % 2) * 16;
+    for (uint32_t i = 0; i < 2; ++i) a_lane[i] = token[i] * (a.channels * 2) + a_chunk;
+    const uint32_t s_lane = token[2] * (bpr * 32) + (col % 2) * 16;
     auto request_sums = [&](uint32_t b) { if (lane < 32) load_to_lds_16(reinterpret_cast<const uint8_t*>(a.sx) + b * 32, s_lane, lds_at + kSumsAt + wave * 512); };
 
     // ---- fragment addresses: chunk 4 (q / 2) + 2 khalf + q % 2 of row col in a slab, chunk 2 P + khalf of row col in a wave's lines
@@ -147,6 +149,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         request_rows(1, slab1);
         request_rows(2, slab2);
         wait_all_loads();
+        asm volatile("" : "+v"(named[0]), "+v"(named[1]));  // looked at from here on: sooner would be a wait for everything older
+        if (named[0] != t.expert || named[1] != t.expert) bad = TSP_ERRBIT_INDEX;
         __syncthreads();
 
         f32x16 acc[MT][2] = {}, blk[MT][2];
@@ -297,8 +301,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
 namespace tsp {
 
+// Half a round of an XCD's 64 workgroups (one, one and a half and two: the same to 0.3 % of a sublayer, 2048 tokens).
+uint32_t stream_gate_up_tail(uint32_t hidden) { return 32 / ((hidden + kUnits - 1) / kUnits); }
+
 int launch_stream_gate_up(const ResidentGateUpArgs& a, hipStream_t s) {
-    const uint32_t groups = (a.task_slots * ((a.hidden + kUnits - 1) / kUnits) + 7) / 8 * 8;
+    const uint32_t groups = 8 * order_pitch(a.task_slots) * ((a.hidden + kUnits - 1) / kUnits);
     if (resident_gate_up_takes(a.channels, a.hidden)) TSP_LAUNCH("gemm_gate_up_swiglu", s, gate_up_stream_kernel<true><<<groups, 256, 0, s>>>(a));
     else TSP_LAUNCH("gemm_gate_up_swiglu", s, gate_up_stream_kernel<false><<<groups, 256, 0, s>>>(a));
     return launch_status("gate_up_stream");

@@ -578,32 +578,39 @@ __global__ __launch_bounds__(256) void to_f16_rows(const void* __restrict__ src,
     if (row < rows) to_f16_row_part<FROM_BF16>(src, src_stride_bytes, dst, sx, row, blockIdx.x, columns, error_word);
 }
 
-// What a grouped product needs before its first matrix instruction: the two task lists (workgroups 0 and 1), each expert's routes (ROUTES: the next
+// What a grouped product needs before its first matrix instruction: the two task lists (workgroups 0 and 1), the order of the second (2), each expert's routes (ROUTES: the next
 // `experts` workgroups; else they are there) and the row conversion (all others) in one launch: a launch of its own costs each of these small kernels
 // more than its work. With ROUTES the lists' workgroups count the ids for themselves.
 struct TaskLists {
     const uint32_t* ids; uint32_t *token_map, *counts;
     uint32_t* tasks0; uint32_t tile0; uint32_t* tasks1; uint32_t tile1; uint32_t experts, selected, tokens;
     bool every_token1;  // list 1 also holds the always-on expert's tasks
+    OrderedTask* order1;  // list 1's tasks in the order a launch takes them (task_order_block), or null
+    uint32_t tail1;
     uint32_t* classes1;  // list 1 is a 64-row list: its tasks by number of rows (task_class_lists_block), or null
 };
 template <bool ROUTES>
 __global__ __launch_bounds__(512) void tasks_and_rows(TaskLists t, const void* __restrict__ src, uint64_t src_stride_bytes, _Float16* __restrict__ dst,
                                                       _Float16* __restrict__ sx, uint32_t rows, uint32_t columns, uint32_t* error_word) {
     __shared__ __attribute__((aligned(16))) uint32_t counted[ROUTES ? 2048 : 4];
-    __shared__ uint32_t totals[24];
-    const uint32_t others = 2 + (ROUTES ? t.experts : 0);
-    if (blockIdx.x < 2) {
+    __shared__ __attribute__((aligned(16))) uint32_t totals[24], kinds[48];
+    const uint32_t others = 3 + (ROUTES ? t.experts : 0);
+    if (blockIdx.x < 3) {
+        if (blockIdx.x == 2 && !t.order1) return;
         const uint32_t* counts = t.counts;
         if constexpr (ROUTES) {
             count_routes_block(t.ids, t.experts, t.selected, t.tokens, counted);
             counts = counted;
         }
+        if (blockIdx.x == 2) {
+            task_order_block(counts, t.order1, t.tail1, t.experts, t.selected, t.tokens, t.every_token1, totals, kinds);
+            return;
+        }
         grouped_tasks_block(counts, blockIdx.x == 0 ? t.tasks0 : t.tasks1, blockIdx.x == 0 ? t.tile0 : t.tile1, t.experts, t.selected, t.tokens,
                             error_word, totals, blockIdx.x == 1 && t.every_token1);
         if (blockIdx.x == 1 && t.classes1) task_class_lists_block(counts, t.classes1, t.experts, t.selected, t.tokens, t.every_token1, totals);
     } else if (ROUTES && blockIdx.x < others) {
-        expert_routes_block<512>(t.ids, t.token_map, t.counts, blockIdx.x - 2, t.experts, t.selected, t.tokens, error_word, totals);
+        expert_routes_block<512>(t.ids, t.token_map, t.counts, blockIdx.x - 3, t.experts, t.selected, t.tokens, error_word, totals);
     } else {
         const uint32_t parts = column_waves(columns), block = blockIdx.x - others, row = block / parts * 8 + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
         if (row < rows) to_f16_row_part<false>(src, src_stride_bytes, dst, sx, row, block % parts, columns, error_word);
@@ -644,12 +651,12 @@ int convert_fragments(const void* src, uint64_t stride, int from_bf16, _Float16*
 int prepare_grouped(const TaskLists& t, const void* src, uint64_t stride, _Float16* dst, _Float16* sx, uint32_t rows, uint32_t columns, uint32_t* err, hipStream_t s) {
     const uint32_t row_groups = (rows + 7) / 8 * column_waves(columns);
     if (t.tokens <= 512) {
-        TSP_LAUNCH("tasks_and_rows", s, tasks_and_rows<true><<<2 + t.experts + row_groups, 512, 0, s>>>(t, src, stride, dst, sx, rows, columns, err));
+        TSP_LAUNCH("tasks_and_rows", s, tasks_and_rows<true><<<3 + t.experts + row_groups, 512, 0, s>>>(t, src, stride, dst, sx, rows, columns, err));
         return launch_status("tasks_and_rows");
     }
     const int rc = tsp_grouped_routes(t.ids, t.token_map, t.counts, t.experts, t.selected, t.tokens, err, s);
     if (rc != TSP_OK) return rc;
-    TSP_LAUNCH("tasks_and_rows", s, tasks_and_rows<false><<<2 + row_groups, 512, 0, s>>>(t, src, stride, dst, sx, rows, columns, err));
+    TSP_LAUNCH("tasks_and_rows", s, tasks_and_rows<false><<<3 + row_groups, 512, 0, s>>>(t, src, stride, dst, sx, rows, columns, err));
     return launch_status("tasks_and_rows");
 }
 
@@ -803,7 +810,7 @@ extern "C" int tsp_grouped_mm(uint32_t encoding, uint32_t layout, const void* ma
     auto* xh = reinterpret_cast<_Float16*>(ws);
     auto* sx = reinterpret_cast<_Float16*>(ws + l.sx);
     auto* task_list = reinterpret_cast<uint32_t*>(ws + l.tasks);
-    const int rc = prepare_grouped(TaskLists{ids, token_map, counts, tasks, 32, task_list, kTaskRows, experts, selected, tokens, false, nullptr}, input, input_stride_bytes, xh, sx,
+    const int rc = prepare_grouped(TaskLists{ids, token_map, counts, tasks, 32, task_list, kTaskRows, experts, selected, tokens, false, nullptr, 0, nullptr}, input, input_stride_bytes, xh, sx,
                                    l.in_rows, columns, error_word, s);
     if (rc != TSP_OK) return rc;
     GemmArgs a{};
@@ -816,7 +823,7 @@ extern "C" int tsp_grouped_mm(uint32_t encoding, uint32_t layout, const void* ma
 
 // ---------------------------------------------------------------- grouped MoE
 namespace {
-struct NaxLayout { uint64_t xh, sx, tasks, classes, hbuf, meta, total; uint32_t bound; };
+struct NaxLayout { uint64_t xh, sx, tasks, classes, hbuf, meta, order, total; uint32_t bound; };
 NaxLayout nax_layout(uint32_t tokens, uint32_t selected, uint32_t experts, uint32_t channels, uint32_t hidden, bool shared = false) {
     NaxLayout l{};
     l.bound = tokens * selected / kTaskRows + experts + (shared ? (tokens + kTaskRows - 1) / kTaskRows : 0);
@@ -826,6 +833,8 @@ NaxLayout nax_layout(uint32_t tokens, uint32_t selected, uint32_t experts, uint3
     l.classes = l.tasks + align256((2 + 2 * uint64_t(l.bound)) * 4);  // the 64-row tasks by number of rows: two counts, two index lists
     l.hbuf = l.classes + align256((2 + 2 * uint64_t(l.bound)) * 4);
     l.meta = l.hbuf + align256(uint64_t(l.bound) * kTaskRows * hidden * 2);  // union records of one chunk of eight tokens
+    l.order = l.meta;  // of the kernels that take them; the others' records lie there
+    static_assert(8 * order_pitch(2048 * 16 / kTaskRows + 512 + 2048 / kTaskRows) * sizeof(OrderedTask) <= 2320 * 4);
     l.total = l.meta + align256(2320 * 4);
     return l;
 }
@@ -955,9 +964,15 @@ int grouped_moe(const tsp_grouped_moe* m, const tsp_shared_expert* shared, void*
     auto* task_list = reinterpret_cast<uint32_t*>(ws + l.tasks);
     auto* hbuf = reinterpret_cast<_Float16*>(ws + l.hbuf);
 
+    // Few rows per expert: the launch is bound by HBM, and the resident kernel's shares of 32 units leave no compute unit waiting for
+    // another (a sublayer of 2048 x 512, 512 experts: 20 tokens 102 us against 114, 100 tokens 216 against 220; 400 tokens 302 against 295, 2048
+    // tokens 478 against 449; 2048 x 768, 128 experts: 50 tokens 143 against 145, 100 tokens 152 against 151, 2048 tokens 408 against 383).
+    // The two add a row's super-blocks up in the same order and with the same roundings.
+    const bool stream_gate_up = fast_gate_up && !(routes < 6 * m->experts && resident_gate_up_takes(m->channels, m->hidden));
+    auto* order = reinterpret_cast<OrderedTask*>(ws + l.order);
     // only the Q4_K gate/up kernels want the activation sums and the column order that goes with them
     rc = prepare_grouped(TaskLists{m->ids, m->token_map, m->counts, m->tasks, 32, task_list, kTaskRows, m->experts, m->selected, m->tokens, shared != nullptr,
-                                   reinterpret_cast<uint32_t*>(ws + l.classes)},
+                                   stream_gate_up ? order : nullptr, stream_gate_up_tail(m->hidden), reinterpret_cast<uint32_t*>(ws + l.classes)},
                          m->x, m->x_stride_bytes, xh, fast_gate_up ? sx : nullptr, m->tokens, m->channels, m->error_word, s);
     if (rc != TSP_OK) return rc;
 
@@ -977,12 +992,8 @@ int grouped_moe(const tsp_grouped_moe* m, const tsp_shared_expert* shared, void*
         r.spec = gu; r.experts = m->experts; r.tokens = m->tokens; r.selected = m->selected; r.channels = m->channels; r.hidden = m->hidden;
         r.tasks = task_list; r.classes = reinterpret_cast<const uint32_t*>(ws + l.classes); r.counts = m->counts; r.token_map = m->token_map; r.ids = m->ids; r.task_slots = l.bound;
         r.hbuf = hbuf; r.error_word = m->error_word;
-        // Few rows per expert: the launch is bound by HBM, and the resident kernel's shares of 32 units leave no compute unit waiting for
-        // another (a sublayer of 2048 x 512, 512 experts: 20 tokens 102 us against 114, 100 tokens 216 against 220; 400 tokens 302 against 295, 2048
-        // tokens 478 against 449; 2048 x 768, 128 experts: 50 tokens 143 against 145, 100 tokens 152 against 151, 2048 tokens 408 against 383).
-        // The two add a row's super-blocks up in the same order and with the same roundings.
-        const bool few = routes < 6 * m->experts;
-        rc = few && resident_gate_up_takes(m->channels, m->hidden) ? launch_resident_gate_up(r, s) : launch_stream_gate_up(r, s);
+        r.order = order;
+        rc = stream_gate_up ? launch_stream_gate_up(r, s) : launch_resident_gate_up(r, s);
     }
     if (rc != TSP_OK) return rc;
     const uint64_t shared_span = shared ? uint64_t(m->tokens) * shared->y_stride_bytes : 0;

@@ -202,6 +202,70 @@ __device__ __forceinline__ void task_class_lists_block(const uint32_t* __restric
     }
 }
 
+// The tasks of a 64-row list in the order in which a launch with a workgroup per (task, column tile) takes them: eight runs, one per XCD, of
+// `order_pitch` places each; a place holds the whole task, so that a workgroup knows from its id alone where to look and asks once, or zero.
+// A task of more than 32 rows takes about half as long again as one of fewer. Every XCD gets an eighth of either kind, the large ones at even distances
+// among the small ones (products of the one beside the other's weights on their way), and its last `tail` are small: what is left running alone when
+// the others have nothing more is short. 2048 tokens, 512 experts, gate/up: 2048 x 512 195 -> 190 us, 2560 x 640 287 -> 281 against list order; no tail 193
+// and 281, all large ones first 200 and 294.
+struct OrderedTask { uint32_t what, task; };  // what: 1 << 31 | rows << 16 | (first row / 64) << 10 | expert; task: index in the list
+constexpr uint32_t order_pitch(uint32_t bound) { return bound / 8 + 2; }
+// One block of 512 threads; experts <= 512, tokens <= 2048. `kinds`: 48 words of LDS, `totals` those of the scans.
+__device__ __forceinline__ void task_order_block(const uint32_t* __restrict__ counts, OrderedTask* __restrict__ out, uint32_t tail, uint32_t experts,
+                                                 uint32_t selected, uint32_t tokens, bool every_token, uint32_t* totals, uint32_t* kinds) {
+    constexpr uint32_t tile = 64;
+    const uint32_t tid = threadIdx.x;
+    const uint32_t extra = every_token ? (tokens + tile - 1) / tile : 0;
+    const uint32_t bound = tokens * selected / tile + experts + extra, pitch = order_pitch(bound);
+    const uint32_t raw = tid < experts ? counts[tid] : 0, count = raw < tokens ? raw : tokens;
+    const uint32_t n = (count + tile - 1) / tile;
+    const uint32_t small = n && count - (n - 1) * tile <= 32 ? 1 : 0;
+    uint32_t scans[3] = {n, small, raw}, sums[3];
+    scan512(scans, sums, totals);
+    const uint32_t extra_small = extra && tokens - (extra - 1) * tile <= 32 ? 1 : 0;
+    const uint32_t total = sums[0], all_small = sums[1] + extra_small, all_large = total + extra - all_small;
+    const uint32_t first = scans[0] - n, first_small = scans[1] - small, first_large = first - first_small;
+    const bool whole = sums[2] == tokens * selected && total + extra <= bound;  // else the list's block flags the batch, and no task is taken up
+    // XCD x has the small tasks from ceil(x all / 8) on and the large ones likewise
+    auto begin = [](uint32_t all, uint32_t x) { return (all * x + 7) / 8; };
+    struct Run { uint32_t small0, large0, early, large; };  // early: small tasks ahead of the tail
+    Run* const runs = reinterpret_cast<Run*>(kinds);
+    if (tid < 8) {
+        const uint32_t s0 = begin(all_small, tid), l0 = begin(all_large, tid), s = begin(all_small, tid + 1) - s0;
+        runs[tid] = Run{s0, l0, s > tail ? s - tail : 0, begin(all_large, tid + 1) - l0};
+        kinds[32 + tid] = whole ? s + begin(all_large, tid + 1) - l0 : 0;
+    }
+    __syncthreads();
+    auto xcd_of = [](uint32_t rank, uint32_t all) { return uint32_t((float(rank * 8) + 0.5f) / float(all)); };  // floor(8 rank / all), both under 2^14
+    auto over = [](uint32_t a, uint32_t b) { return uint32_t((float(a) + 0.5f) / float(b)); };                  // floor(a / b) where a < 2^16, b < 2^9
+    auto put_small = [&](uint32_t rank, OrderedTask t) {
+        const uint32_t x = xcd_of(rank, all_small), i = rank - runs[x].small0;
+        const uint32_t early = runs[x].early, large = runs[x].large;
+        uint32_t before = large;  // large ones ahead of this one
+        if (i < early) { before = over((i + 1) * large + early - 1, early); before = before < large ? before : large; }
+        out[x * pitch + i + before] = t;
+    };
+    auto put_large = [&](uint32_t rank, OrderedTask t) {
+        const uint32_t x = xcd_of(rank, all_large), i = rank - runs[x].large0, large = runs[x].large;
+        out[x * pitch + over(i * (large + runs[x].early), large)] = t;
+    };
+    auto ordered = [&](uint32_t expert, uint32_t i, uint32_t rows, uint32_t task) { return OrderedTask{1u << 31 | (rows < tile ? rows : tile) << 16 | i << 10 | expert, task}; };
+    if (whole) {
+        for (uint32_t i = 0; i < n; ++i) {
+            const OrderedTask t = ordered(tid, i, count - i * tile, first + i);
+            if (small && i + 1 == n) put_small(first_small, t);
+            else put_large(first_large + i, t);
+        }
+        for (uint32_t i = tid; i < extra; i += 512) {
+            const OrderedTask t = ordered(experts, i, tokens - i * tile, total + i);
+            if (extra_small && i + 1 == extra) put_small(sums[1], t);
+            else put_large(total - sums[1] + i, t);
+        }
+    }
+    for (uint32_t x = tid / kWave; x < 8; x += 512 / kWave)
+        for (uint32_t i = kinds[32 + x] + tid % kWave; i < pitch; i += kWave) out[x * pitch + i] = OrderedTask{0, 0};
+}
+
 // The union records of at most 128 routes (T <= 8 tokens x S <= 16 slots): records (expert, <= cap routes) in first-use
 // order. Block layout in 32-bit words: [0..7] header, +8 experts[128], +136 counts[128], +264 tokens[128][8],
 // +1288 routes[128][8]. Thread f < 128 owns flat route f and brings its expert id (`mine`, anything when f >= T S); threads
