@@ -738,9 +738,9 @@ def test_grouped_moe_order_of_tasks(gpu, tsp, orc, synth, loads, always_on):
         assert float(np.median(err)) <= 2e-5 and float(err.max()) <= 4e-3 and nmse(got, declared) <= 1e-7
 
 
-@pytest.mark.parametrize("n,hidden,experts,selected", [(20, 256, 32, 4), (90, 512, 64, 4), (95, 256, 64, 4), (96, 256, 64, 4)])
+@pytest.mark.parametrize("n,hidden,experts,selected", [(20, 256, 32, 4), (90, 512, 64, 4), (95, 256, 64, 4), (96, 256, 64, 4), (255, 256, 32, 4), (256, 256, 32, 4)])
 def test_grouped_moe_2048_columns_few_rows(gpu, tsp, orc, synth, n, hidden, experts, selected):
-    """Either side of six rows per expert, where 2048-column experts change from the resident to the streaming gate/up kernel: loads of none, a
+    """Either side of 32 rows per expert, where 2048-column experts change from the resident to the streaming gate/up kernel: loads of none, a
     few, more than 32 and more than 64 rows, the bounds of the larger cases, and what is reported."""
     channels = 2048
     gate, up, down = synth.matrix(12, 3421, hidden * experts, channels), synth.matrix(12, 3422, hidden * experts, channels), synth.matrix(14, 3423, channels * experts, hidden)
@@ -767,6 +767,31 @@ def test_grouped_moe_2048_columns_few_rows(gpu, tsp, orc, synth, n, hidden, expe
     x[n - 1, 2047] = np.inf
     tsp.planar_nax_grouped_moe(gpu, w, gpu.upload(ids.reshape(-1)), gpu.upload(x), n, selected, scratch)
     assert gpu.error() & tsp.ERRBIT_NONFINITE
+
+
+# persistent workgroups' parts of a launch: none or one of either kind of task, fewer items than workgroups, parts that begin within a task's start, of
+# one kind only and of both; the gate/up kernel with its rows in registers, and the down kernels of either construction
+@pytest.mark.parametrize("dn_type,channels,hidden,experts", [(14, 512, 512, 512), (8, 512, 512, 512), (7, 512, 512, 512), (8, 256, 640, 512), (7, 256, 640, 512), (14, 2048, 256, 64)])
+@pytest.mark.parametrize("loads", [[1], [64], [33, 7], [300, 1, 2, 3, 4, 5], [5] * 60, [70] * 3 + [2] * 40 + [34] * 2, [1] * 64], ids=sum)
+def test_grouped_moe_parts_of_a_launch(gpu, tsp, orc, synth, dn_type, channels, hidden, experts, loads):
+    n = sum(loads)
+    at = np.random.default_rng(n).permutation(experts)[:len(loads)]
+    ids = np.random.default_rng(n + 1).permutation(np.repeat(at, loads)).astype(np.uint32)
+    few = 4  # matrices that the experts share in turn: what they hold does not matter here, which one a row meets does
+
+    def stack(kind, seed, rows, columns):
+        return np.tile(synth.matrix(kind, seed, rows * few, columns).reshape(few, -1), (experts // few, 1)).reshape(-1)
+
+    gate, up, down = stack(12, 3451, hidden, channels), stack(12, 3452, hidden, channels), stack(dn_type, 3453, channels, hidden)
+    w = tsp.PlanarMoeWeights(gpu, 12, dn_type, channels, hidden, experts, gate, up, down)
+    x = synth.round_bf16(synth.activations_f32(3454 + n, (n, channels)))
+    y = tsp.planar_nax_grouped_moe(gpu, w, gpu.upload(ids), gpu.upload(x), n, 1, tsp.GroupedScratch(gpu, n, 1, experts, channels, hidden), y=gpu.full((n, channels), np.nan)).cpu().numpy()
+    assert gpu.error() == 0
+    # the declared staging of the kinds, as in test_grouped_moe_other_planar_kinds
+    _, declared = orc.moe_routed_reference(12, dn_type, gate, up, down, channels, hidden, experts, ids, n, 1, x, stage=4 | (8 if dn_type == 14 else 32), threads=8)
+    scale = np.maximum(1.0, np.sqrt((declared ** 2).mean(axis=1, keepdims=True)))
+    err = np.abs(y - declared) / np.maximum(scale, np.abs(declared))
+    assert float(np.median(err)) <= 2e-5 and float(err.max()) <= 4e-3 and nmse(y, declared) <= 1e-7  # the bounds of the cases above
 
 
 # the down kernel that keeps a task's h rows in LDS: one to six steps of 128 hidden units (six take the requests in two halves), one
@@ -981,9 +1006,9 @@ def test_grouped_moe_q6_down_items(gpu, tsp, orc, synth, experts):
     test_grouped_moe_2048_columns_few_rows(gpu, tsp, orc, synth, 90, 512, experts, 4)
 
 
-# loads on either side of six rows per expert, where 2048-column experts change their gate/up kernel, and of eight items of 128 channels to a
+# loads on either side of 32 rows per expert, where 2048-column experts change their gate/up kernel, and of eight items of 128 channels to a
 # compute unit, where 512 hidden units change their down kernel
-@pytest.mark.parametrize("n,hidden", [(20, 256), (250, 256), (20, 512), (250, 512)])
+@pytest.mark.parametrize("n,hidden", [(20, 256), (250, 256), (20, 512), (250, 512), (1040, 256)])
 def test_grouped_moe_rows_whatever_company(gpu, tsp, synth, n, hidden):
     """The always-on expert's rows have the bits of a separate call, whose two experts and one route a token choose other kernels than the 128
     experts that it rides with, and a token's rows have the bits that they have in a chunk of half the size."""

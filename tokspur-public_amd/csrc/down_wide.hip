@@ -3,8 +3,8 @@
 //
 // The launch is a stream of expert weights from HBM and of f32 results back to it; what it costs is how many requests are on
 // their way. Hence:
-//   * One persistent workgroup of eight waves per compute unit takes an equal contiguous share of the (task, 256 channels) items;
-//     consecutive shares go to one XCD. The task's <= 64 rows of h sit in LDS (80 KB at 640 hidden units), whole, so a wave sums a
+//   * One persistent workgroup of eight waves per compute unit takes a contiguous share of the (task, 256 channels) items, as long as everyone's
+//     (share_begin); consecutive shares go to one XCD. The task's <= 64 rows of h sit in LDS (80 KB at 640 hidden units), whole, so a wave sums a
 //     32-channel tile over all columns by itself: no partial results, and no barrier except where the task changes.
 //   * Weights are requested a whole tile ahead into registers (half a tile where all six steps would not fit them), a step of 128 columns
 //     as the step at hand frees them: 5 x 4 KB per wave in flight at 640 hidden units, whole 128-byte pieces of rows by neighbouring
@@ -82,10 +82,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 
     auto pass = [&](auto mt_tag) {
         constexpr int MT = decltype(mt_tag)::value;
-        const uint32_t of_kind = a.classes[MT - 1];
         const uint32_t* list = a.classes + 2 + (MT - 1) * bound;
-        const uint32_t items = of_kind * units;
-        const uint32_t it0 = uint32_t(uint64_t(items) * share / groups), it1 = uint32_t(uint64_t(items) * (share + 1) / groups);
+        constexpr ItemLengths kLengths = KIND == kQ8 ? ItemLengths{19, 4, 2} : ItemLengths{17, 3, 2};
+        const uint32_t it0 = share_begin<MT>(a.classes, units, share, groups, kLengths), it1 = share_begin<MT>(a.classes, units, share + 1, groups, kLengths);
         if (it0 >= it1) return;
         const uint32_t k0 = it0 / units, k1 = (it1 - 1) / units;  // first and last position in the kind's list
         auto first_unit = [&](uint32_t k) { return k == k0 ? it0 % units : 0; };

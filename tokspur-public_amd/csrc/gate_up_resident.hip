@@ -4,7 +4,7 @@
 // stream and keeps everything else off the memory pipeline:
 //
 //   * One persistent workgroup of eight waves per CU. The launch's work, the (task, 32 hidden units) items in task order,
-//     is cut into equal contiguous shares, one per workgroup; consecutive shares go to workgroups of the same XCD so that
+//     is cut into contiguous shares that take equally long, one per workgroup; consecutive shares go to workgroups of the same XCD so that
 //     the tasks of one expert meet in one L2.
 //   * The K dimension is split over the waves: wave w owns super-block w (columns 256 w .. 256 w + 255) of every weight
 //     row. Its A operands, the task's <= 64 activation rows of those 256 columns, are loaded ONCE per task into registers
@@ -19,12 +19,14 @@
 //     one barrier per tile, and the threads that hold gate and up of the same hidden units apply SwiGLU and store h / 256
 //     as halves, the format the down GEMM reads.
 //   * A wave issues at most one instruction every four cycles and two waves share a SIMD, so what a wave executes per
-//     tile is kept short: unpacking is one mask-or and one packed multiply-add per pair of weights, scales are set up two
+//     tile is kept short: unpacking is one mask and one packed multiply per pair of weights, scales are set up two
 //     sub-blocks at a time, the sigmoid uses the hardware exponential and reciprocal, every lane stores (rows a task
 //     does not have repeat its first row, value and slot alike), and the tasks of at most 32 rows run in a loop of their own that keeps
 //     every address in registers. Measured with the arithmetic, the requests or the barrier taken out in turn, no single
 //     one of them bounds the kernel: what is left is the chain of latencies of one tile (arrival, LDS, matrix results,
-//     barrier, sum) at two waves per SIMD.
+//     barrier, sum) at two waves per SIMD. 203 tokens, 512 experts of 2048 x 512 (562 MB): 126 us with an equal part of either kind of task for every
+//     workgroup, of which four in ten met a large one and ended 15 us behind the others, 113 with equal parts of both on one line (share_begin; 105 the median
+//     workgroup, 5.3 TB/s).
 #include "gate_up_resident.hpp"
 #include "mfma_quant.hpp"
 #include "resident_tasks.hpp"
@@ -99,14 +101,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     const Q4ScaleConsts q4s = q4_scale_consts();
 
     // The tasks come in two kinds, those of at most 32 rows (one row tile: 64 registers of activations) and those of 33..64
-    // (two row tiles, 128 registers), each with its own loop so that neither carries the other's registers. A workgroup takes
-    // the same share of either kind's (task, unit) items: equal work for every workgroup whatever the mix of kinds.
+    // (two row tiles, 128 registers), each with its own loop so that neither carries the other's registers. A workgroup's
+    // share of the items takes as long as everyone's, whatever the mix of kinds (share_begin).
     auto pass = [&](auto mt_tag) {
         constexpr int MT = decltype(mt_tag)::value;
-        const uint32_t of_kind = a.classes[MT - 1];
         const uint32_t* list = a.classes + 2 + (MT - 1) * bound;
-        const uint32_t items = of_kind * units;
-        const uint32_t it0 = uint32_t(uint64_t(items) * share / groups), it1 = uint32_t(uint64_t(items) * (share + 1) / groups);
+        constexpr ItemLengths kLengths{25, 40, 11};
+        const uint32_t it0 = share_begin<MT>(a.classes, units, share, groups, kLengths), it1 = share_begin<MT>(a.classes, units, share + 1, groups, kLengths);
         if (it0 >= it1) return;
         const uint32_t k0 = it0 / units, k1 = (it1 - 1) / units;  // first and last position in the kind's list
         auto first_unit = [&](uint32_t k) { return k == k0 ? it0 % units : 0; };

@@ -964,11 +964,12 @@ int grouped_moe(const tsp_grouped_moe* m, const tsp_shared_expert* shared, void*
     auto* task_list = reinterpret_cast<uint32_t*>(ws + l.tasks);
     auto* hbuf = reinterpret_cast<_Float16*>(ws + l.hbuf);
 
-    // Few rows per expert: the launch is bound by HBM, and the resident kernel's shares of 32 units leave no compute unit waiting for
-    // another (a sublayer of 2048 x 512, 512 experts: 20 tokens 102 us against 114, 100 tokens 216 against 220; 400 tokens 302 against 295, 2048
-    // tokens 478 against 449; 2048 x 768, 128 experts: 50 tokens 143 against 145, 100 tokens 152 against 151, 2048 tokens 408 against 383).
+    // At 2048 columns the resident kernel's parts end together however few the tasks are, and it asks for a task's weights without a start per 128
+    // units; with many rows per expert its exchange between the waves weighs more. A sublayer, resident and streaming: 2048 x 512, 512 experts, 20 tokens 97 us and
+    // 106, 50 152 and 163, 120 214 and 223, 260 255 and 266, 600 310 and 316, 1000 339 and 348, 2048 446 and 443; 2048 x 768, 128 experts, 30 125 and 136,
+    // 150 165 and 173, 500 (31 routes an expert) 203 and 204, 1000 280 and 273.
     // The two add a row's super-blocks up in the same order and with the same roundings.
-    const bool stream_gate_up = fast_gate_up && !(routes < 6 * m->experts && resident_gate_up_takes(m->channels, m->hidden));
+    const bool stream_gate_up = fast_gate_up && !(routes < 32 * m->experts && resident_gate_up_takes(m->channels, m->hidden));
     auto* order = reinterpret_cast<OrderedTask*>(ws + l.order);
     // only the Q4_K gate/up kernels want the activation sums and the column order that goes with them
     rc = prepare_grouped(TaskLists{m->ids, m->token_map, m->counts, m->tasks, 32, task_list, kTaskRows, m->experts, m->selected, m->tokens, shared != nullptr,

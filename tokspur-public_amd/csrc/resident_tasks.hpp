@@ -44,4 +44,21 @@ __device__ __forceinline__ ResidentTask resolve_resident_task(const uint32_t* __
     return t;
 }
 
+// A persistent workgroup's part of a launch's (task, unit) items, of which the tasks of 33 to 64 rows come first and then those of fewer: both
+// kinds lie on one line, which is cut into equal parts. Lengths, in sixteenths of a small task's item: what a kernel takes for a
+// large task's item, and what for the first of a large or small task's on top (rows, tables, the pipeline's start). Most workgroups so work
+// on one kind only, and the two, of which one has more to compute and the other more to fetch in the same time, run side by side. (An equal part
+// of either kind for everyone was a second start, some 15 us, for whoever met a large task at all.) Figures at the kernels; the lengths are least-squares
+// fits to the workgroups' times at 60 to 2048 tokens.
+struct ItemLengths { uint32_t large, large_start, small_start; };
+template <int MT>
+__device__ __forceinline__ uint32_t share_begin(const uint32_t* __restrict__ classes, uint32_t units, uint32_t share, uint32_t groups, const ItemLengths& l) {
+    const uint32_t large_task = units * l.large + l.large_start, small_task = units * 16 + l.small_start, all_large = classes[1] * large_task;
+    const uint32_t at = uint32_t(uint64_t(all_large + classes[0] * small_task) * share / groups);  // at most 1056 tasks of 2048 units
+    const uint32_t task = MT == 2 ? large_task : small_task, item = MT == 2 ? l.large : 16, start = MT == 2 ? l.large_start : l.small_start;
+    const uint32_t from = MT == 2 ? (at < all_large ? at : all_large) : (at > all_large ? at - all_large : 0);
+    const uint32_t k = from / task, into = from - k * task;
+    return k * units + (into > start ? (into - start + item - 1) / item : 0);  // the items that begin ahead of the cut
+}
+
 }  // namespace tsp
