@@ -259,6 +259,28 @@ def test_mixture_golden_and_rows(gpu, orc, synth):
     assert (out[:, channels:] == -3.0).all() and gpu.error() == 0
 
 
+@pytest.mark.parametrize("selected", [8, 10, 3])
+@pytest.mark.parametrize("channels", [4, 508, 512, 516])
+def test_mixture_block_edges(gpu, tsp, orc, synth, selected, channels):
+    # four channels a thread at the edges of a block's 128 threads, and a token whose shared logit is infinite: that one
+    # is reported and its row left alone, the others are right. A sum of S + 1 terms in float32 errs by at most
+    # (S + 3) * 2^-24 of the terms' magnitudes, the sigmoid by 4 * 2^-24 of its term.
+    tokens = 3
+    ex = synth.activations_f32(5, (tokens, selected, channels))
+    w = np.abs(synth.activations_f32(6, (tokens, selected))) / 10
+    sh = synth.activations_f32(7, (tokens, channels))
+    sl = synth.activations_f32(8, tokens)
+    sl[1] = np.inf
+    out = gpu.full((tokens, channels), -3.0)
+    gpu.mixture(gpu.upload(ex), gpu.upload(w), gpu.upload(sh), gpu.upload(sl), channels, selected, tokens, out=out)
+    out = out.cpu().numpy()
+    assert gpu.error() == tsp.ERRBIT_NONFINITE and (out[1] == -3.0).all()
+    for t in (0, 2):
+        want = orc.mixture_reference(ex[t].astype(np.float64), w[t].astype(np.float64), sh[t].astype(np.float64), float(sl[t]))
+        size = np.abs(sh[t]).astype(np.float64) + (np.abs(ex[t]) * w[t][:, None]).astype(np.float64).sum(0)
+        assert (np.abs(out[t] - want) <= (selected + 7) * 2.0 ** -24 * size).all()
+
+
 def test_mixture_errors(gpu, tsp):
     one = gpu.upload(np.ones(4, dtype=np.float32))
     gpu.mixture(gpu.upload(np.ones(8, dtype=np.float32)), gpu.upload(np.array([0.5, -0.5], dtype=np.float32)), one,
