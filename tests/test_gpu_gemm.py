@@ -794,6 +794,36 @@ def test_grouped_moe_parts_of_a_launch(gpu, tsp, orc, synth, dn_type, channels, 
     assert float(np.median(err)) <= 2e-5 and float(err.max()) <= 4e-3 and nmse(y, declared) <= 1e-7  # the bounds of the cases above
 
 
+# tasks at the edges of a row tile, one to sixty-four rows of it live, in rows further apart than they are long: a row past a task's
+# end is zeros in and dropped on the way out, so what lies between the rows stays as it was. Resident and streaming gate/up, the two persistent down kernels
+@pytest.mark.parametrize("dn_type,channels,hidden,experts", [(14, 2048, 512, 128), (8, 2048, 512, 128), (14, 256, 256, 8), (8, 768, 384, 8), (7, 2048, 640, 8)])
+def test_grouped_moe_rows_past_the_end(gpu, tsp, orc, synth, dn_type, channels, hidden, experts):
+    loads = (1, 31, 32, 33, 63, 64, 65)
+    n = sum(loads)
+    ids = np.random.default_rng(77).permutation(np.repeat(np.random.default_rng(78).permutation(experts)[:len(loads)], loads)).astype(np.uint32)
+
+    def stack(kind, seed, rows, columns):  # four matrices that the experts share in turn
+        return np.tile(synth.matrix(kind, seed, rows * 4, columns).reshape(4, -1), (experts // 4, 1)).reshape(-1)
+
+    gate, up, down = stack(12, 3461, hidden, channels), stack(12, 3462, hidden, channels), stack(dn_type, 3463, channels, hidden)
+    w = tsp.PlanarMoeWeights(gpu, 12, dn_type, channels, hidden, experts, gate, up, down)
+    x = synth.round_bf16(synth.activations_f32(3464, (n, channels)))
+    scratch = tsp.GroupedScratch(gpu, n, 1, experts, channels, hidden)
+    results = []
+    for fill in (0.0, np.nan):  # what an earlier call has left in the scratch does not reach the results
+        scratch.workspace.view(dtype=gpu.zeros(1).dtype).fill_(fill)
+        y = gpu.full((n + 1, channels + 8), -7.0)
+        tsp.planar_nax_grouped_moe(gpu, w, gpu.upload(ids), gpu.upload(x), n, 1, scratch, y=y, y_stride=(channels + 8) * 4)
+        y = y.cpu().numpy()
+        assert gpu.error() == 0 and (y[n] == -7.0).all() and (y[:, channels:] == -7.0).all()
+        results.append(y[:n, :channels])
+    assert np.array_equal(results[0].view(np.uint32), results[1].view(np.uint32))
+    _, declared = orc.moe_routed_reference(12, dn_type, gate, up, down, channels, hidden, experts, ids, n, 1, x, stage=4 | (8 if dn_type == 14 else 32), threads=8)
+    scale = np.maximum(1.0, np.sqrt((declared ** 2).mean(axis=1, keepdims=True)))
+    err = np.abs(results[0] - declared) / np.maximum(scale, np.abs(declared))
+    assert float(np.median(err)) <= 2e-5 and float(err.max()) <= 4e-3 and nmse(results[0], declared) <= 1e-7  # the bounds of the cases above
+
+
 # the down kernel that keeps a task's h rows in LDS: one to six steps of 128 hidden units (six take the requests in two halves), one
 # and three groups of 256 channels, tasks of one and of two row tiles
 @pytest.mark.parametrize("dn_type,channels,hidden", [(8, 256, 128), (7, 768, 128), (7, 256, 384), (8, 768, 384), (8, 256, 768), (7, 768, 768)])

@@ -16,7 +16,7 @@ struct ResidentDownArgs {
     const uint32_t* token_map;
     const uint32_t* ids;
     uint32_t task_slots;
-    float* y;                    // [tokens * selected] rows by route, y_stride bytes apart; the whole output spans less than 4 GiB
+    float* y;                    // [tokens * selected] rows by route, y_stride bytes apart; the whole output spans less than 0xffffff00 bytes, and so does shared_y
     uint64_t y_stride;
     uint32_t out_bytes;          // y from its first row's first byte to its last row's last
     float* shared_y;             // the always-on expert's rows by token

@@ -11,15 +11,15 @@
 //     lanes. They turn into fragment order through 4 KB (2 KB) of LDS of the wave's own.
 //   * A tile's results are stored at the beginning of the next one: then the requests outstanding at the head of the loop are the same
 //     from wherever it is entered, and each wait counts exactly. In a task's first round there are none: the buffer they go to
-//     has no bytes, and the hardware drops them. Rows a task does not have go past its end likewise.
+//     has no bytes, and the hardware drops them. Rows a task does not have go past its end likewise; they come from past the end of the
+//     h rows' buffer, as zeros, which take the least power to multiply (a first row repeated: 742.9 us a sublayer as below, now 740.7).
 //   * A weight is the half nearest to d * q (d * q + m), the engine's arithmetic for these kinds: one packed half operation, one
 //     rounding.
 //   * Where the task changes, the next one's rows are on their way before the last results of the old one are stored.
 //
 // Measured (2048 tokens, 512 experts of 2560 x 640, ten selected, 615 tasks; 891 MB of Q8_0 weights and 210 MB of results): 250 us,
 // where the staged kernel's short-lived workgroups took 495 (planar_staged.hip, which stays for other widths). Bound by the
-// stream: 4.9 TB/s counting the rows of heavy experts that are read once per task. Q8_0 at 640 hidden units takes all 256 registers and five
-// in scratch, read again where the task changes.
+// stream: 4.9 TB/s counting the rows of heavy experts that are read once per task.
 #include "down_resident.hpp"
 #include "mfma_quant.hpp"
 #include "resident_tasks.hpp"
@@ -219,11 +219,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         u32x4 piece[kBatch];
         uint32_t route = 0;
         auto request_rows = [&](const ResidentTask& t, int from) {
-            const uint8_t* const src = reinterpret_cast<const uint8_t*>(a.hbuf) + uint64_t(t.task) * (kTaskRows * kColumns * 2);
+            __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(reinterpret_cast<const uint8_t*>(a.hbuf)) + uint64_t(t.task) * (kTaskRows * kColumns * 2), 0, int(t.nrows * (kColumns * 2)), 0x00020000);
 #pragma unroll
-            for (int j = 0; j < kBatch; ++j) {  // a row past the end repeats the first
+            for (int j = 0; j < kBatch; ++j) {  // a row past the end lies past the buffer's and is zeros
                 const uint32_t c = tid + (from + j) * kThreads, r = c / (STEPS * 16);
-                if (from + j < kPieces) piece[j] = *reinterpret_cast<const u32x4*>(src + (r < t.nrows ? r : 0) * (kColumns * 2) + c % (STEPS * 16) * 16);
+                if (from + j < kPieces) piece[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(src, r * (kColumns * 2) + c % (STEPS * 16) * 16, 0, 0));
             }
         };
         auto put_rows = [&](int from) {

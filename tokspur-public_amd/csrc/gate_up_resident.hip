@@ -21,12 +21,13 @@
 //   * A wave issues at most one instruction every four cycles and two waves share a SIMD, so what a wave executes per
 //     tile is kept short: unpacking is one mask and one packed multiply per pair of weights, scales are set up two
 //     sub-blocks at a time, the sigmoid uses the hardware exponential and reciprocal, every lane stores (rows a task
-//     does not have repeat its first row, value and slot alike), and the tasks of at most 32 rows run in a loop of their own that keeps
+//     does not have, zeros, go past the end of its buffer and are dropped), and the tasks of at most 32 rows run in a loop of their own that keeps
 //     every address in registers. Measured with the arithmetic, the requests or the barrier taken out in turn, no single
 //     one of them bounds the kernel: what is left is the chain of latencies of one tile (arrival, LDS, matrix results,
 //     barrier, sum) at two waves per SIMD. 203 tokens, 512 experts of 2048 x 512 (562 MB): 126 us with an equal part of either kind of task for every
 //     workgroup, of which four in ten met a large one and ended 15 us behind the others, 113 with equal parts of both on one line (share_begin; 105 the median
-//     workgroup, 5.3 TB/s).
+//     workgroup, 5.3 TB/s). In a row of launches the clock goes by the power and that is 133; 127 with zeros for the rows a task does not have, where
+//     copies of its first row were.
 #include "gate_up_resident.hpp"
 #include "mfma_quant.hpp"
 #include "resident_tasks.hpp"
@@ -163,9 +164,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                 const uint32_t r = i * 32 + n, rr = r < cur.nrows ? r : 0;
                 rid[i] = cur.shared ? 0 : a.token_map[uint64_t(cur.expert) * a.tokens + cur.start + rr];
                 token[i] = cur.shared ? cur.start + rr : rid[i] / a.selected;
-                // A row past the task's end repeats its first row (and stores what it computes, the first row's h, to the first
-                // row's slot), and a route outside the batch stands in for token 0 (the batch is refused). So every lane stores,
-                // every wave issues the same number of stores per unit, and the waits below can count them.
+                // A route outside the batch stands in for token 0 (the batch is refused).
                 if (!cur.shared && rid[i] >= a.tokens * a.selected) { rid[i] = 0; token[i] = 0; if (cur.ok) bad |= TSP_ERRBIT_INDEX; }
                 if (!cur.ok) token[i] = 0;
             }
@@ -175,8 +174,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                 owner[i] = cur.shared ? cur.expert : a.ids[rid[i]];
                 const _Float16* row = a.xh + uint64_t(token[i]) * (bpr * 256) + wave * 256 + khalf * 16;
 #pragma unroll
-                for (int t = 0; t < 16; ++t) A[i][t] = *reinterpret_cast<const f16x8*>(row + (t / 4) * 64 + ((t / 2) % 2) * 32 + (t % 2) * 8);
-                sxA[i] = *reinterpret_cast<const f16x8*>(a.sx + (uint64_t(token[i]) * bpr + wave) * 16 + khalf * 8);
+                for (int t = 0; t < 16; ++t) A[i][t] = f16x8{};  // a row past the task's end: products of zeros take the least power
+                sxA[i] = f16x8{};
+                if (i * 32 + n < cur.nrows) {
+#pragma unroll
+                    for (int t = 0; t < 16; ++t) A[i][t] = *reinterpret_cast<const f16x8*>(row + (t / 4) * 64 + ((t / 2) % 2) * 32 + (t % 2) * 8);
+                    sxA[i] = *reinterpret_cast<const f16x8*>(a.sx + (uint64_t(token[i]) * bpr + wave) * 16 + khalf * 8);
+                }
             }
 #pragma unroll
             for (int i = 0; i < MT; ++i)
@@ -275,6 +279,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                     // element 2 tid + e of the tile is accumulator 4 (wave / 2) + 2 (lane % 2) + e of fragment lane
                     // 32 (wave % 2) + lane / 2: task row 32 i + 4 wave + 2 (lane % 2) + e, hidden unit lane / 2 of the tile
                     const float up_sum[2] = {s0, s1};
+                    __amdgpu_buffer_rsrc_t h_rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16*>(a.hbuf) + uint64_t(task) * kTaskRows * a.hidden, 0, int(task_rows * a.hidden * 2), 0x00020000);
 #pragma unroll
                     for (int e = 0; e < 2; ++e) {
                         const uint32_t r = i * 32 + 4 * wave + 2 * (lane_now % 2) + e;
@@ -285,13 +290,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                         const _Float16 carried = _Float16(h * 0.00390625f);
                         const uint32_t bits = __builtin_bit_cast(uint16_t, carried), magnitude = bits & 0x7fffu;
                         biggest = biggest > magnitude ? biggest : magnitude;
-                        // uniform base (the task's slots, the unit's columns) + 32-bit lane offset, spelled out: the compiler would
-                        // form a 64-bit address per store
-                        // a row past the task's end has multiplied the first row's activations: the same bits, stored to the first
-                        // row's slot, so that the slots nobody reads cost no traffic (and every lane still stores)
-                        const uint32_t at = ((r < task_rows ? r : 0) * a.hidden + lane_now / 2) * 2;
-                        const _Float16* const base = a.hbuf + (uint64_t(task) * kTaskRows) * a.hidden + unit * 32;
-                        asm volatile("global_store_short %0, %1, %2" ::"v"(at), "v"(bits), "s"(base) : "memory");
+                        // The buffer ends with the task's last row, so a row past it is dropped, and every wave still issues the same
+                        // number of stores per unit: the waits above count them.
+                        __builtin_amdgcn_raw_buffer_store_b16(uint16_t(bits), h_rows, (r * a.hidden + lane_now / 2) * 2, unit * 64, 0);
                     }
                 }
             }

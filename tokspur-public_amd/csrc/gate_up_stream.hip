@@ -24,7 +24,9 @@
 // in turn on another box: 203 -> 191 (2048 x 512), 290 -> 281. Bound by what it fetches and by its instructions at once (2048 x 512 and 2560 x 640): 0.91 and 1.36 GB,
 // the planes once per task, the headers' lines twice, 0.1 GB of rows, in 167 and 250 us without any arithmetic (5.4 TB/s); the arithmetic alone
 // takes 158 and 215 with nothing to wait for, 40 and 46 of it where a super-block's sums are scaled and added. Barriers and reads of rows from LDS are free.
-// Tried: persistent workgroups that request the next item's bytes during the last steps of this
+// Rows past a task's end are zeros: in a run of launches the clock goes by the power, 189 us after a pause and 213 in a row, and there rows of
+// zeros are cheap products (a first row repeated: 213 -> 209, 295 -> 292 at 2560 x 640).
+// Tried: the minima's products a group ahead of their use (the other workgroup's wave fills that time already), persistent workgroups that request the next item's bytes during the last steps of this
 // one (298 for 270), tasks of more than 32 rows first (280), nibbles' lines as non-temporal (285), an expert's tasks on one column tile side by side (they do not
 // meet in L2 either: as many bytes).
 #include "gate_up_resident.hpp"
@@ -45,6 +47,11 @@ static_assert(kLdsBytes <= 80 * 1024, "two workgroups per compute unit");
 
 __device__ __forceinline__ void load_to_lds_4(const void* uniform_base, uint32_t lane_offset, uint32_t lds_base) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds_base), "v"(lane_offset), "s"(uniform_base) : "memory", "m0");
+}
+
+// The same from a buffer: a lane whose offset lies past its end brings zeros, and costs no fetch.
+__device__ __forceinline__ void buffer_to_lds_16(u32x4 buffer, uint32_t lane_offset, uint32_t offset, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds_base), "v"(lane_offset), "s"(buffer), "s"(offset) : "memory", "m0");
 }
 
 // BY_BLOCKS: super-blocks are summed by themselves and then added up, in order, as the resident kernel's waves do, and with its roundings: a row's
@@ -104,7 +111,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     request_lines(up, 0, up_at);
     request_headers(0);
 
-    // ---- the task's rows: a row past the end repeats the first one and is not stored; a route that is not the expert's shows behind the first wait,
+    // ---- the task's rows: a row past the end is zeros and not stored (its sums are the first row's); a route that is not the expert's shows behind the first wait,
     // and the batch is refused. Activations: instruction i covers rows 8 wave + 32 i .. + 7, eight lanes per row; sums: 16 bytes each of 64 rows x 32, sixteen rows per wave.
     uint32_t bad = 0;
     const uint32_t my_rows[3] = {wave * 8 + lane / 8, wave * 8 + lane / 8 + 32, wave * 16 + col / 2};
@@ -126,7 +133,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const uint32_t a_chunk = ((lane % 8) ^ ((4 * wave + lane / 16) % 8)) * 16;
     uint32_t a_lane[2];  // byte offsets: 2048 tokens of 65536 channels at most
 #pragma unroll
-    for (uint32_t i = 0; i < 2; ++i) a_lane[i] = token[i] * (a.channels * 2) + a_chunk;
+    for (uint32_t i = 0; i < 2; ++i) a_lane[i] = my_rows[i] < t.nrows ? token[i] * (a.channels * 2) + a_chunk : 0x80000000u;
+    const uint64_t x_at = reinterpret_cast<uint64_t>(a.xh);
+    const u32x4 x_rows{uint32_t(x_at), uint32_t(x_at >> 32) & 0xffffu, a.tokens * a.channels * 2, 0x00020000u};
     const uint32_t s_lane = token[2] * (bpr * 32) + (col % 2) * 16;
     auto request_sums = [&](uint32_t b) { if (lane < 32) load_to_lds_16(reinterpret_cast<const uint8_t*>(a.sx) + b * 32, s_lane, lds_at + kSumsAt + wave * 512); };
 
@@ -140,9 +149,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     auto run = [&](auto tiles_tag) {
         constexpr int MT = decltype(tiles_tag)::value;
         auto request_rows = [&](uint32_t step, uint32_t slab) {
-            const uint8_t* base = reinterpret_cast<const uint8_t*>(a.xh) + uint64_t(min(step, steps - 1)) * 128;
+            const uint32_t at = min(step, steps - 1) * 128;
 #pragma unroll
-            for (int i = 0; i < MT; ++i) load_to_lds_16(base, a_lane[i], lds_at + slab + i * 4096 + wave * 1024);
+            for (int i = 0; i < MT; ++i) buffer_to_lds_16(x_rows, a_lane[i], at, lds_at + slab + i * 4096 + wave * 1024);
         };
         uint32_t slab = 0, slab1 = kSlab, slab2 = 2 * kSlab;  // this step's, the next, the one after
         request_rows(0, slab);

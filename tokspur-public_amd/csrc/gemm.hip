@@ -1009,7 +1009,7 @@ int grouped_moe(const tsp_grouped_moe* m, const tsp_shared_expert* shared, void*
     // experts of 2048, a sublayer of 600 tokens 396 and 391 us, of 2048 528 and 540). A row's bits are the same from either.
     const bool wide_fits = wide_down_takes(down_type, m->channels, m->hidden) && y_span <= 0xffff0000u;
     const bool wide_first = wide_fits && small && routes >= m->experts;
-    const bool resident = !brief && !wide_first && resident_down_takes(down_type, m->channels, m->hidden) && uint64_t(routes) * m->y_stride_bytes < (1ull << 32) && shared_span < (1ull << 32);
+    const bool resident = !brief && !wide_first && resident_down_takes(down_type, m->channels, m->hidden) && uint64_t(routes) * m->y_stride_bytes < 0xffffff00u && shared_span < 0xffffff00u;
     const bool wide = !resident && wide_fits;
     if (resident || wide) {
         ResidentDownArgs r{};
