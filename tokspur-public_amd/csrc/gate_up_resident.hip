@@ -12,7 +12,9 @@
 //     read twice per task and none passes through LDS.
 //   * Weights go global -> LDS directly (no registers in between), a tile of 32 rows x one 128-byte line of nibbles +
 //     the rows' scale bytes and d/dmin per request, into a wave-private ring of two stages. Eight neighbouring lanes fetch
-//     one whole cache line. Nothing but these requests and the epilogue's stores uses the vector memory counter inside
+//     one whole cache line, of which few are wanted twice (an expert with so few rows has one task): they pass by the caches, 203 tokens of
+//     2048 x 512 235.3 -> 227.1 us a sublayer. (The down kernels and the streaming gate/up lose by it, 143 -> 168 us and 278 -> 285 a launch: there
+//     tasks of one expert and waves side by side share lines.) Nothing but these requests and the epilogue's stores uses the vector memory counter inside
 //     the loop, so each wave waits with an exact count, and since the ring is private no barrier guards it.
 //   * A wave's product over its super-block, d * sum(x * sc*q) - dmin * sum(Sx * mn), is a partial result of a 32 x 32
 //     tile; the eight partials add up through LDS in wave order (a fixed order: results are reproducible bit for bit) with
@@ -92,7 +94,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         const uint8_t* qs = base + uint64_t(unit) * (32 * bpr * 128);
         const uint32_t dst = my_stage_lds + stage_offset;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) load_to_lds_16(qs + q * (8 * bpr * 128), qs_lane, dst + q * 1024);
+        for (int q = 0; q < 4; ++q) load_once_to_lds_16(qs + q * (8 * bpr * 128), qs_lane, dst + q * 1024);
         load_to_lds_16(base, hdr_lane + unit * hdr_unit_step, dst + 4096);
     };
 

@@ -965,9 +965,9 @@ int grouped_moe(const tsp_grouped_moe* m, const tsp_shared_expert* shared, void*
     auto* hbuf = reinterpret_cast<_Float16*>(ws + l.hbuf);
 
     // At 2048 columns the resident kernel's parts end together however few the tasks are, and it asks for a task's weights without a start per 128
-    // units; with many rows per expert its exchange between the waves weighs more. A sublayer, resident and streaming: 2048 x 512, 512 experts, 20 tokens 97 us and
-    // 106, 50 152 and 163, 120 214 and 223, 260 255 and 266, 600 310 and 316, 1000 339 and 348, 2048 446 and 443; 2048 x 768, 128 experts, 30 125 and 136,
-    // 150 165 and 173, 500 (31 routes an expert) 203 and 204, 1000 280 and 273.
+    // units; with many rows per expert its exchange between the waves weighs more. A sublayer, resident and streaming: 2048 x 512, 512 experts, 260 tokens 252 us and
+    // 262, 400 270 and 282, 600 302 and 317, 1000 340 and 348, 1400 (27 routes an expert) 380 and 381, 1800 425 and 419, 2048 449 and 440; 2048 x 768,
+    // 128 experts, 150 162 and 171, 400 186 and 192, 500 (31) 199 and 202, 700 234 and 233, 1000 277 and 271, 1500 354 and 335.
     // The two add a row's super-blocks up in the same order and with the same roundings.
     const bool stream_gate_up = fast_gate_up && !(routes < 32 * m->experts && resident_gate_up_takes(m->channels, m->hidden));
     auto* order = reinterpret_cast<OrderedTask*>(ws + l.order);

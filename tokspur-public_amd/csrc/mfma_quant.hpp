@@ -42,6 +42,10 @@ __device__ __forceinline__ void load_to_lds_16(const void* src, uint32_t lds_bas
 __device__ __forceinline__ void load_to_lds_16(const void* uniform_base, uint32_t lane_offset, uint32_t lds_base) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(lane_offset), "s"(uniform_base) : "memory", "m0");
 }
+// The same for whole lines that hardly anyone will want again: they don't take the place of others in the caches.
+__device__ __forceinline__ void load_once_to_lds_16(const void* uniform_base, uint32_t lane_offset, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds_base), "v"(lane_offset), "s"(uniform_base) : "memory", "m0");
+}
 __device__ __forceinline__ uint32_t lds_address(const void* p) {
     return uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)p));
 }
