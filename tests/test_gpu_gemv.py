@@ -289,6 +289,23 @@ def test_dense_mm_q8_staged_tiles(gpu, tsp, synth, tokens, cols, rows):
     assert (np.abs(got - x.astype(np.float64) @ weight.T) <= bound).all() and gpu.error() == 0
 
 
+@pytest.mark.parametrize("tokens,cols,rows,pad", [(33, 64, 33, 0), (63, 2624, 31, 1), (100, 704, 2500, 0), (203, 704, 2500, 3), (1984, 1088, 600, 0), (1990, 704, 2040, 1),
+                                                  (2047, 192, 2050, 0)])
+def test_dense_mm_q8_staged_tile_shapes(gpu, tsp, synth, tokens, cols, rows, pad):
+    # every tile that raw rows are decoded in (32 x 32, 32 x 32, 32 x 64, 64 x 64, 64 x 96, 128 x 128) and the two launches: ragged edges, a last step of 64 columns, a single
+    # step, rows four bytes off a multiple of sixteen. The bound is that of test_dense_mm_q8_staged_tiles.
+    w = synth.matrix(8, 2500 + cols, rows, cols)
+    x = synth.activations_f32(2501 + tokens, (tokens, cols + pad))
+    out = gpu.full((tokens, rows + 3), -5.0)
+    tsp.dense_mm_q8_staged(gpu, tsp.LAYOUT_GGUF, gpu.upload(w), gpu.upload(x), tokens, cols, rows, out=out, x_stride=(cols + pad) * 4, out_stride=(rows + 3) * 4)
+    got, x = out.cpu().numpy(), x[:, :cols].astype(np.float64)
+    blocks = w.reshape(rows, -1, 34)
+    weight = blocks[:, :, 2:].view(np.int8).astype(np.float64) * np.ascontiguousarray(blocks[:, :, :2]).view(np.float16).astype(np.float64)
+    weight = weight.reshape(rows, cols)
+    bound = (2.0 ** -10 + cols * 2.0 ** -24) * (np.abs(x) @ np.abs(weight).T)
+    assert (np.abs(got[:, :rows] - x @ weight.T) <= bound).all() and (got[:, rows:] == -5.0).all() and gpu.error() == 0
+
+
 @pytest.mark.parametrize("tokens,cols,rows,pad", [(2, 64, 1, 0), (7, 640, 33, 0), (8, 2560, 640, 0), (9, 320, 18, 0), (16, 1088, 47, 12), (5, 2048, 160, 4),
                                                   (23, 2560, 48, 0), (3, 96, 20, 0), (6, 512, 24640, 0), (15, 512, 14020, 0), (11, 1280, 14001, 0),
                                                   (7, 2560, 24577, 0), (14, 2560, 14004, 0), (27, 1024, 14004, 0), (41, 192, 30, 4),

@@ -5,9 +5,8 @@
 // kernel stages, include/tokspur/graph.hpp:860 and kernels/grouped_mm.metal:239-243), the token rows are rounded to halves as
 // well, and the matrix cores multiply the two with f32 accumulation.
 //
-// A short chunk goes through one kernel that decodes both operands on their way into the MFMAs (q8_gemm_split, raw rows). With more
-// tokens every operand would be decoded again and again, ten to forty times over, so one launch decodes both into the workspace and
-// f16_gemm_nt multiplies them.
+// GGUF rows whose tiles go round the chip well are decoded on their way into the MFMAs, together with the token rows (q8_gemm_fused). Else every operand would be
+// decoded too often or much of the chip stand idle: one launch decodes both into the workspace and f16_gemm_nt multiplies them.
 //
 // f16_gemm_nt: a workgroup of four waves owns a 64 x 64 output tile (each wave a 32 x 32 MFMA tile) and walks K in
 // steps of 64 halfs. Every byte travels global -> LDS directly (16 bytes per lane, no registers in between) into a ring
@@ -119,102 +118,162 @@ __global__ __launch_bounds__(256, 2) void f16_gemm_nt(F16GemmArgs a) {
     publish_error(bad, a.error_word);
 }
 
-// A workgroup is one 32 x 32 output tile and its waves take the columns in turns of 64: a chunk of 64 tokens against 640 rows is 40
-// workgroups of eight waves, each wave a chain of five steps. A wave reads a step as it lies (256 bytes of 32 token rows,
-// 17 dwords of 32 weight rows), two steps' requests in flight, and puts it into fragment order through LDS of its own: no barrier
-// until the waves' sums meet, which are added in wave order.
-// Bound by latency: 60 tokens, 2560 -> 640 columns 8.8 us, 640 -> 2560 4.9 (two conversions and a GEMM: 18.7 and 14.4).
-template <int WAVES>
-__global__ __launch_bounds__(WAVES * kWave, 4) void q8_gemm_split(Q8GemmArgs a) {
-    constexpr uint32_t kEdge = 32, kDwords = 17, kWLoads = (kEdge * kDwords + kWave - 1) / kWave, kPitch = kStep + 8;
-    struct WaveLds {
-        _Float16 x[kEdge * kPitch];
-        uint32_t w[kWLoads * kWave];
-    };
-    static_assert(sizeof(WaveLds) >= kEdge * kEdge * 4);
-    __shared__ __attribute__((aligned(16))) WaveLds lds[WAVES];
+using four_floats = f32x4 __attribute__((aligned(4)));
+using four_quants = uint32_t __attribute__((aligned(2)));  // rows and blocks are even byte counts
+
+// GGUF rows and a tile to nearly every compute unit: a workgroup of eight waves owns an MT x NT output tile and takes 128 columns a step. A thread reads eight
+// columns of each 32nd row as they lie (32 bytes of a token row, eight quants and their scale of a matrix row), rounds them to halves and puts them into
+// LDS, DEPTH steps' requests in registers; the waves multiply from there, WM x WN of them side by side and every such group a share of
+// the step's columns, whose sums meet in LDS in the groups' order. Chunk c (16 bytes) of row r sits at position c ^ (r % 16) of the
+// row's 256 bytes: sixteen consecutive lanes touch every bank once, writing and reading. Fragments are requested from LDS before the next step's
+// operands are rounded, and multiplied after that.
+// Bound by a step's chain, some 6 ns for each of the tile's rows, whether the rest of the chip has work or not. Against the 32 x 32 tiles whose waves took 64 columns in turns, or
+// above 600 of them the two launches below, per call, tokens x columns -> rows: 203 x 2560 -> 640 10.2 -> 9.0 us, 450 16.9 -> 12.6, 600 17.5 -> 12.9, 1000
+// 18.9 -> 17.8, 2048 25.1 -> 23.2; 450 x 2048 -> 512 9.9 -> 8.2, 2048 18.4 -> 15.5; 203 x 640 -> 2560 8.6 -> 7.4; 2048 x 768 -> 2048 24.2 -> 19.3. Tried: token rows
+// sixteen bytes to a lane and sixteen quants to a load (2048 x 2560 -> 640 27), operands straight into LDS of the wave that multiplies them (24), the
+// matrix in fragment order by a launch before (22, but 32 for 24.9 at 640 x 2560).
+template <int MT, int NT, int WM, int WN, int DEPTH, int WAVES_PER_SIMD>
+struct FusedShape {
+    static constexpr int kM = MT, kN = NT, kDepth = DEPTH, kRowTiles = MT / 32 / WM, kColumnTiles = NT / 32 / WN, kGroups = 8 / (WM * WN), kPasses = kRowTiles * kColumnTiles;
+    static constexpr uint32_t kStage = (MT + NT) * 256, kLds = 2 * kStage > (kPasses > 1 ? 65536u : 32768u) ? 2 * kStage : (kPasses > 1 ? 65536u : 32768u);
+    static constexpr int kWavesM = WM, kWavesN = WN, kWavesPerSimd = WAVES_PER_SIMD;
+    static_assert(kRowTiles * WM * 32 == MT && kColumnTiles * WN * 32 == NT && kGroups * WM * WN == 8);
+};
+
+template <class S>
+__global__ __launch_bounds__(512, S::kWavesPerSimd) void q8_gemm_fused(Q8GemmArgs a) {
+    constexpr uint32_t MT = S::kM, NT = S::kN, XR = MT / 32, WR = NT / 32, TILES = S::kWavesM * S::kWavesN;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid / kWave)));
-    const uint32_t col = lane % 32, khalf = lane / 32;
-    const uint32_t m0 = blockIdx.y * kEdge, n0 = blockIdx.x * kEdge, steps = a.k / kStep, row_bytes = a.k / 32 * 34;
-    const uint8_t* const w_base = a.w + uint64_t(n0) * row_bytes;
-    uint32_t w_at[kWLoads];
+    // an XCD (workgroup id % 8) takes a run of tiles and with it an eighth of the larger operand and all of the smaller one into its L2
+    const uint32_t n_tiles = (a.n + NT - 1) / NT, m_tiles = (a.m + MT - 1) / MT, tiles = n_tiles * m_tiles, per_xcd = (tiles + 7) / 8;
+    const uint32_t tile = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+    if (blockIdx.x / 8 >= per_xcd || tile >= tiles) return;
+    const bool tall = a.m >= a.n;
+    const uint32_t m0 = (tall ? tile / n_tiles : tile % m_tiles) * MT, n0 = (tall ? tile % n_tiles : tile / m_tiles) * NT;
+    const uint32_t steps = (a.k + 127) / 128, row_bytes = a.k / 32 * 34;
+
+    const uint32_t row = tid / 16, chunk = tid % 16;
+    const uint8_t* x_from[XR];
+    const uint8_t* w_from[WR];
 #pragma unroll
-    for (uint32_t q = 0; q < kWLoads; ++q) {
-        const uint32_t id = q * kWave + lane < kEdge * kDwords ? q * kWave + lane : kEdge * kDwords - 1, r = n0 + id / kDwords;
-        w_at[q] = ((r < a.n ? r : a.n - 1) - n0) * row_bytes + id % kDwords * 4;
+    for (uint32_t i = 0; i < XR; ++i) {  // rows past the matrix re-read its last row (never stored)
+        const uint32_t r = m0 + row + 32 * i;
+        x_from[i] = reinterpret_cast<const uint8_t*>(a.x) + (r < a.m ? r : a.m - 1) * a.x_stride;
     }
-    const uint8_t* x_from[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const uint32_t r = m0 + i * 4 + lane / 16;
-        x_from[i] = reinterpret_cast<const uint8_t*>(a.x) + (r < a.m ? r : a.m - 1) * a.x_stride + lane % 16 * 16;
+    for (uint32_t i = 0; i < WR; ++i) {
+        const uint32_t r = n0 + row + 32 * i;
+        w_from[i] = a.w + uint64_t(r < a.n ? r : a.n - 1) * row_bytes;
     }
-    struct Step { f32x4 x[8]; uint32_t w[kWLoads]; };
-    auto fetch = [&](uint32_t s) {
-        Step t;
+    struct Step { f32x4 x[XR][2]; uint32_t q[WR][2]; uint32_t d[WR]; };
+    auto fetch = [&](uint32_t s, Step& t) {
+        const uint32_t wanted = s * 128 + chunk * 8, column = wanted < a.k ? wanted : chunk * 8 % 64;  // every request unconditional: past the end some others, unused
+        const uint32_t x_at = column * 4, d_at = column / 32 * 34, q_at = d_at + 2 + column % 32;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) t.x[i] = *reinterpret_cast<const f32x4*>(x_from[i] + uint64_t(s) * (kStep * 4));
+        for (uint32_t i = 0; i < XR; ++i) {
+            const four_floats* const from = reinterpret_cast<const four_floats*>(x_from[i] + x_at);
+            t.x[i][0] = from[0]; t.x[i][1] = from[1];
+        }
 #pragma unroll
-        for (uint32_t q = 0; q < kWLoads; ++q) t.w[q] = *reinterpret_cast<const uint32_t*>(w_base + uint64_t(s) * (kDwords * 4) + w_at[q]);
-        return t;
+        for (uint32_t i = 0; i < WR; ++i) {
+            const four_quants* const from = reinterpret_cast<const four_quants*>(w_from[i] + q_at);
+            t.q[i][0] = from[0]; t.q[i][1] = from[1];
+            t.d[i] = *reinterpret_cast<const uint16_t*>(w_from[i] + d_at);
+        }
     };
-    _Float16* const xs = lds[wave].x;
-    uint32_t* const ws = lds[wave].w;
-    uint32_t largest = 0;
-    f32x16 acc{};
-    Step next = fetch(wave < steps ? wave : steps - 1);
-    for (uint32_t s = wave; s < steps; s += WAVES) {
-        const Step now = next;
-        next = fetch(s + WAVES < steps ? s + WAVES : s);
+    const uint32_t put_at = row * 256 + ((chunk ^ (row % 16)) * 16);
+    auto put = [&](uint32_t s, const Step& t) {
+        uint8_t* const to = lds + (s % 2) * S::kStage + put_at;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            f16x4 h;
+        for (uint32_t i = 0; i < XR; ++i) {
+            f16x8 h;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) h[e] = _Float16(now.x[i][e]);
-            const uint2 bits = __builtin_bit_cast(uint2, h);
-            // halves without their signs, two to a word: an exponent of ones carries into the bit above
-            largest |= ((bits.x & 0x7fff7fffu) + 0x04000400u) | ((bits.y & 0x7fff7fffu) + 0x04000400u);
-            *reinterpret_cast<f16x4*>(xs + (i * 4 + lane / 16) * kPitch + lane % 16 * 4) = h;
+            for (int e = 0; e < 8; ++e) h[e] = _Float16(t.x[i][e / 4][e % 4]);
+            *reinterpret_cast<f16x8*>(to + i * 8192) = h;
         }
 #pragma unroll
-        for (uint32_t q = 0; q < kWLoads; ++q) ws[q * kWave + lane] = now.w[q];
-        __builtin_amdgcn_wave_barrier();
-        const uint32_t* const mine = ws + col * kDwords;
-        const uint32_t d_even = mine[0] & 0xffffu, d_odd = mine[8] >> 16;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            // quants 16 (g % 2) + 8 khalf .. + 7 of block g / 2, which starts at byte 34 (g / 2) of the row's 68 with its scale
-            const uint32_t* const q = mine + (g < 2 ? 0 : 9) + g % 2 * 4 + khalf * 2;
-            uint32_t q0 = q[0], q1 = q[1];
-            if (g < 2) {
-                q0 = __builtin_amdgcn_alignbyte(q1, q0, 2);
-                q1 = __builtin_amdgcn_alignbyte(q[2], q1, 2);
-            }
-            const uint32_t d = g < 2 ? d_even : d_odd;
-            const f16x2 d2 = as_h2(d | d << 16);
-            const f16x8 c = quants8(q0, q1);  // exact, as is d: one packed multiply rounds once
+        for (uint32_t i = 0; i < WR; ++i) {
+            const f16x2 d2 = as_h2(t.d[i] | t.d[i] << 16);
+            const f16x8 c = quants8(t.q[i][0], t.q[i][1]);  // exact, as is d: one packed multiply rounds once
             const f16x2 p0 = f16x2{c[0], c[1]} * d2, p1 = f16x2{c[2], c[3]} * d2, p2 = f16x2{c[4], c[5]} * d2, p3 = f16x2{c[6], c[7]} * d2;
-            const f16x8 fb{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
-            const f16x8 fa = *reinterpret_cast<const f16x8*>(xs + col * kPitch + g * 16 + khalf * 8);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa, fb, acc, 0, 0, 0);
+            *reinterpret_cast<f16x8*>(to + MT * 256 + i * 8192) = f16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
         }
-        __builtin_amdgcn_wave_barrier();
+        if (s * 128 + chunk * 8 >= a.k) {  // past the end
+#pragma unroll
+            for (uint32_t i = 0; i < XR + WR; ++i) *reinterpret_cast<u32x4*>(to + i * 8192) = u32x4{};
+        }
+    };
+    const uint32_t group = wave / TILES, wm = wave % TILES / S::kWavesN, wn = wave % S::kWavesN, col = lane % 32, khalf = lane / 32;
+    const uint32_t at = col * 256 + ((khalf ^ (col % 16)) * 16), xs = wm * (S::kRowTiles * 8192) + at, ws = MT * 256 + wn * (S::kColumnTiles * 8192) + at;
+    f32x16 acc[S::kRowTiles][S::kColumnTiles] = {};
+    constexpr uint32_t kSlices = 8 / S::kGroups;  // of sixteen columns
+    struct Fragments { f16x8 x[kSlices][S::kRowTiles], w[kSlices][S::kColumnTiles]; };
+    auto read = [&](uint32_t s, Fragments& f) {
+        const uint8_t* const from = lds + (s % 2) * S::kStage;
+#pragma unroll
+        for (uint32_t j = 0; j < kSlices; ++j) {
+            const uint32_t k = (group * kSlices + j) * 32;
+#pragma unroll
+            for (int i = 0; i < S::kRowTiles; ++i) f.x[j][i] = *reinterpret_cast<const f16x8*>(from + (xs ^ k) + i * 8192);
+#pragma unroll
+            for (int i = 0; i < S::kColumnTiles; ++i) f.w[j][i] = *reinterpret_cast<const f16x8*>(from + (ws ^ k) + i * 8192);
+        }
+    };
+    auto multiply = [&](const Fragments& f) {
+#pragma unroll
+        for (uint32_t j = 0; j < kSlices; ++j)
+#pragma unroll
+            for (int i = 0; i < S::kRowTiles; ++i)
+#pragma unroll
+                for (int c = 0; c < S::kColumnTiles; ++c) acc[i][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.x[j][i], f.w[j][c], acc[i][c], 0, 0, 0);
+    };
+    Step t[S::kDepth];
+#pragma unroll
+    for (uint32_t d = 0; d < S::kDepth; ++d) fetch(d, t[d]);
+    put(0, t[0]);
+    fetch(S::kDepth, t[0]);
+    lds_barrier();
+    for (uint32_t s0 = 0; s0 < steps; s0 += S::kDepth) {
+#pragma unroll
+        for (uint32_t d = 0; d < S::kDepth; ++d) {  // steps past the end are zeros
+            const uint32_t s = s0 + d;
+            Step& next = t[(d + 1) % S::kDepth];
+            Fragments f;
+            read(s, f);
+            __builtin_amdgcn_sched_barrier(0);
+            put(s + 1, next);  // while the fragments are on their way
+            fetch(s + 1 + S::kDepth, next);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(f);
+            lds_barrier();
+        }
     }
-    uint32_t bad = largest & 0x80008000u ? uint32_t(TSP_ERRBIT_NONFINITE) : 0u;
-    // accumulator v: token row 8 (v / 4) + 4 khalf + v % 4 of the tile, weight row `col`; the sums lie over their wave's operands
-    float* const sums = reinterpret_cast<float*>(&lds[wave]);
+    // the groups' sums, added in their order: a 32 x 32 tile of every wave at a time, the next one's beside it in LDS
+    uint32_t bad = 0;  // a token's value that is no finite half makes its whole row so
+    f32x4* const sums = reinterpret_cast<f32x4*>(lds);
 #pragma unroll
-    for (int v = 0; v < 16; ++v) sums[(8 * (v / 4) + 4 * khalf + v % 4) * kEdge + col] = acc[v];
-    __syncthreads();
+    for (int p = 0; p < S::kPasses; ++p) {
+        const f32x16& mine = acc[p / S::kColumnTiles][p % S::kColumnTiles];
+        f32x4* const at_pass = sums + (p % 2) * 2048;
 #pragma unroll
-    for (uint32_t i = tid; i < kEdge * kEdge; i += WAVES * kWave) {
-        float value = 0;
+        for (int b = 0; b < 4; ++b) at_pass[(wave * 4 + b) * 64 + lane] = f32x4{mine[4 * b], mine[4 * b + 1], mine[4 * b + 2], mine[4 * b + 3]};
+        lds_barrier();
+        // quad b of lane l: token rows 8 b + 4 (l / 32) + 0 .. 3 of the tile, weight row l % 32
 #pragma unroll
-        for (int q = 0; q < WAVES; ++q) value += reinterpret_cast<const float*>(&lds[q])[i];
-        const uint32_t m = m0 + i / kEdge, n = n0 + i % kEdge;
-        if (m < a.m && n < a.n) {
-            if (nonfinite(value)) bad = TSP_ERRBIT_NONFINITE;
-            reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(a.out) + m * a.out_stride)[n] = value;
+        for (uint32_t q = tid; q < TILES * 256; q += 512) {
+            const uint32_t which = q / 256, b = q / 64 % 4;
+            f32x4 value = at_pass[(which * 4 + b) * 64 + lane];
+#pragma unroll
+            for (uint32_t g = 1; g < S::kGroups; ++g) value += at_pass[((g * TILES + which) * 4 + b) * 64 + lane];
+            const uint32_t n = n0 + ((which % S::kWavesN) * S::kColumnTiles + p % S::kColumnTiles) * 32 + col;
+            const uint32_t m = m0 + ((which / S::kWavesN) * S::kRowTiles + p / S::kColumnTiles) * 32 + 8 * b + 4 * khalf;
+#pragma unroll
+            for (uint32_t r = 0; r < 4; ++r)
+                if (m + r < a.m && n < a.n) {
+                    if (nonfinite(value[r])) bad = TSP_ERRBIT_NONFINITE;
+                    reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(a.out) + (m + r) * a.out_stride)[n] = value[r];
+                }
         }
     }
     publish_error(bad, a.error_word);
@@ -234,8 +293,6 @@ struct OperandsArgs {
     uint32_t layout, columns, rows, tokens;
     uint32_t* error_word;
 };
-using four_floats = f32x4 __attribute__((aligned(4)));
-using four_quants = uint32_t __attribute__((aligned(2)));  // rows and blocks are even byte counts
 __global__ __launch_bounds__(256) void q8_operands_to_f16(OperandsArgs a) {
     const uint32_t lane = threadIdx.x % kWave, row = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), c8 = blockIdx.y * kWave + lane;
     if (row >= a.rows + a.tokens || c8 * 8 >= a.columns) return;
@@ -278,6 +335,43 @@ __global__ __launch_bounds__(256) void q8_operands_to_f16(OperandsArgs a) {
 
 uint64_t align256(uint64_t v) { return (v + 255) / 256 * 256; }
 
+template <class S>
+int launch_fused(const Q8GemmArgs& a, hipStream_t s) {
+    if constexpr (S::kLds > 65536) {
+        static std::atomic<uint64_t> raised{0};
+        int device = 0;
+        if (setup_pending(raised, &device)) {
+            TSP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q8_gemm_fused<S>), hipFuncAttributeMaxDynamicSharedMemorySize, int(S::kLds)));
+            setup_done(raised, device);
+        }
+    }
+    const uint64_t tiles = uint64_t((a.m + S::kM - 1) / S::kM) * ((a.n + S::kN - 1) / S::kN);
+    TSP_LAUNCH("q8_gemm_fused", s, q8_gemm_fused<S><<<uint32_t((tiles + 7) / 8 * 8), 512, S::kLds, s>>>(a));
+    return launch_status("q8_gemm_fused");
+}
+
+// Which tile, or none for the two launches: the one whose time, as measured, is shortest. A round of 256 workgroups, one to a compute unit, takes so
+// long for each 128 columns and so long to begin and end (20 steps of 2560 columns and 5 of 640, us: 32 x 32 8.5 and 4, 32 x 64 12.9 and 5.9, 64 x 64 16.4 and 7.4, 64 x 96 23.2 and
+// 9, 128 x 128 39 and 15.7); rounds follow each other, so a tile that just fills one is the best. The two launches take 570 ns a step for each round of 64 x 64 tiles,
+// which share the compute units evenly, and the conversion's bytes at 5 TB/s: 2048 x 640 -> 2560 24.9 for 31 with the best tile, 1000 x 640 -> 2560
+// 15.8 for 16.3.
+using FusedLaunch = int (*)(const Q8GemmArgs&, hipStream_t);
+FusedLaunch fused_launch(uint32_t m, uint32_t n, uint32_t k) {
+    struct Choice { uint32_t m, n, step_ns, ends_ns; FusedLaunch launch; };
+    static constexpr Choice choices[] = {{32, 32, 310, 2400, launch_fused<FusedShape<32, 32, 1, 1, 2, 2>>},   {32, 64, 480, 3000, launch_fused<FusedShape<32, 64, 1, 2, 2, 2>>},
+                                         {64, 64, 650, 3400, launch_fused<FusedShape<64, 64, 2, 1, 1, 4>>},   {64, 96, 950, 3700, launch_fused<FusedShape<64, 96, 2, 1, 2, 2>>},
+                                         {128, 128, 1600, 8000, launch_fused<FusedShape<128, 128, 2, 2, 1, 2>>}};
+    const auto tiles = [&](uint32_t tm, uint32_t tn) { return uint64_t((m + tm - 1) / tm) * ((n + tn - 1) / tn); };
+    const uint64_t steps = (k + 127) / 128, staged_tiles = tiles(kTile, kTile), staged_rounds = staged_tiles < 220 ? 220 : staged_tiles;  // in 256ths
+    uint64_t best = steps * (570 * staged_rounds / 256 + (768ull * m + 392ull * n) / 5000) + 4700 + 400 * staged_rounds / 256;
+    FusedLaunch launch = nullptr;
+    for (const Choice& c : choices) {
+        const uint64_t ns = (tiles(c.m, c.n) + 255) / 256 * (steps * c.step_ns + c.ends_ns);
+        if (ns < best) { best = ns; launch = c.launch; }
+    }
+    return launch;
+}
+
 }  // namespace
 
 // workspace: [decoded matrix, halves][token rows, halves]
@@ -305,17 +399,9 @@ extern "C" int tsp_dense_mm_q8_staged(uint32_t layout, const void* matrix, uint6
                     !ranges_overlap(workspace, workspace_bytes, output, out_span),
                 "dense Q8_0 GEMM buffers overlap");
     const auto s = static_cast<hipStream_t>(stream);
-    // Up to 600 tiles of 32 x 32 (two or three rounds over the chip): decoded on the way, else decoded once and multiplied, where a round
-    // costs more than the launch saved (2048 columns x 512 rows: 14.8 against 17.2 us at 400 tiles, 20.7 against 18.1 at 656; 640 x
-    // 2560 8.4 against 9.5 at 560, 12.5 against 11.5 at 1040). f32 rows are read sixteen bytes at a time.
-    const uint64_t tiles = uint64_t((rows + 31) / 32) * ((tokens + 31) / 32);
-    if (layout == TSP_LAYOUT_GGUF && tiles <= 600 && reinterpret_cast<uintptr_t>(input) % 16 == 0 && input_stride_bytes % 16 == 0 &&
-        reinterpret_cast<uintptr_t>(matrix) % 4 == 0) {
+    if (layout == TSP_LAYOUT_GGUF) {
         const Q8GemmArgs a{input, input_stride_bytes, static_cast<const uint8_t*>(matrix), output, output_stride_bytes, tokens, rows, columns, error_word};
-        const dim3 grid((rows + 31) / 32, (tokens + 31) / 32);
-        if (columns >= 2048 && tiles <= 256) TSP_LAUNCH("q8_gemm_split", s, q8_gemm_split<8><<<grid, 512, 0, s>>>(a));
-        else TSP_LAUNCH("q8_gemm_split", s, q8_gemm_split<4><<<grid, 256, 0, s>>>(a));
-        return launch_status("q8_gemm_split");
+        if (const auto launch = fused_launch(tokens, rows, columns)) return launch(a, s);
     }
     _Float16* const w16 = static_cast<_Float16*>(workspace);
     _Float16* const x16 = reinterpret_cast<_Float16*>(static_cast<uint8_t*>(workspace) + align256(uint64_t(rows) * columns * 2));
