@@ -289,8 +289,8 @@ def test_dense_mm_q8_staged_tiles(gpu, tsp, synth, tokens, cols, rows):
     assert (np.abs(got - x.astype(np.float64) @ weight.T) <= bound).all() and gpu.error() == 0
 
 
-@pytest.mark.parametrize("tokens,cols,rows,pad", [(33, 64, 33, 0), (63, 2624, 31, 1), (100, 704, 2500, 0), (203, 704, 2500, 3), (1984, 1088, 600, 0), (1990, 704, 2040, 1),
-                                                  (2047, 192, 2050, 0)])
+@pytest.mark.parametrize("tokens,cols,rows,pad", [(33, 64, 33, 0), (63, 2624, 31, 1), (100, 704, 2500, 0), (203, 704, 2500, 3), (2043, 2112, 701, 0), (1990, 704, 2040, 1),
+                                                  (449, 640, 2500, 0)])
 def test_dense_mm_q8_staged_tile_shapes(gpu, tsp, synth, tokens, cols, rows, pad):
     # every tile that raw rows are decoded in (32 x 32, 32 x 32, 32 x 64, 64 x 64, 64 x 96, 128 x 128) and the two launches: ragged edges, a last step of 64 columns, a single
     # step, rows four bytes off a multiple of sixteen. The bound is that of test_dense_mm_q8_staged_tiles.

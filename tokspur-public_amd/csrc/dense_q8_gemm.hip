@@ -127,11 +127,11 @@ using four_quants = uint32_t __attribute__((aligned(2)));  // rows and blocks ar
 // the step's columns, whose sums meet in LDS in the groups' order. Chunk c (16 bytes) of row r sits at position c ^ (r % 16) of the
 // row's 256 bytes: sixteen consecutive lanes touch every bank once, writing and reading. Fragments are requested from LDS before the next step's
 // operands are rounded, and multiplied after that.
-// Bound by a step's chain, some 6 ns for each of the tile's rows, whether the rest of the chip has work or not. Against the 32 x 32 tiles whose waves took 64 columns in turns, or
-// above 600 of them the two launches below, per call, tokens x columns -> rows: 203 x 2560 -> 640 10.2 -> 9.0 us, 450 16.9 -> 12.6, 600 17.5 -> 12.9, 1000
-// 18.9 -> 17.8, 2048 25.1 -> 23.2; 450 x 2048 -> 512 9.9 -> 8.2, 2048 18.4 -> 15.5; 203 x 640 -> 2560 8.6 -> 7.4; 2048 x 768 -> 2048 24.2 -> 19.3. Tried: token rows
-// sixteen bytes to a lane and sixteen quants to a load (2048 x 2560 -> 640 27), operands straight into LDS of the wave that multiplies them (24), the
-// matrix in fragment order by a launch before (22, but 32 for 24.9 at 640 x 2560).
+// Bound by what a compute unit fetches, some 30 bytes a cycle whether the rest of the chip has work or not (a tile alone takes as long as 256; steps further ahead
+// and a step's rounding beside its products gain nothing). Against the 32 x 32 tiles whose waves took 64 columns in turns, or above 600 of them the two launches below, per call, tokens x
+// columns -> rows, operands from memory: 203 x 2560 -> 640 11.2 -> 10.3 us, 600 19.6 -> 15.3, 800 20.4 -> 14.8; 1000 x 2048 -> 512 17.3 -> 12.4, 2048 19.5 -> 18.6; 800 x 1024 ->
+// 512 10.5 -> 8.1; 203 x 640 -> 2560 8.7 -> 8.1; 2048 x 768 -> 2048 23.9 -> 22.1. Tried: token rows sixteen bytes to a lane and sixteen quants to a load (2048 x 2560 -> 640 27 for
+// 23), operands straight into LDS of the wave that multiplies them (24), the matrix in fragment order by a launch before (22, but 32 for 24.9 at 640 x 2560).
 template <int MT, int NT, int WM, int WN, int DEPTH, int WAVES_PER_SIMD>
 struct FusedShape {
     static constexpr int kM = MT, kN = NT, kDepth = DEPTH, kRowTiles = MT / 32 / WM, kColumnTiles = NT / 32 / WN, kGroups = 8 / (WM * WN), kPasses = kRowTiles * kColumnTiles;
@@ -351,19 +351,21 @@ int launch_fused(const Q8GemmArgs& a, hipStream_t s) {
 }
 
 // Which tile, or none for the two launches: the one whose time, as measured, is shortest. A round of 256 workgroups, one to a compute unit, takes so
-// long for each 128 columns and so long to begin and end (20 steps of 2560 columns and 5 of 640, us: 32 x 32 8.5 and 4, 32 x 64 12.9 and 5.9, 64 x 64 16.4 and 7.4, 64 x 96 23.2 and
-// 9, 128 x 128 39 and 15.7); rounds follow each other, so a tile that just fills one is the best. The two launches take 570 ns a step for each round of 64 x 64 tiles,
-// which share the compute units evenly, and the conversion's bytes at 5 TB/s: 2048 x 640 -> 2560 24.9 for 31 with the best tile, 1000 x 640 -> 2560
-// 15.8 for 16.3.
+// long for each 128 columns and so long to begin and end, between operands that a call before has read and operands from memory (20 steps of 2560 columns,
+// us: 32 x 32 8.5 and 11.6, 32 x 64 12.9 and 15.2, 64 x 64 16.4 and 21.5, 64 x 96 23.2 and 27.2, 128 x 128 39 and 48); rounds follow each other, so a tile that just fills
+// one is the best. The two launches take 570 ns a step for each round of 64 x 64 tiles, which share the compute units evenly, and the conversion's bytes at
+// 5 TB/s; what they read from memory they read once and in long runs, so they keep calls that would gain less than a tenth: 2048 x 2560 -> 640 23.1 and 25.8
+// where 64 x 96 takes 22.3 and 27.2, 1000 x 2560 -> 640 18.4 and 19.8 where 64 x 64 takes 17.6 and 21.7, 2048 x 640 -> 2560 24.9 and 26.3 where 128 x 128 takes 31 and 32.9.
 using FusedLaunch = int (*)(const Q8GemmArgs&, hipStream_t);
 FusedLaunch fused_launch(uint32_t m, uint32_t n, uint32_t k) {
     struct Choice { uint32_t m, n, step_ns, ends_ns; FusedLaunch launch; };
-    static constexpr Choice choices[] = {{32, 32, 310, 2400, launch_fused<FusedShape<32, 32, 1, 1, 2, 2>>},   {32, 64, 480, 3000, launch_fused<FusedShape<32, 64, 1, 2, 2, 2>>},
-                                         {64, 64, 650, 3400, launch_fused<FusedShape<64, 64, 2, 1, 1, 4>>},   {64, 96, 950, 3700, launch_fused<FusedShape<64, 96, 2, 1, 2, 2>>},
-                                         {128, 128, 1600, 8000, launch_fused<FusedShape<128, 128, 2, 2, 1, 2>>}};
+    static constexpr Choice choices[] = {{32, 32, 370, 2500, launch_fused<FusedShape<32, 32, 1, 1, 2, 2>>},   {32, 64, 545, 3000, launch_fused<FusedShape<32, 64, 1, 2, 2, 2>>},
+                                         {64, 64, 760, 3850, launch_fused<FusedShape<64, 64, 2, 1, 1, 4>>},   {64, 96, 980, 5100, launch_fused<FusedShape<64, 96, 2, 1, 2, 2>>},
+                                         {128, 128, 1875, 7500, launch_fused<FusedShape<128, 128, 2, 2, 1, 2>>}};
     const auto tiles = [&](uint32_t tm, uint32_t tn) { return uint64_t((m + tm - 1) / tm) * ((n + tn - 1) / tn); };
     const uint64_t steps = (k + 127) / 128, staged_tiles = tiles(kTile, kTile), staged_rounds = staged_tiles < 220 ? 220 : staged_tiles;  // in 256ths
-    uint64_t best = steps * (570 * staged_rounds / 256 + (768ull * m + 392ull * n) / 5000) + 4700 + 400 * staged_rounds / 256;
+    uint64_t best = steps * (570 * staged_rounds / 256 + (768ull * m + 392ull * n) / 5000) + 4950 + 550 * staged_rounds / 256;
+    best = best * 9 / 10;
     FusedLaunch launch = nullptr;
     for (const Choice& c : choices) {
         const uint64_t ns = (tiles(c.m, c.n) + 255) / 256 * (steps * c.step_ns + c.ends_ns);
