@@ -306,6 +306,33 @@ def test_dense_mm_q8_staged_tile_shapes(gpu, tsp, synth, tokens, cols, rows, pad
     assert (np.abs(got[:, :rows] - x @ weight.T) <= bound).all() and (got[:, rows:] == -5.0).all() and gpu.error() == 0
 
 
+@pytest.mark.parametrize("tokens,cols,rows,kernels", [(63, 2624, 31, ["q8_gemm_fused 32x32"]), (100, 704, 2500, ["q8_gemm_fused 32x64"]), (203, 704, 2500, ["q8_gemm_fused 64x64"]),
+                                                      (2043, 1088, 701, ["q8_gemm_fused 64x96"]), (1990, 704, 2040, ["q8_gemm_fused 128x128"]),
+                                                      (1990, 704, 1021, ["q8_operands_to_f16", "f16_gemm_nt"])])
+def test_dense_mm_q8_staged_kernels(gpu, tsp, synth, tokens, cols, rows, kernels):
+    # Which kernels a call takes, so that each is reached whatever the rule's figures; and in each an infinity and a finite value that
+    # no half holds, one of them in the last token row's last 64 columns, are reported and leave all other token rows right (the bound of test_dense_mm_q8_staged_tiles).
+    w = synth.matrix(8, 2600 + cols, rows, cols)
+    x = synth.activations_f32(2601 + tokens, (tokens, cols))
+    blocks = w.reshape(rows, -1, 34)
+    weight = blocks[:, :, 2:].view(np.int8).astype(np.float64) * np.ascontiguousarray(blocks[:, :, :2]).view(np.float16).astype(np.float64)
+    weight = weight.reshape(rows, cols)
+    declared, bound = x.astype(np.float64) @ weight.T, (2.0 ** -10 + cols * 2.0 ** -24) * (np.abs(x.astype(np.float64)) @ np.abs(weight).T)
+    matrix = gpu.upload(w)
+    tsp.profile_begin()
+    got = tsp.dense_mm_q8_staged(gpu, tsp.LAYOUT_GGUF, matrix, gpu.upload(x), tokens, cols, rows).cpu().numpy()
+    assert sorted(tsp.profile_end()) == sorted(kernels)
+    assert (np.abs(got - declared) <= bound).all() and gpu.error() == 0
+    for at, value in ((tokens - 1, np.inf), (tokens - 1, 1e5), (tokens // 2, -np.inf), (tokens // 2, -1e5)):
+        wrong = x.copy()
+        wrong[at, cols - 3 if at == tokens - 1 else 1] = value
+        got = tsp.dense_mm_q8_staged(gpu, tsp.LAYOUT_GGUF, matrix, gpu.upload(wrong), tokens, cols, rows).cpu().numpy()
+        assert gpu.error() & tsp.ERRBIT_NONFINITE
+        gpu.clear_error()
+        others = np.arange(tokens) != at
+        assert (np.abs(got - declared) <= bound)[others].all()
+
+
 @pytest.mark.parametrize("tokens,cols,rows,pad", [(2, 64, 1, 0), (7, 640, 33, 0), (8, 2560, 640, 0), (9, 320, 18, 0), (16, 1088, 47, 12), (5, 2048, 160, 4),
                                                   (23, 2560, 48, 0), (3, 96, 20, 0), (6, 512, 24640, 0), (15, 512, 14020, 0), (11, 1280, 14001, 0),
                                                   (7, 2560, 24577, 0), (14, 2560, 14004, 0), (27, 1024, 14004, 0), (41, 192, 30, 4),

@@ -336,7 +336,7 @@ __global__ __launch_bounds__(256) void q8_operands_to_f16(OperandsArgs a) {
 uint64_t align256(uint64_t v) { return (v + 255) / 256 * 256; }
 
 template <class S>
-int launch_fused(const Q8GemmArgs& a, hipStream_t s) {
+int launch_fused(const Q8GemmArgs& a, const char* name, hipStream_t s) {
     if constexpr (S::kLds > 65536) {
         static std::atomic<uint64_t> raised{0};
         int device = 0;
@@ -346,7 +346,7 @@ int launch_fused(const Q8GemmArgs& a, hipStream_t s) {
         }
     }
     const uint64_t tiles = uint64_t((a.m + S::kM - 1) / S::kM) * ((a.n + S::kN - 1) / S::kN);
-    TSP_LAUNCH("q8_gemm_fused", s, q8_gemm_fused<S><<<uint32_t((tiles + 7) / 8 * 8), 512, S::kLds, s>>>(a));
+    TSP_LAUNCH(name, s, q8_gemm_fused<S><<<uint32_t((tiles + 7) / 8 * 8), 512, S::kLds, s>>>(a));
     return launch_status("q8_gemm_fused");
 }
 
@@ -356,22 +356,27 @@ int launch_fused(const Q8GemmArgs& a, hipStream_t s) {
 // one is the best. The two launches take 570 ns a step for each round of 64 x 64 tiles, which share the compute units evenly, and the conversion's bytes at
 // 5 TB/s; what they read from memory they read once and in long runs, so they keep calls that would gain less than a tenth: 2048 x 2560 -> 640 23.1 and 25.8
 // where 64 x 96 takes 22.3 and 27.2, 1000 x 2560 -> 640 18.4 and 19.8 where 64 x 64 takes 17.6 and 21.7, 2048 x 640 -> 2560 24.9 and 26.3 where 128 x 128 takes 31 and 32.9.
-using FusedLaunch = int (*)(const Q8GemmArgs&, hipStream_t);
-FusedLaunch fused_launch(uint32_t m, uint32_t n, uint32_t k) {
-    struct Choice { uint32_t m, n, step_ns, ends_ns; FusedLaunch launch; };
-    static constexpr Choice choices[] = {{32, 32, 370, 2500, launch_fused<FusedShape<32, 32, 1, 1, 2, 2>>},   {32, 64, 545, 3000, launch_fused<FusedShape<32, 64, 1, 2, 2, 2>>},
-                                         {64, 64, 760, 3850, launch_fused<FusedShape<64, 64, 2, 1, 1, 4>>},   {64, 96, 980, 5100, launch_fused<FusedShape<64, 96, 2, 1, 2, 2>>},
-                                         {128, 128, 1875, 7500, launch_fused<FusedShape<128, 128, 2, 2, 1, 2>>}};
+struct FusedTile {
+    uint32_t m, n, step_ns, ends_ns;
+    const char* name;  // in a profile window
+    int (*launch)(const Q8GemmArgs&, const char*, hipStream_t);
+};
+const FusedTile* fused_tile(uint32_t m, uint32_t n, uint32_t k) {
+    static constexpr FusedTile choices[] = {{32, 32, 370, 2500, "q8_gemm_fused 32x32", launch_fused<FusedShape<32, 32, 1, 1, 2, 2>>},
+                                            {32, 64, 545, 3000, "q8_gemm_fused 32x64", launch_fused<FusedShape<32, 64, 1, 2, 2, 2>>},
+                                            {64, 64, 760, 3850, "q8_gemm_fused 64x64", launch_fused<FusedShape<64, 64, 2, 1, 1, 4>>},
+                                            {64, 96, 980, 5100, "q8_gemm_fused 64x96", launch_fused<FusedShape<64, 96, 2, 1, 2, 2>>},
+                                            {128, 128, 1875, 7500, "q8_gemm_fused 128x128", launch_fused<FusedShape<128, 128, 2, 2, 1, 2>>}};
     const auto tiles = [&](uint32_t tm, uint32_t tn) { return uint64_t((m + tm - 1) / tm) * ((n + tn - 1) / tn); };
     const uint64_t steps = (k + 127) / 128, staged_tiles = tiles(kTile, kTile), staged_rounds = staged_tiles < 220 ? 220 : staged_tiles;  // in 256ths
     uint64_t best = steps * (570 * staged_rounds / 256 + (768ull * m + 392ull * n) / 5000) + 4950 + 550 * staged_rounds / 256;
     best = best * 9 / 10;
-    FusedLaunch launch = nullptr;
-    for (const Choice& c : choices) {
+    const FusedTile* chosen = nullptr;
+    for (const FusedTile& c : choices) {
         const uint64_t ns = (tiles(c.m, c.n) + 255) / 256 * (steps * c.step_ns + c.ends_ns);
-        if (ns < best) { best = ns; launch = c.launch; }
+        if (ns < best) { best = ns; chosen = &c; }
     }
-    return launch;
+    return chosen;
 }
 
 }  // namespace
@@ -403,7 +408,7 @@ extern "C" int tsp_dense_mm_q8_staged(uint32_t layout, const void* matrix, uint6
     const auto s = static_cast<hipStream_t>(stream);
     if (layout == TSP_LAYOUT_GGUF) {
         const Q8GemmArgs a{input, input_stride_bytes, static_cast<const uint8_t*>(matrix), output, output_stride_bytes, tokens, rows, columns, error_word};
-        if (const auto launch = fused_launch(tokens, rows, columns)) return launch(a, s);
+        if (const FusedTile* tile = fused_tile(tokens, rows, columns)) return tile->launch(a, tile->name, s);
     }
     _Float16* const w16 = static_cast<_Float16*>(workspace);
     _Float16* const x16 = reinterpret_cast<_Float16*>(static_cast<uint8_t*>(workspace) + align256(uint64_t(rows) * columns * 2));
