@@ -307,7 +307,7 @@ def test_dense_mm_q8_staged_tile_shapes(gpu, tsp, synth, tokens, cols, rows, pad
 
 
 @pytest.mark.parametrize("tokens,cols,rows,kernels", [(63, 2624, 31, ["q8_gemm_fused 32x32"]), (100, 704, 2500, ["q8_gemm_fused 32x64"]), (203, 704, 2500, ["q8_gemm_fused 64x64"]),
-                                                      (2043, 1088, 701, ["q8_gemm_fused 64x96"]), (1990, 704, 2040, ["q8_gemm_fused 128x128"]),
+                                                      (2043, 1088, 701, ["q8_gemm_fused 64x96"]), (1990, 704, 2040, ["q8_gemm_fused 128x128"]), (70, 128, 33, ["q8_gemm_split"]), (9, 2624, 33, ["q8_gemm_split"]),
                                                       (1990, 704, 1021, ["q8_operands_to_f16", "f16_gemm_nt"])])
 def test_dense_mm_q8_staged_kernels(gpu, tsp, synth, tokens, cols, rows, kernels):
     # Which kernels a call takes, so that each is reached whatever the rule's figures; and in each an infinity and a finite value that
@@ -331,6 +331,27 @@ def test_dense_mm_q8_staged_kernels(gpu, tsp, synth, tokens, cols, rows, kernels
         gpu.clear_error()
         others = np.arange(tokens) != at
         assert (np.abs(got - declared) <= bound)[others].all()
+
+
+@pytest.mark.parametrize("tokens,cols,rows,pad,kernels", [
+    (400, 64, 640, 0, "split"), (9, 320, 33, 0, "split"), (601, 64, 1601, 0, "split"), (561, 64, 1601, 1, "64x64"), (1001, 64, 1601, 0, "two"), (33, 64, 33, 1, "two"), (700, 192, 1000, 0, "64x64"), (33, 384, 33, 0, "32x32"), (1600, 384, 700, 0, "two"),       # few columns; rows that the first cannot read
+    (1, 2048, 33, 0, "split"), (16, 4096, 65, 4, "split"), (16, 2048, 65, 3, "32x32"), (17, 2048, 65, 0, "32x32"), (16, 1024, 65, 0, "32x32"),  # few tokens
+    (700, 2112, 1024, 0, "two"), (250, 2112, 3100, 0, "64x64"), (1025, 1024, 512, 0, "64x64"), (1025, 1088, 512, 0, "two"), (820, 1088, 512, 0, "32x64"), (1200, 2112, 512, 0, "two")])
+def test_dense_mm_q8_staged_choice(gpu, tsp, synth, tokens, cols, rows, pad, kernels):
+    # Calls that the rule by rounds over the chip alone had made up to 1.5 times as long as they were (few columns, few tokens) or 1.1 times (many columns from memory), and
+    # either side of its limits. The bound is that of test_dense_mm_q8_staged_tiles.
+    w = synth.matrix(8, 2700 + cols, rows, cols)
+    x = synth.activations_f32(2701 + tokens, (tokens, cols + pad))
+    matrix, rows_in = gpu.upload(w), gpu.upload(x)
+    tsp.profile_begin()
+    got = tsp.dense_mm_q8_staged(gpu, tsp.LAYOUT_GGUF, matrix, rows_in, tokens, cols, rows, x_stride=(cols + pad) * 4).cpu().numpy()
+    assert sorted(tsp.profile_end()) == {"split": ["q8_gemm_split"], "two": ["f16_gemm_nt", "q8_operands_to_f16"]}.get(kernels, ["q8_gemm_fused " + kernels])
+    x = x[:, :cols].astype(np.float64)
+    blocks = w.reshape(rows, -1, 34)
+    weight = blocks[:, :, 2:].view(np.int8).astype(np.float64) * np.ascontiguousarray(blocks[:, :, :2]).view(np.float16).astype(np.float64)
+    weight = weight.reshape(rows, cols)
+    bound = (2.0 ** -10 + cols * 2.0 ** -24) * (np.abs(x) @ np.abs(weight).T)
+    assert (np.abs(got - x @ weight.T) <= bound).all() and gpu.error() == 0
 
 
 @pytest.mark.parametrize("tokens,cols,rows,pad", [(2, 64, 1, 0), (7, 640, 33, 0), (8, 2560, 640, 0), (9, 320, 18, 0), (16, 1088, 47, 12), (5, 2048, 160, 4),

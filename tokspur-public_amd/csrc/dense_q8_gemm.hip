@@ -5,8 +5,8 @@
 // kernel stages, include/tokspur/graph.hpp:860 and kernels/grouped_mm.metal:239-243), the token rows are rounded to halves as
 // well, and the matrix cores multiply the two with f32 accumulation.
 //
-// GGUF rows whose tiles go round the chip well are decoded on their way into the MFMAs, together with the token rows (q8_gemm_fused). Else every operand would be
-// decoded too often or much of the chip stand idle: one launch decodes both into the workspace and f16_gemm_nt multiplies them.
+// GGUF rows whose tiles go round the chip well are decoded on their way into the MFMAs, together with the token rows (q8_gemm_fused; q8_gemm_split for few columns or few
+// token rows). Else every operand would be decoded too often or much of the chip stand idle: one launch decodes both into the workspace and f16_gemm_nt multiplies them.
 //
 // f16_gemm_nt: a workgroup of four waves owns a 64 x 64 output tile (each wave a 32 x 32 MFMA tile) and walks K in
 // steps of 64 halfs. Every byte travels global -> LDS directly (16 bytes per lane, no registers in between) into a ring
@@ -113,6 +113,108 @@ __global__ __launch_bounds__(256, 2) void f16_gemm_nt(F16GemmArgs a) {
         if (m < a.m && n < a.n) {
             if (nonfinite(acc[v])) bad = TSP_ERRBIT_NONFINITE;
             reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(a.out) + uint64_t(m) * a.out_stride)[n] = acc[v];
+        }
+    }
+    publish_error(bad, a.error_word);
+}
+
+// A workgroup is one 32 x 32 output tile and its waves take the columns in turns of 64: a chunk of 64 tokens against 640 rows is 40
+// workgroups of eight waves, each wave a chain of five steps. A wave reads a step as it lies (256 bytes of 32 token rows,
+// 17 dwords of 32 weight rows), two steps' requests in flight, and puts it into fragment order through LDS of its own: no barrier
+// until the waves' sums meet, which are added in wave order.
+// For few columns or few token rows, where it has less to begin and to end with than the kernel below: 400 x 64 -> 640 3.2 us, 100 x 3.0, 9 x 5120 -> 1024 15.2 from memory
+// (4.4, 3.6 and 16.5 on 32 x 32 or 32 x 64 tiles of that one, 5.2 and more for 64 columns with two launches). f32 rows are read sixteen bytes at a time.
+template <int WAVES>
+__global__ __launch_bounds__(WAVES * kWave, 4) void q8_gemm_split(Q8GemmArgs a) {
+    constexpr uint32_t kEdge = 32, kDwords = 17, kWLoads = (kEdge * kDwords + kWave - 1) / kWave, kPitch = kStep + 8;
+    struct WaveLds {
+        _Float16 x[kEdge * kPitch];
+        uint32_t w[kWLoads * kWave];
+    };
+    static_assert(sizeof(WaveLds) >= kEdge * kEdge * 4);
+    __shared__ __attribute__((aligned(16))) WaveLds lds[WAVES];
+    const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid / kWave)));
+    const uint32_t col = lane % 32, khalf = lane / 32;
+    const uint32_t m0 = blockIdx.y * kEdge, n0 = blockIdx.x * kEdge, steps = a.k / kStep, row_bytes = a.k / 32 * 34;
+    const uint8_t* const w_base = a.w + uint64_t(n0) * row_bytes;
+    uint32_t w_at[kWLoads];
+#pragma unroll
+    for (uint32_t q = 0; q < kWLoads; ++q) {
+        const uint32_t id = q * kWave + lane < kEdge * kDwords ? q * kWave + lane : kEdge * kDwords - 1, r = n0 + id / kDwords;
+        w_at[q] = ((r < a.n ? r : a.n - 1) - n0) * row_bytes + id % kDwords * 4;
+    }
+    const uint8_t* x_from[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const uint32_t r = m0 + i * 4 + lane / 16;
+        x_from[i] = reinterpret_cast<const uint8_t*>(a.x) + (r < a.m ? r : a.m - 1) * a.x_stride + lane % 16 * 16;
+    }
+    struct Step { f32x4 x[8]; uint32_t w[kWLoads]; };
+    auto fetch = [&](uint32_t s) {
+        Step t;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) t.x[i] = *reinterpret_cast<const f32x4*>(x_from[i] + uint64_t(s) * (kStep * 4));
+#pragma unroll
+        for (uint32_t q = 0; q < kWLoads; ++q) t.w[q] = *reinterpret_cast<const uint32_t*>(w_base + uint64_t(s) * (kDwords * 4) + w_at[q]);
+        return t;
+    };
+    _Float16* const xs = lds[wave].x;
+    uint32_t* const ws = lds[wave].w;
+    uint32_t largest = 0;
+    f32x16 acc{};
+    Step next = fetch(wave < steps ? wave : steps - 1);
+    for (uint32_t s = wave; s < steps; s += WAVES) {
+        const Step now = next;
+        next = fetch(s + WAVES < steps ? s + WAVES : s);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            f16x4 h;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) h[e] = _Float16(now.x[i][e]);
+            const uint2 bits = __builtin_bit_cast(uint2, h);
+            // halves without their signs, two to a word: an exponent of ones carries into the bit above
+            largest |= ((bits.x & 0x7fff7fffu) + 0x04000400u) | ((bits.y & 0x7fff7fffu) + 0x04000400u);
+            *reinterpret_cast<f16x4*>(xs + (i * 4 + lane / 16) * kPitch + lane % 16 * 4) = h;
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < kWLoads; ++q) ws[q * kWave + lane] = now.w[q];
+        __builtin_amdgcn_wave_barrier();
+        const uint32_t* const mine = ws + col * kDwords;
+        const uint32_t d_even = mine[0] & 0xffffu, d_odd = mine[8] >> 16;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            // quants 16 (g % 2) + 8 khalf .. + 7 of block g / 2, which starts at byte 34 (g / 2) of the row's 68 with its scale
+            const uint32_t* const q = mine + (g < 2 ? 0 : 9) + g % 2 * 4 + khalf * 2;
+            uint32_t q0 = q[0], q1 = q[1];
+            if (g < 2) {
+                q0 = __builtin_amdgcn_alignbyte(q1, q0, 2);
+                q1 = __builtin_amdgcn_alignbyte(q[2], q1, 2);
+            }
+            const uint32_t d = g < 2 ? d_even : d_odd;
+            const f16x2 d2 = as_h2(d | d << 16);
+            const f16x8 c = quants8(q0, q1);  // exact, as is d: one packed multiply rounds once
+            const f16x2 p0 = f16x2{c[0], c[1]} * d2, p1 = f16x2{c[2], c[3]} * d2, p2 = f16x2{c[4], c[5]} * d2, p3 = f16x2{c[6], c[7]} * d2;
+            const f16x8 fb{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
+            const f16x8 fa = *reinterpret_cast<const f16x8*>(xs + col * kPitch + g * 16 + khalf * 8);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa, fb, acc, 0, 0, 0);
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+    uint32_t bad = largest & 0x80008000u ? uint32_t(TSP_ERRBIT_NONFINITE) : 0u;
+    // accumulator v: token row 8 (v / 4) + 4 khalf + v % 4 of the tile, weight row `col`; the sums lie over their wave's operands
+    float* const sums = reinterpret_cast<float*>(&lds[wave]);
+#pragma unroll
+    for (int v = 0; v < 16; ++v) sums[(8 * (v / 4) + 4 * khalf + v % 4) * kEdge + col] = acc[v];
+    __syncthreads();
+#pragma unroll
+    for (uint32_t i = tid; i < kEdge * kEdge; i += WAVES * kWave) {
+        float value = 0;
+#pragma unroll
+        for (int q = 0; q < WAVES; ++q) value += reinterpret_cast<const float*>(&lds[q])[i];
+        const uint32_t m = m0 + i / kEdge, n = n0 + i % kEdge;
+        if (m < a.m && n < a.n) {
+            if (nonfinite(value)) bad = TSP_ERRBIT_NONFINITE;
+            reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(a.out) + m * a.out_stride)[n] = value;
         }
     }
     publish_error(bad, a.error_word);
@@ -350,33 +452,54 @@ int launch_fused(const Q8GemmArgs& a, const char* name, hipStream_t s) {
     return launch_status("q8_gemm_fused");
 }
 
-// Which tile, or none for the two launches: the one whose time, as measured, is shortest. A round of 256 workgroups, one to a compute unit, takes so
-// long for each 128 columns and so long to begin and end, between operands that a call before has read and operands from memory (20 steps of 2560 columns,
-// us: 32 x 32 8.5 and 11.6, 32 x 64 12.9 and 15.2, 64 x 64 16.4 and 21.5, 64 x 96 23.2 and 27.2, 128 x 128 39 and 48); rounds follow each other, so a tile that just fills
-// one is the best. The two launches take 570 ns a step for each round of 64 x 64 tiles, which share the compute units evenly, and the conversion's bytes at
-// 5 TB/s; what they read from memory they read once and in long runs, so they keep calls that would gain less than a tenth: 2048 x 2560 -> 640 23.1 and 25.8
-// where 64 x 96 takes 22.3 and 27.2, 1000 x 2560 -> 640 18.4 and 19.8 where 64 x 64 takes 17.6 and 21.7, 2048 x 640 -> 2560 24.9 and 26.3 where 128 x 128 takes 31 and 32.9.
-struct FusedTile {
-    uint32_t m, n, step_ns, ends_ns;
+template <int WAVES>
+int launch_split(const Q8GemmArgs& a, const char* name, hipStream_t s) {
+    TSP_LAUNCH(name, s, q8_gemm_split<WAVES><<<dim3((a.n + 31) / 32, (a.m + 31) / 32), WAVES * kWave, 0, s>>>(a));
+    return launch_status("q8_gemm_split");
+}
+
+struct RawRowsKernel {
     const char* name;  // in a profile window
     int (*launch)(const Q8GemmArgs&, const char*, hipStream_t);
 };
-const FusedTile* fused_tile(uint32_t m, uint32_t n, uint32_t k) {
-    static constexpr FusedTile choices[] = {{32, 32, 370, 2500, "q8_gemm_fused 32x32", launch_fused<FusedShape<32, 32, 1, 1, 2, 2>>},
-                                            {32, 64, 545, 3000, "q8_gemm_fused 32x64", launch_fused<FusedShape<32, 64, 1, 2, 2, 2>>},
-                                            {64, 64, 760, 3850, "q8_gemm_fused 64x64", launch_fused<FusedShape<64, 64, 2, 1, 1, 4>>},
-                                            {64, 96, 980, 5100, "q8_gemm_fused 64x96", launch_fused<FusedShape<64, 96, 2, 1, 2, 2>>},
-                                            {128, 128, 1875, 7500, "q8_gemm_fused 128x128", launch_fused<FusedShape<128, 128, 2, 2, 1, 2>>}};
+constexpr RawRowsKernel kSplit4{"q8_gemm_split", launch_split<4>}, kSplit8{"q8_gemm_split", launch_split<8>}, k32x32{"q8_gemm_fused 32x32", launch_fused<FusedShape<32, 32, 1, 1, 2, 2>>},
+    k32x64{"q8_gemm_fused 32x64", launch_fused<FusedShape<32, 64, 1, 2, 2, 2>>}, k64x64{"q8_gemm_fused 64x64", launch_fused<FusedShape<64, 64, 2, 1, 1, 4>>},
+    k64x96{"q8_gemm_fused 64x96", launch_fused<FusedShape<64, 96, 2, 1, 2, 2>>}, k128x128{"q8_gemm_fused 128x128", launch_fused<FusedShape<128, 128, 2, 2, 1, 2>>};
+
+// Which kernel decodes GGUF rows on their way, or none for the two launches; `aligned`: rows as q8_gemm_split reads them. All forms were timed at some 2300 calls, 64 to 8192
+// columns, 64 to 16 000 matrix rows, 1 to 2048 tokens, with operands at hand, the matrix from memory, and both from memory; times below are the first and the last of these.
+//   * Below 384 columns q8_gemm_fused takes longer to begin and end than its products take: q8_gemm_split up to 600 tiles, 1024 of 64 columns (64 -> 640, 700 tokens 3.5
+//     us and 4.0, 32 x 64 4.7 and 5.3, two launches 5.4 and 6.1; 64 -> 512, 2048 tokens 4.2 and 4.9, two launches 5.8 and 6.5; 256 and 320 columns are even, at 448 32 x 32 takes
+//     0.95 of the time). Beyond that 64 x 64 as below, larger tiles not below 512 columns (1600 tokens, 384 -> 700, 64 x 96 8.8 and 10.8, two launches 8.6 and 10.2).
+//   * Up to 16 tokens from 2048 columns on: q8_gemm_split with eight waves, by operands from memory (9 tokens, 4096 -> 4096 11.6 and 13.3, 32 x 32 11.4 and 14.0).
+//   * Else the smallest tile that goes round in one round of the compute units, since a second costs as much as the first however few are in it. 32 x 32 and 32 x 64
+//     gain whatever they fill (203 tokens, 2560 -> 640 8.6 and 11.5, q8_gemm_split 8.9 and 11.9, two launches 15.5 and 16.3).
+//   * 64 x 64 takes as long for one tile as for all (2048 columns 14.5 and 18.5), the two launches less for fewer (16.8 and 17.1 at 152 tiles, 18.1 and 18.8 at 224): seven tenths
+//     of a round, half of one up to 1024 columns or 256 tokens. Beyond 2048 columns operands from memory make it the slower one (512 rows, 1800 tokens, 4096 columns: 0.93 and
+//     1.09 of the two launches' time) but for so few tokens that they are little (150 tokens, 2560 -> 4096 17.1 and 21.8, two launches 21.6 and 22.6).
+//   * 64 x 96 where 64 x 64 would need two rounds: 78 hundredths of one, 75 up to 1024 columns, and within the same columns (1800 tokens, 1024 -> 640 14.0 -> 12.1 and 15.8 -> 14.7).
+//   * 128 x 128 for four rounds of the two launches: nine tenths of a round, from 2048 columns on of several, 85 hundredths up to 1024 (2048 tokens, 2560 -> 2048 60.7 -> 43.0
+//     and 63.7 -> 51.1; at 75 hundredths even with operands at hand and 1.2 times as long from memory).
+// Against the kernels that were chosen by 600 tiles before there was q8_gemm_fused, 512 columns and more: 0.92 of the time on average, 43 of 1716 calls slower by more than 2.5 % in one
+// of the three states, two in their mean.
+const RawRowsKernel* raw_rows_kernel(uint32_t m, uint32_t n, uint32_t k, bool aligned) {
+    const uint64_t units = 256;
     const auto tiles = [&](uint32_t tm, uint32_t tn) { return uint64_t((m + tm - 1) / tm) * ((n + tn - 1) / tn); };
-    const uint64_t steps = (k + 127) / 128, staged_tiles = tiles(kTile, kTile), staged_rounds = staged_tiles < 220 ? 220 : staged_tiles;  // in 256ths
-    uint64_t best = steps * (570 * staged_rounds / 256 + (768ull * m + 392ull * n) / 5000) + 4950 + 550 * staged_rounds / 256;
-    best = best * 9 / 10;
-    const FusedTile* chosen = nullptr;
-    for (const FusedTile& c : choices) {
-        const uint64_t ns = (tiles(c.m, c.n) + 255) / 256 * (steps * c.step_ns + c.ends_ns);
-        if (ns < best) { best = ns; chosen = &c; }
-    }
-    return chosen;
+    // at most that many rounds, their tiles at least `hundredths` of what they could be
+    const auto fill = [&](uint64_t count, uint32_t hundredths, uint64_t rounds = 1) {
+        const uint64_t r = (count + units - 1) / units;
+        return r <= rounds && count * 100 >= hundredths * r * units;
+    };
+    const uint64_t smallest = tiles(32, 32);
+    const bool split = aligned && smallest <= (k < 128 ? 1024 : 600), few_columns = k <= 1024, few_tokens = m <= 256;
+    if (split && (k < 384 || (m <= 16 && k >= 2048 && smallest <= units))) return k < 2048 ? &kSplit4 : &kSplit8;
+    if (k >= 384 && fill(smallest, 0)) return &k32x32;
+    if (k >= 384 && fill(tiles(32, 64), 0)) return &k32x64;
+    if ((k <= 2048 || few_tokens) && fill(tiles(64, 64), few_columns || (few_tokens && k <= 2048) ? 50 : k <= 2048 ? 70 : 75)) return &k64x64;
+    if (k < 512) return nullptr;
+    if ((k <= 2048 || m <= 320) && fill(tiles(64, 96), few_columns ? 75 : 78)) return &k64x96;
+    if (fill(tiles(128, 128), few_columns ? 85 : 90, k < 2048 ? 1 : ~0ull)) return &k128x128;
+    return nullptr;
 }
 
 }  // namespace
@@ -408,7 +531,8 @@ extern "C" int tsp_dense_mm_q8_staged(uint32_t layout, const void* matrix, uint6
     const auto s = static_cast<hipStream_t>(stream);
     if (layout == TSP_LAYOUT_GGUF) {
         const Q8GemmArgs a{input, input_stride_bytes, static_cast<const uint8_t*>(matrix), output, output_stride_bytes, tokens, rows, columns, error_word};
-        if (const FusedTile* tile = fused_tile(tokens, rows, columns)) return tile->launch(a, tile->name, s);
+        const bool aligned = reinterpret_cast<uintptr_t>(input) % 16 == 0 && input_stride_bytes % 16 == 0 && reinterpret_cast<uintptr_t>(matrix) % 4 == 0;
+        if (const RawRowsKernel* kernel = raw_rows_kernel(tokens, rows, columns, aligned)) return kernel->launch(a, kernel->name, s);
     }
     _Float16* const w16 = static_cast<_Float16*>(workspace);
     _Float16* const x16 = reinterpret_cast<_Float16*>(static_cast<uint8_t*>(workspace) + align256(uint64_t(rows) * columns * 2));
