@@ -482,8 +482,8 @@ constexpr RawRowsKernel kSplit4{"q8_gemm_split", launch_split<4>}, kSplit8{"q8_g
 //     and 63.7 -> 51.1; at 75 hundredths even with operands at hand and 1.2 times as long from memory).
 // Against the kernels that were chosen by 600 tiles before there was q8_gemm_fused, 512 columns and more: 0.92 of the time on average, 43 of 1716 calls slower by more than 2.5 % in one
 // of the three states, two in their mean.
-const RawRowsKernel* raw_rows_kernel(uint32_t m, uint32_t n, uint32_t k, bool aligned) {
-    const uint64_t units = 256;
+// `units`: the device's compute units; figures are for 256.
+const RawRowsKernel* raw_rows_kernel(uint32_t m, uint32_t n, uint32_t k, bool aligned, uint64_t units) {
     const auto tiles = [&](uint32_t tm, uint32_t tn) { return uint64_t((m + tm - 1) / tm) * ((n + tn - 1) / tn); };
     // at most that many rounds, their tiles at least `hundredths` of what they could be
     const auto fill = [&](uint64_t count, uint32_t hundredths, uint64_t rounds = 1) {
@@ -491,7 +491,7 @@ const RawRowsKernel* raw_rows_kernel(uint32_t m, uint32_t n, uint32_t k, bool al
         return r <= rounds && count * 100 >= hundredths * r * units;
     };
     const uint64_t smallest = tiles(32, 32);
-    const bool split = aligned && smallest <= (k < 128 ? 1024 : 600), few_columns = k <= 1024, few_tokens = m <= 256;
+    const bool split = aligned && smallest <= (k < 128 ? 4 * units : units * 75 / 32), few_columns = k <= 1024, few_tokens = m <= 256;
     if (split && (k < 384 || (m <= 16 && k >= 2048 && smallest <= units))) return k < 2048 ? &kSplit4 : &kSplit8;
     if (k >= 384 && fill(smallest, 0)) return &k32x32;
     if (k >= 384 && fill(tiles(32, 64), 0)) return &k32x64;
@@ -532,7 +532,14 @@ extern "C" int tsp_dense_mm_q8_staged(uint32_t layout, const void* matrix, uint6
     if (layout == TSP_LAYOUT_GGUF) {
         const Q8GemmArgs a{input, input_stride_bytes, static_cast<const uint8_t*>(matrix), output, output_stride_bytes, tokens, rows, columns, error_word};
         const bool aligned = reinterpret_cast<uintptr_t>(input) % 16 == 0 && input_stride_bytes % 16 == 0 && reinterpret_cast<uintptr_t>(matrix) % 4 == 0;
-        if (const RawRowsKernel* kernel = raw_rows_kernel(tokens, rows, columns, aligned)) return kernel->launch(a, kernel->name, s);
+        static std::atomic<uint64_t> seen{0};
+        static int units_of[64];
+        int device = 0;
+        if (setup_pending(seen, &device)) {
+            TSP_HIP(hipDeviceGetAttribute(&units_of[device], hipDeviceAttributeMultiprocessorCount, device));
+            setup_done(seen, device);
+        }
+        if (const RawRowsKernel* kernel = raw_rows_kernel(tokens, rows, columns, aligned, units_of[device] > 0 ? uint64_t(units_of[device]) : 256)) return kernel->launch(a, kernel->name, s);
     }
     _Float16* const w16 = static_cast<_Float16*>(workspace);
     _Float16* const x16 = reinterpret_cast<_Float16*>(static_cast<uint8_t*>(workspace) + align256(uint64_t(rows) * columns * 2));
