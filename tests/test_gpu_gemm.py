@@ -824,6 +824,27 @@ def test_grouped_moe_rows_past_the_end(gpu, tsp, orc, synth, dn_type, channels, 
     assert float(np.median(err)) <= 2e-5 and float(err.max()) <= 4e-3 and nmse(results[0], declared) <= 1e-7  # the bounds of the cases above
 
 
+def test_grouped_moe_2048_columns_shared_lines(gpu, tsp, orc, synth):
+    """Experts of four tasks and of five on the resident gate/up kernel, which asks for the lines of the one past the caches and of the other through them, each beside an
+    expert of one task, in both loops (tasks of up to 32 rows and of more); the bounds of the larger cases."""
+    channels, hidden, experts, loads = 2048, 256, 64, (256, 257, 1, 33, 300, 224)
+    n = sum(loads)
+    ids = np.random.default_rng(81).permutation(np.repeat(np.random.default_rng(82).permutation(experts)[:len(loads)], loads)).astype(np.uint32)
+
+    def stack(kind, seed, rows, columns):  # eight matrices that the experts share in turn
+        return np.tile(synth.matrix(kind, seed, rows * 8, columns).reshape(8, -1), (experts // 8, 1)).reshape(-1)
+
+    gate, up, down = stack(12, 3471, hidden, channels), stack(12, 3472, hidden, channels), stack(14, 3473, channels, hidden)
+    w = tsp.PlanarMoeWeights(gpu, 12, 14, channels, hidden, experts, gate, up, down)
+    x = synth.round_bf16(synth.activations_f32(3474, (n, channels)))
+    y = tsp.planar_nax_grouped_moe(gpu, w, gpu.upload(ids), gpu.upload(x), n, 1, tsp.GroupedScratch(gpu, n, 1, experts, channels, hidden), y=gpu.full((n, channels), np.nan)).cpu().numpy()
+    assert gpu.error() == 0
+    _, declared = orc.moe_routed_reference(12, 14, gate, up, down, channels, hidden, experts, ids, n, 1, x, stage=12, threads=8)
+    scale = np.maximum(1.0, np.sqrt((declared ** 2).mean(axis=1, keepdims=True)))
+    err = np.abs(y - declared) / np.maximum(scale, np.abs(declared))
+    assert float(np.median(err)) <= 2e-5 and float(err.max()) <= 4e-3 and nmse(y, declared) <= 1e-7
+
+
 # the down kernel that keeps a task's h rows in LDS: one to six steps of 128 hidden units (six take the requests in two halves), one
 # and three groups of 256 channels, tasks of one and of two row tiles
 @pytest.mark.parametrize("dn_type,channels,hidden", [(8, 256, 128), (7, 768, 128), (7, 256, 384), (8, 768, 384), (8, 256, 768), (7, 768, 768)])
