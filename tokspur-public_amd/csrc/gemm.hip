@@ -593,7 +593,7 @@ template <bool ROUTES>
 __global__ __launch_bounds__(512) void tasks_and_rows(TaskLists t, const void* __restrict__ src, uint64_t src_stride_bytes, _Float16* __restrict__ dst,
                                                       _Float16* __restrict__ sx, uint32_t rows, uint32_t columns, uint32_t* error_word) {
     __shared__ __attribute__((aligned(16))) uint32_t counted[ROUTES ? 2048 : 4];
-    __shared__ __attribute__((aligned(16))) uint32_t totals[24], kinds[48];
+    __shared__ __attribute__((aligned(16))) uint32_t totals[24], kinds[56];
     const uint32_t others = 3 + (ROUTES ? t.experts : 0);
     if (blockIdx.x < 3) {
         if (blockIdx.x == 2 && !t.order1) return;
