@@ -825,8 +825,8 @@ def test_grouped_moe_rows_past_the_end(gpu, tsp, orc, synth, dn_type, channels, 
 
 
 def test_grouped_moe_2048_columns_shared_lines(gpu, tsp, orc, synth):
-    """Experts of four tasks and of five on the resident gate/up kernel, which asks for the lines of the one past the caches and of the other through them, each beside an
-    expert of one task, in both loops (tasks of up to 32 rows and of more); the bounds of the larger cases."""
+    """Experts of four tasks and of five on the resident gate/up kernel, beside experts of one task, in both loops: tasks of up to 32 rows, whose lines are asked for past the
+    caches, and of more, whose lines go through them; the bounds of the larger cases."""
     channels, hidden, experts, loads = 2048, 256, 64, (256, 257, 1, 33, 300, 224)
     n = sum(loads)
     ids = np.random.default_rng(81).permutation(np.repeat(np.random.default_rng(82).permutation(experts)[:len(loads)], loads)).astype(np.uint32)

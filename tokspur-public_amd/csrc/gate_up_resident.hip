@@ -12,9 +12,11 @@
 //     read twice per task and none passes through LDS.
 //   * Weights go global -> LDS directly (no registers in between), a tile of 32 rows x one 128-byte line of nibbles +
 //     the rows' scale bytes and d/dmin per request, into a wave-private ring of two stages. Eight neighbouring lanes fetch
-//     one whole cache line. Where an expert has up to four tasks few of its lines are wanted again while they are there, and they pass by the caches: 203
-//     tokens of 2048 x 512 235.3 -> 227.1 us a sublayer. An expert of more tasks (the always-on one, or tokens that agree) keeps its lines: 1000 tokens that all name
-//     the same ten experts 136.5 -> 133.2, 1600 197.2 -> 190.2. (The down kernels and the streaming gate/up lose by it, 143 -> 168 us and 278 -> 285 a launch: there
+//     one whole cache line. An expert with a task of at most 32 rows has no other, or few, so its lines are not wanted again and pass by the caches: 203
+//     tokens of 2048 x 512 235.3 -> 227.1 us a sublayer. Tasks of more rows keep theirs there, for such tasks of one expert run at the same time (the always-on one's, a busy
+//     one's, all where tokens agree: 1600 tokens that all name the same ten experts 188.6 us for the routed products without, 181.3 with, 700 102.9 and 100.2; an expert of 33 to 64 rows
+//     alone pays for it, 400 tokens of 2048 x 768 and 128 experts 134.1 and 135.9). By each expert's own number of tasks instead, every request looks at a flag, and small calls
+//     lose more (12 tokens 23.0 -> 23.4). (The down kernels and the streaming gate/up lose by passing the caches, 143 -> 168 us and 278 -> 285 a launch: there
 //     tasks of one expert and waves side by side share lines.) Nothing but these requests and the epilogue's stores uses the vector memory counter inside
 //     the loop, so each wave waits with an exact count, and since the ring is private no barrier guards it.
 //   * A wave's product over its super-block, d * sum(x * sc*q) - dmin * sum(Sx * mn), is a partial result of a 32 x 32
@@ -91,10 +93,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         gate = pair;
         up = pair + a.spec.planar_expert_bytes;
     };
-    auto request_tile = [&](const uint8_t* base, uint32_t unit, uint32_t stage_offset, bool once) {  // base: one expert (under 4 GiB), uniform
+    auto request_tile = [&](const uint8_t* base, uint32_t unit, uint32_t stage_offset, auto once_tag) {  // base: one expert (under 4 GiB), uniform
         const uint8_t* qs = base + uint64_t(unit) * (32 * bpr * 128);
         const uint32_t dst = my_stage_lds + stage_offset;
-        if (once) {
+        if constexpr (decltype(once_tag)::value) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) load_once_to_lds_16(qs + q * (8 * bpr * 128), qs_lane, dst + q * 1024);
         } else {
@@ -140,16 +142,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         f16x8 sxA[MT];     // activation sums (k-half 0: the eight sub-block sums' high halves, k-half 1: the residuals)
         // ---- the request cursor runs two tiles ahead of the arithmetic: (list position, unit, gate or up)
         uint32_t rk = k0, runit = first_unit(k0), rj = 0, rstage = 0;
-        bool rdone = false, ronce = false;
+        bool rdone = false;
         const uint8_t *rgate, *rup;
         auto enter_task = [&](uint32_t k) {
             const Info t = info_at(k);
             weight_bases(t, rgate, rup);
-            ronce = !t.shares;
         };
         enter_task(k0);
         auto request_next = [&]() {  // past the end of the share the last tile is requested again (unused)
-            request_tile(rj == 0 ? rgate : rup, runit, rstage, ronce);
+            request_tile(rj == 0 ? rgate : rup, runit, rstage, std::bool_constant<MT == 1>{});
             rstage = rstage + kStageBytes == kStages * kStageBytes ? 0 : rstage + kStageBytes;
             if (rdone) return;
             if (rj == 0) { rj = 1; return; }
@@ -237,7 +238,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             f32x16 blk[MT];
             auto steps = [&](auto p_tag) {
                 constexpr int P = decltype(p_tag)::value;
-                // the scales of sub-blocks 2P (low nibbles) and 2P + 1 (high nibbles, in place as 16 q: scale / 16) as one pair
+                // the factors of sub-blocks 2P (low nibbles, 2^8 sc) and 2P + 1 (high nibbles, in place as 16 q: 2^4 sc) as one pair; d makes up for 2^-16 (kQ4Lift)
                 const f16x2 sc = q4_pair_scale<P>(sm.x, sm.y, q4s);
 #pragma unroll
                 for (int hi = 0; hi < 2; ++hi) {

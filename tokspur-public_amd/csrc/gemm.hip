@@ -967,7 +967,9 @@ int grouped_moe(const tsp_grouped_moe* m, const tsp_shared_expert* shared, void*
     // At 2048 columns the resident kernel's parts end together however few the tasks are, and it asks for a task's weights without a start per 128
     // units; with many rows per expert its exchange between the waves weighs more. A sublayer, resident and streaming: 2048 x 512, 512 experts, 260 tokens 252 us and
     // 262, 400 270 and 282, 600 302 and 317, 1000 340 and 348, 1400 (27 routes an expert) 380 and 381, 1800 425 and 419, 2048 449 and 440; 2048 x 768,
-    // 128 experts, 150 162 and 171, 400 186 and 192, 500 (31) 199 and 202, 700 234 and 233, 1000 277 and 271, 1500 354 and 335.
+    // 128 experts, 150 162 and 171, 400 186 and 192, 500 (31) 199 and 202, 700 234 and 233, 1000 277 and 271, 1500 354 and 335. Only the mean can decide here: tokens that
+    // all name the same few experts have many rows each and would be better off with the streaming one (the launch, 700 tokens on ten experts of 2048 x 512 60 and 45 us,
+    // 1000 73 and 59, 203 on eight of 2048 x 768 33 and 27), but the ids are on the device, and a second launch that finds nothing to do would cost every other call.
     // The two add a row's super-blocks up in the same order and with the same roundings.
     const bool stream_gate_up = fast_gate_up && !(routes < 32 * m->experts && resident_gate_up_takes(m->channels, m->hidden));
     auto* order = reinterpret_cast<OrderedTask*>(ws + l.order);

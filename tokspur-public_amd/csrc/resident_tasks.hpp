@@ -9,11 +9,11 @@ namespace tsp {
 constexpr uint32_t kResidentTaskRows = 64;
 constexpr uint32_t kResidentInfoSlots = 32;  // tasks of a workgroup's share kept in LDS, per pass
 
-struct ResidentTask { uint32_t task, expert, start, nrows; bool shared, ok, shares; };  // shares: one of more than four tasks of its expert
+struct ResidentTask { uint32_t task, expert, start, nrows; bool shared, ok; };
 
-// (task, expert, first row, rows | shared << 8 | ok << 9 | shares << 10): one 16-byte LDS slot per task
+// (task, expert, first row, rows | shared << 8 | ok << 9): one 16-byte LDS slot per task
 __device__ __forceinline__ uint4 pack_resident_task(const ResidentTask& t) {
-    return uint4{t.task, t.expert, t.start, t.nrows | (t.shared ? 256u : 0u) | (t.ok ? 512u : 0u) | (t.shares ? 1024u : 0u)};
+    return uint4{t.task, t.expert, t.start, t.nrows | (t.shared ? 256u : 0u) | (t.ok ? 512u : 0u)};
 }
 // The words are the same in every lane (every lane read the same slot): they go to scalar registers.
 __device__ __forceinline__ ResidentTask unpack_resident_task(const uint4& v) {
@@ -22,7 +22,7 @@ __device__ __forceinline__ ResidentTask unpack_resident_task(const uint4& v) {
     t.expert = __builtin_amdgcn_readfirstlane(v.y);
     t.start = __builtin_amdgcn_readfirstlane(v.z);
     const uint32_t w = __builtin_amdgcn_readfirstlane(v.w);
-    t.nrows = w & 255u; t.shared = (w & 256u) != 0; t.ok = (w & 512u) != 0; t.shares = (w & 1024u) != 0;
+    t.nrows = w & 255u; t.shared = (w & 256u) != 0; t.ok = (w & 512u) != 0;
     return t;
 }
 
@@ -39,7 +39,6 @@ __device__ __forceinline__ ResidentTask resolve_resident_task(const uint32_t* __
     t.shared = has_shared && t.expert == experts;
     const uint32_t count = t.shared ? tokens : t.expert < experts ? counts[t.expert] : 0;
     t.ok = (t.expert < experts || t.shared) && count <= tokens && t.start < count;
-    t.shares = count > 4 * kResidentTaskRows;
     t.nrows = t.ok ? (count - t.start < kResidentTaskRows ? count - t.start : kResidentTaskRows) : 0;
     if (!t.ok) { t.expert = 0; t.start = 0; t.shared = false; }
     return t;
