@@ -277,8 +277,8 @@ def test_dense_mm_q8_staged(gpu, tsp, orc, synth, tokens, cols, rows):
 
 @pytest.mark.parametrize("tokens,cols,rows", [(33, 2048, 31), (31, 2112, 65), (2, 64, 1), (65, 576, 33), (96, 192, 6400), (97, 64, 6401)])
 def test_dense_mm_q8_staged_tiles(gpu, tsp, synth, tokens, cols, rows):
-    # the columns shared out over eight waves (2048 columns and more) or four, fewer steps than waves, ragged tiles; the last shape is
-    # more tiles than that form takes. A weight and an activation are rounded to halves: 2^-11 each, so 2^-10 of the sum of |w| |x|.
+    # one tile and many, fewer steps than waves, a half step at the end, ragged tiles on both sides (which kernel has which call: test_dense_mm_q8_staged_kernels).
+    # A weight and an activation are rounded to halves: 2^-11 each, so 2^-10 of the sum of |w| |x|.
     w = synth.matrix(8, 2400 + cols, rows, cols)
     x = synth.activations_f32(2401 + tokens, (tokens, cols))
     got = tsp.dense_mm_q8_staged(gpu, tsp.LAYOUT_GGUF, gpu.upload(w), gpu.upload(x), tokens, cols, rows).cpu().numpy()

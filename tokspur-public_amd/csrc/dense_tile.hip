@@ -144,8 +144,8 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
     const uint32_t sx_at = kSxAt + (wm * (RT * 32) + col) * 32 + khalf * 16;
 
     const Q4Masks masks = q4_masks();
-    // Rounded weights: masks in scalar registers. What a mask saves in vector registers is not what they wait for, and the loop's order comes out the better one
-    // (2048 x 8192 x 2048 70.9 -> 70.3 us, 1500 x 8192 x 2560 75.0 -> 74.3).
+    // Rounded weights: masks in scalar registers. Two mixed-precision multiply-adds follow each and here, so its rate is not what they wait for, and with the registers left to
+    // other values the loop's order comes out the better one (in vector registers 2048 x 8192 x 2048 takes 70.9 us for 70.3, 1500 x 8192 x 2560 75.0 for 74.3).
     Q4Masks rounded_masks{0x000f000fu, 0x00f000f0u};
     asm volatile("" : "+s"(rounded_masks.lo), "+s"(rounded_masks.hi));
     const Q4ScaleConsts q4s = q4_scale_consts();

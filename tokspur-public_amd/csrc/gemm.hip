@@ -11,8 +11,9 @@
 // The second term (Q4_K minima) is one more MFMA per super-block against the per-sub-block activation
 // sums Sx, carried as a hi+lo pair of f16. Nothing is rounded to f16 that is not an exact integer (Q6_K
 // products above 2048 round to even, a 2^-12 relative step), so results track the f32-dequantised
-// reference to f32-accumulation accuracy, and unpacking costs ~1.4 VALU operations per weight (mask,
-// byte permute into 1024+q, one packed f16 fma) instead of ~3 for convert + f32 fma + f16 round.
+// reference to f32-accumulation accuracy. Unpacking a Q6_K weight costs ~1.4 VALU operations (mask,
+// byte permute into 1024+q, one packed f16 fma) instead of ~3 for convert + f32 fma + f16 round; a Q4_K weight
+// ~1.1: masked nibbles as subnormal halves, times the scale that is (sc*q) * 2^-16, and d carries 2^16 (kQ4Lift).
 //
 // One workgroup = 4 waves = one task (<= 64 activation rows of one expert, or one 64-row slab of a dense
 // matrix) x 256 weight rows. Each wave owns 64 weight rows (two 32-wide MFMA column tiles) and all 64

@@ -178,7 +178,8 @@ __device__ __forceinline__ HdrQ4 decode_hdr_q4k(const RawHdrQ4& r) {
 // instead of a mask and two byte permutes per four. A masked pair of nibbles is two subnormal halves, q * 2^-24 or, where the high ones sit, 16 q * 2^-24;
 // times 2^8 sc or 2^4 sc that is sc * q * 2^-16, as exact as sc * q itself (a scale byte of 255 still fits), in two instructions for two
 // weights, and the block's d makes up for the power of two (kQ4Lift). An and of two vector registers issues at twice the rate of an and-or, or of an and
-// with a scalar register, when two waves share a SIMD (1.0 against 1.9 ns an instruction): hence no bits to be or'ed in, and the masks in vector registers.
+// with a scalar register, when two waves share a SIMD (1.0 against 1.9 ns an instruction): hence no bits to be or'ed in, and the masks in vector registers. (Where what
+// follows an and is two mixed-precision multiply-adds a pair, weights8_q4_swapped, it is not the ands that are waited for: dense_tile.hip keeps its masks for those in scalar registers.)
 struct Q4Masks { uint32_t lo, hi; };
 __device__ __forceinline__ Q4Masks q4_masks() {
     Q4Masks m{0x000f000fu, 0x00f000f0u};
